@@ -160,7 +160,7 @@ def _big_weight(name, shape, seed):
     if name.endswith("norm"):
         return _rand(seed, name, shape, 0.1).add_(1.0)
     leaf = name.rsplit(".", 1)[-1]
-    return _rand(seed, name, shape, {"embed": 1.0, "o": 0.005, "down": 0.005, "w2": 0.002, "router": 0.06}.get(leaf, 0.02))
+    return _rand(seed, name, shape, {"embed": 1.0, "o": 0.0025, "down": 0.0025, "w2": 0.001, "router": 0.06}.get(leaf, 0.02))
 
 
 def _big_kv(cfg, layer, n, seed):
@@ -175,12 +175,13 @@ def _layer_config(case):
 
 
 def _layer_value(name, shape, seed, kind):
-    """One checkpoint tensor of a layered decoder (bf16), each kind of parameter in its usual range.  The norms that
-    Sigudra puts on each sublayer's output are small, so that the residual stream leads."""
+    """One checkpoint tensor of a layered decoder (bf16), each kind of parameter in its usual range.  Single experts add
+    little to the residual stream (a token whose chosen experts nearly tie may go either way): their output is small,
+    as are the norms that Sigudra puts on each sublayer's output, and Gezavik's softmax router decides."""
     leaf = name.rsplit(".", 1)[-1]
     f = lambda uniform=False: _rand(seed, name, shape, dtype=torch.float32, uniform=uniform)  # noqa: E731
     if leaf in ("norm", "norm1", "norm2", "norm1b", "norm2b", "out") and len(shape) == 1:
-        t = (1.0 + 0.1 * f()) * (0.25 if kind == "sigudra" and leaf in ("norm1", "norm2") else 1.0)
+        t = (1.0 + 0.1 * f()) * ({"norm1": 0.25, "norm2": 0.08}.get(leaf, 1.0) if kind == "sigudra" else 1.0)
     elif leaf == "alpha":
         t = 0.4 + 0.4 * f(True)
     elif leaf == "A_log":
@@ -204,6 +205,10 @@ def _layer_value(name, shape, seed, kind):
         t = f()
     else:
         t = f() * shape[-1] ** -0.5
+        if leaf == "down" and ".e" in name:
+            t = 0.15 * t
+        elif leaf == "router" and kind == "gezavik":
+            t = 3.0 * t
     return t.to(torch.bfloat16)
 
 
@@ -435,20 +440,18 @@ def work(case):
 
 
 def tolerance(case):
-    """From the error against float64 that the start's code shows: two to four times it (bf16 sums in another order,
-    and rows whose chosen experts nearly tie)."""
+    """From the error against float64 that bf16 and fp8 show here: two to four times it, sums in another order included;
+    single values of a row whose chosen experts nearly tie may be off by more."""
     kind = case["kind"]
     if kind == "search":       # f32 dot products; rows whose scores nearly tie may change places
         return {"rel": 1e-5, "max": 1e-3, "differ": 0.01}
     if kind == "embed":        # seen: 0.007
         return {"rel": 0.02}
-    if kind == "chat":         # 32 layers in bf16, seen: 0.028
-        return {"rel": 0.07}
-    if kind == "moe":          # fp8 products, seen: 0.03 to 0.035
-        return {"rel": 0.1}
+    if kind in ("chat", "moe"):
+        return {"rel": 0.03}
     if case["dtype"] == "fp32":     # seen: up to 6e-6
         return {"rel": 3e-5, "differ": 0.01}
-    return {"rel": 0.08, "differ": 0.01}      # seen: up to 0.03
+    return {"rel": 0.03, "max": 0.99, "differ": 0.01}
 
 
 # ----------------------------------------------------------------------------------------------
