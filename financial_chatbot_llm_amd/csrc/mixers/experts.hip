@@ -1,0 +1,447 @@
+// Routed feed-forwards: the chosen experts of every token as two grouped matrix products over rows sorted by expert,
+//     act[r] = unit(W1[e] x[token(r)])      W1 [N1, W] per expert (gated: gate and up rows in turns of 16)
+//     ys[r]  = W2[e] act[r]                 W2 [W, F] per expert
+// Three launches and no host read of the bucket sizes:
+//   plan    one block: a stable counting sort of the (token, choice) pairs by expert and the list of row tiles
+//   GEMM 1  gathers the tokens' rows while it stages them, applies the gated unit in its epilogue
+//   GEMM 2  sorted rows in and out; mx_moe_combine sums a token's rows
+// Weights are stored as the MFMA reads them: pieces of 1 KiB, [row group of 16][K step of 64 bytes][64 lanes][16 B],
+// lane l holding row l % 16 and the 16 bytes at 16 * (l / 16); rows and K padded with zeros (whole groups, K to 128 B).
+// Both storage types share the code: a 16-byte operand is 8 bf16 (one 16x16x32 MFMA) or 4 f32 (four 16x16x4 MFMAs whose
+// step j takes K element 4 g + j of both operands).  Accumulation is f32; the unit sees the f32 sums.
+//
+// Two forms, chosen by the rows an expert gets on average (the bucket sizes stay on the device):
+//   tile    128 W rows x 64 or 128 tokens per block, both operands through a two-stage LDS ring filled by LDS-DMA,
+//           two or three blocks per CU: bound by the matrix cores.  4096 tokens, width 2048, 32 experts of 1024, top 4,
+//           bf16: 320 us for both products (650 TFLOP/s); 31 pairs of library products and the host's wait for the
+//           bucket sizes took 1.3 ms.
+//   stream  32 or 64 W rows x 16 tokens per block, the four waves split K and the weights go straight to registers,
+//           1 KiB per load: bound by the weight stream.  64 tokens of the same layer: 49 + 23 us, 5.5 and 5.9 TB/s
+//           (batched library products of all rows with all experts, their unit and combine: 125 us).
+#include "mx_common.h"
+
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+template <int N> struct Steps { static constexpr int value = N; };
+
+enum { UNIT_NONE = 0, UNIT_CLAMP = 1, UNIT_SILU = 2, UNIT_GELU = 3, UNIT_RELU2 = 4 };
+
+// 16 zero bytes: what a lane stages for K positions behind a row's end
+__device__ uint4 g_zero16;
+
+template <typename T> __device__ __forceinline__ f32x4 mma16(uint4 a, uint4 b, f32x4 c);
+template <> __device__ __forceinline__ f32x4 mma16<bf16>(uint4 a, uint4 b, f32x4 c) {
+  union { uint4 u; bf16x8 v; } x, y;
+  x.u = a;
+  y.u = b;
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.v, y.v, c, 0, 0, 0);
+}
+template <> __device__ __forceinline__ f32x4 mma16<float>(uint4 a, uint4 b, f32x4 c) {
+  union { uint4 u; f32x4 v; } x, y;
+  x.u = a;
+  y.u = b;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(x.v[j], y.v[j], c, 0, 0, 0);
+  return c;
+}
+
+struct ExpertGemm {
+  const void* x;        // rows of ldx elements: token rows (top > 0: sorted row r reads row src[r] / top) or sorted rows
+  long ldx;
+  int kbytes;           // bytes of a row that count
+  const int* src;       // sorted row -> pair
+  int top;
+  const int4* tiles;    // (expert, first sorted row, rows, -); rows 0: none
+  int ntiles;           // entries of the list
+  const char* w;        // pieces, expert stride wstride bytes
+  long wstride;
+  int kt;               // pieces per row group
+  int groups;           // row groups
+  void* y;              // sorted rows of ldy elements, columns 0 .. ncol - 1 written
+  long ldy;
+  int ncol;
+  int unit;
+  float limit, alpha;
+  const float* scale;   // per pair, on the expert's input (or null)
+};
+
+// One block: pairs 0 .. P-1 (expert idx[i], identity experts >= E stay out) in a stable order by expert.  Every wave
+// owns a contiguous run of pairs; lanes with equal experts find each other by ballots over the index bits, so no
+// atomics, and pos / src are the same on every run.  Bound by latency: NC > 0 keeps a wave's run of NC * 64 indices in
+// registers, all loads in flight at once (16,384 pairs: 34 us as a loop over memory).  LDS: cnt [waves][E], base [E].
+template <int NC>
+__global__ void __launch_bounds__(1024) expert_plan_kernel(const int* __restrict__ idx, int P, int E, int bits, int mt,
+                                                           int ntiles, int* __restrict__ pos, int* __restrict__ src,
+                                                           int4* __restrict__ tiles) {
+  extern __shared__ int lds[];
+  const int nw = blockDim.x >> 6, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int* cnt = lds + w * E;
+  int* base = lds + nw * E;
+  __shared__ int tiles_used;
+  const int per = NC > 0 ? NC * 64 : (P + nw * 64 - 1) / (nw * 64) * 64, i0 = w * per, i1 = min(P, i0 + per);
+  const int nc = NC > 0 ? NC : (i1 - i0 + 63) / 64;
+  int held[NC > 0 ? NC : 1];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) held[c] = i0 + c * 64 + lane < i1 ? idx[i0 + c * 64 + lane] : E;
+  auto expert = [&](int c) { return NC > 0 ? held[c] : (i0 + c * 64 + lane < i1 ? idx[i0 + c * 64 + lane] : E); };
+  for (int e = threadIdx.x; e < nw * E; e += blockDim.x) lds[e] = 0;
+  __syncthreads();
+  auto peers = [&](int e) {
+    unsigned long long m = __ballot(e < E);
+    for (int b = 0; b < bits; ++b) {
+      const unsigned long long s = __ballot((e >> b) & 1);
+      m &= (e >> b) & 1 ? s : ~s;
+    }
+    return m;
+  };
+#pragma unroll
+  for (int c = 0; c < nc; ++c) {
+    const int e = expert(c);
+    const unsigned long long m = peers(e);
+    if (e < E && __ffsll(m) - 1 == lane) cnt[e] += __popcll(m);
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < E; e += blockDim.x) {        // this expert's first place per wave, and its total
+    int t = 0;
+    for (int v = 0; v < nw; ++v) {
+      const int c = lds[v * E + e];
+      lds[v * E + e] = t;
+      t += c;
+    }
+    base[e] = t;
+  }
+  __syncthreads();
+  if (w == 0) {                                              // exclusive sums over the experts: rows and tiles
+    int rows = 0, nt = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int e = e0 + lane, c = e < E ? base[e] : 0, t = (c + mt - 1) / mt;
+      int sc = c, st = t;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int a = __shfl_up(sc, o, 64), b = __shfl_up(st, o, 64);
+        if (lane >= o) sc += a, st += b;
+      }
+      const int r0 = rows + sc - c, t0 = nt + st - t;
+      if (e < E) base[e] = r0;
+      for (int k = 0; k < t; ++k)
+        if (t0 + k < ntiles) tiles[t0 + k] = make_int4(e, r0 + k * mt, min(mt, c - k * mt), 0);
+      rows += __shfl(sc, 63, 64);
+      nt += __shfl(st, 63, 64);
+    }
+    if (lane == 0) tiles_used = nt;
+  }
+  __syncthreads();
+  for (int t = tiles_used + threadIdx.x; t < ntiles; t += blockDim.x) tiles[t] = make_int4(0, 0, 0, 0);
+#pragma unroll
+  for (int c = 0; c < nc; ++c) {
+    const int i = i0 + c * 64 + lane, e = expert(c);
+    const unsigned long long m = peers(e);
+    if (e < E) {
+      const int at = base[e] + cnt[e] + __popcll(m & ((1ull << lane) - 1));
+      pos[i] = at;
+      src[at] = i;
+    } else if (i < i1) {
+      pos[i] = 0;
+    }
+    __builtin_amdgcn_wave_barrier();                         // every lane has read its count
+    if (e < E && __ffsll(m) - 1 == lane) cnt[e] += __popcll(m);
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+__device__ __forceinline__ float unit_value(int unit, float g, float u, float limit, float alpha) {
+  if (unit == UNIT_CLAMP) {
+    g = fminf(g, limit);
+    u = fminf(fmaxf(u, -limit), limit);
+    return g * mx_sigmoid(alpha * g) * (u + 1.0f);
+  }
+  if (unit == UNIT_SILU) return mx_silu(g) * u;
+  const float z = 0.7978845608028654f * (g + 0.044715f * g * g * g);   // gelu, tanh form
+  return 0.5f * g * (1.0f + mx_tanh(z)) * u;
+}
+
+// four adjacent output columns c .. c + 3 of sorted row r: gate and up sums, or one sum
+template <typename T, bool GLU>
+__device__ __forceinline__ void expert_store(const ExpertGemm& a, long r, int c, f32x4 g, f32x4 u) {
+  if (c >= a.ncol) return;
+  typedef T vec __attribute__((ext_vector_type(4)));
+  if (GLU && a.scale != nullptr) {
+    const float s = a.scale[a.src[r]];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) g[j] *= s, u[j] *= s;
+  }
+  vec o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float v = g[j];
+    if (GLU) v = unit_value(a.unit, g[j], u[j], a.limit, a.alpha);
+    else if (a.unit == UNIT_RELU2) v = fmaxf(v, 0.f) * fmaxf(v, 0.f);
+    o[j] = (T)v;
+  }
+  T* y = static_cast<T*>(a.y) + r * a.ldy + c;
+  if (c + 4 <= a.ncol && a.ldy % 4 == 0) {
+    *reinterpret_cast<vec*>(y) = o;
+  } else {
+    for (int j = 0; j < 4 && c + j < a.ncol; ++j) y[j] = o[j];
+  }
+}
+
+// row of x that sorted row r reads
+__device__ __forceinline__ const char* expert_row(const ExpertGemm& a, int r, int es) {
+  return static_cast<const char*>(a.x) + (a.top > 0 ? a.src[r] / a.top : r) * a.ldx * es;
+}
+
+// ---- tile form ---------------------------------------------------------------------------------------------------
+// 256 threads = 4 waves as 2 (W rows) x 2 (tokens), a wave's 64 x 16 MF sub-tile as 4 x MF accumulators (A = W: a
+// lane's four registers are adjacent output columns).  A stage is 128 bytes of K: the W image keeps the pieces'
+// order, the X image has rows of 128 B whose 16-B chunks are swizzled by (row / 2) % 8 (conflict-free b128 reads).
+template <typename T, int MF, bool GLU>
+__global__ void __launch_bounds__(256, MF == 4 ? 2 : 3) expert_tile_kernel(ExpertGemm a) {
+  constexpr int MT = 32 * MF, WIMG = 16384, STG = WIMG + MT * 128, ES = sizeof(T);
+  constexpr int XP = MT / 32;             // 1-KiB pieces of the X image per wave
+  __shared__ __attribute__((aligned(1024))) char smem[2 * STG];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wa = w >> 1, wb = w & 1, g = lane >> 4, col = lane & 15;
+  // four neighbouring tiles -- mostly one expert's -- take all column blocks in turn on one XCD: their W panels and
+  // token rows meet in its L2; the groups of four go round the XCDs, as the end of the list is empty
+  const int nt = (a.groups + 7) / 8, per = 4 * nt, local = blockIdx.x >> 3;
+  const int t = ((local / per) * 8 + (blockIdx.x & 7)) * 4 + (local % per) % 4, nb = (local % per) / 4;
+  if (t >= a.ntiles) return;
+  const int4 tile = a.tiles[t];
+  const int rows = tile.z;
+  if (rows == 0) return;
+
+  const char* wsrc[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {           // piece p = 4 w + i of the stage: row group p / 2, K step p % 2
+    const int p = 4 * w + i;
+    wsrc[i] = a.w + tile.x * a.wstride + ((long)min(nb * 8 + p / 2, a.groups - 1) * a.kt + p % 2) * 1024 + lane * 16;
+  }
+  const char* xsrc[XP];
+  int xoff[XP];
+#pragma unroll
+  for (int i = 0; i < XP; ++i) {
+    const int r = 8 * (w * XP + i) + lane / 8;
+    xsrc[i] = expert_row(a, tile.y + min(r, rows - 1), ES);
+    xoff[i] = 16 * ((lane % 8) ^ ((r >> 1) & 7));
+  }
+  const char* zero = reinterpret_cast<const char*>(&g_zero16);
+  const unsigned lds0 = (unsigned)(uintptr_t)((__attribute__((address_space(3))) char*)smem);
+  auto load = [&](const char* gp, unsigned dst) {
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep)
+                 : "v"(gp), "s"(dst)
+                 : "memory");
+  };
+  auto stage = [&](int s) {
+    const unsigned buf = lds0 + (s & 1) * STG;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) load(wsrc[i] + (long)s * 2048, buf + (4 * w + i) * 1024);
+#pragma unroll
+    for (int i = 0; i < XP; ++i) {
+      const int off = s * 128 + xoff[i];
+      load(off < a.kbytes ? xsrc[i] + off : zero, buf + WIMG + (w * XP + i) * 1024);
+    }
+  };
+  f32x4 acc[4][MF];
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+#pragma unroll
+    for (int u = 0; u < MF; ++u) acc[f][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int ns = a.kt / 2;
+  stage(0);
+  for (int s = 0; s < ns; ++s) {
+    // this wave's pieces have landed, then everybody's; all reads of the other buffer are done
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (s + 1 < ns) stage(s + 1);
+    const char* wi = smem + (s & 1) * STG + wa * 8192 + lane * 16;
+    const char* xi = smem + (s & 1) * STG + WIMG + (wb * 16 * MF + col) * 128;
+    uint4 av[4][2], bv[MF][2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+      for (int f = 0; f < 4; ++f) av[f][kk] = *reinterpret_cast<const uint4*>(wi + (2 * f + kk) * 1024);
+#pragma unroll
+      for (int u = 0; u < MF; ++u)
+        bv[u][kk] = *reinterpret_cast<const uint4*>(xi + u * 2048 + (((4 * kk + g) ^ ((col >> 1) & 7)) << 4));
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int f = 0; f < 4; ++f)
+#pragma unroll
+        for (int u = 0; u < MF; ++u) acc[f][u] = mma16<T>(av[f][kk], bv[u][kk], acc[f][u]);
+  }
+#pragma unroll
+  for (int u = 0; u < MF; ++u) {
+    const int m = wb * 16 * MF + u * 16 + col;
+    if (m >= rows) continue;
+    const int G = nb * 8 + wa * 4;
+    if (GLU) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        if (G + 2 * q < a.groups)
+          expert_store<T, true>(a, tile.y + m, (G / 2 + q) * 16 + 4 * g, acc[2 * q][u], acc[2 * q + 1][u]);
+    } else {
+#pragma unroll
+      for (int f = 0; f < 4; ++f)
+        if (G + f < a.groups) expert_store<T, false>(a, tile.y + m, (G + f) * 16 + 4 * g, acc[f][u], acc[f][u]);
+    }
+  }
+}
+
+// ---- stream form -------------------------------------------------------------------------------------------------
+// NF row groups x 16 tokens per block; wave w takes the w-th quarter of the pieces, the partial sums meet in LDS.
+template <typename T, int NF, bool GLU>
+__global__ void __launch_bounds__(256) expert_stream_kernel(ExpertGemm a) {
+  constexpr int ES = sizeof(T), UN = 8;
+  __shared__ f32x4 red[4][NF][64];
+  const int4 tile = a.tiles[blockIdx.y];
+  const int rows = tile.z;
+  if (rows == 0) return;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, col = lane & 15;
+  const int G = blockIdx.x * NF;
+  const uint4* wp[NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+    wp[f] = reinterpret_cast<const uint4*>(a.w + tile.x * a.wstride + (long)min(G + f, a.groups - 1) * a.kt * 1024) + lane;
+  const char* xp = expert_row(a, tile.y + min(col, rows - 1), ES) + 16 * g;
+  const char* zero = reinterpret_cast<const char*>(&g_zero16);
+  f32x4 acc[NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int k0 = a.kt * w / 4, k1 = a.kt * (w + 1) / 4;
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  auto steps = [&](int k, auto count) {
+    constexpr int U = decltype(count)::value;
+    uint4 av[U][NF], bv[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+        const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wp[f] + (long)(k + j) * 64));
+        av[j][f] = make_uint4(v.x, v.y, v.z, v.w);
+      }
+      const int off = (k + j) * 64;
+      bv[j] = *reinterpret_cast<const uint4*>(off + 16 * g < a.kbytes ? xp + off : zero);
+    }
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+#pragma unroll
+      for (int f = 0; f < NF; ++f) acc[f] = mma16<T>(av[j][f], bv[j], acc[f]);
+  };
+  int k = k0;
+  for (; k + UN <= k1; k += UN) steps(k, Steps<UN>{});
+  for (; k < k1; ++k) steps(k, Steps<1>{});
+#pragma unroll
+  for (int f = 0; f < NF; ++f) red[w][f][lane] = acc[f];
+  __syncthreads();
+  auto total = [&](int i) {
+    f32x4 s = red[0][i][lane];
+#pragma unroll
+    for (int v = 1; v < 4; ++v) s += red[v][i][lane];
+    return s;
+  };
+  constexpr int ITEMS = GLU ? NF / 2 : NF;
+  for (int f = w; f < ITEMS; f += 4) {
+    if (col >= rows) continue;
+    if (GLU) {
+      if (G + 2 * f < a.groups)
+        expert_store<T, true>(a, tile.y + col, (G / 2 + f) * 16 + 4 * g, total(2 * f), total(2 * f + 1));
+    } else if (G + f < a.groups) {
+      const f32x4 s = total(f);
+      expert_store<T, false>(a, tile.y + col, (G + f) * 16 + 4 * g, s, s);
+    }
+  }
+}
+
+// Tokens per tile, from the rows an expert gets on average.  A tile of 16 streams the weights once per 16 rows, a wider
+// one wastes matrix work on rows that are not there but reads them once.  Both products, width 2048, 32 experts of 1024,
+// bf16 (us, tiles of 16 / 64 / 128): 8 rows on average 81 / 84 / 87, 12: 86 / 85 / 87, 24: 118 / 87 / 89, 48: 172 / 90 /
+// 96, 64: 209 / 127 / 98, 192: - / 183 / 148, 512: - / 355 / 320.  f32 products are bound by the matrix cores much
+// earlier and gain nothing from 128 rows (width 1024, experts of 512): 8: 47 / 69, 24: 68 / 71, 32: 83 / 71 / 119,
+// 96: 161 / 123 / 126, 512: - / 505 / 549.
+int tile_rows(long pairs, int experts, int dt) {
+  const long avg = pairs / experts;
+  if (dt == 1) return avg <= 24 ? 16 : 64;
+  return avg <= 12 ? 16 : (avg <= 56 ? 64 : 128);
+}
+
+template <typename T, bool GLU>
+int expert_launch(const ExpertGemm& a, int mt, hipStream_t st) {
+  if (mt >= 64) {
+    const long grid = (long)((a.ntiles + 31) / 32) * 32 * ((a.groups + 7) / 8);
+    if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
+    if constexpr (sizeof(T) == 2) {
+      if (mt == 128) {
+        expert_tile_kernel<T, 4, GLU><<<(unsigned)grid, 256, 0, st>>>(a);
+        return (int)hipGetLastError();
+      }
+    }
+    expert_tile_kernel<T, 2, GLU><<<(unsigned)grid, 256, 0, st>>>(a);
+  } else {
+    if (a.ntiles > 65535) return (int)hipErrorInvalidValue;
+    const bool wide = (long)a.ntiles * (a.groups / 4) >= 512;       // enough blocks of 64 W rows to fill the chip
+    const dim3 grid((a.groups + (wide ? 3 : 1)) / (wide ? 4 : 2), a.ntiles);
+    if (wide) expert_stream_kernel<T, 4, GLU><<<grid, 256, 0, st>>>(a);
+    else expert_stream_kernel<T, 2, GLU><<<grid, 256, 0, st>>>(a);
+  }
+  return (int)hipGetLastError();
+}
+
+}  // namespace
+
+// h [T, >= W] (row stride ldh), idx int32 [T, top] (>= E: an identity expert, no row here); w1 / w2: pieces as above, k1 / k2
+// pieces per row group, g1 / g2 row groups per expert (gated units: g1 counts gate and up groups); unit: UNIT_*;
+// scale f32 [T, top] on the experts' inputs (gated units) or null; act [T * top, lda], ys [T * top, W]: scratch of the
+// storage type dt, lda >= F a multiple of 16 bytes; iws: ints, pos [T * top] | src
+// [T * top] (each rounded up to 4) | tiles int4 [T * top / 16 + min(T * top, E) + 1]; afterwards pos is every pair's row of ys.
+MX_API int mx_experts(const void* h, long ldh, const int* idx, int T, int top, int E, int W, int F, const void* w1, int k1,
+                      int g1, const void* w2, int k2, int g2, int unit, float limit, float alpha, const float* scale,
+                      void* act, long lda, void* ys, int* iws, int dt, hipStream_t st) {
+  if (T <= 0) return 0;
+  const int es = dt == 1 ? 4 : 2;
+  const long P = (long)T * top;
+  const bool glu = unit == UNIT_CLAMP || unit == UNIT_SILU || unit == UNIT_GELU;
+  if (top < 1 || E < 1 || E > 8192 || P > 0x3fffffff || k1 % 2 || k2 % 2 || (long)k1 * 64 < (long)W * es || (long)k2 * 64 < lda * es ||
+      lda < F || lda * es % 16 || (long)W * es % 16 || ldh * es % 16 || ((size_t)h | (size_t)act | (size_t)w1 | (size_t)w2) % 16 ||
+      (size_t)iws % 16 || (glu ? g1 % 2 || g1 / 2 * 16 < lda : g1 * 16 < lda) || g2 * 16 < W || unit < 0 || unit > UNIT_RELU2 ||
+      (scale != nullptr && !glu))
+    return (int)hipErrorInvalidValue;
+  const int mt = tile_rows(P, E, dt);
+  const int ntiles = (int)(P / mt + (P < E ? P : E));
+  int* pos = iws;
+  int* src = iws + (P + 3) / 4 * 4;
+  int4* tiles = reinterpret_cast<int4*>(src + (P + 3) / 4 * 4);
+  int bits = 0;
+  while ((1 << bits) < E) ++bits;
+  int nw = (int)((P + 63) / 64);
+  nw = nw < 1 ? 1 : (nw > 16 ? 16 : nw);
+  while (nw > 1 && (long)(nw + 1) * E > 16000) --nw;
+  if ((long)(nw + 1) * E * 4 > 65536 - 64) return (int)hipErrorInvalidValue;
+  const long run = (P + nw * 64 - 1) / (nw * 64);            // chunks of 64 pairs per wave
+  const size_t lds = (size_t)(nw + 1) * E * 4;
+#define PLAN(NC) expert_plan_kernel<NC><<<1, nw * 64, lds, st>>>(idx, (int)P, E, bits, mt, ntiles, pos, src, tiles)
+  if (run <= 2) PLAN(2);
+  else if (run <= 8) PLAN(8);
+  else if (run <= 16) PLAN(16);
+  else if (run <= 32) PLAN(32);
+  else PLAN(0);
+#undef PLAN
+  int rc = (int)hipGetLastError();
+  if (rc) return rc;
+  ExpertGemm a{h, ldh, W * es, src, top, tiles, ntiles, (const char*)w1, (long)g1 * k1 * 1024, k1, g1, act, lda, (int)lda,
+               unit, limit, alpha, scale};
+  ExpertGemm b{act, lda, (int)lda * es, src, 0, tiles, ntiles, (const char*)w2, (long)g2 * k2 * 1024, k2, g2, ys, W, W,
+               UNIT_NONE, 0.f, 0.f, nullptr};
+  if (glu) MX_DISPATCH(dt, TT, rc = expert_launch<TT, true>(a, mt, st));
+  else MX_DISPATCH(dt, TT, rc = expert_launch<TT, false>(a, mt, st));
+  if (rc) return rc;
+  MX_DISPATCH(dt, TT, rc = expert_launch<TT, false>(b, mt, st));
+  return rc;
+}

@@ -309,23 +309,33 @@ __global__ void route_biased_kernel(const float* __restrict__ z, const float* __
 }
 
 // out[t] = sum_k w[t,k] * src(t,k) (+ shared[t]):  src is the token's own input row h[t] for an
-// identity expert (index >= E), else row pos[t,k] of the expert-sorted outputs ys.
-template <typename T>
-__global__ void moe_combine_kernel(const T* __restrict__ ys, const int* __restrict__ pos, const int* __restrict__ idx,
+// identity expert (index >= E), else row pos[t,k] of the expert-sorted outputs ys; w null: weights 1.
+// One block per token, V adjacent columns per access (V > 1: rows, strides and W in whole 16-byte units).  Bound by the
+// top + 2 rows it moves: 4096 tokens of 2048 bf16, top 4: 23 us, 72 with single-element accesses.
+template <typename T, int V>
+__global__ void moe_combine_kernel(const T* __restrict__ ys, long sy, const int* __restrict__ pos, const int* __restrict__ idx,
                                    const float* __restrict__ wts, const T* __restrict__ h, long sh,
                                    const T* __restrict__ shared, long ssh, int E, int top, int W,
                                    T* __restrict__ out) {
+  typedef T vec __attribute__((ext_vector_type(V)));
   const long t = blockIdx.x;
-  for (int c = threadIdx.x; c < W; c += blockDim.x) {
-    float acc = shared != nullptr ? ldf(shared + t * ssh + c) : 0.f;
+  for (int c = threadIdx.x * V; c < W; c += blockDim.x * V) {
+    float acc[V];
+    vec v = vec{};
+    if (shared != nullptr) v = *reinterpret_cast<const vec*>(shared + t * ssh + c);
+#pragma unroll
+    for (int j = 0; j < V; ++j) acc[j] = (float)v[j];
     for (int k = 0; k < top; ++k) {
       const int e = idx[t * top + k];
-      const float w = wts[t * top + k];
+      const float w = wts != nullptr ? wts[t * top + k] : 1.f;
       if (w == 0.f) continue;
-      const float v = e >= E ? ldf(h + t * sh + c) : ldf(ys + (long)pos[t * top + k] * W + c);
-      acc += w * v;
+      v = *reinterpret_cast<const vec*>(e >= E ? h + t * sh + c : ys + (long)pos[t * top + k] * sy + c);
+#pragma unroll
+      for (int j = 0; j < V; ++j) acc[j] += w * (float)v[j];
     }
-    stf(out + t * W + c, acc);
+#pragma unroll
+    for (int j = 0; j < V; ++j) v[j] = (T)acc[j];
+    *reinterpret_cast<vec*>(out + t * W + c) = v;
   }
 }
 
@@ -450,11 +460,21 @@ MX_API int mx_route_biased(const float* z, const float* bias, int E, int top, in
   MX_RETURN_LAUNCH();
 }
 
-MX_API int mx_moe_combine(const void* ys, const int* pos, const int* idx, const float* wts, const void* h, long sh,
+MX_API int mx_moe_combine(const void* ys, long sy, const int* pos, const int* idx, const float* wts, const void* h, long sh,
                           const void* shared, long ssh, int E, int top, int W, void* out, int dt, int T,
                           hipStream_t st) {
   if (T <= 0) return 0;
-  MX_DISPATCH(dt, TT, moe_combine_kernel<TT><<<T, 256, 0, st>>>((const TT*)ys, pos, idx, wts, (const TT*)h, sh,
-                                                                (const TT*)shared, ssh, E, top, W, (TT*)out));
+  const int V = dt == 1 ? 4 : 8;                       // elements per 16 bytes
+  const bool vec = W % V == 0 && sy % V == 0 && sh % V == 0 && ssh % V == 0 &&
+                   ((size_t)ys | (size_t)h | (size_t)shared | (size_t)out) % 16 == 0;
+  const int cols = vec ? W / V : W, nt = cols >= 256 ? 256 : (cols + 63) / 64 * 64;
+#define COMBINE(TT, VV)                                                                                               \
+  moe_combine_kernel<TT, VV><<<T, nt, 0, st>>>((const TT*)ys, sy, pos, idx, wts, (const TT*)h, sh, (const TT*)shared, \
+                                               ssh, E, top, W, (TT*)out)
+  if (vec && dt == 1) COMBINE(float, 4);
+  else if (vec) COMBINE(bf16, 8);
+  else if (dt == 1) COMBINE(float, 1);
+  else COMBINE(bf16, 1);
+#undef COMBINE
   MX_RETURN_LAUNCH();
 }

@@ -57,8 +57,8 @@ projection's rank).
 
 Every block declares the rows it needs from a fused in-projection (``in_weight``): a layer stacks
 its mixer's and its feed-forward's rows into ONE GEMM over ``h`` and hands each block its column
-slice.  GEMMs are vendor matrix products (``F.linear`` / ``bmm``) on bf16 or f32 weights; everything
-else runs on the kernels behind :mod:`..ops.mixers`.
+slice.  Plain GEMMs are vendor matrix products (``F.linear`` / ``bmm``) on bf16 or f32 weights; the routed experts and
+everything else run on the kernels behind :mod:`..ops.mixers`.
 """
 from __future__ import annotations
 
@@ -67,25 +67,72 @@ from typing import Callable, Dict, Optional
 import torch
 import torch.nn.functional as F
 
-from ..ops import mixers as mx
+from ..ops import _native as N, mixers as mx
 from .common import AttentionMetadata
 
 Getter = Callable[[str], torch.Tensor]
 
-# steps with at most this many (token, expert) pairs run every expert over every row (no host sync:
-# hipGraph-capturable, and a decode step streams all expert weights anyway); larger steps bucket
-# the rows by expert and read the bucket sizes on the host once per layer
+# on the CPU: steps with at most this many (token, expert) pairs run every expert over every row, larger ones bucket
+# the rows by expert
 DENSE_MAX_PAIRS = 512
 
 
-def _capturing(t: torch.Tensor) -> bool:
-    return t.is_cuda and torch.cuda.is_current_stream_capturing()
+class _ExpertBank:
+    """The expert matrices of a routed feed-forward.  ``first`` / ``second``: per expert W1 [out, in] (or the pair
+    (gate, up)) and W2.  On the GPU they are stored as the grouped kernels read them (:func:`..ops.mixers.experts`),
+    on the CPU as batched right operands [E, in, out]."""
 
+    def __init__(self, first, second, dtype):
+        self.E = len(second)
+        self.native = N.use_native(second[0])
+        if self.native:
+            self.w1, self.w2 = mx.pack_experts(first, dtype), mx.pack_experts(second, dtype)
+        else:
+            cat = [torch.cat(m, 0) if isinstance(m, tuple) else m for m in first]
+            self.w1, self.w2 = (torch.stack([w.t() for w in ws]).to(dtype).contiguous() for ws in (cat, second))
 
-def _expert_stack(ws, dtype) -> torch.Tensor:
-    """Expert matrices [out, in] as one batched right operand [E, in, out], contiguous: batched bf16 products take
-    no transposed view."""
-    return torch.stack([w.t() for w in ws]).to(dtype).contiguous()
+    def num_bytes(self) -> int:
+        return sum(t.numel() * t.element_size() for t in ((self.w1.data, self.w2.data) if self.native else (self.w1, self.w2)))
+
+    def run(self, h: torch.Tensor, idx: torch.Tensor, unit: str, limit: float = 0.0, alpha: float = 0.0,
+            scale: Optional[torch.Tensor] = None):
+        """(ys, pos): row pos[t, k] of ys is expert idx[t, k]'s output for token t (its input times scale[t, k])."""
+        if self.native:
+            return mx.experts(h, idx, self.w1, self.w2, unit, limit, alpha, scale)
+        T, W = h.shape
+        E, top, Fe = self.E, idx.shape[1], self.w2.shape[1]
+
+        def act(x, s):
+            if unit == "relu2":
+                return mx.relu2(x)
+            if unit == "clamped":
+                return mx.glu_clamp(x[:, :Fe], x[:, Fe:], limit, alpha)
+            return mx.glu_act(x[:, :Fe], x[:, Fe:], unit, s)
+
+        if T * top <= DENSE_MAX_PAIRS:
+            # rows an expert was not chosen for get scale 0 and are not read
+            pos = idx.clamp(max=E - 1).long() * T + torch.arange(T, device=h.device)[:, None]
+            s = None
+            if scale is not None:
+                s = torch.zeros(E * T, dtype=torch.float32, device=h.device).scatter_(0, pos.reshape(-1), scale.reshape(-1))
+            x = torch.bmm(h.unsqueeze(0).expand(E, T, W), self.w1).view(E * T, -1)
+            return torch.bmm(act(x, s).view(E, T, Fe), self.w2).view(E * T, W), pos.to(torch.int32)
+        flat = idx.reshape(-1).long()
+        order = torch.argsort(flat, stable=True)
+        offs = [0] + torch.bincount(flat, minlength=E).cumsum(0).tolist()
+        n = offs[E]                                          # rows of real experts (identity experts sort behind them)
+        xs = h.index_select(0, order[:n] // top)
+        live = [(e, offs[e], offs[e + 1]) for e in range(E) if offs[e + 1] > offs[e]]
+        x = torch.empty((n, self.w1.shape[2]), dtype=h.dtype, device=h.device)
+        for e, a, b in live:
+            torch.mm(xs[a:b], self.w1[e], out=x[a:b])
+        y = act(x, scale.reshape(-1)[order[:n]].contiguous() if scale is not None else None)
+        ys = torch.empty((max(n, 1), W), dtype=h.dtype, device=h.device)
+        for e, a, b in live:
+            torch.mm(y[a:b], self.w2[e], out=ys[a:b])
+        pos = torch.empty_like(order)
+        pos[order] = torch.arange(order.numel(), device=order.device)
+        return ys, pos.view(T, top).to(torch.int32)
 
 
 class Mamba2Mixer:
@@ -296,20 +343,19 @@ class RoutedFF:
     def load(self, get: Getter, dtype) -> Optional[torch.Tensor]:
         self.router = get("router").float().contiguous()
         self.correction = get(self.bias_name).float().contiguous()
-        self.w13 = _expert_stack([torch.cat([get(f"e{e}.gate"), get(f"e{e}.up")], 0) for e in range(self.E)], dtype)
-        self.w2 = _expert_stack([get(f"e{e}.down") for e in range(self.E)], dtype)
+        self.bank = _ExpertBank([(get(f"e{e}.gate"), get(f"e{e}.up")) for e in range(self.E)],
+                                [get(f"e{e}.down") for e in range(self.E)], dtype)
         if not self.Fs:
             return None
         self.down_s = get("shared.down").to(dtype).contiguous()
         return torch.cat([get("shared.gate"), get("shared.up")], 0).to(dtype)
 
     def num_bytes(self) -> int:
-        ts = [self.router, self.w13, self.w2] + ([self.down_s] if self.Fs else [])
-        return sum(t.numel() * t.element_size() for t in ts)
+        ts = [self.router] + ([self.down_s] if self.Fs else [])
+        return self.bank.num_bytes() + sum(t.numel() * t.element_size() for t in ts)
 
     def forward(self, h: torch.Tensor, proj: Optional[torch.Tensor]) -> torch.Tensor:
-        T, W = h.shape
-        E, top, Fe = self.E, self.top, self.F
+        top = self.top
         shared = None
         if self.Fs:
             shared = F.linear(mx.glu_clamp(proj[:, :self.Fs], proj[:, self.Fs:2 * self.Fs], self.limit_s, self.alpha),
@@ -319,29 +365,8 @@ class RoutedFF:
         else:
             wts, idx = mx.route_biased(F.linear(h.float(), self.router), self.correction, top, self.score, self.renorm,
                                        self.w_scale)
-        if T * top <= DENSE_MAX_PAIRS or _capturing(h):
-            gu = torch.bmm(h.unsqueeze(0).expand(E, T, W), self.w13).view(E * T, 2 * Fe)
-            act = mx.glu_clamp(gu[:, :Fe], gu[:, Fe:], self.limit, self.alpha)
-            ys = torch.bmm(act.view(E, T, Fe), self.w2).view(E * T, W)
-            rows = torch.arange(T, dtype=torch.int32, device=h.device)[:, None]
-            pos = (idx.clamp(max=E - 1) * T + rows).to(torch.int32)
-            return mx.moe_combine(ys, pos, idx, wts, h, shared, E)
-        flat = idx.reshape(-1).long()
-        order = torch.argsort(flat, stable=True)
-        offs = [0] + torch.bincount(flat, minlength=E + self.I).cumsum(0).tolist()     # host read of the buckets
-        n = offs[E]                                          # rows of real experts (identity experts sort behind them)
-        xs = h.index_select(0, order[:n] // top)
-        live = [(e, offs[e], offs[e + 1]) for e in range(E) if offs[e + 1] > offs[e]]
-        gu = torch.empty((n, 2 * Fe), dtype=h.dtype, device=h.device)
-        for e, a, b in live:
-            torch.mm(xs[a:b], self.w13[e], out=gu[a:b])
-        act = mx.glu_clamp(gu[:, :Fe], gu[:, Fe:], self.limit, self.alpha)             # one launch over all buckets
-        ys = torch.empty((max(n, 1), W), dtype=h.dtype, device=h.device)
-        for e, a, b in live:
-            torch.mm(act[a:b], self.w2[e], out=ys[a:b])
-        pos = torch.empty_like(order)
-        pos[order] = torch.arange(order.numel(), device=order.device)
-        return mx.moe_combine(ys, pos.view(T, top).to(torch.int32), idx, wts, h, shared, E)
+        ys, pos = self.bank.run(h, idx, "clamped", self.limit, self.alpha)
+        return mx.moe_combine(ys, pos, idx, wts, h, shared, self.E)
 
 
 class InputScaledRoutedFF:
@@ -371,46 +396,19 @@ class InputScaledRoutedFF:
 
     def load(self, get: Getter, dtype) -> Optional[torch.Tensor]:
         self.router = get("router").float().contiguous()
-        self.w13 = _expert_stack([torch.cat([get(f"e{e}.gate"), get(f"e{e}.up")], 0) for e in range(self.E)], dtype)
-        self.w2 = _expert_stack([get(f"e{e}.down") for e in range(self.E)], dtype)
+        self.bank = _ExpertBank([(get(f"e{e}.gate"), get(f"e{e}.up")) for e in range(self.E)],
+                                [get(f"e{e}.down") for e in range(self.E)], dtype)
         return None
 
     def num_bytes(self) -> int:
-        return sum(t.numel() * t.element_size() for t in (self.router, self.w13, self.w2))
+        return self.bank.num_bytes() + self.router.numel() * self.router.element_size()
 
     def forward(self, h: torch.Tensor, proj: Optional[torch.Tensor] = None, x32: Optional[torch.Tensor] = None) -> torch.Tensor:
         """``x32``: the f32 input ``h`` was rounded from, when the caller has it: the router then reads the
         unrounded values (fewer swapped near-ties against an exact evaluation)."""
-        T, W = h.shape
-        E, top, Fe = self.E, self.top, self.F
-        wts, idx = mx.route_scores(F.linear(x32 if x32 is not None else h.float(), self.router), top, self.score)
-        ones = torch.ones_like(wts)
-        if T * top <= DENSE_MAX_PAIRS or _capturing(h):
-            # every expert over every row; rows an expert was not chosen for get scale 0 and are not read
-            rows = torch.arange(T, device=h.device)[:, None]
-            pos = idx.long() * T + rows
-            scale = torch.zeros(E * T, dtype=torch.float32, device=h.device).scatter_(0, pos.reshape(-1), wts.reshape(-1))
-            gu = torch.bmm(h.unsqueeze(0).expand(E, T, W), self.w13).view(E * T, 2 * Fe)
-            act = mx.glu_act(gu[:, :Fe], gu[:, Fe:], self.act, scale)
-            ys = torch.bmm(act.view(E, T, Fe), self.w2).view(E * T, W)
-            return mx.moe_combine(ys, pos.to(torch.int32), idx, ones, h, None, E)
-        flat = idx.reshape(-1).long()
-        order = torch.argsort(flat, stable=True)
-        offs = [0] + torch.bincount(flat, minlength=E).cumsum(0).tolist()              # host read of the buckets
-        xs = h.index_select(0, order // top)
-        sc = wts.reshape(-1)[order].contiguous()
-        # one GEMM pair per expert with rows; the activation runs once over all buckets
-        gu = torch.empty((T * top, 2 * Fe), dtype=h.dtype, device=h.device)
-        live = [(e, offs[e], offs[e + 1]) for e in range(E) if offs[e + 1] > offs[e]]
-        for e, a, b in live:
-            torch.mm(xs[a:b], self.w13[e], out=gu[a:b])
-        act = mx.glu_act(gu[:, :Fe], gu[:, Fe:], self.act, sc)
-        ys = torch.empty((T * top, W), dtype=h.dtype, device=h.device)
-        for e, a, b in live:
-            torch.mm(act[a:b], self.w2[e], out=ys[a:b])
-        pos = torch.empty_like(order)
-        pos[order] = torch.arange(order.numel(), device=order.device)
-        return mx.moe_combine(ys, pos.view(T, top).to(torch.int32), idx, ones, h, None, E)
+        wts, idx = mx.route_scores(F.linear(x32 if x32 is not None else h.float(), self.router), self.top, self.score)
+        ys, pos = self.bank.run(h, idx, self.act, scale=wts)
+        return mx.moe_combine(ys, pos, idx, None, h, None, self.E)
 
 
 class TopSoftmaxRoutedFF:
@@ -440,42 +438,21 @@ class TopSoftmaxRoutedFF:
 
     def load(self, get: Getter, dtype) -> Optional[torch.Tensor]:
         self.router = get("router").float().contiguous()
-        self.w1 = _expert_stack([get(f"e{e}.up") for e in range(self.E)], dtype)              # [E, W, F]
-        self.w2 = _expert_stack([get(f"e{e}.down") for e in range(self.E)], dtype)            # [E, F, W]
+        self.bank = _ExpertBank([get(f"e{e}.up") for e in range(self.E)], [get(f"e{e}.down") for e in range(self.E)], dtype)
         if not self.Fs:
             return None
         self.down_s = get("shared.down").to(dtype).contiguous()
         return get("shared.up").to(dtype)
 
     def num_bytes(self) -> int:
-        ts = [self.router, self.w1, self.w2] + ([self.down_s] if self.Fs else [])
-        return sum(t.numel() * t.element_size() for t in ts)
+        ts = [self.router] + ([self.down_s] if self.Fs else [])
+        return self.bank.num_bytes() + sum(t.numel() * t.element_size() for t in ts)
 
     def forward(self, h: torch.Tensor, proj: Optional[torch.Tensor] = None, x32: Optional[torch.Tensor] = None) -> torch.Tensor:
-        T, W = h.shape
-        E, top, Fe = self.E, self.top, self.F
         shared = F.linear(mx.relu2(proj[:, :self.Fs]), self.down_s) if self.Fs else None
-        wts, idx = mx.route_scores(F.linear(x32 if x32 is not None else h.float(), self.router), top, "softmax_top")
-        if T * top <= DENSE_MAX_PAIRS or _capturing(h):
-            up = torch.bmm(h.unsqueeze(0).expand(E, T, W), self.w1).view(E * T, Fe)
-            ys = torch.bmm(mx.relu2(up).view(E, T, Fe), self.w2).view(E * T, W)
-            rows = torch.arange(T, dtype=torch.int32, device=h.device)[:, None]
-            return mx.moe_combine(ys, (idx * T + rows).to(torch.int32), idx, wts, h, shared, E)
-        flat = idx.reshape(-1).long()
-        order = torch.argsort(flat, stable=True)
-        offs = [0] + torch.bincount(flat, minlength=E).cumsum(0).tolist()              # host read of the buckets
-        xs = h.index_select(0, order // top)
-        up = torch.empty((T * top, Fe), dtype=h.dtype, device=h.device)
-        live = [(e, offs[e], offs[e + 1]) for e in range(E) if offs[e + 1] > offs[e]]
-        for e, a, b in live:
-            torch.mm(xs[a:b], self.w1[e], out=up[a:b])
-        act = mx.relu2(up)                                   # one activation launch over all buckets
-        ys = torch.empty((T * top, W), dtype=h.dtype, device=h.device)
-        for e, a, b in live:
-            torch.mm(act[a:b], self.w2[e], out=ys[a:b])
-        pos = torch.empty_like(order)
-        pos[order] = torch.arange(order.numel(), device=order.device)
-        return mx.moe_combine(ys, pos.view(T, top).to(torch.int32), idx, wts, h, shared, E)
+        wts, idx = mx.route_scores(F.linear(x32 if x32 is not None else h.float(), self.router), self.top, "softmax_top")
+        ys, pos = self.bank.run(h, idx, "relu2")
+        return mx.moe_combine(ys, pos, idx, wts, h, shared, self.E)
 
 
 def _f32(get: Getter, name: str) -> torch.Tensor:

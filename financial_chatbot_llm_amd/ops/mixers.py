@@ -265,15 +265,70 @@ def route_biased(z: torch.Tensor, bias: Optional[torch.Tensor], top: int, score:
     return w * scale, idx.to(torch.int32)
 
 
-def moe_combine(ys: Optional[torch.Tensor], pos: torch.Tensor, idx: torch.Tensor, wts: torch.Tensor, h: torch.Tensor,
+class ExpertRows(NamedTuple):
+    """The matrices of all experts as :func:`experts` reads them (see :func:`pack_experts`)."""
+    data: torch.Tensor      # [experts, row groups, K steps of 64 bytes, 4, 16, elements per 16 bytes]
+    rows: int               # rows of one matrix
+    parts: int              # 2: gate and up in turns of 16 rows
+
+
+def pack_experts(mats, dtype: torch.dtype) -> ExpertRows:
+    """``mats``: per expert one matrix [out, in], or the pair (gate, up).  Rows in groups of 16 (a pair's groups take
+    turns) and K in pieces of 64 bytes, each piece stored as the matrix instruction's lanes read it; rows and K are
+    padded with zeros to whole groups and 128 bytes."""
+    pairs = [m if isinstance(m, (tuple, list)) else (m,) for m in mats]
+    E, parts, (n, k) = len(pairs), len(pairs[0]), pairs[0][0].shape
+    el = 16 // torch.empty((), dtype=dtype).element_size()
+    groups, kp = -(-n // 16), -(-k // (8 * el)) * 8 * el
+    full = torch.stack([m.to(dtype) for ms in pairs for m in ms])
+    if (groups * 16, kp) != (n, k):
+        full = F.pad(full, (0, kp - k, 0, groups * 16 - n))
+    data = full.view(E, parts, groups, 16, kp // (4 * el), 4, el).permute(0, 2, 1, 4, 5, 3, 6).contiguous()
+    return ExpertRows(data.view(E, groups * parts, kp // (4 * el), 4, 16, el), n, parts)
+
+
+EXPERT_UNITS = {"clamped": 1, "silu": 2, "gelu_tanh": 3, "relu2": 4}
+
+
+def experts(h: torch.Tensor, idx: torch.Tensor, w1: ExpertRows, w2: ExpertRows, unit: str, limit: float = 0.0, alpha: float = 0.0,
+            scale: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Every token's chosen experts (GPU only): rows ys[pos[t, k]] = W2_e unit(W1_e h[t]) for e = idx[t, k] < experts
+    (identity experts have no row).  ``unit``: "clamped" (g, u of :func:`glu_clamp` with ``limit`` and ``alpha``),
+    "silu" / "gelu_tanh" (act(s g) * (s u), s the pair's entry of ``scale`` f32 [T, top] or 1) or "relu2" (one
+    matrix).  No host read: the rows are sorted by expert on the device.  Returns (ys, pos int32 [T, top])."""
+    T, W = h.shape
+    top, E = idx.shape[1], w1.data.shape[0]
+    el = w1.data.shape[-1]
+    assert h.dtype == w1.data.dtype == w2.data.dtype and idx.dtype == torch.int32 and idx.is_contiguous()
+    assert scale is None or (scale.dtype == torch.float32 and scale.is_contiguous() and scale.shape == idx.shape)
+    wp = -(-W // el) * el
+    if wp != W:                                   # rows in whole 16-byte units
+        h = F.pad(h, (0, wp - W))
+    elif h.stride(1) != 1 or h.stride(0) % el or h.data_ptr() % 16:
+        h = h.contiguous()
+    P = T * top
+    lda = -(-w1.rows // el) * el
+    act = torch.empty((P, lda), dtype=h.dtype, device=h.device)
+    ys = torch.empty((P, wp), dtype=h.dtype, device=h.device)
+    # pos | sorted row -> pair | row tiles of (expert, first row, rows, -), at most P / 16 + experts of them
+    ws = torch.empty(2 * (-(-P // 4) * 4) + 4 * (P // 16 + min(P, E) + 1), dtype=torch.int32, device=h.device)
+    N.mcall("mx_experts", N.ptr(h), h.stride(0), N.ptr(idx), T, top, E, wp, w1.rows, N.ptr(w1.data), w1.data.shape[2],
+            w1.data.shape[1], N.ptr(w2.data), w2.data.shape[2], w2.data.shape[1], EXPERT_UNITS[unit], float(limit),
+            float(alpha), N.ptr(scale), N.ptr(act), lda, N.ptr(ys), N.ptr(ws), _dt(h), N.stream())
+    return ys[:, :W], ws[:P].view(T, top)
+
+
+def moe_combine(ys: Optional[torch.Tensor], pos: torch.Tensor, idx: torch.Tensor, wts: Optional[torch.Tensor], h: torch.Tensor,
                 shared: Optional[torch.Tensor], num_experts: int) -> torch.Tensor:
     """out[t] = sum_k wts[t, k] * src(t, k) (+ shared[t]): src is the token's own input ``h[t]`` for an
-    identity expert (idx >= num_experts), else row ``pos[t, k]`` of the expert outputs ``ys``."""
+    identity expert (idx >= num_experts), else row ``pos[t, k]`` of the expert outputs ``ys``; ``wts`` None: ones."""
     T, W = h.shape
     top = idx.shape[1]
     if N.use_native(h):
         out = torch.empty((T, W), dtype=h.dtype, device=h.device)
-        N.mcall("mx_moe_combine", N.ptr(ys), N.ptr(pos.contiguous()), N.ptr(idx.contiguous()), N.ptr(wts.contiguous()),
+        pos, idx, wts = pos.contiguous(), idx.contiguous(), wts.contiguous() if wts is not None else None
+        N.mcall("mx_moe_combine", N.ptr(_rows(ys)) if ys is not None else None, ys.stride(0) if ys is not None else 0,
+                N.ptr(pos), N.ptr(idx), N.ptr(wts),
                 N.ptr(_rows(h)), h.stride(0), N.ptr(_rows(shared)) if shared is not None else None,
                 shared.stride(0) if shared is not None else 0, num_experts, top, W, N.ptr(out), _dt(h), T, N.stream())
         return out
@@ -285,7 +340,7 @@ def moe_combine(ys: Optional[torch.Tensor], pos: torch.Tensor, idx: torch.Tensor
         if ys is not None and (~ident).any():
             rows = pos[:, k].long().clamp(0, ys.shape[0] - 1)
             src = torch.where(ident[:, None], src, ys.float()[rows])
-        acc += wts[:, k:k + 1] * src
+        acc += (wts[:, k:k + 1] if wts is not None else 1.0) * src
     return acc.to(h.dtype)
 
 
