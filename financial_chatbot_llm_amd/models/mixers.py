@@ -176,7 +176,7 @@ class Mamba2Mixer:
         u = mx.conv_silu(xbc, self.conv_w, self.conv_b, conv_state, meta.seg_cu, meta.seg_state, positions,
                          meta.seg_max_len)
         y = mx.ssm_scan(u, dt, self.dt_bias, self.A_log, self.D, ssm_state, meta.seg_cu, meta.seg_state, positions,
-                        self.H, self.P, self.N, self.G)
+                        self.H, self.P, self.N, self.G, meta.seg_max_len)
         # the gate comes before the norm: rms over silu(z) * y, in norm_groups equal parts
         yn = mx.group_norm(y, self.norm_w, self.eps, self.norm_groups, gate=z, out_dtype=proj.dtype)
         return F.linear(yn, self.o)

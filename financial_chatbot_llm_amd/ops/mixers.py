@@ -382,8 +382,8 @@ def conv_silu(inp: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], 
 
 def ssm_scan(u: torch.Tensor, dt_raw: torch.Tensor, dt_bias: torch.Tensor, A_log: torch.Tensor, D: torch.Tensor,
              state: torch.Tensor, cu: torch.Tensor, slot: torch.Tensor, pos: torch.Tensor, heads: int, vdim: int,
-             nstate: int, groups: int) -> torch.Tensor:
-    """Mamba-2 recurrence, token by token, f32.  ``u`` f32 [T, H*P + 2*G*N] = [x | B | C] (after the
+             nstate: int, groups: int, max_len: int = 0) -> torch.Tensor:
+    """Mamba-2 recurrence in f32 (``max_len``: the longest segment when known; the kernels take long ones in chunks).  ``u`` f32 [T, H*P + 2*G*N] = [x | B | C] (after the
     convolution), ``dt_raw`` [T, H]; per head h of group h // (H / G):
     dt = softplus(dt_raw + dt_bias), S <- exp(-exp(A_log) dt) S + dt x B^T, y = S C + D x.
     ``state`` f32 [slots, H, P, N] is read (unless the segment starts at position 0) and replaced."""
@@ -393,9 +393,11 @@ def ssm_scan(u: torch.Tensor, dt_raw: torch.Tensor, dt_bias: torch.Tensor, A_log
     assert u.dtype == torch.float32 and u.is_contiguous() and C == H * P + 2 * G * Ns
     if N.use_native(u):
         y = torch.empty((T, H * P), dtype=torch.float32, device=u.device)
+        max_len = max_len or T
+        cb = torch.empty((T, G, 64), dtype=torch.float32, device=u.device) if max_len > 1 else None
         N.mcall("mx_ssm_scan", N.ptr(u), C, N.ptr(_rows(dt_raw)), dt_raw.stride(0), _dt(dt_raw), N.ptr(dt_bias),
-                N.ptr(A_log), N.ptr(D), N.ptr(state), N.ptr(cu), N.ptr(slot), N.ptr(pos), N.ptr(y), S, H, P, Ns, G, T,
-                N.stream())
+                N.ptr(A_log), N.ptr(D), N.ptr(state), N.ptr(cu), N.ptr(slot), N.ptr(pos), N.ptr(y), S, int(max_len), H, P, Ns, G,
+                T, N.ptr(cb), N.stream())
         return y
     y = torch.zeros((T, H * P), dtype=torch.float32)
     cul, sll, pl = cu.tolist(), slot.tolist(), pos.tolist()

@@ -1,0 +1,55 @@
+"""The chunked state-space scan against a float64 recurrence and beside the token-by-token kernel: chunk edges, fresh and
+continued segments, padding rows, mixed lengths, slow and very fast decays."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+
+def recurrence(u, dtr, bias, A_log, D, S, H, P, N, G):
+    y = torch.zeros(u.shape[0], H, P, dtype=torch.float64)
+    x, B, C = u[:, :H * P].view(-1, H, P), u[:, H * P:H * P + G * N].view(-1, G, N), u[:, H * P + G * N:].view(-1, G, N)
+    B, C = (t.repeat_interleave(H // G, 1) for t in (B, C))
+    dt = F.softplus(dtr + bias)
+    keep = torch.exp(-torch.exp(A_log) * dt)
+    for t in range(u.shape[0]):
+        S = keep[t, :, None, None] * S + (dt[t, :, None] * x[t])[:, :, None] * B[t][:, None]
+        y[t] = (S * C[t][:, None]).sum(-1) + D[:, None] * x[t]
+    return y.reshape(-1, H * P), S
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,P,N,G,decay", [(2, 64, 128, 2, 1.0), (4, 16, 64, 1, 8.0), (2, 48, 256, 2, 0.1), (4, 32, 128, 2, 60.0)])
+@pytest.mark.parametrize("lens", [[64], [32, 1, 31, 63, 65], [200, 5, 129], [1, 128]])
+def test_chunked_scan(dtype, H, P, N, G, decay, lens):
+    from financial_chatbot_llm_amd.ops import mixers as mx
+    g = torch.Generator().manual_seed(sum(lens) + N)
+    rnd = lambda *s: torch.randn(s, generator=g)  # noqa: E731
+    T, S = sum(lens) + 1, len(lens) + 1           # one padding row at the end
+    cu = torch.tensor([0] + lens + [1]).cumsum(0)
+    slot = torch.tensor([S + 2 - i for i in range(len(lens))] + [-1])
+    starts = [0 if i % 2 == 0 else 70 for i in range(len(lens))] + [0]
+    pos = torch.cat([torch.arange(a, a + n) for a, n in zip(starts, lens + [1])])
+    u, dtr = rnd(T, H * P + 2 * G * N), (rnd(T, H) * 0.5).to(dtype)
+    bias, A_log, D = rnd(H) * 0.5 - 2.0, torch.log(decay * (0.5 + torch.rand(H, generator=g))), rnd(H)
+    state = rnd(S + 3, H, P, N)
+    dev = lambda t: t.cuda() if t.is_floating_point() else t.to("cuda", torch.int32)  # noqa: E731
+    got = {}
+    for name, most in (("chunks", max(lens)), ("tokens", 1)):
+        st = state.cuda()
+        y = mx.ssm_scan(u.cuda(), dtr.cuda(), dev(bias), dev(A_log), dev(D), st, dev(cu), dev(slot), dev(pos), H, P, N, G, most)
+        got[name] = (y.double().cpu(), st.double().cpu())
+    off = {"chunks": 0.0, "tokens": 0.0}
+    for i, n in enumerate(lens):
+        a = int(cu[i])
+        s0 = torch.zeros(H, P, N, dtype=torch.float64) if starts[i] == 0 else state[slot[i]].double()
+        y, s1 = recurrence(u[a:a + n].double(), dtr[a:a + n].double(), bias.double(), A_log.double(), D.double(), s0, H, P, N, G)
+        for name, (gy, gs) in got.items():
+            off[name] = max(off[name], float((gy[a:a + n] - y).norm() / y.norm()), float((gs[slot[i]] - s1).norm() / s1.norm()))
+    used = set(slot[:-1].tolist())
+    for _, gs in got.values():                    # no other slot is touched
+        for k in range(S + 3):
+            assert k in used or torch.equal(gs[k], state[k].double())
+    # f32 sums of up to N + 64 products and one exponential per pair of tokens
+    assert off["chunks"] < 2e-6 and off["chunks"] < 2.0 * off["tokens"] + 3e-7, off
