@@ -2,10 +2,8 @@
 
 Post-LN BERT: embeddings (word + position + type) -> LayerNorm -> 12 x [fused QKV GEMM (+bias)
 -> bidirectional attention -> O GEMM -> add+LayerNorm -> GELU MLP -> add+LayerNorm] -> CLS
-pooling -> L2 normalise.  Queries are packed varlen (no padding FLOPs).  Attention reuses the
-decoder's paged-KV machinery: each layer's K/V go through the RoPE-less KV writer into a small
-scratch paged cache (reused by every layer) and the MFMA prefill kernel runs with
-``causal=False`` at head_dim 64.
+pooling -> L2 normalise.  Queries are packed varlen (no padding FLOPs); attention reads the packed QKV
+rows as they are (``csrc/kernels/encoder.hip``).
 """
 from __future__ import annotations
 
@@ -17,7 +15,6 @@ import torch
 import torch.nn.functional as F
 
 from .. import ops
-from ..ops.attention import KV_BS
 from ..ops.gemm import linear_bias
 from .common import random_tensor
 from .configs import ModelConfig
@@ -30,7 +27,6 @@ class BertEncoder:
         self.dtype = dtype
         self.H, self.nh, self.D = cfg.hidden_size, cfg.num_heads, cfg.head_dim
         self.w: Dict[str, torch.Tensor] = {}
-        self._scratch: Optional[torch.Tensor] = None
 
     def shapes(self) -> Dict[str, tuple]:
         c = self.cfg
@@ -62,12 +58,6 @@ class BertEncoder:
             self.w[k] = v.to(self.device, self.dtype).contiguous()
         return self
 
-    def _kv_scratch(self, nblocks: int):
-        if self._scratch is None or self._scratch.shape[1] < nblocks:
-            self._scratch = torch.zeros((2, max(nblocks, 64), self.nh, KV_BS * self.D), dtype=self.dtype,
-                                        device=self.device)
-        return self._scratch[0], self._scratch[1]
-
     @torch.no_grad()
     def forward(self, ids_list: Sequence[Sequence[int]]) -> torch.Tensor:
         """-> final hidden states [T, H] of the packed batch, plus CLS row indices."""
@@ -77,25 +67,14 @@ class BertEncoder:
         T = int(lens.sum())
         cu = np.zeros(len(lens) + 1, np.int64)
         np.cumsum(lens, out=cu[1:])
-        flat = np.fromiter((t for x in ids_list for t in x), np.int32, T)
-        pos = np.arange(T, dtype=np.int64) - np.repeat(cu[:-1], lens)
-        nbs = (lens + KV_BS - 1) // KV_BS
-        starts = np.zeros(len(lens) + 1, np.int64)
-        np.cumsum(nbs, out=starts[1:])
-        W = int(nbs.max())
-        cols = np.arange(W, dtype=np.int64)
-        bt = np.where(cols[None, :] < nbs[:, None], starts[:-1, None] + cols[None, :], 0).astype(np.int32)
-        slots = (np.repeat(starts[:-1], lens) + pos // KV_BS) * KV_BS + pos % KV_BS
-        ids_t = torch.from_numpy(flat).to(dev)
-        pos_t = torch.from_numpy(pos.astype(np.int32)).to(dev)
-        slots_t = torch.from_numpy(slots.astype(np.int32)).to(dev)
-        cu_t = torch.from_numpy(cu.astype(np.int32)).to(dev)
-        lens_t = torch.from_numpy(lens.astype(np.int32)).to(dev)
-        bt = torch.from_numpy(bt).to(dev)
-        starts = starts.tolist()
-        lens = lens.tolist()
+        # token ids | positions | row bounds: one copy to the device
+        meta = np.empty(2 * T + len(cu), np.int32)
+        meta[:T] = np.fromiter((t for x in ids_list for t in x), np.int32, T)
+        meta[T:2 * T] = np.arange(T, dtype=np.int64) - np.repeat(cu[:-1], lens)
+        meta[2 * T:] = cu
+        ids_t, pos_t, cu_t = torch.from_numpy(meta).to(dev).split([T, T, len(cu)])
+        longest = int(lens.max())
         cu = cu.tolist()
-        kc, vc = self._kv_scratch(starts[-1])
         w = self.w
         e_word = ops.embedding(ids_t, w["word_emb"])
         e_pos = ops.embedding(pos_t, w["pos_emb"])
@@ -105,9 +84,8 @@ class BertEncoder:
         for i in range(c.num_layers):
             p = f"layers.{i}."
             qkv = linear_bias(x, w[p + "qkv"], w[p + "qkv_b"])
-            q = ops.rope_kv_write(qkv, pos_t, None, slots_t, kc, vc, self.nh, self.nh, self.D, apply_rope=False)
-            a = ops.prefill(q, cu_t, lens_t, bt, kc, vc, scale, causal=False, max_q_len=max(lens))
-            o = linear_bias(a.view(T, self.H), w[p + "o"], w[p + "o_b"])
+            a = ops.encoder_attention(qkv, cu_t, longest, self.nh, scale)
+            o = linear_bias(a, w[p + "o"], w[p + "o_b"])
             x = ops.layer_norm(o, w[p + "ln1_g"], w[p + "ln1_b"], c.norm_eps, residual=x)
             h = linear_bias(x, w[p + "fc1"], w[p + "fc1_b"], gelu=True)      # bias + GELU fused
             y = linear_bias(h, w[p + "fc2"], w[p + "fc2_b"])

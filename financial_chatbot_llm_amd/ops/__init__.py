@@ -5,7 +5,7 @@ loudly if the library is missing), CPU tensors run an fp32 PyTorch reference tha
 oracle in the numerics tests.
 """
 from .activation import gelu_, silu_mul
-from .attention import (KV_BS, DecodeWorkspace, decode, default_scale, prefill, rope_cos_sin, rope_kv_write,
+from .attention import (KV_BS, DecodeWorkspace, decode, default_scale, encoder_attention, prefill, rope_cos_sin, rope_kv_write,
                         write_kv_ref)
 from .embedding import embedding
 from .mixers import (DynTanh, conv_act, conv_heads, conv_silu, decay_scan, dyn_tanh_embed, dyn_tanh_residual, distance_buckets, embed_f32,
@@ -18,7 +18,7 @@ from .sampling import (apply_top_k_top_p, fused_lm_head_ok, lm_head_sample, lm_h
                        pick_pairs, sample,
                        sample_shard)
 
-__all__ = ["gelu_", "silu_mul", "KV_BS", "DecodeWorkspace", "decode", "default_scale", "prefill", "rope_cos_sin",
+__all__ = ["gelu_", "silu_mul", "KV_BS", "DecodeWorkspace", "decode", "default_scale", "encoder_attention", "prefill", "rope_cos_sin",
            "rope_kv_write", "write_kv_ref", "embedding", "layer_norm", "rms_norm", "filtered_topk",
            "apply_top_k_top_p", "sample", "conv_silu", "embed_f32", "glu_clamp", "group_norm", "latent_attend",
            "latent_prep", "moe_combine", "relu2", "residual_norm", "route_biased", "ssm_scan", "conv_act", "embed_pairs",

@@ -398,6 +398,25 @@ def prefill(q: torch.Tensor, cu_q: torch.Tensor, ctx_lens: torch.Tensor, block_t
     return out
 
 
+def encoder_attention(qkv: torch.Tensor, cu: torch.Tensor, max_len: int, heads: int, scale: float) -> torch.Tensor:
+    """Bidirectional attention of packed texts: ``qkv`` [T, 3 * heads * D] holds q | k | v, text i owns rows
+    cu[i] : cu[i + 1] and attends within itself; ``max_len``: the longest text.  Returns [T, heads * D]."""
+    T, D = qkv.shape[0], qkv.shape[1] // (3 * heads)
+    if N.use_native(qkv):
+        out = torch.empty((T, heads * D), dtype=qkv.dtype, device=qkv.device)
+        for a in range(0, cu.numel() - 1, 65535):      # texts per launch
+            c = cu[a:a + 65536]
+            N.call("penny_encoder_attention", N.ptr(qkv), qkv.stride(0), N.ptr(c), c.numel() - 1, int(max_len), heads, D,
+                   float(scale), N.ptr(out), N.stream())
+        return out
+    q, k, v = qkv.view(T, 3, heads, D).unbind(1)
+    bounds = cu.tolist()
+    out = torch.empty((T, heads, D), dtype=qkv.dtype)
+    for a, b in zip(bounds, bounds[1:]):
+        out[a:b] = _attend_ref(q[a:b], k[a:b], v[a:b], scale, None)
+    return out.view(T, heads * D)
+
+
 def _lse_ref(q: torch.Tensor, k: torch.Tensor, scale: float, q_offset: Optional[int]) -> torch.Tensor:
     """[Tq, Hq] natural-log sum-exp of the scaled (masked) scores, fp32."""
     G = q.shape[1] // k.shape[1]

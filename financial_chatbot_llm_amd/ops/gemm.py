@@ -750,22 +750,35 @@ def tail_workspace(dev: torch.device) -> Tuple:
     return (N.ptr(part), part.numel(), N.ptr(cnt), cnt.numel(), cus)
 
 
-# bge query batches up to this many tokens run every projection on the tile kernel: the encoder is
-# launch-bound there (~2 ms for 12 layers) and the fused bias / bias+GELU epilogues save launches and
-# passes -- 1.72 vs 2.15 ms for 1 query, 2.12 vs 2.24 ms for 24, 2.18 vs 2.26 ms for 64 (1.5k tokens)
-# against hipBLASLt + the GELU pass; at 4k tokens the per-shape policy decides
-# (profiles/r3_bge_query_tile_vs_hipblaslt.jsonl)
+# bge query batches up to this many tokens run every projection on the framework's kernels: the encoder is
+# launch-bound there and the fused bias / bias+GELU epilogues save launches and passes (1.72 vs 2.15 ms for 1 query, 2.18
+# vs 2.26 ms for 64 (1.5k tokens) against hipBLASLt + the GELU pass, profiles/r3_bge_query_tile_vs_hipblaslt.jsonl); at 4k
+# tokens the per-shape policy decides
 BGE_TILE_MAX_M = 2048
+# ... and up to this many the small-batch kernel, whose blocks of 16 - 32 weight rows fill the chip.  bge projections, us
+# (small / tile): 2304 x 768 4.3 / 17 at 18 rows, 11 / 22 at 256, 20 / 22 at 768, 24 / 22 at 1024; 768 x 3072 8 / 32, 19 / 36,
+# 36 / 38, 36 / 38; 3072 x 768 with GELU 4.5 / 26, 12 / 35, 26 / 36, 30 / 36
+BGE_SMALL_MAX_M = 768
+
+
+def small_bias_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    return (N.use_native(x) and x.dtype == w.dtype == torch.bfloat16 and w.shape[0] % 16 == 0 and w.shape[1] % 32 == 0
+            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.is_contiguous())
 
 
 def linear_bias(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, gelu: bool = False) -> torch.Tensor:
-    """Encoder projection bf16(x @ w.T + b) [-> exact GELU] on the tile kernel with the bias (+GELU)
-    epilogue: always for query-size batches (<= BGE_TILE_MAX_M tokens), by the measured per-shape
+    """Encoder projection bf16(x @ w.T + b) [-> exact GELU]: the small-batch kernel up to BGE_SMALL_MAX_M tokens, the
+    tile kernel with the bias (+GELU) epilogue always up to BGE_TILE_MAX_M tokens and by the measured per-shape
     policy for bulk ingest; hipBLASLt's bias GEMM + the HIP GELU pass otherwise
     (``PENNY_PREFILL_GEMM=0``: always the library)."""
     M, K = x.shape
     N_ = w.shape[0]
     mode = os.environ.get("PENNY_PREFILL_GEMM", "1")
+    if mode == "1" and M <= BGE_SMALL_MAX_M and small_bias_ok(x, w):
+        y = torch.empty((M, N_), dtype=x.dtype, device=x.device)
+        N.call("penny_gemm_bias_small", N.ptr(x), x.stride(0), N.ptr(w), K, N.ptr(y), N_, N.ptr(b), M, N_, int(gelu),
+               N.stream())
+        return y
     if mode != "0" and prefill_ok(x, w) and (M <= BGE_TILE_MAX_M or mode == "force" or
                                             prefill_choice(M, N_, K, "bias_gelu" if gelu else "bias") == "hip"):
         return prefill_gemm(x, w, "bias_gelu" if gelu else "bias", bias=b)

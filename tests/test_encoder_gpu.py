@@ -1,0 +1,50 @@
+"""The encoder's own kernels against plain float32: attention over packed rows (tile edges, one-token texts, both head
+sizes, rows wider than q | k | v) and the biased projections of small batches (edges of the token and row tiles)."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D,H", [(64, 12), (64, 3), (128, 2)])
+@pytest.mark.parametrize("lens", [[1], [18], [64, 63, 65, 1, 16], [130, 7, 200], [300]])
+@pytest.mark.parametrize("pad", [0, 8])
+def test_encoder_attention(D, H, lens, pad):
+    from financial_chatbot_llm_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(D + sum(lens))
+    T = sum(lens)
+    x = torch.randn(T, 3 * H * D + pad, generator=g, device="cuda").to(torch.bfloat16)
+    qkv = x[:, :3 * H * D]
+    cu = torch.tensor([0] + lens).cumsum(0).to("cuda", torch.int32)
+    scale = 1.7 * D ** -0.5
+    if pad:                          # the op's row stride comes from the tensor, the head size from its width
+        assert qkv.stride(0) == 3 * H * D + pad
+    got = ops.encoder_attention(qkv, cu, max(lens), H, scale).float()
+    a = 0
+    for n in lens:
+        q, k, v = qkv[a:a + n].float().reshape(n, 3, H, D).permute(1, 2, 0, 3).contiguous()
+        p = torch.softmax(torch.matmul(q, k.transpose(1, 2).contiguous()) * scale, -1)
+        want = torch.matmul(p, v).permute(1, 0, 2).reshape(n, H * D)
+        # weights and output are rounded to bf16 once each
+        assert float((got[a:a + n] - want).norm() / want.norm()) < 6e-3
+        assert float((got[a:a + n] - want).abs().max()) < 0.03 * float(want.abs().max())
+        a += n
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64, 65, 128, 129, 768])
+@pytest.mark.parametrize("N,K", [(768, 768), (48, 96), (3072, 768), (768, 3072), (16, 32)])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_small_batch_projection(M, N, K, gelu):
+    from financial_chatbot_llm_amd.ops import gemm
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K + 8, generator=g, device="cuda").to(torch.bfloat16)[:, :K]
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    b = torch.randn(N, generator=g, device="cuda").to(torch.bfloat16)
+    assert gemm.small_bias_ok(x, w) and M <= gemm.BGE_SMALL_MAX_M
+    got = gemm.linear_bias(x, w, b, gelu).float()
+    want = x.float() @ w.float().T + b.float()
+    if gelu:
+        want = F.gelu(want)
+    # f32 sums; the result (with gelu also its argument) is rounded to bf16 once
+    assert float((got - want).norm() / want.norm()) < 4e-3
