@@ -458,7 +458,8 @@ class DecodeWorkspace:
     def create(cls, max_batch: int, Hq: int, D: int, max_ctx: int, device, pb: int = 8) -> "DecodeWorkspace":
         nblk = (max_ctx + KV_BS - 1) // KV_BS
         nparts = max(2, (nblk + pb - 1) // pb)
-        stride = max(nparts, 2)
+        # slots per (row, head): the lean kernel may cut a row of a small batch into 16 parts (decode)
+        stride = max(nparts, min(nblk + 1, 17))
         f = dict(dtype=torch.float32, device=device)
         return cls(torch.empty((max_batch, Hq, stride), **f), torch.empty((max_batch, Hq, stride), **f),
                    torch.empty((max_batch, Hq, stride, D), **f), pb, max(nparts, 2), stride,
@@ -473,6 +474,11 @@ _SIDE_STREAMS = {}
 DECODE_LEAN = os.environ.get("PENNY_DECODE_LEAN", "1") != "0"
 LEAN_MIN_B = int(os.environ.get("PENNY_DECODE_LEAN_MIN_B", "1"))
 LEAN_WG_PER_CU = 2          # 242 VGPRs per wave -> 2 waves per SIMD = 2 workgroups per CU
+# blocks a wave takes at least, and how many parts a row may have.  A small batch wants many parts (us, 3 / 5 / 9 / 17 slots
+# per row): 1 row behind 900 tokens 13.7 / 11.9 / 10.6 / 10.0, behind 4000 42 / 28 / 19 / 16, 4 rows behind 4000 66 / 40 / 29 /
+# 24, 32 rows behind 1200 50 / 33 / 38 / 33; 8 and 16 rows rather parts of 4 blocks than of 2 (16 behind 1200: 23.5 and 26.5).
+# From 48 rows on the rows themselves fill the chip and parts only cost the merge (48 behind 1200: 43 us with 4 slots or
+# 17, the merge 4.9 and 7.0).
 LEAN_MIN_PER_WAVE = 2
 # lean kernel flags (attention.hip penny_attention_decode lean_flags): bit 0 = non-temporal K/V loads
 # for the blocks only one row of the step reads (the host marks the shared ones: mark_shared_blocks);
@@ -580,10 +586,13 @@ def decode(q: torch.Tensor, ctx_lens: torch.Tensor, block_tables: torch.Tensor, 
         lean = (DECODE_LEAN and B >= LEAN_MIN_B and ws.lean_meta is not None
                 and ws.lean_meta.numel() >= LEAN_META0 + B + 2)
         pb, nparts = ws.partitioning(B) if not lean else (ws.pb, ws.nparts)
+        min_per_wave = LEAN_MIN_PER_WAVE
+        if lean and B <= 32:
+            nparts, min_per_wave = ws.part_stride, 4 if 4 < B <= 16 else LEAN_MIN_PER_WAVE
         args = [N.ptr(q), N.ptr(ctx_lens), N.ptr(block_tables), N.ptr(k_cache), N.ptr(v_cache), N.ptr(out),
                 N.ptr(ws.part_m), N.ptr(ws.part_l), N.ptr(ws.part_o), B, Hq, Hkv, D, block_tables.shape[1], pb,
                 nparts, ws.part_stride, float(scale)]
-        lean_args = ((_lean_grid(q.device, Hkv), N.ptr(ws.lean_meta), LEAN_MIN_PER_WAVE,
+        lean_args = ((_lean_grid(q.device, Hkv), N.ptr(ws.lean_meta), min_per_wave,
                       LEAN_FLAGS if B >= LEAN_NT_MIN_B else LEAN_FLAGS & ~1) if lean else (0, None, 1, 0))
         N.call("penny_attention_decode", *args, *lean_args, N.stream() if stream is None else stream)
         return out
