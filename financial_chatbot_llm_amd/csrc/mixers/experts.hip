@@ -23,7 +23,6 @@
 namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 template <int N> struct Steps { static constexpr int value = N; };
 
@@ -31,22 +30,6 @@ enum { UNIT_NONE = 0, UNIT_CLAMP = 1, UNIT_SILU = 2, UNIT_GELU = 3, UNIT_RELU2 =
 
 // 16 zero bytes: what a lane stages for K positions behind a row's end
 __device__ uint4 g_zero16;
-
-template <typename T> __device__ __forceinline__ f32x4 mma16(uint4 a, uint4 b, f32x4 c);
-template <> __device__ __forceinline__ f32x4 mma16<bf16>(uint4 a, uint4 b, f32x4 c) {
-  union { uint4 u; bf16x8 v; } x, y;
-  x.u = a;
-  y.u = b;
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.v, y.v, c, 0, 0, 0);
-}
-template <> __device__ __forceinline__ f32x4 mma16<float>(uint4 a, uint4 b, f32x4 c) {
-  union { uint4 u; f32x4 v; } x, y;
-  x.u = a;
-  y.u = b;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(x.v[j], y.v[j], c, 0, 0, 0);
-  return c;
-}
 
 struct ExpertGemm {
   const void* x;        // rows of ldx elements: token rows (top > 0: sorted row r reads row src[r] / top) or sorted rows

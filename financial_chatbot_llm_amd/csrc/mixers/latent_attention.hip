@@ -16,11 +16,11 @@
 //                     softmax denominator of head h also holds exp(sink[h]) (no key, no value).
 #include <stdlib.h>
 
-#include "mx_common.h"
+#include "rows_attend.h"
 
 namespace {
 
-constexpr int PAGE = 64;            // tokens per cache page
+constexpr int PAGE = PAGE_ROWS;
 
 // one block per token; sine and cosine are evaluated once per pair and shared by the key and all heads' queries
 template <typename T>
@@ -215,9 +215,6 @@ latent_attend_kernel(const T* __restrict__ q_lat, const T* __restrict__ q_rot, c
 //                        one bf16 term, or (SPLIT) as two, hi + lo, so that the f32 softmax weights are
 //                        not cut to 8 bits
 // Feature dimensions are zero-padded to multiples of 32 (keys) / 16 (values) in LDS and registers.
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int MKT = 32;             // keys per tile
 constexpr int MLDV = MKT + 8;       // row stride of the transposed value tile
 
@@ -490,15 +487,36 @@ MX_API int mx_latent_prep(const void* kv, long skv, const float* norm_w, float e
 // q_lat [T, H, R], q_rot [T, H, Dr], out [T, H, R] contiguous; cu [S+1] row bounds of the segments,
 // pos [T] positions, bt [S, btw] page tables; gate [T, >=H] slice (row stride sgate) or null; sink f32 [H] or
 // null.  exact != 0: the softmax weights enter the value product of the matrix-core form as two bf16 terms.
-// nsplit > 1 with a workspace ws (f32 [T, H, nsplit, R + 2]) and single-row segments: the key range of
-// each row is walked by nsplit blocks and merged (bf16 matrix-core form only; ignored otherwise).
+// nsplit > 1 with a workspace ws (f32 [rows, H, nsplit, R + 2]): the keys of each row are walked by nsplit blocks and
+// merged (rows_attend.h; the older matrix-core form does so for single-row segments only, the f32-lane form never).
 MX_API int mx_latent_attend(const void* q_lat, const void* q_rot, const void* cache, const int* cu, const int* pos,
                             const int* bt, int btw, const void* gate, long sgate, const float* sink, int exact,
                             int window, float scale, void* out, int dt, int S, int max_len, int H, int R, int Dr,
-                            int nsplit, float* ws, hipStream_t st) {
+                            int nsplit, float* ws, int rows, hipStream_t st) {
   if (S <= 0 || max_len <= 0) return 0;
   if (R > 64 * ATT_RPL) return (int)hipErrorInvalidValue;
   const int D = R + Dr;
+  // rows_attend.h for the latent of 256 with a rotated part of 32 or none, the sizes of this framework's decoders (32 heads,
+  // window 1024, before -> after: 2048 rows of three segments 217 -> 64 us, 256 rows and 30 single ones 405 -> 75, 64 single
+  // rows 85 -> 24, 4 single rows 32 -> 19)
+  if (dt == 0 && R == 256 && (Dr == 32 || Dr == 0) && mx_use_mfma() &&
+      ((size_t)q_lat | (size_t)q_rot | (size_t)cache | (size_t)out) % 16 == 0 && window <= (1 << 30)) {
+    if (ws == nullptr || nsplit < 1) nsplit = 1;
+    const int HB = H < 64 ? H : 64, QT = max_len == 1 ? 1 : 64 / HB;
+    RowsArgs a{q_lat, q_rot, (long)H * R, cache, D, 0, 0, 0, cu, pos, bt, btw, gate, sgate, 0, window, 0, 0,
+               nullptr, 0.f, sink, scale, out, H, 1, QT, HB, nsplit, ws};
+    const dim3 grid((unsigned)((max_len + QT - 1) / QT * nsplit), (H + HB - 1) / HB, S);
+    if (Dr == 32) {
+      if (exact) rows_attend_kernel<bf16, 256, 32, 256, true, 1, 4, 64, false, true><<<grid, 256, 0, st>>>(a);
+      else rows_attend_kernel<bf16, 256, 32, 256, true, 1, 4, 64, false, false><<<grid, 256, 0, st>>>(a);
+    } else {
+      if (exact) rows_attend_kernel<bf16, 256, 0, 256, true, 1, 4, 64, false, true><<<grid, 256, 0, st>>>(a);
+      else rows_attend_kernel<bf16, 256, 0, 256, true, 1, 4, 64, false, false><<<grid, 256, 0, st>>>(a);
+    }
+    if (nsplit > 1)
+      latent_merge_kernel<<<dim3(rows, H), 128, 0, st>>>(ws, (const bf16*)gate, sgate, sink, (bf16*)out, H, R, nsplit);
+    MX_RETURN_LAUNCH();
+  }
   if (dt == 0 && D <= 320 && R <= 256 && mx_use_mfma()) {
     // matrix-core form: 64 (row, head) pairs per block
     const int HB = H < 64 ? H : 64;

@@ -71,6 +71,28 @@ __device__ __forceinline__ float mx_softmax_scale(float m, float l, const float*
   return f / (l * f + expf(sk - M));
 }
 
+// D += A B of a 16 x 16 tile over 64 bytes of K per row: a 16-byte operand is 8 bf16 (one 16x16x32 product) or 4 f32 (four
+// 16x16x4 products, step j taking K element 4 g + j of both sides)
+typedef float mx_f32x4 __attribute__((ext_vector_type(4)));
+template <typename T> __device__ __forceinline__ mx_f32x4 mma16(uint4 a, uint4 b, mx_f32x4 c);
+template <> __device__ __forceinline__ mx_f32x4 mma16<bf16>(uint4 a, uint4 b, mx_f32x4 c) {
+  typedef __bf16 v8 __attribute__((ext_vector_type(8)));
+  union { uint4 u; v8 v; } x, y;
+  x.u = a;
+  y.u = b;
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.v, y.v, c, 0, 0, 0);
+}
+template <> __device__ __forceinline__ mx_f32x4 mma16<float>(uint4 a, uint4 b, mx_f32x4 c) {
+  union { uint4 u; mx_f32x4 v; } x, y;
+  x.u = a;
+  y.u = b;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(x.v[j], y.v[j], c, 0, 0, 0);
+  return c;
+}
+
+constexpr int PAGE_ROWS = 64;            // tokens per cache page
+
 // tanh with one division and no branch.  |z| < 0.6: the fifth convergent of Lambert's continued fraction
 // z / (1 + z^2 / (3 + z^2 / (5 + ...))), relative error below 1e-8 there; beyond: (1 - e) / (1 + e), e = exp(-2|z|)
 __device__ __forceinline__ float mx_tanh(float z) {

@@ -25,11 +25,11 @@
 //                      decoded tokens alike).
 #include <stdlib.h>
 
-#include "mx_common.h"
+#include "rows_attend.h"
 
 namespace {
 
-constexpr int PAGE = 64;            // tokens per cache page
+constexpr int PAGE = PAGE_ROWS;
 
 // first key the query at position p sees: a sliding window of `window` keys, or the start of p's block
 __device__ __forceinline__ int first_key(int p, int window, int chunked) {
@@ -320,10 +320,7 @@ window_attend_kernel(const T* __restrict__ q, long sq, const T* __restrict__ cac
 // Feature dimensions are zero-padded to multiples of 32 (keys) / 16 (values) in LDS and registers.
 // Single-row segments (decode) may split each row's key range over nsplit blocks; the parts
 // (unnormalised output, running maximum, sum) are combined by window_merge_kernel.
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int MKT = 32;             // keys per tile
 constexpr int MLDV = MKT + 8;       // row stride of the transposed value tile
 
@@ -616,19 +613,20 @@ window_attend_mfma_kernel(const bf16* __restrict__ q, long sq, const bf16* __res
 
 // grid (rows, H): combine the nsplit parts of one (row, head)
 // (sigm: the parts are plain sums of independently weighted values)
-__global__ void window_merge_kernel(const float* __restrict__ ws, const bf16* __restrict__ gate, long sgate,
-                                    int gate_elem, const float* __restrict__ sink, bf16* __restrict__ out, int H, int P,
+template <typename T>
+__global__ void window_merge_kernel(const float* __restrict__ ws, const T* __restrict__ gate, long sgate,
+                                    int gate_elem, const float* __restrict__ sink, T* __restrict__ out, int H, int P,
                                     int nsplit, int sigm) {
   const long row = blockIdx.x;
   const int h = blockIdx.y;
   const float* w = ws + (row * H + h) * nsplit * (long)(P + 2);
-  const bf16* ge = gate_elem ? gate + row * sgate + (long)h * P : nullptr;
+  const T* ge = gate_elem ? gate + row * sgate + (long)h * P : nullptr;
   if (sigm) {
-    const float gs = gate != nullptr && !gate_elem ? mx_sigmoid((float)gate[row * sgate + h]) : 1.0f;
+    const float gs = gate != nullptr && !gate_elem ? mx_sigmoid(ldf(gate + row * sgate + h)) : 1.0f;
     for (int r = threadIdx.x; r < P; r += blockDim.x) {
       float a = 0.f;
       for (int i = 0; i < nsplit; ++i) a += w[i * (P + 2) + r];
-      out[(row * H + h) * P + r] = (bf16)(a * gs * (ge != nullptr ? mx_sigmoid((float)ge[r]) : 1.0f));
+      out[(row * H + h) * P + r] = (T)(a * gs * (ge != nullptr ? mx_sigmoid(ldf(ge + r)) : 1.0f));
     }
     return;
   }
@@ -640,14 +638,14 @@ __global__ void window_merge_kernel(const float* __restrict__ ws, const bf16* __
     if (mi != -INFINITY) L += w[i * (P + 2) + P + 1] * expf(mi - M);
   }
   float gsc = 1.0f / L;
-  if (gate != nullptr && !gate_elem) gsc *= mx_sigmoid((float)gate[row * sgate + h]);
+  if (gate != nullptr && !gate_elem) gsc *= mx_sigmoid(ldf(gate + row * sgate + h));
   for (int r = threadIdx.x; r < P; r += blockDim.x) {
     float a = 0.f;
     for (int i = 0; i < nsplit; ++i) {
       const float mi = w[i * (P + 2) + P];
       if (mi != -INFINITY) a += w[i * (P + 2) + r] * expf(mi - M);
     }
-    out[(row * H + h) * P + r] = (bf16)(a * gsc * (ge != nullptr ? mx_sigmoid((float)ge[r]) : 1.0f));
+    out[(row * H + h) * P + r] = (T)(a * gsc * (ge != nullptr ? mx_sigmoid(ldf(ge + r)) : 1.0f));
   }
 }
 
@@ -707,20 +705,49 @@ MX_API int mx_qk_norm_write(const void* q, long sq, const void* k, long sk, cons
 // cap > 0: the scaled score becomes cap * tanh(score / cap) before any bias.  slope (f32 [H], or null):
 // score - slope[h] * (p - j).  rel (f32 [H, rel_len], or null): score + rel[h][min(p - j, rel_len - 1)].  sink (f32 [H], or null; softmax only): exp(sink[h]) in
 // the denominator.  gate_elem != 0: the gate is a [T, >= H*P] slice, one value per output element.
-// nsplit > 1 with a workspace ws (f32 [T, H, nsplit, P + 2]) and single-row segments: the key range of
-// each row is walked by nsplit blocks and merged (bf16 matrix-core form only; ignored otherwise).
+// nsplit > 1 with a workspace ws (f32 [rows, H, nsplit, P + 2]): the keys of each row are walked by nsplit blocks and
+// merged (rows_attend.h; the older matrix-core form does so for single-row segments only, the f32-lane form never).
+// Which form: rows_attend.h for heads of 128 in 16-byte rows, in both types, with softmax weights and no distance table
+// (16 heads over 4, window 1024, before -> after: segments of 390, 400 and 380 rows and 21 single ones 131 -> 44 us; 2433
+// rows from position 0 101 -> 39; 48 single rows 39 -> 24; f32: 577 rows 317 -> 33, 8 single rows 153 -> 17); the older
+// forms for everything else.
 MX_API int mx_window_attend(const void* q, long sq, const void* cache, const int* cu, const int* pos, const int* bt,
                             int btw, const void* gate, long sgate, int gate_elem, int window, int chunked, int keep,
                             const float* head_bias, const float* slope, const float* rel, int rel_len, float cap,
                             const float* sink, float scale, void* out, int dt, int S, int max_len, int H, int G,
-                            int D, int P, int nsplit, float* ws, hipStream_t st) {
+                            int D, int P, int nsplit, float* ws, int rows, hipStream_t st) {
   if (S <= 0 || max_len <= 0) return 0;
   if (P > 64 * WA_CPL || G < 1 || H % G || window < 1 || keep < 0 ||
       (gate_elem && gate == nullptr) || (sink != nullptr && head_bias != nullptr) || (rel != nullptr && rel_len < 1))
     return (int)hipErrorInvalidValue;
   // 2: gate rows that 8-byte accesses may read (bf16)
   const int ge = !gate_elem ? 0 : (P % 4 == 0 && sgate % 4 == 0 && (size_t)gate % 8 == 0 ? 2 : 1);
-  const int rep = H / G;
+  const int rep = H / G, es = dt == 1 ? 4 : 2;
+  if (D == 128 && P == 128 && head_bias == nullptr && rel == nullptr && wa_use_mfma() && sq * es % 16 == 0 &&
+      ((size_t)q | (size_t)cache | (size_t)out) % 16 == 0 && window <= (1 << 30)) {
+    const int HB = rep < 64 ? rep : 64, QT = max_len == 1 ? 1 : 64 / HB;
+    if (ws == nullptr || nsplit < 1) nsplit = 1;
+    RowsArgs a{q, nullptr, sq, cache, G * (D + P), D, G * D, P, cu, pos, bt, btw, gate, sgate, gate_elem, window, chunked, keep,
+               slope, cap, sink, scale, out, H, G, QT, HB, nsplit, ws};
+    const dim3 grid((unsigned)((max_len + QT - 1) / QT * nsplit), G * ((rep + HB - 1) / HB), S);
+    // 64 keys per tile while all blocks find a place at two per CU (64 KB of LDS each; 98 x 4 blocks: 43 us, 32 keys: 55),
+    // 32 keys and four blocks per CU beyond (512 x 4 blocks: 127 us, 64 keys: 137)
+    const bool few = ((long)S + (long)rows * HB / 64) * G * ((rep + HB - 1) / HB) * nsplit <= 512;
+    if (dt == 1) {
+      if (cap > 0.f) rows_attend_kernel<float, 128, 0, 128, false, 1, 4, 32, true, false><<<grid, 256, 0, st>>>(a);
+      else rows_attend_kernel<float, 128, 0, 128, false, 1, 4, 32, false, false><<<grid, 256, 0, st>>>(a);
+    } else if (few) {
+      if (cap > 0.f) rows_attend_kernel<bf16, 128, 0, 128, false, 1, 4, 64, true, true><<<grid, 256, 0, st>>>(a);
+      else rows_attend_kernel<bf16, 128, 0, 128, false, 1, 4, 64, false, true><<<grid, 256, 0, st>>>(a);
+    } else {
+      if (cap > 0.f) rows_attend_kernel<bf16, 128, 0, 128, false, 1, 4, 32, true, true><<<grid, 256, 0, st>>>(a);
+      else rows_attend_kernel<bf16, 128, 0, 128, false, 1, 4, 32, false, true><<<grid, 256, 0, st>>>(a);
+    }
+    if (nsplit > 1)
+      MX_DISPATCH(dt, TT, window_merge_kernel<TT><<<dim3(rows, H), 128, 0, st>>>(
+          ws, (const TT*)gate, sgate, gate_elem, sink, (TT*)out, H, P, nsplit, 0));
+    MX_RETURN_LAUNCH();
+  }
   const bool forms = (cap <= 0.f || head_bias == nullptr) &&
                      (rel == nullptr || (head_bias == nullptr && slope == nullptr && keep == 0));
   if (dt == 0 && D <= 256 && P <= 256 && forms && wa_use_mfma()) {
@@ -756,7 +783,7 @@ MX_API int mx_window_attend(const void* q, long sq, const void* cache, const int
 #undef WINDOW_LAUNCH
     if (nsplit > 1) {
       dim3 g2(S, H);           // single-row segments: row index == segment index
-      window_merge_kernel<<<g2, P >= 128 ? 128 : 64, 0, st>>>(ws, (const bf16*)gate, sgate, ge, sink, (bf16*)out, H, P,
+      window_merge_kernel<bf16><<<g2, P >= 128 ? 128 : 64, 0, st>>>(ws, (const bf16*)gate, sgate, ge, sink, (bf16*)out, H, P,
                                                               nsplit, head_bias != nullptr ? 1 : 0);
     }
     MX_RETURN_LAUNCH();

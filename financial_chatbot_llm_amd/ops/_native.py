@@ -113,7 +113,7 @@ _MIXER_SIGS = {
     "mx_qk_norm_write": [P, c_long, P, c_long, P, c_long, P, P, c_float, c_int, c_int, c_int, P, c_float, P, P, P, P, c_int,
                          c_int, c_int, c_int, c_int, P],
     "mx_window_attend": [P, c_long, P, P, P, P, c_int, P, c_long, c_int, c_int, c_int, c_int, P, P, P, c_int, c_float, P,
-                         c_float, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, P, P],
+                         c_float, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, P, c_int, P],
     "mx_mingru_scan": [P, c_long, P, c_long, P, c_long, c_int, P, P, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int,
                        c_int, P],
     "mx_decay_scan": [P, c_long, P, c_long, c_int, P, c_long, c_int, c_int, P, c_float, P, P, P, P, P, c_int, c_int,
@@ -127,7 +127,7 @@ _MIXER_SIGS = {
     "mx_latent_prep": [P, c_long, P, c_float, P, c_int, c_float, P, P, P, P, c_long, c_int, c_int, P, c_int, c_int, c_int,
                        c_int, c_int, P],
     "mx_latent_attend": [P, P, P, P, P, P, c_int, P, c_long, P, c_int, c_int, c_float, P, c_int, c_int, c_int, c_int, c_int,
-                         c_int, c_int, P, P],
+                         c_int, c_int, P, c_int, P],
 }
 _MIXER_LIB: Optional[ctypes.CDLL] = None
 

@@ -494,18 +494,22 @@ def latent_attend(q_lat: torch.Tensor, q_rot: torch.Tensor, cache: torch.Tensor,
     if N.use_native(q_lat):
         assert q_lat.is_contiguous() and q_rot.is_contiguous() and bt.is_contiguous()
         out = torch.empty((T, H, R), dtype=q_lat.dtype, device=q_lat.device)
-        # decode-size steps (one row per segment) walk each row's keys with several blocks so that a
-        # small batch still fills the chip; the split depends only on static sizes (graph-safe)
+        # steps whose blocks (64 pairs of a row and a head) would leave the chip idle walk each row's keys with several
+        # blocks; the split depends only on static sizes (graph-safe).  R = 256 (64 keys per tile, two blocks per CU; 32
+        # heads, window 1024): 64 single rows take 24 us with 256 blocks, 42 with 1024; 256 rows of one segment and 30 single
+        # ones 72 us unsplit, 69 with 512 blocks
         nsplit, ws = 1, None
-        if max_len == 1 and q_lat.dtype == torch.bfloat16:
-            tiles = (min(window, bt.shape[1] * PAGE) + 31) // 32 + 1
-            nsplit = max(1, min(16, tiles // 2, 1024 // max(S * ((H + 63) // 64), 1)))
+        if q_lat.dtype == torch.bfloat16 and (max_len == 1 or (R == 256 and Dr in (0, 32))):
+            tiles = (min(window + max_len, bt.shape[1] * PAGE) + 31) // 32 + 1
+            blocks = S * ((H + 63) // 64) if max_len == 1 else S + T * H // 64
+            want = 512 if max_len > 1 else 256 if R == 256 and Dr in (0, 32) else 1024
+            nsplit = max(1, min(16, tiles // 2, want // max(blocks, 1)))
             if nsplit > 1:
                 ws = torch.empty((T, H, nsplit, R + 2), dtype=torch.float32, device=q_lat.device)
         N.mcall("mx_latent_attend", N.ptr(q_lat), N.ptr(q_rot), N.ptr(cache), N.ptr(cu), N.ptr(pos), N.ptr(bt),
                 bt.shape[1], N.ptr(_rows(gate)) if gate is not None else None,
                 gate.stride(0) if gate is not None else 0, N.ptr(sink), 1 if exact_weights else 0,
-                int(min(window, 1 << 30)), float(scale), N.ptr(out), _dt(q_lat), S, int(max_len), H, R, Dr, nsplit, N.ptr(ws), N.stream())
+                int(min(window, 1 << 30)), float(scale), N.ptr(out), _dt(q_lat), S, int(max_len), H, R, Dr, nsplit, N.ptr(ws), T, N.stream())
         return out
     out = torch.zeros((T, H, R), dtype=torch.float32)
     rows = cache.view(-1, R + Dr).float()
@@ -1026,12 +1030,16 @@ def window_attend(q: torch.Tensor, cache: torch.Tensor, cu: torch.Tensor, pos: t
     if N.use_native(q):
         assert bt.is_contiguous() and q.dtype == cache.dtype
         out = torch.empty((T, H * P), dtype=q.dtype, device=q.device)
-        # decode-size steps (one row per segment) walk each row's keys with several blocks so that a
-        # small batch still fills the chip; the split depends only on static sizes (graph-safe)
+        # steps whose blocks (64 pairs of a row and a head of one group) would leave the chip idle walk each row's keys with
+        # several blocks; the split depends only on static sizes (graph-safe).  Single rows want 1024 blocks (48 rows of 16
+        # heads over 4, window 1024: 25 us, at 256 blocks 39); with longer segments merging the parts costs more, and 512
+        # are enough (577 rows in f32: 34 us at 468 blocks)
         nsplit, ws = 1, None
-        if max_len == 1 and q.dtype == torch.bfloat16:
-            tiles = (min(window + keep_first, bt.shape[1] * PAGE) + 31) // 32 + 1
-            nsplit = max(1, min(16, tiles // 2, 1024 // max(S * G, 1)))
+        tiled = D == 128 and P == 128 and head_bias is None and rel is None
+        if tiled or (max_len == 1 and q.dtype == torch.bfloat16):
+            tiles = (min(window + keep_first + max_len, bt.shape[1] * PAGE) + 31) // 32 + 1
+            blocks = S * G if max_len == 1 else (S + T * (H // G) // 64) * G
+            nsplit = max(1, min(16, tiles // 2, (1024 if max_len == 1 else 512) // max(blocks, 1)))
             if nsplit > 1:
                 ws = torch.empty((T, H, nsplit, P + 2), dtype=torch.float32, device=q.device)
         N.mcall("mx_window_attend", N.ptr(_rows(q)), q.stride(0), N.ptr(cache), N.ptr(cu), N.ptr(pos), N.ptr(bt), bt.shape[1],
@@ -1039,7 +1047,7 @@ def window_attend(q: torch.Tensor, cache: torch.Tensor, cu: torch.Tensor, pos: t
                 1 if gate_elem else 0, int(min(window, 1 << 30)), 1 if chunked else 0, int(keep_first), N.ptr(head_bias),
                 N.ptr(slopes), N.ptr(rel), rel.shape[1] if rel is not None else 0, float(softcap), N.ptr(sink), float(scale),
                 N.ptr(out),
-                _dt(q), S, int(max_len), H, G, D, P, nsplit, N.ptr(ws), N.stream())
+                _dt(q), S, int(max_len), H, G, D, P, nsplit, N.ptr(ws), T, N.stream())
         return out
     out = torch.zeros((T, H, P), dtype=torch.float32)
     rows = cache.view(-1, Wr).float()
