@@ -19,6 +19,8 @@
 //            the current chunk's dependent steps run; the chunk's outputs leave through LDS as
 //            whole runs.  Steps with few (segment, head) pairs take the variant with more lanes per
 //            column so that the grid still covers the chip.
+//   gla and delta with a segment of 32 rows or more and D <= 256 take chunks of 16 tokens on the f32 matrix
+//   instructions instead (further down).
 //
 // mx_lru_scan: a diagonal recurrence per channel, S <- a S + sqrt(1 - a^2) i u with
 //     a = exp(-8 sigmoid(zr + r_bias) softplus(lam)),  i = sigmoid(zi + i_bias),
@@ -33,6 +35,8 @@
 //   only the current token: z = sigmoid(zp + z_bias), u = xp + x_bias, c = u + 1/2 for u >= 0 and
 //   sigmoid(u) below; output S * silu(gp).  The same two launches (a gates pass that leaves 1 - z, z c
 //   and the SiLU branch in f32, then the recurrence kernel above) or one fused launch for single rows.
+#include <type_traits>
+
 #include "mx_common.h"
 
 namespace {
@@ -441,12 +445,389 @@ int dispatch_matrix_scan(int D, bool wide, Args... args) {
   return launch_matrix_scan<TQ, 32, 16, DELTA>(args...);
 }
 
+// ---- chunks of 16 tokens on the f32 matrix instructions (gla and delta, steps with longer segments).
+// With G_t the product of a chunk's decays up to token t (per key channel), E_t that of the tokens behind t, and
+// w(s, t) = G_t / G_s formed as the running product of the decays between them -- no quotients, no exponents of sums: every
+// factor is the one that the token form applies, and none exceeds 1 --
+//     A[t][s] = sum_d q_t k_s w(s, t)  (s <= t),   M[t][s] = sum_d k_t k_s w(s, t)  (s < t),
+//     delta:  U = T V - W S,  T = (1 + b M)^-1 b,  W = T (k G)   by forward substitution;   gla:  U = V
+//     O = (q G) S + A U,      S <- G_15 S + (k E)^T U.
+// scan_chunk_prep_kernel makes A, T, W, q G, k E of all chunks at once, in the order of the matrix operands: 16 threads per
+// s walk t with w in registers.  scan_chunk_kernel walks the chunks of a (segment, head, 16 value columns): four waves own a
+// quarter of the key channels of S each, in registers, the sums over channels meet in LDS, one barrier per chunk.
+// Bound by the f32 matrix rate where many (segment, head) pairs run (3 D P products per token), by the chain of 26 dependent
+// products per 16 tokens otherwise; the operands come three chunks ahead (one ahead: 144 against 125 us for the chain of 1500
+// tokens).  16 heads, values of 128, token form -> both launches here: delta, D = 128, segments of 1500, 40, 600, 1 and 1
+// tokens 509 -> 175 us (50 of them the preparation), four of 2048 865 -> 421, 64 + 40 + 32 tokens 41 -> 26; gla, D = 64,
+// 279 -> 77, 433 -> 140 and 19 -> 16.  Errors against 64 bits are those of the token form.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int SCC = 16;                  // tokens per chunk
+constexpr int SCAN_LEAST = 32;           // the longest segment from which the chunk form is taken (two chunks; see above)
+
+__host__ __device__ inline long scan_chunk_floats(int DP, bool delta) { return 33L * DP + 256 + (delta ? 256 + 16L * DP : 0); }
+
+// where (s, t) of A and T lies: wave s % 4 reads its 64 consecutive values
+__device__ __forceinline__ int chunk_pair(int s, int t) { return (s & 3) * 64 + (s >> 2) * 16 + t; }
+
+// exp(x) for x <= 0: the product with log2 e in two parts, so that the error is that of the exponential alone
+__device__ __forceinline__ float exp_below(float x) {
+  x = x < -150.f ? -150.f : x;
+  const float h = x * 1.44269502f, l = fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269502f, -h));
+  const float e = __builtin_amdgcn_exp2f(h);
+  return fmaf(e, l * 0.693147182f, e);
+}
+
+// exp(rate * softplus(z)), rate <= 0, without branches (the general functions took half of the chunk preparation's vector
+// instructions: 8192 rows x 16 heads x 128 channels 200 -> 177 us).  log(1 + y) = 2 atanh(s), s = y / (2 + y) <= 1/3, by the
+// series of atanh to s^17, whose rest is below 2^-29 of the sum.
+__device__ __forceinline__ float decay_of(float z, float rate) {
+  const float y = exp_below(-fabsf(z)), d = 2.f + y;
+  float r = __builtin_amdgcn_rcpf(d);
+  r = fmaf(fmaf(-d, r, 1.f), r, r);
+  const float s = y * r, q = s * s;
+  float p = 1.f / 17;
+  p = fmaf(p, q, 1.f / 15);
+  p = fmaf(p, q, 1.f / 13);
+  p = fmaf(p, q, 1.f / 11);
+  p = fmaf(p, q, 1.f / 9);
+  p = fmaf(p, q, 1.f / 7);
+  p = fmaf(p, q, 1.f / 5);
+  p = fmaf(p, q, 1.f / 3);
+  const float s2 = 2.f * s, sp = (z < 0.f ? 0.f : z) + fmaf(s2 * q, p, s2);
+  return exp_below(rate * sp);
+}
+
+// grid (T / 16 + S, H): chunk x of the step; segment s starts at chunk cu[s] / 16 + s
+template <typename TQ, int DP, bool DELTA>
+__global__ void __launch_bounds__(256, 2)
+scan_chunk_prep_kernel(const TQ* __restrict__ q, long sq, const TQ* __restrict__ k, long sk, const float* __restrict__ a,
+                       long sa, const float* __restrict__ a_bias, const float* __restrict__ A_log,
+                       const void* __restrict__ beta, long sbeta, int beta_code, float tau_inv, float* __restrict__ ws,
+                       const int* __restrict__ cu, const int* __restrict__ slot, int S, int H, int G, int D) {
+  constexpr int LD = DP + 4;             // 16 rows at one column meet different banks
+  __shared__ __align__(16) float qs[SCC * LD], ks[SCC * LD], gs[SCC * LD];
+  __shared__ __align__(16) float As[SCC * SCC], Ms[SCC * SCC];
+  __shared__ float bs[SCC];
+  const int h = blockIdx.y, kvh = h / (H / G), tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ci = blockIdx.x;
+  int s = 0;
+  for (int lo = 0, hi = S; lo < hi;) {   // the last segment that starts at or before this chunk
+    const int mid = (lo + hi) >> 1;
+    if (cu[mid] / SCC + mid <= ci) {
+      s = mid;
+      lo = mid + 1;
+    } else {
+      hi = mid;
+    }
+  }
+  const int first = (ci - cu[s] / SCC - s) * SCC, n = cu[s + 1] - cu[s];
+  if (slot[s] < 0 || first < 0 || first >= n) return;
+  const long row0 = cu[s] + first;
+  const int nt = min(SCC, n - first);
+  const float qscale = 1.0f / sqrtf((float)D);
+  const float rate = DELTA ? -expf(A_log[h]) : -tau_inv;
+  constexpr int NE = SCC * DP / 256;     // elements per thread, in rows of its wave; loads are clamped and issued together
+  const int d0 = tid % DP, dc = min(d0, D - 1), tw = wave * 64 / DP;
+  TQ xq[NE], xk[NE];
+  float xa[NE];
+#pragma unroll
+  for (int i = 0; i < NE; ++i) {
+    const long row = row0 + min(tw + i * (256 / DP), nt - 1);
+    xq[i] = (q + row * sq + kvh * D)[dc];
+    xk[i] = (k + row * sk + kvh * D)[dc];
+    xa[i] = (a + row * sa + h * D)[dc];
+  }
+  const float xb = a_bias[h * D + dc];
+#pragma unroll
+  for (int i = 0; i < NE; ++i) {
+    const int t = tw + i * (256 / DP);
+    const bool live = t < nt && d0 < D;
+    const float z = xa[i] + xb;
+    qs[t * LD + d0] = live ? ldf(&xq[i]) * (DELTA ? 1.f : qscale) : 0.f;
+    ks[t * LD + d0] = live ? ldf(&xk[i]) : 0.f;
+    gs[t * LD + d0] = live ? decay_of(DELTA ? z : -z, rate) : 1.f;
+  }
+  As[tid] = Ms[tid] = 0.f;
+  if (DELTA && tid < SCC) bs[tid] = tid < nt ? mx_sigmoid(ld_code(beta, beta_code, (row0 + tid) * sbeta + h)) : 0.f;
+  __syncthreads();
+  if (DELTA) {                           // unit rows of q (scaled) and k
+    for (int r = wave; r < 2 * SCC; r += 4) {
+      float* x = (r & 1 ? ks : qs) + (r >> 1) * LD;
+      float ss = 0.f;
+      for (int d = lane; d < DP; d += 64) ss += x[d] * x[d];
+      ss = mx_wave_sum(ss);
+      const float f = ((r & 1) ? 1.0f : qscale) / sqrtf(ss + 1e-6f);
+      for (int d = lane; d < DP; d += 64) x[d] *= f;
+    }
+    __syncthreads();
+  }
+  {                                      // 16 lanes share s: channels 4 dg .. + 3 of every 64
+    const int sj = tid >> 4, dg = (tid & 15) * 4;
+    f32x4 w[DP / 64];
+#pragma unroll
+    for (int j = 0; j < DP / 64; ++j) w[j] = *reinterpret_cast<const f32x4*>(ks + sj * LD + 64 * j + dg);
+    auto row = [&](int t, auto edge) {   // edge: some of this wave's s lie at or behind t
+      float aq = 0.f, ak = 0.f;
+#pragma unroll
+      for (int j = 0; j < DP / 64; ++j) {
+        const f32x4 qq = *reinterpret_cast<const f32x4*>(qs + t * LD + 64 * j + dg);
+        const f32x4 gg = *reinterpret_cast<const f32x4*>(gs + t * LD + 64 * j + dg);
+        if (!edge.value || t > sj) w[j] *= gg;
+        aq += qq[0] * w[j][0] + qq[1] * w[j][1] + qq[2] * w[j][2] + qq[3] * w[j][3];
+        if (DELTA) {
+          const f32x4 kk = *reinterpret_cast<const f32x4*>(ks + t * LD + 64 * j + dg);
+          ak += kk[0] * w[j][0] + kk[1] * w[j][1] + kk[2] * w[j][2] + kk[3] * w[j][3];
+        }
+      }
+      aq = lane_group_sum<16>(aq);
+      if (DELTA) ak = lane_group_sum<16>(ak);
+      if (dg == 0 && t >= sj) {
+        As[chunk_pair(sj, t)] = aq;
+        if (DELTA && t > sj) Ms[t * SCC + sj] = ak;
+      }
+    };
+#pragma unroll
+    for (int t = 0; t < 4; ++t) row(4 * wave + t, std::true_type{});
+    for (int t = 4 * wave + 4; t < SCC; ++t) row(t, std::false_type{});
+  }
+  __syncthreads();
+  float* out = ws + ((long)ci * H + h) * scan_chunk_floats(DP, DELTA);
+  for (int d = tid; d < DP + (DELTA ? SCC : 0); d += 256) {
+    float x[SCC], g = 1.f;
+#pragma unroll
+    for (int t = 0; t < SCC; ++t) {
+      float r;
+      if (d < DP) {
+        g *= gs[t * LD + d];
+        qs[t * LD + d] *= g;
+        r = ks[t * LD + d] * g;
+      } else {
+        r = t == d - DP ? 1.f : 0.f;
+      }
+      if (DELTA) {
+#pragma unroll
+        for (int i = 0; i < t; ++i) r -= Ms[t * SCC + i] * x[i];
+        x[t] = r * bs[t];
+      }
+    }
+    if (d < DP) {
+      out[32 * DP + d] = g;
+      float e = 1.f;
+#pragma unroll
+      for (int t = SCC - 1; t >= 0; --t) {
+        const float gt = gs[t * LD + d];
+        ks[t * LD + d] *= e;
+        e *= gt;
+        if (DELTA) gs[t * LD + d] = -x[t];
+      }
+    } else if (DELTA) {
+#pragma unroll
+      for (int t = 0; t < SCC; ++t) out[33 * DP + 256 + chunk_pair(d - DP, t)] = x[t];
+    }
+  }
+  __syncthreads();
+  out[33 * DP + tid] = As[tid];
+  for (int e = tid; e < 4 * DP; e += 256) {                      // 16-byte operand pieces: tile e / 64, lane e % 64
+    const int j = (e >> 6) * 16, c = e & 15, g = (e >> 4) & 3;
+    *reinterpret_cast<f32x4*>(out + 4 * e) = *reinterpret_cast<const f32x4*>(qs + c * LD + j + 4 * g);
+    f32x4 x;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x[r] = ks[(4 * g + r) * LD + j + c];
+    *reinterpret_cast<f32x4*>(out + 16 * DP + 4 * e) = x;
+    if (DELTA)
+      *reinterpret_cast<f32x4*>(out + 33 * DP + 512 + 4 * e) = *reinterpret_cast<const f32x4*>(gs + c * LD + j + 4 * g);
+  }
+}
+
+// A token whose value is not finite must not reach the tokens before it through the zeros of A and T: such elements of a
+// chunk (rows 4 g + r of column lane % 16) become zero, and the first one's row is returned (16: none).
+__device__ __forceinline__ int drop_nonfinite(f32x4& x, int g) {
+  bool bad = false;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) bad |= !(fabsf(x[r]) < INFINITY);
+  if (!__any(bad)) return SCC;
+  int first = SCC;
+#pragma unroll
+  for (int r = 3; r >= 0; --r)
+    if (!(fabsf(x[r]) < INFINITY)) {
+      first = 4 * g + r;
+      x[r] = 0.f;
+    }
+  first = min(first, __shfl_xor(first, 16, 64));
+  return min(first, __shfl_xor(first, 32, 64));
+}
+
+// grid (H, ceil(P / 16), S): all column blocks of a head on one chiplet, whose cache then holds the chunk's operands
+template <typename TQ, int DP, int NW, bool DELTA>
+__global__ void __launch_bounds__(NW * 64, 2)
+scan_chunk_kernel(const TQ* __restrict__ v, long sv, const float* __restrict__ ws, float* __restrict__ state,
+                  const int* __restrict__ cu, const int* __restrict__ slot, const int* __restrict__ pos,
+                  float* __restrict__ out, int H, int D, int P) {
+  constexpr int TPW = DP / 16 / NW;      // tiles of 16 key channels per wave
+  __shared__ __align__(16) f32x4 us[2][NW][64];
+  __shared__ __align__(16) f32x4 os[2][NW][64];
+  const int h = blockIdx.x, s = blockIdx.z;
+  const int sl = slot[s], r0 = cu[s], n = cu[s + 1] - r0;
+  if (sl < 0 || n <= 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c = lane & 15;
+  const int col = blockIdx.y * 16 + c;
+  const bool cok = col < P;
+  float* srec = state + ((long)sl * H + h) * D * P;
+  f32x4 S[TPW];
+  const bool fresh = pos[r0] == 0;
+#pragma unroll
+  for (int j = 0; j < TPW; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int d = 16 * (w * TPW + j) + 4 * g + r;
+      S[j][r] = !fresh && cok && d < D ? srec[(long)d * P + col] : 0.f;
+    }
+  const long step = (long)H * scan_chunk_floats(DP, DELTA);
+  const float* base = ws + (long)(r0 / SCC + s) * step + h * scan_chunk_floats(DP, DELTA);
+  const int last = (n - 1) / SCC;
+  struct Chunk {
+    f32x4 q[TPW], k[TPW], w[TPW], g[TPW];
+    TQ v[4];
+    float a, t;
+  };
+  const TQ* vp = v + (long)r0 * sv + h * P + min(col, P - 1);
+  const TQ* vf = vp + 4 * g * sv;
+  auto fetch = [&](Chunk& x, int t0) {   // x: the chunk of tokens t0 .. (behind the end: the last one again)
+    const float* p = base + min(t0 / SCC, last) * step;
+#pragma unroll
+    for (int j = 0; j < TPW; ++j) {
+      const int o = ((w * TPW + j) * 64 + lane) * 4;
+      x.q[j] = *reinterpret_cast<const f32x4*>(p + o);
+      x.k[j] = *reinterpret_cast<const f32x4*>(p + 16 * DP + o);
+      if (DELTA) x.w[j] = *reinterpret_cast<const f32x4*>(p + 33 * DP + 512 + o);
+      x.g[j] = *reinterpret_cast<const f32x4*>(p + 32 * DP + 16 * (w * TPW + j) + 4 * g);
+    }
+    x.a = p[33 * DP + (tid & 255)];
+    if (DELTA) x.t = p[33 * DP + 256 + (tid & 255)];
+    if (t0 + SCC <= n) {                 // (64-bit products are slow: only the tail forms them)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x.v[r] = vf[r * sv];
+      vf += SCC * sv;
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x.v[r] = vp[min(t0 + 4 * g + r, n - 1) * sv];
+    }
+  };
+  auto mine = [&](const f32x4& x) {      // tokens 4 g + w of a tile: this wave's K step (the first four waves')
+    const float y = w == 0 ? x[0] : w == 1 ? x[1] : w == 2 ? x[2] : x[3];
+    return NW == 4 || w < 4 ? y : 0.f;
+  };
+  float* op = out + (long)(r0 + 4 * g + w) * H * P + h * P + col;
+  const long orow = (long)SCC * H * P;
+  auto flush = [&](int t0, int buf) {    // a finished chunk: this wave's rows 4 g + w (the first four waves)
+    const int t = t0 + 4 * g + w;
+    const float* o = reinterpret_cast<const float*>(&os[buf][0][0]) + lane * 4 + (w & 3);
+    float y = (o[0] + o[256]) + (o[512] + o[768]);
+    if (NW == 8) y += (o[1024] + o[1280]) + (o[1536] + o[1792]);
+    if (t < n && cok && w < 4) *op = y;
+    op += orow;
+  };
+  auto walk = [&](Chunk& cur, Chunk& nxt, int t0, int buf) {
+    fetch(nxt, t0 + 3 * SCC);
+    const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 u, o[2] = {zero, zero};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) u[r] = t0 + 4 * g + r < n && cok ? ldf(&cur.v[r]) : 0.f;
+    int bad = drop_nonfinite(u, g);
+    if (DELTA) {
+      // two sums: the many small terms of W S are not rounded at the size of T V
+      f32x4 x[2] = {zero, zero};
+      const f32x4 tv = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.t, mine(u), zero, 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < TPW; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[j & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.w[j][r], S[j][r], x[j & 1], 0, 0, 0);
+      x[0] += TPW > 1 ? x[1] + tv : tv;
+      us[buf][w][lane] = x[0];
+    }
+#pragma unroll
+    for (int j = 0; j < TPW; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[j & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.q[j][r], S[j][r], o[j & 1], 0, 0, 0);
+    // The sum stays on this side of the barrier: moved behind the branches that follow, the vector instruction has been
+    // issued before the matrix instruction's result was there on the path around them.
+    if (TPW > 1) {
+      o[0] += o[1];
+      asm volatile("" : "+v"(o[0]));
+    }
+    __syncthreads();
+    if (DELTA) {
+      u = (us[buf][0][lane] + us[buf][1][lane]) + (us[buf][2][lane] + us[buf][3][lane]);
+      if (NW == 8) u += (us[buf][NW - 4][lane] + us[buf][NW - 3][lane]) + (us[buf][NW - 2][lane] + us[buf][NW - 1][lane]);
+      bad = min(bad, drop_nonfinite(u, g));
+    }
+    if (t0 > 0) flush(t0 - SCC, buf ^ 1);
+    o[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.a, mine(u), o[0], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < TPW; ++j) {
+      S[j] *= cur.g[j];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.k[j][r], u[r], S[j], 0, 0, 0);
+    }
+    if (bad < SCC) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[0][r] = 4 * g + r >= bad ? NAN : o[0][r];
+#pragma unroll
+      for (int j = 0; j < TPW; ++j) S[j] = f32x4{NAN, NAN, NAN, NAN};
+    }
+    os[buf][w][lane] = o[0];
+  };
+  // three chunks ahead: a chunk's step is shorter than the way to memory
+  Chunk x[4];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) fetch(x[i], i * SCC);
+  for (int t0 = 0; t0 < n; t0 += 4 * SCC) {
+    walk(x[0], x[3], t0, 0);
+    if (t0 + SCC >= n) break;
+    walk(x[1], x[0], t0 + SCC, 1);
+    if (t0 + 2 * SCC >= n) break;
+    walk(x[2], x[1], t0 + 2 * SCC, 0);
+    if (t0 + 3 * SCC >= n) break;
+    walk(x[3], x[2], t0 + 3 * SCC, 1);
+  }
+  __syncthreads();
+  flush(last * SCC, last & 1);
+#pragma unroll
+  for (int j = 0; j < TPW; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int d = 16 * (w * TPW + j) + 4 * g + r;
+      if (cok && d < D) srec[(long)d * P + col] = S[j][r];
+    }
+}
+
+template <typename TQ, int TPW, bool DELTA>
+int launch_scan_chunks(const void* q, long sq, const void* k, long sk, const void* v, long sv, const float* a, long sa,
+                       const float* a_bias, const float* A_log, const void* beta, long sbeta, int beta_dt, float tau_inv,
+                       float* ws, float* state, const int* cu, const int* slot, const int* pos, float* out, int S, int T,
+                       int H, int G, int D, int P, hipStream_t st) {
+  scan_chunk_prep_kernel<TQ, 64 * TPW, DELTA><<<dim3(T / SCC + S, H), 256, 0, st>>>(
+      (const TQ*)q, sq, (const TQ*)k, sk, a, sa, a_bias, A_log, beta, sbeta, beta_dt, tau_inv, ws, cu, slot, S, H, G, D);
+  constexpr int NW = TPW <= 2 ? 4 : 8;
+  scan_chunk_kernel<TQ, 64 * TPW, NW, DELTA><<<dim3(H, (P + 15) / 16, S), NW * 64, 0, st>>>((const TQ*)v, sv, ws, state, cu, slot,
+                                                                                          pos, out, H, D, P);
+  MX_RETURN_LAUNCH();
+}
+
 template <typename TQ, bool DELTA>
 int run_matrix_scan(const void* q, long sq, const void* k, long sk, const void* v, long sv, float* a, long sa,
                     const float* a_bias, const float* A_log, const void* beta, long sbeta, int beta_dt, float tau_inv,
-                    float* aux, float* state, const int* cu, const int* slot, const int* pos, float* out, int S, int T,
-                    int H, int G, int D, int P, int max_len, hipStream_t st) {
+                    float* aux, float* ws, float* state, const int* cu, const int* slot, const int* pos, float* out, int S,
+                    int T, int H, int G, int D, int P, int max_len, hipStream_t st) {
   const bool one = max_len == 1;         // every segment is a single row: no chunk staging
+  if (ws != nullptr && max_len >= SCAN_LEAST && D <= 256) {
+#define SCAN_CHUNKS(TPW)                                                                                                  \
+  launch_scan_chunks<TQ, TPW, DELTA>(q, sq, k, sk, v, sv, a, sa, a_bias, A_log, beta, sbeta, beta_dt, tau_inv, ws, state, \
+                                     cu, slot, pos, out, S, T, H, G, D, P, st)
+    return D <= 64 ? SCAN_CHUNKS(1) : D <= 128 ? SCAN_CHUNKS(2) : SCAN_CHUNKS(4);
+#undef SCAN_CHUNKS
+  }
   if (!one)        // single-row steps fold this pass into the scan (one launch less per layer)
     scan_prep_kernel<TQ, DELTA><<<T, 256, 0, st>>>((const TQ*)q, sq, (const TQ*)k, sk, a, sa, a_bias, A_log, beta, sbeta,
                                                    beta_dt, tau_inv, aux, H, G, D);
@@ -466,26 +847,27 @@ int run_matrix_scan(const void* q, long sq, const void* k, long sk, const void* 
 // slice (row stride sa), OVERWRITTEN with the decays; a_bias f32 [H*D]; delta != 0: A_log f32 [H], beta
 // [T, >= H] slice of type beta_dt, aux f32 [T, 2*G + H] scratch; state f32 [slots, H, D, P]; out f32
 // [T, H*P].  T: rows of the step (every row belongs to a segment or is padding); max_len: the longest
-// segment (1: the decode form).
+// segment (1: the decode form).  ws: f32 scratch of
+// (T / 16 + S) * H * scan_chunk_floats(D padded to 64, 128 or 256) values for the chunk form, or null (token form).
 MX_API int mx_matrix_scan(const void* q, long sq, const void* k, long sk, const void* v, long sv, int dt, float* a,
                           long sa, const float* a_bias, const float* A_log, const void* beta, long sbeta, int beta_dt,
-                          float tau, int delta, float* aux, float* state, const int* cu, const int* slot, const int* pos,
-                          float* out, int S, int T, int max_len, int H, int G, int D, int P, hipStream_t st) {
+                          float tau, int delta, float* aux, float* ws, float* state, const int* cu, const int* slot,
+                          const int* pos, float* out, int S, int T, int max_len, int H, int G, int D, int P, hipStream_t st) {
   if (S <= 0 || T <= 0) return 0;
   if (D < 1 || D > 512 || G < 1 || H % G || tau <= 0.f || (delta && (A_log == nullptr || beta == nullptr || aux == nullptr)))
     return (int)hipErrorInvalidValue;
   const float ti = 1.0f / tau;
   if (delta) {
     if (dt == 1)
-      return run_matrix_scan<float, true>(q, sq, k, sk, v, sv, a, sa, a_bias, A_log, beta, sbeta, beta_dt, ti, aux, state,
+      return run_matrix_scan<float, true>(q, sq, k, sk, v, sv, a, sa, a_bias, A_log, beta, sbeta, beta_dt, ti, aux, ws, state,
                                           cu, slot, pos, out, S, T, H, G, D, P, max_len, st);
-    return run_matrix_scan<bf16, true>(q, sq, k, sk, v, sv, a, sa, a_bias, A_log, beta, sbeta, beta_dt, ti, aux, state, cu,
+    return run_matrix_scan<bf16, true>(q, sq, k, sk, v, sv, a, sa, a_bias, A_log, beta, sbeta, beta_dt, ti, aux, ws, state, cu,
                                        slot, pos, out, S, T, H, G, D, P, max_len, st);
   }
   if (dt == 1)
-    return run_matrix_scan<float, false>(q, sq, k, sk, v, sv, a, sa, a_bias, A_log, beta, sbeta, beta_dt, ti, aux, state,
+    return run_matrix_scan<float, false>(q, sq, k, sk, v, sv, a, sa, a_bias, A_log, beta, sbeta, beta_dt, ti, aux, ws, state,
                                          cu, slot, pos, out, S, T, H, G, D, P, max_len, st);
-  return run_matrix_scan<bf16, false>(q, sq, k, sk, v, sv, a, sa, a_bias, A_log, beta, sbeta, beta_dt, ti, aux, state, cu,
+  return run_matrix_scan<bf16, false>(q, sq, k, sk, v, sv, a, sa, a_bias, A_log, beta, sbeta, beta_dt, ti, aux, ws, state, cu,
                                       slot, pos, out, S, T, H, G, D, P, max_len, st);
 }
 

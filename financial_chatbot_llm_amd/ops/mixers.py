@@ -713,6 +713,9 @@ def conv_act(inp: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], s
 # ----------------------------------------------------------------------------------------------
 # matrix-state linear recurrences (gated linear attention, gated delta rule)
 # ----------------------------------------------------------------------------------------------
+SCAN_CHUNK_LEAST = 32         # the longest segment from which the chunk form is taken (see SCAN_LEAST of the kernels)
+
+
 def matrix_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.Tensor, a_bias: torch.Tensor,
                 state: torch.Tensor, cu: torch.Tensor, slot: torch.Tensor, pos: torch.Tensor, heads: int, kv_heads: int,
                 dim: int, vdim: int, mode: str, tau: float = 1.0, A_log: Optional[torch.Tensor] = None,
@@ -721,7 +724,7 @@ def matrix_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.Tens
     [slots, H, dim, vdim], read unless the segment starts at position 0, then replaced), with one
     decay per head and key channel acting on the state's rows.  ``q``/``k`` [T, G*dim], ``v``
     [T, H*vdim] (column slices; head h reads q/k head h // (H/G)), ``a`` f32 [T, H*dim] the decay's
-    pre-activation (the kernels overwrite it with the decays), ``a_bias`` f32 [H*dim].
+    pre-activation (the kernels may overwrite it with the decays), ``a_bias`` f32 [H*dim].
 
     ``mode="gla"``:   g = sigmoid(a + a_bias)^(1/tau);  S <- g S + k v^T;  o = S^T (q dim^-1/2).
     ``mode="delta"``: q, k <- unit vectors (x / sqrt(sum x^2 + 1e-6)), q scaled by dim^-1/2;
@@ -738,10 +741,14 @@ def matrix_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.Tens
     if N.use_native(q):
         out = torch.empty((T, H * P), dtype=torch.float32, device=q.device)
         aux = torch.empty((T, 2 * G + H), dtype=torch.float32, device=q.device) if delta else None
+        ws = None
+        if max_len >= SCAN_CHUNK_LEAST and D <= 256:
+            DP = 64 if D <= 64 else 128 if D <= 128 else 256
+            ws = torch.empty((T // 16 + S, H, 33 * DP + 256 + (16 * DP + 256 if delta else 0)), dtype=torch.float32, device=q.device)
         N.mcall("mx_matrix_scan", N.ptr(_rows(q)), q.stride(0), N.ptr(_rows(k)), k.stride(0), N.ptr(_rows(v)), v.stride(0),
                 _dt(q), N.ptr(_rows(a)), a.stride(0), N.ptr(a_bias), N.ptr(A_log) if delta else None,
                 N.ptr(_rows(beta)) if delta else None, beta.stride(0) if delta else 0, _dt(beta) if delta else 1,
-                float(tau), 1 if delta else 0, N.ptr(aux), N.ptr(state), N.ptr(cu), N.ptr(slot), N.ptr(pos), N.ptr(out), S, T,
+                float(tau), 1 if delta else 0, N.ptr(aux), N.ptr(ws), N.ptr(state), N.ptr(cu), N.ptr(slot), N.ptr(pos), N.ptr(out), S, T,
                 int(max_len), H, G, D, P, N.stream())
         return out
     out = torch.zeros((T, H * P), dtype=torch.float32)
