@@ -132,3 +132,22 @@ __device__ __forceinline__ void better(float& bv, int& bi, float v, int i) {
 }
 
 #define PENNY_RETURN_LAUNCH() return (int)hipGetLastError()
+
+// GELU as max(x, 0) - |x| erfc(|x| / sqrt 2) / 2, without branches: erfc(z) = t Q(t) exp(-z^2), t = 1 / (1 + 0.3 z), Q of
+// degree 8 fitted to a relative error of 2e-8 over z <= 9.5 (beyond, the result is below the smallest f32).  A third of the
+// instructions of x/2 (1 + erff), which a GEMM's epilogue does not hide (36,400 x 3072 x 768: 208 us, with erff 260, the
+// product and bias alone 163), and without its cancellation for negative x: relative error 1.5e-6 for |x| < 5, there 5e-2.
+__device__ __forceinline__ float gelu_erf(float x) {
+  const float t = __builtin_amdgcn_rcpf(fmaf(fabsf(x), 0.2121320366859436f, 1.f));
+  float q = -0.06471703946590424f;
+  q = fmaf(q, t, 0.24254819750785828f);
+  q = fmaf(q, t, -0.25561317801475525f);
+  q = fmaf(q, t, 0.2731974720954895f);
+  q = fmaf(q, t, -0.046815596520900726f);
+  q = fmaf(q, t, 0.10721813142299652f);
+  q = fmaf(q, t, 0.07424121350049973f);
+  q = fmaf(q, t, 0.08534596860408783f);
+  q = fmaf(q, t, 0.08459480851888657f);
+  const float e = q * t * __builtin_amdgcn_exp2f(x * x * -0.72134752f);
+  return fmaf(-fminf(fabsf(x), 64.f), e, fmaxf(x, 0.f));      // (|x| kept finite beside e = 0: gelu(inf) is inf)
+}

@@ -40,7 +40,7 @@ __global__ void gelu_kernel(bf16* __restrict__ x, long n8) {
     float v[8];
     unpack8(*p, v);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = 0.5f * v[k] * (1.f + erff(v[k] * 0.70710678118654752f));
+    for (int k = 0; k < 8; ++k) v[k] = gelu_erf(v[k]);
     *p = pack8(v);
   }
 }

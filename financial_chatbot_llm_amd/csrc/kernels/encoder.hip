@@ -195,7 +195,7 @@ __global__ void __launch_bounds__(512) gemm_bias_small_kernel(const bf16* __rest
       float v = s[r] + (float)bv[r];
       if (GELU) {
         v = (float)(bf16)v;                          // rounded where GEMM-with-bias -> bf16 -> GELU rounds
-        v = 0.5f * v * (1.f + erff(v * 0.70710678118654752f));
+        v = gelu_erf(v);
       }
       y[r] = (bf16)v;
     }

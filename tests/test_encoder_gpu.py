@@ -48,3 +48,20 @@ def test_small_batch_projection(M, N, K, gelu):
         want = F.gelu(want)
     # f32 sums; the result (with gelu also its argument) is rounded to bf16 once
     assert float((got - want).norm() / want.norm()) < 4e-3
+
+
+def test_gelu_over_all_bf16():
+    from financial_chatbot_llm_amd import ops
+    bits = torch.arange(1 << 16, dtype=torch.int32)
+    x = torch.cat([bits[:0x7f81], bits[0x8000:0xff80]]).to(torch.int16).view(torch.bfloat16)   # finite values and +inf
+    x = torch.cat([x, x.new_zeros(-x.numel() % 8)])
+    got = ops.gelu_(x.cuda().clone().view(1, -1)).cpu().view(-1).double()
+    z = x.double()
+    want = 0.5 * z * torch.special.erfc(-z * 0.5 ** 0.5)
+    want[torch.isneginf(want) | torch.isnan(want)] = 0.0
+    fin = torch.isfinite(z)
+    assert torch.isposinf(got[~fin]).all()
+    # one rounding to bf16 (8 significant bits: half a unit in the last place is at most 2^-8; below 2^-126 to zero), and
+    # 3e-7 of x for x > 0, 1e-4 of the result in the negative tail
+    tol = want.abs() * (2.0 ** -8 + 1e-4) + 3e-7 * z.clamp(min=0) * (z.abs() < 10) + 2.0 ** -126
+    assert ((got - want).abs() <= tol)[fin].all(), float(((got - want).abs() / tol)[fin].max())
