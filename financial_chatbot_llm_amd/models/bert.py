@@ -7,17 +7,24 @@ rows as they are (``csrc/kernels/encoder.hip``).
 """
 from __future__ import annotations
 
+import ctypes
 import math
-from typing import Dict, List, Optional, Sequence
+import os
+from typing import Dict, Optional, Sequence, Tuple
 
 import numpy as np
 import torch
 import torch.nn.functional as F
 
 from .. import ops
-from ..ops.gemm import linear_bias
+from ..ops import _native as N
+from ..ops.gemm import BGE_SMALL_MAX_M, linear_bias
 from .common import random_tensor
 from .configs import ModelConfig
+
+
+# a layer's weights, in the order of penny_encoder_layers
+LAYER = ("qkv", "qkv_b", "o", "o_b", "ln1_g", "ln1_b", "fc1", "fc1_b", "fc2", "fc2_b", "ln2_g", "ln2_b")
 
 
 class BertEncoder:
@@ -27,6 +34,9 @@ class BertEncoder:
         self.dtype = dtype
         self.H, self.nh, self.D = cfg.hidden_size, cfg.num_heads, cfg.head_dim
         self.w: Dict[str, torch.Tensor] = {}
+        self.layer_names = [f"layers.{i}.{n}" for i in range(cfg.num_layers) for n in LAYER]
+        shapes = self.shapes()
+        self.layer_shapes = [shapes[n] for n in self.layer_names]
 
     def shapes(self) -> Dict[str, tuple]:
         c = self.cfg
@@ -58,9 +68,38 @@ class BertEncoder:
             self.w[k] = v.to(self.device, self.dtype).contiguous()
         return self
 
-    @torch.no_grad()
-    def forward(self, ids_list: Sequence[Sequence[int]]) -> torch.Tensor:
-        """-> final hidden states [T, H] of the packed batch, plus CLS row indices."""
+    def _embed(self, ids: torch.Tensor, pos: torch.Tensor) -> torch.Tensor:
+        c, w = self.cfg, self.w
+        rows = [w[n] for n in ("word_emb", "pos_emb", "type_emb", "emb_ln_g", "emb_ln_b")]
+        if N.use_native(rows[0]) and self.H in (256, 512, 768, 1024) and \
+                all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.shape[-1] == self.H for t in rows):
+            x = torch.empty((ids.numel(), self.H), dtype=torch.bfloat16, device=ids.device)
+            word, position, kind, g, b = rows
+            N.call("penny_encoder_embed", N.ptr(ids), N.ptr(pos), N.ptr(word), word.shape[0], N.ptr(position),
+                   position.shape[0], N.ptr(kind), N.ptr(g), N.ptr(b), N.ptr(x), x.shape[0], self.H, float(c.norm_eps), N.stream())
+            return x
+        e_word = ops.embedding(ids, w["word_emb"])
+        e_pos = ops.embedding(pos, w["pos_emb"])
+        e_pos = (e_pos.float() + w["type_emb"][0].float()).to(self.dtype)
+        return ops.layer_norm(e_word, w["emb_ln_g"], w["emb_ln_b"], c.norm_eps, residual=e_pos)
+
+    def _small_batch(self, x: torch.Tensor, cu: torch.Tensor, longest: int) -> bool:
+        """All layers of a batch of up to BGE_SMALL_MAX_M tokens in one native call (x in place); False: not a case for it."""
+        T, F_ = x.shape[0], self.cfg.intermediate_size
+        if not (N.use_native(x) and T <= BGE_SMALL_MAX_M and x.dtype == torch.bfloat16 and cu.numel() <= 65536 and
+                self.H % 32 == 0 and F_ % 32 == 0 and os.environ.get("PENNY_PREFILL_GEMM", "1") == "1"):
+            return False
+        w = [self.w[n] for n in self.layer_names]
+        if not all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.device == x.device for t in w) or \
+                [t.shape for t in w] != self.layer_shapes:
+            return False
+        table = (ctypes.c_void_p * len(w))(*[t.data_ptr() for t in w])
+        scratch = torch.empty(T * (6 * self.H + F_), dtype=torch.bfloat16, device=x.device)
+        N.call("penny_encoder_layers", table, self.cfg.num_layers, N.ptr(x), N.ptr(scratch), N.ptr(cu), cu.numel() - 1, longest,
+               T, self.H, self.nh, F_, float(self.cfg.norm_eps), 1.0 / math.sqrt(self.D), N.stream())
+        return True
+
+    def _hidden(self, ids_list: Sequence[Sequence[int]]) -> Tuple[torch.Tensor, np.ndarray, torch.Tensor]:
         c, dev = self.cfg, self.device
         # packed varlen metadata, vectorised on the host (bulk ingest packs 100k+ tokens a call)
         lens = np.fromiter((len(x) for x in ids_list), np.int64, len(ids_list))
@@ -74,12 +113,10 @@ class BertEncoder:
         meta[2 * T:] = cu
         ids_t, pos_t, cu_t = torch.from_numpy(meta).to(dev).split([T, T, len(cu)])
         longest = int(lens.max())
-        cu = cu.tolist()
         w = self.w
-        e_word = ops.embedding(ids_t, w["word_emb"])
-        e_pos = ops.embedding(pos_t, w["pos_emb"])
-        e_pos = (e_pos.float() + w["type_emb"][0].float()).to(self.dtype)
-        x = ops.layer_norm(e_word, w["emb_ln_g"], w["emb_ln_b"], c.norm_eps, residual=e_pos)
+        x = self._embed(ids_t, pos_t)
+        if self._small_batch(x, cu_t, longest):
+            return x, cu, cu_t
         scale = 1.0 / math.sqrt(self.D)
         for i in range(c.num_layers):
             p = f"layers.{i}."
@@ -90,11 +127,21 @@ class BertEncoder:
             h = linear_bias(x, w[p + "fc1"], w[p + "fc1_b"], gelu=True)      # bias + GELU fused
             y = linear_bias(h, w[p + "fc2"], w[p + "fc2_b"])
             x = ops.layer_norm(y, w[p + "ln2_g"], w[p + "ln2_b"], c.norm_eps, residual=x)
-        return x, cu
+        return x, cu, cu_t
+
+    @torch.no_grad()
+    def forward(self, ids_list: Sequence[Sequence[int]]) -> torch.Tensor:
+        """-> final hidden states [T, H] of the packed batch, plus CLS row indices."""
+        x, cu, _ = self._hidden(ids_list)
+        return x, cu.tolist()
 
     @torch.no_grad()
     def encode(self, ids_list: Sequence[Sequence[int]]) -> torch.Tensor:
         """CLS pooling + L2 normalisation (bge convention) -> [n, H] f32."""
-        x, cu = self.forward(ids_list)
-        cls = x[torch.tensor(cu[:-1], device=x.device)]
+        x, cu, cu_t = self._hidden(ids_list)
+        if N.use_native(x) and x.dtype == torch.bfloat16 and cu[-2] < x.shape[0]:
+            out = torch.empty((len(cu) - 1, self.H), dtype=torch.float32, device=x.device)
+            N.call("penny_encoder_pool", N.ptr(x), N.ptr(cu_t), len(cu) - 1, self.H, N.ptr(out), N.stream())
+            return out
+        cls = x[torch.tensor(cu[:-1].tolist(), device=x.device)]
         return F.normalize(cls.float(), dim=-1)

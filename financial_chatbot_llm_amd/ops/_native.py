@@ -28,6 +28,9 @@ P = c_void_p
 _SIGS = {
     "penny_rmsnorm": [P, P, P, P, c_int, c_int, c_float, c_int, P],
     "penny_rmsnorm_slabs": [P, c_int, P, P, P, c_int, c_int, c_float, c_int, P],
+    "penny_encoder_embed": [P, P, P, c_int, P, c_int, P, P, P, P, c_int, c_int, c_float, P],
+    "penny_encoder_pool": [P, P, c_int, c_int, P, P],
+    "penny_encoder_layers": [P, c_int, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, P],
     "penny_layernorm": [P, P, P, P, P, c_int, c_int, c_float, c_int, P],
     "penny_silu_mul": [P, P, c_int, c_int, c_int, P],
     "penny_skinny_gemm": [P, c_int, P, c_int, P, c_int, P, c_int, c_int, c_int, c_int, c_int, c_int, P],

@@ -65,3 +65,39 @@ def test_gelu_over_all_bf16():
     # 3e-7 of x for x > 0, 1e-4 of the result in the negative tail
     tol = want.abs() * (2.0 ** -8 + 1e-4) + 3e-7 * z.clamp(min=0) * (z.abs() < 10) + 2.0 ** -126
     assert ((got - want).abs() <= tol)[fin].all(), float(((got - want).abs() / tol)[fin].max())
+
+
+@pytest.mark.parametrize("lens", [[1], [18], [5, 1, 40, 64, 65], [16] * 48, [500, 268], [500, 269]])
+def test_small_batches_in_one_call(lens, monkeypatch):
+    """The native walk over the layers against the per-layer calls it stands for, bit by bit; 769 tokens take the latter."""
+    from financial_chatbot_llm_amd.models import bert
+    from financial_chatbot_llm_amd.models.configs import get_model_config
+    g = torch.Generator().manual_seed(sum(lens))
+    cfg = get_model_config("bge-base-en")
+    m = bert.BertEncoder.build(cfg, device="cuda", seed=3)
+    ids = [torch.randint(0, cfg.vocab_size, (n,), generator=g).tolist() for n in lens]
+    x, cu = m.forward(ids)
+    e = m.encode(ids)
+    monkeypatch.setattr(m, "_small_batch", lambda *a: False)
+    y, _ = m.forward(ids)
+    assert cu == [0] + torch.tensor(lens).cumsum(0).tolist() and torch.equal(x, y)
+    want = F.normalize(y[torch.tensor(cu[:-1], device="cuda")].float(), dim=-1)
+    assert e.shape == want.shape and float((e - want).abs().max()) < 1e-6      # f32 sums of 768 squares in another order
+
+
+def test_encoder_embed_edges():
+    """Fused embedding rows against the separate ops: last and out-of-table ids, every supported width."""
+    from financial_chatbot_llm_amd import ops
+    from financial_chatbot_llm_amd.ops import _native as N
+    for H in (256, 512, 768, 1024):
+        g = torch.Generator().manual_seed(H)
+        r = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).cuda()  # noqa: E731
+        word, position, kind, w, b = r(50, H), r(9, H), r(2, H), r(H), r(H)
+        ids = torch.tensor([0, 49, 50, 7, 3], dtype=torch.int32, device="cuda")
+        pos = torch.tensor([0, 8, 1, 9, 4], dtype=torch.int32, device="cuda")
+        y = torch.empty(5, H, dtype=torch.bfloat16, device="cuda")
+        N.call("penny_encoder_embed", N.ptr(ids), N.ptr(pos), N.ptr(word), 50, N.ptr(position), 9, N.ptr(kind), N.ptr(w),
+               N.ptr(b), N.ptr(y), 5, H, 1e-12, N.stream())
+        ep = (ops.embedding(pos, position).float() + kind[0].float()).to(torch.bfloat16)
+        want = ops.layer_norm(ops.embedding(ids, word), w, b, 1e-12, residual=ep)
+        assert float((y.float() - want.float()).abs().max()) <= 2.0 ** -6      # a rounding to bf16 below 4
