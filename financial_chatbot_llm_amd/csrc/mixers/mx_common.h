@@ -91,6 +91,20 @@ template <> __device__ __forceinline__ mx_f32x4 mma16<float>(uint4 a, uint4 b, m
   return c;
 }
 
+// four neighbouring elements, as f32
+__device__ __forceinline__ mx_f32x4 ldf4(const float* p) { return *reinterpret_cast<const mx_f32x4*>(p); }
+__device__ __forceinline__ mx_f32x4 ldf4(const bf16* p) {
+  typedef bf16 v4 __attribute__((ext_vector_type(4)));
+  const v4 x = *reinterpret_cast<const v4*>(p);
+  return mx_f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
+}
+template <typename T> __device__ __forceinline__ void stf4(T* p, mx_f32x4 x) {
+  typedef T v4 __attribute__((ext_vector_type(4)));
+  *reinterpret_cast<v4*>(p) = v4{(T)x[0], (T)x[1], (T)x[2], (T)x[3]};
+}
+// rows of `stride` elements of type code dt (1: f32) may be read and written by four
+inline bool mx_by_four(const void* p, long stride, int dt) { return stride % 4 == 0 && (size_t)p % (dt == 1 ? 16 : 8) == 0; }
+
 constexpr int PAGE_ROWS = 64;            // tokens per cache page
 
 // tanh with one division and no branch.  |z| < 0.6: the fifth convergent of Lambert's continued fraction

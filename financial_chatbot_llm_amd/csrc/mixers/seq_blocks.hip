@@ -96,6 +96,68 @@ __global__ void post_norm_kernel(float* __restrict__ x, const TA* __restrict__ a
   }
 }
 
+// The same with the row in registers, by fours, R pieces per thread: one read of every input (2400 rows of 2048 f32 with a
+// bf16 addend and copy: 19 us, through LDS element by element 34).
+template <typename TA, typename TO, int R>
+__global__ void __launch_bounds__(256) post_norm_vec_kernel(float* __restrict__ x, const TA* __restrict__ a, long sa,
+                                                            const float* __restrict__ wa, const TA* __restrict__ b, long sb,
+                                                            const float* __restrict__ wb, const float* __restrict__ w,
+                                                            float eps, TO* __restrict__ out, int W) {
+  __shared__ float scratch[16];
+  const long t = blockIdx.x;
+  const float inv_w = 1.0f / (float)W;
+  const mx_f32x4 zero = mx_f32x4{0.f, 0.f, 0.f, 0.f};
+  mx_f32x4 m[R], xv[R], u[R];
+  auto sum4 = [](mx_f32x4 v) { return (v[0] + v[1]) + (v[2] + v[3]); };
+#pragma unroll
+  for (int c = 0; c < R; ++c) {
+    const int i = 4 * (threadIdx.x + 256 * c);
+    m[c] = xv[c] = u[c] = zero;
+    if (i >= W) continue;
+    xv[c] = ldf4(x + t * W + i);
+    m[c] = a == nullptr ? xv[c] : ldf4(a + t * sa + i);
+    if (b != nullptr) u[c] = ldf4(b + t * sb + i);
+  }
+  if (b != nullptr) {
+    float sa2 = 0.f, sb2 = 0.f;
+#pragma unroll
+    for (int c = 0; c < R; ++c) {
+      sa2 += sum4(m[c] * m[c]);
+      sb2 += sum4(u[c] * u[c]);
+    }
+    sa2 = mx_block_sum(sa2, scratch);
+    sb2 = mx_block_sum(sb2, scratch);
+    const float ka = 1.0f / sqrtf(sa2 * inv_w + eps), kb = 1.0f / sqrtf(sb2 * inv_w + eps);
+#pragma unroll
+    for (int c = 0; c < R; ++c) {
+      const int i = 4 * (threadIdx.x + 256 * c);
+      if (i < W) m[c] = 0.5f * (m[c] * ka * ldf4(wa + i) + u[c] * kb * ldf4(wb + i));
+    }
+  }
+  float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+  for (int c = 0; c < R; ++c) s1 += sum4(m[c]);
+  const float mean = mx_block_sum(s1, scratch) * inv_w;
+#pragma unroll
+  for (int c = 0; c < R; ++c) {
+    if (4 * ((int)threadIdx.x + 256 * c) >= W) continue;
+    const mx_f32x4 d = m[c] - mean;
+    s2 += sum4(d * d);
+  }
+  const float k = 1.0f / sqrtf(mx_block_sum(s2, scratch) * inv_w + eps);
+#pragma unroll
+  for (int c = 0; c < R; ++c) {
+    const int i = 4 * (threadIdx.x + 256 * c);
+    if (i >= W) continue;
+    mx_f32x4 y = (m[c] - mean) * k * ldf4(w + i);
+    if (a != nullptr) {
+      y += xv[c];
+      stf4(x + t * W + i, y);
+    }
+    if (out != nullptr) stf4(out + t * W + i, y);
+  }
+}
+
 // 0.5 z (1 + tanh(u)) with u = sqrt(2/pi) (z + 0.044715 z^3), written as z sigmoid(2u): one exponential
 __device__ __forceinline__ float mx_gelu_tanh(float z) {
   return z * mx_sigmoid(1.5957691216057308f * (z + 0.044715f * z * z * z));
@@ -227,6 +289,33 @@ __global__ void head_norm_gate_kernel(const TI* __restrict__ in, long si, const 
         ldf(r + i) * k * (w != nullptr ? w[i] : 1.f) * mx_act(ldf(gate + t * sg + (long)h * P + i), act));
 }
 
+// The same by fours with L lanes per head (4 L >= P): 2400 rows of 16 heads of 128 15 us, one block per head 30
+template <typename TI, typename TG, typename TO, int L>
+__global__ void __launch_bounds__(256) head_norm_gate_vec_kernel(const TI* __restrict__ in, long si, const float* __restrict__ w,
+                                                                 float eps, const TG* __restrict__ gate, long sg, int act,
+                                                                 TO* __restrict__ out, int H, int P, long total) {
+  const long id = (long)blockIdx.x * (256 / L) + threadIdx.x / L;
+  if (id >= total) return;
+  const long t = id / H;
+  const int h = (int)(id - t * H), i = 4 * (threadIdx.x % L);
+  const bool live = i < P;
+  mx_f32x4 v = mx_f32x4{0.f, 0.f, 0.f, 0.f}, z = v;
+  if (live) {
+    v = ldf4(in + t * si + (long)h * P + i);
+    z = ldf4(gate + t * sg + (long)h * P + i);
+  }
+  float ss = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+#pragma unroll
+  for (int o = 1; o < L; o <<= 1) ss += __shfl_xor(ss, o, 64);
+  const float k = 1.0f / sqrtf(ss / (float)P + eps);
+  if (!live) return;
+  v *= k;
+  if (w != nullptr) v *= ldf4(w + i);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] *= mx_act(z[e], act);
+  stf4(out + id * P + i, v);
+}
+
 }  // namespace
 
 MX_API int mx_embed_pairs(const int* ids, const void* table, const void* pairs, int dt, int mul_prev, int mul_cur,
@@ -247,6 +336,19 @@ MX_API int mx_post_norm(float* x, const void* a, long sa, const float* wa, const
                         int dt_ab, const float* w, float eps, void* out, int dt_out, int T, int W, hipStream_t st) {
   if (T <= 0) return 0;
   if ((size_t)W * sizeof(float) > 60 * 1024 || (a == nullptr && out == nullptr)) return (int)hipErrorInvalidValue;
+  if (W % 4 == 0 && W > 0 && W <= 8192 && ((size_t)x | (size_t)w | (size_t)wa | (size_t)wb) % 16 == 0 &&
+      (a == nullptr || mx_by_four(a, sa, dt_ab)) && (b == nullptr || (a != nullptr && mx_by_four(b, sb, dt_ab))) &&
+      mx_by_four(out, W, dt_out)) {
+#define POST_NORM(R)                                                                                                     \
+  MX_DISPATCH(dt_ab, TA, MX_DISPATCH(dt_out, TO, post_norm_vec_kernel<TA, TO, R><<<T, 256, 0, st>>>(                     \
+      x, (const TA*)a, sa, wa, (const TA*)b, sb, wb, w, eps, (TO*)out, W)))
+    if (W <= 1024) POST_NORM(1);
+    else if (W <= 2048) POST_NORM(2);
+    else if (W <= 4096) POST_NORM(4);
+    else POST_NORM(8);
+#undef POST_NORM
+    MX_RETURN_LAUNCH();
+  }
   const int nt = W >= 1024 ? 512 : 256;
   MX_DISPATCH(dt_ab, TA, MX_DISPATCH(dt_out, TO, post_norm_kernel<TA, TO><<<T, nt, (size_t)W * sizeof(float), st>>>(
       x, (const TA*)a, sa, wa, (const TA*)b, sb, wb, w, eps, (TO*)out, W)));
@@ -291,6 +393,19 @@ MX_API int mx_route_scores(const float* z, int E, int top, int sigmoid_scores, f
 MX_API int mx_head_norm_gate(const void* in, long si, int dt_in, const float* w, float eps, const void* gate, long sg,
                              int dt_gate, int act, void* out, int dt_out, int T, int H, int P, hipStream_t st) {
   if (T <= 0) return 0;
+  if (P % 4 == 0 && P > 0 && P <= 256 && mx_by_four(in, si, dt_in) && mx_by_four(gate, sg, dt_gate) &&
+      mx_by_four(out, P, dt_out) && (size_t)w % 16 == 0 && (long)T * H < (1L << 31)) {
+    const long total = (long)T * H;
+#define HEAD_NORM(L)                                                                                                      \
+  MX_DISPATCH(dt_in, TI, MX_DISPATCH(dt_gate, TG, MX_DISPATCH(dt_out, TO, head_norm_gate_vec_kernel<TI, TG, TO, L>        \
+      <<<(unsigned)((total + 256 / L - 1) / (256 / L)), 256, 0, st>>>((const TI*)in, si, w, eps, (const TG*)gate, sg, act, \
+                                                                      (TO*)out, H, P, total))))
+    if (P <= 64) HEAD_NORM(16);
+    else if (P <= 128) HEAD_NORM(32);
+    else HEAD_NORM(64);
+#undef HEAD_NORM
+    MX_RETURN_LAUNCH();
+  }
   const int nt = P >= 256 ? 256 : (P > 64 ? 128 : 64);
   dim3 grid(T, H);
   MX_DISPATCH(dt_in, TI, MX_DISPATCH(dt_gate, TG, MX_DISPATCH(dt_out, TO, head_norm_gate_kernel<TI, TG, TO>

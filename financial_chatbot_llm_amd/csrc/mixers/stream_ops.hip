@@ -155,6 +155,67 @@ __global__ void group_norm_kernel(const TI* __restrict__ in, long si, const TG* 
   }
 }
 
+// The same by fours, the values of a group in registers: L lanes per group (a part of a wave, or with L = 256 the block), R
+// pieces of four per lane.  Bound by memory (4096 rows of 4096 f32 values in two groups with a bf16 gate: 32 us, element by
+// element with a second read 75).
+template <typename TI, typename TG, typename TO, int L, int R>
+__global__ void __launch_bounds__(256) group_norm_vec_kernel(const TI* __restrict__ in, long si, const TG* __restrict__ gate,
+                                                             long sg, const float* __restrict__ w, float eps,
+                                                             TO* __restrict__ out, long so, int groups, int n, long total) {
+  __shared__ float scratch[16];
+  const long id = (long)blockIdx.x * (256 / L) + threadIdx.x / L;
+  if (id >= total) return;
+  const long t = id / groups;
+  const int g = (int)(id - t * groups), l = threadIdx.x % L;
+  mx_f32x4 v[R];
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < R; ++c) {
+    const int i = 4 * (l + L * c);
+    v[c] = mx_f32x4{0.f, 0.f, 0.f, 0.f};
+    if (i < n) {
+      v[c] = ldf4(in + t * si + (long)g * n + i);
+      if (gate != nullptr) {
+        const mx_f32x4 z = ldf4(gate + t * sg + (long)g * n + i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[c][e] *= mx_silu(z[e]);
+      }
+    }
+    ss += (v[c][0] * v[c][0] + v[c][1] * v[c][1]) + (v[c][2] * v[c][2] + v[c][3] * v[c][3]);
+  }
+  if (L == 256) {
+    ss = mx_block_sum(ss, scratch);
+  } else {
+#pragma unroll
+    for (int o = 1; o < L; o <<= 1) ss += __shfl_xor(ss, o, 64);
+  }
+  const float k = 1.0f / sqrtf(ss / (float)n + eps);
+#pragma unroll
+  for (int c = 0; c < R; ++c) {
+    const int i = 4 * (l + L * c);
+    if (i < n) stf4(out + t * so + (long)g * n + i, v[c] * k * ldf4(w + (long)g * n + i));
+  }
+}
+
+// 16 bytes per thread: 4096 rows of 8192 bf16 21 us, element by element 46
+template <typename T>
+__global__ void __launch_bounds__(256) relu2_vec_kernel(const T* __restrict__ in, long si, T* __restrict__ out, long so, int nv) {
+  const int c = blockIdx.y * 256 + threadIdx.x;
+  if (c >= nv) return;
+  const long t = blockIdx.x;
+  constexpr int H = sizeof(T) == 2 ? 2 : 1;
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    mx_f32x4 v = ldf4(in + t * si + 4 * (H * (long)c + h));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[e] = fmaxf(v[e], 0.f);
+      v[e] *= v[e];
+    }
+    stf4(out + t * so + 4 * (H * (long)c + h), v);
+  }
+}
+
 template <typename T>
 __global__ void relu2_kernel(const T* __restrict__ in, long si, T* __restrict__ out, long so, int n, long total) {
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < total; i += (long)gridDim.x * blockDim.x) {
@@ -411,6 +472,24 @@ MX_API int mx_dyn_tanh(float* x, const void* a, long sa, const int* ids, const v
 MX_API int mx_group_norm(const void* in, long si, int dt_in, const void* gate, long sg, int dt_gate, const float* w,
                          float eps, void* out, long so, int dt_out, int T, int groups, int n, hipStream_t st) {
   if (T <= 0) return 0;
+  if (n % 4 == 0 && n > 0 && n <= 8192 && (size_t)w % 16 == 0 && mx_by_four(in, si, dt_in) && mx_by_four(out, so, dt_out) &&
+      (gate == nullptr || mx_by_four(gate, sg, dt_gate)) && (long)T * groups < (1L << 31)) {
+    const long total = (long)T * groups;
+#define GROUP_NORM(L, R)                                                                                                \
+  MX_DISPATCH(dt_in, TI, MX_DISPATCH(dt_gate, TG, MX_DISPATCH(dt_out, TO, group_norm_vec_kernel<TI, TG, TO, L, R>       \
+      <<<(unsigned)((total + 256 / L - 1) / (256 / L)), 256, 0, st>>>((const TI*)in, si, (const TG*)gate, sg, w, eps,   \
+                                                                      (TO*)out, so, groups, n, total))))
+    if (n <= 64) GROUP_NORM(16, 1);
+    else if (n <= 128) GROUP_NORM(32, 1);
+    else if (n <= 256) GROUP_NORM(64, 1);
+    else if (n <= 512) GROUP_NORM(64, 2);
+    else if (n <= 1024) GROUP_NORM(256, 1);
+    else if (n <= 2048) GROUP_NORM(256, 2);
+    else if (n <= 4096) GROUP_NORM(256, 4);
+    else GROUP_NORM(256, 8);
+#undef GROUP_NORM
+    MX_RETURN_LAUNCH();
+  }
   const int nt = n >= 1024 ? 512 : (n >= 256 ? 256 : 64);
   dim3 grid(T, groups);
   MX_DISPATCH(dt_in, TI, MX_DISPATCH(dt_gate, TG, MX_DISPATCH(dt_out, TO, group_norm_kernel<TI, TG, TO>
@@ -421,6 +500,11 @@ MX_API int mx_group_norm(const void* in, long si, int dt_in, const void* gate, l
 MX_API int mx_relu2(const void* in, long si, void* out, long so, int dt, int T, int n, hipStream_t st) {
   const long total = (long)T * n;
   if (total <= 0) return 0;
+  const int V = dt == 1 ? 4 : 8;
+  if (n % V == 0 && mx_by_four(in, si, dt) && mx_by_four(out, so, dt) && (size_t)n / V <= 65535u * 256u) {
+    MX_DISPATCH(dt, TT, relu2_vec_kernel<TT><<<dim3(T, (n / V + 255) / 256), 256, 0, st>>>((const TT*)in, si, (TT*)out, so, n / V));
+    MX_RETURN_LAUNCH();
+  }
   const int blocks = (int)((total + 255) / 256 < 16384 ? (total + 255) / 256 : 16384);
   MX_DISPATCH(dt, TT, relu2_kernel<TT><<<blocks, 256, 0, st>>>((const TT*)in, si, (TT*)out, so, n, total));
   MX_RETURN_LAUNCH();
