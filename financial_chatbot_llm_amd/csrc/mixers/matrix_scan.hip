@@ -640,24 +640,6 @@ scan_chunk_prep_kernel(const TQ* __restrict__ q, long sq, const TQ* __restrict__
   }
 }
 
-// A token whose value is not finite must not reach the tokens before it through the zeros of A and T: such elements of a
-// chunk (rows 4 g + r of column lane % 16) become zero, and the first one's row is returned (16: none).
-__device__ __forceinline__ int drop_nonfinite(f32x4& x, int g) {
-  bool bad = false;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) bad |= !(fabsf(x[r]) < INFINITY);
-  if (!__any(bad)) return SCC;
-  int first = SCC;
-#pragma unroll
-  for (int r = 3; r >= 0; --r)
-    if (!(fabsf(x[r]) < INFINITY)) {
-      first = 4 * g + r;
-      x[r] = 0.f;
-    }
-  first = min(first, __shfl_xor(first, 16, 64));
-  return min(first, __shfl_xor(first, 32, 64));
-}
-
 // grid (H, ceil(P / 16), S): all column blocks of a head on one chiplet, whose cache then holds the chunk's operands
 template <typename TQ, int DP, int NW, bool DELTA>
 __global__ void __launch_bounds__(NW * 64, 2)
@@ -734,7 +716,7 @@ scan_chunk_kernel(const TQ* __restrict__ v, long sv, const float* __restrict__ w
     f32x4 u, o[2] = {zero, zero};
 #pragma unroll
     for (int r = 0; r < 4; ++r) u[r] = t0 + 4 * g + r < n && cok ? ldf(&cur.v[r]) : 0.f;
-    int bad = drop_nonfinite(u, g);
+    int bad = mx_drop_nonfinite(u, g);
     if (DELTA) {
       // two sums: the many small terms of W S are not rounded at the size of T V
       f32x4 x[2] = {zero, zero};
@@ -760,7 +742,7 @@ scan_chunk_kernel(const TQ* __restrict__ v, long sv, const float* __restrict__ w
     if (DELTA) {
       u = (us[buf][0][lane] + us[buf][1][lane]) + (us[buf][2][lane] + us[buf][3][lane]);
       if (NW == 8) u += (us[buf][NW - 4][lane] + us[buf][NW - 3][lane]) + (us[buf][NW - 2][lane] + us[buf][NW - 1][lane]);
-      bad = min(bad, drop_nonfinite(u, g));
+      bad = min(bad, mx_drop_nonfinite(u, g));
     }
     if (t0 > 0) flush(t0 - SCC, buf ^ 1);
     o[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.a, mine(u), o[0], 0, 0, 0);

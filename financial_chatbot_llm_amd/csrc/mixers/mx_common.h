@@ -105,6 +105,24 @@ template <typename T> __device__ __forceinline__ void stf4(T* p, mx_f32x4 x) {
 // rows of `stride` elements of type code dt (1: f32) may be read and written by four
 inline bool mx_by_four(const void* p, long stride, int dt) { return stride % 4 == 0 && (size_t)p % (dt == 1 ? 16 : 8) == 0; }
 
+// A token whose value is not finite must not reach the tokens before it through the zeros of a triangular factor: such
+// elements of a tile (rows 4 g + r of column lane % 16) become zero, and the first one's row is returned (16: none).
+__device__ __forceinline__ int mx_drop_nonfinite(mx_f32x4& x, int g) {
+  bool bad = false;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) bad |= !(fabsf(x[r]) < INFINITY);
+  if (!__any(bad)) return 16;
+  int first = 16;
+#pragma unroll
+  for (int r = 3; r >= 0; --r)
+    if (!(fabsf(x[r]) < INFINITY)) {
+      first = 4 * g + r;
+      x[r] = 0.f;
+    }
+  first = min(first, __shfl_xor(first, 16, 64));
+  return min(first, __shfl_xor(first, 32, 64));
+}
+
 constexpr int PAGE_ROWS = 64;            // tokens per cache page
 
 // tanh with one division and no branch.  |z| < 0.6: the fifth convergent of Lambert's continued fraction

@@ -385,28 +385,53 @@ ssm_scan_kernel(const float* __restrict__ u, int C, const TD* __restrict__ dt_ra
 //     y_t = e^(c_t) C_t S^T + sum_(s<=t) (C_t . B_s) e^(c_t - c_s) dt_s x_s + D x_t
 //     S  <- e^(c_63) S + sum_s e^(c_63 - c_s) dt_s x_s B_s^T
 // all in f32 (v_mfma_f32_16x16x4_f32; the sums c in f64, so that their differences are good to f32 however far the
-// chunk decays).  C . B is shared by a group's heads: ssd_scores_kernel leaves it in memory once.  Then a block owns 16
-// value channels of one head and walks the chunks of its segment; wave w owns tokens 16 w .. 16 w + 15 of the outputs
-// and N / 4 columns of the state, which the waves exchange through LDS, one barrier per chunk.  Every operand is read
-// from memory in the register layout of its product -- K index 16 j + 4 g + e of step (j, e) for lane group g on both
-// sides -- and the loads of the next chunk are issued as soon as the registers are free.
-// Bound by the matrix cores (80 of these products per wave and chunk) and the exponentials beside them; 2 prompts of
-// 2048, 64 heads of 64 x 128, 2 groups: 285 us and 11 us for the scores, token by token 858 us (a chain of 2048 steps).
+// chunk decays).  Three launches leave to the serial one only products: ssd_scores_kernel makes C . B of a group, which its
+// heads share, and B in operand order; ssd_decay_kernel the factors of every chunk and head, M[t][s] = (C_t . B_s)
+// e^(c_t - c_s) dt_s for s <= t (else 0), E[t] = e^(c_t), F[s] = e^(c_63 - c_s) dt_s; then a block of ssd_scan_kernel owns 16
+// value channels of one head and walks the chunks of its segment: wave w owns tokens 16 w .. 16 w + 15 of the outputs and
+// N / 4 columns of the state, which the waves exchange through LDS, one barrier per chunk.  Every operand is read from memory
+// in the register layout of its product -- K index 16 j + 4 g + e of step (j, e) for lane group g on both sides -- and the
+// loads of the next chunk are issued as soon as the registers are free.
+// Bound by the matrix cores (80 of these products per wave and chunk); 2 prompts of 2048, 64 heads of 64 x 128, 2 groups:
+// 188 us in all, with the factors made in the walk, four value blocks and four waves over, 287 us, token by token 858 us.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int SSD_L = 64;           // tokens per chunk
 constexpr int SSD_LEAST = 32;       // shorter segments go token by token: a chunk costs about as much as 20 steps
 
 __device__ __forceinline__ f32x4 mma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
-// grid (chunks, G, S): cb[(row t, group)][s] = C_t . B_s for the tokens s of t's chunk up to t's tile of 16
+// Scratch of a chunk -- segment s starts at chunk cu[s] / 64 + s --: per group C . B [64][64] (s up to t's tile of 16) and B in
+// operand order [N / 16][4][64 lanes][4 tokens]; per head M in operand order [10 tiles (w, j <= w)][64 lanes][4], E, F.
+constexpr int SSD_HEAD = 10 * 256 + 2 * SSD_L;
+__host__ __device__ inline long ssd_group_floats(int N) { return 64L * SSD_L + 64L * N; }
+__host__ __device__ inline long ssd_chunk_floats(int N, int G, int H) { return G * ssd_group_floats(N) + (long)H * SSD_HEAD; }
+
+// the last segment that starts at or before chunk ci
+__device__ __forceinline__ int ssd_segment(const int* cu, int S, int ci) {
+  int s = 0;
+  for (int lo = 0, hi = S; lo < hi;) {
+    const int mid = (lo + hi) >> 1;
+    if (cu[mid] / SSD_L + mid <= ci) {
+      s = mid;
+      lo = mid + 1;
+    } else {
+      hi = mid;
+    }
+  }
+  return s;
+}
+
+// grid (T / 64 + S, G)
 template <int NTW>
-__global__ void __launch_bounds__(256) ssd_scores_kernel(const float* __restrict__ u, int C, const int* __restrict__ cu,
-                                                         const int* __restrict__ slot, float* __restrict__ cb, int inner, int G) {
+__global__ void __launch_bounds__(256, 2) ssd_scores_kernel(const float* __restrict__ u, int C, const int* __restrict__ cu,
+                                                            const int* __restrict__ slot, float* __restrict__ ws, int S, int H,
+                                                            int inner, int G) {
   constexpr int N = 64 * NTW, NJ = N / 16;
-  const int s = blockIdx.z, grp = blockIdx.y, c0 = blockIdx.x * SSD_L;
-  const int r0 = cu[s], n = cu[s + 1] - r0;
-  if (slot[s] < 0 || n < SSD_LEAST || c0 >= n) return;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
+  const int ci = blockIdx.x, grp = blockIdx.y, s = ssd_segment(cu, S, ci);
+  const int r0 = cu[s], n = cu[s + 1] - r0, c0 = (ci - r0 / SSD_L - s) * SSD_L;
+  if (slot[s] < 0 || n < SSD_LEAST || c0 < 0 || c0 >= n) return;
+  float* cb = ws + ci * ssd_chunk_floats(N, G, H) + grp * ssd_group_floats(N);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, c = lane & 15;
   const float* ub = u + inner + grp * N + 4 * g;
   const float* cr = ub + (long)G * N + (long)(r0 + min(c0 + 16 * w + c, n - 1)) * C;
   f32x4 cv[NJ];
@@ -424,35 +449,87 @@ __global__ void __launch_bounds__(256) ssd_scores_kernel(const float* __restrict
       a1 = mma4(cv[j][3], bv[3], a1);
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int t = c0 + 16 * w + 4 * g + r;
-      if (t < n) cb[((long)(r0 + t) * G + grp) * SSD_L + 16 * st + c] = a0[r] + a1[r];
-    }
+    for (int r = 0; r < 4; ++r) cb[(16 * w + 4 * g + r) * SSD_L + 16 * st + c] = a0[r] + a1[r];
+  }
+  // B: wave w's tokens 16 w + 4 g + e, column 16 i + c
+  float* bt = cb + SSD_L * SSD_L;
+  const float* bp = u + inner + grp * N + c;
+#pragma unroll
+  for (int i = 0; i < NJ; ++i) {
+    f32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = bp[(long)(r0 + min(c0 + 16 * w + 4 * g + e, n - 1)) * C + 16 * i];
+    *reinterpret_cast<f32x4*>(bt + ((i * 4 + w) * 64 + lane) * 4) = v;
   }
 }
 
-// grid (P / 16, H, S)
-template <typename TD, int NTW>
-__global__ void __launch_bounds__(256, 2)
-ssd_scan_kernel(const float* __restrict__ u, int C, const TD* __restrict__ dt_raw, long sdt, const float* __restrict__ dt_bias,
-                const float* __restrict__ A_log, const float* __restrict__ Dp, float* __restrict__ state,
-                const float* __restrict__ cb, const int* __restrict__ cu, const int* __restrict__ slot,
+// grid (T / 64 + S, H)
+template <typename TD>
+__global__ void __launch_bounds__(256) ssd_decay_kernel(const TD* __restrict__ dt_raw, long sdt,
+                                                        const float* __restrict__ dt_bias, const float* __restrict__ A_log,
+                                                        const int* __restrict__ cu, const int* __restrict__ slot,
+                                                        float* __restrict__ ws, int S, int H, int G, int N) {
+  __shared__ double cums[4][SSD_L];      // a copy per wave
+  __shared__ float dts[4][SSD_L];
+  const int ci = blockIdx.x, h = blockIdx.y, s = ssd_segment(cu, S, ci);
+  const int r0 = cu[s], n = cu[s + 1] - r0, c0 = (ci - r0 / SSD_L - s) * SSD_L;
+  if (slot[s] < 0 || n < SSD_LEAST || c0 < 0 || c0 >= n) return;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, c = lane & 15;
+  const float A = -expf(A_log[h]);
+  const float raw = ldf(dt_raw + (long)(r0 + min(c0 + lane, n - 1)) * sdt + h);
+  const float dt = c0 + lane < n ? mx_softplus(raw + dt_bias[h]) : 0.f;
+  double a = (double)(A * dt);
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const double v = __shfl_up(a, o, 64);
+    if (lane >= o) a += v;
+  }
+  cums[w][lane] = a;
+  dts[w][lane] = dt;
+  __builtin_amdgcn_wave_barrier();
+  const double* cw = cums[w];
+  float* chunk = ws + ci * ssd_chunk_floats(N, G, H);
+  const float* cb = chunk + h / (H / G) * ssd_group_floats(N) + (16 * w + c) * SSD_L + 4 * g;
+  float* out = chunk + G * ssd_group_floats(N) + (long)h * SSD_HEAD;
+  const double ct = cw[16 * w + c];
+  for (int j = 0; j <= w; ++j) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(cb + 16 * j);
+    f32x4 m;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int t = 16 * j + 4 * g + e;
+      m[e] = t <= 16 * w + c ? v[e] * expf((float)(ct - cw[t])) * dts[w][t] : 0.f;
+    }
+    *reinterpret_cast<f32x4*>(out + ((w * (w + 1) / 2 + j) * 64 + lane) * 4) = m;
+  }
+  if (w == 0) {
+    out[2560 + lane] = expf((float)a);
+    out[2560 + SSD_L + lane] = dt * expf((float)(cw[SSD_L - 1] - a));
+  }
+}
+
+// grid (H, P / 16, S): the value blocks of a head on one chiplet, whose cache then holds the chunk's factors
+template <int NTW>
+__global__ void __launch_bounds__(256, NTW == 4 ? 1 : 2)
+ssd_scan_kernel(const float* __restrict__ u, int C, const float* __restrict__ Dp, float* __restrict__ state,
+                const float* __restrict__ ws, const int* __restrict__ cu, const int* __restrict__ slot,
                 const int* __restrict__ pos, float* __restrict__ y, int H, int P, int G) {
   constexpr int N = 64 * NTW, NJ = N / 16;
   __shared__ __attribute__((aligned(16))) float sbuf[2][16][N + 4];   // the state, [p][n]: rows 4 banks apart
-  __shared__ __attribute__((aligned(16))) double cums[4][SSD_L];       // a copy per wave
-  __shared__ __attribute__((aligned(16))) float dts[4][SSD_L];
-  const int s = blockIdx.z, h = blockIdx.y, p0 = blockIdx.x * 16;
+  const int s = blockIdx.z, h = blockIdx.x, p0 = blockIdx.y * 16;
   const int sl = slot[s], r0 = cu[s], n = cu[s + 1] - r0;
   if (sl < 0 || n < SSD_LEAST) return;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, c = lane & 15;
-  const int grp = h / (H / G), inner = H * P;
-  const float A = -expf(A_log[h]), bias = dt_bias[h], Dh = Dp[h];
+  const int grp = h / (H / G), inner = H * P, last = (n - 1) / SSD_L;
+  const float Dh = Dp[h];
+  const long step = ssd_chunk_floats(N, G, H);
+  const float* base = ws + (long)(r0 / SSD_L + s) * step;
+  const float* bbase = base + grp * ssd_group_floats(N) + SSD_L * SSD_L + (NTW * w * 256 + lane) * 4;
+  const float* hbase = base + G * ssd_group_floats(N) + (long)h * SSD_HEAD;
   const float* ux = u + (long)r0 * C + h * P + p0 + c;
-  const float* ub = u + (long)r0 * C + inner + grp * N + 16 * NTW * w + c;
   const float* uc = u + (long)r0 * C + inner + (G + grp) * N + 4 * g;
-  const float* cbr = cb + ((long)r0 * G + grp) * SSD_L + 4 * g;
   float* sp = state + (((long)sl * H + h) * P + p0 + 4 * g) * N + 16 * NTW * w + c;
+  float* yp = y + (long)(r0 + 16 * w + 4 * g) * inner + h * P + p0 + c;
 
   f32x4 st[NTW];                          // S[p0 + 4 g + r][16 (NTW w + i) + c]
 #pragma unroll
@@ -463,50 +540,65 @@ ssd_scan_kernel(const float* __restrict__ u, int C, const TD* __restrict__ dt_ra
       sbuf[0][4 * g + r][16 * (NTW * w + i) + c] = st[i][r];
     }
 
-  f32x4 cv[NJ], cbv[4], xv[4], bv[NTW][4];
-  float raw;
-  auto load_c = [&](int c0) {
-    const float* p = uc + (long)min(c0 + 16 * w + c, n - 1) * C;
+  f32x4 cv[NJ], mv[4], xv[4], bv[NTW][4], fv[4], ev;
+  float keep;
+  auto load_c = [&](int k) {              // k: the chunk (behind the end: the last one again)
+    const float* p = uc + (long)min(k * SSD_L + 16 * w + c, n - 1) * C;
 #pragma unroll
     for (int j = 0; j < NJ; ++j) cv[j] = *reinterpret_cast<const f32x4*>(p + 16 * j);
   };
-  auto load_cb = [&](int c0) {
-    const float* p = cbr + (long)min(c0 + 16 * w + c, n - 1) * G * SSD_L;
+  auto load_m = [&](int k) {
+    const float* p = hbase + min(k, last) * step;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      if (j <= w) cbv[j] = *reinterpret_cast<const f32x4*>(p + 16 * j);
+      if (j <= w) mv[j] = *reinterpret_cast<const f32x4*>(p + ((w * (w + 1) / 2 + j) * 64 + lane) * 4);
+    ev = *reinterpret_cast<const f32x4*>(p + 2560 + 16 * w + 4 * g);
   };
-  auto load_xb = [&](int c0) {
+  auto load_b = [&](int k) {
+    const float* p = bbase + min(k, last) * step;
+    const float* f = hbase + min(k, last) * step + 2560;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 4; ++j) {
+      fv[j] = *reinterpret_cast<const f32x4*>(f + SSD_L + 16 * j + 4 * g);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const long o = (long)min(c0 + 16 * j + 4 * g + e, n - 1) * C;
-        xv[j][e] = ux[o];
-#pragma unroll
-        for (int i = 0; i < NTW; ++i) bv[i][j][e] = ub[o + 16 * i];
-      }
-  };
-  auto load_dt = [&](int c0) { raw = ldf(dt_raw + (long)(r0 + min(c0 + lane, n - 1)) * sdt + h); };
-  load_dt(0);
-  load_c(0);
-  load_cb(0);
-  load_xb(0);
-  for (int c0 = 0, b = 0; c0 < n; c0 += SSD_L, b ^= 1) {
-    {                                     // this chunk's steps and running log decays, token = lane
-      const float dt = c0 + lane < n ? mx_softplus(raw + bias) : 0.f;
-      double a = (double)(A * dt);
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const double v = __shfl_up(a, o, 64);
-        if (lane >= o) a += v;
-      }
-      cums[w][lane] = a;
-      dts[w][lane] = dt;
+      for (int i = 0; i < NTW; ++i) bv[i][j] = *reinterpret_cast<const f32x4*>(p + (i * 4 + j) * 256);
     }
-    load_dt(c0 + SSD_L);
+    keep = f[SSD_L - 1];
+  };
+  auto load_x = [&](int k) {
+    const int t0 = k * SSD_L + 4 * g;
+    if (k < last) {
+      const float* p = ux + (long)t0 * C;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) xv[j][e] = p[(16 * j + e) * C];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) xv[j][e] = ux[(long)min(t0 + 16 * j + e, n - 1) * C];
+    }
+  };
+  load_c(0);
+  load_m(0);
+  load_x(0);
+  load_b(0);
+  for (int k = 0; k <= last; ++k) {
+    const int b = k & 1, left = n - k * SSD_L;
+    // a value that is not finite spoils the tokens from its own on and its row of the state, nothing before
+    int bad = SSD_L;
+    const f32x4 xt = w == 0 ? xv[0] : (w == 1 ? xv[1] : (w == 2 ? xv[2] : xv[3]));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (left < SSD_L) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) xv[j][e] = 16 * j + 4 * g + e < left ? xv[j][e] : 0.f;
+      }
+      const int at = mx_drop_nonfinite(xv[j], g);
+      bad = min(bad, at < 16 ? 16 * j + at : SSD_L);
+    }
     __syncthreads();                      // the state of the last chunk is in sbuf[b]
-    const double* cw = cums[w];
     // what the state before the chunk gives
     f32x4 y0 = {0.f, 0.f, 0.f, 0.f}, y1 = y0;
 #pragma unroll
@@ -517,48 +609,48 @@ ssd_scan_kernel(const float* __restrict__ u, int C, const TD* __restrict__ dt_ra
       y0 = mma4(cv[j][2], sv[2], y0);
       y1 = mma4(cv[j][3], sv[3], y1);
     }
-    load_c(c0 + SSD_L);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) y0[r] = (y0[r] + y1[r]) * expf((float)cw[16 * w + 4 * g + r]);
+    load_c(k + 1);
+    y0 = (y0 + y1) * ev;
     // the chunk's own tokens up to this one
-    const double ct = cw[16 * w + c];
     y1 = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       if (j > w) continue;
-      f32x4 m;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int t = 16 * j + 4 * g + e;
-        m[e] = t <= 16 * w + c ? cbv[j][e] * expf((float)(ct - cw[t])) * dts[w][t] : 0.f;
-      }
-      y0 = mma4(m[0], xv[j][0], y0);
-      y1 = mma4(m[1], xv[j][1], y1);
-      y0 = mma4(m[2], xv[j][2], y0);
-      y1 = mma4(m[3], xv[j][3], y1);
+      y0 = mma4(mv[j][0], xv[j][0], y0);
+      y1 = mma4(mv[j][1], xv[j][1], y1);
+      y0 = mma4(mv[j][2], xv[j][2], y0);
+      y1 = mma4(mv[j][3], xv[j][3], y1);
     }
-    load_cb(c0 + SSD_L);
-    const f32x4 xt = w == 0 ? xv[0] : (w == 1 ? xv[1] : (w == 2 ? xv[2] : xv[3]));
+    load_m(k + 1);
+    y0 += y1;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int t = c0 + 16 * w + 4 * g + r;
-      if (t < n) y[(long)(r0 + t) * inner + h * P + p0 + c] = y0[r] + y1[r] + Dh * xt[r];
+      const int t = 16 * w + 4 * g + r;
+      y0[r] = t >= bad ? NAN : y0[r] + Dh * xt[r];
+      if (t < left) yp[(long)r * inner] = y0[r];
     }
+    yp += (long)SSD_L * inner;
     // the state after the chunk
-    const double cl = cw[SSD_L - 1];
-    const float keep = expf((float)cl);
 #pragma unroll
     for (int i = 0; i < NTW; ++i) st[i] *= keep;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 4; ++j) {
+      const f32x4 a = xv[j] * fv[j];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int t = 16 * j + 4 * g + e;
-        const float a = xv[j][e] * (dts[w][t] * expf((float)(cl - cw[t])));
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int i = 0; i < NTW; ++i) st[i] = mma4(a, bv[i][j][e], st[i]);
+        for (int i = 0; i < NTW; ++i) st[i] = mma4(a[e], bv[i][j][e], st[i]);
+    }
+    load_x(k + 1);
+    load_b(k + 1);
+    if (__any(bad < SSD_L)) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const bool spoilt = __shfl(bad, 4 * g + r, 64) < SSD_L;
+#pragma unroll
+        for (int i = 0; i < NTW; ++i) st[i][r] = spoilt ? NAN : st[i][r];
       }
-    load_xb(c0 + SSD_L);
+    }
 #pragma unroll
     for (int i = 0; i < NTW; ++i)
 #pragma unroll
@@ -603,26 +695,27 @@ MX_API int mx_conv_silu(const void* in, long si, int dt, const float* w, const f
 }
 
 // u f32 [rows, C = H*P + 2*G*N]; dt_raw [rows, H] slice (stride sdt, type dt_code); state f32
-// [slots, H, P, N]; y f32 [rows, H*P]; max_len: the longest segment; cb: f32 [rows, G, 64] scratch of the chunked form,
-// or null (token by token).
+// [slots, H, P, N]; y f32 [rows, H*P]; max_len: the longest segment; ws: f32 scratch of
+// (rows / 64 + S) * ssd_chunk_floats(N, G, H) values for the chunked form, or null (token by token).
 // The chunked form takes states of 64, 128 or 256 columns, value sizes in whole tiles of 16 and 16-byte rows.
 MX_API int mx_ssm_scan(const float* u, int C, const void* dt_raw, long sdt, int dt_code, const float* dt_bias,
                        const float* A_log, const float* D, float* state, const int* cu, const int* slot,
                        const int* pos, float* y, int S, int max_len, int H, int P, int N, int G, int cu_rows_bound,
-                       float* cb, hipStream_t st) {
+                       float* ws, hipStream_t st) {
   if (S <= 0) return 0;
   if (N > SCAN_NS * 16 || G < 1 || H % G) return (int)hipErrorInvalidValue;
   if ((long)cu_rows_bound * C >= (1L << 31)) return (int)hipErrorInvalidValue;
   const bool vecu = (N % 4 == 0) && ((H * P) % 4 == 0) && (C % 4 == 0);
-  const bool chunked = cb != nullptr && max_len >= SSD_LEAST && (N == 64 || N == 128 || N == 256) && P % 16 == 0 && vecu &&
-                       ((size_t)u | (size_t)cb) % 16 == 0 && H <= 65535 && S <= 65535;
+  const bool chunked = ws != nullptr && max_len >= SSD_LEAST && (N == 64 || N == 128 || N == 256) && P % 16 == 0 && vecu &&
+                       ((size_t)u | (size_t)ws) % 16 == 0 && H <= 65535 && S <= 65535;
   if (chunked) {
-    const dim3 gs((max_len + SSD_L - 1) / SSD_L, G, S), g2(P / 16, H, S);
+    const int chunks = cu_rows_bound / SSD_L + S;
 #define SSD(NTW)                                                                                                 \
   do {                                                                                                           \
-    ssd_scores_kernel<NTW><<<gs, 256, 0, st>>>(u, C, cu, slot, cb, H * P, G);                                    \
-    MX_DISPATCH(dt_code, TT, ssd_scan_kernel<TT, NTW><<<g2, 256, 0, st>>>(                                       \
-        u, C, (const TT*)dt_raw, sdt, dt_bias, A_log, D, state, cb, cu, slot, pos, y, H, P, G));                 \
+    ssd_scores_kernel<NTW><<<dim3(chunks, G), 256, 0, st>>>(u, C, cu, slot, ws, S, H, H * P, G);                 \
+    MX_DISPATCH(dt_code, TT, ssd_decay_kernel<TT><<<dim3(chunks, H), 256, 0, st>>>(                              \
+        (const TT*)dt_raw, sdt, dt_bias, A_log, cu, slot, ws, S, H, G, N));                                      \
+    ssd_scan_kernel<NTW><<<dim3(H, P / 16, S), 256, 0, st>>>(u, C, D, state, ws, cu, slot, pos, y, H, P, G);     \
   } while (0)
     if (N == 64) SSD(1);
     else if (N == 128) SSD(2);

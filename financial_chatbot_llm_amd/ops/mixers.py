@@ -394,10 +394,12 @@ def ssm_scan(u: torch.Tensor, dt_raw: torch.Tensor, dt_bias: torch.Tensor, A_log
     if N.use_native(u):
         y = torch.empty((T, H * P), dtype=torch.float32, device=u.device)
         max_len = max_len or T
-        cb = torch.empty((T, G, 64), dtype=torch.float32, device=u.device) if max_len > 1 else None
+        ws = None
+        if max_len >= 32 and Ns in (64, 128, 256):          # the chunked form's factors (ssd_chunk_floats of the kernels)
+            ws = torch.empty((T // 64 + S, G * 64 * (64 + Ns) + H * 2688), dtype=torch.float32, device=u.device)
         N.mcall("mx_ssm_scan", N.ptr(u), C, N.ptr(_rows(dt_raw)), dt_raw.stride(0), _dt(dt_raw), N.ptr(dt_bias),
                 N.ptr(A_log), N.ptr(D), N.ptr(state), N.ptr(cu), N.ptr(slot), N.ptr(pos), N.ptr(y), S, int(max_len), H, P, Ns, G,
-                T, N.ptr(cb), N.stream())
+                T, N.ptr(ws), N.stream())
         return y
     y = torch.zeros((T, H * P), dtype=torch.float32)
     cul, sll, pl = cu.tolist(), slot.tolist(), pos.tolist()

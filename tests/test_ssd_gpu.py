@@ -53,3 +53,25 @@ def test_chunked_scan(dtype, H, P, N, G, decay, lens):
             assert k in used or torch.equal(gs[k], state[k].double())
     # f32 sums of up to N + 64 products and one exponential per pair of tokens
     assert off["chunks"] < 2e-6 and off["chunks"] < 2.0 * off["tokens"] + 3e-7, off
+
+
+def test_not_finite():
+    """An infinite input reaches no earlier token and no other channel."""
+    from financial_chatbot_llm_amd.ops import mixers as mx
+    H, P, N, G, T = 2, 32, 64, 1, 150
+    g = torch.Generator().manual_seed(1)
+    u, dtr = torch.randn(T, H * P + 2 * G * N, generator=g), torch.randn(T, H, generator=g)
+    bias, A_log, D = torch.zeros(H), torch.zeros(H), torch.ones(H)
+    cu, slot, pos = torch.tensor([0, T]), torch.tensor([0]), torch.arange(T)
+    dev = lambda t: t.cuda() if t.is_floating_point() else t.to("cuda", torch.int32)  # noqa: E731
+    out = []
+    for bad in (None, 85):
+        v, st = u.clone(), torch.zeros(1, H, P, N).cuda()
+        if bad is not None:
+            v[bad, 5] = float("inf")
+        y = mx.ssm_scan(*(dev(t) for t in (v, dtr, bias, A_log, D)), st, dev(cu), dev(slot), dev(pos), H, P, N, G, T)
+        out.append((y.cpu(), st.cpu()))
+    (y, st), (z, sz) = out
+    assert torch.equal(y[:85], z[:85]) and not torch.isfinite(z[85:, 5]).any() and not torch.isfinite(sz[0, 0, 5]).any()
+    y[:, 5], z[:, 5], st[0, 0, 5], sz[0, 0, 5] = 0, 0, 0, 0
+    assert torch.equal(y, z) and torch.equal(st, sz)
