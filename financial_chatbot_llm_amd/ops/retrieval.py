@@ -1,7 +1,8 @@
 """K15: filtered exact top-k over an HBM-resident corpus (user_id == u AND date >= t)."""
 from __future__ import annotations
 
-from typing import Tuple
+import threading
+from typing import Dict, Tuple
 
 import torch
 
@@ -30,21 +31,21 @@ def filtered_topk_ref(corpus, user_codes, dates, queries, q_user, q_floor, ks, k
     return ids, scores, counts
 
 
-class _Workspace:
-    def __init__(self):
-        self.key = None
-
-    def get(self, nq: int, cap: int, device):
-        key = (nq, cap, str(device))
-        if self.key != key:
-            self.counts = torch.empty((nq,), dtype=torch.int32, device=device)
-            self.cand = torch.empty((nq, cap), dtype=torch.int32, device=device)
-            self.scores = torch.empty((nq, cap), dtype=torch.float32, device=device)
-            self.key = key
-        return self.counts, self.cand, self.scores
+# candidate lists, one set per (device, stream, thread): the calls of a thread on a stream run in order.  At most eight sets;
+# the kernels leave counts at zero.
+_WS: Dict[Tuple[int, int, int], Tuple[Tuple[int, int], Tuple[torch.Tensor, torch.Tensor, torch.Tensor]]] = {}
 
 
-_WS = _Workspace()
+def _workspace(nq: int, cap: int, device: torch.device) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    key = (device.index or 0, N.stream(), threading.get_ident())
+    ent = _WS.get(key)
+    if ent is None or ent[0] != (nq, cap):
+        if len(_WS) >= 8:
+            _WS.clear()
+        ent = _WS[key] = ((nq, cap), (torch.zeros((nq, 32), dtype=torch.int32, device=device),
+                                      torch.empty((nq, cap), dtype=torch.int32, device=device),
+                                      torch.empty((nq, cap), dtype=torch.float32, device=device)))
+    return ent[1]
 
 
 def filtered_topk(corpus: torch.Tensor, user_codes: torch.Tensor, dates: torch.Tensor, queries: torch.Tensor,
@@ -60,21 +61,23 @@ def filtered_topk(corpus: torch.Tensor, user_codes: torch.Tensor, dates: torch.T
                                ks[i:i + 64], kmax, cap) for i in range(0, nq, 64)]
         return tuple(torch.cat(x) for x in zip(*parts))
     cap = max(SORT_CAP, min(cap, corpus.shape[0]))
-    counts, cand, scores = _WS.get(nq, cap, corpus.device)
-    out_ids = torch.full((nq, kmax), -1, dtype=torch.int32, device=corpus.device)
-    out_scores = torch.zeros((nq, kmax), dtype=torch.float32, device=corpus.device)
+    counts, cand, scores = _workspace(nq, cap, corpus.device)
+    out_ids = torch.empty((nq, kmax), dtype=torch.int32, device=corpus.device)
+    out_scores = torch.empty((nq, kmax), dtype=torch.float32, device=corpus.device)
     out_count = torch.empty((nq,), dtype=torch.int32, device=corpus.device)
+    oc = torch.empty((nq,), dtype=torch.int32, pin_memory=True)      # written by the kernel itself
     queries = queries.to(torch.bfloat16).contiguous()
     # converted inputs bound to names: as N.ptr(x.to(...)) temporaries they would be freed before
     # the launch and the next conversion could reuse (overwrite) their memory on the stream
     qu, qf, kk = q_user.to(torch.int32).contiguous(), q_floor.to(torch.int64).contiguous(), ks.to(torch.int32).contiguous()
     N.call("penny_filtered_topk", N.ptr(corpus), N.ptr(user_codes), N.ptr(dates), corpus.shape[0], D,
            N.ptr(queries), N.ptr(qu), N.ptr(qf), N.ptr(kk), nq, kmax, N.ptr(counts), N.ptr(cand), N.ptr(scores), cap,
-           N.ptr(out_ids), N.ptr(out_scores), N.ptr(out_count), N.stream())
-    oc = out_count.cpu()
-    big = (oc < 0).nonzero().flatten().tolist()
-    for i in big:  # > SORT_CAP candidates: finish on device with torch.topk
-        total = -int(oc[i])
+           N.ptr(out_ids), N.ptr(out_scores), N.ptr(out_count), N.ptr(oc), N.stream())
+    torch.cuda.current_stream(corpus.device).synchronize()
+    for i, c in enumerate(oc.tolist()):  # > SORT_CAP candidates: finish on device with torch.topk
+        if c >= 0:
+            continue
+        total = -c
         k = min(int(ks[i]), total, kmax)
         if total <= cap:
             s, j = torch.topk(scores[i, :total], k)
@@ -84,5 +87,5 @@ def filtered_topk(corpus: torch.Tensor, user_codes: torch.Tensor, dates: torch.T
             full = (corpus.float() @ queries[i].float()).masked_fill(~mask, float("-inf"))
             s, j = torch.topk(full, k)
             out_ids[i, :k], out_scores[i, :k] = j.to(torch.int32), s
-        oc[i] = k
-    return out_ids, out_scores, oc.to(corpus.device)
+        out_count[i] = k
+    return out_ids, out_scores, out_count

@@ -1,0 +1,46 @@
+"""Filtered top-k: candidate counts around the ranking's and the sort's limits, several calls through one workspace, ties and
+scores that are not numbers, corpus sizes around a block's share."""
+import pytest
+import torch
+
+from financial_chatbot_llm_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def corpus(sizes, N, D, seed):
+    """N rows; user u + 1 owns sizes[u] of them, the rest belong to user 0."""
+    g = torch.Generator().manual_seed(seed)
+    users = torch.zeros(N, dtype=torch.int32)
+    perm, o = torch.randperm(N, generator=g), 0
+    for u, n in enumerate(sizes):
+        users[perm[o:o + n]] = u + 1
+        o += n
+    x = torch.randint(-3, 4, (N, D), generator=g).to(torch.bfloat16)      # whole numbers: exact sums, many ties
+    dates = torch.randint(0, 1000, (N,), generator=g)
+    q = torch.randint(-3, 4, (len(sizes) + 1, D), generator=g).to(torch.bfloat16)
+    return x, users, dates, q
+
+
+@pytest.mark.parametrize("sizes,N,D", [([0, 1, 2], 3, 8), ([5, 255, 256, 257, 300], 1100, 64), ([1024, 1, 700, 8192], 12000, 64),
+                                       ([9000], 9001, 8), ([100] * 40, 4097, 768)])
+def test_sizes(sizes, N, D):
+    x, users, dates, q = corpus(sizes, N, D, len(sizes))
+    nq, kmax = len(sizes) + 1, 300
+    who = torch.tensor([u + 1 for u in range(len(sizes))] + [len(sizes) + 5], dtype=torch.int32)
+    dev = [t.cuda() for t in (x, users, dates, q, who)]
+    for since, k in ((0, kmax), (500, 10), (0, 1)):
+        floor, ks = torch.full((nq,), since, dtype=torch.int64), torch.full((nq,), k, dtype=torch.int32)
+        got = ops.filtered_topk(*dev, floor.cuda(), ks.cuda(), kmax)
+        want = ops.filtered_topk(x, users, dates, q, who, floor, ks, kmax)
+        assert torch.equal(got[2].cpu(), want[2]) and torch.equal(got[1].cpu(), want[1])
+        small = torch.tensor([n <= 8192 for n in sizes] + [True])          # the library's top-k breaks ties its own way
+        assert torch.equal(got[0].cpu()[small], want[0][small])
+
+
+def test_not_a_number():
+    x, users, dates, q = corpus([200], 300, 64, 7)
+    x[users.nonzero().flatten()[:3]] = float("nan")
+    ids, _, count = ops.filtered_topk(x.cuda(), users.cuda(), dates.cuda(), q[:1].cuda(), torch.tensor([1]).cuda(),
+                                      torch.tensor([0]).cuda(), torch.tensor([200]).cuda(), 200)
+    assert int(count[0]) == 200 and set(ids[0].tolist()) == set(users.nonzero().flatten().tolist())
