@@ -695,7 +695,7 @@ MX_API int mx_conv_silu(const void* in, long si, int dt, const float* w, const f
 }
 
 // u f32 [rows, C = H*P + 2*G*N]; dt_raw [rows, H] slice (stride sdt, type dt_code); state f32
-// [slots, H, P, N]; y f32 [rows, H*P]; max_len: the longest segment; ws: f32 scratch of
+// [slots, H, P, N]; y f32 [rows, H*P]; max_len: no segment is longer; ws: f32 scratch of
 // (rows / 64 + S) * ssd_chunk_floats(N, G, H) values for the chunked form, or null (token by token).
 // The chunked form takes states of 64, 128 or 256 columns, value sizes in whole tiles of 16 and 16-byte rows.
 MX_API int mx_ssm_scan(const float* u, int C, const void* dt_raw, long sdt, int dt_code, const float* dt_bias,
@@ -722,7 +722,7 @@ MX_API int mx_ssm_scan(const float* u, int C, const void* dt_raw, long sdt, int 
     else SSD(4);
 #undef SSD
     const int rc = (int)hipGetLastError();
-    if (rc || S == 1) return rc;                         // one segment, and it was a long one
+    if (rc) return rc;                                   // (max_len is a bound: every segment may still be a short one)
   }
   const int below = chunked ? SSD_LEAST : 0x7fffffff;
   dim3 grid((P + SCAN_PT - 1) / SCAN_PT, H, S);

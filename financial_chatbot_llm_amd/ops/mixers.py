@@ -383,8 +383,9 @@ def conv_silu(inp: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], 
 def ssm_scan(u: torch.Tensor, dt_raw: torch.Tensor, dt_bias: torch.Tensor, A_log: torch.Tensor, D: torch.Tensor,
              state: torch.Tensor, cu: torch.Tensor, slot: torch.Tensor, pos: torch.Tensor, heads: int, vdim: int,
              nstate: int, groups: int, max_len: int = 0) -> torch.Tensor:
-    """Mamba-2 recurrence in f32 (``max_len``: the longest segment when known; the kernels take long ones in chunks).  ``u`` f32 [T, H*P + 2*G*N] = [x | B | C] (after the
-    convolution), ``dt_raw`` [T, H]; per head h of group h // (H / G):
+    """Mamba-2 recurrence in f32 (``max_len``: no segment is longer, all rows when left out; the kernels take long segments
+    in chunks).  ``u`` f32 [T, H*P + 2*G*N] = [x | B | C] (after the convolution), ``dt_raw`` [T, H]; per head h of group
+    h // (H / G):
     dt = softplus(dt_raw + dt_bias), S <- exp(-exp(A_log) dt) S + dt x B^T, y = S C + D x.
     ``state`` f32 [slots, H, P, N] is read (unless the segment starts at position 0) and replaced."""
     T, C = u.shape

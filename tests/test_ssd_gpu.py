@@ -75,3 +75,22 @@ def test_not_finite():
     assert torch.equal(y[:85], z[:85]) and not torch.isfinite(z[85:, 5]).any() and not torch.isfinite(sz[0, 0, 5]).any()
     y[:, 5], z[:, 5], st[0, 0, 5], sz[0, 0, 5] = 0, 0, 0, 0
     assert torch.equal(y, z) and torch.equal(st, sz)
+
+
+@pytest.mark.parametrize("n", [0, 1, 20, 31, 40])
+@pytest.mark.parametrize("most", [[], [40]])
+def test_one_segment_in_a_longer_buffer(n, most):
+    """The rows behind the last segment belong to nobody: ``max_len`` left out, or given as the buffer's rows, is a bound."""
+    from financial_chatbot_llm_amd.ops import mixers as mx
+    H, P, N, G, T = 2, 16, 64, 1, 40
+    g = torch.Generator().manual_seed(n)
+    args = [torch.randn(T, H * P + 2 * G * N, generator=g), torch.randn(T, H, generator=g), torch.randn(H, generator=g) - 2.0,
+            torch.zeros(H), torch.ones(H)]
+    state = torch.randn(3, H, P, N, generator=g)
+    meta = [torch.tensor([0, n]), torch.tensor([2]), torch.arange(T) + 9]
+    dev = lambda t: t.cuda() if t.is_floating_point() else t.to("cuda", torch.int32)  # noqa: E731
+    got_state, want_state = state.cuda(), state.clone()
+    got = mx.ssm_scan(*map(dev, args), got_state, *map(dev, meta), H, P, N, G, *most)
+    want = mx.ssm_scan(*args, want_state, *meta, H, P, N, G)
+    # f32 sums of up to N + 40 products on both sides
+    assert torch.allclose(got[:n].cpu(), want[:n], rtol=1e-5, atol=1e-4) and torch.allclose(got_state.cpu(), want_state, rtol=1e-5, atol=1e-4)
