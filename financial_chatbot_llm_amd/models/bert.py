@@ -90,7 +90,7 @@ class BertEncoder:
                 self.H % 32 == 0 and F_ % 32 == 0 and os.environ.get("PENNY_PREFILL_GEMM", "1") == "1"):
             return False
         w = [self.w[n] for n in self.layer_names]
-        if not all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.device == x.device for t in w) or \
+        if not all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.device == x.device and t.data_ptr() % 16 == 0 for t in w) or \
                 [t.shape for t in w] != self.layer_shapes:
             return False
         table = (ctypes.c_void_p * len(w))(*[t.data_ptr() for t in w])

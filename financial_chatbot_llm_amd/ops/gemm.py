@@ -762,8 +762,17 @@ BGE_SMALL_MAX_M = 768
 
 
 def small_bias_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
-    return (N.use_native(x) and x.dtype == w.dtype == torch.bfloat16 and w.shape[0] % 16 == 0 and w.shape[1] % 32 == 0
-            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.is_contiguous())
+    """Whether the small-batch kernel takes these operands; other types, shapes and views off its alignment are left to the
+    paths behind it (which also refuse shapes that do not fit)."""
+    return (N.use_native(x) and x.dtype == w.dtype == torch.bfloat16 and x.device == w.device and w.shape[0] % 16 == 0
+            and w.shape[1] % 32 == 0 and w.shape[1] == x.shape[1] and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and w.is_contiguous() and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+
+
+def _bias_row(b: Optional[torch.Tensor], w: torch.Tensor) -> bool:
+    """Whether ``b`` is a bias the small-batch kernel reads."""
+    return (b is not None and b.dtype == torch.bfloat16 and b.device == w.device and b.shape == w.shape[:1]
+            and b.is_contiguous() and b.data_ptr() % 8 == 0)
 
 
 def linear_bias(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, gelu: bool = False) -> torch.Tensor:
@@ -774,7 +783,7 @@ def linear_bias(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, gelu: bool = 
     M, K = x.shape
     N_ = w.shape[0]
     mode = os.environ.get("PENNY_PREFILL_GEMM", "1")
-    if mode == "1" and M <= BGE_SMALL_MAX_M and small_bias_ok(x, w):
+    if mode == "1" and M <= BGE_SMALL_MAX_M and small_bias_ok(x, w) and _bias_row(b, w):
         y = torch.empty((M, N_), dtype=x.dtype, device=x.device)
         N.call("penny_gemm_bias_small", N.ptr(x), x.stride(0), N.ptr(w), K, N.ptr(y), N_, N.ptr(b), M, N_, int(gelu),
                N.stream())

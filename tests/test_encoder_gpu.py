@@ -50,6 +50,33 @@ def test_small_batch_projection(M, N, K, gelu):
     assert float((got - want).norm() / want.norm()) < 4e-3
 
 
+def test_projections_the_small_kernel_does_not_take():
+    """What the library product takes is answered by it, what it refuses is refused."""
+    from financial_chatbot_llm_amd.ops import gemm
+    g = torch.Generator(device="cuda").manual_seed(5)
+    M, N, K = 9, 48, 96
+    flat = torch.randn(N * K + M * K + N + 8, generator=g, device="cuda").to(torch.bfloat16)
+    x, w, b = flat[:M * K].view(M, K), flat[M * K:M * K + N * K].view(N, K), flat[-N - 8:-8]
+    off = flat[1:1 + N * K].view(N, K)                                        # two bytes off the kernel's 16
+    for args in ((x, w, None), (x, off, b), (x, w, flat[3:3 + N]), (x, w, flat[:2 * N:2]), (flat[1:1 + M * K].view(M, K), w, b)):
+        want = args[0].float() @ args[1].float().T + (args[2].float() if args[2] is not None else 0.0)
+        assert float((gemm.linear_bias(*args).float() - want).norm() / want.norm()) < 4e-3      # one rounding to bf16
+    for args in ((x, w, b.float()), (x[:, :64], w, b), (x, w, b[:16]), (x, w.float(), b)):
+        with pytest.raises(RuntimeError):
+            gemm.linear_bias(*args)
+
+
+def test_a_layer_weight_off_the_alignment():
+    from financial_chatbot_llm_amd.models.bert import BertEncoder
+    from financial_chatbot_llm_amd.models.configs import get_model_config
+    m = BertEncoder.build(get_model_config("bert-tiny"), "cuda")
+    want = m.encode([[5, 6, 7]])
+    for name in ("layers.0.o_b", "layers.1.ln1_g"):                          # slices of a flat buffer
+        t = m.w[name]
+        m.w[name] = torch.cat([t.new_zeros(4), t])[4:]
+    assert torch.allclose(m.encode([[5, 6, 7]]), want, atol=2e-2)            # other kernels, bf16 activations
+
+
 def test_gelu_over_all_bf16():
     from financial_chatbot_llm_amd import ops
     bits = torch.arange(1 << 16, dtype=torch.int32)
