@@ -2,7 +2,7 @@
 from __future__ import annotations
 
 import threading
-from typing import Dict, Tuple
+from typing import List, Tuple
 
 import torch
 
@@ -31,21 +31,31 @@ def filtered_topk_ref(corpus, user_codes, dates, queries, q_user, q_floor, ks, k
     return ids, scores, counts
 
 
-# candidate lists, one set per (device, stream, thread): the calls of a thread on a stream run in order.  At most eight sets;
-# the kernels leave counts at zero.
-_WS: Dict[Tuple[int, int, int], Tuple[Tuple[int, int], Tuple[torch.Tensor, torch.Tensor, torch.Tensor]]] = {}
+# Candidate lists that no call holds: (device, stream, set), at most eight, the longest unused dropped first.  A set serves the
+# calls of one stream, whatever their sizes; a call takes one (or makes it), so two threads never share it, and hands it back
+# when its kernels have left the counters at zero again -- a call that fails does not.
+_Set = Tuple[torch.Tensor, torch.Tensor, torch.Tensor]
+_FREE: List[Tuple[int, int, _Set]] = []
+_LOCK = threading.Lock()
+_KEEP = 8
 
 
-def _workspace(nq: int, cap: int, device: torch.device) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    key = (device.index or 0, N.stream(), threading.get_ident())
-    ent = _WS.get(key)
-    if ent is None or ent[0] != (nq, cap):
-        if len(_WS) >= 8:
-            _WS.clear()
-        ent = _WS[key] = ((nq, cap), (torch.zeros((nq, 32), dtype=torch.int32, device=device),
-                                      torch.empty((nq, cap), dtype=torch.int32, device=device),
-                                      torch.empty((nq, cap), dtype=torch.float32, device=device)))
-    return ent[1]
+def _take(n: int, device: torch.device, stream: int) -> _Set:
+    """Counters [64, 32] of zeros, rows and scores of at least ``n`` candidates."""
+    with _LOCK:
+        for i, (d, s, ws) in enumerate(_FREE):
+            if d == device.index and s == stream and ws[1].numel() >= n:
+                return _FREE.pop(i)[2]
+    n = 1 << (n - 1).bit_length()          # few sizes: a smaller call fits behind a larger one
+    return (torch.zeros((64, 32), dtype=torch.int32, device=device), torch.empty(n, dtype=torch.int32, device=device),
+            torch.empty(n, dtype=torch.float32, device=device))
+
+
+def _hand_back(ws: _Set, device: torch.device, stream: int) -> None:
+    with _LOCK:
+        # smaller sets of the stream that nobody holds have no use beside this one
+        _FREE[:] = [f for f in _FREE if f[:2] != (device.index, stream) or f[2][1].numel() >= ws[1].numel()][1 - _KEEP:]
+        _FREE.append((device.index, stream, ws))
 
 
 def filtered_topk(corpus: torch.Tensor, user_codes: torch.Tensor, dates: torch.Tensor, queries: torch.Tensor,
@@ -61,7 +71,9 @@ def filtered_topk(corpus: torch.Tensor, user_codes: torch.Tensor, dates: torch.T
                                ks[i:i + 64], kmax, cap) for i in range(0, nq, 64)]
         return tuple(torch.cat(x) for x in zip(*parts))
     cap = max(SORT_CAP, min(cap, corpus.shape[0]))
-    counts, cand, scores = _workspace(nq, cap, corpus.device)
+    stream = N.stream()
+    ws = _take(nq * cap, corpus.device, stream)
+    counts, cand, scores = ws                                        # the lists: nq rows of cap entries
     out_ids = torch.empty((nq, kmax), dtype=torch.int32, device=corpus.device)
     out_scores = torch.empty((nq, kmax), dtype=torch.float32, device=corpus.device)
     out_count = torch.empty((nq,), dtype=torch.int32, device=corpus.device)
@@ -72,7 +84,7 @@ def filtered_topk(corpus: torch.Tensor, user_codes: torch.Tensor, dates: torch.T
     qu, qf, kk = q_user.to(torch.int32).contiguous(), q_floor.to(torch.int64).contiguous(), ks.to(torch.int32).contiguous()
     N.call("penny_filtered_topk", N.ptr(corpus), N.ptr(user_codes), N.ptr(dates), corpus.shape[0], D,
            N.ptr(queries), N.ptr(qu), N.ptr(qf), N.ptr(kk), nq, kmax, N.ptr(counts), N.ptr(cand), N.ptr(scores), cap,
-           N.ptr(out_ids), N.ptr(out_scores), N.ptr(out_count), N.ptr(oc), N.stream())
+           N.ptr(out_ids), N.ptr(out_scores), N.ptr(out_count), N.ptr(oc), stream)
     torch.cuda.current_stream(corpus.device).synchronize()
     for i, c in enumerate(oc.tolist()):  # > SORT_CAP candidates: finish on device with torch.topk
         if c >= 0:
@@ -80,12 +92,13 @@ def filtered_topk(corpus: torch.Tensor, user_codes: torch.Tensor, dates: torch.T
         total = -c
         k = min(int(ks[i]), total, kmax)
         if total <= cap:
-            s, j = torch.topk(scores[i, :total], k)
-            out_ids[i, :k], out_scores[i, :k] = cand[i, :total][j], s
+            s, j = torch.topk(scores[i * cap:i * cap + total], k)
+            out_ids[i, :k], out_scores[i, :k] = cand[i * cap:i * cap + total][j], s
         else:
             mask = (user_codes == q_user[i]) & (dates >= q_floor[i])
             full = (corpus.float() @ queries[i].float()).masked_fill(~mask, float("-inf"))
             s, j = torch.topk(full, k)
             out_ids[i, :k], out_scores[i, :k] = j.to(torch.int32), s
         out_count[i] = k
+    _hand_back(ws, corpus.device, stream)
     return out_ids, out_scores, out_count

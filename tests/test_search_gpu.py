@@ -44,3 +44,59 @@ def test_not_a_number():
     ids, _, count = ops.filtered_topk(x.cuda(), users.cuda(), dates.cuda(), q[:1].cuda(), torch.tensor([1]).cuda(),
                                       torch.tensor([0]).cuda(), torch.tensor([200]).cuda(), 200)
     assert int(count[0]) == 200 and set(ids[0].tolist()) == set(users.nonzero().flatten().tolist())
+
+
+def test_workspaces(monkeypatch):
+    """Batches of several sizes share a set of lists, threads do not, and one whose call failed is not used again."""
+    import threading
+
+    from financial_chatbot_llm_amd.ops import retrieval
+    sizes = [5, 300, 40, 700, 1, 90]
+    x, users, dates, q = corpus(sizes, 3000, 64, 11)
+    who, floor, ks = torch.arange(1, 7, dtype=torch.int32), torch.zeros(6, dtype=torch.int64), torch.full((6,), 50, dtype=torch.int32)
+    rows, rest = [t.cuda() for t in (x, users, dates)], [t.cuda() for t in (q[:6], who, floor, ks)]
+    want = ops.filtered_topk(x, users, dates, q[:6], who, floor, ks, 50)
+    made, zeros = [], torch.zeros
+
+    def counted(*a, **k):
+        made.append(zeros(*a, **k))
+        return made[-1]
+
+    def check(n):
+        for g, w in zip(ops.filtered_topk(*rows, *(t[:n] for t in rest), 50), want):
+            assert torch.equal(g.cpu(), w[:n])
+
+    monkeypatch.setattr(retrieval, "_FREE", [])
+    monkeypatch.setattr(torch, "zeros", counted)
+    check(6)
+    for n in (1, 5, 2, 6, 3):
+        check(n)
+    assert len(made) == 1                                  # one set, made by the first call
+    call = retrieval.N.call
+
+    def fails(name, *args):                                # behind the filter: the counters are not back at zero
+        made[-1].fill_(2)
+        torch.cuda.synchronize()
+        raise RuntimeError(name)
+
+    monkeypatch.setattr(retrieval.N, "call", fails)
+    with pytest.raises(RuntimeError):
+        check(6)
+    monkeypatch.setattr(retrieval.N, "call", call)
+    check(6)
+    assert len(made) == 2
+    errors = []
+
+    def worker():
+        try:
+            for n in (2, 6, 4) * 5:
+                check(n)
+        except BaseException as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=worker) for _ in range(12)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors and len(retrieval._FREE) <= 8
