@@ -179,6 +179,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) rows_attend_kernel(R
   const float sl2 = a.scale * 1.4426950408889634f;
   const float cap_k = CAP ? 2.885390081777927f * a.scale / a.cap : 0.f;
 
+  const int t_begin = ti;
   int buf = 0;
   if (ti <= t_end) stage(ti, 0);
   for (; ti <= t_end; ++ti, buf ^= 1) {
@@ -290,13 +291,73 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) rows_attend_kernel(R
     }
   }
   typedef T out4 __attribute__((ext_vector_type(4)));
+  const T* gate = static_cast<const T*>(a.gate);
+  auto part_of = [&](long rw, int head) { return a.ws + ((rw * a.H + head) * a.nsplit + split) * (long)(P + 2); };
+  auto out_of = [&](long rw, int head) { return static_cast<T*>(a.out) + (rw * a.H + head) * P; };
+  auto gate_of = [&](long rw, int head) { return a.gate_elem ? gate + rw * a.sgate + (long)head * P : nullptr; };
+  auto scale_of = [&](float mn, float lt, long rw, int head) {
+    const float gs = mx_softmax_scale(mn, lt, a.sink, head);
+    return gate != nullptr && !a.gate_elem ? gs * mx_sigmoid(ldf(gate + rw * a.sgate + head)) : gs;
+  };
 #pragma unroll
   for (int b = 0; b < MB; ++b) {
     l[b] = rows_sum4(l[b]);
+    // A key that a pair does not see has weight zero, but zero times a value that is not finite is not zero: pairs whose sums
+    // came out so beside finite weights are walked again, by the whole wave, over the keys they see and no others.  (Looking
+    // for them costs 0.2 - 0.4 us of bf16 calls of 17 - 300 us, up to 3 % in f32: 48 single rows 59.4 -> 61.5 us.)
+    float zero_if_finite = 0.f;
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) zero_if_finite = fmaf(o[b][i][r], 0.f, zero_if_finite);
+    unsigned long long again = __ballot(zero_if_finite != 0.f && qok[b] && l[b] < INFINITY);
+    again |= again >> 32;
+    again = (again | again >> 16) & 0xffff;
+    for (; again != 0; again &= again - 1) {
+      const int at = __ffsll(again) - 1, head = __shfl(hd[b], at, 64), p = __shfl(pq[b], at, 64), p_lo = __shfl(pq_lo[b], at, 64);
+      const long rw = r0 + t0 + ((w * MB + b) * 16 + at) / nh;
+      const float sl = __shfl(slp[b], at, 64);
+      const T* q1 = static_cast<const T*>(a.q) + rw * a.sq + (long)head * D1;
+      const T* q2 = static_cast<const T*>(a.q2) + (rw * a.H + head) * D2;
+      float wm = -INFINITY, wl = 0.f, acc[(P + 63) / 64] = {};
+      for (int i = t_begin; i <= t_end; ++i) {
+        const int k0 = key0(i);
+        const T* tile = static_cast<const T*>(a.cache) +
+                        ((long)a.bt[(long)s * a.btw + k0 / PAGE_ROWS] * PAGE_ROWS + k0 % PAGE_ROWS) * a.Wr;
+        for (int j = k0; j < k0 + KT && j <= p; ++j) {
+          if (j < p_lo && j >= a.keep) continue;
+          const T* kr = tile + (long)(j - k0) * a.Wr + kvh * a.kstep;
+          const T* vr = tile + (long)(j - k0) * a.Wr + a.voff + kvh * a.vstep;
+          float x = 0.f;
+          for (int d = lane; d < D; d += 64) x += ldf(d < D1 ? q1 + d : q2 + (d - D1)) * ldf(kr + d);
+          x = mx_wave_sum(x) * a.scale;
+          if (CAP) x = a.cap * tanhf(x / a.cap);
+          x = x * 1.4426950408889634f + sl * (float)(j - p);
+          const float mn = fmaxf(wm, x), f = __builtin_amdgcn_exp2f(wm - mn), wt = __builtin_amdgcn_exp2f(x - mn);
+          wl = wl * f + wt;
+          wm = mn;
+#pragma unroll
+          for (int u = 0; u < (P + 63) / 64; ++u)
+            if (P % 64 == 0 || lane + 64 * u < P) acc[u] = acc[u] * f + wt * ldf(vr + lane + 64 * u);
+        }
+      }
+      wm *= 0.6931471805599453f;
+      const float gs = a.nsplit > 1 ? 1.f : scale_of(wm, wl, rw, head);
+      const T* ge = gate_of(rw, head);
+#pragma unroll
+      for (int u = 0; u < (P + 63) / 64; ++u) {
+        const int d = lane + 64 * u;
+        if (P % 64 != 0 && d >= P) continue;
+        if (a.nsplit > 1) part_of(rw, head)[d] = acc[u];
+        else stf(out_of(rw, head) + d, acc[u] * gs * (ge != nullptr ? mx_sigmoid(ldf(ge + d)) : 1.f));
+      }
+      if (a.nsplit > 1 && lane < 2) part_of(rw, head)[P + lane] = lane == 0 ? wm : wl;
+      if (c == at) qok[b] = false;                               // written
+    }
     if (!qok[b]) continue;
     const float mn = m[b] * 0.6931471805599453f;                 // of the natural exponent
     if (a.nsplit > 1) {
-      float* x = a.ws + ((row[b] * a.H + hd[b]) * a.nsplit + split) * (long)(P + 2);
+      float* x = part_of(row[b], hd[b]);
       typedef float f32x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
       for (int i = 0; i < NT; ++i) {
@@ -309,11 +370,9 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) rows_attend_kernel(R
       }
       continue;
     }
-    float gs = mx_softmax_scale(mn, l[b], a.sink, hd[b]);
-    const T* gate = static_cast<const T*>(a.gate);
-    if (gate != nullptr && !a.gate_elem) gs *= mx_sigmoid(ldf(gate + row[b] * a.sgate + hd[b]));
-    T* dst = static_cast<T*>(a.out) + (row[b] * a.H + hd[b]) * P + 4 * g;
-    const T* ge = a.gate_elem ? gate + row[b] * a.sgate + (long)hd[b] * P + 4 * g : nullptr;
+    const float gs = scale_of(mn, l[b], row[b], hd[b]);
+    T* dst = out_of(row[b], hd[b]) + 4 * g;
+    const T* ge = a.gate_elem ? gate_of(row[b], hd[b]) + 4 * g : nullptr;
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
       out4 x;

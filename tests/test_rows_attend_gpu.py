@@ -88,3 +88,59 @@ def test_latent(segs, H, Dr, window, exact):
         return mx.latent_attend(f(ql), f(qr), f(cache), f(cu), f(pos), f(bt), window, R ** -0.5, max(n for n, _ in segs),
                                 gate=f(gate), sink=f(sink), exact_weights=exact)
     check(run(lambda t: t.cuda()), run(lambda t: t.float() if t.is_floating_point() else t), dt, 0.0 if exact else 2.0 ** -9)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads,opt", [((4, 4), {"window": 1 << 40}), ((6, 2), {"window": 40, "keep_first": 3}),
+                                       ((16, 4), {"window": 64, "chunked": True, "softcap": 5.0, "slopes": True, "sink": True})])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_window_not_finite(dt, heads, opt, bad):
+    """A key or value that is not finite reaches the rows that see its token and no others."""
+    g = torch.Generator().manual_seed(9)
+    (H, G), D = heads, 128
+    segs = [(150, 150), (1, 130), (40, 100)]
+    cu, pos, bt, total = pages(segs, g)
+    cache = rows(segs, bt, total, G * 2 * D, dt, g)
+    q = torch.randn((int(cu[-1]), H * D), generator=g).to(dt)
+    opt = dict(opt)
+    if opt.pop("sink", False):
+        opt["sink"] = torch.randn(H, generator=g)
+    if opt.pop("slopes", False):
+        opt["slopes"] = torch.rand(H, generator=g) * 0.1
+
+    def run(f, cache):
+        o = {k: f(v) if torch.is_tensor(v) else v for k, v in opt.items()}
+        return mx.window_attend(f(q), f(cache), f(cu), f(pos), f(bt), scale=D ** -0.5, max_len=150, heads=H, kv_heads=G, dim=D,
+                                vdim=D, **o)
+    want = run(lambda t: t.float() if t.is_floating_point() else t, cache)
+    token = [101, 37, 75]                                             # one of every segment
+    sees = torch.zeros(int(cu[-1]), dtype=torch.bool)
+    for i, j in enumerate(token):
+        for r in range(int(cu[i]), int(cu[i + 1])):
+            p = int(pos[r])
+            low = p // opt["window"] * opt["window"] if opt.get("chunked") else p - opt["window"] + 1
+            sees[r] = j <= p and (j >= low or j < opt.get("keep_first", 0))
+        cache[bt[i, j // 64], j % 64, G * D + 5::D] = bad             # a value of every key head
+        cache[bt[i, j // 64], j % 64, :G * D:D] = bad if i == 2 else 0.5
+    got = run(lambda t: t.cuda(), cache).cpu()
+    check(got[~sees], want[~sees], dt)
+    assert not torch.isfinite(got[sees].float().view(-1, H, D)[:, :, 5]).any() and 0 < int(sees.sum()) < len(sees)
+
+
+def test_latent_not_finite():
+    g = torch.Generator().manual_seed(10)
+    dt, R, Dr, H = torch.bfloat16, 256, 32, 3
+    segs = [(100, 130), (1, 70)]
+    cu, pos, bt, total = pages(segs, g)
+    cache = rows(segs, bt, total, R + Dr, dt, g)
+    ql, qr = (torch.randn((101, H, n), generator=g).to(dt) for n in (R, Dr))
+
+    def run(f, cache):
+        return mx.latent_attend(f(ql), f(qr), f(cache), f(cu), f(pos), f(bt), 50, R ** -0.5, 100)
+    want = run(lambda t: t.float() if t.is_floating_point() else t, cache)
+    cache[bt[0, 1], 90 - 64, 7] = float("nan")                        # token 90 of the first segment
+    cache[bt[1, 0], 3, 7] = float("inf")                              # left the window long ago
+    sees = torch.cat([(pos[:100] >= 90) & (pos[:100] < 140), torch.zeros(1, dtype=torch.bool)])
+    got = run(lambda t: t.cuda(), cache).cpu()
+    check(got[~sees], want[~sees], dt, 2.0 ** -9)
+    assert not torch.isfinite(got[sees].float()).any()
