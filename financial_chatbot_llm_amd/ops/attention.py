@@ -402,18 +402,25 @@ def encoder_attention(qkv: torch.Tensor, cu: torch.Tensor, max_len: int, heads: 
     """Bidirectional attention of packed texts: ``qkv`` [T, 3 * heads * D] holds q | k | v, text i owns rows
     cu[i] : cu[i + 1] and attends within itself; ``max_len``: the longest text.  Returns [T, heads * D]."""
     T, D = qkv.shape[0], qkv.shape[1] // (3 * heads)
+    if qkv.dim() != 2 or qkv.shape[1] != 3 * heads * D:
+        raise ValueError(f"expected [tokens, 3 * {heads} * head size] rows, got {tuple(qkv.shape)}")
     if N.use_native(qkv):
+        # the kernel reads bf16 rows and 32-bit bounds as they lie
+        if qkv.dtype != torch.bfloat16 or qkv.stride(1) != 1:
+            raise ValueError("the encoder's attention takes bf16 rows with unit column stride")
+        cu = cu.to(qkv.device, torch.int32).contiguous()
         out = torch.empty((T, heads * D), dtype=qkv.dtype, device=qkv.device)
         for a in range(0, cu.numel() - 1, 65535):      # texts per launch
             c = cu[a:a + 65536]
             N.call("penny_encoder_attention", N.ptr(qkv), qkv.stride(0), N.ptr(c), c.numel() - 1, int(max_len), heads, D,
                    float(scale), N.ptr(out), N.stream())
         return out
-    q, k, v = qkv.view(T, 3, heads, D).unbind(1)
+    q, k, v = qkv.reshape(T, 3, heads, D).unbind(1)
     bounds = cu.tolist()
-    out = torch.empty((T, heads, D), dtype=qkv.dtype)
+    out = torch.empty((T, heads, D), dtype=qkv.dtype, device=qkv.device)
     for a, b in zip(bounds, bounds[1:]):
-        out[a:b] = _attend_ref(q[a:b], k[a:b], v[a:b], scale, None)
+        if b > a:
+            out[a:b] = _attend_ref(q[a:b], k[a:b], v[a:b], scale, None)
     return out.view(T, heads * D)
 
 

@@ -32,6 +32,23 @@ def test_encoder_attention(D, H, lens, pad):
         a += n
 
 
+def test_encoder_attention_takes_bf16_rows(monkeypatch):
+    from financial_chatbot_llm_amd import ops
+    from financial_chatbot_llm_amd.ops import _native
+    g = torch.Generator(device="cuda").manual_seed(3)
+    lens, H, D = [5, 70, 0, 1], 2, 64
+    qkv = torch.randn(sum(lens), 3 * H * D, generator=g, device="cuda").to(torch.bfloat16)
+    cu = torch.tensor([0] + lens).cumsum(0).cuda()                            # 64-bit bounds
+    for x in (qkv.float(), qkv.half(), qkv.t().contiguous().t(), qkv[:, :-1]):
+        with pytest.raises(ValueError):
+            ops.encoder_attention(x, cu, 70, H, 0.125)
+    got = ops.encoder_attention(qkv, cu, 70, H, 0.125)
+    monkeypatch.setattr(_native, "_FORCE_TORCH_OPS", True)                     # plain torch on the same device
+    for x in (qkv, torch.cat([qkv, qkv], 1)[:, :3 * H * D]):
+        want = ops.encoder_attention(x, cu, 70, H, 0.125)
+        assert want.device == qkv.device and float((got.float() - want.float()).norm() / want.float().norm()) < 8e-3
+
+
 @pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64, 65, 128, 129, 768])
 @pytest.mark.parametrize("N,K", [(768, 768), (48, 96), (3072, 768), (768, 3072), (16, 32)])
 @pytest.mark.parametrize("gelu", [False, True])
