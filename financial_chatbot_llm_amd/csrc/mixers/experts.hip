@@ -63,7 +63,6 @@ __global__ void __launch_bounds__(1024) expert_plan_kernel(const int* __restrict
   const int nw = blockDim.x >> 6, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   int* cnt = lds + w * E;
   int* base = lds + nw * E;
-  __shared__ int tiles_used;
   const int per = NC > 0 ? NC * 64 : (P + nw * 64 - 1) / (nw * 64) * 64, i0 = w * per, i1 = min(P, i0 + per);
   const int nc = NC > 0 ? NC : (i1 - i0 + 63) / 64;
   int held[NC > 0 ? NC : 1];
@@ -115,10 +114,9 @@ __global__ void __launch_bounds__(1024) expert_plan_kernel(const int* __restrict
       rows += __shfl(sc, 63, 64);
       nt += __shfl(st, 63, 64);
     }
-    if (lane == 0) tiles_used = nt;
+    for (int t = nt + lane; t < ntiles; t += 64) tiles[t] = make_int4(0, 0, 0, 0);
   }
   __syncthreads();
-  for (int t = tiles_used + threadIdx.x; t < ntiles; t += blockDim.x) tiles[t] = make_int4(0, 0, 0, 0);
 #pragma unroll
   for (int c = 0; c < nc; ++c) {
     const int i = i0 + c * 64 + lane, e = expert(c);
@@ -405,8 +403,7 @@ MX_API int mx_experts(const void* h, long ldh, const int* idx, int T, int top, i
   while ((1 << bits) < E) ++bits;
   int nw = (int)((P + 63) / 64);
   nw = nw < 1 ? 1 : (nw > 16 ? 16 : nw);
-  while (nw > 1 && (long)(nw + 1) * E > 16000) --nw;
-  if ((long)(nw + 1) * E * 4 > 65536 - 64) return (int)hipErrorInvalidValue;
+  while (nw > 1 && (long)(nw + 1) * E > 16384) --nw;         // counts per wave and the sums in 64 KB of LDS: 8192 experts
   const long run = (P + nw * 64 - 1) / (nw * 64);            // chunks of 64 pairs per wave
   const size_t lds = (size_t)(nw + 1) * E * 4;
 #define PLAN(NC) expert_plan_kernel<NC><<<1, nw * 64, lds, st>>>(idx, (int)P, E, bits, mt, ntiles, pos, src, tiles)

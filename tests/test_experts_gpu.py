@@ -101,3 +101,10 @@ def test_expert_plan_run_lengths(T):
     """The sort's forms by the length of a wave's run (2, 8, 16 and 32 chunks in registers, a loop beyond)."""
     for top in (1, 2):
         check(torch.bfloat16, T, 16, 16, 5, top, "relu2", ident=1)
+
+
+@pytest.mark.parametrize("E", [8184, 8185, 8192])
+def test_most_experts(E):
+    """As many as the routing kernels choose from; few pairs, and more than a wave's run of them."""
+    check(torch.float32, 40, 8, 8, E, 3, "relu2")
+    check(torch.float32, 900, 8, 8, E, 2, "relu2", skew=True)
