@@ -665,9 +665,20 @@ struct LeanPlan {
   int per_wave;  // units per wave
 };
 
+// How many slots of the workspace a row may use (many: all of them; nparts: one per pb blocks of the longest context) and how
+// many blocks a wave takes at least follow from the contexts, whatever the table and the workspace could hold (us, 32 heads over
+// 8).  Up to 4 rows want many parts whatever lies behind them (3 / 5 / 9 / 16 slots: 1 row behind 900 tokens 13.7 / 11.9 / 10.6 /
+// 10.0, behind 4000 42 / 28 / 19 / 15, 4 rows behind 4000 66 / 40 / 29 / 21), up to 32 rows while their contexts are short (a slot
+// per 8 blocks / 16 slots: 8 rows behind 400 16.4 / 10.6, 20 behind 1200 27.2 / 23.2, 32 behind 900 33 / 24; but 8 behind 4000
+// 28.3 / 29.4).  From 48 rows on the rows themselves fill the chip and parts only cost the merge.  Among the short ones, when a
+// wave would get about one block and rows are not so short that few parts are left, parts of 4 blocks are better than of 2: 12 /
+// 16 / 20 / 32 rows behind 1200, 900, 900 and 900 18.5 / 18.3 / 19.8 / 24.0 and 19.9 / 19.3 / 23.2 / 25.3; but 12 rows behind 800
+// 16.4 and 16.2, 32 behind 400 (7 blocks each) 18.4 and 14.6.
+constexpr int LEAN_FEW_ROWS = 4, LEAN_SOME_ROWS = 32, LEAN_SHORT_BLOCKS = 24;
+
 // s_pre[0..B]: exclusive prefix sums of the per-row block counts
 __device__ __forceinline__ LeanPlan lean_plan(int* s_pre, int* s_w, const int* __restrict__ ctx_lens, int B,
-                                              int nwaves, int nparts, int min_per_wave) {
+                                              int nwaves, int nparts, int many, int min_per_wave) {
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   int c[4], sum = 0, mx = 0;
 #pragma unroll
@@ -703,6 +714,10 @@ __device__ __forceinline__ LeanPlan lean_plan(int* s_pre, int* s_w, const int* _
   }
   if (t == 0) s_pre[B] = total;
   __syncthreads();
+  if (B <= LEAN_FEW_ROWS || (B <= LEAN_SOME_ROWS && maxn <= LEAN_SHORT_BLOCKS)) {
+    nparts = many;
+    if (B > LEAN_FEW_ROWS && 4 * total > 3 * nwaves && total <= 2 * nwaves && total >= 8 * B) min_per_wave *= 2;
+  }
   // a segment of n blocks meets at most ceil(n / per_wave) + 1 waves: keep that <= nparts slots
   const int want = (total + nwaves - 1) / nwaves;
   const int cap = (maxn + nparts - 2) / (nparts - 1);
@@ -740,7 +755,7 @@ __global__ void __launch_bounds__(256) decode_lean_kernel(
   constexpr int KC = D / 32, DT = D / 16;
   __shared__ int s_pre[LEAN_MAX_B + 1];
   __shared__ int s_w[8];
-  const LeanPlan pl = lean_plan(s_pre, s_w, ctx_lens, B, gridDim.x / Hkv * 4, nparts, min_per_wave);
+  const LeanPlan pl = lean_plan(s_pre, s_w, ctx_lens, B, gridDim.x / Hkv * 4, nparts, part_stride, min_per_wave);
   if (blockIdx.x == 0) {
     for (int i = threadIdx.x; i <= B; i += 256) meta[LEAN_META0 + i] = s_pre[i];
     if (threadIdx.x == 0) meta[LEAN_META0 + B + 1] = pl.per_wave;
@@ -866,7 +881,7 @@ __global__ void __launch_bounds__(256) decode_lean_kernel(
         }
       } else {
         const long pi = ((long)b * Hq + hq) * part_stride + (chunk - seg0 / pl.per_wave);
-        PENNY_DASSERT(chunk - seg0 / pl.per_wave < nparts);
+        PENNY_DASSERT(chunk - seg0 / pl.per_wave < part_stride);
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4*>(part_o + pi * D + 16 * dt + 4 * g) = o[dt];
         if (g == 0) {

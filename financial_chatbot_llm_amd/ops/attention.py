@@ -465,8 +465,8 @@ class DecodeWorkspace:
     def create(cls, max_batch: int, Hq: int, D: int, max_ctx: int, device, pb: int = 8) -> "DecodeWorkspace":
         nblk = (max_ctx + KV_BS - 1) // KV_BS
         nparts = max(2, (nblk + pb - 1) // pb)
-        # slots per (row, head): the lean kernel may cut a row of a small batch into 16 parts (decode)
-        stride = max(nparts, min(nblk + 1, 17))
+        # slots per (row, head): the lean kernel may cut a row of a small batch into 15 parts (lean_plan of attention.hip)
+        stride = max(nparts, min(nblk + 1, 16))
         f = dict(dtype=torch.float32, device=device)
         return cls(torch.empty((max_batch, Hq, stride), **f), torch.empty((max_batch, Hq, stride), **f),
                    torch.empty((max_batch, Hq, stride, D), **f), pb, max(nparts, 2), stride,
@@ -481,13 +481,7 @@ _SIDE_STREAMS = {}
 DECODE_LEAN = os.environ.get("PENNY_DECODE_LEAN", "1") != "0"
 LEAN_MIN_B = int(os.environ.get("PENNY_DECODE_LEAN_MIN_B", "1"))
 LEAN_WG_PER_CU = 2          # 242 VGPRs per wave -> 2 waves per SIMD = 2 workgroups per CU
-# blocks a wave takes at least, and how many parts a row may have.  Up to 4 rows want many parts whatever lies behind them (us,
-# 3 / 5 / 9 / 17 slots per row: 1 row behind 900 tokens 13.7 / 11.9 / 10.6 / 10.0, behind 4000 42 / 28 / 19 / 16, 4 rows behind
-# 4000 66 / 40 / 29 / 24), up to 32 rows while their contexts are short (a slot per 8 blocks / 17 slots: 8 rows behind 400
-# 16.4 / 11.6, 20 behind 1200 35.9 / 24.8, 32 behind 1200 37 / 31; but 16 behind 2500 31.2 / 35.1, 8 behind 4000 28.6 / 31.6).
-# Between one and two blocks per wave, parts of 4 blocks (half the waves) are better than of 2: 16 / 20 / 24 rows behind 1200
-# 20.7 / 24.8 / 25.8 and 23.6 / 27.3 / 27.8.  From 48 rows on the rows themselves fill the chip and parts only cost the merge.
-LEAN_SPLIT_BLOCKS = 24
+# blocks a wave takes at least (lean_plan of attention.hip takes twice as many for some small batches)
 LEAN_MIN_PER_WAVE = 2
 # lean kernel flags (attention.hip penny_attention_decode lean_flags): bit 0 = non-temporal K/V loads
 # for the blocks only one row of the step reads (the host marks the shared ones: mark_shared_blocks);
@@ -595,16 +589,10 @@ def decode(q: torch.Tensor, ctx_lens: torch.Tensor, block_tables: torch.Tensor, 
         lean = (DECODE_LEAN and B >= LEAN_MIN_B and ws.lean_meta is not None
                 and ws.lean_meta.numel() >= LEAN_META0 + B + 2)
         pb, nparts = ws.partitioning(B) if not lean else (ws.pb, ws.nparts)
-        min_per_wave = LEAN_MIN_PER_WAVE
-        width = block_tables.shape[1]
-        if lean and (B <= 4 or (B <= 32 and width <= LEAN_SPLIT_BLOCKS)):
-            nparts = ws.part_stride
-            if 256 < B * width <= 512:
-                min_per_wave = 4
         args = [N.ptr(q), N.ptr(ctx_lens), N.ptr(block_tables), N.ptr(k_cache), N.ptr(v_cache), N.ptr(out),
                 N.ptr(ws.part_m), N.ptr(ws.part_l), N.ptr(ws.part_o), B, Hq, Hkv, D, block_tables.shape[1], pb,
                 nparts, ws.part_stride, float(scale)]
-        lean_args = ((_lean_grid(q.device, Hkv), N.ptr(ws.lean_meta), min_per_wave,
+        lean_args = ((_lean_grid(q.device, Hkv), N.ptr(ws.lean_meta), LEAN_MIN_PER_WAVE,
                       LEAN_FLAGS if B >= LEAN_NT_MIN_B else LEAN_FLAGS & ~1) if lean else (0, None, 1, 0))
         N.call("penny_attention_decode", *args, *lean_args, N.stream() if stream is None else stream)
         return out
