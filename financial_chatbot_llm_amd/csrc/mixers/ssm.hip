@@ -396,22 +396,32 @@ ssm_scan_kernel(const float* __restrict__ u, int C, const TD* __restrict__ dt_ra
 // 188 us in all, with the factors made in the walk, four value blocks and four waves over, 287 us, token by token 858 us.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int SSD_L = 64;           // tokens per chunk
-constexpr int SSD_LEAST = 32;       // shorter segments go token by token: a chunk costs about as much as 20 steps
+constexpr int SSD_LEAST = 32;       // shorter segments of a step in chunks go token by token: a chunk costs about 20 steps
 
 __device__ __forceinline__ f32x4 mma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
-// Scratch of a chunk -- segment s starts at chunk cu[s] / 64 + s --: per group C . B [64][64] (s up to t's tile of 16) and B in
+// Scratch of a chunk: per group C . B [64][64] (s up to t's tile of 16) and B in
 // operand order [N / 16][4][64 lanes][4 tokens]; per head M in operand order [10 tiles (w, j <= w)][64 lanes][4], E, F.
 constexpr int SSD_HEAD = 10 * 256 + 2 * SSD_L;
 __host__ __device__ inline long ssd_group_floats(int N) { return 64L * SSD_L + 64L * N; }
 __host__ __device__ inline long ssd_chunk_floats(int N, int G, int H) { return G * ssd_group_floats(N) + (long)H * SSD_HEAD; }
+
+// max_len is a bound: the only segment of a step may be of any length, and needs no fourth launch whatever it is
+__host__ __device__ inline int ssd_least(int S) { return S == 1 ? 1 : SSD_LEAST; }
+
+// The chunk that segment s, from row r0 on, starts at: no two segments of SSD_LEAST rows or more share one, and the shorter
+// ones, which have none, do not move it by more than the rows before it allow.
+__host__ __device__ inline int ssd_first(int r0, int s) { return r0 / SSD_L + (s < r0 / SSD_LEAST ? s : r0 / SSD_LEAST); }
+
+// all chunks of S segments in T rows
+__host__ __device__ inline int ssd_chunks(int T, int S) { return ssd_first(T, S) > 1 ? ssd_first(T, S) : 1; }
 
 // the last segment that starts at or before chunk ci
 __device__ __forceinline__ int ssd_segment(const int* cu, int S, int ci) {
   int s = 0;
   for (int lo = 0, hi = S; lo < hi;) {
     const int mid = (lo + hi) >> 1;
-    if (cu[mid] / SSD_L + mid <= ci) {
+    if (ssd_first(cu[mid], mid) <= ci) {
       s = mid;
       lo = mid + 1;
     } else {
@@ -421,15 +431,15 @@ __device__ __forceinline__ int ssd_segment(const int* cu, int S, int ci) {
   return s;
 }
 
-// grid (T / 64 + S, G)
+// grid (ssd_chunks(T, S), G)
 template <int NTW>
 __global__ void __launch_bounds__(256, 2) ssd_scores_kernel(const float* __restrict__ u, int C, const int* __restrict__ cu,
                                                             const int* __restrict__ slot, float* __restrict__ ws, int S, int H,
                                                             int inner, int G) {
   constexpr int N = 64 * NTW, NJ = N / 16;
   const int ci = blockIdx.x, grp = blockIdx.y, s = ssd_segment(cu, S, ci);
-  const int r0 = cu[s], n = cu[s + 1] - r0, c0 = (ci - r0 / SSD_L - s) * SSD_L;
-  if (slot[s] < 0 || n < SSD_LEAST || c0 < 0 || c0 >= n) return;
+  const int r0 = cu[s], n = cu[s + 1] - r0, c0 = (ci - ssd_first(r0, s)) * SSD_L;
+  if (slot[s] < 0 || n < ssd_least(S) || c0 < 0 || c0 >= n) return;
   float* cb = ws + ci * ssd_chunk_floats(N, G, H) + grp * ssd_group_floats(N);
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, c = lane & 15;
   const float* ub = u + inner + grp * N + 4 * g;
@@ -463,7 +473,7 @@ __global__ void __launch_bounds__(256, 2) ssd_scores_kernel(const float* __restr
   }
 }
 
-// grid (T / 64 + S, H)
+// grid (ssd_chunks(T, S), H)
 template <typename TD>
 __global__ void __launch_bounds__(256) ssd_decay_kernel(const TD* __restrict__ dt_raw, long sdt,
                                                         const float* __restrict__ dt_bias, const float* __restrict__ A_log,
@@ -472,8 +482,8 @@ __global__ void __launch_bounds__(256) ssd_decay_kernel(const TD* __restrict__ d
   __shared__ double cums[4][SSD_L];      // a copy per wave
   __shared__ float dts[4][SSD_L];
   const int ci = blockIdx.x, h = blockIdx.y, s = ssd_segment(cu, S, ci);
-  const int r0 = cu[s], n = cu[s + 1] - r0, c0 = (ci - r0 / SSD_L - s) * SSD_L;
-  if (slot[s] < 0 || n < SSD_LEAST || c0 < 0 || c0 >= n) return;
+  const int r0 = cu[s], n = cu[s + 1] - r0, c0 = (ci - ssd_first(r0, s)) * SSD_L;
+  if (slot[s] < 0 || n < ssd_least(S) || c0 < 0 || c0 >= n) return;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, c = lane & 15;
   const float A = -expf(A_log[h]);
   const float raw = ldf(dt_raw + (long)(r0 + min(c0 + lane, n - 1)) * sdt + h);
@@ -518,12 +528,12 @@ ssd_scan_kernel(const float* __restrict__ u, int C, const float* __restrict__ Dp
   __shared__ __attribute__((aligned(16))) float sbuf[2][16][N + 4];   // the state, [p][n]: rows 4 banks apart
   const int s = blockIdx.z, h = blockIdx.x, p0 = blockIdx.y * 16;
   const int sl = slot[s], r0 = cu[s], n = cu[s + 1] - r0;
-  if (sl < 0 || n < SSD_LEAST) return;
+  if (sl < 0 || n < ssd_least(gridDim.z)) return;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, c = lane & 15;
   const int grp = h / (H / G), inner = H * P, last = (n - 1) / SSD_L;
   const float Dh = Dp[h];
   const long step = ssd_chunk_floats(N, G, H);
-  const float* base = ws + (long)(r0 / SSD_L + s) * step;
+  const float* base = ws + (long)ssd_first(r0, s) * step;
   const float* bbase = base + grp * ssd_group_floats(N) + SSD_L * SSD_L + (NTW * w * 256 + lane) * 4;
   const float* hbase = base + G * ssd_group_floats(N) + (long)h * SSD_HEAD;
   const float* ux = u + (long)r0 * C + h * P + p0 + c;
@@ -696,7 +706,7 @@ MX_API int mx_conv_silu(const void* in, long si, int dt, const float* w, const f
 
 // u f32 [rows, C = H*P + 2*G*N]; dt_raw [rows, H] slice (stride sdt, type dt_code); state f32
 // [slots, H, P, N]; y f32 [rows, H*P]; max_len: no segment is longer; ws: f32 scratch of
-// (rows / 64 + S) * ssd_chunk_floats(N, G, H) values for the chunked form, or null (token by token).
+// max(1, rows / 64 + min(S, rows / 32)) * ssd_chunk_floats(N, G, H) values for the chunked form, or null (token by token).
 // The chunked form takes states of 64, 128 or 256 columns, value sizes in whole tiles of 16 and 16-byte rows.
 MX_API int mx_ssm_scan(const float* u, int C, const void* dt_raw, long sdt, int dt_code, const float* dt_bias,
                        const float* A_log, const float* D, float* state, const int* cu, const int* slot,
@@ -709,7 +719,7 @@ MX_API int mx_ssm_scan(const float* u, int C, const void* dt_raw, long sdt, int 
   const bool chunked = ws != nullptr && max_len >= SSD_LEAST && (N == 64 || N == 128 || N == 256) && P % 16 == 0 && vecu &&
                        ((size_t)u | (size_t)ws) % 16 == 0 && H <= 65535 && S <= 65535;
   if (chunked) {
-    const int chunks = cu_rows_bound / SSD_L + S;
+    const int chunks = ssd_chunks(cu_rows_bound, S);
 #define SSD(NTW)                                                                                                 \
   do {                                                                                                           \
     ssd_scores_kernel<NTW><<<dim3(chunks, G), 256, 0, st>>>(u, C, cu, slot, ws, S, H, H * P, G);                 \
@@ -722,7 +732,7 @@ MX_API int mx_ssm_scan(const float* u, int C, const void* dt_raw, long sdt, int 
     else SSD(4);
 #undef SSD
     const int rc = (int)hipGetLastError();
-    if (rc) return rc;                                   // (max_len is a bound: every segment may still be a short one)
+    if (rc || S == 1) return rc;
   }
   const int below = chunked ? SSD_LEAST : 0x7fffffff;
   dim3 grid((P + SCAN_PT - 1) / SCAN_PT, H, S);

@@ -380,11 +380,29 @@ def conv_silu(inp: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], 
     return out
 
 
+def _ssm_in_chunks(T: int, S: int, max_len: int, state: int) -> bool:
+    """Whether a step of S segments and T rows goes in chunks rather than token by token (``state``: numbers in a state).
+
+    An estimate of both forms' times in us.  Token by token: the longest chain, or the rows (staged by 32) and the states
+    moved, about added where they are alike.  In chunks: three launches more, the products (64 rows at a time) and the same
+    states, moved by single rows after the chunks and not beside them.  64 heads of 64 x 128, tokens / chunks: one segment of
+    48 rows 17.9 / 17.6, of 64 20.7 / 18.1, of 256 69 / 28; four of 32 27.5 / 29.8, of 40 38 / 32; one of 64 beside 8 single
+    rows 24 / 27, of 96 32 / 30; one of 192 beside 64 single rows 76 / 81, of 256 90 / 84.  32 heads: one of 64 beside 8
+    single rows 21 / 24; four of 96 beside 64 55 / 61, of 128 64 / 61."""
+    if max_len < 32:
+        return False
+    size = state / (64 * 64 * 128)
+    moved = 0.75 * S * size
+    staged, padded = (-(-max_len // n) * n / max_len for n in (32, 64))
+    tokens = ((5.5 + 0.27 * max_len) ** 4 + (0.165 * max(T - S, 0) * staged * size + moved) ** 4) ** 0.25
+    return 16.5 + 0.2 * S + 0.047 * T * padded * size + moved < tokens
+
+
 def ssm_scan(u: torch.Tensor, dt_raw: torch.Tensor, dt_bias: torch.Tensor, A_log: torch.Tensor, D: torch.Tensor,
              state: torch.Tensor, cu: torch.Tensor, slot: torch.Tensor, pos: torch.Tensor, heads: int, vdim: int,
              nstate: int, groups: int, max_len: int = 0) -> torch.Tensor:
-    """Mamba-2 recurrence in f32 (``max_len``: no segment is longer, all rows when left out; the kernels take long segments
-    in chunks).  ``u`` f32 [T, H*P + 2*G*N] = [x | B | C] (after the convolution), ``dt_raw`` [T, H]; per head h of group
+    """Mamba-2 recurrence in f32 (``max_len``: no segment is longer, all rows when left out; steps of long segments go in
+    chunks).  ``u`` f32 [T, H*P + 2*G*N] = [x | B | C] (after the convolution), ``dt_raw`` [T, H]; per head h of group
     h // (H / G):
     dt = softplus(dt_raw + dt_bias), S <- exp(-exp(A_log) dt) S + dt x B^T, y = S C + D x.
     ``state`` f32 [slots, H, P, N] is read (unless the segment starts at position 0) and replaced."""
@@ -396,8 +414,8 @@ def ssm_scan(u: torch.Tensor, dt_raw: torch.Tensor, dt_bias: torch.Tensor, A_log
         y = torch.empty((T, H * P), dtype=torch.float32, device=u.device)
         max_len = max_len or T
         ws = None
-        if max_len >= 32 and Ns in (64, 128, 256):          # the chunked form's factors (ssd_chunk_floats of the kernels)
-            ws = torch.empty((T // 64 + S, G * 64 * (64 + Ns) + H * 2688), dtype=torch.float32, device=u.device)
+        if Ns in (64, 128, 256) and _ssm_in_chunks(T, S, max_len, H * P * Ns):          # the factors: ssd_chunk_floats of the kernels
+            ws = torch.empty((max(1, T // 64 + min(S, T // 32)), G * 64 * (64 + Ns) + H * 2688), dtype=torch.float32, device=u.device)
         N.mcall("mx_ssm_scan", N.ptr(u), C, N.ptr(_rows(dt_raw)), dt_raw.stride(0), _dt(dt_raw), N.ptr(dt_bias),
                 N.ptr(A_log), N.ptr(D), N.ptr(state), N.ptr(cu), N.ptr(slot), N.ptr(pos), N.ptr(y), S, int(max_len), H, P, Ns, G,
                 T, N.ptr(ws), N.stream())
