@@ -93,7 +93,7 @@ matrix_scan_kernel(const TQ* __restrict__ q, long sq, const TQ* __restrict__ k, 
                    const int* __restrict__ cu, const int* __restrict__ slot, const int* __restrict__ pos,
                    float* __restrict__ out, int H, int G, int D, int P, const float* __restrict__ a_bias,
                    const float* __restrict__ A_log, const void* __restrict__ beta, long sbeta, int beta_code,
-                   float tau_inv) {
+                   float tau_inv, int most) {
   constexpr bool DELTA = MODE == 1, FIXED = MODE == 2;
   constexpr int DP = RPL * LPC;          // padded key size
   constexpr int CB = 256 / LPC;          // columns per block
@@ -110,7 +110,7 @@ matrix_scan_kernel(const TQ* __restrict__ q, long sq, const TQ* __restrict__ k, 
   const int sl = slot[s];
   if (sl < 0) return;
   const int r0 = cu[s], n = cu[s + 1] - r0;
-  if (n <= 0) return;
+  if (n <= 0 || n > most) return;        // longer ones are not this launch's
   const int h = blockIdx.y, kvh = h / (H / G);
   const int tid = threadIdx.x, part = tid % LPC, cl = tid / LPC;
   const int c0 = blockIdx.x * CB, col = c0 + cl;
@@ -421,17 +421,17 @@ template <typename TQ, int RPL, int LPC, int DELTA>
 int launch_matrix_scan(const void* q, long sq, const void* k, long sk, const void* v, long sv, const float* g, long sa,
                        const float* aux, float* state, const int* cu, const int* slot, const int* pos, float* out, int S,
                        int H, int G, int D, int P, const float* a_bias, const float* A_log, const void* beta, long sbeta,
-                       int beta_dt, float tau_inv, bool one, hipStream_t st) {
+                       int beta_dt, float tau_inv, bool one, int most, hipStream_t st) {
   constexpr int CB = 256 / LPC;
   dim3 grid((P + CB - 1) / CB, H, S);
   if (one)
     matrix_scan_kernel<TQ, RPL, LPC, DELTA, true><<<grid, 256, 0, st>>>(
         (const TQ*)q, sq, (const TQ*)k, sk, (const TQ*)v, sv, g, sa, aux, state, cu, slot, pos, out, H, G, D, P, a_bias,
-        A_log, beta, sbeta, beta_dt, tau_inv);
+        A_log, beta, sbeta, beta_dt, tau_inv, most);
   else
     matrix_scan_kernel<TQ, RPL, LPC, DELTA, false><<<grid, 256, 0, st>>>(
         (const TQ*)q, sq, (const TQ*)k, sk, (const TQ*)v, sv, g, sa, aux, state, cu, slot, pos, out, H, G, D, P, a_bias,
-        A_log, beta, sbeta, beta_dt, tau_inv);
+        A_log, beta, sbeta, beta_dt, tau_inv, most);
   MX_RETURN_LAUNCH();
 }
 
@@ -503,7 +503,7 @@ __global__ void __launch_bounds__(256, 2)
 scan_chunk_prep_kernel(const TQ* __restrict__ q, long sq, const TQ* __restrict__ k, long sk, const float* __restrict__ a,
                        long sa, const float* __restrict__ a_bias, const float* __restrict__ A_log,
                        const void* __restrict__ beta, long sbeta, int beta_code, float tau_inv, float* __restrict__ ws,
-                       const int* __restrict__ cu, const int* __restrict__ slot, int S, int H, int G, int D) {
+                       const int* __restrict__ cu, const int* __restrict__ slot, int S, int H, int G, int D, int least) {
   constexpr int LD = DP + 4;             // 16 rows at one column meet different banks
   __shared__ __align__(16) float qs[SCC * LD], ks[SCC * LD], gs[SCC * LD];
   __shared__ __align__(16) float As[SCC * SCC], Ms[SCC * SCC];
@@ -522,7 +522,7 @@ scan_chunk_prep_kernel(const TQ* __restrict__ q, long sq, const TQ* __restrict__
     }
   }
   const int first = (ci - cu[s] / SCC - s) * SCC, n = cu[s + 1] - cu[s];
-  if (slot[s] < 0 || first < 0 || first >= n) return;
+  if (slot[s] < 0 || n < (DELTA ? least : 1) || first < 0 || first >= n) return;
   const long row0 = cu[s] + first;
   const int nt = min(SCC, n - first);
   const float qscale = 1.0f / sqrtf((float)D);
@@ -645,13 +645,13 @@ template <typename TQ, int DP, int NW, bool DELTA>
 __global__ void __launch_bounds__(NW * 64, 2)
 scan_chunk_kernel(const TQ* __restrict__ v, long sv, const float* __restrict__ ws, float* __restrict__ state,
                   const int* __restrict__ cu, const int* __restrict__ slot, const int* __restrict__ pos,
-                  float* __restrict__ out, int H, int D, int P) {
+                  float* __restrict__ out, int H, int D, int P, int least) {
   constexpr int TPW = DP / 16 / NW;      // tiles of 16 key channels per wave
   __shared__ __align__(16) f32x4 us[2][NW][64];
   __shared__ __align__(16) f32x4 os[2][NW][64];
   const int h = blockIdx.x, s = blockIdx.z;
   const int sl = slot[s], r0 = cu[s], n = cu[s + 1] - r0;
-  if (sl < 0 || n <= 0) return;
+  if (sl < 0 || n < (DELTA ? least : 1)) return;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c = lane & 15;
   const int col = blockIdx.y * 16 + c;
   const bool cok = col < P;
@@ -788,12 +788,12 @@ template <typename TQ, int TPW, bool DELTA>
 int launch_scan_chunks(const void* q, long sq, const void* k, long sk, const void* v, long sv, const float* a, long sa,
                        const float* a_bias, const float* A_log, const void* beta, long sbeta, int beta_dt, float tau_inv,
                        float* ws, float* state, const int* cu, const int* slot, const int* pos, float* out, int S, int T,
-                       int H, int G, int D, int P, hipStream_t st) {
+                       int H, int G, int D, int P, int least, hipStream_t st) {
   scan_chunk_prep_kernel<TQ, 64 * TPW, DELTA><<<dim3(T / SCC + S, H), 256, 0, st>>>(
-      (const TQ*)q, sq, (const TQ*)k, sk, a, sa, a_bias, A_log, beta, sbeta, beta_dt, tau_inv, ws, cu, slot, S, H, G, D);
+      (const TQ*)q, sq, (const TQ*)k, sk, a, sa, a_bias, A_log, beta, sbeta, beta_dt, tau_inv, ws, cu, slot, S, H, G, D, least);
   constexpr int NW = TPW <= 2 ? 4 : 8;
   scan_chunk_kernel<TQ, 64 * TPW, NW, DELTA><<<dim3(H, (P + 15) / 16, S), NW * 64, 0, st>>>((const TQ*)v, sv, ws, state, cu, slot,
-                                                                                          pos, out, H, D, P);
+                                                                                          pos, out, H, D, P, least);
   MX_RETURN_LAUNCH();
 }
 
@@ -802,25 +802,35 @@ int run_matrix_scan(const void* q, long sq, const void* k, long sk, const void* 
                     const float* a_bias, const float* A_log, const void* beta, long sbeta, int beta_dt, float tau_inv,
                     float* aux, float* ws, float* state, const int* cu, const int* slot, const int* pos, float* out, int S,
                     int T, int H, int G, int D, int P, int max_len, hipStream_t st) {
-  const bool one = max_len == 1;         // every segment is a single row: no chunk staging
-  if (ws != nullptr && max_len >= SCAN_LEAST && D <= 256) {
+  // Steps of segments that are short on average are decode rows beside a prompt or two.  In the delta form a single row takes a
+  // chunk as long as 16 do, and the single-row form a quarter of that: with more than 256 blocks' worth of rows the single ones
+  // go there (16 heads of 128 x 128, us, all in chunks / apart / token form: 64 single rows beside 32 rows 96 / 50 / 92, 16 beside
+  // 128 41 / 38 / 64; with longer prompts the rows hide behind the chain: 32 beside 1000 119 / 124 / 340), and steps below that
+  // of at most two full chunks stay in the token form (8 heads, 21 beside three of 32 33 / 37 / 28).  Gla's chunks are cheaper.
+  const bool rows = DELTA && T < 32L * S;
+  const bool split = rows && max_len >= SCAN_LEAST && max_len <= 256 && (long)S * H * P > 256L * 128 && ws != nullptr && D <= 256;
+  const bool chunks = split || (ws != nullptr && max_len >= SCAN_LEAST && D <= 256 && !(rows && S >= 16 && max_len < 48));
+  if (chunks) {
+    const int least = split ? 2 : 1;
 #define SCAN_CHUNKS(TPW)                                                                                                  \
   launch_scan_chunks<TQ, TPW, DELTA>(q, sq, k, sk, v, sv, a, sa, a_bias, A_log, beta, sbeta, beta_dt, tau_inv, ws, state, \
-                                     cu, slot, pos, out, S, T, H, G, D, P, st)
-    return D <= 64 ? SCAN_CHUNKS(1) : D <= 128 ? SCAN_CHUNKS(2) : SCAN_CHUNKS(4);
+                                     cu, slot, pos, out, S, T, H, G, D, P, least, st)
+    const int rc = D <= 64 ? SCAN_CHUNKS(1) : D <= 128 ? SCAN_CHUNKS(2) : SCAN_CHUNKS(4);
 #undef SCAN_CHUNKS
+    if (rc || !split) return rc;
   }
+  const bool one = max_len == 1 || split;          // single rows: no chunk staging
   if (!one)        // single-row steps fold this pass into the scan (one launch less per layer)
     scan_prep_kernel<TQ, DELTA><<<T, 256, 0, st>>>((const TQ*)q, sq, (const TQ*)k, sk, a, sa, a_bias, A_log, beta, sbeta,
                                                    beta_dt, tau_inv, aux, H, G, D);
   // the longest segment sets the step's duration: count the segments that can be about that long (a
   // prompt chunk beside many single decode rows is still one long chain)
-  const long seff = max_len > 0 ? (S < (T + max_len - 1) / max_len ? S : (T + max_len - 1) / max_len) : S;
+  const long seff = max_len > 0 && !split ? (S < (T + max_len - 1) / max_len ? S : (T + max_len - 1) / max_len) : S;
   const int lpc = D <= 128 ? 4 : (D <= 256 ? 8 : 16);
   const long blocks = seff * H * ((P + 256 / lpc - 1) / (256 / lpc));
   return dispatch_matrix_scan<TQ, DELTA>(D, blocks < 512, q, sq, k, sk, v, sv, (const float*)a, sa, (const float*)aux, state,
                                          cu, slot, pos, out, S, H, G, D, P, a_bias, A_log, beta, sbeta, beta_dt, tau_inv,
-                                         one, st);
+                                         one, split ? 1 : 0x7fffffff, st);
 }
 
 }  // namespace
@@ -871,10 +881,10 @@ MX_API int mx_decay_scan(const void* q, long sq, const void* k, long sk, int dt_
   if (dt_qk == 1)
     return dispatch_matrix_scan<float, 2>(D, blocks < 512, q, sq, k, sk, v, sv, (const float*)nullptr, 0L,
                                           (const float*)nullptr, state, cu, slot, pos, out, S, H, H, D, P, decay,
-                                          (const float*)nullptr, (const void*)nullptr, 0L, code, out_scale, one, st);
+                                          (const float*)nullptr, (const void*)nullptr, 0L, code, out_scale, one, 0x7fffffff, st);
   return dispatch_matrix_scan<bf16, 2>(D, blocks < 512, q, sq, k, sk, v, sv, (const float*)nullptr, 0L,
                                        (const float*)nullptr, state, cu, slot, pos, out, S, H, H, D, P, decay,
-                                       (const float*)nullptr, (const void*)nullptr, 0L, code, out_scale, one, st);
+                                       (const float*)nullptr, (const void*)nullptr, 0L, code, out_scale, one, 0x7fffffff, st);
 }
 
 // u f32 [T, R], OVERWRITTEN with the GeLU branch; z f32 [blocks, T, 2 * R / blocks], OVERWRITTEN with the gates; y [T, >= R] slice (row stride

@@ -94,3 +94,26 @@ def test_not_finite(mode, where):
     assert not torch.isfinite(col).any() and not torch.isfinite(state[5, 0, :, 5]).all()
     if where == "v":                                                  # only that value column
         assert torch.equal(got.view(-1, H, P)[:n, 0, 6], clean.view(-1, H, P)[:n, 0, 6])
+
+
+@pytest.mark.parametrize("mode", ["gla", "delta"])
+@pytest.mark.parametrize("lens", [[1] * 30 + [33, 2, 0, 17] + [1] * 20, [32] + [1] * 7, [31, 32, 1, 1, 2, 3, 0, 1, 1], [70] * 7 + [1],
+                                  [40] * 3 + [1] * 4, [32] * 8])
+@pytest.mark.parametrize("D,P,dt", [(64, 16, torch.bfloat16), (128, 48, torch.float32), (256, 20, torch.bfloat16)])
+def test_single_rows_beside_chunks(mode, lens, D, P, dt):
+    """Steps short on average give their single rows to the single-row form, others take them along."""
+    g = torch.Generator().manual_seed(len(lens) + D)
+    H, G, T, S = 4, 2, sum(lens) + 2, len(lens)
+    r = lambda *s: torch.randn(s, generator=g)  # noqa: E731
+    x = [r(T, G * D).to(dt), r(T, G * D).to(dt), r(T, H * P).to(dt), r(T, H * D), r(H * D) * 0.1, r(S, H, D, P)]
+    slot = torch.randperm(S, generator=g).int()
+    slot[min(3, S - 1)] = -1                                          # padding
+    meta = [torch.tensor([0] + lens).cumsum(0).int(), slot, torch.cat([torch.arange(n) + i % 2 for i, n in enumerate(lens + [2])]).int()]
+    opt = {"A_log": r(H) * 0.5, "beta": r(T, H).to(dt)} if mode == "delta" else {"tau": 16.0}
+    got = [t.cuda() for t in x]
+    out = mx.matrix_scan(*got, *(t.cuda() for t in meta), H, G, D, P, mode, max_len=max(lens),
+                         **{k: v.cuda() if torch.is_tensor(v) else v for k, v in opt.items()}).cpu()
+    want = mx.matrix_scan(*x, *meta, H, G, D, P, mode, **opt)
+    live = torch.cat([torch.full((n,), bool(slot[i] >= 0)) for i, n in enumerate(lens)] + [torch.zeros(2, dtype=torch.bool)])
+    # f32 on both sides: each of <= 70 tokens rounds the state and its products a few times
+    assert torch.allclose(out[live], want[live], rtol=1e-4, atol=2e-4) and torch.allclose(got[5].cpu(), x[5], rtol=1e-4, atol=2e-4)
