@@ -732,12 +732,7 @@ scan_chunk_kernel(const TQ* __restrict__ v, long sv, const float* __restrict__ w
     for (int j = 0; j < TPW; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[j & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.q[j][r], S[j][r], o[j & 1], 0, 0, 0);
-    // The sum stays on this side of the barrier: moved behind the branches that follow, the vector instruction has been
-    // issued before the matrix instruction's result was there on the path around them.
-    if (TPW > 1) {
-      o[0] += o[1];
-      asm volatile("" : "+v"(o[0]));
-    }
+    if (TPW > 1) o[0] += o[1];
     __syncthreads();
     if (DELTA) {
       u = (us[buf][0][lane] + us[buf][1][lane]) + (us[buf][2][lane] + us[buf][3][lane]);
