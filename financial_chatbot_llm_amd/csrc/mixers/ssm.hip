@@ -675,13 +675,16 @@ ssd_scan_kernel(const float* __restrict__ u, int C, const float* __restrict__ Dp
 }  // namespace
 
 // in: [rows, C] slice (row stride si) of the in-projection; out: f32 [rows, C]; state f32 [slots, K-1, C]
-// act: 0 none, 1 SiLU; in_bias (optional, [C]) is added to every input before the convolution
+// act: 0 none, 1 SiLU; in_bias (optional, [C]) is added to every input before the convolution; rows: those of the step
+// By four channels (conv4_kernel) from where memory is the bound: a quarter of the threads with eight inputs each in flight is
+// the slower start for less, and for segments of fewer than eight tokens (bf16, us, by one / by four: 64 single rows of 4608
+// 7.1 / 11.0; 512 rows of 4608 15.6 / 17.1; 1024 19.1 / 18.9; 2048 rows of 8192 36 / 28; 512 segments of 4 rows of 4608 38 / 40).
 MX_API int mx_conv_act(const void* in, long si, int dt, const float* w, const float* bias, const float* in_bias, int act,
                        float* state, const int* cu, const int* slot, const int* pos, float* out, int S, int max_len,
-                       int C, int K, hipStream_t st) {
+                       int rows, int C, int K, hipStream_t st) {
   if (S <= 0 || max_len <= 0) return 0;
   if (K < 1 || K > MAX_TAPS || act < 0 || act > 1) return (int)hipErrorInvalidValue;
-  if (K == 4 && C % 4 == 0 && mx_by_four(in, si, dt) &&
+  if (K == 4 && C % 4 == 0 && rows >= 8L * S && (long)rows * C >= 4500000 && mx_by_four(in, si, dt) &&
       ((size_t)w | (size_t)bias | (size_t)in_bias | (size_t)state | (size_t)out) % 16 == 0) {
     const dim3 grid((C / 4 + 255) / 256, (max_len + CONV_TT - 1) / CONV_TT, S);
     MX_DISPATCH(dt, TT, conv4_kernel<TT><<<grid, 256, 0, st>>>((const TT*)in, si, w, bias, in_bias, act, state, cu, slot, pos,
@@ -699,9 +702,9 @@ MX_API int mx_conv_act(const void* in, long si, int dt, const float* w, const fl
 }
 
 MX_API int mx_conv_silu(const void* in, long si, int dt, const float* w, const float* bias, float* state,
-                        const int* cu, const int* slot, const int* pos, float* out, int S, int max_len, int C, int K,
+                        const int* cu, const int* slot, const int* pos, float* out, int S, int max_len, int rows, int C, int K,
                         hipStream_t st) {
-  return mx_conv_act(in, si, dt, w, bias, nullptr, 1, state, cu, slot, pos, out, S, max_len, C, K, st);
+  return mx_conv_act(in, si, dt, w, bias, nullptr, 1, state, cu, slot, pos, out, S, max_len, rows, C, K, st);
 }
 
 // u f32 [rows, C = H*P + 2*G*N]; dt_raw [rows, H] slice (stride sdt, type dt_code); state f32

@@ -103,8 +103,8 @@ _MIXER_SIGS = {
     "mx_moe_combine": [P, c_long, P, P, P, P, c_long, P, c_long, c_int, c_int, c_int, P, c_int, c_int, P],
     "mx_experts": [P, c_long, P, c_int, c_int, c_int, c_int, c_int, P, c_int, c_int, P, c_int, c_int, c_int, c_float, c_float,
                    P, P, c_long, P, P, c_int, P],
-    "mx_conv_silu": [P, c_long, c_int, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, P],
-    "mx_conv_act": [P, c_long, c_int, P, P, P, c_int, P, P, P, P, P, c_int, c_int, c_int, c_int, P],
+    "mx_conv_silu": [P, c_long, c_int, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, P],
+    "mx_conv_act": [P, c_long, c_int, P, P, P, c_int, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, P],
     "mx_embed_pairs": [P, P, P, c_int, c_int, c_int, c_int, P, P, P, P, P, c_int, c_int, c_int, c_int, P],
     "mx_post_norm": [P, P, c_long, P, P, c_long, P, c_int, P, c_float, P, c_int, c_int, c_int, P],
     "mx_glu_act": [P, c_long, P, c_long, P, c_int, P, c_long, c_int, c_int, c_int, P],

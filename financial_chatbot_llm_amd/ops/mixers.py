@@ -359,7 +359,7 @@ def conv_silu(inp: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], 
     if N.use_native(inp):
         out = torch.empty((T, C), dtype=torch.float32, device=inp.device)
         N.mcall("mx_conv_silu", N.ptr(_rows(inp)), inp.stride(0), _dt(inp), N.ptr(w), N.ptr(bias), N.ptr(state),
-                N.ptr(cu), N.ptr(slot), N.ptr(pos), N.ptr(out), S, int(max_len), C, K, N.stream())
+                N.ptr(cu), N.ptr(slot), N.ptr(pos), N.ptr(out), S, int(max_len), T, C, K, N.stream())
         return out
     out = torch.zeros((T, C), dtype=torch.float32)
     cul, sll, pl = cu.tolist(), slot.tolist(), pos.tolist()
@@ -711,7 +711,7 @@ def conv_act(inp: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], s
     if N.use_native(inp):
         out = torch.empty((T, C), dtype=torch.float32, device=inp.device)
         N.mcall("mx_conv_act", N.ptr(_rows(inp)), inp.stride(0), _dt(inp), N.ptr(w), N.ptr(bias), N.ptr(in_bias),
-                ACTS[act], N.ptr(state), N.ptr(cu), N.ptr(slot), N.ptr(pos), N.ptr(out), S, int(max_len), C, K, N.stream())
+                ACTS[act], N.ptr(state), N.ptr(cu), N.ptr(slot), N.ptr(pos), N.ptr(out), S, int(max_len), T, C, K, N.stream())
         return out
     out = torch.zeros((T, C), dtype=torch.float32)
     cul, sll, pl = cu.tolist(), slot.tolist(), pos.tolist()

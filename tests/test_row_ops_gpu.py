@@ -105,3 +105,25 @@ def test_conv(dt, pad, C, K):
                           in_bias=ib.cuda())
         near(got[live.cuda()], want[live], torch.float32)
         near(ds, cs, torch.float32)
+
+
+@pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("pad", [0, 4, 1])
+@pytest.mark.parametrize("lens", [[900, 33, 70, 8, 2, 1, 100], [8] * 130])
+def test_conv_by_four(dt, pad, lens):
+    """Enough rows for the form by four channels, and layouts that it leaves to the other one."""
+    C, K, T, S = 4612, 4, sum(lens), len(lens)
+    g = torch.Generator().manual_seed(T)
+    x, w, b, ib, state = rand(g, T, C, dt=dt), rand(g, C, K), rand(g, C), rand(g, C), rand(g, S + 1, K - 1, C)
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    slot = torch.randperm(S + 1, generator=g)[:S].int()
+    slot[3] = -1
+    pos = torch.cat([torch.arange(n) + (9 if i % 2 else 0) for i, n in enumerate(lens)]).int()
+    live = torch.cat([torch.full((n,), int(s) >= 0) for n, s in zip(lens, slot)])
+    for act in ("silu", "none"):
+        cs, ds = state.clone(), state.cuda()
+        want = mx.conv_act(x, w, b, cs, cu, slot, pos, max(lens), act, in_bias=ib)
+        got = mx.conv_act(view(x, pad, 0), w.cuda(), b.cuda(), ds, cu.cuda(), slot.cuda(), pos.cuda(), max(lens), act,
+                          in_bias=ib.cuda())
+        near(got[live.cuda()], want[live], torch.float32)
+        near(ds, cs, torch.float32)
