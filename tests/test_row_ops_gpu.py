@@ -54,6 +54,17 @@ def test_head_norm_gate(dt, pad, off, H, P):
 
 
 @pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("pad,off", [(0, 0), (4, 4), (1, 0)])
+@pytest.mark.parametrize("T,H,P", [(22000, 3, 4), (1400, 3, 64), (530, 5, 100), (1025, 2, 128), (342, 3, 256), (513, 2, 256)])
+def test_head_norm_gate_of_many_heads(dt, pad, off, T, H, P):
+    g = torch.Generator().manual_seed(P)
+    o, z, w = rand(g, T, H * P), rand(g, T, H * P, dt=dt), rand(g, P)
+    for act in ("silu", "sigmoid"):
+        want = mx.head_norm_gate(o, w, 1e-5, z, H, act, dt)
+        near(mx.head_norm_gate(view(o, pad, off), w.cuda(), 1e-5, view(z, pad, off), H, act, dt), want, dt)
+
+
+@pytest.mark.parametrize("dt", DTS)
 @pytest.mark.parametrize("pad", [0, 4, 1])
 @pytest.mark.parametrize("W", [4, 1024, 1028, 2048, 4100, 8192, 8196, 777])
 def test_post_norm(dt, pad, W):
