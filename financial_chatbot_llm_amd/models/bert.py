@@ -18,7 +18,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from ..ops import _native as N
-from ..ops.gemm import BGE_SMALL_MAX_M, linear_bias
+from ..ops.gemm import BGE_SMALL_MAX_M, SMALL_MAX_MADS, linear_bias
 from .common import random_tensor
 from .configs import ModelConfig
 
@@ -84,10 +84,12 @@ class BertEncoder:
         return ops.layer_norm(e_word, w["emb_ln_g"], w["emb_ln_b"], c.norm_eps, residual=e_pos)
 
     def _small_batch(self, x: torch.Tensor, cu: torch.Tensor, longest: int) -> bool:
-        """All layers of a batch of up to BGE_SMALL_MAX_M tokens in one native call (x in place); False: not a case for it."""
+        """All layers of a batch of up to BGE_SMALL_MAX_M tokens (fewer in wide models) in one native call (x in place); False:
+        not a case for it."""
         T, F_ = x.shape[0], self.cfg.intermediate_size
-        if not (N.use_native(x) and T <= BGE_SMALL_MAX_M and x.dtype == torch.bfloat16 and cu.numel() <= 65536 and
-                self.H % 32 == 0 and F_ % 32 == 0 and os.environ.get("PENNY_PREFILL_GEMM", "1") == "1"):
+        if not (N.use_native(x) and T <= BGE_SMALL_MAX_M and T * self.H * max(F_, 3 * self.H) < SMALL_MAX_MADS and
+                x.dtype == torch.bfloat16 and cu.numel() <= 65536 and self.H % 32 == 0 and F_ % 32 == 0 and
+                os.environ.get("PENNY_PREFILL_GEMM", "1") == "1"):
             return False
         w = [self.w[n] for n in self.layer_names]
         if not all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.device == x.device and t.data_ptr() % 16 == 0 for t in w) or \

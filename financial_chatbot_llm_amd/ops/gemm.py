@@ -759,6 +759,19 @@ BGE_TILE_MAX_M = 2048
 # (small / tile): 2304 x 768 4.3 / 17 at 18 rows, 11 / 22 at 256, 20 / 22 at 768, 24 / 22 at 1024; 768 x 3072 8 / 32, 19 / 36,
 # 36 / 38, 36 / 38; 3072 x 768 with GELU 4.5 / 26, 12 / 35, 26 / 36, 30 / 36
 BGE_SMALL_MAX_M = 768
+# Every block of it reads its own rows of both operands, about 9 TB/s from the caches, so that wide layers reach the tile
+# kernel's time sooner: at about 2^31 multiply-adds (8192 x 2048 at 128 rows 38 / 35, at 512 88 / 41; 4096 x 1024 at 512
+# 26 / 26, at 768 35 / 26; 1024 x 4096 at 640 45 / 41).  Shapes that the tile kernel does not take have the library's product
+# behind them, whose splits of K win with few columns (384 x 1536, us small / library: 18 rows 5.3 / 5.3, 64 9.0 / 5.3; 1152 x 384:
+# 400 rows 4.9 / 5.7, 512 6.9 / 5.8).
+SMALL_MAX_MADS = 1 << 31
+
+
+def small_bias_wins(M: int, N_: int, K: int) -> bool:
+    """Whether the small-batch kernel is the fastest for a projection of M tokens."""
+    if M > BGE_SMALL_MAX_M or M * N_ * K >= SMALL_MAX_MADS:
+        return False
+    return N_ % 256 == 0 and K % 64 == 0 or M <= 32 or (K <= 512 and M * N_ < 1 << 19)
 
 
 def small_bias_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -783,7 +796,7 @@ def linear_bias(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, gelu: bool = 
     M, K = x.shape
     N_ = w.shape[0]
     mode = os.environ.get("PENNY_PREFILL_GEMM", "1")
-    if mode == "1" and M <= BGE_SMALL_MAX_M and small_bias_ok(x, w) and _bias_row(b, w):
+    if mode == "1" and small_bias_wins(M, N_, K) and small_bias_ok(x, w) and _bias_row(b, w):
         y = torch.empty((M, N_), dtype=x.dtype, device=x.device)
         N.call("penny_gemm_bias_small", N.ptr(x), x.stride(0), N.ptr(w), K, N.ptr(y), N_, N.ptr(b), M, N_, int(gelu),
                N.stream())

@@ -145,3 +145,10 @@ def test_encoder_embed_edges():
         ep = (ops.embedding(pos, position).float() + kind[0].float()).to(torch.bfloat16)
         want = ops.layer_norm(ops.embedding(ids, word), w, b, 1e-12, residual=ep)
         assert float((y.float() - want.float()).abs().max()) <= 2.0 ** -6      # a rounding to bf16 below 4
+
+
+def test_projection_form_follows_its_shape():
+    """Shapes of which each form was measured faster."""
+    from financial_chatbot_llm_amd.ops.gemm import small_bias_wins as small
+    assert all(small(*s) for s in ((768, 2304, 768), (768, 768, 3072), (400, 1152, 384), (18, 384, 1536), (64, 8192, 2048), (511, 4096, 1024)))
+    assert not any(small(*s) for s in ((769, 768, 768), (512, 1152, 384), (64, 384, 1536), (128, 8192, 2048), (768, 4096, 1024)))
