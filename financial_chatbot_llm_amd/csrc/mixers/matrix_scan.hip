@@ -804,7 +804,20 @@ int run_matrix_scan(const void* q, long sq, const void* k, long sk, const void* 
   // of at most two full chunks stay in the token form (8 heads, 21 beside three of 32 33 / 37 / 28).  Gla's chunks are cheaper.
   const bool rows = DELTA && T < 32L * S;
   const bool split = rows && max_len >= SCAN_LEAST && max_len <= 256 && (long)S * H * P > 256L * 128 && ws != nullptr && D <= 256;
-  const bool chunks = split || (ws != nullptr && max_len >= SCAN_LEAST && D <= 256 && !(rows && S >= 16 && max_len < 48));
+  // the longest segment sets the step's duration: count the segments that can be about that long (a
+  // prompt chunk beside many single decode rows is still one long chain)
+  const long seff = max_len > 0 && !split ? (S < (T + max_len - 1) / max_len ? S : (T + max_len - 1) / max_len) : S;
+  // Keys pad to 64 or 128 channels in chunks and not in the token form.  Where its blocks of 64 value columns fill the chip its
+  // chains no longer matter, and it is the faster form (us, token / chunks of 32 segments of 100 tokens, 64 heads with values of
+  // 64: delta, keys of 16 134 / 319, 64 240 / 341, 128 517 / 521; gla, 32 100 / 142, 64 183 / 126; 16 segments of 40, 32 heads,
+  // delta, 64: 45 / 54).
+  const long blocks64 = seff * H * ((P + 63) / 64);
+  const bool brief = max_len < 64;
+  long full = 1L << 62;
+  if (D <= 32) full = DELTA || brief ? 256 : 512;
+  else if (DELTA && D <= 96) full = brief ? 256 : D <= 64 ? 512 : 1024;
+  const bool chunks = split || (ws != nullptr && max_len >= SCAN_LEAST && D <= 256 && !(rows && S >= 16 && max_len < 48) &&
+                                blocks64 < full);
   if (chunks) {
     const int least = split ? 2 : 1;
 #define SCAN_CHUNKS(TPW)                                                                                                  \
@@ -818,9 +831,6 @@ int run_matrix_scan(const void* q, long sq, const void* k, long sk, const void* 
   if (!one)        // single-row steps fold this pass into the scan (one launch less per layer)
     scan_prep_kernel<TQ, DELTA><<<T, 256, 0, st>>>((const TQ*)q, sq, (const TQ*)k, sk, a, sa, a_bias, A_log, beta, sbeta,
                                                    beta_dt, tau_inv, aux, H, G, D);
-  // the longest segment sets the step's duration: count the segments that can be about that long (a
-  // prompt chunk beside many single decode rows is still one long chain)
-  const long seff = max_len > 0 && !split ? (S < (T + max_len - 1) / max_len ? S : (T + max_len - 1) / max_len) : S;
   const int lpc = D <= 128 ? 4 : (D <= 256 ? 8 : 16);
   const long blocks = seff * H * ((P + 256 / lpc - 1) / (256 / lpc));
   return dispatch_matrix_scan<TQ, DELTA>(D, blocks < 512, q, sq, k, sk, v, sv, (const float*)a, sa, (const float*)aux, state,

@@ -117,3 +117,23 @@ def test_single_rows_beside_chunks(mode, lens, D, P, dt):
     live = torch.cat([torch.full((n,), bool(slot[i] >= 0)) for i, n in enumerate(lens)] + [torch.zeros(2, dtype=torch.bool)])
     # f32 on both sides: each of <= 70 tokens rounds the state and its products a few times
     assert torch.allclose(out[live], want[live], rtol=1e-4, atol=2e-4) and torch.allclose(got[5].cpu(), x[5], rtol=1e-4, atol=2e-4)
+
+
+@pytest.mark.parametrize("mode", ["gla", "delta"])
+@pytest.mark.parametrize("D,H,P,lens", [(32, 16, 64, [40] * 16), (16, 32, 64, [70] * 16), (64, 32, 64, [65] * 16), (48, 16, 64, [33, 50] * 8),
+                                        (96, 16, 64, [40] * 16), (32, 16, 64, [65] * 3)])
+def test_many_chains(mode, D, H, P, lens):
+    """Steps on both sides of the line from which small keys go token by token."""
+    g = torch.Generator().manual_seed(D + len(lens))
+    T, S = sum(lens), len(lens)
+    r = lambda *s: torch.randn(s, generator=g)  # noqa: E731
+    x = [r(T, H * D), r(T, H * D), r(T, H * P), r(T, H * D), r(H * D) * 0.1, r(S, H, D, P)]
+    meta = [torch.tensor([0] + lens).cumsum(0).int(), torch.randperm(S, generator=g).int(),
+            torch.cat([torch.arange(n) + i % 2 for i, n in enumerate(lens)]).int()]
+    opt = {"A_log": r(H) * 0.5, "beta": r(T, H)} if mode == "delta" else {"tau": 16.0}
+    got = [t.cuda() for t in x]
+    out = mx.matrix_scan(*got, *(t.cuda() for t in meta), H, H, D, P, mode, max_len=max(lens),
+                         **{k: v.cuda() if torch.is_tensor(v) else v for k, v in opt.items()}).cpu()
+    want = mx.matrix_scan(*x, *meta, H, H, D, P, mode, **opt)
+    # f32 on both sides: each of <= 70 tokens rounds the state and its products a few times
+    assert torch.allclose(out, want, rtol=1e-4, atol=2e-4) and torch.allclose(got[5].cpu(), x[5], rtol=1e-4, atol=2e-4)
