@@ -347,10 +347,22 @@ __global__ void __launch_bounds__(256) expert_stream_kernel(ExpertGemm a) {
 // 96, 64: 209 / 127 / 98, 192: - / 183 / 148, 512: - / 355 / 320.  f32 products are bound by the matrix cores much
 // earlier and gain nothing from 128 rows (width 1024, experts of 512): 8: 47 / 69, 24: 68 / 71, 32: 83 / 71 / 119,
 // 96: 161 / 123 / 126, 512: - / 505 / 549.
-int tile_rows(long pairs, int experts, int dt) {
+//
+// Beyond the line to wider tiles a few experts' column blocks may leave the chip idle, and a block's chain of stages, of about
+// 1 us each and more with larger matrices, then takes longer than the weights streamed once per 16 rows by many small blocks.
+// Both are estimated (us; `bytes`: an expert's two matrices; `stages`: of one block of each product): 4 experts of 4096 x 2048,
+// tiles of 16 / 64: 32 rows on average 58 / 132, f32 126 / 569, 96 rows 120 / 122; 8 of 8192 x 2048: 24 rows 165 / 238, 48 rows
+// 274 / 245; 2 of 4096 x 1024: 64 rows 32 / 87; 16 of 768 x 2048: 24 rows 35 / 48, 48 rows 56 / 50.
+// Of the wide tiles, 64 rows also for more when few experts' wider ones would be fewer than the CUs (`columns`: column blocks of
+// the smaller product): 4 experts of 4096 x 2048, 128 rows 126 / 156, 8 of 8192 x 2048, 128 rows 231 / 310, 256 rows 353 / 305.
+int tile_rows(long pairs, int experts, int dt, double bytes, int stages, int columns) {
   const long avg = pairs / experts;
-  if (dt == 1) return avg <= 24 ? 16 : 64;
-  return avg <= 12 ? 16 : (avg <= 56 ? 64 : 128);
+  if (avg <= (dt == 1 ? 24 : 12)) return 16;
+  const double live = pairs < experts ? pairs : experts, memory = live * bytes / 5.2e6;
+  const double chain = stages * (dt == 1 ? 1.15 + bytes * 20e-9 : 0.7 + bytes * 9.5e-9);
+  const double again = (pairs / 16.0 + live / 2) * bytes / (dt == 1 ? 7.0e6 : 7.9e6);
+  if (15 + (again > memory ? again : memory) < 12 + (chain > memory ? chain : memory) && pairs / 16 + experts <= 65535) return 16;
+  return dt == 1 || avg <= 56 || (experts <= 8 && (experts + pairs / 128) * columns < 300) ? 64 : 128;
 }
 
 template <typename T, bool GLU>
@@ -394,7 +406,8 @@ MX_API int mx_experts(const void* h, long ldh, const int* idx, int T, int top, i
       (size_t)iws % 16 || (glu ? g1 % 2 || g1 / 2 * 16 < lda : g1 * 16 < lda) || g2 * 16 < W || unit < 0 || unit > UNIT_RELU2 ||
       (scale != nullptr && !glu))
     return (int)hipErrorInvalidValue;
-  const int mt = tile_rows(P, E, dt);
+  const int mt = tile_rows(P, E, dt, 1024.0 * ((double)g1 * k1 + (double)g2 * k2), (k1 + k2) / 2,
+                           ((g1 < g2 ? g1 : g2) + 7) / 8);
   const int ntiles = (int)(P / mt + (P < E ? P : E));
   int* pos = iws;
   int* src = iws + (P + 3) / 4 * 4;

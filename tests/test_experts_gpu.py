@@ -108,3 +108,13 @@ def test_most_experts(E):
     """As many as the routing kernels choose from; few pairs, and more than a wave's run of them."""
     check(torch.float32, 40, 8, 8, E, 3, "relu2")
     check(torch.float32, 900, 8, 8, E, 2, "relu2", skew=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,W,F_,E,top,unit", [
+    (100, 512, 1024, 2, 1, "relu2"),       # few experts: tiles of 16 rows far beyond the average from which many take 64
+    (130, 2048, 520, 3, 2, "clamped"),
+    (700, 512, 1024, 2, 1, "silu"),        # ... and past the line
+])
+def test_few_experts(dtype, T, W, F_, E, top, unit):
+    check(dtype, T, W, F_, E, top, unit)
