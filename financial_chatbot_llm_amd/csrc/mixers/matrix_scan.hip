@@ -19,8 +19,8 @@
 //            the current chunk's dependent steps run; the chunk's outputs leave through LDS as
 //            whole runs.  Steps with few (segment, head) pairs take the variant with more lanes per
 //            column so that the grid still covers the chip.
-//   gla and delta with a segment of 32 rows or more and D <= 256 take chunks of 16 tokens on the f32 matrix
-//   instructions instead (further down).
+//   gla and delta with D <= 256 take chunks of 16 tokens on the f32 matrix instructions instead (further down) in steps
+//   with a segment of 32 rows or more, but for those that run_matrix_scan keeps here.
 //
 // mx_lru_scan: a diagonal recurrence per channel, S <- a S + sqrt(1 - a^2) i u with
 //     a = exp(-8 sigmoid(zr + r_bias) softplus(lam)),  i = sigmoid(zi + i_bias),
@@ -453,8 +453,8 @@ int dispatch_matrix_scan(int D, bool wide, Args... args) {
 //     delta:  U = T V - W S,  T = (1 + b M)^-1 b,  W = T (k G)   by forward substitution;   gla:  U = V
 //     O = (q G) S + A U,      S <- G_15 S + (k E)^T U.
 // scan_chunk_prep_kernel makes A, T, W, q G, k E of all chunks at once, in the order of the matrix operands: 16 threads per
-// s walk t with w in registers.  scan_chunk_kernel walks the chunks of a (segment, head, 16 value columns): four waves own a
-// quarter of the key channels of S each, in registers, the sums over channels meet in LDS, one barrier per chunk.
+// s walk t with w in registers.  scan_chunk_kernel walks the chunks of a (segment, head, 16 value columns): the waves (four, eight for
+// keys of 129 - 256) own equal parts of the key channels of S, in registers, the sums over channels meet in LDS, one barrier per chunk.
 // Bound by the f32 matrix rate where many (segment, head) pairs run (3 D P products per token), by the chain of 26 dependent
 // products per 16 tokens otherwise; the operands come three chunks ahead (one ahead: 144 against 125 us for the chain of 1500
 // tokens).  16 heads, values of 128, token form -> both launches here: delta, D = 128, segments of 1500, 40, 600, 1 and 1
@@ -841,8 +841,8 @@ int run_matrix_scan(const void* q, long sq, const void* k, long sk, const void* 
 }  // namespace
 
 // q, k [rows, G*D] and v [rows, H*P] slices of storage type dt (row strides sq, sk, sv); a f32 [T, H*D]
-// slice (row stride sa), OVERWRITTEN with the decays; a_bias f32 [H*D]; delta != 0: A_log f32 [H], beta
-// [T, >= H] slice of type beta_dt, aux f32 [T, 2*G + H] scratch; state f32 [slots, H, D, P]; out f32
+// slice (row stride sa), which the token form of longer segments overwrites with the decays; a_bias f32 [H*D]; delta != 0: A_log f32 [H], beta
+// [T, >= H] slice of type beta_dt, aux f32 [T, 2*G + H] scratch of that form; state f32 [slots, H, D, P]; out f32
 // [T, H*P].  T: rows of the step (every row belongs to a segment or is padding); max_len: the longest
 // segment (1: the decode form).  ws: f32 scratch of
 // (T / 16 + S) * H * scan_chunk_floats(D padded to 64, 128 or 256) values for the chunk form, or null (token form).

@@ -11,8 +11,8 @@
 //            dt = softplus(dt_raw + dt_bias[h]);  a = exp(-exp(A_log[h]) * dt)
 //            S <- a * S + dt * x_t (outer) B_t;   y_t = S C_t + D[h] * x_t
 //          u rows are laid out [x: H*P | B: G*N | C: G*N].
-//          Segments of SSD_LEAST tokens or more run in chunks of 64 on the f32 matrix instructions (ssd_scan_kernel),
-//          shorter ones token by token (ssm_scan_kernel).
+//          Steps with long segments, by the caller's choice, run those of SSD_LEAST tokens or more in chunks of 64 on the
+//          f32 matrix instructions (ssd_scan_kernel); all else goes token by token (ssm_scan_kernel).
 #include <type_traits>
 
 #include "mx_common.h"

@@ -734,7 +734,7 @@ def conv_act(inp: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], s
 # ----------------------------------------------------------------------------------------------
 # matrix-state linear recurrences (gated linear attention, gated delta rule)
 # ----------------------------------------------------------------------------------------------
-SCAN_CHUNK_LEAST = 32         # the longest segment from which the chunk form is taken (see SCAN_LEAST of the kernels)
+SCAN_CHUNK_LEAST = 32         # the longest segment from which the chunk form is possible (SCAN_LEAST of the kernels)
 
 
 def matrix_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.Tensor, a_bias: torch.Tensor,
@@ -751,7 +751,7 @@ def matrix_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.Tens
     ``mode="delta"``: q, k <- unit vectors (x / sqrt(sum x^2 + 1e-6)), q scaled by dim^-1/2;
                       g = exp(-exp(A_log[h]) softplus(a + a_bias));  b = sigmoid(beta[t, h]);
                       S <- g S;  u = b (v - S^T k);  S <- S + k u^T;  o = S^T q.
-    ``max_len``: the longest segment when known (1 selects the kernels' single-row form).
+    ``max_len``: the longest segment when known (1 selects the kernels' single-row form, left out the token form).
     Returns o f32 [T, H*vdim]."""
     T = q.shape[0]
     H, G, D, P = heads, kv_heads, dim, vdim
