@@ -338,15 +338,21 @@ PENNY_API int penny_encoder_pool(const void* x, const int* cu, int texts, int H,
 PENNY_API int penny_layernorm(const void* x, const void* res, const void* g, const void* b, void* y, int T, int H, float eps,
                               int add_residual, hipStream_t stream);
 
+constexpr int PENNY_MISALIGNED = -1;
+
 // All layers of a small batch: x [T, H] bf16 is replaced by the last layer's output.  w: 12 pointers per layer -- qkv, its
 // bias, o, its bias, the first norm's weight and bias, fc1, its bias, fc2, its bias, the second norm's weight and bias, each
 // contiguous bf16.  ws: T * (6 H + F) bf16.  Shapes as penny_gemm_bias_small, penny_encoder_attention and penny_layernorm take
-// them.  The launches of one layer take the host 8 x 2.5 us here and 8 x 7 from Python, where the kernels of a single query
+// them; PENNY_MISALIGNED, and nothing launched, for a weight off their 16 bytes (asked here: 144 weights take 18 us in Python).
+// The launches of one layer take the host 8 x 2.5 us here and 8 x 7 from Python, where the kernels of a single query
 // (18 tokens, 12 layers of 768) run for 440 us in all: 815 -> 497 us for the query.
 PENNY_API int penny_encoder_layers(const void* const* w, int layers, void* x, void* ws, const int* cu, int texts, int max_len,
                                    int T, int H, int heads, int F, float eps, float scale, hipStream_t stream) {
   if (T <= 0) return 0;
   if (heads < 1 || H % heads || H % 8 || F % 8) return (int)hipErrorInvalidValue;
+  size_t at = 0;
+  for (int i = 0; i < 12 * layers; ++i) at |= (size_t)w[i];
+  if (at % 16) return PENNY_MISALIGNED;
   bf16* qkv = static_cast<bf16*>(ws);
   bf16 *a = qkv + (long)T * 3 * H, *o = a + (long)T * H, *mid = o + (long)T * H, *h = mid + (long)T * H;
   int rc = 0;

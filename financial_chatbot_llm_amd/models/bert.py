@@ -92,14 +92,16 @@ class BertEncoder:
                 os.environ.get("PENNY_PREFILL_GEMM", "1") == "1"):
             return False
         w = [self.w[n] for n in self.layer_names]
-        if not all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.device == x.device and t.data_ptr() % 16 == 0 for t in w) or \
+        if not all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.device == x.device for t in w) or \
                 [t.shape for t in w] != self.layer_shapes:
             return False
         table = (ctypes.c_void_p * len(w))(*[t.data_ptr() for t in w])
         scratch = torch.empty(T * (6 * self.H + F_), dtype=torch.bfloat16, device=x.device)
-        N.call("penny_encoder_layers", table, self.cfg.num_layers, N.ptr(x), N.ptr(scratch), N.ptr(cu), cu.numel() - 1, longest,
-               T, self.H, self.nh, F_, float(self.cfg.norm_eps), 1.0 / math.sqrt(self.D), N.stream())
-        return True
+        rc = N.load().penny_encoder_layers(table, self.cfg.num_layers, N.ptr(x), N.ptr(scratch), N.ptr(cu), cu.numel() - 1, longest,
+                                           T, self.H, self.nh, F_, float(self.cfg.norm_eps), 1.0 / math.sqrt(self.D), N.stream())
+        if rc > 0:
+            raise RuntimeError(f"penny_encoder_layers failed with hipError {rc}")
+        return rc == 0                       # else a weight off the kernels' 16 bytes, and nothing was launched
 
     def _hidden(self, ids_list: Sequence[Sequence[int]]) -> Tuple[torch.Tensor, np.ndarray, torch.Tensor]:
         c, dev = self.cfg, self.device
