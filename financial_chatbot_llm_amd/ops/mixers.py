@@ -32,6 +32,7 @@ segment whose first row is at position 0 starts from zero state whatever its slo
 """
 from __future__ import annotations
 
+import functools
 from typing import NamedTuple, Optional, Tuple
 
 import torch
@@ -497,6 +498,24 @@ def _sink_softmax(sc: torch.Tensor, sink: Optional[torch.Tensor]) -> torch.Tenso
     return torch.softmax(torch.cat([sc, extra], -1), -1)[..., :-1]
 
 
+@functools.lru_cache(maxsize=1024)          # the estimate takes 1 - 5 us
+def _key_parts(keys: int, blocks: int, most_blocks: int, pairs: int, width: int, dtype: torch.dtype) -> int:
+    """How many blocks walk the keys of the same queries in the tiled attention (at most ``most_blocks`` over ``blocks``), for
+    ``keys`` a query block may see and ``pairs`` (row, head) results of ``width`` values.
+
+    The cheapest by an estimate in us: a walk of 0.75 per tile of 32 keys in bf16 and 2.8 in f32, once per 512 blocks, and with
+    parts a second launch that reads them all.  Unsplit / in 2 / as chosen (window 1 << 30, 16 heads over 4): 8 prompts of 100 rows
+    7.9 / 21.1 / 7.9, one of 1000 29 / 35 / 29, of 300 rows behind 600 beside 30 single rows 30.0 / 25.7 / 25.7, of 64 rows behind
+    836 25.5 / 18.3 / 15.4; one row behind 1000 25.3 / 17.3 / 13.7, behind 100 6.7 / 7.9 / 6.7; in f32 8 of 100 17.6 / 27.4 / 17.6,
+    one row behind 100 15.9 / 12.3 / 12.3."""
+    tiles = (keys + 31) // 32 + 1
+    walk, merge = 0.75 if dtype == torch.bfloat16 else 2.8, 1.84e-6 * pairs * (width + 2)
+
+    def cost(n: int) -> float:
+        return walk * tiles / n * max(1, -(-blocks * n // 512)) + (2.5 + 4e-4 * pairs + (merge + 0.5) * n if n > 1 else 0.0)
+    return min(range(1, max(1, min(16, tiles // 2, most_blocks // max(blocks, 1))) + 1), key=cost)
+
+
 def latent_attend(q_lat: torch.Tensor, q_rot: torch.Tensor, cache: torch.Tensor, cu: torch.Tensor, pos: torch.Tensor,
                   bt: torch.Tensor, window: int, scale: float, max_len: int,
                   gate: Optional[torch.Tensor] = None, sink: Optional[torch.Tensor] = None,
@@ -515,16 +534,18 @@ def latent_attend(q_lat: torch.Tensor, q_rot: torch.Tensor, cache: torch.Tensor,
     if N.use_native(q_lat):
         assert q_lat.is_contiguous() and q_rot.is_contiguous() and bt.is_contiguous()
         out = torch.empty((T, H, R), dtype=q_lat.dtype, device=q_lat.device)
-        # steps whose blocks (64 pairs of a row and a head) would leave the chip idle walk each row's keys with several
+        # steps whose blocks (64 pairs of a row and a head) would leave the chip idle may walk each row's keys with several
         # blocks; the split depends only on static sizes (graph-safe).  R = 256 (64 keys per tile, two blocks per CU; 32
-        # heads, window 1024): 64 single rows take 24 us with 256 blocks, 42 with 1024; 256 rows of one segment and 30 single
-        # ones 72 us unsplit, 69 with 512 blocks
+        # heads, window 1024): 64 single rows take 24 us with 256 blocks, 42 with 1024
         nsplit, ws = 1, None
-        if q_lat.dtype == torch.bfloat16 and (max_len == 1 or (R == 256 and Dr in (0, 32))):
-            tiles = (min(window + max_len, bt.shape[1] * PAGE) + 31) // 32 + 1
+        tiled = R == 256 and Dr in (0, 32)
+        if q_lat.dtype == torch.bfloat16 and (max_len == 1 or tiled):
+            keys = min(window + min(max_len, 64), bt.shape[1] * PAGE)      # a block's rows are 64 at most
             blocks = S * ((H + 63) // 64) if max_len == 1 else S + T * H // 64
-            want = 512 if max_len > 1 else 256 if R == 256 and Dr in (0, 32) else 1024
-            nsplit = max(1, min(16, tiles // 2, want // max(blocks, 1)))
+            if tiled:
+                nsplit = _key_parts(keys, blocks, 512 if max_len > 1 else 256, T * H, R, q_lat.dtype)
+            else:
+                nsplit = max(1, min(16, ((keys + 31) // 32 + 1) // 2, 1024 // max(blocks, 1)))
             if nsplit > 1:
                 ws = torch.empty((T, H, nsplit, R + 2), dtype=torch.float32, device=q_lat.device)
         N.mcall("mx_latent_attend", N.ptr(q_lat), N.ptr(q_rot), N.ptr(cache), N.ptr(cu), N.ptr(pos), N.ptr(bt),
@@ -1058,16 +1079,20 @@ def window_attend(q: torch.Tensor, cache: torch.Tensor, cu: torch.Tensor, pos: t
     if N.use_native(q):
         assert bt.is_contiguous() and q.dtype == cache.dtype
         out = torch.empty((T, H * P), dtype=q.dtype, device=q.device)
-        # steps whose blocks (64 pairs of a row and a head of one group) would leave the chip idle walk each row's keys with
-        # several blocks; the split depends only on static sizes (graph-safe).  Single rows want 1024 blocks (48 rows of 16
+        # steps whose blocks (64 pairs of a row and a head of one group) would leave the chip idle may walk each row's keys with
+        # several blocks; the split depends only on static sizes (graph-safe).  Single rows may take 1024 blocks (48 rows of 16
         # heads over 4, window 1024: 25 us, at 256 blocks 39); with longer segments merging the parts costs more, and 512
         # are enough (577 rows in f32: 34 us at 468 blocks)
         nsplit, ws = 1, None
         tiled = D == 128 and P == 128 and head_bias is None and rel is None
         if tiled or (max_len == 1 and q.dtype == torch.bfloat16):
-            tiles = (min(window + keep_first + max_len, bt.shape[1] * PAGE) + 31) // 32 + 1
+            keys = min(window + keep_first + min(max_len, 64), bt.shape[1] * PAGE)     # a block's rows are 64 at most
             blocks = S * G if max_len == 1 else (S + T * (H // G) // 64) * G
-            nsplit = max(1, min(16, tiles // 2, (1024 if max_len == 1 else 512) // max(blocks, 1)))
+            most = 1024 if max_len == 1 else 512
+            if tiled:
+                nsplit = _key_parts(keys, blocks, most, T * H, P, q.dtype)
+            else:
+                nsplit = max(1, min(16, ((keys + 31) // 32 + 1) // 2, most // max(blocks, 1)))
             if nsplit > 1:
                 ws = torch.empty((T, H, nsplit, P + 2), dtype=torch.float32, device=q.device)
         N.mcall("mx_window_attend", N.ptr(_rows(q)), q.stride(0), N.ptr(cache), N.ptr(cu), N.ptr(pos), N.ptr(bt), bt.shape[1],

@@ -144,3 +144,27 @@ def test_latent_not_finite():
     got = run(lambda t: t.cuda(), cache).cpu()
     check(got[~sees], want[~sees], dt, 2.0 ** -9)
     assert not torch.isfinite(got[sees].float()).any()
+
+
+def test_parts_follow_the_walk():
+    """Steps of which each split was measured faster: (rows, context) of the segments, 16 heads over 4, window 1 << 30."""
+    bf, f32 = torch.bfloat16, torch.float32
+
+    def parts(segs, dt):
+        T, S, longest, pages_ = sum(n for n, _ in segs), len(segs), max(n for n, _ in segs), max((c + 63) // 64 for _, c in segs)
+        blocks = S * 4 if longest == 1 else (S + T * 4 // 64) * 4
+        return mx._key_parts(pages_ * 64, blocks, 1024 if longest == 1 else 512, T * 16, 128, dt)
+    for segs in ([(100, 100)] * 8, [(100, 100)], [(512, 512)], [(1000, 1000)], [(40, 40)] * 16, [(1, 100)] * 8):
+        assert parts(segs, bf) == 1, segs
+    assert parts([(100, 100)] * 8, f32) == parts([(33, 33)], f32) == 1
+    assert parts([(300, 900)] + [(1, 700)] * 30, bf) == parts([(1, 100)], f32) == 2
+    assert 3 <= parts([(64, 900)], bf) <= 6 and 4 <= parts([(1, 1000)], bf) <= 8 and parts([(64, 900)], f32) >= 6
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("nsplit", [1, 2, 5, 16])
+def test_any_number_of_parts(dt, nsplit, monkeypatch):
+    """More parts than a row has tiles among them: those are empty."""
+    monkeypatch.setattr(mx, "_key_parts", lambda *a: nsplit)
+    test_window(dt, LONG, (6, 2), {"window": 63, "keep_first": 5})
+    test_window(dt, SINGLES, (8, 1), {"window": 130, "keep_first": 70, "gate": "head", "sink": True})
