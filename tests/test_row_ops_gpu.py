@@ -97,6 +97,14 @@ def test_relu2(dt, pad, off, n):
 
 
 @pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("n", [120, 128, 252, 256])
+def test_relu2_of_narrow_rows(dt, n):
+    """On both sides of the widths from which rows go by 16 bytes."""
+    x = rand(torch.Generator().manual_seed(n), 300, n, dt=dt)
+    assert torch.equal(mx.relu2(x.cuda()).cpu(), mx.relu2(x))
+
+
+@pytest.mark.parametrize("dt", DTS)
 @pytest.mark.parametrize("pad", [0, 4, 1])
 @pytest.mark.parametrize("C,K", [(4, 4), (1028, 4), (30, 4), (64, 3)])
 def test_conv(dt, pad, C, K):
