@@ -1,9 +1,9 @@
 // BERT / bge encoder (K14) kernels of their own: bidirectional attention straight over the packed QKV rows, and the
 // biased projections of small batches.
 //
-//   penny_encoder_attention   every text attends within itself; texts are short (a query or a transaction: 6 - 128
-//                             tokens), so a 64-token tile of one (text, head) is a whole problem and no paged cache is
-//                             written first.
+//   penny_encoder_attention   every text attends within itself; most are short (a query or a transaction: 6 - 128
+//                             tokens), so a 64-token tile of one (text, head) is about a whole problem, and no paged cache
+//                             is written first.
 //   penny_gemm_bias_small     bf16(x w^T + b) [-> exact GELU] for up to a few hundred rows.
 //   penny_encoder_embed       word + position + type rows and their layer norm in one pass.
 //   penny_encoder_layers      the launches of all layers of a small batch, from one call.
@@ -26,6 +26,9 @@ __device__ __forceinline__ f32x4 mfma16(const bf16x8& a, const bf16x8& b, const 
 // in base 2, O^T += V^T P^T with the value tile transposed in LDS and P straight from the score registers (K slot 8 g + i
 // holds keys 4 g + i and 16 + 4 g + i).  Bound by the QKV rows read and the output written: 1024 texts of 6 - 64 tokens
 // (36k), 12 heads of 64: 61 us (3.6 TB/s); the paged form took 202 us for the cache write and 72 us for the attention.
+// Longer texts read each other's keys once per 64 queries and wave, without prefetch: the attention alone is slower than the
+// paged one from 64 tokens on, but not with its cache write (32,768 tokens, us, write + paged / this: texts of 128 239 + 39 / 75, of
+// 256 236 + 65 / 125, of 512 237 + 100 / 227; 8 texts of 512 25 + 20 / 38).
 template <int D>
 __global__ void __launch_bounds__(256) encoder_attention_kernel(const bf16* __restrict__ qkv, long ld,
                                                                 const int* __restrict__ cu, int H, float scale_log2,
