@@ -14,8 +14,8 @@
 // Bound by the LDS reads of the operands and the vector instructions of the softmax (four segments of 2048 rows, 16 heads
 // over 4, window 1024: 127 us, 0.6 PFLOP/s with the second weight term).  16 pairs per wave (MB = 1): 32 halve the operand
 // reads but leave two waves per SIMD (bf16 heads of 128: 56 against 43 us for 1190 rows) or spill (latent: 108 against 65).
-// A block's serial walk is what a small step waits for: the launcher splits the keys over nsplit blocks then
-// (unnormalised parts: o | m | l, merged afterwards).
+// A block's serial walk is what a small step waits for: the caller splits the keys over nsplit blocks where that is shorter
+// than reading the parts back (unnormalised: o | m | l, merged afterwards).
 #pragma once
 #include "mx_common.h"
 
