@@ -134,6 +134,72 @@ __global__ void __launch_bounds__(1024) expert_plan_kernel(const int* __restrict
   }
 }
 
+// The same plan by one block per expert, for more pairs than one block sorts in the time of a launch.  Every block counts all
+// pairs (LDS atomics into a row of bins per wave), so it knows its expert's first row and tile without the other blocks, and
+// then places its own expert's pairs: one ballot per chunk of 64 instead of one per bit of the index.  Same pos, src and tiles
+// as above.  Bound by the latency of reading the indices and of the count.  Us in one block / here, 32 experts: 20,260 pairs
+// 30.7 / 9.6, 4,736: 10.5 / 4.9, 2,048: 4.6 / 4.1, 1,536: 4.5 / 4.0, 1,024 and fewer: alike; 8 and 256 experts draw the same
+// line (1,024 pairs 3.8 / 3.8 and 6.6 / 6.6, 4,096: 7.6 / 4.7 and 13.8 / 4.8).  LDS: cnt [16][E], total [E].
+template <int NC>
+__global__ void __launch_bounds__(1024) expert_plan_wide_kernel(const int* __restrict__ idx, int P, int E, int mt, int ntiles,
+                                                                int* __restrict__ pos, int* __restrict__ src,
+                                                                int4* __restrict__ tiles) {
+  extern __shared__ int lds[];
+  __shared__ int own[4];                                     // first row, first tile, rows, tiles of all experts
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, me = blockIdx.x;
+  int* cnt = lds + w * E;
+  int* total = lds + 16 * E;
+  const int i0 = w * NC * 64 + lane;
+  int held[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) held[c] = i0 + c * 64 < P ? idx[i0 + c * 64] : -1;
+  for (int e = threadIdx.x; e < 16 * E; e += 1024) lds[e] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+    if ((unsigned)held[c] < (unsigned)E) atomicAdd(cnt + held[c], 1);
+  __syncthreads();
+  for (int e = threadIdx.x; e < E; e += 1024) {
+    int t = 0;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) t += lds[v * E + e];
+    total[e] = t;
+  }
+  __syncthreads();
+  if (w == 0) {
+    int rows = 0, nt = 0;                                    // of the experts before this one
+    int all = 0;
+    for (int e = lane; e < E; e += 64) {
+      const int c = total[e], t = (c + mt - 1) / mt;
+      if (e < me) rows += c, nt += t;
+      all += t;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) rows += __shfl_xor(rows, o, 64), nt += __shfl_xor(nt, o, 64), all += __shfl_xor(all, o, 64);
+    if (lane == 0) own[0] = rows, own[1] = nt, own[2] = total[me], own[3] = all;
+  }
+  __syncthreads();
+  const int row0 = own[0], tile0 = own[1], n = own[2], all = own[3];
+  for (int k = threadIdx.x; k * mt < n; k += 1024)
+    if (tile0 + k < ntiles) tiles[tile0 + k] = make_int4(me, row0 + k * mt, min(mt, n - k * mt), 0);
+  if (me == 0)
+    for (int t = all + threadIdx.x; t < ntiles; t += 1024) tiles[t] = make_int4(0, 0, 0, 0);
+  int at = row0;
+  for (int v = 0; v < w; ++v) at += lds[v * E + me];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const unsigned long long m = __ballot(held[c] == me);
+    if (held[c] == me) {
+      const int r = at + __popcll(m & ((1ull << lane) - 1));
+      pos[i0 + c * 64] = r;
+      src[r] = i0 + c * 64;
+    } else if (me == 0 && held[c] >= E) {
+      pos[i0 + c * 64] = 0;
+    }
+    at += __popcll(m);
+  }
+}
+
 __device__ __forceinline__ float unit_value(int unit, float g, float u, float limit, float alpha) {
   if (unit == UNIT_CLAMP) {
     g = fminf(g, limit);
@@ -412,6 +478,8 @@ MX_API int mx_experts(const void* h, long ldh, const int* idx, int T, int top, i
   int* pos = iws;
   int* src = iws + (P + 3) / 4 * 4;
   int4* tiles = reinterpret_cast<int4*>(src + (P + 3) / 4 * 4);
+  // one block per expert beyond 1024 pairs (every block reads them all: up to 512 experts, 35 KB of counts)
+  const bool wide = P > 1024 && P <= 32 * 1024 && E <= 512;
   int bits = 0;
   while ((1 << bits) < E) ++bits;
   int nw = (int)((P + 63) / 64);
@@ -420,11 +488,17 @@ MX_API int mx_experts(const void* h, long ldh, const int* idx, int T, int top, i
   const long run = (P + nw * 64 - 1) / (nw * 64);            // chunks of 64 pairs per wave
   const size_t lds = (size_t)(nw + 1) * E * 4;
 #define PLAN(NC) expert_plan_kernel<NC><<<1, nw * 64, lds, st>>>(idx, (int)P, E, bits, mt, ntiles, pos, src, tiles)
-  if (run <= 2) PLAN(2);
+#define WIDE(NC) expert_plan_wide_kernel<NC><<<E, 1024, (size_t)17 * E * 4, st>>>(idx, (int)P, E, mt, ntiles, pos, src, tiles)
+  if (wide && P <= 4 * 1024) WIDE(4);
+  else if (wide && P <= 8 * 1024) WIDE(8);
+  else if (wide && P <= 16 * 1024) WIDE(16);
+  else if (wide) WIDE(32);
+  else if (run <= 2) PLAN(2);
   else if (run <= 8) PLAN(8);
   else if (run <= 16) PLAN(16);
   else if (run <= 32) PLAN(32);
   else PLAN(0);
+#undef WIDE
 #undef PLAN
   int rc = (int)hipGetLastError();
   if (rc) return rc;

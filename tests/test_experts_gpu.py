@@ -118,3 +118,24 @@ def test_most_experts(E):
 ])
 def test_few_experts(dtype, T, W, F_, E, top, unit):
     check(dtype, T, W, F_, E, top, unit)
+
+
+@pytest.mark.parametrize("E", [1, 3, 64, 65, 512, 513])
+@pytest.mark.parametrize("T", [256, 257, 1023, 1025, 2049, 4097, 8192, 8193])
+def test_expert_plan_is_the_stable_sort(E, T):
+    """One block (512 experts or 1024 pairs and fewer, 32768 and more) and a block per expert: every pair's place is that of the
+    stable sort by expert, identity experts behind; some experts get no pair, one may get nearly all."""
+    from financial_chatbot_llm_amd.ops import mixers as mx
+    top, W = 4, 8
+    g = torch.Generator().manual_seed(T + E)
+    for skew in (False, True):
+        idx = torch.randint(0, E + 2, (T, top), generator=g)
+        if skew:
+            idx = torch.where(torch.rand(T, top, generator=g) < 0.9, E // 2, idx)
+        w1 = mx.pack_experts([torch.ones(8, W, device="cuda")] * E, torch.float32)
+        w2 = mx.pack_experts([torch.ones(W, 8, device="cuda")] * E, torch.float32)
+        _, pos = mx.experts(torch.ones(T, W, device="cuda"), idx.int().cuda(), w1, w2, "relu2")
+        flat = idx.flatten()
+        want = torch.empty(T * top, dtype=torch.int32)
+        want[torch.argsort(flat, stable=True)] = torch.arange(T * top, dtype=torch.int32)
+        assert torch.equal(pos.cpu().flatten(), torch.where(flat < E, want, 0))
