@@ -433,8 +433,9 @@ latent_attend_mfma_kernel(const bf16* __restrict__ q_lat, const bf16* __restrict
 }
 
 // grid (rows, H): combine the nsplit parts of one (row, head)
-__global__ void latent_merge_kernel(const float* __restrict__ ws, const bf16* __restrict__ gate, long sgate,
-                                    const float* __restrict__ sink, bf16* __restrict__ out, int H, int R, int nsplit) {
+template <typename T>
+__global__ void latent_merge_kernel(const float* __restrict__ ws, const T* __restrict__ gate, long sgate,
+                                    const float* __restrict__ sink, T* __restrict__ out, int H, int R, int nsplit) {
   const long row = blockIdx.x;
   const int h = blockIdx.y;
   const float* w = ws + (row * H + h) * nsplit * (long)(R + 2);
@@ -446,14 +447,14 @@ __global__ void latent_merge_kernel(const float* __restrict__ ws, const bf16* __
     if (mi != -INFINITY) L += w[i * (R + 2) + R + 1] * expf(mi - M);
   }
   float gsc = 1.0f / L;
-  if (gate != nullptr) gsc *= mx_sigmoid((float)gate[row * sgate + h]);
+  if (gate != nullptr) gsc *= mx_sigmoid(ldf(gate + row * sgate + h));
   for (int r = threadIdx.x; r < R; r += blockDim.x) {
     float a = 0.f;
     for (int i = 0; i < nsplit; ++i) {
       const float mi = w[i * (R + 2) + R];
       if (mi != -INFINITY) a += w[i * (R + 2) + r] * expf(mi - M);
     }
-    out[(row * H + h) * R + r] = (bf16)(a * gsc);
+    stf(out + (row * H + h) * R + r, a * gsc);
   }
 }
 
@@ -488,7 +489,7 @@ MX_API int mx_latent_prep(const void* kv, long skv, const float* norm_w, float e
 // pos [T] positions, bt [S, btw] page tables; gate [T, >=H] slice (row stride sgate) or null; sink f32 [H] or
 // null.  exact != 0: the softmax weights enter the value product of the matrix-core form as two bf16 terms.
 // nsplit > 1 with a workspace ws (f32 [rows, H, nsplit, R + 2]): the keys of each row are walked by nsplit blocks and
-// merged (rows_attend.h; the older matrix-core form does so for single-row segments only, the f32-lane form never).
+// merged (rows_attend.h, bf16 and f32; the older matrix-core form does so for single-row segments only, the f32-lane form never).
 MX_API int mx_latent_attend(const void* q_lat, const void* q_rot, const void* cache, const int* cu, const int* pos,
                             const int* bt, int btw, const void* gate, long sgate, const float* sink, int exact,
                             int window, float scale, void* out, int dt, int S, int max_len, int H, int R, int Dr,
@@ -496,17 +497,22 @@ MX_API int mx_latent_attend(const void* q_lat, const void* q_rot, const void* ca
   if (S <= 0 || max_len <= 0) return 0;
   if (R > 64 * ATT_RPL) return (int)hipErrorInvalidValue;
   const int D = R + Dr;
-  // rows_attend.h for the latent of 256 with a rotated part of 32 or none, the sizes of this framework's decoders (32 heads,
-  // window 1024, before -> after: 2048 rows of three segments 217 -> 64 us, 256 rows and 30 single ones 405 -> 75, 64 single
-  // rows 85 -> 24, 4 single rows 32 -> 19)
-  if (dt == 0 && R == 256 && (Dr == 32 || Dr == 0) && mx_use_mfma() &&
+  // rows_attend.h for the latent of 256 with a rotated part of 32 or none, the sizes of this framework's decoders (window 1024,
+  // before -> after; 32 heads, bf16: 2048 rows of three segments 217 -> 64 us, 256 rows and 30 single ones 405 -> 75, 64 single
+  // rows 85 -> 24, 4 single rows 32 -> 19; 8 heads, f32, where the walk is a chain of f32 products: 2 single rows behind 1443
+  // 572 -> 42, 64 behind 1100 737 -> 93, three times 200 rows behind 692 1457 -> 103, 24 rows alone 55 -> 16; 32 heads, f32,
+  // twice 2048 rows 13.7 -> 1.28 ms)
+  if (R == 256 && (Dr == 32 || Dr == 0) && mx_use_mfma() &&
       ((size_t)q_lat | (size_t)q_rot | (size_t)cache | (size_t)out) % 16 == 0 && window <= (1 << 30)) {
     if (ws == nullptr || nsplit < 1) nsplit = 1;
     const int HB = H < 64 ? H : 64, QT = max_len == 1 ? 1 : 64 / HB;
     RowsArgs a{q_lat, q_rot, (long)H * R, cache, D, 0, 0, 0, cu, pos, bt, btw, gate, sgate, 0, window, 0, 0,
                nullptr, 0.f, sink, scale, out, H, 1, QT, HB, nsplit, ws};
     const dim3 grid((unsigned)((max_len + QT - 1) / QT * nsplit), (H + HB - 1) / HB, S);
-    if (Dr == 32) {
+    if (dt == 1) {
+      if (Dr == 32) rows_attend_kernel<float, 256, 32, 256, true, 1, 4, 32, false, false><<<grid, 256, 0, st>>>(a);
+      else rows_attend_kernel<float, 256, 0, 256, true, 1, 4, 32, false, false><<<grid, 256, 0, st>>>(a);
+    } else if (Dr == 32) {
       if (exact) rows_attend_kernel<bf16, 256, 32, 256, true, 1, 4, 64, false, true><<<grid, 256, 0, st>>>(a);
       else rows_attend_kernel<bf16, 256, 32, 256, true, 1, 4, 64, false, false><<<grid, 256, 0, st>>>(a);
     } else {
@@ -514,7 +520,8 @@ MX_API int mx_latent_attend(const void* q_lat, const void* q_rot, const void* ca
       else rows_attend_kernel<bf16, 256, 0, 256, true, 1, 4, 64, false, false><<<grid, 256, 0, st>>>(a);
     }
     if (nsplit > 1)
-      latent_merge_kernel<<<dim3(rows, H), 128, 0, st>>>(ws, (const bf16*)gate, sgate, sink, (bf16*)out, H, R, nsplit);
+      MX_DISPATCH(dt, TT, latent_merge_kernel<TT><<<dim3(rows, H), 128, 0, st>>>(ws, (const TT*)gate, sgate, sink, (TT*)out, H,
+                                                                                R, nsplit));
     MX_RETURN_LAUNCH();
   }
   if (dt == 0 && D <= 320 && R <= 256 && mx_use_mfma()) {
@@ -539,7 +546,7 @@ MX_API int mx_latent_attend(const void* q_lat, const void* q_rot, const void* ca
 #undef LATENT_LAUNCH
     if (nsplit > 1) {
       dim3 g2(S, H);           // single-row segments: row index == segment index
-      latent_merge_kernel<<<g2, R >= 128 ? 128 : 64, 0, st>>>(ws, (const bf16*)gate, sgate, sink, (bf16*)out, H, R, nsplit);
+      latent_merge_kernel<bf16><<<g2, R >= 128 ? 128 : 64, 0, st>>>(ws, (const bf16*)gate, sgate, sink, (bf16*)out, H, R, nsplit);
     }
     MX_RETURN_LAUNCH();
   }

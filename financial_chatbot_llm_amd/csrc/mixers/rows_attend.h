@@ -63,9 +63,11 @@ __device__ __forceinline__ float rows_sum4(float v) {
 // chunk swizzle of a tile row (CH 16-byte chunks per row): chunk c lies at c ^ z(row).
 // Rows of whole 256 bytes: 16 rows at one chunk (key reads) meet 16 different ones; bf16: rows 4 g .. 4 g + 7 at a pair of
 // chunks (transposed value reads) different pairs; f32: rows 0, 4, 8, 12 at four chunks (value reads) different fours.
-// 576-byte rows are 64 bytes apart in the banks by themselves: two bits do.
+// 576-byte rows are 64 bytes apart in the banks by themselves: two bits do.  1152-byte rows (f32) are 128 bytes apart: three
+// bits of the row pair; value reads then meet in pairs, which the f32 products they feed hide.
 template <int CH, int ES> __device__ __forceinline__ int rows_swz(int row) {
   if (CH % 16 == 0) return ES == 2 ? ((row & 7) << 1) ^ ((row >> 3) & 1) : (((row >> 2) & 3) << 2) | (row & 3);
+  if (CH % 8 == 0) return (row >> 1) & 7;
   return ((row >> 3) & 1) | ((row >> 1) & 2);
 }
 

@@ -539,7 +539,7 @@ def latent_attend(q_lat: torch.Tensor, q_rot: torch.Tensor, cache: torch.Tensor,
         # heads, window 1024): 64 single rows take 24 us with 256 blocks, 42 with 1024
         nsplit, ws = 1, None
         tiled = R == 256 and Dr in (0, 32)
-        if q_lat.dtype == torch.bfloat16 and (max_len == 1 or tiled):
+        if tiled or (q_lat.dtype == torch.bfloat16 and max_len == 1):
             keys = min(window + min(max_len, 64), bt.shape[1] * PAGE)      # a block's rows are 64 at most
             blocks = S * ((H + 63) // 64) if max_len == 1 else S + T * H // 64
             if tiled:

@@ -168,3 +168,20 @@ def test_any_number_of_parts(dt, nsplit, monkeypatch):
     monkeypatch.setattr(mx, "_key_parts", lambda *a: nsplit)
     test_window(dt, LONG, (6, 2), {"window": 63, "keep_first": 5})
     test_window(dt, SINGLES, (8, 1), {"window": 130, "keep_first": 70, "gate": "head", "sink": True})
+
+
+@pytest.mark.parametrize("segs", [SINGLES, RAGGED, LONG], ids=["singles", "ragged", "long"])
+@pytest.mark.parametrize("H,Dr,window", [(1, 32, 1), (8, 32, 1024), (70, 0, 1 << 40), (3, 0, 64), (32, 32, 65)])
+def test_latent_f32(segs, H, Dr, window):
+    g = torch.Generator().manual_seed(16)
+    dt, R = torch.float32, 256
+    cu, pos, bt, total = pages(segs, g)
+    T = int(cu[-1])
+    cache = rows(segs, bt, total, R + Dr, dt, g)
+    ql, qr = (torch.randn((T, H, n), generator=g).to(dt) for n in (R, Dr))
+    gate, sink = torch.randn((T, H), generator=g), torch.randn(H, generator=g)
+
+    def run(f):
+        return mx.latent_attend(f(ql), f(qr), f(cache), f(cu), f(pos), f(bt), window, R ** -0.5, max(n for n, _ in segs),
+                                gate=f(gate), sink=f(sink) if H > 1 else None)
+    check(run(lambda t: t.cuda()), run(lambda t: t), dt)
