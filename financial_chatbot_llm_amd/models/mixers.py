@@ -361,10 +361,9 @@ class RoutedFF:
             shared = F.linear(mx.glu_clamp(proj[:, :self.Fs], proj[:, self.Fs:2 * self.Fs], self.limit_s, self.alpha),
                               self.down_s)
         if self.score == "softmax_top":
-            wts, idx = mx.route_scores(F.linear(h.float(), self.router, self.correction), top, "softmax_top")
+            wts, idx = mx.router_scores(h, self.router, self.correction, top, "softmax_top")
         else:
-            wts, idx = mx.route_biased(F.linear(h.float(), self.router), self.correction, top, self.score, self.renorm,
-                                       self.w_scale)
+            wts, idx = mx.router_biased(h, self.router, self.correction, top, self.score, self.renorm, self.w_scale)
         ys, pos = self.bank.run(h, idx, "clamped", self.limit, self.alpha)
         return mx.moe_combine(ys, pos, idx, wts, h, shared, self.E)
 
@@ -406,7 +405,7 @@ class InputScaledRoutedFF:
     def forward(self, h: torch.Tensor, proj: Optional[torch.Tensor] = None, x32: Optional[torch.Tensor] = None) -> torch.Tensor:
         """``x32``: the f32 input ``h`` was rounded from, when the caller has it: the router then reads the
         unrounded values (fewer swapped near-ties against an exact evaluation)."""
-        wts, idx = mx.route_scores(F.linear(x32 if x32 is not None else h.float(), self.router), self.top, self.score)
+        wts, idx = mx.router_scores(x32 if x32 is not None else h, self.router, None, self.top, self.score)
         ys, pos = self.bank.run(h, idx, self.act, scale=wts)
         return mx.moe_combine(ys, pos, idx, None, h, None, self.E)
 
@@ -450,7 +449,7 @@ class TopSoftmaxRoutedFF:
 
     def forward(self, h: torch.Tensor, proj: Optional[torch.Tensor] = None, x32: Optional[torch.Tensor] = None) -> torch.Tensor:
         shared = F.linear(mx.relu2(proj[:, :self.Fs]), self.down_s) if self.Fs else None
-        wts, idx = mx.route_scores(F.linear(x32 if x32 is not None else h.float(), self.router), self.top, "softmax_top")
+        wts, idx = mx.router_scores(x32 if x32 is not None else h, self.router, None, self.top, "softmax_top")
         ys, pos = self.bank.run(h, idx, "relu2")
         return mx.moe_combine(ys, pos, idx, wts, h, shared, self.E)
 
