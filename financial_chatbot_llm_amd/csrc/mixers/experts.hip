@@ -37,7 +37,7 @@ struct ExpertGemm {
   int kbytes;           // bytes of a row that count
   const int* src;       // sorted row -> pair
   int top;
-  const int4* tiles;    // (expert, first sorted row, rows, -); rows 0: none
+  const int4* tiles;    // (expert, first sorted row, rows, -), then entries without rows; the first one's w: how many have rows
   int ntiles;           // entries of the list
   const char* w;        // pieces, expert stride wstride bytes
   long wstride;
@@ -115,6 +115,7 @@ __global__ void __launch_bounds__(1024) expert_plan_kernel(const int* __restrict
       nt += __shfl(st, 63, 64);
     }
     for (int t = nt + lane; t < ntiles; t += 64) tiles[t] = make_int4(0, 0, 0, 0);
+    if (lane == 0) tiles[0].w = nt;
   }
   __syncthreads();
 #pragma unroll
@@ -181,7 +182,7 @@ __global__ void __launch_bounds__(1024) expert_plan_wide_kernel(const int* __res
   __syncthreads();
   const int row0 = own[0], tile0 = own[1], n = own[2], all = own[3];
   for (int k = threadIdx.x; k * mt < n; k += 1024)
-    if (tile0 + k < ntiles) tiles[tile0 + k] = make_int4(me, row0 + k * mt, min(mt, n - k * mt), 0);
+    if (tile0 + k < ntiles) tiles[tile0 + k] = make_int4(me, row0 + k * mt, min(mt, n - k * mt), tile0 + k == 0 ? all : 0);
   if (me == 0)
     for (int t = all + threadIdx.x; t < ntiles; t += 1024) tiles[t] = make_int4(0, 0, 0, 0);
   int at = row0;
@@ -242,6 +243,22 @@ __device__ __forceinline__ const char* expert_row(const ExpertGemm& a, int r, in
   return static_cast<const char*>(a.x) + (a.top > 0 ? a.src[r] / a.top : r) * a.ldx * es;
 }
 
+// (tile, column block) of this block among `cols` column blocks, or false.  Every XCD takes an equal run of the tiles that have
+// rows, in groups of four neighbouring ones -- mostly one expert's -- through all column blocks in turn, so that their W panels
+// and token rows meet in its L2.  (Fixed groups dealt to the XCDs leave some of them idle: 16 tiles of 256 rows by 16 column
+// blocks ran on four.)
+__device__ __forceinline__ bool expert_place(const ExpertGemm& a, int cols, int& t, int& nb) {
+  const int live = a.tiles[0].w, nwg = live * cols;
+  int id = blockIdx.x;
+  if (id >= nwg) return false;
+  const int xcd = id & 7, q = nwg >> 3, r = nwg & 7;
+  id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (id >> 3);
+  const int grp = id / (4 * cols), in = id - grp * 4 * cols, gm = min(live - 4 * grp, 4);
+  t = 4 * grp + in % gm;
+  nb = in / gm;
+  return true;
+}
+
 // ---- tile form ---------------------------------------------------------------------------------------------------
 // 256 threads = 4 waves as 2 (W rows) x 2 (tokens), a wave's 64 x 16 MF sub-tile as 4 x MF accumulators (A = W: a
 // lane's four registers are adjacent output columns).  A stage is 128 bytes of K: the W image keeps the pieces'
@@ -253,14 +270,10 @@ __global__ void __launch_bounds__(256, MF == 4 ? 2 : 3) expert_tile_kernel(Exper
   __shared__ __attribute__((aligned(1024))) char smem[2 * STG];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wa = w >> 1, wb = w & 1, g = lane >> 4, col = lane & 15;
-  // four neighbouring tiles -- mostly one expert's -- take all column blocks in turn on one XCD: their W panels and
-  // token rows meet in its L2; the groups of four go round the XCDs, as the end of the list is empty
-  const int nt = (a.groups + 7) / 8, per = 4 * nt, local = blockIdx.x >> 3;
-  const int t = ((local / per) * 8 + (blockIdx.x & 7)) * 4 + (local % per) % 4, nb = (local % per) / 4;
-  if (t >= a.ntiles) return;
+  int t, nb;
+  if (!expert_place(a, (a.groups + 7) / 8, t, nb)) return;
   const int4 tile = a.tiles[t];
   const int rows = tile.z;
-  if (rows == 0) return;
 
   const char* wsrc[4];
 #pragma unroll
@@ -434,7 +447,7 @@ int tile_rows(long pairs, int experts, int dt, double bytes, int stages, int col
 template <typename T, bool GLU>
 int expert_launch(const ExpertGemm& a, int mt, hipStream_t st) {
   if (mt >= 64) {
-    const long grid = (long)((a.ntiles + 31) / 32) * 32 * ((a.groups + 7) / 8);
+    const long grid = (long)a.ntiles * ((a.groups + 7) / 8);
     if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
     if constexpr (sizeof(T) == 2) {
       if (mt == 128) {
