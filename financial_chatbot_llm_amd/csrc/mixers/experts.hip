@@ -10,14 +10,18 @@
 // Both storage types share the code: a 16-byte operand is 8 bf16 (one 16x16x32 MFMA) or 4 f32 (four 16x16x4 MFMAs whose
 // step j takes K element 4 g + j of both operands).  Accumulation is f32; the unit sees the f32 sums.
 //
-// Two forms, chosen by the rows an expert gets on average (the bucket sizes stay on the device):
+// Three forms, chosen by the rows an expert gets on average (the bucket sizes stay on the device):
 //   tile    128 W rows x 64 or 128 tokens per block, both operands through a two-stage LDS ring filled by LDS-DMA,
-//           two or three blocks per CU: bound by the matrix cores.  4096 tokens, width 2048, 32 experts of 1024, top 4,
-//           bf16: 320 us for both products (650 TFLOP/s); 31 pairs of library products and the host's wait for the
+//           two or three blocks per CU: bound by the operand reads.  4096 tokens, width 2048, 32 experts of 1024, top 4,
+//           bf16: 300 us for both products (650 TFLOP/s); 31 pairs of library products and the host's wait for the
 //           bucket sizes took 1.3 ms.
+//   wide    256 W rows x 256 tokens per block, bf16: bound by the matrix cores and, with few rounds of blocks, by the last one
+//           (5065 tokens of the same layer: 366 -> 315 us, 8192: 515 -> 420, 930 TFLOP/s).
 //   stream  32 or 64 W rows x 16 tokens per block, the four waves split K and the weights go straight to registers,
 //           1 KiB per load: bound by the weight stream.  64 tokens of the same layer: 49 + 23 us, 5.5 and 5.9 TB/s
 //           (batched library products of all rows with all experts, their unit and combine: 125 us).
+#include <math.h>
+
 #include "mx_common.h"
 
 namespace {
@@ -37,7 +41,8 @@ struct ExpertGemm {
   int kbytes;           // bytes of a row that count
   const int* src;       // sorted row -> pair
   int top;
-  const int4* tiles;    // (expert, first sorted row, rows, -), then entries without rows; the first one's w: how many have rows
+  const int4* tiles;    // (expert, first sorted row, rows, -), then entries without rows; the one before the first: how many have
+                        // rows, how many of them more than half a tile of 256
   int ntiles;           // entries of the list
   const char* w;        // pieces, expert stride wstride bytes
   long wstride;
@@ -115,7 +120,7 @@ __global__ void __launch_bounds__(1024) expert_plan_kernel(const int* __restrict
       nt += __shfl(st, 63, 64);
     }
     for (int t = nt + lane; t < ntiles; t += 64) tiles[t] = make_int4(0, 0, 0, 0);
-    if (lane == 0) tiles[0].w = nt;
+    if (lane == 0) tiles[-1] = make_int4(nt, nt, 0, 0);
   }
   __syncthreads();
 #pragma unroll
@@ -137,28 +142,32 @@ __global__ void __launch_bounds__(1024) expert_plan_kernel(const int* __restrict
 
 // The same plan by one block per expert, for more pairs than one block sorts in the time of a launch.  Every block counts all
 // pairs (LDS atomics into a row of bins per wave), so it knows its expert's first row and tile without the other blocks, and
-// then places its own expert's pairs: one ballot per chunk of 64 instead of one per bit of the index.  Same pos, src and tiles
-// as above.  Bound by the latency of reading the indices and of the count.  Us in one block / here, 32 experts: 20,260 pairs
-// 30.7 / 9.6, 4,736: 10.5 / 4.9, 2,048: 4.6 / 4.1, 1,536: 4.5 / 4.0, 1,024 and fewer: alike; 8 and 256 experts draw the same
-// line (1,024 pairs 3.8 / 3.8 and 6.6 / 6.6, 4,096: 7.6 / 4.7 and 13.8 / 4.8).  LDS: cnt [16][E], total [E].
+// then places its own expert's pairs: one ballot per chunk of 64 instead of one per bit of the index.  Same pos and src as
+// above, and the same tiles, but that tiles of 256 rows at most half full come last.  Bound by the latency of reading the indices
+// and of the count.  Us in one block / here, 32 experts: 20,260 pairs 30.7 / 9.6, 4,736: 10.5 / 4.9, 2,048: 4.6 / 4.1, 1,536: 4.5 /
+// 4.0, 1,024 and fewer: alike; 8 and 256 experts draw the same line (1,024 pairs 3.8 / 3.8 and 6.6 / 6.6, 4,096: 7.6 / 4.7 and 13.8 /
+// 4.8).  NC > 0: NC * 1024 pairs at most, held in registers; 0: any number, read twice.  LDS: cnt [16][E], total [E].
 template <int NC>
 __global__ void __launch_bounds__(1024) expert_plan_wide_kernel(const int* __restrict__ idx, int P, int E, int mt, int ntiles,
                                                                 int* __restrict__ pos, int* __restrict__ src,
                                                                 int4* __restrict__ tiles) {
   extern __shared__ int lds[];
-  __shared__ int own[4];                                     // first row, first tile, rows, tiles of all experts
+  __shared__ int own[4];                                     // first row, first tile, first tile of the last ones, full tiles
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, me = blockIdx.x;
   int* cnt = lds + w * E;
   int* total = lds + 16 * E;
-  const int i0 = w * NC * 64 + lane;
-  int held[NC];
+  const int nc = NC > 0 ? NC : (P + 1023) / 1024, i0 = w * nc * 64 + lane;
+  int held[NC > 0 ? NC : 1];
 #pragma unroll
   for (int c = 0; c < NC; ++c) held[c] = i0 + c * 64 < P ? idx[i0 + c * 64] : -1;
+  auto expert = [&](int c) { return NC > 0 ? held[c] : (i0 + c * 64 < P ? idx[i0 + c * 64] : -1); };
   for (int e = threadIdx.x; e < 16 * E; e += 1024) lds[e] = 0;
   __syncthreads();
 #pragma unroll
-  for (int c = 0; c < NC; ++c)
-    if ((unsigned)held[c] < (unsigned)E) atomicAdd(cnt + held[c], 1);
+  for (int c = 0; c < nc; ++c) {
+    const int e = expert(c);
+    if ((unsigned)e < (unsigned)E) atomicAdd(cnt + e, 1);
+  }
   __syncthreads();
   for (int e = threadIdx.x; e < E; e += 1024) {
     int t = 0;
@@ -167,34 +176,45 @@ __global__ void __launch_bounds__(1024) expert_plan_wide_kernel(const int* __res
     total[e] = t;
   }
   __syncthreads();
+  const int half = mt == 256 ? 128 : 0;
+  auto begun = [&](int c) { return c % mt != 0 && c % mt <= half; };       // the last tile is one of the small ones
   if (w == 0) {
-    int rows = 0, nt = 0;                                    // of the experts before this one
-    int all = 0;
+    int rows = 0, full = 0, small = 0, fulls = 0, smalls = 0;
     for (int e = lane; e < E; e += 64) {
-      const int c = total[e], t = (c + mt - 1) / mt;
-      if (e < me) rows += c, nt += t;
-      all += t;
+      const int c = total[e], sm = begun(c), fl = (c + mt - 1) / mt - sm;
+      if (e < me) rows += c, full += fl, small += sm;
+      fulls += fl;
+      smalls += sm;
     }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) rows += __shfl_xor(rows, o, 64), nt += __shfl_xor(nt, o, 64), all += __shfl_xor(all, o, 64);
-    if (lane == 0) own[0] = rows, own[1] = nt, own[2] = total[me], own[3] = all;
+    for (int o = 32; o > 0; o >>= 1) {
+      rows += __shfl_xor(rows, o, 64), full += __shfl_xor(full, o, 64), small += __shfl_xor(small, o, 64);
+      fulls += __shfl_xor(fulls, o, 64), smalls += __shfl_xor(smalls, o, 64);
+    }
+    if (lane == 0) {
+      own[0] = rows, own[1] = full, own[2] = fulls + small, own[3] = fulls + smalls;
+      if (me == 0) tiles[-1] = make_int4(fulls + smalls, fulls, 0, 0);
+    }
   }
   __syncthreads();
-  const int row0 = own[0], tile0 = own[1], n = own[2], all = own[3];
-  for (int k = threadIdx.x; k * mt < n; k += 1024)
-    if (tile0 + k < ntiles) tiles[tile0 + k] = make_int4(me, row0 + k * mt, min(mt, n - k * mt), tile0 + k == 0 ? all : 0);
+  const int row0 = own[0], tile0 = own[1], small0 = own[2], all = own[3], n = total[me];
+  for (int k = threadIdx.x; k * mt < n; k += 1024) {
+    const int at = n - k * mt < mt && begun(n) ? small0 : tile0 + k;
+    if (at < ntiles) tiles[at] = make_int4(me, row0 + k * mt, min(mt, n - k * mt), 0);
+  }
   if (me == 0)
     for (int t = all + threadIdx.x; t < ntiles; t += 1024) tiles[t] = make_int4(0, 0, 0, 0);
   int at = row0;
   for (int v = 0; v < w; ++v) at += lds[v * E + me];
 #pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const unsigned long long m = __ballot(held[c] == me);
-    if (held[c] == me) {
+  for (int c = 0; c < nc; ++c) {
+    const int e = expert(c);
+    const unsigned long long m = __ballot(e == me);
+    if (e == me) {
       const int r = at + __popcll(m & ((1ull << lane) - 1));
       pos[i0 + c * 64] = r;
       src[r] = i0 + c * 64;
-    } else if (me == 0 && held[c] >= E) {
+    } else if (me == 0 && e >= E) {
       pos[i0 + c * 64] = 0;
     }
     at += __popcll(m);
@@ -243,18 +263,23 @@ __device__ __forceinline__ const char* expert_row(const ExpertGemm& a, int r, in
   return static_cast<const char*>(a.x) + (a.top > 0 ? a.src[r] / a.top : r) * a.ldx * es;
 }
 
-// (tile, column block) of this block among `cols` column blocks, or false.  Every XCD takes an equal run of the tiles that have
-// rows, in groups of four neighbouring ones -- mostly one expert's -- through all column blocks in turn, so that their W panels
-// and token rows meet in its L2.  (Fixed groups dealt to the XCDs leave some of them idle: 16 tiles of 256 rows by 16 column
-// blocks ran on four.)
+// (tile, column block) of this block among `cols` column blocks, or false.  Every XCD takes an equal run of the full tiles, in
+// groups of four neighbouring ones -- mostly one expert's -- through all column blocks in turn, so that their W panels and token
+// rows meet in its L2, then one of the small tiles.  (Fixed groups dealt to the XCDs leave some of them idle: 16 tiles of 256 rows
+// by 16 column blocks ran on four.)
 __device__ __forceinline__ bool expert_place(const ExpertGemm& a, int cols, int& t, int& nb) {
-  const int live = a.tiles[0].w, nwg = live * cols;
-  int id = blockIdx.x;
-  if (id >= nwg) return false;
-  const int xcd = id & 7, q = nwg >> 3, r = nwg & 7;
+  const int4 head = a.tiles[-1];
+  int id = blockIdx.x, first = 0, live = head.y;
+  if (id >= live * cols) {
+    id -= live * cols;
+    first = live;
+    live = head.x - first;
+    if (id >= live * cols) return false;
+  }
+  const int nwg = live * cols, xcd = id & 7, q = nwg >> 3, r = nwg & 7;
   id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (id >> 3);
   const int grp = id / (4 * cols), in = id - grp * 4 * cols, gm = min(live - 4 * grp, 4);
-  t = 4 * grp + in % gm;
+  t = first + 4 * grp + in % gm;
   nb = in / gm;
   return true;
 }
@@ -355,6 +380,168 @@ __global__ void __launch_bounds__(256, MF == 4 ? 2 : 3) expert_tile_kernel(Exper
   }
 }
 
+// ---- wide tile form (bf16) ---------------------------------------------------------------------------------------
+// 256 W rows x 256 tokens per block, 8 waves as 2 (W rows) x 4 (tokens), a wave's 128 x 64 sub-tile as 8 x 4 accumulators:
+// a third fewer operand reads per product than the 64 x 64 sub-tiles above, which are bound by them.  A K tile (64 elements) is
+// four half tiles of 16 KiB -- W rows 0-63 of both wave rows, tokens 0-127, tokens 128-255, W rows 64-127 of both wave rows -- in
+// two stages, and runs as four phases of {operand reads; one half tile of prefetch; barrier; 16 MFMAs; barrier}.  A half tile is
+// staged again one phase after its last read, so three stay in flight across every barrier and the waits are counted, never a
+// drain.  The waves of the second row run one barrier behind, so that a SIMD's two waves alternate between reading and
+// multiplying.  A tile of at most 128 rows leaves out the products of the second half of its tokens.  One block per CU.
+__device__ __forceinline__ void wide_bar() { __builtin_amdgcn_s_barrier(); }
+template <int N> __device__ __forceinline__ void wide_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
+template <bool GLU>
+__global__ void __launch_bounds__(512) expert_wide_kernel(ExpertGemm a) {
+  typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+  union Frag {
+    uint4 u;
+    bf16x8 v;
+  };
+  constexpr int HALF = 16384, STG = 4 * HALF, W0 = 0, X0 = 1, X1 = 2, W1 = 3;
+  __shared__ __attribute__((aligned(1024))) char smem[2 * STG];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wa = w >> 2, wb = w & 3, g = lane >> 4, col = lane & 15;
+  int tl, nb;
+  if (!expert_place(a, (a.groups + 15) / 16, tl, nb)) return;
+  const int4 tile = a.tiles[tl];
+  const int rows = tile.z;
+
+  const char* src[4][2];                  // piece i of half tile h: this lane's 16 bytes of K tile 0
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int lr = 16 * w + 8 * i + (lane >> 3), ch = (lane & 7) ^ ((lr >> 1) & 7);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int G = min(nb * 16 + wa * 8 + wb + 4 * q, a.groups - 1);               // wave w stages row group w of the half
+      src[q ? W1 : W0][i] = a.w + tile.x * a.wstride + ((long)G * a.kt + i) * 1024 + lane * 16;
+      src[q ? X1 : X0][i] = expert_row(a, tile.y + min(128 * q + lr, rows - 1), 2) + 16 * ch;
+    }
+  }
+  const unsigned lds0 = (unsigned)(uintptr_t)((__attribute__((address_space(3))) char*)smem);
+  auto stage = [&](int h, int t, unsigned buf) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const unsigned dst = buf + h * HALF + (2 * w + i) * 1024;
+      const char* gp = src[h][i] + (long)t * (h == W0 || h == W1 ? 2048 : 128);
+      unsigned keep;
+      asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+                   : "=&s"(keep)
+                   : "v"(gp), "s"(dst)
+                   : "memory");
+    }
+  };
+  const int rowoff = col * 128, ch0 = (g ^ ((col >> 1) & 7)) << 4, ch1 = ((4 + g) ^ ((col >> 1) & 7)) << 4;
+  Frag av[4][2], b0[2][2], b1[2][2], c0[2][2];
+  auto read_w = [&](const char* half) {
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+        av[f][kk].u = *reinterpret_cast<const uint4*>(half + ((wa * 4 + f) * 2 + kk) * 1024 + lane * 16);
+  };
+  auto read_x = [&](const char* half, Frag (&b)[2][2]) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const char* r = half + (wb * 32 + t * 16) * 128 + rowoff;
+      b[t][0].u = *reinterpret_cast<const uint4*>(r + ch0);
+      b[t][1].u = *reinterpret_cast<const uint4*>(r + ch1);
+    }
+  };
+  f32x4 acc[8][4];
+#pragma unroll
+  for (int f = 0; f < 8; ++f)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const bool second = rows > 128;
+  auto phase = [&](auto F0c, auto T0c, const Frag (&bb)[2][2]) {
+    constexpr int F0 = decltype(F0c)::value, T0 = decltype(T0c)::value;
+    wide_bar();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    if (T0 == 0 || second) {
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int f = 0; f < 4; ++f)
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+            acc[F0 + f][T0 + t] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[f][kk].v, bb[t][kk].v, acc[F0 + f][T0 + t], 0, 0, 0);
+      __builtin_amdgcn_s_setprio(0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    wide_bar();
+  };
+  const int nt = a.kt / 2;
+#pragma unroll
+  for (int h = 0; h < 4; ++h) stage(h, 0, lds0);
+  if (nt > 1) {
+#pragma unroll
+    for (int h = 0; h < 3; ++h) stage(h, 1, lds0 + STG);
+    wide_wait<6>();
+  } else {
+    wide_wait<0>();
+  }
+  wide_bar();
+  // The second wave row's extra barrier (the first row passes it after the loop).  A W half is staged again by the wave row that
+  // reads it; an X half by the other row at least one barrier after this row's reads of it have returned (lgkmcnt(0) before the
+  // row's next barrier); the counted wait of a K tile's last phase precedes both rows' barriers before the next tile's reads.
+  if (wa == 1) wide_bar();
+  auto ktile = [&](int t, Frag (&bc)[2][2], Frag (&bn)[2][2]) {
+    const char* cur = smem + (t & 1) * STG;
+    const char* nx = smem + ((t + 1) & 1) * STG;
+    const unsigned lcur = lds0 + (t & 1) * STG, lnxt = lds0 + ((t + 1) & 1) * STG;
+    const bool more1 = t + 1 < nt, more2 = t + 2 < nt;
+    read_w(cur + W0 * HALF);
+    if (more1) stage(W1, t + 1, lnxt);
+    phase(Steps<0>{}, Steps<0>{}, bc);
+    read_x(cur + X1 * HALF, b1);
+    if (more2) stage(W0, t + 2, lcur);
+    phase(Steps<0>{}, Steps<2>{}, b1);
+    read_w(cur + W1 * HALF);
+    if (more2) {
+      stage(X0, t + 2, lcur);
+      wide_wait<8>();                     // W0 and X0 of tile t + 1 have landed: four younger half tiles may be in flight
+    } else {
+      wide_wait<0>();
+    }
+    phase(Steps<4>{}, Steps<2>{}, b1);
+    if (more1) read_x(nx + X0 * HALF, bn);
+    if (more2) {
+      stage(X1, t + 2, lcur);
+      wide_wait<6>();                     // tile t + 1 whole
+    } else {
+      wide_wait<0>();
+    }
+    phase(Steps<4>{}, Steps<0>{}, bc);
+  };
+  read_x(smem + X0 * HALF, b0);
+  int t = 0;
+  for (; t + 1 < nt; t += 2) {
+    ktile(t, b0, c0);
+    ktile(t + 1, c0, b0);
+  }
+  if (t < nt) ktile(t, b0, c0);
+  if (wa == 0) wide_bar();
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int m = (u >> 1) * 128 + wb * 32 + (u & 1) * 16 + col, G = nb * 16 + wa * 8;
+    if (m >= rows) continue;
+    if (GLU) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (G + 2 * q < a.groups)
+          expert_store<bf16, true>(a, tile.y + m, (G / 2 + q) * 16 + 4 * g, acc[2 * q][u], acc[2 * q + 1][u]);
+    } else {
+#pragma unroll
+      for (int f = 0; f < 8; ++f)
+        if (G + f < a.groups) expert_store<bf16, false>(a, tile.y + m, (G + f) * 16 + 4 * g, acc[f][u], acc[f][u]);
+    }
+  }
+}
+
 // ---- stream form -------------------------------------------------------------------------------------------------
 // NF row groups x 16 tokens per block; wave w takes the w-th quarter of the pieces, the partial sums meet in LDS.
 template <typename T, int NF, bool GLU>
@@ -432,21 +619,57 @@ __global__ void __launch_bounds__(256) expert_stream_kernel(ExpertGemm a) {
 // Both are estimated (us; `bytes`: an expert's two matrices; `stages`: of one block of each product): 4 experts of 4096 x 2048,
 // tiles of 16 / 64: 32 rows on average 58 / 132, f32 126 / 569, 96 rows 120 / 122; 8 of 8192 x 2048: 24 rows 165 / 238, 48 rows
 // 274 / 245; 2 of 4096 x 1024: 64 rows 32 / 87; 16 of 768 x 2048: 24 rows 35 / 48, 48 rows 56 / 50.
-// Of the wide tiles, 64 rows also for more when few experts' wider ones would be fewer than the CUs (`columns`: column blocks of
-// the smaller product): 4 experts of 4096 x 2048, 128 rows 126 / 156, 8 of 8192 x 2048, 128 rows 231 / 310, 256 rows 353 / 305.
-int tile_rows(long pairs, int experts, int dt, double bytes, int stages, int columns) {
+//
+// Among the larger tiles the choice is by an estimate too: the rounds of blocks over the CUs (3, 2 and 1 blocks of 64, 128 and 256
+// rows on each) times a block's stages at 1.35 (1.15 where the CUs are not full), 1.38 and 1.85 us; an expert's last tile is half
+// full on average, and a small one of 256 rows takes half the time.  Us for tiles of 64 / 128 / 256, bf16, experts' rows spread by a factor of about 1.3 (5 for the
+// second figures): 32 experts of 1024 x 2048: 64 rows on average 102 / 100 / 95 (96 / 127 / 117), 128: 129 / 138 / 114 (132 / 139 / 142),
+// 192: 165 / 146 / 156 (168 / 142 / 147), 256: 202 / 192 / 176 (189 / 188 / 174), 431: 290 / 256 / 245 (271 / 250 / 214), 633: 397 / 360 /
+// 307 (371 / 325 / 298), 1024: 586 / 513 / 457 (570 / 505 / 447); of 512 x 1024: 128: 40 / 44 / 63, 256: 61 / 73 / 72, 431: 84 / 86 / 92,
+// 633: 112 / 120 / 134; 8 of 2048 x 4096: 128: 145 / 136 / 144, 192: 197 / 138 / 157, 256: 204 / 216 / 167, 1250: 745 / 625 / 492; 64 of 768 x
+// 2048: 64: 155 / 154 / 156, 128: 211 / 205 / 182, 512: 522 / 477 / 419; 4 plain ones of 4096 x 2048: 175: 67 / 79 / 68, 375: 95 / 92 / 142,
+// 1000: 179 / 202 / 189.
+struct Product {
+  int groups, kt;
+};
+
+double wide_time(double avg, int experts, int mt, const Product* p) {
+  double us = 0;
+  for (int i = 0; i < 2; ++i) {
+    const int cols = mt == 256 ? (p[i].groups + 15) / 16 : (p[i].groups + 7) / 8;
+    double r = mt == 256 ? experts * (avg / 256 + 0.25) * cols / 256 + 0.2
+                         : experts * (avg / mt + 0.5) * cols / (mt == 128 ? 512 : 768);
+    if (r < 3) r = floor(r) + fmin(1.0, 2 * (r - floor(r)));      // the last of a few rounds leaves CUs idle
+    us += fmax(r, 1.0) * (p[i].kt / 2 * (mt == 256 ? 1.85 : mt == 128 ? 1.38 : r < 1 ? 1.15 : 1.35) + (mt == 256 ? 5 : 0));
+  }
+  return us;
+}
+
+// `whole`: rows are whole stages of K, which the form of 256 rows asks for
+int tile_rows(long pairs, int experts, int dt, const Product* p, bool whole) {
   const long avg = pairs / experts;
   if (avg <= (dt == 1 ? 24 : 12)) return 16;
+  const double bytes = 1024.0 * ((double)p[0].groups * p[0].kt + (double)p[1].groups * p[1].kt);
+  const int stages = (p[0].kt + p[1].kt) / 2;
   const double live = pairs < experts ? pairs : experts, memory = live * bytes / 5.2e6;
   const double chain = stages * (dt == 1 ? 1.15 + bytes * 20e-9 : 0.7 + bytes * 9.5e-9);
   const double again = (pairs / 16.0 + live / 2) * bytes / (dt == 1 ? 7.0e6 : 7.9e6);
   if (15 + (again > memory ? again : memory) < 12 + (chain > memory ? chain : memory) && pairs / 16 + experts <= 65535) return 16;
-  return dt == 1 || avg <= 56 || (experts <= 8 && (experts + pairs / 128) * columns < 300) ? 64 : 128;
+  if (dt == 1) return 64;
+  const double t64 = wide_time((double)pairs / experts, experts, 64, p), t128 = wide_time((double)pairs / experts, experts, 128, p);
+  // (below 512 rows an expert's panels are read by one or two blocks of 256, whose stages in flight do not cover a first touch of
+  // memory: inside a model, 148 rows on average took 142 us with 256, 124 with 128, and 431 rows 254 and 246)
+  if (whole && avg >= 512 && wide_time((double)pairs / experts, experts, 256, p) < fmin(t64, t128)) return 256;
+  return t64 < 0.95 * t128 ? 64 : 128;                              // 64 where it is clearly the shorter
 }
 
 template <typename T, bool GLU>
 int expert_launch(const ExpertGemm& a, int mt, hipStream_t st) {
-  if (mt >= 64) {
+  if (mt == 256) {
+    const long grid = (long)a.ntiles * ((a.groups + 15) / 16);
+    if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
+    if constexpr (sizeof(T) == 2) expert_wide_kernel<GLU><<<(unsigned)grid, 512, 0, st>>>(a);
+  } else if (mt >= 64) {
     const long grid = (long)a.ntiles * ((a.groups + 7) / 8);
     if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
     if constexpr (sizeof(T) == 2) {
@@ -485,14 +708,14 @@ MX_API int mx_experts(const void* h, long ldh, const int* idx, int T, int top, i
       (size_t)iws % 16 || (glu ? g1 % 2 || g1 / 2 * 16 < lda : g1 * 16 < lda) || g2 * 16 < W || unit < 0 || unit > UNIT_RELU2 ||
       (scale != nullptr && !glu))
     return (int)hipErrorInvalidValue;
-  const int mt = tile_rows(P, E, dt, 1024.0 * ((double)g1 * k1 + (double)g2 * k2), (k1 + k2) / 2,
-                           ((g1 < g2 ? g1 : g2) + 7) / 8);
+  // the plan by one block per expert beyond 1024 pairs (every block reads them all: up to 512 experts, 35 KB of counts)
+  const bool wide = P > 1024 && E <= 512;
+  const Product products[2] = {{g1, k1}, {g2, k2}};
+  const int mt = tile_rows(P, E, dt, products, wide && (long)k1 * 64 == (long)W * es && (long)k2 * 64 == lda * es);
   const int ntiles = (int)(P / mt + (P < E ? P : E));
   int* pos = iws;
   int* src = iws + (P + 3) / 4 * 4;
-  int4* tiles = reinterpret_cast<int4*>(src + (P + 3) / 4 * 4);
-  // one block per expert beyond 1024 pairs (every block reads them all: up to 512 experts, 35 KB of counts)
-  const bool wide = P > 1024 && P <= 32 * 1024 && E <= 512;
+  int4* tiles = reinterpret_cast<int4*>(src + (P + 3) / 4 * 4) + 1;
   int bits = 0;
   while ((1 << bits) < E) ++bits;
   int nw = (int)((P + 63) / 64);
@@ -505,7 +728,8 @@ MX_API int mx_experts(const void* h, long ldh, const int* idx, int T, int top, i
   if (wide && P <= 4 * 1024) WIDE(4);
   else if (wide && P <= 8 * 1024) WIDE(8);
   else if (wide && P <= 16 * 1024) WIDE(16);
-  else if (wide) WIDE(32);
+  else if (wide && P <= 32 * 1024) WIDE(32);
+  else if (wide) WIDE(0);
   else if (run <= 2) PLAN(2);
   else if (run <= 8) PLAN(8);
   else if (run <= 16) PLAN(16);

@@ -139,3 +139,14 @@ def test_expert_plan_is_the_stable_sort(E, T):
         want = torch.empty(T * top, dtype=torch.int32)
         want[torch.argsort(flat, stable=True)] = torch.arange(T * top, dtype=torch.int32)
         assert torch.equal(pos.cpu().flatten(), torch.where(flat < E, want, 0))
+
+
+@pytest.mark.parametrize("T,W,F_,E,top,unit,kw", [
+    (1700, 2048, 1024, 8, 3, "clamped", {}),             # 637 rows on average: tiles of 256 rows, the last one of half the experts small
+    (1600, 2112, 1088, 8, 3, "silu", {"skew": True}),    # an odd number of K tiles; two experts with most of the rows
+    (1700, 2048, 1088, 8, 3, "gelu_tanh", {"strided": True, "ident": 1}),      # a column block beyond the last group
+    (4000, 768, 1024, 16, 4, "relu2", {"ident": 2}),
+    (1700, 2056, 1024, 8, 3, "clamped", {}),             # rows in no whole K tile: 128 tokens
+])
+def test_experts_of_many_rows(T, W, F_, E, top, unit, kw):
+    check(torch.bfloat16, T, W, F_, E, top, unit, **kw)
