@@ -12,7 +12,9 @@
 //                     the score registers -- as two bf16 terms hi + lo, so that f32 weights are not cut to 8 bits (HILO), one
 //                     bf16 term, or f32
 // Bound by the LDS reads of the operands and the vector instructions of the softmax (four segments of 2048 rows, 16 heads
-// over 4, window 1024: 127 us, 0.6 PFLOP/s with the second weight term).  16 pairs per wave (MB = 1): 32 halve the operand
+// over 4, window 1024: 127 us, 0.6 PFLOP/s with the second weight term).  Operands read a group ahead of their products, the page
+// of a tile read a tile ahead of its copies and weights rounded in pairs took 4 - 7 % off in bf16 (prompts of 540, 300 and 327 rows
+// behind 1000 - 2500 beside 21 rows: 70.2 -> 65.4 us) and 7 - 20 % in f32 (254 -> 228; latents, 2 single rows behind 1443: 42 -> 34).  16 pairs per wave (MB = 1): 32 halve the operand
 // reads but leave two waves per SIMD (bf16 heads of 128: 56 against 43 us for 1190 rows) or spill (latent: 108 against 65).
 // A block's serial walk is what a small step waits for: the caller splits the keys over nsplit blocks where that is shorter
 // than reading the parts back (unnormalised: o | m | l, merged afterwards).
@@ -24,6 +26,7 @@ namespace {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 struct RowsArgs {
   const void *q, *q2;            // queries: head h of row t at q + t * sq + h * D1 (elements), its second part at q2 + (t * H + h) * D2
@@ -78,6 +81,12 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) rows_attend_kernel(R
   constexpr int KS = KB / 64, NT = P / 16, KTT = KT / 16, KI = KIMG / 1024, VI = SHARED ? 0 : KT * VB / 1024;
   constexpr int KPW = (KI + NW - 1) / NW, VPW = (VI + NW - 1) / NW;      // 1-KiB pieces per wave
   constexpr bool BF = ES == 2;
+  // Two waves per SIMD or fewer (64 keys per tile, or f32) do not hide the LDS latency by themselves: operands are read a group
+  // ahead of the products that use them.
+  constexpr bool AHEAD = KT == 64 || !BF;
+  constexpr int TP = BF && KS <= 4 ? 2 : 1, GK = BF ? KS : KS % 3 == 0 ? 3 : 2, GV = NT % 4 == 0 ? 4 : 1;
+  constexpr int NVG = BF ? NT / GV : 4 * (NT / GV);
+  static_assert(KTT % TP == 0 && KS % GK == 0, "operand groups");
   static_assert(KB % 64 == 0 && P % 16 == 0 && KIMG % 1024 == 0 && KT % 32 == 0 && PAGE_ROWS % KT == 0, "tile shape");
   __shared__ __attribute__((aligned(1024))) char smem[2 * STG];
   const int rep = a.H / a.G, hblocks = (rep + a.HB - 1) / a.HB;
@@ -159,10 +168,11 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) rows_attend_kernel(R
                  : "v"(gp), "s"(dst)
                  : "memory");
   };
-  auto stage = [&](int i, int buf) {
+  auto page_of = [&](int i) { return a.bt[(long)s * a.btw + key0(i) / PAGE_ROWS]; };
+  auto stage = [&](int i, int buf, int page) {
     const int k0 = key0(i), last = p_last - k0;
     const char* src = static_cast<const char*>(a.cache) +
-                      ((long)a.bt[(long)s * a.btw + k0 / PAGE_ROWS] * PAGE_ROWS + k0 % PAGE_ROWS) * a.Wr * ES;
+                      ((long)__builtin_amdgcn_readfirstlane(page) * PAGE_ROWS + k0 % PAGE_ROWS) * a.Wr * ES;
     const unsigned dst = lds0 + buf * STG;
 #pragma unroll
     for (int j = 0; j < KPW; ++j)
@@ -183,28 +193,94 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) rows_attend_kernel(R
 
   const int t_begin = ti;
   int buf = 0;
-  if (ti <= t_end) stage(ti, 0);
+  // a tile's page is read a tile before its copies are issued, which would wait for it
+  int page = ti < t_end ? page_of(ti + 1) : 0;
+  if (ti <= t_end) stage(ti, 0, page_of(ti));
   for (; ti <= t_end; ++ti, buf ^= 1) {
     // this wave's pieces have landed, then everybody's; all reads of the other stage are done
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (ti < t_end) stage(ti + 1, buf ^ 1);
+    if (ti < t_end) stage(ti + 1, buf ^ 1, page);
+    if (ti + 1 < t_end) page = page_of(ti + 2);
     if (!wave_live) continue;
     const char* kt = smem + buf * STG;
     const int k0 = key0(ti);
     const bool whole = k0 + KT - 1 <= p_first && k0 >= lo_last;   // every pair sees every key
     f32x4 st[MB][KTT];
+    uint4 kf[2][TP][GK];
+    auto read_keys = [&](int i, uint4 (&f)[TP][GK]) {            // group i: TP key tiles of 16, GK steps of K
+      const int t = i / (KS / GK) * TP, k = i % (KS / GK) * GK;
 #pragma unroll
-    for (int t = 0; t < KTT; ++t) {
+      for (int x = 0; x < TP; ++x)
+#pragma unroll
+        for (int y = 0; y < GK; ++y)
+          f[x][y] = *reinterpret_cast<const uint4*>(kt + krd + (t + x) * 16 * KB + (((4 * (k + y) + g) ^ zc) << 4));
+    };
+#pragma unroll
+    for (int t = 0; t < KTT; ++t)
 #pragma unroll
       for (int b = 0; b < MB; ++b) st[b][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (AHEAD) read_keys(0, kf[0]);
 #pragma unroll
-      for (int k = 0; k < KS; ++k) {
-        const uint4 kf = *reinterpret_cast<const uint4*>(kt + krd + t * 16 * KB + (((4 * k + g) ^ zc) << 4));
+    for (int i = 0; i < KTT / TP * (KS / GK); ++i) {
+      if (!AHEAD) read_keys(i, kf[i & 1]);
+      else if (i + 1 < KTT / TP * (KS / GK)) read_keys(i + 1, kf[(i + 1) & 1]);
+      if (AHEAD) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int b = 0; b < MB; ++b) st[b][t] = mma16<T>(kf, qf[b][k], st[b][t]);
-      }
+      for (int y = 0; y < GK; ++y)
+#pragma unroll
+        for (int x = 0; x < TP; ++x)
+#pragma unroll
+          for (int b = 0; b < MB; ++b) {
+            const int t = i / (KS / GK) * TP + x, k = i % (KS / GK) * GK + y;
+            st[b][t] = mma16<T>(kf[i & 1][x][y], qf[b][k], st[b][t]);
+          }
+      if (AHEAD) __builtin_amdgcn_sched_barrier(0);
     }
-    bf16x8 ph[MB][KTT / 2], pl[MB][KTT / 2];
+    // value operands, by groups of GV column tiles (f32: of one key step as well); the first group is on its way during the softmax
+    const char* vt = kt + VBASE + vr * VROWB;
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    union VFrag {
+      s16x4 s[2];
+      bf16x8 v;
+    };
+    VFrag vb[2][GV][KTT / 2];
+    float vf[2][GV][KTT];
+    auto read_values = [&](int i) {
+      if constexpr (BF) {
+        const int cz = ((c & 3) >> 1) ^ zv, half = (c & 1) * 8;
+#pragma unroll
+        for (int x = 0; x < GV; ++x) {
+          const char* v0 = vt + (((2 * (i * GV + x)) ^ cz) << 4) + half;
+#pragma unroll
+          for (int u = 0; u < KTT / 2; ++u) {
+            VFrag& f = vb[i & 1][x][u];
+            f.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(v0 + 32 * u * VROWB));
+            f.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(v0 + (32 * u + 16) * VROWB));
+          }
+        }
+      } else {
+        // step (t, r): K index g is key 16 t + 4 g + r; the row's swizzle is that of row 4 g, but for its low two bits
+        const int r = i / (NT / GV), i0 = i % (NT / GV) * GV;
+#pragma unroll
+        for (int x = 0; x < GV; ++x) {
+          const char* v0 = vt + r * VROWB + (((4 * (i0 + x) + (c >> 2)) ^ rows_swz<VC, ES>(vr + r)) << 4) + (c & 3) * 4;
+#pragma unroll
+          for (int t = 0; t < KTT; ++t) vf[i & 1][x][t] = *reinterpret_cast<const float*>(v0 + 16 * t * VROWB);
+        }
+      }
+    };
+    if (AHEAD) {
+      read_values(0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    union Pair {
+      bf16x2 v;
+      unsigned u;
+    };
+    union Weights {
+      unsigned u[4];
+      bf16x8 v;
+    } ph[MB][KTT / 2], pl[MB][KTT / 2];
 #pragma unroll
     for (int b = 0; b < MB; ++b) {
       float mt = -INFINITY;
@@ -225,7 +301,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) rows_attend_kernel(R
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int j = k0 + 16 * t + 4 * g + r;
-            if (!(j <= pq[b] && (j >= pq_lo[b] || j < a.keep))) st[b][t][r] = -INFINITY;
+            st[b][t][r] = (j <= pq[b]) & ((j >= pq_lo[b]) | (j < a.keep)) ? st[b][t][r] : -INFINITY;
           }
       }
 #pragma unroll
@@ -246,50 +322,54 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) rows_attend_kernel(R
       for (int t = 0; t < KTT; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float p = __builtin_amdgcn_exp2f(st[b][t][r] - mref);
-          l[b] += p;
-          if (BF) {
-            const bf16 hi = (bf16)p;
-            ph[b][t / 2][4 * (t & 1) + r] = hi;
-            if (HILO) pl[b][t / 2][4 * (t & 1) + r] = (bf16)(p - (float)hi);
-          } else {
-            st[b][t][r] = p;
-          }
+          st[b][t][r] = __builtin_amdgcn_exp2f(st[b][t][r] - mref);
+          l[b] += st[b][t][r];
         }
+      if constexpr (BF) {
+#pragma unroll
+        for (int t = 0; t < KTT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; r += 2) {                       // by two: one conversion each
+            const float p0 = st[b][t][r], p1 = st[b][t][r + 1];
+            Pair hi, lo;
+            hi.v = bf16x2{(bf16)p0, (bf16)p1};
+            ph[b][t / 2].u[2 * (t & 1) + r / 2] = hi.u;
+            if (HILO) {
+              lo.v = bf16x2{(bf16)(p0 - __uint_as_float(hi.u << 16)), (bf16)(p1 - __uint_as_float(hi.u & 0xffff0000u))};
+              pl[b][t / 2].u[2 * (t & 1) + r / 2] = lo.u;
+            }
+          }
+      }
     }
-    const char* vt = kt + VBASE + vr * VROWB;
-    if constexpr (BF) {
-      typedef short s16x4 __attribute__((ext_vector_type(4)));
-      const int cz = ((c & 3) >> 1) ^ zv, half = (c & 1) * 8;
 #pragma unroll
-      for (int i = 0; i < NT; ++i) {
-        const char* v0 = vt + (((2 * i) ^ cz) << 4) + half;
+    for (int i = 0; i < NVG; ++i) {
+      if (!AHEAD) read_values(i);
+      else if (i + 1 < NVG) read_values(i + 1);
+      if (AHEAD) __builtin_amdgcn_sched_barrier(0);
+      if constexpr (BF) {
 #pragma unroll
-        for (int u = 0; u < KTT / 2; ++u) {
-          union { s16x4 s[2]; bf16x8 v; } f;
-          f.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(v0 + 32 * u * VROWB));
-          f.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(v0 + (32 * u + 16) * VROWB));
+        for (int u = 0; u < KTT / 2; ++u)
 #pragma unroll
           for (int b = 0; b < MB; ++b) {
-            o[b][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.v, ph[b][u], o[b][i], 0, 0, 0);
-            if (HILO) o[b][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.v, pl[b][u], o[b][i], 0, 0, 0);
+#pragma unroll
+            for (int x = 0; x < GV; ++x)
+              o[b][i * GV + x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vb[i & 1][x][u].v, ph[b][u].v, o[b][i * GV + x], 0, 0, 0);
+            if (HILO)
+#pragma unroll
+              for (int x = 0; x < GV; ++x)
+                o[b][i * GV + x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vb[i & 1][x][u].v, pl[b][u].v, o[b][i * GV + x], 0, 0, 0);
           }
-        }
+      } else {
+        const int r = i / (NT / GV), i0 = i % (NT / GV) * GV;
+#pragma unroll
+        for (int t = 0; t < KTT; ++t)
+#pragma unroll
+          for (int x = 0; x < GV; ++x)
+#pragma unroll
+            for (int b = 0; b < MB; ++b)
+              o[b][i0 + x] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i & 1][x][t], st[b][t][r], o[b][i0 + x], 0, 0, 0);
       }
-    } else {
-      // step (t, r): K index g is key 16 t + 4 g + r; the row's swizzle is that of row 4 g, but for its low two bits
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int i = 0; i < NT; ++i) {
-          const char* v0 = vt + r * VROWB + (((4 * i + (c >> 2)) ^ rows_swz<VC, ES>(vr + r)) << 4) + (c & 3) * 4;
-#pragma unroll
-          for (int t = 0; t < KTT; ++t) {
-            const float v = *reinterpret_cast<const float*>(v0 + 16 * t * VROWB);
-#pragma unroll
-            for (int b = 0; b < MB; ++b) o[b][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, st[b][t][r], o[b][i], 0, 0, 0);
-          }
-        }
+      if (AHEAD) __builtin_amdgcn_sched_barrier(0);
     }
   }
   typedef T out4 __attribute__((ext_vector_type(4)));
