@@ -65,37 +65,6 @@ __device__ __forceinline__ float rows_sum4(float v) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-// Blocks are numbered over the row tiles that the segments have, one after the other (at most rows / QT + S of them): a grid of the
-// longest segment's tiles for every segment is mostly empty blocks in a step of prompts and single rows, and its live ones meet on
-// few CUs (prompts of 540, 300 and 327 rows behind contexts of 1000 - 2500 beside 21 rows, 16 heads over 4, window 1024: 34 x 4 x 24
-// blocks, 376 of them live, took 65 us in bf16 and 227 in f32, numbered so 45 and 159).  S: 0 for one block per segment.
-__device__ __forceinline__ bool rows_place(const RowsArgs& a, int id, int& s, int& t0) {
-  const int lane = threadIdx.x & 63;
-  if (a.S <= 1) {
-    s = a.S == 0 ? id : 0;
-    t0 = a.S == 0 ? 0 : id * a.QT;
-    return t0 < a.cu[s + 1] - a.cu[s];
-  }
-  for (int base = 0; base < a.S; base += 64) {
-    const int i = base + lane, n = i < a.S ? a.cu[i + 1] - a.cu[i] : 0, tiles = (n + a.QT - 1) / a.QT;
-    int upto = tiles;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int x = __shfl_up(upto, o, 64);
-      if (lane >= o) upto += x;
-    }
-    const unsigned long long past = __ballot(upto > id);
-    if (past != 0) {
-      const int at = __ffsll(past) - 1;
-      s = base + at;
-      t0 = (id - __builtin_amdgcn_readlane(upto - tiles, at)) * a.QT;
-      return true;
-    }
-    id -= __builtin_amdgcn_readlane(upto, 63);
-  }
-  return false;
-}
-
 // chunk swizzle of a tile row (CH 16-byte chunks per row): chunk c lies at c ^ z(row).
 // Rows of whole 256 bytes: 16 rows at one chunk (key reads) meet 16 different ones; bf16: rows 4 g .. 4 g + 7 at a pair of
 // chunks (transposed value reads) different pairs; f32: rows 0, 4, 8, 12 at four chunks (value reads) different fours.
@@ -126,7 +95,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) rows_attend_kernel(R
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, c = lane & 15;
   const int split = blockIdx.x % a.nsplit;
   int s, t0;
-  if (!rows_place(a, blockIdx.x / a.nsplit, s, t0)) return;
+  if (!mx_tile_place(a.cu, a.S, a.QT, blockIdx.x / a.nsplit, s, t0)) return;      // (in a grid of dead blocks: 65 us for 45, in f32 227 for 159)
   const int r0 = a.cu[s], n = a.cu[s + 1] - r0;
   const int nq = min(a.QT, n - t0), kvh = blockIdx.y / hblocks, hg0 = (blockIdx.y % hblocks) * a.HB;
   const int nh = min(a.HB, rep - hg0), h0 = kvh * rep + hg0;

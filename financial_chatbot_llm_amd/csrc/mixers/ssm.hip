@@ -22,23 +22,25 @@ namespace {
 constexpr int CONV_TT = 32;   // tokens per block of the convolution
 constexpr int MAX_TAPS = 8;
 
-// grid (ceil(C/256), ceil(max_len/CONV_TT), S)
+// Both forms: the thread of a segment's first tile is the only one that reads the slot's history of its channels (a tile has more
+// rows than the taps reach back), and it replaces it by the segment's last K-1 inputs, upward, reading entry j + n before it
+// writes entry j.  (A launch of its own for that took 4.6 - 5.6 us behind each convolution.)
+
+// grid (ceil(C/256), tiles of the segments)
 template <typename T>
 __global__ void conv_silu_kernel(const T* __restrict__ in, long si, const float* __restrict__ w,
-                                 const float* __restrict__ bias, const float* __restrict__ in_bias, int act,
-                                 const float* __restrict__ state,
+                                 const float* __restrict__ bias, const float* __restrict__ in_bias, int act, float* state,
                                  const int* __restrict__ cu, const int* __restrict__ slot, const int* __restrict__ pos,
-                                 float* __restrict__ out, int C, int K) {
-  const int s = blockIdx.z;
+                                 float* __restrict__ out, int S, int C, int K) {
+  int s, t0;
+  if (!mx_tile_place(cu, S, CONV_TT, blockIdx.y, s, t0)) return;
   const int sl = slot[s];
   if (sl < 0) return;
   const int r0 = cu[s], n = cu[s + 1] - r0;
-  const int t0 = blockIdx.y * CONV_TT;
-  if (t0 >= n) return;
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= C) return;
   const bool fresh = pos[r0] == 0;
-  const float* st = state + (long)sl * (K - 1) * C;
+  float* st = state + (long)sl * (K - 1) * C;
   float wk[MAX_TAPS], win[MAX_TAPS];
   const float ib = in_bias != nullptr ? in_bias[c] : 0.f;   // added to every real input (the history holds biased inputs)
 #pragma unroll
@@ -54,6 +56,11 @@ __global__ void conv_silu_kernel(const T* __restrict__ in, long si, const float*
       win[k + 1] = j >= 0 ? ldf(in + (long)(r0 + j) * si + c) + ib : (fresh ? 0.f : st[(long)(K - 1 + j) * C + c]);
     }
   }
+  if (t0 == 0)
+    for (int j = 0; j < K - 1; ++j) {
+      const int i = n - (K - 1) + j;             // local index of the input that lands in entry j
+      st[(long)j * C + c] = i >= 0 ? ldf(in + (long)(r0 + i) * si + c) + ib : (fresh ? 0.f : st[(long)(j + n) * C + c]);
+    }
   const float b = bias != nullptr ? bias[c] : 0.f;
   const int t1 = min(t0 + CONV_TT, n);
   for (int i = t0; i < t1; ++i) {
@@ -77,13 +84,14 @@ constexpr int CONV_V = 8;
 template <typename T>
 __global__ void __launch_bounds__(256) conv4_kernel(const T* __restrict__ in, long si, const float* __restrict__ w,
                                                     const float* __restrict__ bias, const float* __restrict__ in_bias, int act,
-                                                    const float* __restrict__ state, const int* __restrict__ cu,
+                                                    float* state, const int* __restrict__ cu,
                                                     const int* __restrict__ slot, const int* __restrict__ pos,
-                                                    float* __restrict__ out, int C) {
-  const int s = blockIdx.z, sl = slot[s];
+                                                    float* __restrict__ out, int S, int C) {
+  int s, t0;
+  if (!mx_tile_place(cu, S, CONV_TT, blockIdx.y, s, t0)) return;
+  const int sl = slot[s];
   if (sl < 0) return;
-  const int r0 = cu[s], n = cu[s + 1] - r0, t0 = blockIdx.y * CONV_TT;
-  if (t0 >= n) return;
+  const int r0 = cu[s], n = cu[s + 1] - r0;
   const int c = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (c >= C) return;
   const bool fresh = pos[r0] == 0;
@@ -105,6 +113,15 @@ __global__ void __launch_bounds__(256) conv4_kernel(const T* __restrict__ in, lo
     if (j >= 0) x[k] = ldf4(in + (long)(r0 + j) * si + c) + ib;
     else if (!fresh) x[k] = ldf4(state + ((long)sl * 3 + 3 + j) * C + c);
   }
+  if (t0 == 0) {                         // x[0 .. 2] is the history
+    float* st = state + (long)sl * 3 * C + c;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const int i = n - 3 + j;
+      const mx_f32x4 old = j + n == 1 ? x[1] : x[2];       // entry j + n, 1 or 2
+      stf4(st + (long)j * C, i >= 0 ? ldf4(in + (long)(r0 + i) * si + c) + ib : old);
+    }
+  }
   const int t1 = min(t0 + CONV_TT, n);
   for (int i0 = t0; i0 < t1; i0 += CONV_V) {
 #pragma unroll
@@ -123,31 +140,6 @@ __global__ void __launch_bounds__(256) conv4_kernel(const T* __restrict__ in, lo
     }
 #pragma unroll
     for (int k = 0; k < 3; ++k) x[k] = x[CONV_V + k];
-  }
-}
-
-// grid (ceil(C/256), S): the slot's last K-1 inputs after this chunk.  Runs after conv_silu_kernel
-// of the same step (same stream).  One thread owns a channel's K-1 entries and walks them upward,
-// reading entry j + n before it writes entry j, so the shift is safe in place.
-template <typename T>
-__global__ void conv_state_kernel(const T* __restrict__ in, long si, const float* __restrict__ in_bias, float* __restrict__ state,
-                                  const int* __restrict__ cu, const int* __restrict__ slot, const int* __restrict__ pos,
-                                  int C, int K) {
-  const int s = blockIdx.y;
-  const int sl = slot[s];
-  if (sl < 0) return;
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= C) return;
-  const int r0 = cu[s], n = cu[s + 1] - r0;
-  if (n <= 0) return;
-  const bool fresh = pos[r0] == 0;
-  float* st = state + (long)sl * (K - 1) * C;
-  for (int j = 0; j < K - 1; ++j) {
-    const int i = n - (K - 1) + j;             // local index of the input that lands in entry j
-    float v;
-    if (i >= 0) v = ldf(in + (long)(r0 + i) * si + c) + (in_bias != nullptr ? in_bias[c] : 0.f);
-    else v = fresh ? 0.f : st[(long)(j + n) * C + c];
-    st[(long)j * C + c] = v;
   }
 }
 
@@ -686,17 +678,13 @@ MX_API int mx_conv_act(const void* in, long si, int dt, const float* w, const fl
   if (K < 1 || K > MAX_TAPS || act < 0 || act > 1) return (int)hipErrorInvalidValue;
   if (K == 4 && C % 4 == 0 && rows >= 8L * S && (long)rows * C >= 4500000 && mx_by_four(in, si, dt) &&
       ((size_t)w | (size_t)bias | (size_t)in_bias | (size_t)state | (size_t)out) % 16 == 0) {
-    const dim3 grid((C / 4 + 255) / 256, (max_len + CONV_TT - 1) / CONV_TT, S);
+    const dim3 grid((C / 4 + 255) / 256, mx_tile_count(S, rows, max_len, CONV_TT));
     MX_DISPATCH(dt, TT, conv4_kernel<TT><<<grid, 256, 0, st>>>((const TT*)in, si, w, bias, in_bias, act, state, cu, slot, pos,
-                                                               out, C));
+                                                               out, mx_tile_segments(S, max_len), C));
   } else {
-    dim3 grid((C + 255) / 256, (max_len + CONV_TT - 1) / CONV_TT, S);
+    const dim3 grid((C + 255) / 256, mx_tile_count(S, rows, max_len, CONV_TT));
     MX_DISPATCH(dt, TT, conv_silu_kernel<TT><<<grid, 256, 0, st>>>((const TT*)in, si, w, bias, in_bias, act, state, cu,
-                                                                   slot, pos, out, C, K));
-  }
-  if (K > 1) {
-    dim3 g2((C + 255) / 256, S);
-    MX_DISPATCH(dt, TT, conv_state_kernel<TT><<<g2, 256, 0, st>>>((const TT*)in, si, in_bias, state, cu, slot, pos, C, K));
+                                                                   slot, pos, out, mx_tile_segments(S, max_len), C, K));
   }
   MX_RETURN_LAUNCH();
 }

@@ -99,7 +99,7 @@ _MIXER_SIGS = {
     "mx_route_biased": [P, P, c_int, c_int, c_int, c_int, c_float, P, P, c_int, P],
     "mx_dyn_tanh": [P, P, c_long, P, P, c_int, c_float, c_int, c_float, P, P, c_float, P, P, P, c_int, c_int, c_int, P],
     "mx_conv_heads": [P, c_long, c_int, P, c_int, P, P, P, c_float, c_float, c_int, P, P, P, P, P, P, c_int, c_int, c_int,
-                      c_int, c_int, c_int, P],
+                      c_int, c_int, c_int, c_int, P],
     "mx_moe_combine": [P, c_long, P, P, P, P, c_long, P, c_long, c_int, c_int, c_int, P, c_int, c_int, P],
     "mx_experts": [P, c_long, P, c_int, c_int, c_int, c_int, c_int, P, c_int, c_int, P, c_int, c_int, c_int, c_float, c_float,
                    P, P, c_long, P, P, c_int, P],

@@ -1030,7 +1030,7 @@ def conv_heads(proj: torch.Tensor, w: torch.Tensor, state: Optional[torch.Tensor
         out = torch.empty((T, H * D), dtype=proj.dtype, device=proj.device)
         N.mcall("mx_conv_heads", N.ptr(_rows(proj)), proj.stride(0), _dt(proj), N.ptr(w), K, N.ptr(state) if K > 1 else None,
                 N.ptr(q_norm), N.ptr(k_norm), float(eps), float(temp_coef), int(temp_every), N.ptr(cu), N.ptr(slot),
-                N.ptr(pos), N.ptr(slots), N.ptr(cache) if G else None, N.ptr(out), S, int(max_len), H, G, D, P, N.stream())
+                N.ptr(pos), N.ptr(slots), N.ptr(cache) if G else None, N.ptr(out), S, int(max_len), T, H, G, D, P, N.stream())
         return out
     u = proj[:, :C].float()
     y = torch.zeros((T, C), dtype=torch.float32)

@@ -1,0 +1,80 @@
+"""Kernels whose blocks are numbered over the segments' row tiles: more segments than a wave scans at once, empty ones, prompts
+beside single rows, one long segment; against the CPU forms, with the histories that the convolutions leave behind."""
+import pytest
+import torch
+
+from financial_chatbot_llm_amd.ops import mixers as mx
+
+pytestmark = pytest.mark.gpu
+
+
+def layout(name):
+    g = torch.Generator().manual_seed(7)
+    lens = {"many": torch.randint(0, 70, (150,), generator=g).tolist() + [1] * 40 + [33, 32, 31, 0],
+            "singles": [1] * 130, "one": [777], "two": [3, 1], "wave": [2] * 63 + [40] + [5]}[name]
+    ctx = [n + (i % 3) * 20 for i, n in enumerate(lens)]                     # every third starts at position 0
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    pos = torch.cat([torch.arange(c - n, c) for n, c in zip(lens, ctx)]).int()
+    slot = torch.randperm(len(lens), generator=g).int()
+    slot[len(lens) // 2] = -1 if len(lens) > 4 else slot[len(lens) // 2]     # padding: skipped
+    return lens, ctx, cu, pos, slot, g
+
+
+LAYOUTS = ["many", "singles", "one", "two", "wave"]
+
+
+@pytest.mark.parametrize("name", LAYOUTS)
+@pytest.mark.parametrize("dt,K,C", [(torch.bfloat16, 4, 260), (torch.float32, 3, 65), (torch.bfloat16, 8, 64), (torch.float32, 1, 32),
+                                    (torch.bfloat16, 4, 6400)])             # the last: by four channels where rows are many
+def test_convolution_and_history(name, dt, K, C):
+    lens, _, cu, pos, slot, g = layout(name)
+    T = int(cu[-1])
+    x = torch.randn((T, C + 8), generator=g).to(dt)[:, :C]
+    w, b, ib = torch.randn((C, K), generator=g), torch.randn(C, generator=g), torch.randn(C, generator=g)
+    st = torch.randn((len(lens), K - 1, C), generator=g)
+    want_st, got_st = st.clone(), st.cuda()
+    want = mx.conv_act(x.float(), w, b, want_st, cu, slot, pos, max(lens), in_bias=ib)
+    got = mx.conv_act(x.cuda(), w.cuda(), b.cuda(), got_st, cu.cuda(), slot.cuda(), pos.cuda(), max(lens), in_bias=ib.cuda())
+    live = torch.zeros(T, dtype=torch.bool)
+    for s in range(len(lens)):
+        live[int(cu[s]):int(cu[s + 1])] = int(slot[s]) >= 0
+    assert torch.allclose(got.cpu()[live], want[live], rtol=1e-4, atol=1e-4)
+    assert torch.equal(got_st.cpu(), want_st)
+
+
+@pytest.mark.parametrize("name", LAYOUTS)
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_conv_heads(name, dt):
+    lens, _, cu, pos, slot, g = layout(name)
+    T, H, G, D, P, K = int(cu[-1]), 6, 2, 24, 20, 4
+    C = (H + G) * D + G * P
+    x = torch.randn((T, C), generator=g).to(dt)
+    w, n = torch.randn((C, K), generator=g), torch.rand(D, generator=g)
+    st, slots = torch.randn((len(lens), K - 1, C), generator=g), torch.randperm(T, generator=g).int()
+    cache = torch.zeros((T, G * (D + P)), dtype=dt)
+
+    def run(f, st, cache):
+        return mx.conv_heads(f(x), f(w), st, f(n), f(n), 1e-5, f(cu), f(slot), f(pos), f(slots), cache, max(lens), H, G, D, P, 0.1, 16)
+    want_st, want_c, got_st, got_c = st.clone(), cache.clone(), st.cuda(), cache.cuda()
+    want, got = run(lambda t: t, want_st, want_c), run(lambda t: t.cuda(), got_st, got_c)
+    tol = dict(rtol=2.0 ** -7, atol=2.0 ** -7) if dt == torch.bfloat16 else dict(rtol=1e-4, atol=1e-4)
+    assert torch.allclose(got.float().cpu(), want.float(), **tol) and torch.allclose(got_c.float().cpu(), want_c.float(), **tol)
+    assert torch.equal(got_st.cpu(), want_st)
+
+
+@pytest.mark.parametrize("name", LAYOUTS)
+def test_attention(name):
+    lens, ctx, cu, pos, _, g = layout(name)
+    T, H, G, D = int(cu[-1]), 8, 2, 128
+    need = [max(1, (c + 63) // 64) for c in ctx]
+    bt = torch.zeros((len(lens), max(need)), dtype=torch.int32)
+    o = 0
+    for i, m in enumerate(need):
+        bt[i, :m] = torch.arange(o, o + m)
+        o += m
+    cache, q = torch.randn((o * 64, G * 2 * D), generator=g).to(torch.bfloat16), torch.randn((T, H * D), generator=g).to(torch.bfloat16)
+
+    def run(f):
+        return mx.window_attend(f(q), f(cache), f(cu), f(pos), f(bt), 50, D ** -0.5, max(lens), H, G, D, D)
+    want, got = run(lambda t: t.float() if t.is_floating_point() else t), run(lambda t: t.cuda()).float().cpu()
+    assert ((got - want).abs() <= want.abs() * 2.0 ** -8 + 5 * 2.0 ** -19).all()
