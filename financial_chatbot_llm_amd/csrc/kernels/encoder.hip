@@ -136,9 +136,13 @@ __global__ void __launch_bounds__(256) encoder_attention_kernel(const bf16* __re
 // Bound by latency: a bge projection has 1 - 5 MB of weights, a few microseconds at HBM rate, and the point is enough
 // blocks to ask for them at once.  18 rows, N x K = 2304 x 768: 4.3 us, the 256 x 256 tile kernel 17 us (its 9 tiles split
 // K over the idle CUs and meet in a second phase); 768 x 3072: 8 and 32 us.
-template <int NF, int MF, bool GELU>
+// SLAB: gridDim.z slices of K, slice z's sums to f32 slab z [M, N] (no bias): a long K over few column tiles is 48 blocks that
+// each read 100 KB of weights and twice that of X (18 x 768 x 3072: 8.7 us, in four slices 4.8; the norm that adds
+// them 3.3 us instead of 2.8).
+enum { SMALL_BIAS = 0, SMALL_GELU = 1, SMALL_SLAB = 2 };
+template <int NF, int MF, int EPI>
 __global__ void __launch_bounds__(512) gemm_bias_small_kernel(const bf16* __restrict__ X, int ldx, const bf16* __restrict__ W,
-                                                              int K, bf16* __restrict__ Y, int ldy,
+                                                              int K, void* __restrict__ Yv, int ldy,
                                                               const bf16* __restrict__ bias, int M, int N) {
   constexpr int UN = NF * MF >= 4 ? 3 : 4;
   __shared__ f32x4 red[8][NF * MF][64];
@@ -155,8 +159,9 @@ __global__ void __launch_bounds__(512) gemm_bias_small_kernel(const bf16* __rest
   for (int f = 0; f < NF; ++f)
 #pragma unroll
     for (int u = 0; u < MF; ++u) acc[f][u] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int kt = K / 32, k1 = kt * (w + 1) / 8;
-  int k = kt * w / 8;
+  const int kt = K / 32, part = EPI == SMALL_SLAB ? blockIdx.z * 8 + w : w, parts = EPI == SMALL_SLAB ? gridDim.z * 8 : 8;
+  const int k1 = kt * (part + 1) / parts;
+  int k = kt * part / parts;
   Frag a[UN][NF], b[UN][MF];
   for (; k + UN <= k1; k += UN) {
 #pragma unroll
@@ -194,12 +199,17 @@ __global__ void __launch_bounds__(512) gemm_bias_small_kernel(const bf16* __rest
     f32x4 s = red[0][it][lane];
 #pragma unroll
     for (int i = 1; i < 8; ++i) s += red[i][it][lane];
+    if constexpr (EPI == SMALL_SLAB) {
+      *reinterpret_cast<f32x4*>(static_cast<float*>(Yv) + ((long)blockIdx.z * M + m) * N + n) = s;
+      continue;
+    }
+    bf16* Y = static_cast<bf16*>(Yv);
     const bf16x4 bv = *reinterpret_cast<const bf16x4*>(bias + n);
     bf16x4 y;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       float v = s[r] + (float)bv[r];
-      if (GELU) {
+      if (EPI == SMALL_GELU) {
         v = (float)(bf16)v;                          // rounded where GEMM-with-bias -> bf16 -> GELU rounds
         v = gelu_erf(v);
       }
@@ -237,11 +247,11 @@ PENNY_API int penny_gemm_bias_small(const void* X, int ldx, const void* W, int K
   do {                                                                                                                   \
     const dim3 grid((N + 16 * NF - 1) / (16 * NF), (M + 16 * MF - 1) / (16 * MF));                                       \
     if (gelu)                                                                                                            \
-      gemm_bias_small_kernel<NF, MF, true><<<grid, 512, 0, stream>>>((const bf16*)X, ldx, (const bf16*)W, K, (bf16*)Y,   \
-                                                                     ldy, (const bf16*)bias, M, N);                      \
+      gemm_bias_small_kernel<NF, MF, SMALL_GELU><<<grid, 512, 0, stream>>>((const bf16*)X, ldx, (const bf16*)W, K, Y,    \
+                                                                           ldy, (const bf16*)bias, M, N);                \
     else                                                                                                                 \
-      gemm_bias_small_kernel<NF, MF, false><<<grid, 512, 0, stream>>>((const bf16*)X, ldx, (const bf16*)W, K, (bf16*)Y,  \
-                                                                      ldy, (const bf16*)bias, M, N);                     \
+      gemm_bias_small_kernel<NF, MF, SMALL_BIAS><<<grid, 512, 0, stream>>>((const bf16*)X, ldx, (const bf16*)W, K, Y,    \
+                                                                           ldy, (const bf16*)bias, M, N);                \
   } while (0)
   if (M <= 16) SMALL(1, 1);
   else if (M <= 32) SMALL(1, 2);
@@ -311,6 +321,111 @@ __global__ void __launch_bounds__(256) encoder_pool_kernel(const bf16* __restric
   for (int d = lane; d < H; d += 64) out[(long)i * H + d] = (float)r[d] / n;
 }
 
+// One wave per row: y = LN(bf16(sum of the S slabs + bias) + res); H = 256 C4, arithmetic of layernorm_wave_kernel
+template <int C4>
+__global__ void __launch_bounds__(256) layernorm_slab_kernel(const float* __restrict__ P, int S, const bf16* __restrict__ bias,
+                                                             const bf16* __restrict__ res, const bf16* __restrict__ g,
+                                                             const bf16* __restrict__ b, bf16* __restrict__ y, int T, float eps) {
+  constexpr int H = 256 * C4;
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (row >= T) return;
+  f32x4 p[C4];
+  bf16x4 rv[C4], bv[C4], gg[C4], bb[C4];
+#pragma unroll
+  for (int c = 0; c < C4; ++c) {
+    const int at = lane + 64 * c;
+    p[c] = reinterpret_cast<const f32x4*>(P + (long)row * H)[at];
+    rv[c] = reinterpret_cast<const bf16x4*>(res + (long)row * H)[at];
+    bv[c] = reinterpret_cast<const bf16x4*>(bias)[at];
+    gg[c] = reinterpret_cast<const bf16x4*>(g)[at];
+    bb[c] = reinterpret_cast<const bf16x4*>(b)[at];
+  }
+#pragma unroll 4
+  for (int i = 1; i < S; ++i)
+#pragma unroll
+    for (int c = 0; c < C4; ++c) p[c] += reinterpret_cast<const f32x4*>(P + ((long)i * T + row) * H)[lane + 64 * c];
+  float v[C4][4], s = 0.f, sq = 0.f;
+#pragma unroll
+  for (int c = 0; c < C4; ++c)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[c][i] = (float)(bf16)(p[c][i] + (float)bv[c][i]) + (float)rv[c][i];
+      s += v[c][i];
+    }
+  const float mu = wave_sum(s) / (float)H;
+#pragma unroll
+  for (int c = 0; c < C4; ++c)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float d = v[c][i] - mu;
+      sq += d * d;
+    }
+  const float inv = rsqrtf(wave_sum(sq) / (float)H + eps);
+#pragma unroll
+  for (int c = 0; c < C4; ++c) {
+    bf16x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = (bf16)((v[c][i] - mu) * inv * (float)gg[c][i] + (float)bb[c][i]);
+    reinterpret_cast<bf16x4*>(y + (long)row * H)[lane + 64 * c] = o;
+  }
+}
+
+// Slices of K for the second projection of the feed-forward: as many as bring its blocks near the CUs, 512 of K each at least;
+// 1: not split.  A query of 12 layers of 768 x 3072, us unsplit / in 2 / 3 / 4 / 6: 6 tokens 422 / 412 / 419 / 414 / 414, 18: 467 / 438 /
+// 437 / 441 / 451, 32: 505 / 472 / 466 / 459 / 466, 48: 599 / 536 / 521 / 511 / 523, 64: 634 / 565 / 550 / 545 / 556, 84: 680 / 611 / 623 / 621 /
+// 611, 109: 701 / 627 / 652 / 637 / 640, 179: 743 / 658 / 633 / 669 / 645.
+int small_slices(int M, int N, int K) {
+  if (N != 256 && N != 512 && N != 768 && N != 1024) return 1;
+  const long blocks = M <= 128 ? (long)(N / 16) * ((M + 63) / 64) : (long)((N + 31) / 32) * ((M + 63) / 64);
+  const long s = 216 / blocks, most = K / 512;
+  return (int)(s < most ? (s > 1 ? s : 1) : (most > 1 ? most : 1));
+}
+
+// y = bf16(sum of the S slabs + bias), four columns per thread
+__global__ void __launch_bounds__(256) slab_bias_kernel(const float* __restrict__ P, int S, const bf16* __restrict__ bias,
+                                                        bf16* __restrict__ y, int ldy, int M, int N) {
+  const int c = N / 4, i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= M * c) return;
+  const int row = i / c, n = i % c * 4;
+  f32x4 p = *reinterpret_cast<const f32x4*>(P + (long)row * N + n);
+#pragma unroll 4
+  for (int z = 1; z < S; ++z) p += *reinterpret_cast<const f32x4*>(P + ((long)z * M + row) * N + n);
+  const bf16x4 bv = *reinterpret_cast<const bf16x4*>(bias + n);
+  bf16x4 o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) o[j] = (bf16)(p[j] + (float)bv[j]);
+  *reinterpret_cast<bf16x4*>(y + (long)row * ldy + n) = o;
+}
+
+// S slices of K of X W^T to f32 slabs [S, M, N]
+int small_slabs(const void* X, int ldx, const void* W, float* slabs, int S, int M, int N, int K, hipStream_t stream) {
+#define SLABS(NF, MF)                                                                                                    \
+  gemm_bias_small_kernel<NF, MF, SMALL_SLAB><<<dim3((N + 16 * NF - 1) / (16 * NF), (M + 16 * MF - 1) / (16 * MF), S), 512, 0, stream>>>( \
+      (const bf16*)X, ldx, (const bf16*)W, K, slabs, N, nullptr, M, N)
+  if (M <= 16) SLABS(1, 1);
+  else if (M <= 32) SLABS(1, 2);
+  else if (M <= 128) SLABS(1, 4);
+  else SLABS(2, 4);
+#undef SLABS
+  return (int)hipGetLastError();
+}
+
+// y = LN(bf16(X W^T + bias) + res) by slabs
+int small_slab_norm(const void* X, const void* W, const void* bias, const void* res, const void* g, const void* b, void* y, float* slabs,
+                    int S, int M, int N, int K, float eps, hipStream_t stream) {
+  const int rc = small_slabs(X, K, W, slabs, S, M, N, K, stream);
+  if (rc) return rc;
+#define NORM(C4)                                                                                                        \
+  layernorm_slab_kernel<C4><<<(M + 3) / 4, 256, 0, stream>>>(slabs, S, (const bf16*)bias, (const bf16*)res, (const bf16*)g, \
+                                                             (const bf16*)b, (bf16*)y, M, eps)
+  if (N == 256) NORM(1);
+  else if (N == 512) NORM(2);
+  else if (N == 768) NORM(3);
+  else NORM(4);
+#undef NORM
+  PENNY_RETURN_LAUNCH();
+}
+
 }  // namespace
 
 // ids, pos [T] int32; word [nword, H], position [npos, H], type [>= 1, H], g, b [H], y [T, H] bf16; H = 256, 512, 768 or 1024
@@ -338,6 +453,22 @@ PENNY_API int penny_encoder_pool(const void* x, const int* cu, int texts, int H,
   PENNY_RETURN_LAUNCH();
 }
 
+PENNY_API int penny_encoder_slices(int T, int H, int F) { return small_slices(T, H, F); }
+
+// penny_gemm_bias_small without GELU by S = penny_encoder_slices(M, N, K) > 1 slices; slabs: f32 [S, M, N].  The sums are those of
+// the layers' slab norm.
+PENNY_API int penny_gemm_bias_small_split(const void* X, int ldx, const void* W, int K, void* Y, int ldy, const void* bias, int M, int N,
+                                          float* slabs, int S, hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (S < 2 || S != small_slices(M, N, K) || K % 32 || ldx % 8 || ldy % 4 || ((size_t)X | (size_t)W | (size_t)slabs) % 16 ||
+      ((size_t)Y | (size_t)bias) % 8)
+    return (int)hipErrorInvalidValue;
+  const int rc = small_slabs(X, ldx, W, slabs, S, M, N, K, stream);
+  if (rc) return rc;
+  slab_bias_kernel<<<(M * (N / 4) + 255) / 256, 256, 0, stream>>>(slabs, S, (const bf16*)bias, (bf16*)Y, ldy, M, N);
+  PENNY_RETURN_LAUNCH();
+}
+
 PENNY_API int penny_layernorm(const void* x, const void* res, const void* g, const void* b, void* y, int T, int H, float eps,
                               int add_residual, hipStream_t stream);
 
@@ -345,7 +476,7 @@ constexpr int PENNY_MISALIGNED = -1;
 
 // All layers of a small batch: x [T, H] bf16 is replaced by the last layer's output.  w: 12 pointers per layer -- qkv, its
 // bias, o, its bias, the first norm's weight and bias, fc1, its bias, fc2, its bias, the second norm's weight and bias, each
-// contiguous bf16.  ws: T * (6 H + F) bf16.  Shapes as penny_gemm_bias_small, penny_encoder_attention and penny_layernorm take
+// contiguous bf16.  ws: T * (6 H + F) bf16, then f32 slabs [penny_encoder_slices(T, H, F), T, H] where that is more than 1.  Shapes as penny_gemm_bias_small, penny_encoder_attention and penny_layernorm take
 // them; PENNY_MISALIGNED, and nothing launched, for a weight off their 16 bytes (asked here: 144 weights take 18 us in Python).
 // The launches of one layer take the host 8 x 2.5 us here and 8 x 7 from Python, where the kernels of a single query
 // (18 tokens, 12 layers of 768) run for 440 us in all: 815 -> 497 us for the query.
@@ -358,6 +489,8 @@ PENNY_API int penny_encoder_layers(const void* const* w, int layers, void* x, vo
   if (at % 16) return PENNY_MISALIGNED;
   bf16* qkv = static_cast<bf16*>(ws);
   bf16 *a = qkv + (long)T * 3 * H, *o = a + (long)T * H, *mid = o + (long)T * H, *h = mid + (long)T * H;
+  float* slabs = reinterpret_cast<float*>(h + (long)T * F);
+  const int slices = small_slices(T, H, F);
   int rc = 0;
   for (int i = 0; i < layers && rc == 0; ++i, w += 12) {
     rc = penny_gemm_bias_small(x, H, w[0], H, qkv, 3 * H, w[1], T, 3 * H, 0, stream);
@@ -365,8 +498,12 @@ PENNY_API int penny_encoder_layers(const void* const* w, int layers, void* x, vo
     if (rc == 0) rc = penny_gemm_bias_small(a, H, w[2], H, o, H, w[3], T, H, 0, stream);
     if (rc == 0) rc = penny_layernorm(o, x, w[4], w[5], mid, T, H, eps, 1, stream);
     if (rc == 0) rc = penny_gemm_bias_small(mid, H, w[6], H, h, F, w[7], T, F, 1, stream);
-    if (rc == 0) rc = penny_gemm_bias_small(h, F, w[8], F, o, H, w[9], T, H, 0, stream);
-    if (rc == 0) rc = penny_layernorm(o, mid, w[10], w[11], x, T, H, eps, 1, stream);
+    if (rc == 0 && slices > 1) {
+      rc = small_slab_norm(h, w[8], w[9], mid, w[10], w[11], x, slabs, slices, T, H, F, eps, stream);
+    } else {
+      if (rc == 0) rc = penny_gemm_bias_small(h, F, w[8], F, o, H, w[9], T, H, 0, stream);
+      if (rc == 0) rc = penny_layernorm(o, mid, w[10], w[11], x, T, H, eps, 1, stream);
+    }
   }
   return rc;
 }

@@ -96,8 +96,10 @@ class BertEncoder:
                 [t.shape for t in w] != self.layer_shapes:
             return False
         table = (ctypes.c_void_p * len(w))(*[t.data_ptr() for t in w])
-        scratch = torch.empty(T * (6 * self.H + F_), dtype=torch.bfloat16, device=x.device)
-        rc = N.load().penny_encoder_layers(table, self.cfg.num_layers, N.ptr(x), N.ptr(scratch), N.ptr(cu), cu.numel() - 1, longest,
+        lib = N.load()
+        slices = lib.penny_encoder_slices(T, self.H, F_)
+        scratch = torch.empty(T * (6 * self.H + F_ + (2 * slices * self.H if slices > 1 else 0)), dtype=torch.bfloat16, device=x.device)
+        rc = lib.penny_encoder_layers(table, self.cfg.num_layers, N.ptr(x), N.ptr(scratch), N.ptr(cu), cu.numel() - 1, longest,
                                            T, self.H, self.nh, F_, float(self.cfg.norm_eps), 1.0 / math.sqrt(self.D), N.stream())
         if rc > 0:
             raise RuntimeError(f"penny_encoder_layers failed with hipError {rc}")

@@ -31,6 +31,8 @@ _SIGS = {
     "penny_encoder_embed": [P, P, P, c_int, P, c_int, P, P, P, P, c_int, c_int, c_float, P],
     "penny_encoder_pool": [P, P, c_int, c_int, P, P],
     "penny_encoder_layers": [P, c_int, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, P],
+    "penny_gemm_bias_small_split": [P, c_int, P, c_int, P, c_int, P, c_int, c_int, P, c_int, P],
+    "penny_encoder_slices": [c_int, c_int, c_int],
     "penny_layernorm": [P, P, P, P, P, c_int, c_int, c_float, c_int, P],
     "penny_silu_mul": [P, P, c_int, c_int, c_int, P],
     "penny_skinny_gemm": [P, c_int, P, c_int, P, c_int, P, c_int, c_int, c_int, c_int, c_int, c_int, P],

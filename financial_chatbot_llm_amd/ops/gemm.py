@@ -798,6 +798,12 @@ def linear_bias(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, gelu: bool = 
     mode = os.environ.get("PENNY_PREFILL_GEMM", "1")
     if mode == "1" and small_bias_wins(M, N_, K) and small_bias_ok(x, w) and _bias_row(b, w):
         y = torch.empty((M, N_), dtype=x.dtype, device=x.device)
+        slices = 1 if gelu else N.load().penny_encoder_slices(M, N_, K)
+        if slices > 1:                   # a long K over few column tiles
+            slabs = torch.empty((slices, M, N_), dtype=torch.float32, device=x.device)
+            N.call("penny_gemm_bias_small_split", N.ptr(x), x.stride(0), N.ptr(w), K, N.ptr(y), N_, N.ptr(b), M, N_, N.ptr(slabs),
+                   slices, N.stream())
+            return y
         N.call("penny_gemm_bias_small", N.ptr(x), x.stride(0), N.ptr(w), K, N.ptr(y), N_, N.ptr(b), M, N_, int(gelu),
                N.stream())
         return y

@@ -129,6 +129,21 @@ def test_small_batches_in_one_call(lens, monkeypatch):
     assert e.shape == want.shape and float((e - want).abs().max()) < 1e-6      # f32 sums of 768 squares in another order
 
 
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64, 65, 128, 129, 256, 257])
+@pytest.mark.parametrize("N,K", [(256, 1024), (512, 2080), (768, 3072), (1024, 4096), (768, 1536), (1024, 96)])
+def test_sliced_projection(M, N, K):
+    """A long K over few columns goes by slices where those fill the chip; the norm behind it adds them up to the same values."""
+    from financial_chatbot_llm_amd.ops import _native as nat, gemm
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)  # noqa: E731
+    x, w, b = r(M, K + 8)[:, :K], r(N, K) * K ** -0.5, r(N)
+    S = nat.load().penny_encoder_slices(M, N, K)
+    assert 1 <= S <= max(1, K // 512) and nat.load().penny_encoder_slices(18, 768, 3072) == 4
+    got = gemm.linear_bias(x, w, b).float()
+    want = x.double() @ w.double().T + b.double()
+    assert float((got - want).norm() / want.norm()) < 4e-3                        # one rounding to bf16
+
+
 def test_encoder_embed_edges():
     """Fused embedding rows against the separate ops: last and out-of-table ids, every supported width."""
     from financial_chatbot_llm_amd import ops
