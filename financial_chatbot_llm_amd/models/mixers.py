@@ -227,8 +227,8 @@ class LatentAttentionMixer:
         self.dq_norm = get("dq.norm").float().contiguous()
         self.dkv_norm = get("dkv.norm").float().contiguous()
         self.uq = get("uq").to(dtype).contiguous()
-        self.uk = get("uk").to(dtype).view(self.H, self.dn, self.R).contiguous()      # [H, dn, R]
-        self.uv_t = get("uv").to(dtype).view(self.H, self.dv, self.R).transpose(1, 2).contiguous()  # [H, R, dv]
+        self.uk = mx.HeadLinear(get("uk").to(dtype).view(self.H, self.dn, self.R).transpose(1, 2))    # [H, R, dn]
+        self.uv = mx.HeadLinear(get("uv").to(dtype).view(self.H, self.dv, self.R))                    # [H, dv, R]
         self.o = get("o").to(dtype).contiguous()
         self.rot.to(self.uq.device)
         if self.rot.freq is None:
@@ -237,7 +237,7 @@ class LatentAttentionMixer:
         return torch.cat([get("dq"), get("dkv")] + ([get("g")] if self.gated else []), 0).to(dtype)
 
     def num_bytes(self) -> int:
-        return sum(t.numel() * t.element_size() for t in (self.uq, self.uk, self.uv_t, self.o))
+        return sum(t.numel() * t.element_size() for t in (self.uq, self.o)) + self.uk.num_bytes() + self.uv.num_bytes()
 
     def forward(self, proj: torch.Tensor, positions: torch.Tensor, meta: AttentionMetadata, cache) -> torch.Tensor:
         rows = cache[1]
@@ -253,11 +253,10 @@ class LatentAttentionMixer:
                                q, H, dn + dr, dn, R, dr, self.rot.mscale)
         # fold each head's key up-projection into its query: q_lat[h] = W_uk[h]^T q_nope[h]
         q_nope = q.view(T, H, dn + dr)[:, :, :dn]
-        q_lat = torch.bmm(q_nope.transpose(0, 1), self.uk).transpose(0, 1).contiguous()   # [T, H, R]
+        q_lat = self.uk(q_nope)                                              # [T, H, R]
         o_lat = mx.latent_attend(q_lat, q_rot, rows, meta.seg_cu, positions, meta.seg_bt, self.window, self.scale,
                                  meta.seg_max_len, gate=gate, sink=self.sink, exact_weights=self.exact_weights)
-        o = torch.bmm(o_lat.transpose(0, 1), self.uv_t).transpose(0, 1).reshape(T, H * self.dv)
-        return F.linear(o, self.o)
+        return F.linear(self.uv(o_lat).view(T, H * self.dv), self.o)
 
 
 class SinkLatentAttentionMixer(LatentAttentionMixer):
@@ -1049,14 +1048,14 @@ class PlainLatentAttentionMixer:
 
     def load(self, get: Getter, dtype) -> torch.Tensor:
         self.dkv_norm = _f32(get, "dkv.norm")
-        self.uk = get("uk").to(dtype).view(self.H, self.D, self.R).contiguous()                       # [H, D, R]
-        self.uv_t = get("uv").to(dtype).view(self.H, self.P, self.R).transpose(1, 2).contiguous()     # [H, R, P]
+        self.uk = mx.HeadLinear(get("uk").to(dtype).view(self.H, self.D, self.R).transpose(1, 2))     # [H, R, D]
+        self.uv = mx.HeadLinear(get("uv").to(dtype).view(self.H, self.P, self.R))                     # [H, P, R]
         self.o = get("o").to(dtype).contiguous()
         self.no_freq = torch.zeros(0, dtype=torch.float32, device=self.o.device)
         return torch.cat([get("q"), get("dkv")], 0).to(dtype)
 
     def num_bytes(self) -> int:
-        return sum(t.numel() * t.element_size() for t in (self.uk, self.uv_t, self.o))
+        return self.o.numel() * self.o.element_size() + self.uk.num_bytes() + self.uv.num_bytes()
 
     def forward(self, proj: torch.Tensor, positions: torch.Tensor, meta: AttentionMetadata, cache) -> torch.Tensor:
         rows = cache[1]
@@ -1066,11 +1065,10 @@ class PlainLatentAttentionMixer:
         # the normed latent into the cache (no rotated part: the returned rotated query part is empty)
         q_rot = mx.latent_prep(proj[:, self.nq:self.nq + R], self.dkv_norm, self.eps, self.no_freq, 0, positions,
                                meta.slots, rows, q, H, D, D, R, 0)
-        q_lat = torch.bmm(q.reshape(T, H, D).transpose(0, 1), self.uk).transpose(0, 1).contiguous()     # [T, H, R]
+        q_lat = self.uk(q.unflatten(1, (H, D)))                                                         # [T, H, R]
         o_lat = mx.latent_attend(q_lat, q_rot, rows, meta.seg_cu, positions, meta.seg_bt, self.window, self.scale,
                                  meta.seg_max_len)
-        o = torch.bmm(o_lat.transpose(0, 1), self.uv_t).transpose(0, 1).reshape(T, H * self.P)
-        return F.linear(o, self.o)
+        return F.linear(self.uv(o_lat).view(T, H * self.P), self.o)
 
 
 class ConvAttentionMixer:

@@ -130,6 +130,7 @@ _MIXER_SIGS = {
                       c_float, c_float, P, c_int, P, c_long, c_int, P, P, c_long, c_int, P, c_long, c_float, c_int, P],
     "mx_logit_cap": [P, c_int, c_float, c_float, c_long, P],
     "mx_ssm_scan": [P, c_int, P, c_long, c_int, P, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, P, P],
+    "mx_head_linear": [P, c_long, c_long, P, P, c_int, c_int, c_int, c_int, c_int, P],
     "mx_latent_prep": [P, c_long, P, c_float, P, c_int, c_float, P, P, P, P, c_long, c_int, c_int, P, c_int, c_int, c_int,
                        c_int, c_int, P],
     "mx_latent_attend": [P, P, P, P, P, P, c_int, P, c_long, P, c_int, c_int, c_float, P, c_int, c_int, c_int, c_int, c_int,

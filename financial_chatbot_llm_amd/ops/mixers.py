@@ -534,6 +534,36 @@ def _sink_softmax(sc: torch.Tensor, sink: Optional[torch.Tensor]) -> torch.Tenso
     return torch.softmax(torch.cat([sc, extra], -1), -1)[..., :-1]
 
 
+class HeadLinear:
+    """y[t, h] = W[h] x[t, h]: a matrix per head, ``w`` [H, N, K].  On the GPU the rows of heads are read and written where they lie
+    (``mx_head_linear``); sizes that the kernel does not take (N in whole 16, rows of whole 64 bytes) and the CPU go through a
+    batched product."""
+
+    def __init__(self, w: torch.Tensor):
+        H, self.N, K = w.shape
+        self.native = N.use_native(w) and w.dtype in (torch.bfloat16, torch.float32) and self.N % 16 == 0 and \
+            K * w.element_size() % 64 == 0 and H <= 65535
+        # the batched product's right operand lies as it reads it
+        self.w = w.contiguous() if self.native else w.transpose(1, 2).contiguous()
+
+    def __call__(self, x: torch.Tensor) -> torch.Tensor:
+        """x [T, H, K] (any strides) -> [T, H, N] contiguous."""
+        T, H, K = x.shape
+        if not self.native:
+            return torch.bmm(x.transpose(0, 1), self.w).transpose(0, 1).contiguous()
+        if x.dtype != self.w.dtype or (H, K) != (self.w.shape[0], self.w.shape[2]):
+            raise ValueError("one row of the matrices' width per head, of their type")
+        es = x.element_size()
+        if x.stride(2) != 1 or x.stride(0) * es % 16 or x.stride(1) * es % 16 or x.data_ptr() % 16:
+            x = x.clone(memory_format=torch.contiguous_format)
+        y = torch.empty((T, H, self.N), dtype=x.dtype, device=x.device)
+        N.mcall("mx_head_linear", N.ptr(x), x.stride(0), x.stride(1), N.ptr(self.w), N.ptr(y), T, H, self.N, K, _dt(x), N.stream())
+        return y
+
+    def num_bytes(self) -> int:
+        return self.w.numel() * self.w.element_size()
+
+
 @functools.lru_cache(maxsize=1024)          # the estimate takes 1 - 5 us
 def _key_parts(keys: int, blocks: int, most_blocks: int, pairs: int, width: int, dtype: torch.dtype) -> int:
     """How many blocks walk the keys of the same queries in the tiled attention (at most ``most_blocks`` over ``blocks``), for
