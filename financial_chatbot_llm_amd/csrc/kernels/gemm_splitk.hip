@@ -179,7 +179,8 @@ __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restr
   X += (long)m0 * ldx;
   if constexpr (EPI == SK_SILU || EPI == SK_BF16) Y += (long)m0 * ldy;
   PENNY_DASSERT(M > 0 && (EPI != SK_SAMPLE || gridDim.y == 1));
-  PENNY_DASSERT((tile + 1) * 16 * NF <= N && K % (64 * BKM * S) == 0);
+  PENNY_DASSERT((tile + 1) * 16 * NF <= N || (WROW && N % 16 == 0 && tile * 16 * NF < N && (EPI == SK_BF16 || EPI == SK_SLAB)));
+  PENNY_DASSERT(K % (64 * BKM * S) == 0);
   const int n0 = tile * 16 * NF;
   const int kc = K / S, k0 = s * kc;
   const int nst = kc / (64 * BKM);              // ring slots to stream
@@ -197,7 +198,8 @@ __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restr
     if (q < 2 * NF && WROW) {
       const int r = q * 8 + (lane >> 3);                    // weight row within the tile
       const int c = xswz(r, lane & 7);
-      src[i] = reinterpret_cast<const char*>(Wt + (long)(n0 + r) * K + k0 + 8 * c);
+      // the last tile of N % (16 NF) != 0 (penny_linear_rows) reads its last row again; those columns are not stored
+      src[i] = reinterpret_cast<const char*>(Wt + (long)min(n0 + r, N - 1) * K + k0 + 8 * c);
       step[i] = 128;       // 64 k per stage
       dst[i] = q * 1024;
     } else if (q < 2 * NF) {
@@ -276,6 +278,7 @@ __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restr
       if (m >= M) continue;
 #pragma unroll
       for (int f = 0; f < FW; ++f) {
+        if (WROW && n0 + (wa * FW + f) * 16 >= N) break;
         bf16x4 o;
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[r] = (bf16)acc[f][t][r];
@@ -331,6 +334,7 @@ __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restr
 #pragma unroll
     for (int f = 0; f < FW; ++f) {
       const int n = n0 + (wa * FW + f) * 16 + 4 * g;
+      if (WROW && n >= N) break;
       *reinterpret_cast<f32x4*>(ps + (long)m * N + n) = acc[f][t];
     }
   }
@@ -396,7 +400,7 @@ int launch_any(int wrow, bool pair_ok, dim3 grid, hipStream_t st, A... args) {
 
 template <int NF, int MT, int WA>
 int launch(const void* X, int ldx, const void* Wt, int K, float* P, int M, int N, int S, int wrow, hipStream_t st) {
-  return launch_any<NF, MT, WA, SK_SLAB, 8>(wrow, (K / S) % 128 == 0, dim3((N / (16 * NF)) * S, (M + 16 * MT - 1) / (16 * MT)), st, (const bf16*)X,
+  return launch_any<NF, MT, WA, SK_SLAB, 8>(wrow, (K / S) % 128 == 0, dim3(((N + 16 * NF - 1) / (16 * NF)) * S, (M + 16 * MT - 1) / (16 * MT)), st, (const bf16*)X,
                                             ldx, (const bf16*)Wt, K, P, M, N, S, (bf16*)nullptr, 0, SkSample{});
 }
 
@@ -411,7 +415,7 @@ int launch_silu(const void* X, int ldx, const void* Wt, int K, void* Y, int ldy,
 template <int NF, int MT, int WA>
 int launch_bf16(const void* X, int ldx, const void* Wt, int K, void* Y, int ldy, int M, int N, int wrow,
                 hipStream_t st) {
-  return launch_any<NF, MT, WA, SK_BF16, 16>(wrow, K % 128 == 0, dim3(N / (16 * NF), (M + 16 * MT - 1) / (16 * MT)), st, (const bf16*)X, ldx,
+  return launch_any<NF, MT, WA, SK_BF16, 16>(wrow, K % 128 == 0, dim3((N + 16 * NF - 1) / (16 * NF), (M + 16 * MT - 1) / (16 * MT)), st, (const bf16*)X, ldx,
                                              (const bf16*)Wt, K, (float*)nullptr, M, N, 1, (bf16*)Y, ldy, SkSample{});
 }
 
@@ -586,6 +590,35 @@ PENNY_API int penny_splitk_gemm_bf16(const void* X, int ldx, const void* Wt, int
   BF_CASE(16, 1, 1, 2)
 #undef BF_CASE
   return (int)hipErrorInvalidValue;
+}
+
+// Y [M, N] = X [M, K] x W [N, K]^T in bf16 for the few rows of a decode step, W row-major: slabs == null streams W once
+// (S = 1), else S slices of K leave f32 slabs [S, M, N] that a second launch adds.  One entry for both, so that a step that
+// the host bounds pays for one call.  Contract (checked): 1 <= M <= 96, N % 16 == 0 (the last tile of 16 * nf columns may be
+// part-filled), nf in {2, 4}, K % (64 * S) == 0, ldx % 8 == 0, ldy % 8 == 0.
+PENNY_API int penny_linear_rows(const void* X, int ldx, const void* W, int K, void* Y, int ldy, int M, int N, void* slabs,
+                                int S, int nf, int paired, hipStream_t st) {
+  if (M <= 0) return 0;
+  if (M > 96 || N <= 0 || N % 16 || (nf != 2 && nf != 4) || S < 1 || (S > 1) != (slabs != nullptr) || K <= 0 ||
+      K % (64 * S) || ldx % 8 || ldy % 8)
+    return (int)hipErrorInvalidValue;
+  const int wrow = paired ? 3 : 1, mt = (M + 15) / 16;
+  float* p = static_cast<float*>(slabs);
+  int rc;
+#define LR_CASE(MT_, WA_)                                                                                    \
+  if (mt <= MT_) {                                                                                           \
+    if (S > 1) rc = nf == 2 ? launch<2, MT_, WA_>(X, ldx, W, K, p, M, N, S, wrow, st)                        \
+                            : launch<4, MT_, WA_>(X, ldx, W, K, p, M, N, S, wrow, st);                       \
+    else rc = nf == 2 ? launch_bf16<2, MT_, WA_>(X, ldx, W, K, Y, ldy, M, N, wrow, st)                       \
+                      : launch_bf16<4, MT_, WA_>(X, ldx, W, K, Y, ldy, M, N, wrow, st);                      \
+  } else
+  LR_CASE(2, 2)
+  LR_CASE(4, 1)
+  LR_CASE(6, 2)
+  return (int)hipErrorInvalidValue;
+#undef LR_CASE
+  if (rc || S == 1) return rc;
+  return penny_splitk_reduce(slabs, S, M, N, Y, ldy, nullptr, 0, st);
 }
 
 // Weight-streaming LM head + sampler (K11 + K12) for decode batches, full vocabulary or a TP rank's

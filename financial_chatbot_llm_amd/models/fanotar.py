@@ -26,9 +26,9 @@ from __future__ import annotations
 from typing import Dict
 
 import torch
-import torch.nn.functional as F
 
 from ..ops import mixers as mx
+from ..ops.gemm import project
 from .common import AttentionMetadata, HybridCache
 from .configs import ModelConfig
 from .layered import Layer, LayeredDecoder
@@ -151,13 +151,13 @@ class FanotarModel(LayeredDecoder):
         x, h = mx.dyn_tanh_embed(ids, self.embed, self.embed_scale, self.embed_dt, self.layers[0].dt["norm1"], dt)
         for i, l in enumerate(self.layers):
             m = l.mixer
-            y = m.forward(F.linear(h, l.w_in), positions, meta, kv.layers[i],
+            y = m.forward(project(h, l.w_in), positions, meta, kv.layers[i],
                           kv_cache=kv.layers[m.kv_from] if m.kv_from is not None else None)
             nxt = self.layers[i + 1].dt["norm1"] if i + 1 < n else self.final_dt
             # the norm of this sublayer's output, the residual sum and the norm of what comes next: one pass
             h = mx.dyn_tanh_residual(x, y, l.dt["norm1b"], l.dt["norm2"] if l.ff is not None else nxt, dt)
             if l.ff is not None:
-                y = l.ff.forward(h, F.linear(h, l.w_ff) if l.w_ff is not None else None)
+                y = l.ff.forward(h, project(h, l.w_ff) if l.w_ff is not None else None)
                 h = mx.dyn_tanh_residual(x, y, l.dt["norm2b"], nxt, dt)
             if self.capture is not None:
                 self.capture.append(x.clone())

@@ -20,9 +20,9 @@ import math
 from typing import Dict, List, Optional
 
 import torch
-import torch.nn.functional as F
 
 from ..ops import mixers as mx
+from ..ops.gemm import project
 from .common import AttentionMetadata, HybridCache
 from .configs import ModelConfig
 from .layered import Layer, LayeredDecoder
@@ -102,7 +102,7 @@ class GezavikModel(LayeredDecoder):
         h = mx.residual_norm(x, self.layers[0].norm1, eps, out_dtype=self.dtype)
         n = len(self.layers)
         for i, l in enumerate(self.layers):
-            proj = F.linear(h, l.w_in)
+            proj = project(h, l.w_in)
             nm = l.mixer.in_rows
             a = l.mixer.forward(proj[:, :nm], positions, meta, kv.layers[i])
             b = l.ff.forward(h, proj[:, nm:]) if l.ff is not None else None

@@ -15,8 +15,8 @@ import math
 from typing import Callable, Dict, List, NamedTuple, Optional
 
 import torch
-import torch.nn.functional as F
 
+from ..ops.gemm import project
 from .common import HybridCache, param_seed
 from .configs import ModelConfig
 from .mixers import MIXERS
@@ -218,4 +218,4 @@ class LayeredDecoder:
         return self.head
 
     def logits(self, h: torch.Tensor) -> torch.Tensor:
-        return F.linear(h, self.head)
+        return project(h, self.head)

@@ -57,8 +57,8 @@ projection's rank).
 
 Every block declares the rows it needs from a fused in-projection (``in_weight``): a layer stacks
 its mixer's and its feed-forward's rows into ONE GEMM over ``h`` and hands each block its column
-slice.  Plain GEMMs are vendor matrix products (``F.linear`` / ``bmm``) on bf16 or f32 weights; the routed experts and
-everything else run on the kernels behind :mod:`..ops.mixers`.
+slice.  Plain GEMMs on bf16 weights stream through the framework's kernels for a decode step's few rows and are library
+products for the rest (:func:`..ops.gemm.project`); everything else runs on the kernels behind :mod:`..ops.mixers`.
 """
 from __future__ import annotations
 
@@ -68,6 +68,7 @@ import torch
 import torch.nn.functional as F
 
 from ..ops import _native as N, mixers as mx
+from ..ops.gemm import project
 from .common import AttentionMetadata
 
 Getter = Callable[[str], torch.Tensor]
@@ -179,7 +180,7 @@ class Mamba2Mixer:
                         self.H, self.P, self.N, self.G, meta.seg_max_len)
         # the gate comes before the norm: rms over silu(z) * y, in norm_groups equal parts
         yn = mx.group_norm(y, self.norm_w, self.eps, self.norm_groups, gate=z, out_dtype=proj.dtype)
-        return F.linear(yn, self.o)
+        return project(yn, self.o)
 
 
 class LatentAttentionMixer:
@@ -247,7 +248,7 @@ class LatentAttentionMixer:
         cq = mx.group_norm(proj[:, :a], self.dq_norm, self.eps, 1)
         kv = proj[:, a:a + R + dr]
         gate = proj[:, a + R + dr:a + R + dr + H] if self.gated else None
-        q = F.linear(cq, self.uq)                                            # [T, H * (dn + dr)]
+        q = project(cq, self.uq)                                            # [T, H * (dn + dr)]
         # latent row + shared rotated key into the cache; every head's rotated query part
         q_rot = mx.latent_prep(kv, self.dkv_norm, self.eps, self.rot.freq, self.rot_dims, positions, meta.slots, rows,
                                q, H, dn + dr, dn, R, dr, self.rot.mscale)
@@ -256,7 +257,7 @@ class LatentAttentionMixer:
         q_lat = self.uk(q_nope)                                              # [T, H, R]
         o_lat = mx.latent_attend(q_lat, q_rot, rows, meta.seg_cu, positions, meta.seg_bt, self.window, self.scale,
                                  meta.seg_max_len, gate=gate, sink=self.sink, exact_weights=self.exact_weights)
-        return F.linear(self.uv(o_lat).view(T, H * self.dv), self.o)
+        return project(self.uv(o_lat).view(T, H * self.dv), self.o)
 
 
 class SinkLatentAttentionMixer(LatentAttentionMixer):
@@ -297,10 +298,10 @@ class DenseFF:
         if self.gated:
             gate, up = proj[:, :self.ff], proj[:, self.ff:2 * self.ff]
             if self.act == "clamped":
-                return F.linear(mx.glu_clamp(gate, up, self.limit, self.alpha), self.down)
-            return F.linear(mx.glu_act(gate, up, self.act), self.down)
+                return project(mx.glu_clamp(gate, up, self.limit, self.alpha), self.down)
+            return project(mx.glu_act(gate, up, self.act), self.down)
         up = proj[:, :self.ff]
-        return F.linear(mx.relu2(up) if self.act == "relu2" else mx.glu_act(up, None, self.act), self.down)
+        return project(mx.relu2(up) if self.act == "relu2" else mx.glu_act(up, None, self.act), self.down)
 
 
 class RoutedFF:
@@ -357,8 +358,8 @@ class RoutedFF:
         top = self.top
         shared = None
         if self.Fs:
-            shared = F.linear(mx.glu_clamp(proj[:, :self.Fs], proj[:, self.Fs:2 * self.Fs], self.limit_s, self.alpha),
-                              self.down_s)
+            shared = project(mx.glu_clamp(proj[:, :self.Fs], proj[:, self.Fs:2 * self.Fs], self.limit_s, self.alpha),
+                             self.down_s)
         if self.score == "softmax_top":
             wts, idx = mx.router_scores(h, self.router, self.correction, top, "softmax_top")
         else:
@@ -447,7 +448,7 @@ class TopSoftmaxRoutedFF:
         return self.bank.num_bytes() + sum(t.numel() * t.element_size() for t in ts)
 
     def forward(self, h: torch.Tensor, proj: Optional[torch.Tensor] = None, x32: Optional[torch.Tensor] = None) -> torch.Tensor:
-        shared = F.linear(mx.relu2(proj[:, :self.Fs]), self.down_s) if self.Fs else None
+        shared = project(mx.relu2(proj[:, :self.Fs]), self.down_s) if self.Fs else None
         wts, idx = mx.router_scores(x32 if x32 is not None else h, self.router, None, self.top, "softmax_top")
         ys, pos = self.bank.run(h, idx, "relu2")
         return mx.moe_combine(ys, pos, idx, wts, h, shared, self.E)
@@ -512,8 +513,8 @@ class ChannelDeltaMixer:
         o = mx.matrix_scan(u[:, :nq], u[:, nq:2 * nq], u[:, 2 * nq:], a, self.dt_bias, st["S"], meta.seg_cu,
                            meta.seg_state, positions, H, self.G, self.D, self.P, "delta", A_log=self.A_log, beta=beta,
                            max_len=meta.seg_max_len)
-        gate = F.linear(proj[:, C + H + self.ra:C + H + self.ra + self.rg], self.g2)
-        return F.linear(mx.head_norm_gate(o, self.norm_w, self.eps, gate, H, "sigmoid", proj.dtype), self.o)
+        gate = project(proj[:, C + H + self.ra:C + H + self.ra + self.rg], self.g2)
+        return project(mx.head_norm_gate(o, self.norm_w, self.eps, gate, H, "sigmoid", proj.dtype), self.o)
 
 
 class GLAMixer:
@@ -558,7 +559,7 @@ class GLAMixer:
                            meta.seg_cu, meta.seg_state, positions, self.H, self.H, self.D, self.P, "gla", tau=self.tau,
                            max_len=meta.seg_max_len)
         gate = proj[:, 2 * nq + nv:2 * nq + 2 * nv]
-        return F.linear(mx.head_norm_gate(o, self.norm_w, self.eps, gate, self.H, "silu", proj.dtype), self.o)
+        return project(mx.head_norm_gate(o, self.norm_w, self.eps, gate, self.H, "silu", proj.dtype), self.o)
 
 
 class WindowAttentionMixer:
@@ -605,7 +606,7 @@ class WindowAttentionMixer:
         gate = proj[:, nq + nk + nv:nq + nk + nv + self.H]
         o = mx.window_attend(q, rows, meta.seg_cu, positions, meta.seg_bt, self.window, self.scale, meta.seg_max_len,
                              self.H, self.G, self.D, self.P, gate=gate)
-        return F.linear(o, self.o)
+        return project(o, self.o)
 
 
 class GatedLRUMixer:
@@ -652,7 +653,7 @@ class GatedLRUMixer:
         z = torch.bmm(u.view(T, B, bs).transpose(0, 1), self.w_ri)             # [B, T, 2 bs]: r | i pre-activations
         s = mx.lru_scan(u, z, B, self.r_b, self.i_b, self.lam, proj[:, :R], self.y_b, st["S"], meta.seg_cu,
                         meta.seg_state, positions, proj.dtype, max_len=meta.seg_max_len)
-        return F.linear(s, self.o)
+        return project(s, self.o)
 
 
 def _decays(spec: Dict, heads: int) -> torch.Tensor:
@@ -702,7 +703,7 @@ class LightningMixer:
         o = mx.decay_scan(proj[:, :nq], proj[:, nq:2 * nq], proj[:, 2 * nq:2 * nq + nv], self.decay, st["S"], meta.seg_cu,
                           meta.seg_state, positions, self.H, self.D, self.P, act="silu", max_len=meta.seg_max_len)
         gate = proj[:, 2 * nq + nv:2 * nq + 2 * nv]
-        return F.linear(mx.head_norm_gate(o, self.norm_w, self.eps, gate, 1, "sigmoid", proj.dtype), self.o)
+        return project(mx.head_norm_gate(o, self.norm_w, self.eps, gate, 1, "sigmoid", proj.dtype), self.o)
 
 
 class _Rotary:
@@ -765,7 +766,7 @@ class RetentionMixer:
         o = mx.decay_scan(q, k, proj[:, 2 * nq:2 * nq + nv], self.decay, st["S"], meta.seg_cu, meta.seg_state, positions,
                           self.H, self.D, self.P, max_len=meta.seg_max_len)
         gate = proj[:, 2 * nq + nv:2 * nq + 2 * nv]
-        return F.linear(mx.head_norm_gate(o, None, self.eps, gate, self.H, "silu", proj.dtype), self.o)
+        return project(mx.head_norm_gate(o, None, self.eps, gate, self.H, "silu", proj.dtype), self.o)
 
 
 class ChunkAttentionMixer:
@@ -818,7 +819,7 @@ class ChunkAttentionMixer:
                              self.rot.mscale, norm_eps=self.eps, k_out=rows, slots=meta.slots, v=kraw)
         o = mx.window_attend(q, rows, meta.seg_cu, positions, meta.seg_bt, self.chunk or (1 << 30), self.scale,
                              meta.seg_max_len, self.H, self.G, self.D, self.P, chunked=bool(self.chunk))
-        return F.linear(o, self.o)
+        return project(o, self.o)
 
 
 class ParallelMixer:
@@ -909,7 +910,7 @@ class SigmoidAttentionMixer:
                              meta.slots, rows)
         o = mx.window_attend(q, rows, meta.seg_cu, positions, meta.seg_bt, self.window, self.scale, meta.seg_max_len,
                              self.H, self.G, self.D, self.P, head_bias=self.pb)
-        return F.linear(o, self.o)
+        return project(o, self.o)
 
 
 class MinGRUMixer:
@@ -942,7 +943,7 @@ class MinGRUMixer:
         R = self.R
         s = mx.mingru_scan(proj[:, :R], proj[:, R:2 * R], proj[:, 2 * R:3 * R], self.z_b, self.x_b, cache[1]["S"],
                            meta.seg_cu, meta.seg_state, positions, proj.dtype, max_len=meta.seg_max_len)
-        return F.linear(s, self.o)
+        return project(s, self.o)
 
 
 class WeightedParallelMixer(ParallelMixer):
@@ -1017,7 +1018,7 @@ class SinkWindowAttentionMixer:
                              v_mix=v_first, v_lam=self.lam)
         o = mx.window_attend(q, rows, meta.seg_cu, positions, meta.seg_bt, self.window, self.scale, meta.seg_max_len,
                              self.H, self.G, self.D, self.P, keep_first=self.keep)
-        return F.linear(o, self.o)
+        return project(o, self.o)
 
 
 class PlainLatentAttentionMixer:
@@ -1068,7 +1069,7 @@ class PlainLatentAttentionMixer:
         q_lat = self.uk(q.unflatten(1, (H, D)))                                                         # [T, H, R]
         o_lat = mx.latent_attend(q_lat, q_rot, rows, meta.seg_cu, positions, meta.seg_bt, self.window, self.scale,
                                  meta.seg_max_len)
-        return F.linear(self.uv(o_lat).view(T, H * self.P), self.o)
+        return project(self.uv(o_lat).view(T, H * self.P), self.o)
 
 
 class ConvAttentionMixer:
@@ -1147,7 +1148,7 @@ class ConvAttentionMixer:
         o = mx.window_attend(q, rows, meta.seg_cu, positions, meta.seg_bt, self.window, self.scale, meta.seg_max_len,
                              self.H, self.G, self.D, self.P, gate=proj[:, self.C:self.C + self.no], slopes=self.slopes,
                              sink=self.sink)
-        return F.linear(o, self.o)
+        return project(o, self.o)
 
 
 class _GroupedAttention:
@@ -1247,7 +1248,7 @@ class CappedAttentionMixer(_GroupedAttention):
         gate = proj[:, nq + nk + nv:nq + nk + nv + self.H]
         o = mx.window_attend(q, rows, meta.seg_cu, positions, meta.seg_bt, self.window, self.scale, meta.seg_max_len,
                              self.H, self.G, self.D, self.P, gate=gate, sink=self.sink, softcap=self.softcap)
-        return F.linear(o, self.o)
+        return project(o, self.o)
 
 
 MIXERS = {"mamba2": Mamba2Mixer, "latent_attention": LatentAttentionMixer, "channel_delta": ChannelDeltaMixer,

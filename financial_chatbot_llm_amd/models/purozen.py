@@ -28,9 +28,9 @@ from __future__ import annotations
 from typing import Dict
 
 import torch
-import torch.nn.functional as F
 
 from ..ops import mixers as mx
+from ..ops.gemm import project
 from .common import AttentionMetadata, HybridCache
 from .configs import ModelConfig
 from .layered import Layer, LayeredDecoder
@@ -149,7 +149,7 @@ class PurozenModel(LayeredDecoder):
         v_first = None
         for i, l in enumerate(self.layers):
             m = l.mixer
-            proj = F.linear(h, l.w_in)                                      # mixer rows | gate rows
+            proj = project(h, l.w_in)                                      # mixer rows | gate rows
             gate = proj[:, m.in_rows:m.in_rows + W]
             mults = (1.0, 1.0)
             if m.kind == "parallel":
@@ -167,7 +167,7 @@ class PurozenModel(LayeredDecoder):
             h = mx.residual_norm(x, l.norm2 if l.ff is not None else nxt, eps, a=y, b=y2, mult=mults[0], mult_b=mults[1],
                                  gate=gate, gate_bias=l.rg_b[1], out_dtype=dt)
             if l.ff is not None:
-                proj = F.linear(h, l.w_ff)                                  # up rows | gate rows
+                proj = project(h, l.w_ff)                                  # up rows | gate rows
                 y = l.ff.forward(h, proj)
                 h = mx.residual_norm(x, nxt, eps, a=y, gate=proj[:, l.ff.in_rows:l.ff.in_rows + W], gate_bias=l.rg_b[2],
                                      out_dtype=dt)

@@ -23,9 +23,9 @@ from __future__ import annotations
 from typing import Dict
 
 import torch
-import torch.nn.functional as F
 
 from ..ops import mixers as mx
+from ..ops.gemm import project
 from .common import AttentionMetadata, HybridCache
 from .configs import ModelConfig
 from .layered import Layer, LayeredDecoder
@@ -129,13 +129,13 @@ class SigudraModel(LayeredDecoder):
             x = mx.embed_f32(ids, self.embed)
         h = x if dt == torch.float32 else x.to(dt)
         for i, l in enumerate(self.layers):
-            m = l.mixer.forward(F.linear(h, l.w_in), positions, meta, kv.layers[i])
+            m = l.mixer.forward(project(h, l.w_in), positions, meta, kv.layers[i])
             if isinstance(m, tuple):          # two mixers side by side: half the sum of their RMS norms
                 h = mx.post_norm_add(x, m[0], l.norm1, eps, dt, b=m[1], wa=l.mixer.out_w[0], wb=l.mixer.out_w[1])
             else:
                 h = mx.post_norm_add(x, m, l.norm1, eps, dt)
             if l.ff is not None:
-                f = l.ff.forward(h, F.linear(h, l.w_ff) if l.w_ff is not None else None, x32=x)
+                f = l.ff.forward(h, project(h, l.w_ff) if l.w_ff is not None else None, x32=x)
                 h = mx.post_norm_add(x, f, l.norm2, eps, dt)
             if self.capture is not None:
                 self.capture.append(x.clone())

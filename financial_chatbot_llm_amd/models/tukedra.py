@@ -31,6 +31,7 @@ import torch
 import torch.nn.functional as F
 
 from ..ops import mixers as mx
+from ..ops.gemm import project
 from .common import AttentionMetadata, HybridCache
 from .configs import ModelConfig
 from .layered import Layer, LayeredDecoder
@@ -139,7 +140,7 @@ class TukedraModel(LayeredDecoder):
 
     def logits(self, h: torch.Tensor) -> torch.Tensor:
         # scale and cap in f32: the head product is rounded once, not again after the tanh
-        return mx.logit_cap(F.linear(h, self.head).float(), self.logit_scale, self.logit_softcap)
+        return mx.logit_cap(project(h, self.head).float(), self.logit_scale, self.logit_softcap)
 
     # -- forward -----------------------------------------------------------------------------------
     def forward(self, ids: torch.Tensor, positions: torch.Tensor, meta: AttentionMetadata, kv: HybridCache) -> torch.Tensor:
@@ -155,7 +156,7 @@ class TukedraModel(LayeredDecoder):
             done = l.hc[1]
             if l.ff is not None:
                 h = mx.hyper_mix(x, y, done[2], done[1], l.hc[2][0], l.norm2, eps, dt)
-                y = l.ff.forward(h, F.linear(h, l.w_ff) if l.w_ff is not None else None)
+                y = l.ff.forward(h, project(h, l.w_ff) if l.w_ff is not None else None)
                 done = l.hc[2]
             nxt = self.layers[i + 1] if i + 1 < n else None
             # the write-back of this layer's last sublayer, fused with the read and norm of what comes next

@@ -1,0 +1,44 @@
+"""Projections of a decode step's few rows (``ops.gemm.project``) against float64: one launch and slices of K, part-filled last
+tiles, edges of the row tiles, strided rows, and the calls that keep the library's product."""
+import pytest
+import torch
+
+from financial_chatbot_llm_amd.ops import gemm as G
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M", [1, 2, 15, 16, 17, 33, 63, 64, 65, 96, 97])
+@pytest.mark.parametrize("N_,K", [(512, 64), (528, 128), (2048, 2048), (4096, 2048), (7216, 448), (2064, 3072), (10256, 192),
+                                  (10240, 128), (1024, 4096), (2048, 4160), (500, 128), (512, 96)])
+def test_against_float64(M, N_, K):
+    g = torch.Generator().manual_seed(M + N_ + K)
+    w = (torch.randn((N_, K), generator=g) * K ** -0.5).to(torch.bfloat16).cuda()
+    rows = torch.randn((M, K + 24), generator=g).to(torch.bfloat16).cuda()
+    for off in (0, 16, 3):                                   # 3: rows off the kernel's 16 bytes
+        x = rows[:, off:off + K]
+        y = G.project(x, w)
+        want = x.double() @ w.double().t()
+        assert y.is_contiguous() and y.shape == (M, N_) and y.dtype == torch.bfloat16
+        # one rounding of the result to eight significant bits; K f32 products of values of order K^-0.5
+        assert ((y.double() - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -18 * K ** 0.5).all()
+
+
+def test_rule():
+    assert G.rows_config(64, 2048, 4096) == (2, 4) and G.rows_config(64, 4096, 2048) == (2, 2) and G.rows_config(1, 7216, 2048) == (2, 1)
+    assert G.rows_config(96, 12864, 2048) == (4, 1)
+    for M, N_, K in ((97, 2048, 4096), (65, 2048, 2048), (1, 500, 128), (1, 504, 128), (1, 512, 96)):
+        assert G.rows_config(M, N_, K) is None
+
+
+def test_other_calls_keep_the_library():
+    w = torch.randn((512, 128), device="cuda")
+    x = torch.randn((3, 128), device="cuda")
+    assert torch.equal(G.project(x, w), torch.nn.functional.linear(x, w))
+    wb, xb = w.bfloat16(), x.bfloat16()
+    assert G.project(xb[None], wb).shape == (1, 3, 512) and G.project(xb[0], wb).shape == (512,)
+    assert G.project(xb, wb.clone().requires_grad_()).requires_grad
+    with pytest.raises(RuntimeError):
+        G.project(xb, w)
+    with pytest.raises(RuntimeError):
+        G.project(xb[:, :64], wb)
