@@ -37,7 +37,7 @@ def _dual_stream(device) -> "torch.cuda.Stream":
     if key not in _DUAL_STREAMS:
         _DUAL_STREAMS[key] = torch.cuda.Stream(device=device)
     return _DUAL_STREAMS[key]
-from ..ops.gemm import (interleave16, linear, linear_tiled, prefill_qkv_rope, qkv_rope_fused, tile_weight,
+from ..ops.gemm import (few_ok, few_rows, interleave16, linear, linear_tiled, prefill_qkv_rope, qkv_rope_fused, tile_weight,
                         tiled_only, uses_tiled_weight)
 from ..parallel.layers import shard_cols, shard_rows, shard_sections, vocab_range
 from .common import AttentionMetadata, KVCache, random_tensor
@@ -252,6 +252,14 @@ class DecoderModel:
             # pass (no all-reduce in between), unlike the row-parallel O / down projections
             qkv = linear(h, self.w[p + "qkv"], wt=self.wt.get(p + "qkv"), slabs=True)
             q = ops.rope_kv_write(qkv, positions, self.cos_sin, meta.slots, kc, vc, self.hq, self.hkv, self.D)
+        attn = self.attend(q, meta, kc, vc, scale, qpre)
+        out = linear(attn.view(T, self.hq * self.D), self.w[p + "o"], wt=self.wt.get(p + "o"),
+                     slabs=self.tp_size == 1, fuse_residual=fuse_residual)
+        return comm.tp_all_reduce(out) if self.tp_size > 1 and reduce else out
+
+    def attend(self, q: torch.Tensor, meta: AttentionMetadata, kc: torch.Tensor, vc: torch.Tensor, scale: float,
+               qpre: bool = False) -> torch.Tensor:
+        """The step's attention over the paged cache: prefill rows first, then one row per decoding sequence."""
         attn = torch.empty_like(q)
         tp = meta.num_prefill_tokens
         side = None
@@ -278,9 +286,26 @@ class DecoderModel:
         elif meta.num_decode > 0:
             ops.decode(q[tp:], meta.ctx_lens_d, meta.block_tables_d, kc, vc, scale,
                        workspace=meta.decode_ws, out=attn[tp:])
-        out = linear(attn.view(T, self.hq * self.D), self.w[p + "o"], wt=self.wt.get(p + "o"),
-                     slabs=self.tp_size == 1, fuse_residual=fuse_residual)
-        return comm.tp_all_reduce(out) if self.tp_size > 1 and reduce else out
+        return attn
+
+    def takes_few(self, T: int) -> bool:
+        """Does a step of ``T`` rows take :meth:`forward_few`?  The layers' projections are alike: the first one's decide."""
+        return T <= 4 and self.tp_size == 1 and type(self).mlp is DecoderModel.mlp and all(
+            few_ok(T, self.wt.get("layers.0." + n), norm) for n, norm in (("qkv", True), ("o", False), ("gate_up", True), ("down", False)))
+
+    def forward_few(self, ids: torch.Tensor, positions: torch.Tensor, meta: AttentionMetadata, kv: KVCache) -> torch.Tensor:
+        """One to four rows: each projection takes its norm, its SiLU or its residual add into its own launch."""
+        eps, x = self.cfg.norm_eps, self.embed(ids)
+        for i in range(self.cfg.num_layers):
+            p = f"layers.{i}."
+            kc, vc = kv.k(i), kv.v(i)
+            qkv = few_rows(x, self.wt[p + "qkv"], "slab", self.w[p + "in_norm"], eps)
+            q = ops.rope_kv_write(qkv, positions, self.cos_sin, meta.slots, kc, vc, self.hq, self.hkv, self.D)
+            attn = self.attend(q, meta, kc, vc, self.scale)
+            few_rows(attn.view(-1, self.hq * self.D), self.wt[p + "o"], "add", residual=x)
+            a = few_rows(x, self.wt[p + "gate_up"], "silu", self.w[p + "post_norm"], eps)
+            few_rows(a, self.wt[p + "down"], "add", residual=x)
+        return ops.rms_norm(x, self.w["final_norm"], eps)
 
     def uses_sp(self, T: int) -> bool:
         return (self.sequence_parallel and self.tp_size > 1 and T >= self.sp_min_tokens
@@ -462,6 +487,8 @@ class DecoderModel:
     def forward(self, ids: torch.Tensor, positions: torch.Tensor, meta: AttentionMetadata, kv: KVCache) -> torch.Tensor:
         if self.uses_sp(ids.shape[0]):
             return self.forward_sp(ids, positions, meta, kv)
+        if self.takes_few(ids.shape[0]):
+            return self.forward_few(ids, positions, meta, kv)
         c = self.cfg
         x = self.embed(ids)
         residual = x

@@ -290,6 +290,39 @@ def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return F.linear(x, w)
 
 
+FEW_FORMS = {"slab": 0, "add": 1, "silu": 2}
+
+
+def few_ok(M: int, wt: Optional[torch.Tensor], norm: bool) -> bool:
+    """Can ``few_rows`` run ``M`` rows through this ``tile_weight`` copy (``norm``: with an RMS norm in front)?
+
+    Up to four rows, measured with the launches it replaces (us, weights beyond the caches, 1 and 4 rows): Llama-3-8B's norm +
+    QKV 14.0 / 10.4 and 14.4 / 12.5, O + norm 11.8 / 7.7 and 11.6 / 8.4, norm + gate|up + SiLU 48.2 / 39.6 and 52.1 / 40.3, down + norm
+    27.1 / 20.4 and 27.1 / 20.9.  ``PENNY_SPLITK=0`` or ``PENNY_GATEUP=0`` turn it off with the other streaming kernels."""
+    if wt is None or wt.dtype != torch.bfloat16 or not N.use_native(wt) or "0" in (os.environ.get("PENNY_SPLITK", "1"), os.environ.get("PENNY_GATEUP", "1")):
+        return False
+    K = wt.shape[1] * 32
+    return 1 <= M <= 4 and wt.shape[0] % 2 == 0 and K % 512 == 0 and M * (2 * K + 64) <= 116 * 1024 and (not norm or K <= 4096)
+
+
+def few_rows(x: torch.Tensor, wt: torch.Tensor, form: str, norm: Optional[torch.Tensor] = None, eps: float = 0.0,
+             residual: Optional[torch.Tensor] = None) -> Union[torch.Tensor, "Slabs"]:
+    """One to four rows through a ``tile_weight`` copy in one launch (``penny_few_rows``), RMS-normed with ``norm`` first where it is
+    given.  "slab": f32 sums as one slab; "add": added to ``residual`` in place; "silu": ``wt`` is the interleave16 gate|up weight and the
+    result SiLU(gate) * up."""
+    M, K = x.shape
+    N_ = wt.shape[0] * 16
+    if form == "slab":
+        y = torch.empty((1, M, N_), dtype=torch.float32, device=x.device)
+    elif form == "silu":
+        y = torch.empty((M, N_ // 2), dtype=x.dtype, device=x.device)
+    else:
+        y = residual
+    N.call("penny_few_rows", N.ptr(x), x.stride(0), N.ptr(norm), float(eps), N.ptr(wt), K, N_, N.ptr(y), y.stride(-2), M, FEW_FORMS[form],
+           N.stream())
+    return Slabs(y) if form == "slab" else y
+
+
 # "tiled": the decode kernels stream a fragment-tiled copy of each measured projection (made once
 # at load, ``tile_weight``; 3-10 % faster for gate|up); "rowmajor": they always stream the
 # row-major weights directly (no extra HBM).  Shapes without a tiled copy use row-major anyway.

@@ -1,0 +1,80 @@
+"""Projections of one to four rows with their norm, SiLU or residual add (``ops.gemm.few_rows``) against float64 of the same
+roundings, at both LDS sizes and part-filled threads, and the decoder's step of few rows against the general one."""
+import pytest
+import torch
+
+from financial_chatbot_llm_amd.ops import gemm as G
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("form,N_,K,norm", [("slab", 48, 512, True), ("slab", 96, 4096, True), ("slab", 32, 1536, False), ("add", 16, 512, False),
+                                            ("add", 80, 4096, False), ("add", 48, 14336, False), ("silu", 32, 512, True),
+                                            ("silu", 96, 2560, True), ("silu", 64, 4096, True), ("silu", 64, 6144, False)])
+def test_against_float64(M, form, N_, K, norm):
+    gen = torch.Generator().manual_seed(M + N_ + K)
+    rnd = lambda *s: torch.randn(s, generator=gen).to(torch.bfloat16).cuda()          # noqa: E731
+    x, w, res = rnd(M, K + 8)[:, :K], rnd(N_, K) * K ** -0.5, rnd(M, N_)
+    nw = 1 + 0.1 * rnd(K) if norm else None
+    h = x.double()
+    if norm:
+        h = (x.float() * torch.rsqrt(x.float().pow(2).mean(-1, keepdim=True) + 1e-5)).bfloat16()
+        h = (h.float() * nw.float()).bfloat16().double()
+    want = h @ w.double().t()
+    # a half unit of a norm that falls the other way moves a value of h by 2^-8 of it: a sum of K of them, few of which do
+    tol = 2.0 ** -18 * K ** 0.5 + (2.0 ** -8 * 4 * K ** -0.5 * h.abs().max() if norm else 0.0)
+    ulp = lambda t: t.abs() * 2.0 ** -8                                                # noqa: E731
+    before = res.clone()
+    y = G.few_rows(x, G.tile_weight(w), form, nw, 1e-5, residual=res)
+    if form == "slab":
+        assert y.P.shape == (1, M, N_) and ((y.P[0].double() - want).abs() <= tol + want.abs() * 2.0 ** -20).all()
+    elif form == "add":
+        assert y is res and ((y.double() - (before.double() + want)).abs() <= tol + ulp(want) + ulp(before.double() + want)).all()
+    else:
+        gate, up = (want.view(M, -1, 2, 16)[:, :, i].reshape(M, -1) for i in (0, 1))
+        ref = gate * torch.sigmoid(gate) * up
+        # gate, up, their unit and the product are each rounded once; the unit's slope is 1.1 at most
+        bound = ulp(ref) * 2 + (ulp(gate) + tol) * 1.1 * up.abs() + (ulp(up) + tol) * gate.abs() + tol
+        assert y.shape == (M, N_ // 2) and ((y.double() - ref).abs() <= bound).all()
+
+
+def test_refused():
+    x, wt = torch.zeros((2, 4096), device="cuda", dtype=torch.bfloat16), G.tile_weight(torch.zeros((64, 4096), device="cuda", dtype=torch.bfloat16))
+    assert G.few_ok(4, wt, True) and not G.few_ok(5, wt, True) and not G.few_ok(1, None, False)
+    assert not G.few_ok(1, torch.empty((4, 256, 64, 8), device="cuda", dtype=torch.bfloat16), True)       # a norm over 8192 columns
+    with pytest.raises(RuntimeError):
+        G.few_rows(torch.zeros((5, 4096), device="cuda", dtype=torch.bfloat16), wt, "slab")
+    with pytest.raises(RuntimeError):
+        G.few_rows(x, wt, "add", norm=x[0], residual=torch.zeros((2, 64), device="cuda", dtype=torch.bfloat16))
+
+
+@pytest.mark.parametrize("T", [1, 3, 4])
+def test_decoder_step(T, monkeypatch):
+    """The same step through :meth:`forward_few` and through the general layers, from the same cache."""
+    from financial_chatbot_llm_amd.models.common import AttentionMetadata, KVCache
+    from financial_chatbot_llm_amd.models.configs import ModelConfig
+    from financial_chatbot_llm_amd.models.llama import LlamaModel
+    from financial_chatbot_llm_amd.ops.attention import DecodeWorkspace
+    cfg = ModelConfig(name="few", arch="llama", vocab_size=512, hidden_size=1024, intermediate_size=2048, num_layers=2, num_heads=8,
+                      num_kv_heads=2, head_dim=128, max_position=512)
+    model = LlamaModel(cfg, device="cuda").init_random(3)
+    assert not model.takes_few(T)                            # no streamed copies of these sizes
+    model.wt = {n: G.tile_weight(w) for n, w in model.w.items() if n.endswith((".qkv", ".o", ".down", ".gate_up"))}
+    assert model.takes_few(T) and not model.takes_few(5)
+    pos = torch.full((T,), 70, dtype=torch.int32, device="cuda")
+    ids = torch.arange(T, dtype=torch.int32, device="cuda") * 7
+    bt = torch.arange(2 * T, dtype=torch.int32, device="cuda").view(T, 2)
+    outs = []
+    for few in (True, False):
+        kv = KVCache(cfg.num_layers, 2 * T, 2, 128, device="cuda")
+        for i in range(cfg.num_layers):
+            for c in (kv.k(i), kv.v(i)):
+                c.copy_(torch.randn(c.shape, generator=torch.Generator().manual_seed(i)).to(c.dtype))
+        meta = AttentionMetadata(num_prefill_tokens=0, num_decode=T, slots=(bt[:, 1].long() * 64 + 6).to(torch.int32),
+                                 ctx_lens_d=pos + 1, block_tables_d=bt, decode_ws=DecodeWorkspace.create(T, 8, 128, 512, "cuda"))
+        monkeypatch.setattr(LlamaModel, "takes_few", lambda self, t, few=few: few)
+        outs.append((model.forward(ids, pos, meta, kv).float(), kv.k(1).float(), kv.v(1).float()))
+    for a, b in zip(*outs):
+        # both round the same values to eight bits in a different order of f32 sums: at most a unit per layer of the largest
+        assert (a - b).abs().max() <= 4 * 2.0 ** -8 * b.abs().max()
