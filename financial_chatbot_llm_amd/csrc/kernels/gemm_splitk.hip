@@ -592,29 +592,78 @@ PENNY_API int penny_splitk_gemm_bf16(const void* X, int ldx, const void* Wt, int
   return (int)hipErrorInvalidValue;
 }
 
-// Y [M, N] = X [M, K] x W [N, K]^T in bf16 for the few rows of a decode step, W row-major: slabs == null streams W once
-// (S = 1), else S slices of K leave f32 slabs [S, M, N] that a second launch adds.  One entry for both, so that a step that
-// the host bounds pays for one call.  Contract (checked): 1 <= M <= 96, N % 16 == 0 (the last tile of 16 * nf columns may be
-// part-filled), nf in {2, 4}, K % (64 * S) == 0, ldx % 8 == 0, ldy % 8 == 0.
+namespace {
+
+// What a block of penny_linear_rows takes for 2048 of K beyond its fixed 2.8 us, by its 16 nf columns and 16 mt rows
+struct RowsTile {
+  int nf, mt;
+  float us;
+};
+constexpr RowsTile kRowsTiles[] = {{2, 2, 4.6f}, {2, 4, 6.5f}, {4, 2, 6.7f},  {2, 6, 8.2f},  {4, 4, 9.8f},   {2, 8, 9.9f},  {4, 6, 11.7f},
+                                   {8, 2, 12.3f}, {4, 8, 15.f}, {8, 4, 15.3f}, {8, 6, 21.f}, {4, 12, 19.2f}, {8, 8, 24.f}};
+
+}  // namespace
+
+// The tile and split of penny_linear_rows for M rows: nf | mt << 8 | S << 16, or 0 where the library's product is to be taken.
+//
+// A block's ring takes a CU's LDS, so the blocks run in rounds of 256, each round for as long as its tile's K: a product is the
+// faster the smaller the tile, as long as one round holds all blocks; with few blocks K is cut in 2 or 4 (a second launch and
+// a pass over the slabs: 2 us and 1 us per MB).  Against the library, weights beyond the caches, us library / here: 2048 x 4096
+// 1 row 14.8 / 8.4, 64 13.9 / 10.1; 4096 x 2048 64 12.2 / 8.7, 256 13.7 / 13.7; 7232 x 2048 64 12.9 / 11.4, 256 24.2 / 19.9; 12864 x 2048 64 16.1 /
+// 15.4, 160 24.6 / 23.6; 2048 x 2048 64 8.9 / 7.2, 256 9.9 / 9.8, 512 12.0 / 13.0; 6464 x 1024 64 11.7 / 7.3, 256 15.1 / 12.0; 2048 x 1024 256 8.7 / 6.4, 768
+// 10.1 / 9.4; 1024 x 3072 64 10.0 / 7.0, 256 9.1 / 10.3; 1024 x 1024 64 8.6 / 5.1, 512 8.6 / 6.4.  A library call costs the host 20 - 24 us as well,
+// this one 8: a step of many small launches is bounded by that.  So products of up to 20 us are taken up to 512 rows, where some
+// are up to a tenth slower than the library's, and from there, as the device becomes the bound, ever shorter ones, to 16 us at 1024
+// rows and 8 at 2048.  Whole passes of 400, 600 and 1000 tokens, three hybrid decoders of width 1024, us: 1538 -> 1086, 1739 -> 1347, 1399 ->
+// 935; 1540 -> 1160, 1730 -> 1378, 1440 -> 976; 1570 -> 1399, 1790 -> 1526, 1505 -> 1125; width 2048 at 400: 1811 -> 1789, 1789 -> 1769, 1657
+// -> 1650.  Up to 96 rows, the steps of captured decodes, all but the longest are taken (14912 x 2048, 96 rows: 18.7 / 18.3).
+PENNY_API int penny_linear_rows_plan(int M, int N, int K) {
+  if (M <= 0 || M > 2048 || N < 512 || N % 16 || K <= 0 || K % 64) return 0;
+  int plan = 0;
+  float best = M <= 96 ? 60.f : M <= 512 ? 20.f : 20.f - (M - 512) / 128.f;
+  for (int S = 1; S <= 4; S *= 2) {
+    if (S > 1 && (K % (64 * S) || K / S < 256)) break;
+    for (const RowsTile& t : kRowsTiles) {
+      const long blocks = (long)((N + 16 * t.nf - 1) / (16 * t.nf)) * ((M + 16 * t.mt - 1) / (16 * t.mt)) * S;
+      if (S > 1 && blocks > 256) continue;
+      const float us = (blocks + 255) / 256 * (2.8f + t.us * (K / S) / 2048.f) + (S > 1 ? 2.f + 4e-6f * S * M * N : 0.f);
+      if (us < best) best = us, plan = t.nf | t.mt << 8 | S << 16;
+    }
+  }
+  return plan;
+}
+
+// Y [M, N] = X [M, K] x W [N, K]^T in bf16 for up to about two thousand rows, W row-major: slabs == null streams W once (S = 1), else
+// S slices of K leave f32 slabs [S, M, N] that a second launch adds.  One entry for both, so that a step that the host bounds
+// pays for one call.  nf, mt: a block's columns and rows in units of 16, one of kRowsTiles.  Contract (checked): N % 16 == 0 (the last
+// tile may be part-filled), K % (64 * S) == 0, ldx % 8 == 0, ldy % 8 == 0.
 PENNY_API int penny_linear_rows(const void* X, int ldx, const void* W, int K, void* Y, int ldy, int M, int N, void* slabs,
-                                int S, int nf, int paired, hipStream_t st) {
+                                int S, int nf, int mt, int paired, hipStream_t st) {
   if (M <= 0) return 0;
-  if (M > 96 || N <= 0 || N % 16 || (nf != 2 && nf != 4) || S < 1 || (S > 1) != (slabs != nullptr) || K <= 0 ||
+  if (M > (1 << 20) || N <= 0 || N % 16 || (nf != 2 && nf != 4 && nf != 8) || S < 1 || (S > 1) != (slabs != nullptr) || K <= 0 ||
       K % (64 * S) || ldx % 8 || ldy % 8)
     return (int)hipErrorInvalidValue;
-  const int wrow = paired ? 3 : 1, mt = (M + 15) / 16;
+  const int wrow = paired ? 3 : 1;
   float* p = static_cast<float*>(slabs);
   int rc;
-#define LR_CASE(MT_, WA_)                                                                                    \
-  if (mt <= MT_) {                                                                                           \
-    if (S > 1) rc = nf == 2 ? launch<2, MT_, WA_>(X, ldx, W, K, p, M, N, S, wrow, st)                        \
-                            : launch<4, MT_, WA_>(X, ldx, W, K, p, M, N, S, wrow, st);                       \
-    else rc = nf == 2 ? launch_bf16<2, MT_, WA_>(X, ldx, W, K, Y, ldy, M, N, wrow, st)                       \
-                      : launch_bf16<4, MT_, WA_>(X, ldx, W, K, Y, ldy, M, N, wrow, st);                      \
+#define LR_CASE(NF_, MT_, WA_)                                                       \
+  if (nf == NF_ && mt == MT_) {                                                      \
+    if (S > 1) rc = launch<NF_, MT_, WA_>(X, ldx, W, K, p, M, N, S, wrow, st);       \
+    else rc = launch_bf16<NF_, MT_, WA_>(X, ldx, W, K, Y, ldy, M, N, wrow, st);      \
   } else
-  LR_CASE(2, 2)
-  LR_CASE(4, 1)
-  LR_CASE(6, 2)
+  LR_CASE(2, 2, 2)
+  LR_CASE(2, 4, 1)
+  LR_CASE(4, 2, 2)
+  LR_CASE(2, 6, 2)
+  LR_CASE(4, 4, 1)
+  LR_CASE(2, 8, 1)
+  LR_CASE(4, 6, 2)
+  LR_CASE(8, 2, 2)
+  LR_CASE(4, 8, 1)
+  LR_CASE(8, 4, 2)
+  LR_CASE(8, 6, 2)
+  LR_CASE(4, 12, 1)
+  LR_CASE(8, 8, 2)
   return (int)hipErrorInvalidValue;
 #undef LR_CASE
   if (rc || S == 1) return rc;

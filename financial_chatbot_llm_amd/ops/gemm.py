@@ -19,7 +19,6 @@ with ``bench/kernels.py`` (profiles named next to each table).
 """
 from __future__ import annotations
 
-import functools
 import os
 from typing import Dict, List, Optional, Tuple, Union
 
@@ -252,41 +251,28 @@ def splitk_bf16(x: torch.Tensor, w: torch.Tensor, N_: int, nf: int, rowmajor: bo
     return y
 
 
-@functools.lru_cache(maxsize=1024)
-def rows_config(M: int, N_: int, K: int) -> Optional[Tuple[int, int]]:
-    """(nf, S) of ``penny_linear_rows`` for a few rows on a row-major weight, or None: the library's product.
-
-    32 columns per block (nf 2) up to 320 blocks, then 64; K in slices while the blocks then fit the 256 CUs and a slice keeps 512.
-    Measured on weights beyond the caches (us, library / here, 1 and 64 rows): 2048 x 4096 14.8 / 8.4 and 14.2 / 10.3, 4096 x 2048
-    12.1 / 9.2 and 12.6 / 9.7, 7232 x 2048 12.8 / 9.2 and 13.1 / 11.5, 12288 x 2048 16.0 / 12.4 and 16.5 / 15.2, 32768 x 2048 34.0 / 27.8
-    and 34.7 / 32.8, 2048 x 768 7.1 / 5.4 and 7.8 / 5.5; a call costs the host 7 - 9 us less as well.  At 96 rows 7232 x 2048 takes 14.0 / 12.9,
-    2048 x 6144 17.6 / 14.6, but sliced short products lose (2048 x 2048 8.5 / 9.3), and from 128 rows most do."""
-    if N_ < 512 or N_ % 16 or K % 64 or not 1 <= M <= 96:
-        return None
-    nf = 2 if N_ <= 320 * 32 else 4
-    S = 1
-    while S < 4 and -(-N_ // (16 * nf)) * 2 * S <= 256 and K // (2 * S) >= 512 and K % (128 * S) == 0:
-        S *= 2
-    if M > 64 and S > 1 and K <= 2048:
-        return None
-    return nf, S
+def rows_config(M: int, N_: int, K: int) -> Optional[Tuple[int, int, int]]:
+    """(nf, mt, S) of ``penny_linear_rows`` for M rows on a row-major weight, or None: the library's product (the rule and its
+    measurements stand at ``penny_linear_rows_plan``)."""
+    plan = N.load().penny_linear_rows_plan(M, N_, K)
+    return (plan & 255, plan >> 8 & 255, plan >> 16) if plan else None
 
 
 def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """y = x @ w.T: the streaming kernels for the rows of a decode step (``rows_config``), the library's product for the rest."""
-    if w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and N.use_native(x):
-        M, K = x.shape
-        cfg = rows_config(M, w.shape[0], K)
-        ldx = x.stride(0)
-        if cfg is not None and x.stride(1) == 1 and ldx % 8 == 0 and ldx >= K and w.is_contiguous() and x.data_ptr() % 16 == 0 and \
-                w.data_ptr() % 16 == 0 and w.device == x.device and not (w.requires_grad or x.requires_grad):
-            nf, S = cfg
-            N_ = w.shape[0]
-            y = torch.empty((M, N_), dtype=x.dtype, device=x.device)
-            slabs = torch.empty((S, M, N_), dtype=torch.float32, device=x.device) if S > 1 else None
-            N.call("penny_linear_rows", N.ptr(x), ldx, N.ptr(w), K, N.ptr(y), N_, M, N_, N.ptr(slabs) if S > 1 else None, S, nf,
-                   PAIR_MODE != "0", N.stream())
-            return y
+    """y = x @ w.T: the streaming kernels for up to about two thousand rows (``rows_config``), the library's product for the rest."""
+    if w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 2 and N.use_native(x):
+        (M, K), N_ = x.shape, w.shape[0]
+        ldx, xp, wp = x.stride(0), x.data_ptr(), w.data_ptr()
+        if M <= 2048 and K == w.shape[1] and (xp | wp) % 16 == 0 and ldx % 8 == 0 and ldx >= K and x.stride(1) == 1 and \
+                w.is_contiguous() and w.device == x.device and not (w.requires_grad or x.requires_grad):
+            plan = N.load().penny_linear_rows_plan(M, N_, K)
+            if plan:
+                S = plan >> 16
+                y = torch.empty((M, N_), dtype=x.dtype, device=x.device)
+                slabs = torch.empty((S, M, N_), dtype=torch.float32, device=x.device) if S > 1 else None
+                N.call("penny_linear_rows", xp, ldx, wp, K, y.data_ptr(), N_, M, N_, N.ptr(slabs), S, plan & 255, plan >> 8 & 255,
+                       PAIR_MODE != "0", N.stream())
+                return y
     return F.linear(x, w)
 
 

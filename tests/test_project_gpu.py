@@ -1,5 +1,5 @@
-"""Projections of a decode step's few rows (``ops.gemm.project``) against float64: one launch and slices of K, part-filled last
-tiles, edges of the row tiles, strided rows, and the calls that keep the library's product."""
+"""Projections of a decode step's few rows (``ops.gemm.project``) against float64: one launch and slices of K, all tiles,
+part-filled ones, edges of the rule, strided rows, and the calls that keep the library's product."""
 import pytest
 import torch
 
@@ -8,9 +8,9 @@ from financial_chatbot_llm_amd.ops import gemm as G
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("M", [1, 2, 15, 16, 17, 33, 63, 64, 65, 96, 97])
+@pytest.mark.parametrize("M", [1, 2, 15, 16, 17, 33, 63, 64, 65, 96, 97, 160, 256, 400, 1000, 1024, 1500, 2048, 2049])
 @pytest.mark.parametrize("N_,K", [(512, 64), (528, 128), (2048, 2048), (4096, 2048), (7216, 448), (2064, 3072), (10256, 192),
-                                  (10240, 128), (1024, 4096), (2048, 4160), (500, 128), (512, 96)])
+                                  (10240, 128), (1024, 4096), (1024, 1024), (5168, 1024), (2048, 4160), (500, 128), (512, 96)])
 def test_against_float64(M, N_, K):
     g = torch.Generator().manual_seed(M + N_ + K)
     w = (torch.randn((N_, K), generator=g) * K ** -0.5).to(torch.bfloat16).cuda()
@@ -24,10 +24,29 @@ def test_against_float64(M, N_, K):
         assert ((y.double() - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -18 * K ** 0.5).all()
 
 
+def test_every_tile():
+    """Each tile and split that the launcher knows, with part-filled tiles on both sides."""
+    from financial_chatbot_llm_amd.ops import _native as N
+    g = torch.Generator().manual_seed(1)
+    w = (torch.randn((528, 512), generator=g) * 512 ** -0.5).to(torch.bfloat16).cuda()
+    x = torch.randn((150, 512), generator=g).to(torch.bfloat16).cuda()
+    want = x.double() @ w.double().t()
+    for nf, mt in ((2, 2), (2, 4), (4, 2), (2, 6), (4, 4), (2, 8), (4, 6), (8, 2), (4, 8), (8, 4), (8, 6), (4, 12), (8, 8)):
+        for S in (1, 2, 4):
+            for paired in (0, 1):
+                y = torch.zeros((151, 528), dtype=torch.bfloat16, device="cuda")
+                slabs = torch.empty((S, 150, 528), device="cuda") if S > 1 else None
+                N.call("penny_linear_rows", N.ptr(x), 512, N.ptr(w), 512, N.ptr(y), 528, 150, 528, N.ptr(slabs), S, nf, mt, paired, N.stream())
+                assert ((y[:150].double() - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -18 * 512 ** 0.5).all(), (nf, mt, S, paired)
+                assert (y[150] == 0).all()
+    with pytest.raises(RuntimeError):
+        N.call("penny_linear_rows", N.ptr(x), 512, N.ptr(w), 512, N.ptr(y), 528, 150, 528, None, 1, 2, 16, 1, N.stream())
+
+
 def test_rule():
-    assert G.rows_config(64, 2048, 4096) == (2, 4) and G.rows_config(64, 4096, 2048) == (2, 2) and G.rows_config(1, 7216, 2048) == (2, 1)
-    assert G.rows_config(96, 12864, 2048) == (4, 1)
-    for M, N_, K in ((97, 2048, 4096), (65, 2048, 2048), (1, 500, 128), (1, 504, 128), (1, 512, 96)):
+    assert G.rows_config(64, 2048, 4096) == (2, 4, 4) and G.rows_config(64, 4096, 2048) == (2, 2, 1) and G.rows_config(1, 7216, 2048) == (2, 2, 1)
+    assert G.rows_config(256, 2048, 2048) == (2, 4, 1) and G.rows_config(512, 1024, 1024) == (2, 4, 1)
+    for M, N_, K in ((600, 4096, 2048), (700, 1024, 4096), (300, 12864, 2048), (2049, 512, 64), (1, 500, 128), (1, 504, 128), (1, 512, 96)):
         assert G.rows_config(M, N_, K) is None
 
 
