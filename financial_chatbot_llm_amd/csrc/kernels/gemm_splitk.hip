@@ -37,10 +37,11 @@ __device__ __forceinline__ void vmcnt_barrier() {
 union Frag {
   uint4 u;
   bf16x8 v;
+  f32x4 f;
 };
 
 // epilogues of splitk_gemm_kernel
-enum { SK_SLAB = 0, SK_SILU = 1, SK_BF16 = 2, SK_SAMPLE = 3 };
+enum { SK_SLAB = 0, SK_SILU = 1, SK_BF16 = 2, SK_SAMPLE = 3, SK_F32 = 4 };
 
 // SK_SAMPLE (the streaming LM head + K12 sampler): per-row temperature (<= 0: greedy) and seed;
 // pv / pi [M, pstride] partial (best score, token) per (row, workgroup tile, wave row).  Token
@@ -101,8 +102,10 @@ __device__ __forceinline__ void wait_stage(int younger) {
 // alias-scope metadata, which is what lets hipcc's waitcnt pass leave the younger stages' LDS-DMA
 // in flight -- without it the pass cannot tell them apart from this stage and drains vmcnt(0)
 // before the first ds_read of every stage (measured: the ring then degenerates to one stage).
-template <int FW, int TW, int WBYTES, bool WROW>
-__device__ __forceinline__ void stage_mma(const char* __restrict__ base, f32x4 (&acc)[FW][TW], int wa, int wb,
+// F32: the same 16 bytes are four f32 channels 4g .. 4g + 3; the j-th of each lane make one 16x16x4 product, added into a sum of its own
+// (chains a quarter as long: error of K = 1024 in one slice 5.8e-7 with one sum, 2.9e-7 with four, the library 2.9 - 5.8e-7)
+template <int FW, int TW, int WBYTES, bool WROW, bool F32 = false>
+__device__ __forceinline__ void stage_mma(const char* __restrict__ base, f32x4 (&acc)[F32 ? 4 : 1][FW][TW], int wa, int wb,
                                           int lane, int g, int col) {
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) {
@@ -125,11 +128,17 @@ __device__ __forceinline__ void stage_mma(const char* __restrict__ base, f32x4 (
     for (int f = 0; f < FW; ++f)
 #pragma unroll
       for (int t = 0; t < TW; ++t)
-        acc[f][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[f].v, xf[t].v, acc[f][t], 0, 0, 0);
+        if constexpr (F32) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[j][f][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[f].f[j], xf[t].f[j], acc[j][f][t], 0, 0, 0);
+        } else {
+          acc[0][f][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[f].v, xf[t].v, acc[0][f][t], 0, 0, 0);
+        }
   }
 }
 
 // Epilogues (EPI):
+//   SK_F32    SK_SLAB for f32 operands, which are addressed as twice as many 16-bit columns (K, ldx);
 //   SK_SLAB   f32 partial slabs P [S, M, N] (reduced by the consumer's row pass);
 //   SK_SILU   W is the 16-row-interleaved gate|up weight (ops/gemm.py interleave16) and S == 1: the
 //             epilogue writes Y[m, f] = silu(gate) * up as bf16 [M, N/2] (ldy) instead of f32 slabs --
@@ -179,7 +188,7 @@ __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restr
   X += (long)m0 * ldx;
   if constexpr (EPI == SK_SILU || EPI == SK_BF16) Y += (long)m0 * ldy;
   PENNY_DASSERT(M > 0 && (EPI != SK_SAMPLE || gridDim.y == 1));
-  PENNY_DASSERT((tile + 1) * 16 * NF <= N || (WROW && N % 16 == 0 && tile * 16 * NF < N && (EPI == SK_BF16 || EPI == SK_SLAB)));
+  PENNY_DASSERT((tile + 1) * 16 * NF <= N || (WROW && N % 16 == 0 && tile * 16 * NF < N && (EPI == SK_BF16 || EPI == SK_SLAB || EPI == SK_F32)));
   PENNY_DASSERT(K % (64 * BKM * S) == 0);
   const int n0 = tile * 16 * NF;
   const int kc = K / S, k0 = s * kc;
@@ -230,11 +239,14 @@ __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restr
                                          (lds_void_t*)(base + u * SBYTES + dst[i]), 16, 0, 0);
   };
 
-  f32x4 acc[FW][TW];
+  constexpr int SUMS = EPI == SK_F32 ? 4 : 1;
+  f32x4 sums[SUMS][FW][TW];
 #pragma unroll
-  for (int f = 0; f < FW; ++f)
+  for (int i = 0; i < SUMS; ++i)
 #pragma unroll
-    for (int t = 0; t < TW; ++t) acc[f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int f = 0; f < FW; ++f)
+#pragma unroll
+      for (int t = 0; t < TW; ++t) sums[i][f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
 #pragma unroll
   for (int j = 0; j < NBUF - 1; ++j)
@@ -246,7 +258,14 @@ __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restr
     if (j + NBUF - 1 < nst) stage(j + NBUF - 1);
 #pragma unroll
     for (int u = 0; u < BKM; ++u)
-      stage_mma<FW, TW, WBYTES, WROW>(smem + (j % NBUF) * SLOT + u * SBYTES, acc, wa, wb, lane, g, col);
+      stage_mma<FW, TW, WBYTES, WROW, EPI == SK_F32>(smem + (j % NBUF) * SLOT + u * SBYTES, sums, wa, wb, lane, g, col);
+  }
+  f32x4(&acc)[FW][TW] = sums[0];
+  if constexpr (EPI == SK_F32) {
+#pragma unroll
+    for (int f = 0; f < FW; ++f)
+#pragma unroll
+      for (int t = 0; t < TW; ++t) acc[f][t] = (acc[f][t] + sums[1][f][t]) + (sums[2][f][t] + sums[3][f][t]);
   }
 
   if constexpr (SILU) {
@@ -402,6 +421,30 @@ template <int NF, int MT, int WA>
 int launch(const void* X, int ldx, const void* Wt, int K, float* P, int M, int N, int S, int wrow, hipStream_t st) {
   return launch_any<NF, MT, WA, SK_SLAB, 8>(wrow, (K / S) % 128 == 0, dim3(((N + 16 * NF - 1) / (16 * NF)) * S, (M + 16 * MT - 1) / (16 * MT)), st, (const bf16*)X,
                                             ldx, (const bf16*)Wt, K, P, M, N, S, (bf16*)nullptr, 0, SkSample{});
+}
+
+template <int NF, int MT, int WA>
+int launch_f32(const void* X, int ldx, const void* W, int K, float* P, int M, int N, int S, int paired, hipStream_t st) {
+  const dim3 grid(((N + 16 * NF - 1) / (16 * NF)) * S, (M + 16 * MT - 1) / (16 * MT));
+  if constexpr (pair_fits<NF, MT, 150, 16>()) {
+    if (paired && (K / S) % 64 == 0) {
+      hipLaunchKernelGGL((splitk_gemm_kernel<NF, MT, WA, SK_F32, true, 150, 16, 2>), grid, dim3(256), 0, st, (const bf16*)X, 2 * ldx,
+                         (const bf16*)W, 2 * K, P, M, N, S, (bf16*)nullptr, 0, SkSample{});
+      return (int)hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((splitk_gemm_kernel<NF, MT, WA, SK_F32, true, 150, 16>), grid, dim3(256), 0, st, (const bf16*)X, 2 * ldx, (const bf16*)W,
+                     2 * K, P, M, N, S, (bf16*)nullptr, 0, SkSample{});
+  return (int)hipGetLastError();
+}
+
+// Y[m, n] = sum_s P[s, m, n], four outputs per thread
+__global__ void __launch_bounds__(256) splitk_reduce_f32_kernel(const f32x4* __restrict__ P, int S, long quads, f32x4* __restrict__ Y) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= quads) return;
+  f32x4 v = P[i];
+  for (int s = 1; s < S; ++s) v += P[s * quads + i];
+  Y[i] = v;
 }
 
 template <int NF, int MT, int WA>
@@ -597,10 +640,11 @@ namespace {
 // What a block of penny_linear_rows takes for 2048 of K beyond its fixed 2.8 us, by its 16 nf columns and 16 mt rows
 struct RowsTile {
   int nf, mt;
-  float us;
+  float us, us32;                        // bf16, f32 (the tiles that f32 takes)
 };
-constexpr RowsTile kRowsTiles[] = {{2, 2, 4.6f}, {2, 4, 6.5f}, {4, 2, 6.7f},  {2, 6, 8.2f},  {4, 4, 9.8f},   {2, 8, 9.9f},  {4, 6, 11.7f},
-                                   {8, 2, 12.3f}, {4, 8, 15.f}, {8, 4, 15.3f}, {8, 6, 21.f}, {4, 12, 19.2f}, {8, 8, 24.f}};
+constexpr RowsTile kRowsTiles[] = {{2, 2, 4.6f, 13.6f}, {2, 4, 6.5f, 23.4f}, {4, 2, 6.7f, 24.4f}, {2, 6, 8.2f, 33.f}, {4, 4, 9.8f, 0.f},
+                                   {2, 8, 9.9f, 0.f},   {4, 6, 11.7f, 0.f},  {8, 2, 12.3f, 0.f},  {4, 8, 15.f, 0.f},  {8, 4, 15.3f, 0.f},
+                                   {8, 6, 21.f, 0.f},   {4, 12, 19.2f, 0.f}, {8, 8, 24.f, 0.f}};
 
 }  // namespace
 
@@ -617,39 +661,51 @@ constexpr RowsTile kRowsTiles[] = {{2, 2, 4.6f}, {2, 4, 6.5f}, {4, 2, 6.7f},  {2
 // rows and 8 at 2048.  Whole passes of 400, 600 and 1000 tokens, three hybrid decoders of width 1024, us: 1538 -> 1086, 1739 -> 1347, 1399 ->
 // 935; 1540 -> 1160, 1730 -> 1378, 1440 -> 976; 1570 -> 1399, 1790 -> 1526, 1505 -> 1125; width 2048 at 400: 1811 -> 1789, 1789 -> 1769, 1657
 // -> 1650.  Up to 96 rows, the steps of captured decodes, all but the longest are taken (14912 x 2048, 96 rows: 18.7 / 18.3).
-PENNY_API int penny_linear_rows_plan(int M, int N, int K) {
-  if (M <= 0 || M > 2048 || N < 512 || N % 16 || K <= 0 || K % 64) return 0;
+//
+// f32 (a sixteenth of the matrix rate; the four smallest tiles): the library's tiles are 1.1 - 1.3 times faster from 40 - 100 rows on where
+// the device counts (1024 x 3072, 64 rows 10.6 / 12.3; 2048 x 1024 at 150 11.4 / 14.7) and slower below (1024 x 1024 1 row 8.3 / 6.2, 64 8.7 / 7.3;
+// 2048 x 1024 16 rows 8.8 / 6.9; 1024 x 3072 10.9 / 9.0), so up to 256 rows the products of up to 11 us are taken.  Steps at width 1024: 14
+// rows decoding 956 -> 812, 50 1023 -> 916; 200 tokens, where the host is the bound, 1575 -> 1355.  Errors against 64 bits at most the library's
+// (K = 1024 1.6 - 2.9e-7 of the norm against 2.9 - 5.8e-7, K = 3072 2.0 - 2.6e-7 against 5.0e-7).
+PENNY_API int penny_linear_rows_plan(int M, int N, int K, int f32) {
+  if (M <= 0 || M > (f32 ? 256 : 2048) || N < 512 || N % 16 || K <= 0 || K % (f32 ? 32 : 64)) return 0;
   int plan = 0;
-  float best = M <= 96 ? 60.f : M <= 512 ? 20.f : 20.f - (M - 512) / 128.f;
-  for (int S = 1; S <= 4; S *= 2) {
+  float best = f32 ? 11.f : M <= 96 ? 60.f : M <= 512 ? 20.f : 20.f - (M - 512) / 128.f;
+  for (int S = 1; S <= (f32 ? 8 : 4); S *= 2) {
     if (S > 1 && (K % (64 * S) || K / S < 256)) break;
-    for (const RowsTile& t : kRowsTiles) {
+    for (int i = 0; i < (f32 ? 4 : (int)(sizeof(kRowsTiles) / sizeof(kRowsTiles[0]))); ++i) {
+      const RowsTile& t = kRowsTiles[i];
       const long blocks = (long)((N + 16 * t.nf - 1) / (16 * t.nf)) * ((M + 16 * t.mt - 1) / (16 * t.mt)) * S;
       if (S > 1 && blocks > 256) continue;
-      const float us = (blocks + 255) / 256 * (2.8f + t.us * (K / S) / 2048.f) + (S > 1 ? 2.f + 4e-6f * S * M * N : 0.f);
+      const float us = (blocks + 255) / 256 * (2.8f + (f32 ? t.us32 : t.us) * (K / S) / 2048.f) + (S > 1 ? 2.f + 4e-6f * S * M * N : 0.f);
       if (us < best) best = us, plan = t.nf | t.mt << 8 | S << 16;
     }
   }
   return plan;
 }
 
-// Y [M, N] = X [M, K] x W [N, K]^T in bf16 for up to about two thousand rows, W row-major: slabs == null streams W once (S = 1), else
+// Y [M, N] = X [M, K] x W [N, K]^T in bf16 or f32 (f32 != 0) for up to about two thousand rows, W row-major: slabs == null streams W once (S = 1), else
 // S slices of K leave f32 slabs [S, M, N] that a second launch adds.  One entry for both, so that a step that the host bounds
 // pays for one call.  nf, mt: a block's columns and rows in units of 16, one of kRowsTiles.  Contract (checked): N % 16 == 0 (the last
-// tile may be part-filled), K % (64 * S) == 0, ldx % 8 == 0, ldy % 8 == 0.
-PENNY_API int penny_linear_rows(const void* X, int ldx, const void* W, int K, void* Y, int ldy, int M, int N, void* slabs,
-                                int S, int nf, int mt, int paired, hipStream_t st) {
+// tile may be part-filled), K % (64 * S) == 0 (f32: 32 * S), rows of x in whole 16 bytes, y contiguous.
+PENNY_API int penny_linear_rows(const void* X, int ldx, const void* W, int K, void* Y, int M, int N, void* slabs, int S, int nf, int mt,
+                                int f32, int paired, hipStream_t st) {
   if (M <= 0) return 0;
-  if (M > (1 << 20) || N <= 0 || N % 16 || (nf != 2 && nf != 4 && nf != 8) || S < 1 || (S > 1) != (slabs != nullptr) || K <= 0 ||
-      K % (64 * S) || ldx % 8 || ldy % 8)
+  if (M > (1 << 20) || N <= 0 || N % 16 || S < 1 || (S > 1) != (slabs != nullptr) || K <= 0 || K % ((f32 ? 32 : 64) * S) ||
+      K > (1 << 28) || ldx % (f32 ? 4 : 8))
     return (int)hipErrorInvalidValue;
-  const int wrow = paired ? 3 : 1;
-  float* p = static_cast<float*>(slabs);
+  float* p = static_cast<float*>(f32 && S == 1 ? Y : slabs);
   int rc;
-#define LR_CASE(NF_, MT_, WA_)                                                       \
-  if (nf == NF_ && mt == MT_) {                                                      \
-    if (S > 1) rc = launch<NF_, MT_, WA_>(X, ldx, W, K, p, M, N, S, wrow, st);       \
-    else rc = launch_bf16<NF_, MT_, WA_>(X, ldx, W, K, Y, ldy, M, N, wrow, st);      \
+#define LR_CASE(NF_, MT_, WA_)                                                                     \
+  if (nf == NF_ && mt == MT_) {                                                                    \
+    if (f32) {                                                                                     \
+      if constexpr (NF_ * MT_ <= 12) rc = launch_f32<NF_, MT_, WA_>(X, ldx, W, K, p, M, N, S, paired, st); \
+      else return (int)hipErrorInvalidValue;                                                       \
+    } else if (S > 1) {                                                                            \
+      rc = launch<NF_, MT_, WA_>(X, ldx, W, K, p, M, N, S, paired ? 3 : 1, st);                    \
+    } else {                                                                                       \
+      rc = launch_bf16<NF_, MT_, WA_>(X, ldx, W, K, Y, N, M, N, paired ? 3 : 1, st);               \
+    }                                                                                              \
   } else
   LR_CASE(2, 2, 2)
   LR_CASE(2, 4, 1)
@@ -667,7 +723,10 @@ PENNY_API int penny_linear_rows(const void* X, int ldx, const void* W, int K, vo
   return (int)hipErrorInvalidValue;
 #undef LR_CASE
   if (rc || S == 1) return rc;
-  return penny_splitk_reduce(slabs, S, M, N, Y, ldy, nullptr, 0, st);
+  if (!f32) return penny_splitk_reduce(slabs, S, M, N, Y, N, nullptr, 0, st);
+  const long quads = (long)M * N / 4;
+  splitk_reduce_f32_kernel<<<dim3((unsigned)((quads + 255) / 256)), 256, 0, st>>>((const f32x4*)slabs, S, quads, (f32x4*)Y);
+  return (int)hipGetLastError();
 }
 
 // Weight-streaming LM head + sampler (K11 + K12) for decode batches, full vocabulary or a TP rank's

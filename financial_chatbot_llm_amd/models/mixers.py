@@ -509,7 +509,7 @@ class ChannelDeltaMixer:
         u = mx.conv_act(proj[:, :C], self.conv_w, None, st["conv"], meta.seg_cu, meta.seg_state, positions,
                         meta.seg_max_len, "silu")
         beta = proj[:, C:C + H]
-        a = F.linear(proj[:, C + H:C + H + self.ra].float(), self.a2)
+        a = project(proj[:, C + H:C + H + self.ra].float(), self.a2)
         o = mx.matrix_scan(u[:, :nq], u[:, nq:2 * nq], u[:, 2 * nq:], a, self.dt_bias, st["S"], meta.seg_cu,
                            meta.seg_state, positions, H, self.G, self.D, self.P, "delta", A_log=self.A_log, beta=beta,
                            max_len=meta.seg_max_len)
@@ -554,7 +554,7 @@ class GLAMixer:
     def forward(self, proj: torch.Tensor, positions: torch.Tensor, meta: AttentionMetadata, cache) -> torch.Tensor:
         st = cache[1]
         nq, nv = self.nq, self.nv
-        a = F.linear(proj[:, 2 * nq + 2 * nv:2 * nq + 2 * nv + self.ra].float(), self.a2)
+        a = project(proj[:, 2 * nq + 2 * nv:2 * nq + 2 * nv + self.ra].float(), self.a2)
         o = mx.matrix_scan(proj[:, :nq], proj[:, nq:2 * nq], proj[:, 2 * nq:2 * nq + nv], a, self.a2_b, st["S"],
                            meta.seg_cu, meta.seg_state, positions, self.H, self.H, self.D, self.P, "gla", tau=self.tau,
                            max_len=meta.seg_max_len)

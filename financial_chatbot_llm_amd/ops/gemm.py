@@ -251,26 +251,28 @@ def splitk_bf16(x: torch.Tensor, w: torch.Tensor, N_: int, nf: int, rowmajor: bo
     return y
 
 
-def rows_config(M: int, N_: int, K: int) -> Optional[Tuple[int, int, int]]:
+def rows_config(M: int, N_: int, K: int, dtype: torch.dtype = torch.bfloat16) -> Optional[Tuple[int, int, int]]:
     """(nf, mt, S) of ``penny_linear_rows`` for M rows on a row-major weight, or None: the library's product (the rule and its
     measurements stand at ``penny_linear_rows_plan``)."""
-    plan = N.load().penny_linear_rows_plan(M, N_, K)
+    plan = N.load().penny_linear_rows_plan(M, N_, K, dtype == torch.float32)
     return (plan & 255, plan >> 8 & 255, plan >> 16) if plan else None
 
 
 def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """y = x @ w.T: the streaming kernels for up to about two thousand rows (``rows_config``), the library's product for the rest."""
-    if w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 2 and N.use_native(x):
-        (M, K), N_ = x.shape, w.shape[0]
+    """y = x @ w.T in bf16 or f32: the streaming kernels for up to about two thousand rows (``rows_config``), the library's product for
+    the rest."""
+    dt = x.dtype
+    if dt == w.dtype and (dt == torch.bfloat16 or dt == torch.float32) and x.dim() == 2 and w.dim() == 2 and N.use_native(x):
+        (M, K), N_, f32 = x.shape, w.shape[0], dt == torch.float32
         ldx, xp, wp = x.stride(0), x.data_ptr(), w.data_ptr()
-        if M <= 2048 and K == w.shape[1] and (xp | wp) % 16 == 0 and ldx % 8 == 0 and ldx >= K and x.stride(1) == 1 and \
+        if M <= 2048 and K == w.shape[1] and (xp | wp) % 16 == 0 and ldx % (4 if f32 else 8) == 0 and ldx >= K and x.stride(1) == 1 and \
                 w.is_contiguous() and w.device == x.device and not (w.requires_grad or x.requires_grad):
-            plan = N.load().penny_linear_rows_plan(M, N_, K)
+            plan = N.load().penny_linear_rows_plan(M, N_, K, f32)
             if plan:
                 S = plan >> 16
-                y = torch.empty((M, N_), dtype=x.dtype, device=x.device)
+                y = torch.empty((M, N_), dtype=dt, device=x.device)
                 slabs = torch.empty((S, M, N_), dtype=torch.float32, device=x.device) if S > 1 else None
-                N.call("penny_linear_rows", xp, ldx, wp, K, y.data_ptr(), N_, M, N_, N.ptr(slabs), S, plan & 255, plan >> 8 & 255,
+                N.call("penny_linear_rows", xp, ldx, wp, K, y.data_ptr(), M, N_, N.ptr(slabs), S, plan & 255, plan >> 8 & 255, f32,
                        PAIR_MODE != "0", N.stream())
                 return y
     return F.linear(x, w)

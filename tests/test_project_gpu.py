@@ -11,36 +11,40 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 2, 15, 16, 17, 33, 63, 64, 65, 96, 97, 160, 256, 400, 1000, 1024, 1500, 2048, 2049])
 @pytest.mark.parametrize("N_,K", [(512, 64), (528, 128), (2048, 2048), (4096, 2048), (7216, 448), (2064, 3072), (10256, 192),
                                   (10240, 128), (1024, 4096), (1024, 1024), (5168, 1024), (2048, 4160), (500, 128), (512, 96)])
-def test_against_float64(M, N_, K):
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_against_float64(dt, M, N_, K):
     g = torch.Generator().manual_seed(M + N_ + K)
-    w = (torch.randn((N_, K), generator=g) * K ** -0.5).to(torch.bfloat16).cuda()
-    rows = torch.randn((M, K + 24), generator=g).to(torch.bfloat16).cuda()
+    w = (torch.randn((N_, K), generator=g) * K ** -0.5).to(dt).cuda()
+    rows = torch.randn((M, K + 24), generator=g).to(dt).cuda()
+    e = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -20
     for off in (0, 16, 3):                                   # 3: rows off the kernel's 16 bytes
         x = rows[:, off:off + K]
         y = G.project(x, w)
         want = x.double() @ w.double().t()
-        assert y.is_contiguous() and y.shape == (M, N_) and y.dtype == torch.bfloat16
-        # one rounding of the result to eight significant bits; K f32 products of values of order K^-0.5
-        assert ((y.double() - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -18 * K ** 0.5).all()
+        assert y.is_contiguous() and y.shape == (M, N_) and y.dtype == dt
+        # one rounding of the result (bf16: to eight significant bits); K f32 products of values of order K^-0.5
+        assert ((y.double() - want).abs() <= want.abs() * e + 2.0 ** -18 * K ** 0.5).all()
 
 
 def test_every_tile():
     """Each tile and split that the launcher knows, with part-filled tiles on both sides."""
     from financial_chatbot_llm_amd.ops import _native as N
     g = torch.Generator().manual_seed(1)
-    w = (torch.randn((528, 512), generator=g) * 512 ** -0.5).to(torch.bfloat16).cuda()
-    x = torch.randn((150, 512), generator=g).to(torch.bfloat16).cuda()
-    want = x.double() @ w.double().t()
-    for nf, mt in ((2, 2), (2, 4), (4, 2), (2, 6), (4, 4), (2, 8), (4, 6), (8, 2), (4, 8), (8, 4), (8, 6), (4, 12), (8, 8)):
+    w32 = (torch.randn((528, 512), generator=g) * 512 ** -0.5).cuda()
+    x32 = torch.randn((150, 512), generator=g).cuda()
+    for f32, nf, mt in [(1, nf, mt) for nf, mt in ((2, 2), (2, 4), (4, 2), (2, 6))] + [(0, nf, mt) for nf, mt in ((2, 2), (2, 4), (4, 2), (2, 6), (4, 4), (2, 8), (4, 6), (8, 2), (4, 8), (8, 4), (8, 6), (4, 12), (8, 8))]:
+        dt = torch.float32 if f32 else torch.bfloat16
+        w, x = w32.to(dt), x32.to(dt)
+        want = x.double() @ w.double().t()
         for S in (1, 2, 4):
             for paired in (0, 1):
-                y = torch.zeros((151, 528), dtype=torch.bfloat16, device="cuda")
+                y = torch.zeros((151, 528), dtype=dt, device="cuda")
                 slabs = torch.empty((S, 150, 528), device="cuda") if S > 1 else None
-                N.call("penny_linear_rows", N.ptr(x), 512, N.ptr(w), 512, N.ptr(y), 528, 150, 528, N.ptr(slabs), S, nf, mt, paired, N.stream())
-                assert ((y[:150].double() - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -18 * 512 ** 0.5).all(), (nf, mt, S, paired)
+                N.call("penny_linear_rows", N.ptr(x), 512, N.ptr(w), 512, N.ptr(y), 150, 528, N.ptr(slabs), S, nf, mt, f32, paired, N.stream())
+                assert ((y[:150].double() - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -18 * 512 ** 0.5).all(), (f32, nf, mt, S, paired)
                 assert (y[150] == 0).all()
     with pytest.raises(RuntimeError):
-        N.call("penny_linear_rows", N.ptr(x), 512, N.ptr(w), 512, N.ptr(y), 528, 150, 528, None, 1, 2, 16, 1, N.stream())
+        N.call("penny_linear_rows", N.ptr(x), 512, N.ptr(w), 512, N.ptr(y), 150, 528, None, 1, 2, 16, 0, 1, N.stream())
 
 
 def test_rule():
@@ -53,7 +57,8 @@ def test_rule():
 def test_other_calls_keep_the_library():
     w = torch.randn((512, 128), device="cuda")
     x = torch.randn((3, 128), device="cuda")
-    assert torch.equal(G.project(x, w), torch.nn.functional.linear(x, w))
+    assert torch.equal(G.project(x.half(), w.half()), torch.nn.functional.linear(x.half(), w.half()))
+    assert G.rows_config(257, 512, 128, torch.float32) is None
     wb, xb = w.bfloat16(), x.bfloat16()
     assert G.project(xb[None], wb).shape == (1, 3, 512) and G.project(xb[0], wb).shape == (512,)
     assert G.project(xb, wb.clone().requires_grad_()).requires_grad
