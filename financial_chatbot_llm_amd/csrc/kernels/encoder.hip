@@ -235,6 +235,46 @@ PENNY_API int penny_encoder_attention(const void* qkv, long ld, const int* cu, i
   PENNY_RETURN_LAUNCH();
 }
 
+// gemm_splitk.hip
+extern "C" int penny_bias_rows_tile(int M, int N, int K);
+extern "C" int penny_bias_rows(const void* X, int ldx, const void* W, int K, void* Y, int ldy, const void* bias, int M, int N, int gelu, int nf,
+                               int mt, hipStream_t st);
+
+namespace {
+
+// Slices of K for the second projection of the feed-forward: as many as bring its blocks near the CUs, 512 of K each at least;
+// 1: not split.  A query of 12 layers of 768 x 3072, us unsplit / in 2 / 3 / 4 / 6: 6 tokens 422 / 412 / 419 / 414 / 414, 18: 467 / 438 /
+// 437 / 441 / 451, 32: 505 / 472 / 466 / 459 / 466, 48: 599 / 536 / 521 / 511 / 523, 64: 634 / 565 / 550 / 545 / 556, 84: 680 / 611 / 623 / 621 /
+// 611, 109: 701 / 627 / 652 / 637 / 640, 179: 743 / 658 / 633 / 669 / 645.
+int few_slices(int M, int N, int K) {
+  if (N != 256 && N != 512 && N != 768 && N != 1024) return 1;
+  const long blocks = M <= 128 ? (long)(N / 16) * ((M + 63) / 64) : (long)((N + 31) / 32) * ((M + 63) / 64);
+  const long s = 216 / blocks, most = K / 512;
+  return (int)(s < most ? (s > 1 ? s : 1) : (most > 1 ? most : 1));
+}
+
+}  // namespace
+
+// The tile (nf | mt << 8) with which a projection goes through the LDS ring of gemm_splitk.hip instead of the kernel above, or 0.
+// Blocks of the kernel above read both operands for themselves, which costs more with every further row tile; the ring's tiles share
+// them, one round of blocks for all. Us, above (its slices included) or the tile kernel / ring: 2304 x 768 18 rows 4.0 / 4.8, 48 5.5 / 4.8,
+// 128 9.3 / 5.8, 256 11.0 / 6.7, 768 20.1 / 11.0, 1536 21.3 / 16.8, 2048 21.6 / 24.8 (two rounds); 768 x 768 48 5.0 / 4.5, 768 10.6 / 6.3, 1536
+// 20.2 / 9.0; 3072 x 768 with GELU 128 9.6 / 6.2, 768 24.5 / 15.4, 1024 27.8 / 19.0; 768 x 3072 48 8.8 / 10.0, 192 (in slices, which
+// the next norm adds) 8.8 / 10.4, 256 11 / 10.4, 768 35.1 / 15.6, 2048 38.4 / 27.5; 4096 x 1024 512 31.4 / 14.0; 1024 x 4096 128 20.5 / 12.7.  Widths that
+// the tile kernel does not take have the library behind them: 1152 x 384 256 4.5 / 4.2, 1024 8.0 / 6.9, 2048 9.5 / 10.2; 384 x 1536 64 - 192 4.9 /
+// 6.5: not there.
+PENNY_API int penny_bias_rows_plan(int M, int N, int K) {
+  if (M <= 32 || N < 16 || N % 16 || K < 64 || K % 64 || M > (N % 256 == 0 ? 2048 : K <= 1024 ? 1024 : 0)) return 0;
+  if (M <= 192 && few_slices(M, N, K) > 1) return 0;
+  return penny_bias_rows_tile(M, N, K);
+}
+
+namespace {
+
+int small_slices(int M, int N, int K) { return penny_bias_rows_plan(M, N, K) ? 1 : few_slices(M, N, K); }
+
+}  // namespace
+
 // Y [M, N] (row stride ldy) = bf16(X W^T + bias) [-> exact GELU]; W [N, K] contiguous; N % 16 == 0, K % 32 == 0, rows in
 // whole 16 bytes
 PENNY_API int penny_gemm_bias_small(const void* X, int ldx, const void* W, int K, void* Y, int ldy, const void* bias, int M,
@@ -243,6 +283,8 @@ PENNY_API int penny_gemm_bias_small(const void* X, int ldx, const void* W, int K
   if (N % 16 || K % 32 || ldx % 8 || ldy % 4 || ((size_t)X | (size_t)W) % 16 || ((size_t)Y | (size_t)bias) % 8 ||
       (M + 15) / 16 > 65535)
     return (int)hipErrorInvalidValue;
+  if (const int tile = penny_bias_rows_plan(M, N, K))
+    return penny_bias_rows(X, ldx, W, K, Y, ldy, bias, M, N, gelu, tile & 255, tile >> 8, stream);
 #define SMALL(NF, MF)                                                                                                    \
   do {                                                                                                                   \
     const dim3 grid((N + 16 * NF - 1) / (16 * NF), (M + 16 * MF - 1) / (16 * MF));                                       \
@@ -368,17 +410,6 @@ __global__ void __launch_bounds__(256) layernorm_slab_kernel(const float* __rest
     for (int i = 0; i < 4; ++i) o[i] = (bf16)((v[c][i] - mu) * inv * (float)gg[c][i] + (float)bb[c][i]);
     reinterpret_cast<bf16x4*>(y + (long)row * H)[lane + 64 * c] = o;
   }
-}
-
-// Slices of K for the second projection of the feed-forward: as many as bring its blocks near the CUs, 512 of K each at least;
-// 1: not split.  A query of 12 layers of 768 x 3072, us unsplit / in 2 / 3 / 4 / 6: 6 tokens 422 / 412 / 419 / 414 / 414, 18: 467 / 438 /
-// 437 / 441 / 451, 32: 505 / 472 / 466 / 459 / 466, 48: 599 / 536 / 521 / 511 / 523, 64: 634 / 565 / 550 / 545 / 556, 84: 680 / 611 / 623 / 621 /
-// 611, 109: 701 / 627 / 652 / 637 / 640, 179: 743 / 658 / 633 / 669 / 645.
-int small_slices(int M, int N, int K) {
-  if (N != 256 && N != 512 && N != 768 && N != 1024) return 1;
-  const long blocks = M <= 128 ? (long)(N / 16) * ((M + 63) / 64) : (long)((N + 31) / 32) * ((M + 63) / 64);
-  const long s = 216 / blocks, most = K / 512;
-  return (int)(s < most ? (s > 1 ? s : 1) : (most > 1 ? most : 1));
 }
 
 // y = bf16(sum of the S slabs + bias), four columns per thread

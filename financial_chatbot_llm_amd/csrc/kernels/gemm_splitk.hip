@@ -41,7 +41,7 @@ union Frag {
 };
 
 // epilogues of splitk_gemm_kernel
-enum { SK_SLAB = 0, SK_SILU = 1, SK_BF16 = 2, SK_SAMPLE = 3, SK_F32 = 4 };
+enum { SK_SLAB = 0, SK_SILU = 1, SK_BF16 = 2, SK_SAMPLE = 3, SK_F32 = 4, SK_BIAS = 5 };
 
 // SK_SAMPLE (the streaming LM head + K12 sampler): per-row temperature (<= 0: greedy) and seed;
 // pv / pi [M, pstride] partial (best score, token) per (row, workgroup tile, wave row).  Token
@@ -52,6 +52,8 @@ struct SkSample {
   float* pv;
   int* pi;
   int pstride, voff, vvalid;
+  const bf16* bias;                      // SK_BIAS
+  int gelu;
 };
 
 // X image: token row r of a stage lives at byte r*128; its logical 16-B chunk c (k = 8c..8c+7) at
@@ -138,6 +140,7 @@ __device__ __forceinline__ void stage_mma(const char* __restrict__ base, f32x4 (
 }
 
 // Epilogues (EPI):
+//   SK_BIAS   SK_BF16 with a bias row and, where asked for, the exact GELU of the rounded sum (encoder projections);
 //   SK_F32    SK_SLAB for f32 operands, which are addressed as twice as many 16-bit columns (K, ldx);
 //   SK_SLAB   f32 partial slabs P [S, M, N] (reduced by the consumer's row pass);
 //   SK_SILU   W is the 16-row-interleaved gate|up weight (ops/gemm.py interleave16) and S == 1: the
@@ -186,9 +189,9 @@ __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restr
   const int Mtot = M, m0 = blockIdx.y * 16 * MT;
   M = min(Mtot - m0, 16 * MT);
   X += (long)m0 * ldx;
-  if constexpr (EPI == SK_SILU || EPI == SK_BF16) Y += (long)m0 * ldy;
+  if constexpr (EPI == SK_SILU || EPI == SK_BF16 || EPI == SK_BIAS) Y += (long)m0 * ldy;
   PENNY_DASSERT(M > 0 && (EPI != SK_SAMPLE || gridDim.y == 1));
-  PENNY_DASSERT((tile + 1) * 16 * NF <= N || (WROW && N % 16 == 0 && tile * 16 * NF < N && (EPI == SK_BF16 || EPI == SK_SLAB || EPI == SK_F32)));
+  PENNY_DASSERT((tile + 1) * 16 * NF <= N || (WROW && N % 16 == 0 && tile * 16 * NF < N && (EPI == SK_BF16 || EPI == SK_BIAS || EPI == SK_SLAB || EPI == SK_F32)));
   PENNY_DASSERT(K % (64 * BKM * S) == 0);
   const int n0 = tile * 16 * NF;
   const int kc = K / S, k0 = s * kc;
@@ -289,7 +292,7 @@ __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restr
     }
     return;
   }
-  if constexpr (EPI == SK_BF16) {
+  if constexpr (EPI == SK_BF16 || EPI == SK_BIAS) {
     // lane holds W rows n = 16f + 4g + r (r = 0..3) for token 16t + col: one 8-B store per fragment
 #pragma unroll
     for (int t = 0; t < TW; ++t) {
@@ -299,8 +302,17 @@ __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restr
       for (int f = 0; f < FW; ++f) {
         if (WROW && n0 + (wa * FW + f) * 16 >= N) break;
         bf16x4 o;
+        if constexpr (EPI == SK_BIAS) {
+          const bf16x4 bv = *reinterpret_cast<const bf16x4*>(sa.bias + n0 + (wa * FW + f) * 16 + 4 * g);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = (bf16)acc[f][t][r];
+          for (int r = 0; r < 4; ++r) {
+            const bf16 v = (bf16)(acc[f][t][r] + (float)bv[r]);
+            o[r] = sa.gelu ? (bf16)gelu_erf((float)v) : v;     // the roundings of gemm_bias_small_kernel
+          }
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[r] = (bf16)acc[f][t][r];
+        }
         *reinterpret_cast<bf16x4*>(Y + (long)m * ldy + n0 + (wa * FW + f) * 16 + 4 * g) = o;
       }
     }
@@ -727,6 +739,46 @@ PENNY_API int penny_linear_rows(const void* X, int ldx, const void* W, int K, vo
   const long quads = (long)M * N / 4;
   splitk_reduce_f32_kernel<<<dim3((unsigned)((quads + 255) / 256)), 256, 0, st>>>((const f32x4*)slabs, S, quads, (f32x4*)Y);
   return (int)hipGetLastError();
+}
+
+// The tile of penny_bias_rows for M rows: the fastest that runs all its blocks in one round; 0: none does
+extern "C" int penny_bias_rows_tile(int M, int N, int K) {
+  int tile = 0;
+  float best = 1e9f;
+  for (const RowsTile& t : kRowsTiles) {
+    const long blocks = (long)((N + 16 * t.nf - 1) / (16 * t.nf)) * ((M + 16 * t.mt - 1) / (16 * t.mt));
+    if (blocks <= 256 && t.us < best) best = t.us, tile = t.nf | t.mt << 8;
+  }
+  return tile;
+}
+
+// Y [M, N] (row stride ldy) = bf16(X W^T + bias) [-> exact GELU] on the same tiles, for penny_gemm_bias_small
+extern "C" int penny_bias_rows(const void* X, int ldx, const void* W, int K, void* Y, int ldy, const void* bias, int M, int N, int gelu, int nf, int mt,
+                    hipStream_t st) {
+  if (M <= 0) return 0;
+  if (M > (1 << 20) || N <= 0 || N % 16 || K <= 0 || K % 64 || ldx % 8 || ldy % 4) return (int)hipErrorInvalidValue;
+  SkSample sa{};
+  sa.bias = static_cast<const bf16*>(bias);
+  sa.gelu = gelu;
+#define BR_CASE(NF_, MT_, WA_)                                                                                          \
+  if (nf == NF_ && mt == MT_)                                                                                           \
+    return launch_any<NF_, MT_, WA_, SK_BIAS, 16>(3, K % 128 == 0, dim3((N + 16 * NF_ - 1) / (16 * NF_), (M + 16 * MT_ - 1) / (16 * MT_)), \
+                                                  st, (const bf16*)X, ldx, (const bf16*)W, K, (float*)nullptr, M, N, 1, (bf16*)Y, ldy, sa);
+  BR_CASE(2, 2, 2)
+  BR_CASE(2, 4, 1)
+  BR_CASE(4, 2, 2)
+  BR_CASE(2, 6, 2)
+  BR_CASE(4, 4, 1)
+  BR_CASE(2, 8, 1)
+  BR_CASE(4, 6, 2)
+  BR_CASE(8, 2, 2)
+  BR_CASE(4, 8, 1)
+  BR_CASE(8, 4, 2)
+  BR_CASE(8, 6, 2)
+  BR_CASE(4, 12, 1)
+  BR_CASE(8, 8, 2)
+#undef BR_CASE
+  return (int)hipErrorInvalidValue;
 }
 
 // Weight-streaming LM head + sampler (K11 + K12) for decode batches, full vocabulary or a TP rank's

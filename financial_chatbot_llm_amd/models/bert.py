@@ -84,10 +84,11 @@ class BertEncoder:
         return ops.layer_norm(e_word, w["emb_ln_g"], w["emb_ln_b"], c.norm_eps, residual=e_pos)
 
     def _small_batch(self, x: torch.Tensor, cu: torch.Tensor, longest: int) -> bool:
-        """All layers of a batch of up to BGE_SMALL_MAX_M tokens (fewer in wide models) in one native call (x in place); False:
-        not a case for it."""
+        """All layers of a batch of up to BGE_SMALL_MAX_M tokens (fewer in wide models), or of more where every projection is one round
+        of blocks, in one native call (x in place); False: not a case for it."""
         T, F_ = x.shape[0], self.cfg.intermediate_size
-        if not (N.use_native(x) and T <= BGE_SMALL_MAX_M and T * self.H * max(F_, 3 * self.H) < SMALL_MAX_MADS and
+        if not (N.use_native(x) and (T <= BGE_SMALL_MAX_M and T * self.H * max(F_, 3 * self.H) < SMALL_MAX_MADS or T <= 2048 and all(
+                N.load().penny_bias_rows_plan(T, n, k) for n, k in ((3 * self.H, self.H), (self.H, self.H), (F_, self.H), (self.H, F_)))) and
                 x.dtype == torch.bfloat16 and cu.numel() <= 65536 and self.H % 32 == 0 and F_ % 32 == 0 and
                 os.environ.get("PENNY_PREFILL_GEMM", "1") == "1"):
             return False

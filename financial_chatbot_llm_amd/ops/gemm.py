@@ -849,14 +849,15 @@ def _bias_row(b: Optional[torch.Tensor], w: torch.Tensor) -> bool:
 
 
 def linear_bias(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, gelu: bool = False) -> torch.Tensor:
-    """Encoder projection bf16(x @ w.T + b) [-> exact GELU]: the small-batch kernel up to BGE_SMALL_MAX_M tokens, the
-    tile kernel with the bias (+GELU) epilogue always up to BGE_TILE_MAX_M tokens and by the measured per-shape
+    """Encoder projection bf16(x @ w.T + b) [-> exact GELU]: the small-batch kernels up to BGE_SMALL_MAX_M tokens and where one round of
+    blocks holds them all (``penny_bias_rows_plan``), the tile kernel with the bias (+GELU) epilogue always up to BGE_TILE_MAX_M tokens and by the measured per-shape
     policy for bulk ingest; hipBLASLt's bias GEMM + the HIP GELU pass otherwise
     (``PENNY_PREFILL_GEMM=0``: always the library)."""
     M, K = x.shape
     N_ = w.shape[0]
     mode = os.environ.get("PENNY_PREFILL_GEMM", "1")
-    if mode == "1" and small_bias_wins(M, N_, K) and small_bias_ok(x, w) and _bias_row(b, w):
+    if mode == "1" and (small_bias_wins(M, N_, K) or M <= 2048 and N.use_native(x) and N.load().penny_bias_rows_plan(M, N_, K)) and \
+            small_bias_ok(x, w) and _bias_row(b, w):
         y = torch.empty((M, N_), dtype=x.dtype, device=x.device)
         slices = 1 if gelu else N.load().penny_encoder_slices(M, N_, K)
         if slices > 1:                   # a long K over few column tiles
