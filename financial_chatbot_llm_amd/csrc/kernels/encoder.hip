@@ -4,7 +4,7 @@
 //   penny_encoder_attention   every text attends within itself; most are short (a query or a transaction: 6 - 128
 //                             tokens), so a 64-token tile of one (text, head) is about a whole problem, and no paged cache
 //                             is written first.
-//   penny_gemm_bias_small     bf16(x w^T + b) [-> exact GELU] for up to a few hundred rows.
+//   penny_gemm_bias_small     bf16(x w^T + b) [-> exact GELU] for up to some two thousand rows, most of them on gemm_splitk.hip's tiles.
 //   penny_encoder_embed       word + position + type rows and their layer norm in one pass.
 //   penny_encoder_layers      the launches of all layers of a small batch, from one call.
 //   penny_encoder_pool        the texts' first rows, normalised.

@@ -251,16 +251,9 @@ def splitk_bf16(x: torch.Tensor, w: torch.Tensor, N_: int, nf: int, rowmajor: bo
     return y
 
 
-def rows_config(M: int, N_: int, K: int, dtype: torch.dtype = torch.bfloat16) -> Optional[Tuple[int, int, int]]:
-    """(nf, mt, S) of ``penny_linear_rows`` for M rows on a row-major weight, or None: the library's product (the rule and its
-    measurements stand at ``penny_linear_rows_plan``)."""
-    plan = N.load().penny_linear_rows_plan(M, N_, K, dtype == torch.float32)
-    return (plan & 255, plan >> 8 & 255, plan >> 16) if plan else None
-
-
 def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """y = x @ w.T in bf16 or f32: the streaming kernels for up to about two thousand rows (``rows_config``), the library's product for
-    the rest."""
+    """y = x @ w.T in bf16 or f32: the streaming kernels for up to about two thousand rows (``penny_linear_rows_plan``), the library's
+    product for the rest."""
     dt = x.dtype
     if dt == w.dtype and (dt == torch.bfloat16 or dt == torch.float32) and x.dim() == 2 and w.dim() == 2 and N.use_native(x):
         (M, K), N_, f32 = x.shape, w.shape[0], dt == torch.float32
@@ -815,11 +808,12 @@ def tail_workspace(dev: torch.device) -> Tuple:
 # vs 2.26 ms for 64 (1.5k tokens) against hipBLASLt + the GELU pass, profiles/r3_bge_query_tile_vs_hipblaslt.jsonl); at 4k
 # tokens the per-shape policy decides
 BGE_TILE_MAX_M = 2048
-# ... and up to this many the small-batch kernel, whose blocks of 16 - 32 weight rows fill the chip.  bge projections, us
-# (small / tile): 2304 x 768 4.3 / 17 at 18 rows, 11 / 22 at 256, 20 / 22 at 768, 24 / 22 at 1024; 768 x 3072 8 / 32, 19 / 36,
-# 36 / 38, 36 / 38; 3072 x 768 with GELU 4.5 / 26, 12 / 35, 26 / 36, 30 / 36
+# ... and up to this many the small-batch entry, on the tiles of gemm_splitk.hip's ring from 33 rows on (penny_bias_rows_plan, which
+# goes beyond this number where one round of blocks holds a projection) and blocks of 16 - 32 weight rows below and beside them.  bge
+# projections, us (small / 256 x 256 tiles): 2304 x 768 4.0 / 17 at 18 rows, 6.7 / 22 at 256, 11 / 22 at 768, 13.6 / 22 at 1024; 768 x 3072 6.9 / 32,
+# 10.4 / 36, 15.6 / 38, 18.4 / 38; 3072 x 768 with GELU 4.2 / 26, 8.2 / 35, 15.4 / 36, 19 / 36
 BGE_SMALL_MAX_M = 768
-# Every block of it reads its own rows of both operands, about 9 TB/s from the caches, so that wide layers reach the tile
+# Off the ring every block reads its own rows of both operands, about 9 TB/s from the caches, so that wide layers reach the tile
 # kernel's time sooner: at about 2^31 multiply-adds (8192 x 2048 at 128 rows 38 / 35, at 512 88 / 41; 4096 x 1024 at 512
 # 26 / 26, at 768 35 / 26; 1024 x 4096 at 640 45 / 41).  Shapes that the tile kernel does not take have the library's product
 # behind them, whose splits of K win with few columns (384 x 1536, us small / library: 18 rows 5.3 / 5.3, 64 9.0 / 5.3; 1152 x 384:
