@@ -3,7 +3,8 @@
 //
 // At one row a layer of Llama-3-8B is 436 MB of weights, 75 us at the rate of a large copy; the split-K kernels
 // (gemm_splitk.hip) with their separate norms, slab sums and reduce-SiLU pass take ten launches for it, of which the small
-// ones last 3 - 5 us each whatever they do: 101 us with 26 of them beside the weights, 78 here.  A workgroup owns 16 rows of W (a
+// ones last 3 - 5 us each whatever they do: 101 us with 26 of them beside the weights, 78 here, and
+// the QKV form rotates and writes the cache as well (13.2 -> 10.7).  A workgroup owns 16 rows of W (a
 // pair of gate and up groups) over all of K: its waves divide K, so no slabs, and each keeps 8 - 16 pieces of 1 KiB of W in flight
 // in registers; the tokens' rows lie in LDS.  W's first pieces are issued before the norm waits for its row, so that the
 // norm costs about its own latency once per launch.  Bound by the memory rate (5.9 TB/s for gate|up, 5.75 for the down
@@ -11,13 +12,14 @@
 // W: tile_weight's copy -- a piece is one A operand of the 16x16x32 matrix instruction -- and the tokens are its columns: one
 // instruction per KiB of W whatever the number of rows.
 #include "common.h"
+#include "kv_layout.h"
 
 namespace {
 
 constexpr int FEW_ROWS = 4;              // tokens at most
 constexpr int FEW_PAD = 64;              // bytes behind a token's row in LDS: four tokens at one k meet different banks
 
-enum { FEW_SLAB = 0, FEW_ADD = 1, FEW_SILU = 2 };
+enum { FEW_SLAB = 0, FEW_ADD = 1, FEW_SILU = 2, FEW_ROPE = 3 };
 
 struct FewRows {
   const bf16* x;                         // [M, K], row stride ldx
@@ -27,18 +29,27 @@ struct FewRows {
   long ldx, ldy;
   int M, N, K;
   float eps;
+  // FEW_ROPE (heads of 128): y is q [M, Hq, 128]
+  const int* positions;
+  const float* cos_sin;                  // [positions, 128]: cos of 64 frequencies, then sin
+  const int* slots;                      // of the paged cache; < 0: not written
+  bf16* kc;
+  bf16* vc;
+  int Hq, Hkv;
 };
 
 // NORM: K <= 4096.  XB: bytes of LDS for the rows; NW waves; DEPTH pieces of W in flight per wave.
 template <int EPI, bool NORM, int XB, int NW, int DEPTH>
 __global__ void __launch_bounds__(NW * 64) few_rows_kernel(FewRows a) {
-  constexpr int GROUPS = EPI == FEW_SILU ? 2 : 1, KW = NW / GROUPS, THREADS = NW * 64;
+  constexpr int GROUPS = EPI == FEW_SILU || EPI == FEW_ROPE ? 2 : 1, KW = NW / GROUPS, THREADS = NW * 64;
   __shared__ __attribute__((aligned(16))) char xs[XB];
   __shared__ f32x4 part[NW][64];
   __shared__ float sums[NW][FEW_ROWS];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, col = lane & 15;
   const int pitch = a.K * 2 + FEW_PAD, pieces = a.K / 32;
-  const int group = blockIdx.x * GROUPS + w / KW, part_k = w % KW;
+  // FEW_ROPE: a block owns the pairs of a rotation, row groups r and r + 4 of a head's eight
+  const int group = EPI == FEW_ROPE ? (blockIdx.x >> 2) * 8 + (blockIdx.x & 3) + 4 * (w / KW) : blockIdx.x * GROUPS + w / KW;
+  const int part_k = w % KW;
   const int p0 = pieces * part_k / KW, p1 = pieces * (part_k + 1) / KW;
   PENNY_DASSERT(a.M >= 1 && a.M <= FEW_ROWS && a.M * pitch <= XB && group * 16 < a.N);
 
@@ -159,6 +170,43 @@ __global__ void __launch_bounds__(NW * 64) few_rows_kernel(FewRows a) {
 #pragma unroll
     for (int i = 1; i < KW; ++i) sum[s] += part[s * KW + i][lane];
   }
+  if constexpr (EPI == FEW_ROPE) {         // as rope_kv_kernel with slabs: sums rounded to bf16, rotated in f32, rounded
+    const int h = blockIdx.x >> 2, d = 16 * (blockIdx.x & 3) + 4 * g, slot = a.slots[col];
+    float x1[4], x2[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x1[i] = (float)(bf16)sum[0][i], x2[i] = (float)(bf16)sum[1][i];
+    if (h < a.Hq + a.Hkv) {
+      const float* cs = a.cos_sin + (long)a.positions[col] * 128 + d;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float co = cs[i], si = cs[64 + i], p = x1[i], q = x2[i];
+        x1[i] = p * co - q * si;
+        x2[i] = q * co + p * si;
+      }
+    }
+    bf16x4 o1, o2;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o1[i] = (bf16)x1[i], o2[i] = (bf16)x2[i];
+    const long blk = slot >= 0 ? slot / KV_BS : 0;
+    const int off = slot >= 0 ? slot % KV_BS : 0;
+    if (h < a.Hq) {
+      bf16* dst = static_cast<bf16*>(a.y) + ((long)col * a.Hq + h) * 128 + d;
+      *reinterpret_cast<bf16x4*>(dst) = o1;
+      *reinterpret_cast<bf16x4*>(dst + 64) = o2;
+    } else if (slot >= 0 && h < a.Hq + a.Hkv) {   // four adjacent channels lie in one 16-byte piece
+      bf16* dst = a.kc + (blk * a.Hkv + h - a.Hq) * (long)(KV_BS * 128);
+      *reinterpret_cast<bf16x4*>(dst + k_index(off, d, 128)) = o1;
+      *reinterpret_cast<bf16x4*>(dst + k_index(off, d + 64, 128)) = o2;
+    } else if (slot >= 0) {
+      bf16* dst = a.vc + (blk * a.Hkv + h - a.Hq - a.Hkv) * (long)(KV_BS * 128);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        dst[v_index(off, d + i, 128)] = o1[i];
+        dst[v_index(off, d + 64 + i, 128)] = o2[i];
+      }
+    }
+    return;
+  }
   const int n = blockIdx.x * 16 + 4 * g;   // this lane's four adjacent outputs of token col
   if constexpr (EPI == FEW_SLAB) {
     *reinterpret_cast<f32x4*>(static_cast<float*>(a.y) + col * a.ldy + n) = sum[0];
@@ -183,11 +231,12 @@ __global__ void __launch_bounds__(NW * 64) few_rows_kernel(FewRows a) {
 // Waves of a block and pieces in flight per wave, us of one row (four rows) on weights beyond the caches.  gate|up of 28672 x 4096: 8
 // waves x 16 pieces 39.6 (40.3), 8 x 8 39.5 (40.6), 4 x 16 40.9 (40.2), 16 x 8 41.0 (45.7); QKV of 6144 x 4096: 8 x 12 10.4 (12.5), 8 x 16
 // 11.3 (12.8), 4 x 16 11.2 (11.5); the adding form, 4096 x 14336: 16 x 8 20.4 (20.9), 8 x 24 21.0 (22.2), 4096 x 4096: 7.7 (8.4) and 9.1
-// (9.8).  With loads that stay in the caches these were 42.3, 11.0, 22.8 and 8.5.
+// (9.8); QKV with its rotation and cache write behind it 16 x 8 10.7 (12.7), 16 x 12 11.3 (13.0), 8 x 16 13.8 (14.9), as two launches 13.2 (15.5).
+// With loads that stay in the caches these were 42.3, 11.0, 22.8 and 8.5.
 template <int EPI, bool NORM>
 int launch_few(const FewRows& a, hipStream_t st) {
-  const dim3 grid(a.N / (EPI == FEW_SILU ? 32 : 16));
-  constexpr int NW = EPI == FEW_ADD ? 16 : 8, D = EPI == FEW_SILU ? 16 : EPI == FEW_SLAB ? 12 : 8;
+  const dim3 grid(a.N / (EPI == FEW_SILU || EPI == FEW_ROPE ? 32 : 16));
+  constexpr int NW = EPI == FEW_ADD || EPI == FEW_ROPE ? 16 : 8, D = EPI == FEW_SILU ? 16 : EPI == FEW_SLAB ? 12 : 8;
   if (a.M * (a.K * 2 + FEW_PAD) <= 33 * 1024) few_rows_kernel<EPI, NORM, 33 * 1024, NW, D><<<grid, NW * 64, 0, st>>>(a);
   else if constexpr (!NORM) few_rows_kernel<EPI, NORM, 116 * 1024, NW, D><<<grid, NW * 64, 0, st>>>(a);
   return (int)hipGetLastError();
@@ -195,18 +244,31 @@ int launch_few(const FewRows& a, hipStream_t st) {
 
 }  // namespace
 
-// y = [norm of] X [M, K] x W [N, K]^T, W as tile_weight's copy.  form 0: f32 [M, N]; 1: added to the bf16 rows of y in place;
-// 2: W is the interleave16 gate|up weight, y bf16 [M, N / 2] = SiLU(gate) * up.  norm == null: no norm.
+// y = [norm of] X [M, K] x W [N, K]^T, W as tile_weight's copy.  form 0: norm, f32 [M, N]; 1: added to the bf16 rows of y in place;
+// 2: norm, W is the interleave16 gate|up weight, y bf16 [M, N / 2] = SiLU(gate) * up.
 // Contract (checked): 1 <= M <= 4, N % 16 == 0 (form 2: 32), K % 512 == 0, M * (2 K + 64) <= 116 KiB; with a norm
 // K <= 4096; ldx % 8 == 0, ldy % 4 == 0.
 PENNY_API int penny_few_rows(const void* X, int ldx, const void* norm, float eps, const void* Wt, int K, int N, void* y, int ldy,
                              int M, int form, hipStream_t stream) {
   if (M <= 0) return 0;
   if (M > FEW_ROWS || N <= 0 || K <= 0 || N % (form == FEW_SILU ? 32 : 16) || K % 512 || ldx % 8 || ldy % 4 || form < 0 || form > 2 ||
-      (long)M * (2L * K + FEW_PAD) > 116 * 1024 || (norm && K > 4096))
+      (long)M * (2L * K + FEW_PAD) > 116 * 1024 || (form == FEW_ADD ? norm != nullptr : !norm || K > 4096))
     return (int)hipErrorInvalidValue;
   const FewRows a{(const bf16*)X, (const bf16*)norm, (const char*)Wt, y, ldx, ldy, M, N, K, eps};
-  if (form == FEW_SLAB) return norm ? launch_few<FEW_SLAB, true>(a, stream) : launch_few<FEW_SLAB, false>(a, stream);
-  if (form == FEW_ADD) return norm ? (int)hipErrorInvalidValue : launch_few<FEW_ADD, false>(a, stream);
-  return norm ? launch_few<FEW_SILU, true>(a, stream) : launch_few<FEW_SILU, false>(a, stream);
+  return form == FEW_SLAB ? launch_few<FEW_SLAB, true>(a, stream) : form == FEW_ADD ? launch_few<FEW_ADD, false>(a, stream) : launch_few<FEW_SILU, true>(a, stream);
+}
+
+// QKV [norm of] X [M, K] x W^T of heads of 128 with the rotation and the paged cache's write behind it (rope_kv.hip): q [M, Hq, 128] bf16,
+// k and v of slots >= 0 into the caches.  W: tile_weight's copy of [(Hq + 2 Hkv) * 128, K].  Contract (checked): 1 <= M <= 4, K % 512 == 0,
+// M * (2 K + 64) <= 33 KiB, ldx % 8 == 0, a norm and K <= 4096.
+PENNY_API int penny_few_qkv_rope(const void* X, int ldx, const void* norm, float eps, const void* Wt, int K, const int* positions,
+                                 const float* cos_sin, const int* slots, void* q, void* kc, void* vc, int M, int Hq, int Hkv,
+                                 hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (M > FEW_ROWS || !norm || K <= 0 || K % 512 || K > 4096 || ldx % 8 || Hq < 1 || Hkv < 1 || !positions || !cos_sin || !slots)
+    return (int)hipErrorInvalidValue;
+  FewRows a{(const bf16*)X, (const bf16*)norm, (const char*)Wt, q, ldx, 0, M, (Hq + 2 * Hkv) * 128, K, eps};
+  a.positions = positions, a.cos_sin = cos_sin, a.slots = slots;
+  a.kc = (bf16*)kc, a.vc = (bf16*)vc, a.Hq = Hq, a.Hkv = Hkv;
+  return launch_few<FEW_ROPE, true>(a, stream);
 }

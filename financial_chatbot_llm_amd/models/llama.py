@@ -37,7 +37,7 @@ def _dual_stream(device) -> "torch.cuda.Stream":
     if key not in _DUAL_STREAMS:
         _DUAL_STREAMS[key] = torch.cuda.Stream(device=device)
     return _DUAL_STREAMS[key]
-from ..ops.gemm import (few_ok, few_rows, interleave16, linear, linear_tiled, prefill_qkv_rope, qkv_rope_fused, tile_weight,
+from ..ops.gemm import (few_ok, few_qkv_rope, few_rows, interleave16, linear, linear_tiled, prefill_qkv_rope, qkv_rope_fused, tile_weight,
                         tiled_only, uses_tiled_weight)
 from ..parallel.layers import shard_cols, shard_rows, shard_sections, vocab_range
 from .common import AttentionMetadata, KVCache, random_tensor
@@ -290,17 +290,21 @@ class DecoderModel:
 
     def takes_few(self, T: int) -> bool:
         """Does a step of ``T`` rows take :meth:`forward_few`?  The layers' projections are alike: the first one's decide."""
-        return T <= 4 and self.tp_size == 1 and type(self).mlp is DecoderModel.mlp and all(
+        return T <= 4 and self.tp_size == 1 and type(self).mlp is DecoderModel.mlp and \
+            type(self).attention is DecoderModel.attention and all(
             few_ok(T, self.wt.get("layers.0." + n), norm) for n, norm in (("qkv", True), ("o", False), ("gate_up", True), ("down", False)))
 
     def forward_few(self, ids: torch.Tensor, positions: torch.Tensor, meta: AttentionMetadata, kv: KVCache) -> torch.Tensor:
-        """One to four rows: each projection takes its norm, its SiLU or its residual add into its own launch."""
+        """One to four rows: each projection takes its norm, its rotation and cache write, its SiLU or its residual add into its own launch."""
         eps, x = self.cfg.norm_eps, self.embed(ids)
         for i in range(self.cfg.num_layers):
             p = f"layers.{i}."
             kc, vc = kv.k(i), kv.v(i)
-            qkv = few_rows(x, self.wt[p + "qkv"], "slab", self.w[p + "in_norm"], eps)
-            q = ops.rope_kv_write(qkv, positions, self.cos_sin, meta.slots, kc, vc, self.hq, self.hkv, self.D)
+            if self.D == 128:
+                q = few_qkv_rope(x, self.wt[p + "qkv"], self.w[p + "in_norm"], eps, positions, self.cos_sin, meta.slots, kc, vc, self.hq, self.hkv)
+            else:
+                qkv = few_rows(x, self.wt[p + "qkv"], "slab", self.w[p + "in_norm"], eps)
+                q = ops.rope_kv_write(qkv, positions, self.cos_sin, meta.slots, kc, vc, self.hq, self.hkv, self.D)
             attn = self.attend(q, meta, kc, vc, self.scale)
             few_rows(attn.view(-1, self.hq * self.D), self.wt[p + "o"], "add", residual=x)
             a = few_rows(x, self.wt[p + "gate_up"], "silu", self.w[p + "post_norm"], eps)

@@ -288,9 +288,9 @@ def few_ok(M: int, wt: Optional[torch.Tensor], norm: bool) -> bool:
 
 def few_rows(x: torch.Tensor, wt: torch.Tensor, form: str, norm: Optional[torch.Tensor] = None, eps: float = 0.0,
              residual: Optional[torch.Tensor] = None) -> Union[torch.Tensor, "Slabs"]:
-    """One to four rows through a ``tile_weight`` copy in one launch (``penny_few_rows``), RMS-normed with ``norm`` first where it is
-    given.  "slab": f32 sums as one slab; "add": added to ``residual`` in place; "silu": ``wt`` is the interleave16 gate|up weight and the
-    result SiLU(gate) * up."""
+    """One to four rows through a ``tile_weight`` copy in one launch (``penny_few_rows``).  "slab": RMS-normed with ``norm`` first, f32 sums
+    as one slab; "add": added to ``residual`` in place; "silu": normed, ``wt`` the interleave16 gate|up weight and the result
+    SiLU(gate) * up."""
     M, K = x.shape
     N_ = wt.shape[0] * 16
     if form == "slab":
@@ -302,6 +302,16 @@ def few_rows(x: torch.Tensor, wt: torch.Tensor, form: str, norm: Optional[torch.
     N.call("penny_few_rows", N.ptr(x), x.stride(0), N.ptr(norm), float(eps), N.ptr(wt), K, N_, N.ptr(y), y.stride(-2), M, FEW_FORMS[form],
            N.stream())
     return Slabs(y) if form == "slab" else y
+
+
+def few_qkv_rope(x: torch.Tensor, wt: torch.Tensor, norm: torch.Tensor, eps: float, positions: torch.Tensor, cos_sin: torch.Tensor,
+                 slots: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, Hq: int, Hkv: int) -> torch.Tensor:
+    """``few_rows`` of a QKV projection with ``ops.rope_kv_write`` behind it, heads of 128: the rotated q [M, Hq, 128]."""
+    M, K = x.shape
+    q = torch.empty((M, Hq, 128), dtype=x.dtype, device=x.device)
+    N.call("penny_few_qkv_rope", N.ptr(x), x.stride(0), N.ptr(norm), float(eps), N.ptr(wt), K, N.ptr(positions), N.ptr(cos_sin), N.ptr(slots),
+           N.ptr(q), N.ptr(k_cache), N.ptr(v_cache), M, Hq, Hkv, N.stream())
+    return q
 
 
 # "tiled": the decode kernels stream a fragment-tiled copy of each measured projection (made once

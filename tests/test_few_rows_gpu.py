@@ -9,9 +9,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("M", [1, 2, 3, 4])
-@pytest.mark.parametrize("form,N_,K,norm", [("slab", 48, 512, True), ("slab", 96, 4096, True), ("slab", 32, 1536, False), ("add", 16, 512, False),
+@pytest.mark.parametrize("form,N_,K,norm", [("slab", 48, 512, True), ("slab", 96, 4096, True), ("slab", 32, 1536, True), ("add", 16, 512, False),
                                             ("add", 80, 4096, False), ("add", 48, 14336, False), ("silu", 32, 512, True),
-                                            ("silu", 96, 2560, True), ("silu", 64, 4096, True), ("silu", 64, 6144, False)])
+                                            ("silu", 96, 2560, True), ("silu", 64, 4096, True)])
 def test_against_float64(M, form, N_, K, norm):
     gen = torch.Generator().manual_seed(M + N_ + K)
     rnd = lambda *s: torch.randn(s, generator=gen).to(torch.bfloat16).cuda()          # noqa: E731
@@ -39,12 +39,32 @@ def test_against_float64(M, form, N_, K, norm):
         assert y.shape == (M, N_ // 2) and ((y.double() - ref).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("M,Hq,Hkv,K", [(1, 32, 8, 4096), (2, 3, 1, 512), (3, 8, 2, 1024), (4, 4, 4, 4096)])
+def test_qkv_rope(M, Hq, Hkv, K):
+    """The rotating, cache-writing form against the two launches that it stands for: a skipped slot, both ends of a page."""
+    from financial_chatbot_llm_amd import ops
+    gen = torch.Generator().manual_seed(M + K)
+    x, w = (torch.randn(s, generator=gen).to(torch.bfloat16).cuda() for s in ((M, K), ((Hq + 2 * Hkv) * 128, K)))
+    wt, nw, cs = G.tile_weight(w * K ** -0.5), torch.ones(K, device="cuda").bfloat16(), torch.randn((300, 128), generator=gen).cuda()
+    pos = torch.tensor([0, 299, 64, 17][:M], dtype=torch.int32, device="cuda")
+    slots = torch.tensor([64, 191, -1, 0][:M], dtype=torch.int32, device="cuda")
+    caches = [torch.full((3, Hkv, 64 * 128), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(4)]
+    q = G.few_qkv_rope(x, wt, nw, 1e-5, pos, cs, slots, caches[0], caches[1], Hq, Hkv)
+    want = ops.rope_kv_write(G.few_rows(x, wt, "slab", nw, 1e-5), pos, cs, slots, caches[2], caches[3], Hq, Hkv, 128)
+    for a, b in ((q, want), (caches[0], caches[2]), (caches[1], caches[3])):
+        # the f32 sums of K differ in their order: another rounding to eight bits before the rotation and after it, of values up to the largest
+        assert a.shape == b.shape and (a.float() - b.float()).abs().max() <= 4 * 2.0 ** -8 * b.float().abs().max()
+        assert ((a == 7.0) == (b == 7.0)).float().mean() > 0.999            # the same places are written
+
+
 def test_refused():
     x, wt = torch.zeros((2, 4096), device="cuda", dtype=torch.bfloat16), G.tile_weight(torch.zeros((64, 4096), device="cuda", dtype=torch.bfloat16))
     assert G.few_ok(4, wt, True) and not G.few_ok(5, wt, True) and not G.few_ok(1, None, False)
     assert not G.few_ok(1, torch.empty((4, 256, 64, 8), device="cuda", dtype=torch.bfloat16), True)       # a norm over 8192 columns
     with pytest.raises(RuntimeError):
-        G.few_rows(torch.zeros((5, 4096), device="cuda", dtype=torch.bfloat16), wt, "slab")
+        G.few_rows(torch.zeros((5, 4096), device="cuda", dtype=torch.bfloat16), wt, "slab", norm=x[0])
+    with pytest.raises(RuntimeError):
+        G.few_rows(x, wt, "slab")
     with pytest.raises(RuntimeError):
         G.few_rows(x, wt, "add", norm=x[0], residual=torch.zeros((2, 64), device="cuda", dtype=torch.bfloat16))
 
