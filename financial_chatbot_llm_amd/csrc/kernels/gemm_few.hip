@@ -17,6 +17,7 @@
 namespace {
 
 constexpr int FEW_ROWS = 4;              // tokens at most
+constexpr int FEW_CHUNKS = 7168;         // 16-byte chunks of the rows at most: 4 x 14336, 3 x 18944, 2 x 28672, 1 x 57344 values in 112 KiB
 constexpr int FEW_PAD = 64;              // bytes behind a token's row in LDS: four tokens at one k meet different banks
 
 enum { FEW_SLAB = 0, FEW_ADD = 1, FEW_SILU = 2, FEW_ROPE = 3 };
@@ -38,9 +39,10 @@ struct FewRows {
   int Hq, Hkv;
 };
 
-// NORM: K <= 4096.  XB: bytes of LDS for the rows; NW waves; DEPTH pieces of W in flight per wave.
-template <int EPI, bool NORM, int XB, int NW, int DEPTH>
+// NORM: K <= 4096.  CHUNKS: the rows' 16-byte chunks, M * K / 8 at most; NW waves; DEPTH pieces of W in flight per wave.
+template <int EPI, bool NORM, int CHUNKS, int NW, int DEPTH>
 __global__ void __launch_bounds__(NW * 64) few_rows_kernel(FewRows a) {
+  constexpr int XB = CHUNKS * 16 + FEW_ROWS * FEW_PAD;
   constexpr int GROUPS = EPI == FEW_SILU || EPI == FEW_ROPE ? 2 : 1, KW = NW / GROUPS, THREADS = NW * 64;
   __shared__ __attribute__((aligned(16))) char xs[XB];
   __shared__ f32x4 part[NW][64];
@@ -51,11 +53,12 @@ __global__ void __launch_bounds__(NW * 64) few_rows_kernel(FewRows a) {
   const int group = EPI == FEW_ROPE ? (blockIdx.x >> 2) * 8 + (blockIdx.x & 3) + 4 * (w / KW) : blockIdx.x * GROUPS + w / KW;
   const int part_k = w % KW;
   const int p0 = pieces * part_k / KW, p1 = pieces * (part_k + 1) / KW;
-  PENNY_DASSERT(a.M >= 1 && a.M <= FEW_ROWS && a.M * pitch <= XB && group * 16 < a.N);
+  PENNY_DASSERT(a.M >= 1 && a.M <= FEW_ROWS && a.M * (a.K / 8) <= CHUNKS && group * 16 < a.N);
 
   // every load is issued without a branch, so that none waits for another: indices behind the end read the last chunk again
   constexpr int NC = !NORM ? 0 : THREADS < 512 ? 512 / THREADS : 1;   // NORM: chunks of a token per thread
-  constexpr int XR = NORM ? FEW_ROWS * NC : (XB > 64 * 1024 ? 7168 : 2048) / THREADS;
+  static_assert(CHUNKS % THREADS == 0, "every chunk has a thread");
+  constexpr int XR = NORM ? FEW_ROWS * NC : CHUNKS / THREADS;
   const int kc = a.K / 8, all = a.M * kc, tid = threadIdx.x;
   uint4 xv[XR], nv[NORM ? NC : 1];
   auto row_of = [&](int i) { return (i >= kc) + (i >= 2 * kc) + (i >= 3 * kc); };
@@ -237,8 +240,8 @@ template <int EPI, bool NORM>
 int launch_few(const FewRows& a, hipStream_t st) {
   const dim3 grid(a.N / (EPI == FEW_SILU || EPI == FEW_ROPE ? 32 : 16));
   constexpr int NW = EPI == FEW_ADD || EPI == FEW_ROPE ? 16 : 8, D = EPI == FEW_SILU ? 16 : EPI == FEW_SLAB ? 12 : 8;
-  if (a.M * (a.K * 2 + FEW_PAD) <= 33 * 1024) few_rows_kernel<EPI, NORM, 33 * 1024, NW, D><<<grid, NW * 64, 0, st>>>(a);
-  else if constexpr (!NORM) few_rows_kernel<EPI, NORM, 116 * 1024, NW, D><<<grid, NW * 64, 0, st>>>(a);
+  if (a.M * (a.K / 8) <= 2048) few_rows_kernel<EPI, NORM, 2048, NW, D><<<grid, NW * 64, 0, st>>>(a);
+  else if constexpr (!NORM) few_rows_kernel<EPI, NORM, FEW_CHUNKS, NW, D><<<grid, NW * 64, 0, st>>>(a);
   return (int)hipGetLastError();
 }
 
@@ -246,13 +249,13 @@ int launch_few(const FewRows& a, hipStream_t st) {
 
 // y = [norm of] X [M, K] x W [N, K]^T, W as tile_weight's copy.  form 0: norm, f32 [M, N]; 1: added to the bf16 rows of y in place;
 // 2: norm, W is the interleave16 gate|up weight, y bf16 [M, N / 2] = SiLU(gate) * up.
-// Contract (checked): 1 <= M <= 4, N % 16 == 0 (form 2: 32), K % 512 == 0, M * (2 K + 64) <= 116 KiB; with a norm
+// Contract (checked): 1 <= M <= 4, N % 16 == 0 (form 2: 32), K % 512 == 0, M * K <= 8 * FEW_CHUNKS; with a norm
 // K <= 4096; ldx % 8 == 0, ldy % 4 == 0.
 PENNY_API int penny_few_rows(const void* X, int ldx, const void* norm, float eps, const void* Wt, int K, int N, void* y, int ldy,
                              int M, int form, hipStream_t stream) {
   if (M <= 0) return 0;
   if (M > FEW_ROWS || N <= 0 || K <= 0 || N % (form == FEW_SILU ? 32 : 16) || K % 512 || ldx % 8 || ldy % 4 || form < 0 || form > 2 ||
-      (long)M * (2L * K + FEW_PAD) > 116 * 1024 || (form == FEW_ADD ? norm != nullptr : !norm || K > 4096))
+      (long)M * K > 8 * FEW_CHUNKS || (form == FEW_ADD ? norm != nullptr : !norm || K > 4096))
     return (int)hipErrorInvalidValue;
   const FewRows a{(const bf16*)X, (const bf16*)norm, (const char*)Wt, y, ldx, ldy, M, N, K, eps};
   return form == FEW_SLAB ? launch_few<FEW_SLAB, true>(a, stream) : form == FEW_ADD ? launch_few<FEW_ADD, false>(a, stream) : launch_few<FEW_SILU, true>(a, stream);
@@ -260,7 +263,7 @@ PENNY_API int penny_few_rows(const void* X, int ldx, const void* norm, float eps
 
 // QKV [norm of] X [M, K] x W^T of heads of 128 with the rotation and the paged cache's write behind it (rope_kv.hip): q [M, Hq, 128] bf16,
 // k and v of slots >= 0 into the caches.  W: tile_weight's copy of [(Hq + 2 Hkv) * 128, K].  Contract (checked): 1 <= M <= 4, K % 512 == 0,
-// M * (2 K + 64) <= 33 KiB, ldx % 8 == 0, a norm and K <= 4096.
+// ldx % 8 == 0, a norm and K <= 4096.
 PENNY_API int penny_few_qkv_rope(const void* X, int ldx, const void* norm, float eps, const void* Wt, int K, const int* positions,
                                  const float* cos_sin, const int* slots, void* q, void* kc, void* vc, int M, int Hq, int Hkv,
                                  hipStream_t stream) {

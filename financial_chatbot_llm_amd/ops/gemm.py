@@ -283,7 +283,7 @@ def few_ok(M: int, wt: Optional[torch.Tensor], norm: bool) -> bool:
     if wt is None or wt.dtype != torch.bfloat16 or not N.use_native(wt) or "0" in (os.environ.get("PENNY_SPLITK", "1"), os.environ.get("PENNY_GATEUP", "1")):
         return False
     K = wt.shape[1] * 32
-    return 1 <= M <= 4 and wt.shape[0] % 2 == 0 and K % 512 == 0 and M * (2 * K + 64) <= 116 * 1024 and (not norm or K <= 4096)
+    return 1 <= M <= 4 and wt.shape[0] % 2 == 0 and K % 512 == 0 and M * K <= 57344 and (not norm or K <= 4096)
 
 
 def few_rows(x: torch.Tensor, wt: torch.Tensor, form: str, norm: Optional[torch.Tensor] = None, eps: float = 0.0,

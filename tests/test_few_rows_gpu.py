@@ -98,3 +98,21 @@ def test_decoder_step(T, monkeypatch):
     for a, b in zip(*outs):
         # both round the same values to eight bits in a different order of f32 sums: at most a unit per layer of the largest
         assert (a - b).abs().max() <= 4 * 2.0 ** -8 * b.abs().max()
+
+
+# The most rows of x that a block holds (7168 chunks of 16 bytes), and one step of K beyond
+@pytest.mark.parametrize("M,K", [(1, 57344), (2, 28672), (3, 18944), (4, 14336)])
+def test_widest_rows(M, K):
+    gen = torch.Generator().manual_seed(K)
+    rnd = lambda *s: torch.randn(s, generator=gen).to(torch.bfloat16).cuda()          # noqa: E731
+    x, w = rnd(M, K + 512), rnd(32, K + 512) * K ** -0.5
+    res = torch.zeros((M, 32), dtype=torch.bfloat16, device="cuda")
+    wide = G.tile_weight(w)
+    assert not G.few_ok(M, wide, False)
+    with pytest.raises(RuntimeError):
+        G.few_rows(x, wide, "add", residual=res)
+    x, w = x[:, :K], w[:, :K].contiguous()
+    wt = G.tile_weight(w)
+    assert G.few_ok(M, wt, False)
+    y, want = G.few_rows(x, wt, "add", residual=res), x.double() @ w.double().t()
+    assert ((y.double() - want).abs() <= 2.0 ** -18 * K ** 0.5 + want.abs() * 2.0 ** -8).all()
