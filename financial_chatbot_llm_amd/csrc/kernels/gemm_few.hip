@@ -250,12 +250,13 @@ int launch_few(const FewRows& a, hipStream_t st) {
 // y = [norm of] X [M, K] x W [N, K]^T, W as tile_weight's copy.  form 0: norm, f32 [M, N]; 1: added to the bf16 rows of y in place;
 // 2: norm, W is the interleave16 gate|up weight, y bf16 [M, N / 2] = SiLU(gate) * up.
 // Contract (checked): 1 <= M <= 4, N % 16 == 0 (form 2: 32), K % 512 == 0, M * K <= 8 * FEW_CHUNKS; with a norm
-// K <= 4096; ldx % 8 == 0, ldy % 4 == 0.
+// K <= 4096; ldx % 8 == 0, ldy % 4 == 0; x, norm, W and f32 y in whole 16 bytes, bf16 y in 8.
 PENNY_API int penny_few_rows(const void* X, int ldx, const void* norm, float eps, const void* Wt, int K, int N, void* y, int ldy,
                              int M, int form, hipStream_t stream) {
   if (M <= 0) return 0;
   if (M > FEW_ROWS || N <= 0 || K <= 0 || N % (form == FEW_SILU ? 32 : 16) || K % 512 || ldx % 8 || ldy % 4 || form < 0 || form > 2 ||
-      (long)M * K > 8 * FEW_CHUNKS || (form == FEW_ADD ? norm != nullptr : !norm || K > 4096))
+      (long)M * K > 8 * FEW_CHUNKS || (form == FEW_ADD ? norm != nullptr : !norm || K > 4096) ||
+      ((size_t)X | (size_t)norm | (size_t)Wt) % 16 || !X || !Wt || !y || (size_t)y % (form == FEW_SLAB ? 16 : 8))
     return (int)hipErrorInvalidValue;
   const FewRows a{(const bf16*)X, (const bf16*)norm, (const char*)Wt, y, ldx, ldy, M, N, K, eps};
   return form == FEW_SLAB ? launch_few<FEW_SLAB, true>(a, stream) : form == FEW_ADD ? launch_few<FEW_ADD, false>(a, stream) : launch_few<FEW_SILU, true>(a, stream);
@@ -263,12 +264,13 @@ PENNY_API int penny_few_rows(const void* X, int ldx, const void* norm, float eps
 
 // QKV [norm of] X [M, K] x W^T of heads of 128 with the rotation and the paged cache's write behind it (rope_kv.hip): q [M, Hq, 128] bf16,
 // k and v of slots >= 0 into the caches.  W: tile_weight's copy of [(Hq + 2 Hkv) * 128, K].  Contract (checked): 1 <= M <= 4, K % 512 == 0,
-// ldx % 8 == 0, a norm and K <= 4096.
+// ldx % 8 == 0, a norm and K <= 4096; x, norm, W and the caches in whole 16 bytes.
 PENNY_API int penny_few_qkv_rope(const void* X, int ldx, const void* norm, float eps, const void* Wt, int K, const int* positions,
                                  const float* cos_sin, const int* slots, void* q, void* kc, void* vc, int M, int Hq, int Hkv,
                                  hipStream_t stream) {
   if (M <= 0) return 0;
-  if (M > FEW_ROWS || !norm || K <= 0 || K % 512 || K > 4096 || ldx % 8 || Hq < 1 || Hkv < 1 || !positions || !cos_sin || !slots)
+  if (M > FEW_ROWS || !norm || K <= 0 || K % 512 || K > 4096 || ldx % 8 || Hq < 1 || Hkv < 1 || !positions || !cos_sin || !slots ||
+      !X || !Wt || !q || !kc || !vc || ((size_t)X | (size_t)norm | (size_t)Wt | (size_t)q | (size_t)kc | (size_t)vc) % 16)
     return (int)hipErrorInvalidValue;
   FewRows a{(const bf16*)X, (const bf16*)norm, (const char*)Wt, q, ldx, 0, M, (Hq + 2 * Hkv) * 128, K, eps};
   a.positions = positions, a.cos_sin = cos_sin, a.slots = slots;

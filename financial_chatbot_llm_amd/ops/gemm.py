@@ -286,11 +286,25 @@ def few_ok(M: int, wt: Optional[torch.Tensor], norm: bool) -> bool:
     return 1 <= M <= 4 and wt.shape[0] % 2 == 0 and K % 512 == 0 and M * K <= 57344 and (not norm or K <= 4096)
 
 
+def _few_operands(x: torch.Tensor, wt: torch.Tensor, norm: Optional[torch.Tensor]) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
+    """``x`` and ``norm`` as the few-row kernels read them: rows of the copy's K in bf16, in whole 16 bytes (cloned where they are not)."""
+    K = wt.shape[1] * 32
+    bf = torch.bfloat16
+    if x.dtype != bf or wt.dtype != bf or x.shape[1] != K or not wt.is_contiguous():
+        raise ValueError(f"bf16 rows of {K} values and their tile_weight copy are needed, got {x.dtype} {tuple(x.shape)} and {wt.dtype}")
+    if norm is not None and (norm.dtype != bf or norm.shape != (K,) or not norm.is_contiguous()):
+        raise ValueError(f"the norm's weight is {K} bf16 values, got {norm.dtype} {tuple(norm.shape)}")
+    if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16:
+        x = x.clone(memory_format=torch.contiguous_format)
+    return x, norm.clone() if norm is not None and norm.data_ptr() % 16 else norm
+
+
 def few_rows(x: torch.Tensor, wt: torch.Tensor, form: str, norm: Optional[torch.Tensor] = None, eps: float = 0.0,
              residual: Optional[torch.Tensor] = None) -> Union[torch.Tensor, "Slabs"]:
     """One to four rows through a ``tile_weight`` copy in one launch (``penny_few_rows``).  "slab": RMS-normed with ``norm`` first, f32 sums
     as one slab; "add": added to ``residual`` in place; "silu": normed, ``wt`` the interleave16 gate|up weight and the result
     SiLU(gate) * up."""
+    x, norm = _few_operands(x, wt, norm)
     M, K = x.shape
     N_ = wt.shape[0] * 16
     if form == "slab":
@@ -299,6 +313,8 @@ def few_rows(x: torch.Tensor, wt: torch.Tensor, form: str, norm: Optional[torch.
         y = torch.empty((M, N_ // 2), dtype=x.dtype, device=x.device)
     else:
         y = residual
+        if y is None or y.dtype != x.dtype or y.shape != (M, N_) or y.stride(1) != 1:
+            raise ValueError(f"the residual is bf16 [{M}, {N_}] in rows")
     N.call("penny_few_rows", N.ptr(x), x.stride(0), N.ptr(norm), float(eps), N.ptr(wt), K, N_, N.ptr(y), y.stride(-2), M, FEW_FORMS[form],
            N.stream())
     return Slabs(y) if form == "slab" else y
@@ -307,7 +323,14 @@ def few_rows(x: torch.Tensor, wt: torch.Tensor, form: str, norm: Optional[torch.
 def few_qkv_rope(x: torch.Tensor, wt: torch.Tensor, norm: torch.Tensor, eps: float, positions: torch.Tensor, cos_sin: torch.Tensor,
                  slots: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, Hq: int, Hkv: int) -> torch.Tensor:
     """``few_rows`` of a QKV projection with ``ops.rope_kv_write`` behind it, heads of 128: the rotated q [M, Hq, 128]."""
+    x, norm = _few_operands(x, wt, norm)
     M, K = x.shape
+    if wt.shape[0] != (Hq + 2 * Hkv) * 8 or k_cache.dtype != x.dtype or v_cache.dtype != x.dtype or not (
+            k_cache.is_contiguous() and v_cache.is_contiguous()):
+        raise ValueError(f"{Hq} + 2 * {Hkv} heads of 128 and bf16 caches are needed")
+    if cos_sin.dtype != torch.float32 or cos_sin.shape[-1] != 128 or not cos_sin.is_contiguous() or any(
+            t.dtype != torch.int32 or t.shape[0] < M or not t.is_contiguous() for t in (positions, slots)):
+        raise ValueError("positions and slots are int32, a value per row; the table f32 rows of 128")
     q = torch.empty((M, Hq, 128), dtype=x.dtype, device=x.device)
     N.call("penny_few_qkv_rope", N.ptr(x), x.stride(0), N.ptr(norm), float(eps), N.ptr(wt), K, N.ptr(positions), N.ptr(cos_sin), N.ptr(slots),
            N.ptr(q), N.ptr(k_cache), N.ptr(v_cache), M, Hq, Hkv, N.stream())

@@ -116,3 +116,29 @@ def test_widest_rows(M, K):
     assert G.few_ok(M, wt, False)
     y, want = G.few_rows(x, wt, "add", residual=res), x.double() @ w.double().t()
     assert ((y.double() - want).abs() <= 2.0 ** -18 * K ** 0.5 + want.abs() * 2.0 ** -8).all()
+
+
+def test_operands():
+    """Rows and a norm off 16 bytes give the same as aligned ones; what does not fit the weight is refused before any launch."""
+    gen = torch.Generator().manual_seed(5)
+    rnd = lambda *s: torch.randn(s, generator=gen).to(torch.bfloat16).cuda()          # noqa: E731
+    K, Hq, Hkv = 512, 2, 1
+    wt, x, nw, res = G.tile_weight(rnd(512, K)), rnd(3, K + 9), rnd(K + 3), rnd(3, 512)
+    for xo in (x[:, 3:K + 3], x[:, 8:K + 8], rnd(K, 3).t()):
+        assert torch.equal(G.few_rows(xo, wt, "slab", nw[3:]).P, G.few_rows(xo.contiguous().clone(), wt, "slab", nw[3:].clone()).P)
+    xo, nw = x[:, :K].contiguous(), nw[:K].contiguous()
+    for bad in (lambda: G.few_rows(x[:, :K - 32], wt, "slab", nw), lambda: G.few_rows(rnd(3, 2 * K), wt, "add", residual=res),
+                lambda: G.few_rows(xo.float(), wt, "slab", nw), lambda: G.few_rows(xo, wt.float(), "slab", nw),
+                lambda: G.few_rows(xo, wt, "silu", nw.float()), lambda: G.few_rows(xo, wt, "silu", nw[:-8]),
+                lambda: G.few_rows(xo, wt, "add"), lambda: G.few_rows(xo, wt, "add", residual=res.float()),
+                lambda: G.few_rows(xo, wt, "add", residual=res[:2]), lambda: G.few_rows(xo, wt, "add", residual=rnd(512, 3).t())):
+        with pytest.raises(ValueError):
+            bad()
+    with pytest.raises(RuntimeError):                        # added in place: it cannot be cloned
+        G.few_rows(xo, wt, "add", residual=rnd(3 * 516 + 1)[1:].view(3, 516)[:, :512])
+    pos, cs, cache = torch.zeros(3, dtype=torch.int32, device="cuda"), torch.zeros((4, 128), device="cuda"), rnd(1, 1, 64 * 128)
+    good = dict(x=xo, wt=wt, norm=nw, eps=1e-5, positions=pos, cos_sin=cs, slots=pos, k_cache=cache, v_cache=cache.clone(), Hq=Hq, Hkv=Hkv)
+    assert G.few_qkv_rope(**good).shape == (3, Hq, 128)
+    for k, v in dict(x=rnd(3, K - 32), norm=nw.float(), positions=pos.long(), slots=pos[:2], cos_sin=cs.half(), k_cache=cache.float(), Hq=3).items():
+        with pytest.raises(ValueError):
+            G.few_qkv_rope(**dict(good, **{k: v}))
