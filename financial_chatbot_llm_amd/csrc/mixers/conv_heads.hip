@@ -24,13 +24,13 @@ __global__ void __launch_bounds__(CH_WAVES * 64)
 conv_heads_kernel(const T* __restrict__ in, long si, const float* __restrict__ w, int K, float* state,
                   const float* __restrict__ qw, const float* __restrict__ kw, float eps, float tcoef, int tevery,
                   const int* __restrict__ cu, const int* __restrict__ slot, const int* __restrict__ pos,
-                  const int* __restrict__ slots, T* __restrict__ cache, T* __restrict__ qout, int S, int H, int G, int D, int P) {
+                  const int* __restrict__ slots, T* __restrict__ cache, T* __restrict__ qout, int S, int per, int H, int G, int D, int P) {
   static_assert(TT >= KM - 1, "tiles behind the first must not reach the slot's history");
   typedef T vt __attribute__((ext_vector_type(VE)));
   constexpr int NV = NC * VE;
   int s, t0;
   const int unit = blockIdx.y * CH_WAVES + (threadIdx.x >> 6);
-  if (unit >= H + 2 * G || !mx_tile_place(cu, S, TT, blockIdx.x, s, t0)) return;     // wave-uniform, no block barrier below
+  if (unit >= H + 2 * G || !mx_tile_place<1>(cu, S, per, TT, blockIdx.x, s, t0)) return;     // wave-uniform, no block barrier below
   const int r0 = cu[s], n = cu[s + 1] - r0;
   const int lane = threadIdx.x & 63;
   const bool isq = unit < H, isv = unit >= H + G;
@@ -166,10 +166,10 @@ MX_API int mx_conv_heads(const void* in, long si, int dt, const float* w, int K,
   const int units = H + 2 * G;
 #define CH_LAUNCH(VE, NC, KM, TT)                                                                                     \
   do {                                                                                                                \
-    dim3 grid(mx_tile_count(S, rows, max_len, TT), (units + CH_WAVES - 1) / CH_WAVES);                                \
+    dim3 grid(mx_tile_count(S, rows, max_len, TT, 6), (units + CH_WAVES - 1) / CH_WAVES);                             \
     MX_DISPATCH(dt, TY, conv_heads_kernel<TY, VE, NC, KM, TT><<<grid, CH_WAVES * 64, 0, st>>>(                        \
         (const TY*)in, si, w, K, state, qw, kw, eps, tcoef, tevery, cu, slot, pos, slots, (TY*)cache, (TY*)qout,       \
-        mx_tile_segments(S, max_len), H, G, D, P));                                                                   \
+        S, mx_tile_per(S, rows, max_len, TT, 6), H, G, D, P));                                                         \
   } while (0)
 #define CH_TAPS(VE, NC)                     \
   do {                                      \

@@ -507,8 +507,8 @@ MX_API int mx_latent_attend(const void* q_lat, const void* q_rot, const void* ca
     if (ws == nullptr || nsplit < 1) nsplit = 1;
     const int HB = H < 64 ? H : 64, QT = max_len == 1 ? 1 : 64 / HB;
     RowsArgs a{q_lat, q_rot, (long)H * R, cache, D, 0, 0, 0, cu, pos, bt, btw, gate, sgate, 0, window, 0, 0,
-               nullptr, 0.f, sink, scale, out, H, 1, QT, HB, mx_tile_segments(S, max_len), nsplit, ws};
-    const dim3 grid((unsigned)(mx_tile_count(S, rows, max_len, QT) * nsplit), (H + HB - 1) / HB);
+               nullptr, 0.f, sink, scale, out, H, 1, QT, HB, S, mx_tile_per(S, rows, max_len, QT, 4), nsplit, ws};
+    const dim3 grid((unsigned)(mx_tile_count(S, rows, max_len, QT, 4) * nsplit), (H + HB - 1) / HB);
     if (dt == 1) {
       if (Dr == 32) rows_attend_kernel<float, 256, 32, 256, true, 1, 4, 32, false, false><<<grid, 256, 0, st>>>(a);
       else rows_attend_kernel<float, 256, 0, 256, true, 1, 4, 32, false, false><<<grid, 256, 0, st>>>(a);

@@ -123,40 +123,73 @@ __device__ __forceinline__ int mx_drop_nonfinite(mx_f32x4& x, int g) {
   return min(first, __shfl_xor(first, 32, 64));
 }
 
-// Blocks numbered over the tiles of `tile` rows that the segments have, one after the other (rows / tile + S of them at most):
-// block id's segment and its first row there, false behind the last.  A grid of the longest segment's tiles for every segment is
-// mostly empty blocks in a step of prompts and single rows, and its live ones meet on few CUs (prompts of 540, 300 and 327 rows
-// beside 21 single rows: an attention's 34 x 4 x 24 blocks, 376 of them live, did 31 us of work per CU in 65 us).  By a scan of the
-// row counts, 64 segments at a time; S = 0: one block per segment (each of one row at most).
-__device__ __forceinline__ bool mx_tile_place(const int* __restrict__ cu, int S, int tile, int id, int& s, int& t0) {
+// Blocks numbered over the tiles of `tile` rows that the segments have: block id's segment and its first row there, or false.
+// per > 0: every segment has that many blocks, the longest segment's tiles.  In a step of prompts and single rows most of those
+// would be empty and the live ones meet on few CUs (prompts of 540, 300 and 327 rows beside 21 single rows: an attention's 34 x
+// 4 x 24 blocks, 376 of them live, did 31 us of work per CU in 65 us), so with per = 0 the tiles are numbered one segment after the
+// other (rows / tile + S of them at most) and found by a scan of the row counts, 64 lanes with NL segments each at a time.
+template <int NL>
+__device__ __forceinline__ bool mx_tile_scan(const int* __restrict__ cu, int S, int tile, int id, int& s, int& t0) {
   const int lane = threadIdx.x & 63;
-  if (S <= 1) {
-    s = S == 0 ? id : 0;
-    t0 = S == 0 ? 0 : id * tile;
-    return t0 < cu[s + 1] - cu[s];
-  }
-  for (int base = 0; base < S; base += 64) {
-    const int i = base + lane, n = i < S ? cu[i + 1] - cu[i] : 0, tiles = (n + tile - 1) / tile;
-    int upto = tiles;
+  for (int base = 0; base < S; base += 64 * NL) {
+    int c[NL + 1], tiles[NL], sum = 0;
+#pragma unroll
+    for (int k = 0; k <= NL; ++k) c[k] = cu[min(base + NL * lane + k, S)];
+#pragma unroll
+    for (int k = 0; k < NL; ++k) sum += tiles[k] = (c[k + 1] - c[k] + tile - 1) / tile;
+    int upto = sum;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const int x = __shfl_up(upto, o, 64);
       if (lane >= o) upto += x;
     }
     const unsigned long long past = __ballot(upto > id);
-    if (past != 0) {
-      const int at = __ffsll(past) - 1;
-      s = base + at;
-      t0 = (id - __builtin_amdgcn_readlane(upto - tiles, at)) * tile;
-      return true;
+    if (past == 0) {
+      id -= __builtin_amdgcn_readlane(upto, 63);
+      continue;
     }
-    id -= __builtin_amdgcn_readlane(upto, 63);
+    const int at = __ffsll(past) - 1, first = base + NL * at;
+    id -= __builtin_amdgcn_readlane(upto - sum, at);
+    s = first;
+#pragma unroll
+    for (int k = 0; k < NL - 1; ++k) {                       // of the lane's segments the one that holds the block
+      const int t = __builtin_amdgcn_readlane(tiles[k], at);
+      if (s == first + k && id >= t) id -= t, ++s;
+    }
+    t0 = id * tile;
+    return true;
   }
   return false;
 }
-// its number of blocks, and the S to pass
-inline int mx_tile_count(int S, int rows, int max_len, int tile) { return max_len == 1 ? S : S + rows / tile; }
-inline int mx_tile_segments(int S, int max_len) { return max_len == 1 ? 0 : S; }
+// NL: 4 shortens the scan's chain (a window's 1,024 segments 130.7 -> 121.4 us, 4,096 of them 717 -> 538), 1 has the fewer instructions
+// (convolutions, whose blocks are many and short: 512 segments 30.7 us, with 4 32.5).
+template <int NL>
+__device__ __forceinline__ bool mx_tile_place(const int* __restrict__ cu, int S, int per, int tile, int id, int& s, int& t0) {
+  if (per > 0) {
+    s = per == 1 ? id : id / per;
+    if (s >= S) return false;
+    t0 = (id - s * per) * tile;
+    return t0 < cu[s + 1] - cu[s];
+  }
+  return S <= 64 ? mx_tile_scan<1>(cu, S, tile, id, s, t0) : mx_tile_scan<NL>(cu, S, tile, id, s, t0);
+}
+
+// Blocks per segment, or 0 for the scan: where the longest segment's tiles for every segment are no more blocks than the scan's
+// (segments alike, or as short as a tile), a block finds its place without it.  (32 segments of 5 rows, tiles of 16: an attention
+// in f32 28.6 -> 20.3 us.)  Beside very many segments empty blocks are cheaper than the scan, up to slack S / 1024 of the scan's blocks
+// in all, by the kernel's work per block: 1,023 single rows and a prompt of 64, convolution 52.5 us by the scan, 37.7 so; 2,047 and 130
+// 125 and 69, their window attention 270 and 206; 511 and 64 25.7 and 23.6; convolved heads of 1,023 and 20 42 and 30, 100 43 and 50.
+inline int mx_tile_per(int S, int rows, int max_len, int tile, int slack = 0) {
+  long per = ((long)max_len + tile - 1) / tile;
+  const long scan = (long)S + rows / tile;
+  if (per * S <= scan) return (int)per;
+  per |= 1;                              // single rows' only tiles, every 2nd or 4th or 8th block, would meet on a few XCDs
+  return per * S <= scan + scan * S * slack / 1024 ? (int)per : 0;
+}
+inline int mx_tile_count(int S, int rows, int max_len, int tile, int slack = 0) {
+  const int per = mx_tile_per(S, rows, max_len, tile, slack);
+  return per > 0 ? per * S : S + rows / tile;
+}
 
 constexpr int PAGE_ROWS = 64;            // tokens per cache page
 

@@ -44,7 +44,7 @@ struct RowsArgs {
   float scale;
   void* out;                     // [T, H * P]
   int H, G, QT, HB;
-  int S;                         // segments, or 0: a block per segment (each of one row at most)
+  int S, per;                    // segments, row tiles of each (0: numbered by a scan)
   int nsplit;
   float* ws;                     // nsplit > 1: [T, H, nsplit, P + 2]
 };
@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) rows_attend_kernel(R
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, c = lane & 15;
   const int split = blockIdx.x % a.nsplit;
   int s, t0;
-  if (!mx_tile_place(a.cu, a.S, a.QT, blockIdx.x / a.nsplit, s, t0)) return;      // (in a grid of dead blocks: 65 us for 45, in f32 227 for 159)
+  if (!mx_tile_place<4>(a.cu, a.S, a.per, a.QT, blockIdx.x / a.nsplit, s, t0)) return;
   const int r0 = a.cu[s], n = a.cu[s + 1] - r0;
   const int nq = min(a.QT, n - t0), kvh = blockIdx.y / hblocks, hg0 = (blockIdx.y % hblocks) * a.HB;
   const int nh = min(a.HB, rep - hg0), h0 = kvh * rep + hg0;

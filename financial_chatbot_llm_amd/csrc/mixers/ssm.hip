@@ -31,9 +31,9 @@ template <typename T>
 __global__ void conv_silu_kernel(const T* __restrict__ in, long si, const float* __restrict__ w,
                                  const float* __restrict__ bias, const float* __restrict__ in_bias, int act, float* state,
                                  const int* __restrict__ cu, const int* __restrict__ slot, const int* __restrict__ pos,
-                                 float* __restrict__ out, int S, int C, int K) {
+                                 float* __restrict__ out, int S, int per, int C, int K) {
   int s, t0;
-  if (!mx_tile_place(cu, S, CONV_TT, blockIdx.y, s, t0)) return;
+  if (!mx_tile_place<1>(cu, S, per, CONV_TT, blockIdx.y, s, t0)) return;
   const int sl = slot[s];
   if (sl < 0) return;
   const int r0 = cu[s], n = cu[s + 1] - r0;
@@ -86,9 +86,9 @@ __global__ void __launch_bounds__(256) conv4_kernel(const T* __restrict__ in, lo
                                                     const float* __restrict__ bias, const float* __restrict__ in_bias, int act,
                                                     float* state, const int* __restrict__ cu,
                                                     const int* __restrict__ slot, const int* __restrict__ pos,
-                                                    float* __restrict__ out, int S, int C) {
+                                                    float* __restrict__ out, int S, int per, int C) {
   int s, t0;
-  if (!mx_tile_place(cu, S, CONV_TT, blockIdx.y, s, t0)) return;
+  if (!mx_tile_place<1>(cu, S, per, CONV_TT, blockIdx.y, s, t0)) return;
   const int sl = slot[s];
   if (sl < 0) return;
   const int r0 = cu[s], n = cu[s + 1] - r0;
@@ -676,15 +676,16 @@ MX_API int mx_conv_act(const void* in, long si, int dt, const float* w, const fl
                        int rows, int C, int K, hipStream_t st) {
   if (S <= 0 || max_len <= 0) return 0;
   if (K < 1 || K > MAX_TAPS || act < 0 || act > 1) return (int)hipErrorInvalidValue;
+  const int per = mx_tile_per(S, rows, max_len, CONV_TT, 4);
   if (K == 4 && C % 4 == 0 && rows >= 8L * S && (long)rows * C >= 4500000 && mx_by_four(in, si, dt) &&
       ((size_t)w | (size_t)bias | (size_t)in_bias | (size_t)state | (size_t)out) % 16 == 0) {
-    const dim3 grid((C / 4 + 255) / 256, mx_tile_count(S, rows, max_len, CONV_TT));
+    const dim3 grid((C / 4 + 255) / 256, mx_tile_count(S, rows, max_len, CONV_TT, 4));
     MX_DISPATCH(dt, TT, conv4_kernel<TT><<<grid, 256, 0, st>>>((const TT*)in, si, w, bias, in_bias, act, state, cu, slot, pos,
-                                                               out, mx_tile_segments(S, max_len), C));
+                                                               out, S, per, C));
   } else {
-    const dim3 grid((C + 255) / 256, mx_tile_count(S, rows, max_len, CONV_TT));
+    const dim3 grid((C + 255) / 256, mx_tile_count(S, rows, max_len, CONV_TT, 4));
     MX_DISPATCH(dt, TT, conv_silu_kernel<TT><<<grid, 256, 0, st>>>((const TT*)in, si, w, bias, in_bias, act, state, cu,
-                                                                   slot, pos, out, mx_tile_segments(S, max_len), C, K));
+                                                                   slot, pos, out, S, per, C, K));
   }
   MX_RETURN_LAUNCH();
 }

@@ -728,8 +728,8 @@ MX_API int mx_window_attend(const void* q, long sq, const void* cache, const int
     const int HB = rep < 64 ? rep : 64, QT = max_len == 1 ? 1 : 64 / HB;
     if (ws == nullptr || nsplit < 1) nsplit = 1;
     RowsArgs a{q, nullptr, sq, cache, G * (D + P), D, G * D, P, cu, pos, bt, btw, gate, sgate, gate_elem, window, chunked, keep,
-               slope, cap, sink, scale, out, H, G, QT, HB, mx_tile_segments(S, max_len), nsplit, ws};
-    const dim3 grid((unsigned)(mx_tile_count(S, rows, max_len, QT) * nsplit), G * ((rep + HB - 1) / HB));
+               slope, cap, sink, scale, out, H, G, QT, HB, S, mx_tile_per(S, rows, max_len, QT, 4), nsplit, ws};
+    const dim3 grid((unsigned)(mx_tile_count(S, rows, max_len, QT, 4) * nsplit), G * ((rep + HB - 1) / HB));
     // 64 keys per tile while all blocks find a place at two per CU (64 KB of LDS each; 98 x 4 blocks: 43 us, 32 keys: 55),
     // 32 keys and four blocks per CU beyond (512 x 4 blocks: 127 us, 64 keys: 137)
     const bool few = ((long)S + (long)rows * HB / 64) * G * ((rep + HB - 1) / HB) * nsplit <= 512;

@@ -1,5 +1,5 @@
 """Kernels whose blocks are numbered over the segments' row tiles: more segments than a wave scans at once, empty ones, prompts
-beside single rows, one long segment; against the CPU forms, with the histories that the convolutions leave behind."""
+beside single rows, one long segment, segments alike; against the CPU forms, with the histories that the convolutions leave behind."""
 import pytest
 import torch
 
@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 def layout(name):
     g = torch.Generator().manual_seed(7)
     lens = {"many": torch.randint(0, 70, (150,), generator=g).tolist() + [1] * 40 + [33, 32, 31, 0],
-            "singles": [1] * 130, "one": [777], "two": [3, 1], "wave": [2] * 63 + [40] + [5]}[name]
+            "singles": [1] * 130, "one": [777], "two": [3, 1], "wave": [2] * 63 + [40] + [5],
+            "alike": [17] * 30 + [0, 20, 32], "scans": [1] * 254 + [40, 0, 0, 33, 1, 70] + [2, 0] * 130 + [65]}[name]
     ctx = [n + (i % 3) * 20 for i, n in enumerate(lens)]                     # every third starts at position 0
     cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
     pos = torch.cat([torch.arange(c - n, c) for n, c in zip(lens, ctx)]).int()
@@ -20,7 +21,7 @@ def layout(name):
     return lens, ctx, cu, pos, slot, g
 
 
-LAYOUTS = ["many", "singles", "one", "two", "wave"]
+LAYOUTS = ["many", "singles", "one", "two", "wave", "alike", "scans"]
 
 
 @pytest.mark.parametrize("name", LAYOUTS)
