@@ -26,14 +26,14 @@ constexpr int MAX_TAPS = 8;
 // rows than the taps reach back), and it replaces it by the segment's last K-1 inputs, upward, reading entry j + n before it
 // writes entry j.  (A launch of its own for that took 4.6 - 5.6 us behind each convolution.)
 
-// grid (ceil(C/256), tiles of the segments)
+// grid (ceil(C/256), tiles of the segments, in y and z: one of them holds 65535 of 32 rows)
 template <typename T>
 __global__ void conv_silu_kernel(const T* __restrict__ in, long si, const float* __restrict__ w,
                                  const float* __restrict__ bias, const float* __restrict__ in_bias, int act, float* state,
                                  const int* __restrict__ cu, const int* __restrict__ slot, const int* __restrict__ pos,
                                  float* __restrict__ out, int S, int per, int C, int K) {
   int s, t0;
-  if (!mx_tile_place<1>(cu, S, per, CONV_TT, blockIdx.y, s, t0)) return;
+  if (!mx_tile_place<1>(cu, S, per, CONV_TT, blockIdx.z * gridDim.y + blockIdx.y, s, t0)) return;
   const int sl = slot[s];
   if (sl < 0) return;
   const int r0 = cu[s], n = cu[s + 1] - r0;
@@ -88,7 +88,7 @@ __global__ void __launch_bounds__(256) conv4_kernel(const T* __restrict__ in, lo
                                                     const int* __restrict__ slot, const int* __restrict__ pos,
                                                     float* __restrict__ out, int S, int per, int C) {
   int s, t0;
-  if (!mx_tile_place<1>(cu, S, per, CONV_TT, blockIdx.y, s, t0)) return;
+  if (!mx_tile_place<1>(cu, S, per, CONV_TT, blockIdx.z * gridDim.y + blockIdx.y, s, t0)) return;
   const int sl = slot[s];
   if (sl < 0) return;
   const int r0 = cu[s], n = cu[s + 1] - r0;
@@ -676,14 +676,15 @@ MX_API int mx_conv_act(const void* in, long si, int dt, const float* w, const fl
                        int rows, int C, int K, hipStream_t st) {
   if (S <= 0 || max_len <= 0) return 0;
   if (K < 1 || K > MAX_TAPS || act < 0 || act > 1) return (int)hipErrorInvalidValue;
-  const int per = mx_tile_per(S, rows, max_len, CONV_TT, 4);
+  const int per = mx_tile_per(S, rows, max_len, CONV_TT, 4), tiles = mx_tile_count(S, rows, max_len, CONV_TT, 4);
+  const int tz = (tiles + 65534) / 65535, ty = (tiles + tz - 1) / tz;
   if (K == 4 && C % 4 == 0 && rows >= 8L * S && (long)rows * C >= 4500000 && mx_by_four(in, si, dt) &&
       ((size_t)w | (size_t)bias | (size_t)in_bias | (size_t)state | (size_t)out) % 16 == 0) {
-    const dim3 grid((C / 4 + 255) / 256, mx_tile_count(S, rows, max_len, CONV_TT, 4));
+    const dim3 grid((C / 4 + 255) / 256, ty, tz);
     MX_DISPATCH(dt, TT, conv4_kernel<TT><<<grid, 256, 0, st>>>((const TT*)in, si, w, bias, in_bias, act, state, cu, slot, pos,
                                                                out, S, per, C));
   } else {
-    const dim3 grid((C + 255) / 256, mx_tile_count(S, rows, max_len, CONV_TT, 4));
+    const dim3 grid((C + 255) / 256, ty, tz);
     MX_DISPATCH(dt, TT, conv_silu_kernel<TT><<<grid, 256, 0, st>>>((const TT*)in, si, w, bias, in_bias, act, state, cu,
                                                                    slot, pos, out, S, per, C, K));
   }

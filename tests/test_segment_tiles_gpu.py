@@ -43,6 +43,22 @@ def test_convolution_and_history(name, dt, K, C):
     assert torch.equal(got_st.cpu(), want_st)
 
 
+@pytest.mark.parametrize("K", [3, 4])                                       # 4: by four channels
+def test_convolution_of_many_rows(K):
+    """More row tiles than a launch holds in its second dimension (65535 of 32 rows), against torch's own convolution."""
+    T, C = 2_200_000, 4
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x, w, b = (torch.randn(s, generator=g, device="cuda") for s in ((T, C), (C, K), (C,)))
+    cu, pos = torch.tensor([0, 1_200_000, T]).int().cuda(), torch.cat([torch.arange(1_200_000), torch.arange(1_000_000)]).int().cuda()
+    st = torch.randn((2, K - 1, C), device="cuda")
+    y = mx.conv_silu(x, w, b, st, cu, torch.arange(2).int().cuda(), pos, 1_200_000)
+    for s, (a, e) in enumerate(((0, 1_200_000), (1_200_000, T))):
+        assert torch.equal(st[s], x[e - K + 1:e])
+        h = torch.nn.functional.pad(x[a:e].double(), (0, 0, K - 1, 0))
+        want = torch.nn.functional.silu(sum(h[k:k + e - a] * w[:, k].double() for k in range(K)) + b.double())
+        assert ((y[a:e] - want).abs() <= 2.0 ** -20 * (8 + want.abs())).all()
+
+
 @pytest.mark.parametrize("name", LAYOUTS)
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 def test_conv_heads(name, dt):
