@@ -13,11 +13,14 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// Most tokens of the rows form, by one and by four per block.  34 experts, us as library product and choice / rows by 1 / by 4 /
-// tile, width 2048, bf16: 1 token 14.8 / 7.9 / 10.5 / 13.1, 64: 17.8 / 8.4 / 10.8 / 17.9, 256: 19.0 / 9.1 / 11.0 / 18.0, 512: 19.8 /
-// 12.4 / 11.3 / 18.0, 1024: 22.2 / 21.0 / 12.4 / 18.3, 1280: 24.6 / 25.9 / 21.6 / 18.7, 5065: 38 / - / 52 / 30; width 1024 draws the
-// same lines.  f32 has no conversion to save: 64 tokens 13.7 / 8.4 / 10.7 / 20.0, 1024: 14.0 / 22.8 / 12.2 / 20.4, 2048: 16.3 / 39 / 22 /
-// 21, 5065: 23 / - / 54 / 34, so beyond 1024 rows the caller keeps the library's product.
+// Most tokens of the rows form, by one and by four per block.  Every block reads all of W, so the kernel's time grows with E x W and
+// the library's hardly does; the rule of the calls that come here is ops.mixers.router_takes.  Us, conversion, library product and
+// choice / here, W in the memory-side cache, 34 experts of width 2048, bf16: 1 token 15.7 / 10.2, 64: 17.4 / 10.6, 256: 18.3 / 10.9, 512: 19.7 /
+// 14.6, 1024: 22.5 / 14.9, 2048: 27.8 / 18.8, 5000: 36.6 / 30.2, 16000: 82.6 / 49.9 (in a decode step, W from HBM, 64 tokens take 13.9); f32 64: 13.5 / 10.3,
+// 1024: 15.4 / 12.5.  8 of 2048: 64: 17.6 / 4.5, 5000: 33.5 / 14.3; 32 of 8192: 64: 34.5 / 16.1, 5000: 84 / 79; 48 of 4096: 64: 19.6 / 16.2, 1024:
+// 29.5 / 23.3, 5000: 51 / 60; f32 64: 17.0 / 15.6, 1024: 17.6 / 19.3; 48 of 8192 64: 25 / 27.  64 of 2048: 64: 17.4 / 15.5, 512 (by four, whose sums no
+// longer fit the registers): 19.5 / 33.4, 2048: 30.9 / 27.6, 5000: 41 / 46; f32 64: 14.8 / 15.9; of 1024: 64: 16.9 / 11.6, 5000: 32.8 / 30.8; f32 64: 12.3 /
+// 12.0; of 4096: 64: 19.8 / 22.2.
 constexpr int ROWS_1 = 256, ROWS_4 = 1024;
 
 enum { ROUTE_SOFTMAX = 0, ROUTE_SIGMOID = 1, ROUTE_SOFTMAX_TOP = 2 };
@@ -182,8 +185,9 @@ __global__ void __launch_bounds__(512, 4) router_tile_kernel(Router a) {
 
 template <typename T, int NF> void router_launch(const Router& a, hipStream_t st) {
   if (a.T <= ROWS_1) router_rows_kernel<T, 4 * NF, 1><<<a.T, 1024, 0, st>>>(a);
-  else if (a.T <= ROWS_4) router_rows_kernel<T, 4 * NF, 4><<<(a.T + 3) / 4, 1024, 0, st>>>(a);
-  else if constexpr (sizeof(T) == 2) router_tile_kernel<T, NF><<<(a.T + 15) / 16, 512, 0, st>>>(a);
+  else if (a.T <= ROWS_4) {
+    if constexpr (NF <= 3) router_rows_kernel<T, 4 * NF, 4><<<(a.T + 3) / 4, 1024, 0, st>>>(a);
+  } else if constexpr (sizeof(T) == 2) router_tile_kernel<T, NF><<<(a.T + 15) / 16, 512, 0, st>>>(a);
 }
 
 }  // namespace
@@ -191,13 +195,15 @@ template <typename T, int NF> void router_launch(const Router& a, hipStream_t st
 // h [T, W] of type dt (row stride ldh), w f32 [E, W], zbias f32 [E] or null: logits z = w h + zbias.  score: 0 softmax over all
 // entries, 1 sigmoid, 2 softmax over the chosen logits.  biased != 0: the largest score + bias (f32 [E] or null) are chosen,
 // weighted by the score itself; else the largest logits.  renorm != 0: weights divided by their sum (+ 1e-20); times wscale.
-// outw, outi [T, top].  E <= 64, W % 32 == 0, 16-byte rows.  The tile form is for bf16: f32 takes at most ROWS_4 rows.
+// outw, outi [T, top].  E <= 64, W % 32 == 0, 16-byte rows.  The tile form is for bf16: f32 takes at most ROWS_4 rows.  More than 48
+// entries take no rows between ROWS_1 and ROWS_4.
 MX_API int mx_router(const void* h, long ldh, int dt, const float* w, const float* zbias, const float* bias, int biased,
                      int score, int renorm, float wscale, int E, int top, int W, float* outw, int* outi, int T,
                      hipStream_t st) {
   if (T <= 0) return 0;
   if (E < 1 || E > 64 || top < 1 || top > E || W < 32 || W % 32 || ldh * (dt == 1 ? 4 : 2) % 16 ||
-      ((size_t)h | (size_t)w) % 16 || score < 0 || score > 2 || (biased && score == ROUTE_SOFTMAX_TOP) || (dt == 1 && T > ROWS_4))
+      ((size_t)h | (size_t)w) % 16 || score < 0 || score > 2 || (biased && score == ROUTE_SOFTMAX_TOP) || (dt == 1 && T > ROWS_4) ||
+      (E > 48 && T > ROWS_1 && T <= ROWS_4))
     return (int)hipErrorInvalidValue;
   const Router a{h, ldh, w, zbias, bias, biased, score, renorm, wscale, E, top, W, T, outw, outi};
   MX_DISPATCH(dt, TT, switch ((E + 15) / 16) {

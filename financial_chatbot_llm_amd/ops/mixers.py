@@ -266,14 +266,29 @@ def route_biased(z: torch.Tensor, bias: Optional[torch.Tensor], top: int, score:
     return w * scale, idx.to(torch.int32)
 
 
+def router_takes(T: int, E: int, W: int, f32: bool) -> bool:
+    """Is ``mx_router`` the faster way for ``T`` rows, ``E`` entries, ``W`` columns?  Its kernels work in sixteens of entries (figures beside
+    them): up to 32 entries always; up to 48 in matrices that it reads faster than the library's three launches start; beyond, by one row
+    per block or on the matrix cores and in yet narrower ones.  f32 has no conversion to save and no matrix form."""
+    if W % 32 or W > 8192 or E > 64 or (f32 and T > 1024):
+        return False
+    if E <= 32:
+        return True
+    if E <= 48:
+        return W <= 2048 or (W <= 4096 and T <= (256 if f32 else 1024))
+    if T <= 256:
+        return W <= (1024 if f32 else 2048)
+    return T > 1024 and (W <= 1024 or (W <= 2048 and T <= 4096))
+
+
 def _router(h: torch.Tensor, w: torch.Tensor, zbias, bias, biased: bool, top: int, score: str, renorm: bool, scale: float):
     """``mx_router`` where it serves the call (up to 64 entries, whole groups of 32 columns, 16-byte rows) and is the faster way
-    (f32: 1024 rows at most), else None."""
+    (:func:`router_takes`), else None."""
     T, W = h.shape
     E = w.shape[0]
     es = h.element_size()
-    if not N.use_native(h) or E > 64 or W % 32 or T == 0 or (h.dtype == torch.float32 and T > 1024) or h.dtype not in (torch.bfloat16, torch.float32) or not w.is_contiguous() or \
-            h.stride(1) != 1 or h.stride(0) * es % 16 or h.data_ptr() % 16 or w.data_ptr() % 16:
+    if not N.use_native(h) or T == 0 or h.dtype not in (torch.bfloat16, torch.float32) or not router_takes(T, E, W, h.dtype == torch.float32) or \
+            not w.is_contiguous() or h.stride(1) != 1 or h.stride(0) * es % 16 or h.data_ptr() % 16 or w.data_ptr() % 16:
         return None
     outw = torch.empty((T, top), dtype=torch.float32, device=h.device)
     outi = torch.empty((T, top), dtype=torch.int32, device=h.device)
