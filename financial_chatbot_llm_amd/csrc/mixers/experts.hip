@@ -660,7 +660,10 @@ int tile_rows(long pairs, int experts, int dt, const Product* p, bool whole) {
   // (below 512 rows an expert's panels are read by one or two blocks of 256, whose stages in flight do not cover a first touch of
   // memory: inside a model, 148 rows on average took 142 us with 256, 124 with 128, and 431 rows 254 and 246)
   if (whole && avg >= 512 && wide_time((double)pairs / experts, experts, 256, p) < fmin(t64, t128)) return 256;
-  return t64 < 0.95 * t128 ? 64 : 128;                              // 64 where it is clearly the shorter
+  // 64 where it is clearly the shorter, and while most experts' only tile is less than half of one of 128: uneven buckets then pay for
+  // the wider (plan and products, 200 and 300 tokens most of which go to an eighth of the experts: 64 of 512 x 1024, top 6, 128 rows 66 and 71 us,
+  // 64 rows 47 and 51; 32 of 1024 x 2048, top 4, 120 and 126, 94 and 97; evenly spread 43 - 45 and 42, 91 - 92 and 86)
+  return avg <= 56 || t64 < 0.95 * t128 ? 64 : 128;
 }
 
 template <typename T, bool GLU>
@@ -690,6 +693,13 @@ int expert_launch(const ExpertGemm& a, int mt, hipStream_t st) {
 }
 
 }  // namespace
+
+// Rows of a tile (16: the stream form) that mx_experts takes for `pairs` over E experts with these products
+MX_API int mx_experts_tile(int pairs, int E, int dt, int g1, int k1, int g2, int k2, int whole) {
+  if (pairs < 1 || E < 1) return 0;
+  const Product products[2] = {{g1, k1}, {g2, k2}};
+  return tile_rows(pairs, E, dt, products, whole != 0 && pairs > 1024 && E <= 512);
+}
 
 // h [T, >= W] (row stride ldh), idx int32 [T, top] (>= E: an identity expert, no row here); w1 / w2: pieces as above, k1 / k2
 // pieces per row group, g1 / g2 row groups per expert (gated units: g1 counts gate and up groups); unit: UNIT_*;

@@ -108,6 +108,7 @@ _MIXER_SIGS = {
     "mx_conv_heads": [P, c_long, c_int, P, c_int, P, P, P, c_float, c_float, c_int, P, P, P, P, P, P, c_int, c_int, c_int,
                       c_int, c_int, c_int, c_int, P],
     "mx_moe_combine": [P, c_long, P, P, P, P, c_long, P, c_long, c_int, c_int, c_int, P, c_int, c_int, P],
+    "mx_experts_tile": [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int],
     "mx_experts": [P, c_long, P, c_int, c_int, c_int, c_int, c_int, P, c_int, c_int, P, c_int, c_int, c_int, c_float, c_float,
                    P, P, c_long, P, P, c_int, P],
     "mx_conv_silu": [P, c_long, c_int, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, P],

@@ -120,6 +120,14 @@ def test_few_experts(dtype, T, W, F_, E, top, unit):
     check(dtype, T, W, F_, E, top, unit)
 
 
+def test_tile_rule():
+    """Few rows per expert on average keep tiles of 64 whatever the estimate says of even buckets."""
+    from financial_chatbot_llm_amd.ops import _native as N
+    tile = lambda T, top, E, W, F_: N.load_mixers().mx_experts_tile(T * top, E, 0, F_ // 8, W // 32, W // 16, F_ // 32, 1)     # noqa: E731
+    assert [tile(T, 6, 64, 1024, 512) for T in (100, 200, 300, 600, 1000)] == [16, 64, 64, 64, 128]
+    assert tile(300, 4, 32, 2048, 1024) == 64 and tile(1100, 4, 32, 2048, 1024) == 128 and tile(5065, 4, 32, 2048, 1024) == 256
+
+
 @pytest.mark.parametrize("E", [1, 3, 64, 65, 512, 513])
 @pytest.mark.parametrize("T", [256, 257, 1023, 1025, 2049, 4097, 8192, 8193])
 def test_expert_plan_is_the_stable_sort(E, T):
