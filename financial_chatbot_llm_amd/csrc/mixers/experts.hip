@@ -263,10 +263,12 @@ __device__ __forceinline__ const char* expert_row(const ExpertGemm& a, int r, in
   return static_cast<const char*>(a.x) + (a.top > 0 ? a.src[r] / a.top : r) * a.ldx * es;
 }
 
-// (tile, column block) of this block among `cols` column blocks, or false.  Every XCD takes an equal run of the full tiles, in
-// groups of four neighbouring ones -- mostly one expert's -- through all column blocks in turn, so that their W panels and token
-// rows meet in its L2, then one of the small tiles.  (Fixed groups dealt to the XCDs leave some of them idle: 16 tiles of 256 rows
-// by 16 column blocks ran on four.)
+// (tile, column block) of this block among `cols` column blocks, or false.  Groups of four neighbouring tiles -- mostly one expert's --
+// take all column blocks in turn on one XCD, so that their W panels and token rows meet in its L2, and go round the XCDs: a busy
+// expert's groups, which share their panels, and those of the small ones, which stream them, spread over all memory paths (64
+// experts of 512 x 1024, 700 tokens most of which go to 8: runs of neighbouring groups per XCD 75 us, dealt round 68).  What is left
+// behind whole rounds of groups is dealt by equal runs: 16 tiles of 256 rows by 16 column blocks would run on four XCDs.  Small
+// tiles come last, the same way.
 __device__ __forceinline__ bool expert_place(const ExpertGemm& a, int cols, int& t, int& nb) {
   const int4 head = a.tiles[-1];
   int id = blockIdx.x, first = 0, live = head.y;
@@ -276,10 +278,17 @@ __device__ __forceinline__ bool expert_place(const ExpertGemm& a, int cols, int&
     live = head.x - first;
     if (id >= live * cols) return false;
   }
-  const int nwg = live * cols, xcd = id & 7, q = nwg >> 3, r = nwg & 7;
-  id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (id >> 3);
-  const int grp = id / (4 * cols), in = id - grp * 4 * cols, gm = min(live - 4 * grp, 4);
-  t = first + 4 * grp + in % gm;
+  const int xcd = id & 7, k = id >> 3, rounds = live >> 5, dealt = rounds * 4 * cols;        // 32 tiles a round
+  if (k < dealt) {
+    const int grp = k / (4 * cols), in = k - grp * 4 * cols;
+    t = first + (grp * 8 + xcd) * 4 + (in & 3);
+    nb = in >> 2;
+    return true;
+  }
+  const int left = live - 32 * rounds, nwg = left * cols, q = nwg >> 3, r = nwg & 7;
+  id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + k - dealt;
+  const int grp = id / (4 * cols), in = id - grp * 4 * cols, gm = min(left - 4 * grp, 4);
+  t = first + 32 * rounds + 4 * grp + in % gm;
   nb = in / gm;
   return true;
 }

@@ -155,6 +155,8 @@ def test_expert_plan_is_the_stable_sort(E, T):
     (1700, 2048, 1088, 8, 3, "gelu_tanh", {"strided": True, "ident": 1}),      # a column block beyond the last group
     (4000, 768, 1024, 16, 4, "relu2", {"ident": 2}),
     (1700, 2056, 1024, 8, 3, "clamped", {}),             # rows in no whole K tile: 128 tokens
+    (300, 256, 136, 64, 6, "silu", {"skew": True}),      # tiles of 64: one and more whole rounds of groups over the XCDs and a rest
+    (700, 256, 136, 60, 6, "clamped", {}),
 ])
 def test_experts_of_many_rows(T, W, F_, E, top, unit, kw):
     check(torch.bfloat16, T, W, F_, E, top, unit, **kw)
