@@ -246,7 +246,10 @@ namespace {
 // 1: not split.  A query of 12 layers of 768 x 3072, us unsplit / in 2 / 3 / 4 / 6: 6 tokens 422 / 412 / 419 / 414 / 414, 18: 467 / 438 /
 // 437 / 441 / 451, 32: 505 / 472 / 466 / 459 / 466, 48: 599 / 536 / 521 / 511 / 523, 64: 634 / 565 / 550 / 545 / 556, 84: 680 / 611 / 623 / 621 /
 // 611, 109: 701 / 627 / 652 / 637 / 640, 179: 743 / 658 / 633 / 669 / 645.
+// As a call of its own the slices' sum is a launch more, so not where K is short: 1024 x 1024 7 rows unsplit 3.7, in 2 slices 5.6, 18: 4.4 / 6.0; 512 x
+// 2048 7: 5.0 / 5.8, 18: 6.6 / 6.3; 768 x 3072 7: 6.4 / 6.5, 18: 8.8 / 7.0.
 int few_slices(int M, int N, int K) {
+  if (K < (M <= 16 ? 3072 : 2048)) return 1;
   if (N != 256 && N != 512 && N != 768 && N != 1024) return 1;
   const long blocks = M <= 128 ? (long)(N / 16) * ((M + 63) / 64) : (long)((N + 31) / 32) * ((M + 63) / 64);
   const long s = 216 / blocks, most = K / 512;
@@ -262,9 +265,11 @@ int few_slices(int M, int N, int K) {
 // 20.2 / 9.0; 3072 x 768 with GELU 128 9.6 / 6.2, 768 24.5 / 15.4, 1024 27.8 / 19.0; 768 x 3072 48 8.8 / 10.0, 192 (in slices, which
 // the next norm adds) 8.8 / 10.4, 256 11 / 10.4, 768 35.1 / 15.6, 2048 38.4 / 27.5; 4096 x 1024 512 31.4 / 14.0; 1024 x 4096 128 20.5 / 12.7.  Widths that
 // the tile kernel does not take have the library behind them: 1152 x 384 256 4.5 / 4.2, 1024 8.0 / 6.9, 2048 9.5 / 10.2; 384 x 1536 64 - 192 4.9 /
-// 6.5: not there.
+// 6.5: not there.  Nor where K is as long as many rows (2048 x 8192 1000 rows 67.9 / 65.6, 1280 70.0 / 78.3, 2048 79.4 / 90.8), nor for few rows and
+// a short K, whose ring has nothing to fill (1152 x 384 33 rows 3.5 / 3.9).
 PENNY_API int penny_bias_rows_plan(int M, int N, int K) {
-  if (M <= 32 || N < 16 || N % 16 || K < 64 || K % 64 || M > (N % 256 == 0 ? 2048 : K <= 1024 ? 1024 : 0)) return 0;
+  if (M <= (K < 512 ? 40 : 32) || N < 16 || N % 16 || K < 64 || K % 64 || M > (N % 256 == 0 ? 2048 : K <= 1024 ? 1024 : 0) || (long)M * K > 1 << 23)
+    return 0;
   if (M <= 192 && few_slices(M, N, K) > 1) return 0;
   return penny_bias_rows_tile(M, N, K);
 }

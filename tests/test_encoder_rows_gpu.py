@@ -60,3 +60,18 @@ def test_walk_of_longer_batches(lens, monkeypatch):
     monkeypatch.setattr(m, "_small_batch", lambda *a: False)
     y, _ = m.forward(ids)
     assert torch.equal(x, y)
+
+
+def test_rule():
+    """Slices of K and the ring only where they are the faster way."""
+    from financial_chatbot_llm_amd.ops import _native as nat
+    lib = nat.load()
+    assert [lib.penny_encoder_slices(*a) > 1 for a in ((7, 1024, 1024), (18, 1024, 1024), (150, 1024, 1024), (16, 512, 2048), (17, 512, 2048),
+                                                       (16, 768, 3072), (18, 512, 1984))] == [False, False, False, False, True, True, False]
+    assert [lib.penny_bias_rows_plan(*a) > 0 for a in ((33, 1024, 1024), (190, 1024, 1024), (1024, 2048, 8192), (1025, 2048, 8192), (2048, 1024, 4096),
+                                                       (40, 1152, 384), (41, 1152, 384), (33, 1152, 512))] == [True, True, True, False, True, False, True, True]
+
+
+@pytest.mark.parametrize("M,N,K", [(7, 1024, 1024), (18, 1024, 1024), (33, 1024, 1024), (190, 1024, 1024), (16, 512, 2048), (17, 512, 2048), (40, 1152, 384)])
+def test_at_the_rule(M, N, K):
+    test_against_float64(M, N, K, False)
