@@ -560,6 +560,8 @@ class HeadLinear:
             K * w.element_size() % 64 == 0 and H <= 65535
         # the batched product's right operand lies as it reads it
         self.w = w.contiguous() if self.native else w.transpose(1, 2).contiguous()
+        if self.native and self.w.data_ptr() % 16:
+            self.w = self.w.clone()
 
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
         """x [T, H, K] (any strides) -> [T, H, N] contiguous."""

@@ -25,3 +25,9 @@ def test_against_float64(dt, T, H, N, K):
         # one rounding of the result to eight significant bits (half a unit: 2^-8 of it at most); sums of K f32 products
         e = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -20
         assert ((y.double().cpu() - want).abs() <= want.abs() * e + 2.0 ** -18 * K ** 0.5).all()
+
+
+def test_weights_off_16_bytes():
+    """A part of a flat buffer of weights, as a loader may hand it over."""
+    w, x = torch.randn(3 * 32 * 64 + 3, device="cuda")[3:].view(3, 32, 64), torch.randn((5, 3, 64), device="cuda")
+    assert ((mx.HeadLinear(w)(x).double() - (x.double()[:, :, None] * w.double()).sum(-1)).abs() <= 2.0 ** -18 * 64).all()
