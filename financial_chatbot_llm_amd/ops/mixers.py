@@ -551,25 +551,41 @@ def _sink_softmax(sc: torch.Tensor, sink: Optional[torch.Tensor]) -> torch.Tenso
 
 class HeadLinear:
     """y[t, h] = W[h] x[t, h]: a matrix per head, ``w`` [H, N, K].  On the GPU the rows of heads are read and written where they lie
-    (``mx_head_linear``); sizes that the kernel does not take (N in whole 16, rows of whole 64 bytes) and the CPU go through a
-    batched product."""
+    (``mx_head_linear``); sizes that the kernel does not take (N in whole 16, rows of whole 64 bytes), those that it would serve
+    slower (:meth:`_most_rows`) and the CPU go through a batched product."""
 
     def __init__(self, w: torch.Tensor):
-        H, self.N, K = w.shape
+        H, self.N, self.K = w.shape
+        self.H, self.dtype = H, w.dtype
         self.native = N.use_native(w) and w.dtype in (torch.bfloat16, torch.float32) and self.N % 16 == 0 and \
-            K * w.element_size() % 64 == 0 and H <= 65535
-        # the batched product's right operand lies as it reads it
-        self.w = w.contiguous() if self.native else w.transpose(1, 2).contiguous()
-        if self.native and self.w.data_ptr() % 16:
-            self.w = self.w.clone()
+            self.K * w.element_size() % 64 == 0 and H <= 65535
+        self.most = self._most_rows()
+        # the kernel's matrices, in whole 16 bytes, and the batched product's, whose right operand lies as it reads it: what calls need
+        self.w = self.wt = None
+        if self.most > 0:
+            self.w = w.contiguous()
+            if self.w.data_ptr() % 16:
+                self.w = self.w.clone()
+        if self.most < 1 << 40:
+            self.wt = w.transpose(1, 2).contiguous()
+
+    def _most_rows(self) -> int:
+        """Rows that the kernel serves faster.  Every wave reads its columns of W for itself, so the library's tiles win where a head's
+        matrix is large, or K is and the rows are many.  Us, batched product with its copies / here, heads x N x K: bf16 8 x 512 x 512 64
+        rows 9.7 / 23.4, 8192 91 / 177; 16 x 256 x 256 64: 12.1 / 7.8, 8192: 82 / 97; 32 x 128 x 256 2048: 30 / 27, 8192: 105 / 98, 16384: 206 /
+        223; 32 x 256 x 128 16384: 284 / 260; f32 16 x 96 x 256 2048: 28.5 / 27.0, 8192: 87 / 99; 32 x 128 x 256 512: 20.3 / 19.0, 2048: 56 / 60;
+        16 x 256 x 96 16384: 276 / 218."""
+        if not self.native or self.N * self.K > 32768:
+            return 0
+        return 1 << 40 if self.K <= self.N else (32768 if self.dtype == torch.float32 else 262144) // self.H
 
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
         """x [T, H, K] (any strides) -> [T, H, N] contiguous."""
         T, H, K = x.shape
-        if not self.native:
-            return torch.bmm(x.transpose(0, 1), self.w).transpose(0, 1).contiguous()
-        if x.dtype != self.w.dtype or (H, K) != (self.w.shape[0], self.w.shape[2]):
+        if self.native and (x.dtype != self.dtype or (H, K) != (self.H, self.K)):
             raise ValueError("one row of the matrices' width per head, of their type")
+        if T > self.most:
+            return torch.bmm(x.transpose(0, 1), self.wt).transpose(0, 1).contiguous()
         es = x.element_size()
         if x.stride(2) != 1 or x.stride(0) * es % 16 or x.stride(1) * es % 16 or x.data_ptr() % 16:
             x = x.clone(memory_format=torch.contiguous_format)
@@ -578,7 +594,7 @@ class HeadLinear:
         return y
 
     def num_bytes(self) -> int:
-        return self.w.numel() * self.w.element_size()
+        return sum(w.numel() * w.element_size() for w in (self.w, self.wt) if w is not None)
 
 
 @functools.lru_cache(maxsize=1024)          # the estimate takes 1 - 5 us

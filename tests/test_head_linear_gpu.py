@@ -31,3 +31,23 @@ def test_weights_off_16_bytes():
     """A part of a flat buffer of weights, as a loader may hand it over."""
     w, x = torch.randn(3 * 32 * 64 + 3, device="cuda")[3:].view(3, 32, 64), torch.randn((5, 3, 64), device="cuda")
     assert ((mx.HeadLinear(w)(x).double() - (x.double()[:, :, None] * w.double()).sum(-1)).abs() <= 2.0 ** -18 * 64).all()
+
+
+@pytest.mark.parametrize("dt,T,H,N,K,native", [
+    (torch.bfloat16, 8192, 32, 128, 256, True), (torch.bfloat16, 8193, 32, 128, 256, False), (torch.float32, 1024, 32, 128, 256, True),
+    (torch.float32, 1025, 32, 128, 256, False), (torch.float32, 1025, 32, 256, 128, True), (torch.bfloat16, 3, 2, 512, 96, False),
+    (torch.bfloat16, 3, 2, 256, 128, True), (torch.bfloat16, 3, 2, 256, 160, False)])
+def test_rule(dt, T, H, N, K, native, monkeypatch):
+    """Large matrices, and a long K beside many rows, keep the batched product."""
+    from financial_chatbot_llm_amd.ops import _native as nat
+    calls = []
+    mcall = nat.mcall
+    monkeypatch.setattr(nat, "mcall", lambda name, *a: (calls.append(name), mcall(name, *a))[1])
+    g = torch.Generator(device="cuda").manual_seed(T)
+    w = torch.randn((H, N, K), generator=g, device="cuda").mul_(K ** -0.5).to(dt)
+    x = torch.randn((T, H, K), generator=g, device="cuda").to(dt)
+    y = mx.HeadLinear(w)(x)
+    assert calls == (["mx_head_linear"] if native else [])
+    want = (x[:50].double()[:, :, None] * w.double()).sum(-1)
+    e = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -20
+    assert ((y[:50].double() - want).abs() <= want.abs() * e + 2.0 ** -18 * K ** 0.5).all()
