@@ -696,6 +696,18 @@ PENNY_API int penny_linear_rows_plan(int M, int N, int K, int f32) {
   return plan;
 }
 
+// The same for launches that a graph replays, where the host's share of a library call does not count: only what the device runs faster.
+// Up to 96 rows (f32: 32) that is all of the above.  Beyond, us in replayed graphs, library / here: bf16 7232 x 2048 160 rows 17.4 / 16.1, 256
+// 24.8 / 20.2; 4096 x 2048 192 21.5 / 12.4; 6464 x 1024 256 15.0 / 12.0; 2048 x 6144 (in slices) 192 22.6 / 17.7; but 2048 x 4096 unsplit 192 15.9 / 16.7, 12864
+// x 2048 128 19.5 / 21.2, 32000 x 1024 128 18.8 / 20.5.  f32 2048 x 1024 48 11.3 / 9.9, 1024 x 2048 64 11.3 / 10.6, 2048 x 32 256 3.9 / 3.1; but 1024 x 3072 48
+// 10.9 / 12.4, 3616 x 1024 48 12.1 / 12.6, 1024 x 1024 80 8.2 / 9.0, 256 8.8 / 11.2, 2048 x 1024 128 11.6 / 11.8.
+PENNY_API int penny_linear_rows_replay_plan(int M, int N, int K, int f32) {
+  const int plan = penny_linear_rows_plan(M, N, K, f32);
+  if (M <= (f32 ? 32 : 96)) return plan;
+  if (f32) return K <= 64 || (M <= 64 && (long)N * K <= 2048 * 1024) ? plan : 0;
+  return N <= 8192 && (K < 4096 || plan >> 16 > 1) ? plan : 0;
+}
+
 // Y [M, N] = X [M, K] x W [N, K]^T in bf16 or f32 (f32 != 0) for up to about two thousand rows, W row-major: slabs == null streams W once (S = 1), else
 // S slices of K leave f32 slabs [S, M, N] that a second launch adds.  One entry for both, so that a step that the host bounds
 // pays for one call.  nf, mt: a block's columns and rows in units of 16, one of kRowsTiles.  Contract (checked): N % 16 == 0 (the last

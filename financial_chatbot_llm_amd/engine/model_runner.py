@@ -24,6 +24,7 @@ from .. import ops
 from ..models.common import AttentionMetadata, KVCache
 from ..ops import attention as _attn
 from ..ops.attention import KV_BS, DecodeWorkspace, mark_shared_blocks, prefill_plan
+from ..ops.gemm import replayed
 from ..parallel import comm
 from ..utils.logging import get_logger
 from ..utils.profiling import marker
@@ -674,6 +675,10 @@ class ModelRunner:
         return self._dual
 
     def _run_static(self, B: int, filtered: bool = False) -> torch.Tensor:
+        with replayed():
+            return self._static_step(B, filtered)
+
+    def _static_step(self, B: int, filtered: bool) -> torch.Tensor:
         s = self._static
         self._gather_pending(s["ids"], s["src"][:B], 0)
         if self.dual_decode and B >= self.dual_min_batch:

@@ -19,7 +19,9 @@ with ``bench/kernels.py`` (profiles named next to each table).
 """
 from __future__ import annotations
 
+import contextlib
 import os
+import threading
 from typing import Dict, List, Optional, Tuple, Union
 
 import torch
@@ -251,16 +253,32 @@ def splitk_bf16(x: torch.Tensor, w: torch.Tensor, N_: int, nf: int, rowmajor: bo
     return y
 
 
+_REPLAYED = threading.local()
+
+
+@contextlib.contextmanager
+def replayed():
+    """Launches of this thread's block are for a graph, its warm-up included (the library's kernels have to be loaded before the
+    capture): ``project`` then chooses by the device's time alone, as no host time is paid on a replay."""
+    before = getattr(_REPLAYED, "on", False)
+    _REPLAYED.on = True
+    try:
+        yield
+    finally:
+        _REPLAYED.on = before
+
+
 def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """y = x @ w.T in bf16 or f32: the streaming kernels for up to about two thousand rows (``penny_linear_rows_plan``), the library's
-    product for the rest."""
+    """y = x @ w.T in bf16 or f32: the streaming kernels for up to about two thousand rows (``penny_linear_rows_plan``; inside
+    :func:`replayed` ``penny_linear_rows_replay_plan``), the library's product for the rest."""
     dt = x.dtype
     if dt == w.dtype and (dt == torch.bfloat16 or dt == torch.float32) and x.dim() == 2 and w.dim() == 2 and N.use_native(x):
         (M, K), N_, f32 = x.shape, w.shape[0], dt == torch.float32
         ldx, xp, wp = x.stride(0), x.data_ptr(), w.data_ptr()
         if M <= 2048 and K == w.shape[1] and (xp | wp) % 16 == 0 and ldx % (4 if f32 else 8) == 0 and ldx >= K and x.stride(1) == 1 and \
                 w.is_contiguous() and w.device == x.device and not (w.requires_grad or x.requires_grad):
-            plan = N.load().penny_linear_rows_plan(M, N_, K, f32)
+            rule = N.load().penny_linear_rows_replay_plan if M > 32 and getattr(_REPLAYED, "on", False) else N.load().penny_linear_rows_plan
+            plan = rule(M, N_, K, f32)
             if plan:
                 S = plan >> 16
                 y = torch.empty((M, N_), dtype=dt, device=x.device)

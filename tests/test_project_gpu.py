@@ -72,3 +72,52 @@ def test_other_calls_keep_the_library():
         G.project(xb, w)
     with pytest.raises(RuntimeError):
         G.project(xb[:, :64], wb)
+
+
+@pytest.mark.parametrize("dt,M,N_,K,eager,graph", [
+    (torch.bfloat16, 96, 32000, 1024, True, True), (torch.bfloat16, 128, 12864, 2048, True, False), (torch.bfloat16, 192, 2048, 4096, True, False),
+    (torch.bfloat16, 192, 2048, 6144, True, True), (torch.bfloat16, 256, 7232, 2048, True, True), (torch.float32, 32, 3616, 1024, True, True),
+    (torch.float32, 48, 3616, 1024, True, False), (torch.float32, 64, 2048, 1024, True, True), (torch.float32, 80, 1024, 1024, True, False),
+    (torch.float32, 256, 2048, 32, True, True)])
+def test_replayed(dt, M, N_, K, eager, graph, monkeypatch):
+    """A step that a graph replays takes only the products that the device runs faster; its warm-up takes the same, other threads do not."""
+    import threading
+    from financial_chatbot_llm_amd.ops import _native as N
+    calls = []
+    call = N.call
+    monkeypatch.setattr(N, "call", lambda name, *a: (calls.append(name), call(name, *a))[1])
+    g = torch.Generator(device="cuda").manual_seed(M)
+    w = (torch.randn((N_, K), generator=g, device="cuda") * K ** -0.5).to(dt)
+    x = torch.randn((M, K), generator=g, device="cuda").to(dt)
+    native = lambda f: (calls.clear(), f(), bool(calls))[2]                            # noqa: E731
+    assert native(lambda: G.project(x, w)) is eager
+    with G.replayed():
+        assert native(lambda: G.project(x, w)) is graph
+        other = []
+        t = threading.Thread(target=lambda: other.append(native(lambda: G.project(x, w))))
+        t.start()
+        t.join()
+        assert other == [eager]
+        torch.cuda.synchronize()
+        cg = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(cg):
+            y = G.project(x, w)
+        assert native(lambda: G.project(x, w)) is graph
+    assert native(lambda: G.project(x, w)) is eager
+    e = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -20
+    for i in range(3):
+        x.copy_(torch.randn((M, K), generator=g, device="cuda"))
+        cg.replay()
+        want = x.double() @ w.double().t()
+        assert ((y.double() - want).abs() <= want.abs() * e + 2.0 ** -18 * K ** 0.5).all()
+
+
+def test_the_runner_says_so(monkeypatch):
+    """The engine's graphs, and the passes that warm them up, are made inside ``replayed``."""
+    from financial_chatbot_llm_amd.engine.model_runner import ModelRunner
+    seen = []
+    monkeypatch.setattr(ModelRunner, "_static_step", lambda self, B, filtered: seen.append((B, filtered, getattr(G._REPLAYED, "on", False))))
+    r = ModelRunner.__new__(ModelRunner)
+    r._run_static(3)
+    r._run_static(4, filtered=True)
+    assert seen == [(3, False, True), (4, True, True)] and not getattr(G._REPLAYED, "on", False)
