@@ -236,7 +236,7 @@ PENNY_API int penny_encoder_attention(const void* qkv, long ld, const int* cu, i
 }
 
 // gemm_splitk.hip
-extern "C" int penny_bias_rows_tile(int M, int N, int K);
+extern "C" int penny_bias_rows_tile(int M, int N);
 extern "C" int penny_bias_rows(const void* X, int ldx, const void* W, int K, void* Y, int ldy, const void* bias, int M, int N, int gelu, int nf,
                                int mt, hipStream_t st);
 
@@ -271,7 +271,7 @@ PENNY_API int penny_bias_rows_plan(int M, int N, int K) {
   if (M <= (K < 512 ? 40 : 32) || N < 16 || N % 16 || K < 64 || K % 64 || M > (N % 256 == 0 ? 2048 : K <= 1024 ? 1024 : 0) || (long)M * K > 1 << 23)
     return 0;
   if (M <= 192 && few_slices(M, N, K) > 1) return 0;
-  return penny_bias_rows_tile(M, N, K);
+  return penny_bias_rows_tile(M, N);
 }
 
 namespace {
@@ -512,8 +512,8 @@ constexpr int PENNY_MISALIGNED = -1;
 
 // All layers of a small batch: x [T, H] bf16 is replaced by the last layer's output.  w: 12 pointers per layer -- qkv, its
 // bias, o, its bias, the first norm's weight and bias, fc1, its bias, fc2, its bias, the second norm's weight and bias, each
-// contiguous bf16.  ws: T * (6 H + F) bf16, then f32 slabs [penny_encoder_slices(T, H, F), T, H] where that is more than 1.  Shapes as penny_gemm_bias_small, penny_encoder_attention and penny_layernorm take
-// them; PENNY_MISALIGNED, and nothing launched, for a weight off their 16 bytes (asked here: 144 weights take 18 us in Python).
+// contiguous bf16.  ws: T * (6 H + F) bf16, then f32 slabs [penny_encoder_slices(T, H, F), T, H] where that is more than 1.  Shapes as
+// penny_gemm_bias_small, penny_encoder_attention and penny_layernorm take them; PENNY_MISALIGNED, and nothing launched, for a weight off their 16 bytes (asked here: 144 weights take 18 us in Python).
 // The launches of one layer take the host 8 x 2.5 us here and 8 x 7 from Python, where the kernels of a single query
 // (18 tokens, 12 layers of 768) run for 440 us in all: 815 -> 497 us for the query.
 PENNY_API int penny_encoder_layers(const void* const* w, int layers, void* x, void* ws, const int* cu, int texts, int max_len,

@@ -413,26 +413,28 @@ constexpr bool pair_fits() {
 }
 
 // one launch of splitk_gemm_kernel<NF, MT, WA, EPI, *, 150, MAXB, *> with the W layout / stage pairing
-// of wrow (runtime) mapped onto the template arguments
-template <int NF, int MT, int WA, int EPI, int MAXB, class... A>
+// of wrow (runtime) mapped onto the template arguments.  ROWS: row-major weights only (the entries whose last tile of columns may be
+// part-filled, which the tiled copy's form does not know).
+template <int NF, int MT, int WA, int EPI, int MAXB, bool ROWS = false, class... A>
 int launch_any(int wrow, bool pair_ok, dim3 grid, hipStream_t st, A... args) {
   const bool rm = wrow & 1;
+  if (ROWS && !rm) return (int)hipErrorInvalidValue;
   if constexpr (pair_fits<NF, MT, 150, MAXB>()) {
     if ((wrow & 2) && pair_ok) {
       if (rm) hipLaunchKernelGGL((splitk_gemm_kernel<NF, MT, WA, EPI, true, 150, MAXB, 2>), grid, dim3(256), 0, st, args...);
-      else hipLaunchKernelGGL((splitk_gemm_kernel<NF, MT, WA, EPI, false, 150, MAXB, 2>), grid, dim3(256), 0, st, args...);
+      else if constexpr (!ROWS) hipLaunchKernelGGL((splitk_gemm_kernel<NF, MT, WA, EPI, false, 150, MAXB, 2>), grid, dim3(256), 0, st, args...);
       return (int)hipGetLastError();
     }
   }
   if (rm) hipLaunchKernelGGL((splitk_gemm_kernel<NF, MT, WA, EPI, true, 150, MAXB>), grid, dim3(256), 0, st, args...);
-  else hipLaunchKernelGGL((splitk_gemm_kernel<NF, MT, WA, EPI, false, 150, MAXB>), grid, dim3(256), 0, st, args...);
+  else if constexpr (!ROWS) hipLaunchKernelGGL((splitk_gemm_kernel<NF, MT, WA, EPI, false, 150, MAXB>), grid, dim3(256), 0, st, args...);
   return (int)hipGetLastError();
 }
 
-template <int NF, int MT, int WA>
+template <int NF, int MT, int WA, bool ROWS = false>
 int launch(const void* X, int ldx, const void* Wt, int K, float* P, int M, int N, int S, int wrow, hipStream_t st) {
-  return launch_any<NF, MT, WA, SK_SLAB, 8>(wrow, (K / S) % 128 == 0, dim3(((N + 16 * NF - 1) / (16 * NF)) * S, (M + 16 * MT - 1) / (16 * MT)), st, (const bf16*)X,
-                                            ldx, (const bf16*)Wt, K, P, M, N, S, (bf16*)nullptr, 0, SkSample{});
+  return launch_any<NF, MT, WA, SK_SLAB, 8, ROWS>(wrow, (K / S) % 128 == 0, dim3(((N + 16 * NF - 1) / (16 * NF)) * S, (M + 16 * MT - 1) / (16 * MT)), st,
+                                                  (const bf16*)X, ldx, (const bf16*)Wt, K, P, M, N, S, (bf16*)nullptr, 0, SkSample{});
 }
 
 template <int NF, int MT, int WA>
@@ -467,11 +469,11 @@ int launch_silu(const void* X, int ldx, const void* Wt, int K, void* Y, int ldy,
                                                           ldy, SkSample{});
 }
 
-template <int NF, int MT, int WA>
+template <int NF, int MT, int WA, bool ROWS = false>
 int launch_bf16(const void* X, int ldx, const void* Wt, int K, void* Y, int ldy, int M, int N, int wrow,
                 hipStream_t st) {
-  return launch_any<NF, MT, WA, SK_BF16, 16>(wrow, K % 128 == 0, dim3((N + 16 * NF - 1) / (16 * NF), (M + 16 * MT - 1) / (16 * MT)), st, (const bf16*)X, ldx,
-                                             (const bf16*)Wt, K, (float*)nullptr, M, N, 1, (bf16*)Y, ldy, SkSample{});
+  return launch_any<NF, MT, WA, SK_BF16, 16, ROWS>(wrow, K % 128 == 0, dim3((N + 16 * NF - 1) / (16 * NF), (M + 16 * MT - 1) / (16 * MT)), st,
+                                                   (const bf16*)X, ldx, (const bf16*)Wt, K, (float*)nullptr, M, N, 1, (bf16*)Y, ldy, SkSample{});
 }
 
 // the streaming LM head: row-major W (wrow) or its fragment-tiled copy; ring budget 150 KiB (one
@@ -726,9 +728,9 @@ PENNY_API int penny_linear_rows(const void* X, int ldx, const void* W, int K, vo
       if constexpr (NF_ * MT_ <= 12) rc = launch_f32<NF_, MT_, WA_>(X, ldx, W, K, p, M, N, S, paired, st); \
       else return (int)hipErrorInvalidValue;                                                       \
     } else if (S > 1) {                                                                            \
-      rc = launch<NF_, MT_, WA_>(X, ldx, W, K, p, M, N, S, paired ? 3 : 1, st);                    \
+      rc = launch<NF_, MT_, WA_, true>(X, ldx, W, K, p, M, N, S, paired ? 3 : 1, st);              \
     } else {                                                                                       \
-      rc = launch_bf16<NF_, MT_, WA_>(X, ldx, W, K, Y, N, M, N, paired ? 3 : 1, st);               \
+      rc = launch_bf16<NF_, MT_, WA_, true>(X, ldx, W, K, Y, N, M, N, paired ? 3 : 1, st);         \
     }                                                                                              \
   } else
   LR_CASE(2, 2, 2)
@@ -754,7 +756,7 @@ PENNY_API int penny_linear_rows(const void* X, int ldx, const void* W, int K, vo
 }
 
 // The tile of penny_bias_rows for M rows: the fastest that runs all its blocks in one round; 0: none does
-extern "C" int penny_bias_rows_tile(int M, int N, int K) {
+extern "C" int penny_bias_rows_tile(int M, int N) {
   int tile = 0;
   float best = 1e9f;
   for (const RowsTile& t : kRowsTiles) {
@@ -774,7 +776,7 @@ extern "C" int penny_bias_rows(const void* X, int ldx, const void* W, int K, voi
   sa.gelu = gelu;
 #define BR_CASE(NF_, MT_, WA_)                                                                                          \
   if (nf == NF_ && mt == MT_)                                                                                           \
-    return launch_any<NF_, MT_, WA_, SK_BIAS, 16>(3, K % 128 == 0, dim3((N + 16 * NF_ - 1) / (16 * NF_), (M + 16 * MT_ - 1) / (16 * MT_)), \
+    return launch_any<NF_, MT_, WA_, SK_BIAS, 16, true>(3, K % 128 == 0, dim3((N + 16 * NF_ - 1) / (16 * NF_), (M + 16 * MT_ - 1) / (16 * MT_)), \
                                                   st, (const bf16*)X, ldx, (const bf16*)W, K, (float*)nullptr, M, N, 1, (bf16*)Y, ldy, sa);
   BR_CASE(2, 2, 2)
   BR_CASE(2, 4, 1)

@@ -497,7 +497,8 @@ GATEUP_SPLITK: Dict[Tuple[int, int], List[Tuple[int, int, int, int, bool]]] = {
     # hipBLASLt from 32 rows
     (57344, 8192): [(1, 1, 8, 2, True), (2, 16, 4, 2, True)],
     # Llama-3-8B at one row: S4 nf2 + reduce-SiLU with paired stages 44.4 us vs the fused kernel's 50.3
-    # (r5_decode_gemm_paired_stages_ab.jsonl)
+    # (r5_decode_gemm_paired_stages_ab.jsonl); steps of one to four rows go through few_rows instead, so this is for
+    # the layers called one by one (a context-parallel shard's last row)
     (28672, 4096): [(1, 1, 4, 2, False)],
 }
 
