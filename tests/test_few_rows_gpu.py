@@ -142,3 +142,42 @@ def test_operands():
     for k, v in dict(x=rnd(3, K - 32), norm=nw.float(), positions=pos.long(), slots=pos[:2], cos_sin=cs.half(), k_cache=cache.float(), Hq=3).items():
         with pytest.raises(ValueError):
             G.few_qkv_rope(**dict(good, **{k: v}))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("prompts,rows", [([(70, 3)], []), ([(0, 4)], []), ([(64, 1)], []), ([(127, 2)], [40]), ([(0, 1), (62, 2)], [130]), ([], [5, 64, 191])])
+def test_decoder_step_of_prompts(D, prompts, rows, monkeypatch):
+    """Heads that take the slab form and its rotation pass, and short prompts -- whole ones, tails behind a cached prefix and over a page's
+    end -- alone and beside decoding rows, through :meth:`forward_few` and through the general layers."""
+    from financial_chatbot_llm_amd.models.common import AttentionMetadata, KVCache
+    from financial_chatbot_llm_amd.models.configs import ModelConfig
+    from financial_chatbot_llm_amd.models.llama import LlamaModel
+    from financial_chatbot_llm_amd.ops.attention import DecodeWorkspace
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")                  # noqa: E731
+    cfg = ModelConfig(name="few", arch="llama", vocab_size=512, hidden_size=1024, intermediate_size=2048, num_layers=2, num_heads=1024 // D,
+                      num_kv_heads=256 // D, head_dim=D, max_position=512)
+    model = LlamaModel(cfg, device="cuda").init_random(4)
+    model.wt = {n: G.tile_weight(w) for n, w in model.w.items() if n.endswith((".qkv", ".o", ".down", ".gate_up"))}
+    segs = prompts + [(c, 1) for c in rows]
+    T, tp, n = sum(k for _, k in segs), sum(k for _, k in prompts), len(prompts)
+    assert model.takes_few(T)
+    pos = [a + j for a, k in segs for j in range(k)]
+    bt = torch.arange(4 * len(segs), dtype=torch.int32, device="cuda").view(len(segs), 4)
+    slots = i32([(4 * i + (a + j) // 64) * 64 + (a + j) % 64 for i, (a, k) in enumerate(segs) for j in range(k)])
+    meta = AttentionMetadata(slots=slots, num_prefill_tokens=tp, num_decode=len(rows), decode_ws=DecodeWorkspace.create(4, model.hq, D, 512, "cuda"))
+    if prompts:
+        meta.cu_q, meta.ctx_lens_p = i32([sum(k for _, k in prompts[:i]) for i in range(n + 1)]), i32([a + k for a, k in prompts])
+        meta.block_tables_p, meta.max_q_len = bt[:n].contiguous(), max(k for _, k in prompts)
+    if rows:
+        meta.ctx_lens_d, meta.block_tables_d = i32([c + 1 for c in rows]), bt[n:].contiguous()
+    outs = []
+    for few in (True, False):
+        kv = KVCache(cfg.num_layers, 4 * len(segs), model.hkv, D, device="cuda")
+        for i in range(cfg.num_layers):
+            for c in (kv.k(i), kv.v(i)):
+                c.copy_(torch.randn(c.shape, generator=torch.Generator().manual_seed(i)).to(c.dtype))
+        monkeypatch.setattr(LlamaModel, "takes_few", lambda self, t, few=few: few)
+        outs.append((model.forward(i32(range(3, 3 + T)), i32(pos), meta, kv).float(), kv.k(0).float(), kv.k(1).float(), kv.v(1).float()))
+    for a, b in zip(*outs):
+        # both round the same values to eight bits in a different order of f32 sums: at most a unit per layer of the largest
+        assert (a - b).abs().max() <= 4 * 2.0 ** -8 * b.abs().max()
