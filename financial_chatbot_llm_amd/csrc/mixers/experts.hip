@@ -2,7 +2,8 @@
 //     act[r] = unit(W1[e] x[token(r)])      W1 [N1, W] per expert (gated: gate and up rows in turns of 16)
 //     ys[r]  = W2[e] act[r]                 W2 [W, F] per expert
 // Three launches and no host read of the bucket sizes:
-//   plan    one block: a stable counting sort of the (token, choice) pairs by expert and the list of row tiles
+//   plan    a stable counting sort of the (token, choice) pairs by expert and the list of row tiles: one block, beyond 1024 pairs one
+//           per expert
 //   GEMM 1  gathers the tokens' rows while it stages them, applies the gated unit in its epilogue
 //   GEMM 2  sorted rows in and out; mx_moe_combine sums a token's rows
 // Weights are stored as the MFMA reads them: pieces of 1 KiB, [row group of 16][K step of 64 bytes][64 lanes][16 B],
@@ -631,8 +632,9 @@ __global__ void __launch_bounds__(256) expert_stream_kernel(ExpertGemm a) {
 //
 // Among the larger tiles the choice is by an estimate too: the rounds of blocks over the CUs (3, 2 and 1 blocks of 64, 128 and 256
 // rows on each) times a block's stages at 1.35 (1.15 where the CUs are not full), 1.38 and 1.85 us; an expert's last tile is half
-// full on average, and a small one of 256 rows takes half the time.  Us for tiles of 64 / 128 / 256, bf16, experts' rows spread by a factor of about 1.3 (5 for the
-// second figures): 32 experts of 1024 x 2048: 64 rows on average 102 / 100 / 95 (96 / 127 / 117), 128: 129 / 138 / 114 (132 / 139 / 142),
+// full on average, and a small one of 256 rows takes half the time.  Us for tiles of 64 / 128 / 256, bf16, experts' rows spread by a
+// factor of about 1.3 (5 for the second figures): 32 experts of 1024 x 2048: 64 rows on average 102 / 100 / 95 (96 / 127 / 117), 128:
+// 129 / 138 / 114 (132 / 139 / 142),
 // 192: 165 / 146 / 156 (168 / 142 / 147), 256: 202 / 192 / 176 (189 / 188 / 174), 431: 290 / 256 / 245 (271 / 250 / 214), 633: 397 / 360 /
 // 307 (371 / 325 / 298), 1024: 586 / 513 / 457 (570 / 505 / 447); of 512 x 1024: 128: 40 / 44 / 63, 256: 61 / 73 / 72, 431: 84 / 86 / 92,
 // 633: 112 / 120 / 134; 8 of 2048 x 4096: 128: 145 / 136 / 144, 192: 197 / 138 / 157, 256: 204 / 216 / 167, 1250: 745 / 625 / 492; 64 of 768 x

@@ -57,8 +57,9 @@ projection's rank).
 
 Every block declares the rows it needs from a fused in-projection (``in_weight``): a layer stacks
 its mixer's and its feed-forward's rows into ONE GEMM over ``h`` and hands each block its column
-slice.  Plain GEMMs on bf16 weights stream through the framework's kernels for a decode step's few rows and are library
-products for the rest (:func:`..ops.gemm.project`); everything else runs on the kernels behind :mod:`..ops.mixers`.
+slice.  Plain GEMMs stream through the framework's kernels where those are the faster way -- bf16 up to some two thousand rows, f32
+up to 256, products short enough for it -- and are library products for the rest (:func:`..ops.gemm.project`); everything else
+runs on the kernels behind :mod:`..ops.mixers`.
 """
 from __future__ import annotations
 

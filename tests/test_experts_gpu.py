@@ -131,7 +131,7 @@ def test_tile_rule():
 @pytest.mark.parametrize("E", [1, 3, 64, 65, 512, 513])
 @pytest.mark.parametrize("T", [256, 257, 1023, 1025, 2049, 4097, 8192, 8193])
 def test_expert_plan_is_the_stable_sort(E, T):
-    """One block (512 experts or 1024 pairs and fewer, 32768 and more) and a block per expert: every pair's place is that of the
+    """One block (more than 512 experts, or 1024 pairs and fewer) and a block per expert (beyond 32768 pairs in a loop): every pair's place is that of the
     stable sort by expert, identity experts behind; some experts get no pair, one may get nearly all."""
     from financial_chatbot_llm_amd.ops import mixers as mx
     top, W = 4, 8
