@@ -131,18 +131,107 @@ __global__ void __launch_bounds__(256) encoder_attention_kernel(const bf16* __re
   }
 }
 
-// grid (W rows / (16 NF), token tiles of 16 MF), 8 waves that split K in pieces of 32.  Both operands go from memory
-// straight to registers (W rows and token rows, 64 bytes of a row per four lanes); the partial sums meet in LDS.
-// Bound by latency: a bge projection has 1 - 5 MB of weights, a few microseconds at HBM rate, and the point is enough
-// blocks to ask for them at once.  18 rows, N x K = 2304 x 768: 4.3 us, the 256 x 256 tile kernel 17 us (its 9 tiles split
-// K over the idle CUs and meet in a second phase); 768 x 3072: 8 and 32 us.
+enum { SMALL_BIAS = 0, SMALL_GELU = 1, SMALL_SLAB = 2 };
+
+// bf16(s + bias) [-> exact GELU] of four adjacent columns
+template <int EPI> __device__ __forceinline__ void small_store(const f32x4& s, const bf16* bias, bf16* y) {
+  const bf16x4 bv = *reinterpret_cast<const bf16x4*>(bias);
+  bf16x4 o;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    float v = s[r] + (float)bv[r];
+    if (EPI == SMALL_GELU) {
+      v = (float)(bf16)v;                            // rounded where GEMM-with-bias -> bf16 -> GELU rounds
+      v = gelu_erf(v);
+    }
+    o[r] = (bf16)v;
+  }
+  *reinterpret_cast<bf16x4*>(y) = o;
+}
+
+// Up to 32 rows: grid (16 W rows, -, slices of K), MF tiles of 16 tokens.  Eight waves fetch both operands of 256 UN of K at a time as the
+// matrix instruction reads them and leave them in LDS; then one wave per token tile runs the products as ONE chain over K.  That
+// is the order of the LDS ring's sums (gemm_splitk.hip), which takes more rows: a text's embedding is the same bit by bit alone and
+// beside others.  Bound by latency: a bge projection has 1 - 5 MB of weights, a few microseconds at HBM rate, and the point is enough
+// blocks to ask for them at once.  18 rows, N x K = 2304 x 768: 4.5 us (eight waves that multiply an eighth of K each and add up, in
+// another order, 4.1; the 256 x 256 tile kernel 17), 768 x 768 4.2 (3.8), 3072 x 768 4.7 (4.3).
 // SLAB: gridDim.z slices of K, slice z's sums to f32 slab z [M, N] (no bias): a long K over few column tiles is 48 blocks that
 // each read 100 KB of weights and twice that of X (18 x 768 x 3072: 8.7 us, in four slices 4.8; the norm that adds
 // them 3.3 us instead of 2.8).
-enum { SMALL_BIAS = 0, SMALL_GELU = 1, SMALL_SLAB = 2 };
+template <int MF, int EPI, int UN>
+__global__ void __launch_bounds__(512) gemm_bias_chain_kernel(const bf16* __restrict__ X, int ldx, const bf16* __restrict__ W, int K,
+                                                              void* __restrict__ Yv, int ldy, const bf16* __restrict__ bias, int M, int N) {
+  constexpr int CH = 8 * UN;                           // steps of 32 of K at a time
+  __shared__ bf16x8 ops[CH][1 + MF][64];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, c = lane & 15;
+  const int n0 = blockIdx.x * 16, steps = K / 32 / gridDim.z, k0 = blockIdx.z * steps;
+  const bf16* wp = W + (long)(n0 + c) * K + 8 * g;
+  const bf16* xp[MF];
+#pragma unroll
+  for (int u = 0; u < MF; ++u) xp[u] = X + (long)min(16 * u + c, M - 1) * ldx + 8 * g;
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 v[UN][1 + MF];
+  auto fetch = [&](int at) {
+#pragma unroll
+    for (int i = 0; i < UN; ++i) {
+      const int k = min(at + w + 8 * i, steps - 1) + k0;       // no branch: all loads are asked for at once
+      v[i][0] = *reinterpret_cast<const bf16x8*>(wp + (long)k * 32);
+#pragma unroll
+      for (int u = 0; u < MF; ++u) v[i][1 + u] = *reinterpret_cast<const bf16x8*>(xp[u] + (long)k * 32);
+    }
+  };
+  fetch(0);
+  for (int at = 0; at < steps; at += CH) {
+    if (at > 0) __syncthreads();                       // the products of the steps before are done
+#pragma unroll
+    for (int i = 0; i < UN; ++i)
+#pragma unroll
+      for (int u = 0; u <= MF; ++u) ops[w + 8 * i][u][lane] = v[i][u];
+    __syncthreads();
+    if (at + CH < steps) fetch(at + CH);
+    if (w < MF) {
+      // operands a group ahead of their products: the chain waits for the matrix pipe only
+      const int n = min(CH, steps - at);
+      bf16x8 a[2][4], b[2][4];
+      auto read = [&](int s, int k) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[s][i] = ops[min(k + i, CH - 1)][0][lane], b[s][i] = ops[min(k + i, CH - 1)][1 + w][lane];
+      };
+      read(0, 0);
+#pragma unroll
+      for (int k = 0; k < CH; k += 4) {
+        if (k + 4 < CH) read((k / 4 + 1) & 1, k + 4);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (k + i < n) acc = mfma16(a[(k / 4) & 1][i], b[(k / 4) & 1][i], acc);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  const int m = 16 * w + c, n = n0 + 4 * g;
+  if (w >= MF || m >= M) return;
+  if constexpr (EPI == SMALL_SLAB) *reinterpret_cast<f32x4*>(static_cast<float*>(Yv) + ((long)blockIdx.z * M + m) * N + n) = acc;
+  else small_store<EPI>(acc, bias + n, static_cast<bf16*>(Yv) + (long)m * ldy + n);
+}
+
+template <int EPI>
+void launch_chain(const void* X, int ldx, const void* W, int K, void* Y, int ldy, const void* bias, int M, int N, int S, hipStream_t st) {
+  const dim3 grid(N / 16, 1, S);
+  const int un = K / S > 768 ? 4 : (K / S + 255) / 256;
+#define CHAIN(MF, UN) \
+  if (un == UN && MF == (M <= 16 ? 1 : 2)) \
+    gemm_bias_chain_kernel<MF, EPI, UN><<<grid, 512, 0, st>>>((const bf16*)X, ldx, (const bf16*)W, K, Y, ldy, (const bf16*)bias, M, N);
+  CHAIN(1, 1) CHAIN(1, 2) CHAIN(1, 3) CHAIN(1, 4) CHAIN(2, 1) CHAIN(2, 2) CHAIN(2, 3) CHAIN(2, 4)
+#undef CHAIN
+}
+
+// The sizes that neither that kernel nor the ring take: grid (W rows / (16 NF), token tiles of 16 MF), 8 waves that split K in pieces of 32.
+// Both operands go from memory straight to registers (W rows and token rows, 64 bytes of a row per four lanes); the
+// partial sums meet in LDS.
 template <int NF, int MF, int EPI>
 __global__ void __launch_bounds__(512) gemm_bias_small_kernel(const bf16* __restrict__ X, int ldx, const bf16* __restrict__ W,
-                                                              int K, void* __restrict__ Yv, int ldy,
+                                                              int K, bf16* __restrict__ Y, int ldy,
                                                               const bf16* __restrict__ bias, int M, int N) {
   constexpr int UN = NF * MF >= 4 ? 3 : 4;
   __shared__ f32x4 red[8][NF * MF][64];
@@ -159,9 +248,8 @@ __global__ void __launch_bounds__(512) gemm_bias_small_kernel(const bf16* __rest
   for (int f = 0; f < NF; ++f)
 #pragma unroll
     for (int u = 0; u < MF; ++u) acc[f][u] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int kt = K / 32, part = EPI == SMALL_SLAB ? blockIdx.z * 8 + w : w, parts = EPI == SMALL_SLAB ? gridDim.z * 8 : 8;
-  const int k1 = kt * (part + 1) / parts;
-  int k = kt * part / parts;
+  const int kt = K / 32, k1 = kt * (w + 1) / 8;
+  int k = kt * w / 8;
   Frag a[UN][NF], b[UN][MF];
   for (; k + UN <= k1; k += UN) {
 #pragma unroll
@@ -199,23 +287,7 @@ __global__ void __launch_bounds__(512) gemm_bias_small_kernel(const bf16* __rest
     f32x4 s = red[0][it][lane];
 #pragma unroll
     for (int i = 1; i < 8; ++i) s += red[i][it][lane];
-    if constexpr (EPI == SMALL_SLAB) {
-      *reinterpret_cast<f32x4*>(static_cast<float*>(Yv) + ((long)blockIdx.z * M + m) * N + n) = s;
-      continue;
-    }
-    bf16* Y = static_cast<bf16*>(Yv);
-    const bf16x4 bv = *reinterpret_cast<const bf16x4*>(bias + n);
-    bf16x4 y;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float v = s[r] + (float)bv[r];
-      if (EPI == SMALL_GELU) {
-        v = (float)(bf16)v;                          // rounded where GEMM-with-bias -> bf16 -> GELU rounds
-        v = gelu_erf(v);
-      }
-      y[r] = (bf16)v;
-    }
-    *reinterpret_cast<bf16x4*>(Y + (long)m * ldy + n) = y;
+    small_store<EPI>(s, bias + n, Y + (long)m * ldy + n);
   }
 }
 
@@ -236,49 +308,57 @@ PENNY_API int penny_encoder_attention(const void* qkv, long ld, const int* cu, i
 }
 
 // gemm_splitk.hip
-extern "C" int penny_bias_rows_tile(int M, int N);
-extern "C" int penny_bias_rows(const void* X, int ldx, const void* W, int K, void* Y, int ldy, const void* bias, int M, int N, int gelu, int nf,
+extern "C" int penny_bias_rows_tile(int M, int N, int S);
+extern "C" int penny_bias_rows(const void* X, int ldx, const void* W, int K, void* Y, int ldy, const void* bias, int M, int N, int gelu, int slices, int nf,
                                int mt, hipStream_t st);
+extern "C" int penny_rows_slabs(const void* X, int ldx, const void* W, int K, float* slabs, int M, int N, int S, int nf, int mt, int paired,
+                                hipStream_t st);
 
 namespace {
 
-// Slices of K for the second projection of the feed-forward: as many as bring its blocks near the CUs, 512 of K each at least;
-// 1: not split.  A query of 12 layers of 768 x 3072, us unsplit / in 2 / 3 / 4 / 6: 6 tokens 422 / 412 / 419 / 414 / 414, 18: 467 / 438 /
-// 437 / 441 / 451, 32: 505 / 472 / 466 / 459 / 466, 48: 599 / 536 / 521 / 511 / 523, 64: 634 / 565 / 550 / 545 / 556, 84: 680 / 611 / 623 / 621 /
-// 611, 109: 701 / 627 / 652 / 637 / 640, 179: 743 / 658 / 633 / 669 / 645.
-// As a call of its own the slices' sum is a launch more, so not where K is short: 1024 x 1024 7 rows unsplit 3.7, in 2 slices 5.6, 18: 4.4 / 6.0; 512 x
-// 2048 7: 5.0 / 5.8, 18: 6.6 / 6.3; 768 x 3072 7: 6.4 / 6.5, 18: 8.8 / 7.0.
-int few_slices(int M, int N, int K) {
-  if (K < (M <= 16 ? 3072 : 2048)) return 1;
-  if (N != 256 && N != 512 && N != 768 && N != 1024) return 1;
-  const long blocks = M <= 128 ? (long)(N / 16) * ((M + 63) / 64) : (long)((N + 31) / 32) * ((M + 63) / 64);
-  const long s = 216 / blocks, most = K / 512;
-  return (int)(s < most ? (s > 1 ? s : 1) : (most > 1 ? most : 1));
+// Weights whose rows beyond 32 the ring takes
+bool ring_shape(int N, int K) { return N >= 16 && N % 16 == 0 && K >= 64 && K % 64 == 0 && (N % 256 == 0 || K <= 1024); }
+
+// Slices of K for the second projection of the feed-forward: as many as bring its blocks near the CUs, 512 of K each at least; 1: not
+// split.  By the weight alone, for the same reason: a query embedded beside others would else rank its near-ties otherwise than
+// alone, and the prompt that is made of them would miss the prefix cache.  A query of 12 layers of 768 x 3072, us unsplit / in 2 / 3 / 4 / 6: 6
+// tokens 422 / 412 / 419 / 414 / 414, 18: 467 / 438 / 437 / 441 / 451, 32: 505 / 472 / 466 / 459 / 466, 48: 599 / 536 / 521 / 511 / 523, 64: 634 / 565 /
+// 550 / 545 / 556, 84: 680 / 611 / 623 / 621 / 611, 109: 701 / 627 / 652 / 637 / 640, 179: 743 / 658 / 633 / 669 / 645.  As a call of its own the
+// slices' sum is a launch more, so not where K is short: 1024 x 1024 7 rows unsplit 3.7, in 2 slices 5.6, 18: 4.4 / 6.0; 512 x 2048 7: 5.0 / 5.8,
+// 18: 6.6 / 6.3; 768 x 3072 7: 6.4 / 6.5, 18: 8.8 / 7.0.
+int few_slices(int N, int K) {
+  if (K < 3072 || !ring_shape(N, K) || (N != 256 && N != 512 && N != 768 && N != 1024)) return 1;
+  int s = 256 / (N / 16);
+  if (s > K / 512) s = K / 512;
+  while (K % (64 * s)) --s;
+  return s;
 }
+
+// Parts of K that are summed for themselves and then added in turn, one order of the sums for all numbers of rows: the slices above; of a
+// long K that has none the eighths that gemm_bias_small_kernel's waves take (2048 x 8192 7 rows 16.1 us, as one chain 19.5; the ring adds
+// them up at no cost); else K is one chain.
+int sum_parts(int N, int K) {
+  const int s = few_slices(N, K);
+  return s > 1 ? s : K > 1024 && K % 512 == 0 && ring_shape(N, K) ? 8 : 1;
+}
+
+// The slices as slabs that the next pass adds: up to 192 rows; beyond, the ring adds them itself
+int small_slices(int M, int N, int K) { return M <= 192 ? few_slices(N, K) : 1; }
 
 }  // namespace
 
-// The tile (nf | mt << 8) with which a projection goes through the LDS ring of gemm_splitk.hip instead of the kernel above, or 0.
-// Blocks of the kernel above read both operands for themselves, which costs more with every further row tile; the ring's tiles share
+// The tile (nf | mt << 8) with which a projection goes through the LDS ring of gemm_splitk.hip instead of the kernels above, or 0.
+// Blocks of the kernel that splits K read both operands for themselves, which costs more with every further row tile; the ring's tiles share
 // them, one round of blocks for all. Us, above (its slices included) or the tile kernel / ring: 2304 x 768 18 rows 4.0 / 4.8, 48 5.5 / 4.8,
 // 128 9.3 / 5.8, 256 11.0 / 6.7, 768 20.1 / 11.0, 1536 21.3 / 16.8, 2048 21.6 / 24.8 (two rounds); 768 x 768 48 5.0 / 4.5, 768 10.6 / 6.3, 1536
-// 20.2 / 9.0; 3072 x 768 with GELU 128 9.6 / 6.2, 768 24.5 / 15.4, 1024 27.8 / 19.0; 768 x 3072 48 8.8 / 10.0, 192 (in slices, which
-// the next norm adds) 8.8 / 10.4, 256 11 / 10.4, 768 35.1 / 15.6, 2048 38.4 / 27.5; 4096 x 1024 512 31.4 / 14.0; 1024 x 4096 128 20.5 / 12.7.  Widths that
+// 20.2 / 9.0; 3072 x 768 with GELU 128 9.6 / 6.2, 768 24.5 / 15.4, 1024 27.8 / 19.0; 768 x 3072 48 8.6 / 7.0, 192 (in slices,
+// on either side, with the launch that adds them) 11.4 / 9.5, 256 (unsplit) 11 / 10.4, 768 35.1 / 15.6, 2048 38.4 / 27.5; 4096 x 1024 512 31.4 / 14.0; 1024 x 4096 128 20.5 / 12.7.  Widths that
 // the tile kernel does not take have the library behind them: 1152 x 384 256 4.5 / 4.2, 1024 8.0 / 6.9, 2048 9.5 / 10.2; 384 x 1536 64 - 192 4.9 /
-// 6.5: not there.  Nor where K is as long as many rows (2048 x 8192 1000 rows 67.9 / 65.6, 1280 70.0 / 78.3, 2048 79.4 / 90.8), nor for few rows and
-// a short K, whose ring has nothing to fill (1152 x 384 33 rows 3.5 / 3.9).
+// 6.5: not there.  Nor where K is as long as many rows (2048 x 8192 1000 rows 67.9 / 65.6, 1280 70.0 / 78.3, 2048 79.4 / 90.8).
 PENNY_API int penny_bias_rows_plan(int M, int N, int K) {
-  if (M <= (K < 512 ? 40 : 32) || N < 16 || N % 16 || K < 64 || K % 64 || M > (N % 256 == 0 ? 2048 : K <= 1024 ? 1024 : 0) || (long)M * K > 1 << 23)
-    return 0;
-  if (M <= 192 && few_slices(M, N, K) > 1) return 0;
-  return penny_bias_rows_tile(M, N);
+  if (M <= 32 || !ring_shape(N, K) || M > (N % 256 == 0 ? 2048 : 1024) || (long)M * K > 1 << 23 || small_slices(M, N, K) > 1) return 0;
+  return penny_bias_rows_tile(M, N, 1);
 }
-
-namespace {
-
-int small_slices(int M, int N, int K) { return penny_bias_rows_plan(M, N, K) ? 1 : few_slices(M, N, K); }
-
-}  // namespace
 
 // Y [M, N] (row stride ldy) = bf16(X W^T + bias) [-> exact GELU]; W [N, K] contiguous; N % 16 == 0, K % 32 == 0, rows in
 // whole 16 bytes
@@ -288,17 +368,24 @@ PENNY_API int penny_gemm_bias_small(const void* X, int ldx, const void* W, int K
   if (N % 16 || K % 32 || ldx % 8 || ldy % 4 || ((size_t)X | (size_t)W) % 16 || ((size_t)Y | (size_t)bias) % 8 ||
       (M + 15) / 16 > 65535)
     return (int)hipErrorInvalidValue;
-  if (const int tile = penny_bias_rows_plan(M, N, K))
-    return penny_bias_rows(X, ldx, W, K, Y, ldy, bias, M, N, gelu, tile & 255, tile >> 8, stream);
+  const bool sliced = few_slices(N, K) > 1;
+  if (M <= 32 && ring_shape(N, K) && (sum_parts(N, K) == 1 || (gelu && sliced))) {
+    if (gelu) launch_chain<SMALL_GELU>(X, ldx, W, K, Y, ldy, bias, M, N, 1, stream);
+    else launch_chain<SMALL_BIAS>(X, ldx, W, K, Y, ldy, bias, M, N, 1, stream);
+    PENNY_RETURN_LAUNCH();
+  }
+  // (GELU behind a weight of slices: no slabs there, one chain throughout)
+  if (const int tile = gelu && M > 32 && small_slices(M, N, K) > 1 ? penny_bias_rows_tile(M, N, 1) : penny_bias_rows_plan(M, N, K))
+    return penny_bias_rows(X, ldx, W, K, Y, ldy, bias, M, N, gelu, gelu && sliced ? 1 : sum_parts(N, K), tile & 255, tile >> 8, stream);
 #define SMALL(NF, MF)                                                                                                    \
   do {                                                                                                                   \
     const dim3 grid((N + 16 * NF - 1) / (16 * NF), (M + 16 * MF - 1) / (16 * MF));                                       \
     if (gelu)                                                                                                            \
-      gemm_bias_small_kernel<NF, MF, SMALL_GELU><<<grid, 512, 0, stream>>>((const bf16*)X, ldx, (const bf16*)W, K, Y,    \
-                                                                           ldy, (const bf16*)bias, M, N);                \
+      gemm_bias_small_kernel<NF, MF, SMALL_GELU><<<grid, 512, 0, stream>>>((const bf16*)X, ldx, (const bf16*)W, K,       \
+                                                                           (bf16*)Y, ldy, (const bf16*)bias, M, N);      \
     else                                                                                                                 \
-      gemm_bias_small_kernel<NF, MF, SMALL_BIAS><<<grid, 512, 0, stream>>>((const bf16*)X, ldx, (const bf16*)W, K, Y,    \
-                                                                           ldy, (const bf16*)bias, M, N);                \
+      gemm_bias_small_kernel<NF, MF, SMALL_BIAS><<<grid, 512, 0, stream>>>((const bf16*)X, ldx, (const bf16*)W, K,       \
+                                                                           (bf16*)Y, ldy, (const bf16*)bias, M, N);      \
   } while (0)
   if (M <= 16) SMALL(1, 1);
   else if (M <= 32) SMALL(1, 2);
@@ -433,16 +520,13 @@ __global__ void __launch_bounds__(256) slab_bias_kernel(const float* __restrict_
   *reinterpret_cast<bf16x4*>(y + (long)row * ldy + n) = o;
 }
 
-// S slices of K of X W^T to f32 slabs [S, M, N]
+// S = few_slices(N, K) slices of K of X W^T to f32 slabs [S, M, N], up to 192 rows (192 x 1024 and 4 slices: 192 blocks of 4 x 4)
 int small_slabs(const void* X, int ldx, const void* W, float* slabs, int S, int M, int N, int K, hipStream_t stream) {
-#define SLABS(NF, MF)                                                                                                    \
-  gemm_bias_small_kernel<NF, MF, SMALL_SLAB><<<dim3((N + 16 * NF - 1) / (16 * NF), (M + 16 * MF - 1) / (16 * MF), S), 512, 0, stream>>>( \
-      (const bf16*)X, ldx, (const bf16*)W, K, slabs, N, nullptr, M, N)
-  if (M <= 16) SLABS(1, 1);
-  else if (M <= 32) SLABS(1, 2);
-  else if (M <= 128) SLABS(1, 4);
-  else SLABS(2, 4);
-#undef SLABS
+  if (M > 32) {
+    const int tile = penny_bias_rows_tile(M, N, S);
+    return tile ? penny_rows_slabs(X, ldx, W, K, slabs, M, N, S, tile & 255, tile >> 8, 1, stream) : (int)hipErrorInvalidValue;
+  }
+  launch_chain<SMALL_SLAB>(X, ldx, W, K, slabs, N, nullptr, M, N, S, stream);
   return (int)hipGetLastError();
 }
 
@@ -513,7 +597,8 @@ constexpr int PENNY_MISALIGNED = -1;
 // All layers of a small batch: x [T, H] bf16 is replaced by the last layer's output.  w: 12 pointers per layer -- qkv, its
 // bias, o, its bias, the first norm's weight and bias, fc1, its bias, fc2, its bias, the second norm's weight and bias, each
 // contiguous bf16.  ws: T * (6 H + F) bf16, then f32 slabs [penny_encoder_slices(T, H, F), T, H] where that is more than 1.  Shapes as
-// penny_gemm_bias_small, penny_encoder_attention and penny_layernorm take them; PENNY_MISALIGNED, and nothing launched, for a weight off their 16 bytes (asked here: 144 weights take 18 us in Python).
+// penny_gemm_bias_small, penny_encoder_attention and penny_layernorm take them; PENNY_MISALIGNED, and nothing launched, for a weight off
+// their 16 bytes (asked here: 144 weights take 18 us in Python).
 // The launches of one layer take the host 8 x 2.5 us here and 8 x 7 from Python, where the kernels of a single query
 // (18 tokens, 12 layers of 768) run for 440 us in all: 815 -> 497 us for the query.
 PENNY_API int penny_encoder_layers(const void* const* w, int layers, void* x, void* ws, const int* cu, int texts, int max_len,

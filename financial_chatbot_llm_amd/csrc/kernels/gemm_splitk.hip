@@ -53,7 +53,7 @@ struct SkSample {
   int* pi;
   int pstride, voff, vvalid;
   const bf16* bias;                      // SK_BIAS
-  int gelu;
+  int gelu, slices;
 };
 
 // X image: token row r of a stage lives at byte r*128; its logical 16-B chunk c (k = 8c..8c+7) at
@@ -140,7 +140,8 @@ __device__ __forceinline__ void stage_mma(const char* __restrict__ base, f32x4 (
 }
 
 // Epilogues (EPI):
-//   SK_BIAS   SK_BF16 with a bias row and, where asked for, the exact GELU of the rounded sum (encoder projections);
+//   SK_BIAS   SK_BF16 with a bias row and, where asked for, the exact GELU of the rounded sum (encoder projections).  Each of
+//             sa.slices slices of K is summed by itself and the slices then in turn, as by slabs: the same sums in every form;
 //   SK_F32    SK_SLAB for f32 operands, which are addressed as twice as many 16-bit columns (K, ldx);
 //   SK_SLAB   f32 partial slabs P [S, M, N] (reduced by the consumer's row pass);
 //   SK_SILU   W is the 16-row-interleaved gate|up weight (ops/gemm.py interleave16) and S == 1: the
@@ -255,13 +256,37 @@ __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restr
   for (int j = 0; j < NBUF - 1; ++j)
     if (j < nst) stage(j);
 
-  for (int j = 0; j < nst; ++j) {
-    // stages j+1 .. min(j+NBUF-2, nst-1) may stay in flight
-    wait_stage<LOADS * BKM, NBUF - 2>(min(NBUF - 2, nst - 1 - j));
-    if (j + NBUF - 1 < nst) stage(j + NBUF - 1);
+  auto stream = [&](int j0, int j1) {
+    for (int j = j0; j < j1; ++j) {
+      // stages j+1 .. min(j+NBUF-2, nst-1) may stay in flight
+      wait_stage<LOADS * BKM, NBUF - 2>(min(NBUF - 2, nst - 1 - j));
+      if (j + NBUF - 1 < nst) stage(j + NBUF - 1);
 #pragma unroll
-    for (int u = 0; u < BKM; ++u)
-      stage_mma<FW, TW, WBYTES, WROW, EPI == SK_F32>(smem + (j % NBUF) * SLOT + u * SBYTES, sums, wa, wb, lane, g, col);
+      for (int u = 0; u < BKM; ++u)
+        stage_mma<FW, TW, WBYTES, WROW, EPI == SK_F32>(smem + (j % NBUF) * SLOT + u * SBYTES, sums, wa, wb, lane, g, col);
+    }
+  };
+  if constexpr (EPI == SK_BIAS) {                    // K % (64 BKM slices) == 0
+    const int per = nst / sa.slices;
+    f32x4 total[FW][TW];
+    stream(0, per);
+    for (int j0 = per; j0 < nst; j0 += per) {
+#pragma unroll
+      for (int f = 0; f < FW; ++f)
+#pragma unroll
+        for (int t = 0; t < TW; ++t) {
+          total[f][t] = j0 == per ? sums[0][f][t] : total[f][t] + sums[0][f][t];
+          sums[0][f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      stream(j0, j0 + per);
+    }
+    if (per < nst)
+#pragma unroll
+      for (int f = 0; f < FW; ++f)
+#pragma unroll
+        for (int t = 0; t < TW; ++t) sums[0][f][t] = total[f][t] + sums[0][f][t];
+  } else {
+    stream(0, nst);
   }
   f32x4(&acc)[FW][TW] = sums[0];
   if constexpr (EPI == SK_F32) {
@@ -710,6 +735,22 @@ PENNY_API int penny_linear_rows_replay_plan(int M, int N, int K, int f32) {
   return N <= 8192 && (K < 4096 || plan >> 16 > 1) ? plan : 0;
 }
 
+#define ROWS_TILES(CASE) \
+  CASE(2, 2, 2) CASE(2, 4, 1) CASE(4, 2, 2) CASE(2, 6, 2) CASE(4, 4, 1) CASE(2, 8, 1) CASE(4, 6, 2) CASE(8, 2, 2) CASE(4, 8, 1) CASE(8, 4, 2) \
+  CASE(8, 6, 2) CASE(4, 12, 1) CASE(8, 8, 2)
+
+// S slices of K of X W^T (bf16, W row-major) to f32 slabs [S, M, N]
+extern "C" int penny_rows_slabs(const void* X, int ldx, const void* W, int K, float* slabs, int M, int N, int S, int nf, int mt, int paired,
+                                hipStream_t st) {
+  if (M <= 0) return 0;
+  if (M > (1 << 20) || N <= 0 || N % 16 || S < 1 || K <= 0 || K % (64 * S) || ldx % 8) return (int)hipErrorInvalidValue;
+#define SLABS_CASE(NF_, MT_, WA_) \
+  if (nf == NF_ && mt == MT_) return launch<NF_, MT_, WA_, true>(X, ldx, W, K, slabs, M, N, S, paired ? 3 : 1, st);
+  ROWS_TILES(SLABS_CASE)
+#undef SLABS_CASE
+  return (int)hipErrorInvalidValue;
+}
+
 // Y [M, N] = X [M, K] x W [N, K]^T in bf16 or f32 (f32 != 0) for up to about two thousand rows, W row-major: slabs == null streams W once (S = 1), else
 // S slices of K leave f32 slabs [S, M, N] that a second launch adds.  One entry for both, so that a step that the host bounds
 // pays for one call.  nf, mt: a block's columns and rows in units of 16, one of kRowsTiles.  Contract (checked): N % 16 == 0 (the last
@@ -728,24 +769,12 @@ PENNY_API int penny_linear_rows(const void* X, int ldx, const void* W, int K, vo
       if constexpr (NF_ * MT_ <= 12) rc = launch_f32<NF_, MT_, WA_>(X, ldx, W, K, p, M, N, S, paired, st); \
       else return (int)hipErrorInvalidValue;                                                       \
     } else if (S > 1) {                                                                            \
-      rc = launch<NF_, MT_, WA_, true>(X, ldx, W, K, p, M, N, S, paired ? 3 : 1, st);              \
+      rc = penny_rows_slabs(X, ldx, W, K, p, M, N, S, nf, mt, paired, st);                         \
     } else {                                                                                       \
       rc = launch_bf16<NF_, MT_, WA_, true>(X, ldx, W, K, Y, N, M, N, paired ? 3 : 1, st);         \
     }                                                                                              \
   } else
-  LR_CASE(2, 2, 2)
-  LR_CASE(2, 4, 1)
-  LR_CASE(4, 2, 2)
-  LR_CASE(2, 6, 2)
-  LR_CASE(4, 4, 1)
-  LR_CASE(2, 8, 1)
-  LR_CASE(4, 6, 2)
-  LR_CASE(8, 2, 2)
-  LR_CASE(4, 8, 1)
-  LR_CASE(8, 4, 2)
-  LR_CASE(8, 6, 2)
-  LR_CASE(4, 12, 1)
-  LR_CASE(8, 8, 2)
+  ROWS_TILES(LR_CASE)
   return (int)hipErrorInvalidValue;
 #undef LR_CASE
   if (rc || S == 1) return rc;
@@ -755,42 +784,33 @@ PENNY_API int penny_linear_rows(const void* X, int ldx, const void* W, int K, vo
   return (int)hipGetLastError();
 }
 
-// The tile of penny_bias_rows for M rows: the fastest that runs all its blocks in one round; 0: none does
-extern "C" int penny_bias_rows_tile(int M, int N) {
+// The tile of penny_bias_rows (S = 1) or penny_rows_slabs for M rows: the fastest that runs all its blocks in one round; 0: none does
+extern "C" int penny_bias_rows_tile(int M, int N, int S) {
   int tile = 0;
   float best = 1e9f;
   for (const RowsTile& t : kRowsTiles) {
-    const long blocks = (long)((N + 16 * t.nf - 1) / (16 * t.nf)) * ((M + 16 * t.mt - 1) / (16 * t.mt));
+    const long blocks = (long)((N + 16 * t.nf - 1) / (16 * t.nf)) * ((M + 16 * t.mt - 1) / (16 * t.mt)) * S;
     if (blocks <= 256 && t.us < best) best = t.us, tile = t.nf | t.mt << 8;
   }
   return tile;
 }
 
-// Y [M, N] (row stride ldy) = bf16(X W^T + bias) [-> exact GELU] on the same tiles, for penny_gemm_bias_small
-extern "C" int penny_bias_rows(const void* X, int ldx, const void* W, int K, void* Y, int ldy, const void* bias, int M, int N, int gelu, int nf, int mt,
-                    hipStream_t st) {
+// Y [M, N] (row stride ldy) = bf16(X W^T + bias) [-> exact GELU] on the same tiles, for penny_gemm_bias_small; the sums are those of
+// penny_rows_slabs in `slices` slices, added in turn
+extern "C" int penny_bias_rows(const void* X, int ldx, const void* W, int K, void* Y, int ldy, const void* bias, int M, int N, int gelu, int slices, int nf,
+                               int mt, hipStream_t st) {
   if (M <= 0) return 0;
-  if (M > (1 << 20) || N <= 0 || N % 16 || K <= 0 || K % 64 || ldx % 8 || ldy % 4) return (int)hipErrorInvalidValue;
+  if (M > (1 << 20) || N <= 0 || N % 16 || K <= 0 || slices < 1 || K % (64 * slices) || ldx % 8 || ldy % 4)
+    return (int)hipErrorInvalidValue;
   SkSample sa{};
   sa.bias = static_cast<const bf16*>(bias);
   sa.gelu = gelu;
+  sa.slices = slices;
 #define BR_CASE(NF_, MT_, WA_)                                                                                          \
   if (nf == NF_ && mt == MT_)                                                                                           \
-    return launch_any<NF_, MT_, WA_, SK_BIAS, 16, true>(3, K % 128 == 0, dim3((N + 16 * NF_ - 1) / (16 * NF_), (M + 16 * MT_ - 1) / (16 * MT_)), \
+    return launch_any<NF_, MT_, WA_, SK_BIAS, 16, true>(3, K / slices % 128 == 0, dim3((N + 16 * NF_ - 1) / (16 * NF_), (M + 16 * MT_ - 1) / (16 * MT_)), \
                                                   st, (const bf16*)X, ldx, (const bf16*)W, K, (float*)nullptr, M, N, 1, (bf16*)Y, ldy, sa);
-  BR_CASE(2, 2, 2)
-  BR_CASE(2, 4, 1)
-  BR_CASE(4, 2, 2)
-  BR_CASE(2, 6, 2)
-  BR_CASE(4, 4, 1)
-  BR_CASE(2, 8, 1)
-  BR_CASE(4, 6, 2)
-  BR_CASE(8, 2, 2)
-  BR_CASE(4, 8, 1)
-  BR_CASE(8, 4, 2)
-  BR_CASE(8, 6, 2)
-  BR_CASE(4, 12, 1)
-  BR_CASE(8, 8, 2)
+  ROWS_TILES(BR_CASE)
 #undef BR_CASE
   return (int)hipErrorInvalidValue;
 }
