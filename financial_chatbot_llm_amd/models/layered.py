@@ -15,8 +15,9 @@ import math
 from typing import Callable, Dict, List, NamedTuple, Optional
 
 import torch
+import torch.nn.functional as F
 
-from ..ops.gemm import project
+from ..ops.gemm import project, transformed
 from .common import HybridCache, param_seed
 from .configs import ModelConfig
 from .mixers import MIXERS
@@ -218,4 +219,4 @@ class LayeredDecoder:
         return self.head
 
     def logits(self, h: torch.Tensor) -> torch.Tensor:
-        return project(h, self.head)
+        return F.linear(h, self.head) if transformed(h) else project(h, self.head)

@@ -26,6 +26,7 @@ from typing import Dict, List, Optional, Tuple, Union
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import _native as N
 from .activation import silu_mul
@@ -268,11 +269,19 @@ def replayed():
         _REPLAYED.on = before
 
 
+def transformed(x: torch.Tensor) -> bool:
+    """Is ``x`` more than its data: under vmap, forward-mode differentiation or a trace, or of a tensor class of its own?  A launch on its
+    data pointer would lose that, so that an entry point that such code may call keeps torch's own operation for it."""
+    return type(x) is not torch.Tensor or torch._C._functorch.peek_interpreter_stack() is not None or forward_ad._current_level >= 0 or \
+        torch.jit.is_tracing()
+
+
 def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """y = x @ w.T in bf16 or f32: the streaming kernels for up to about two thousand rows (``penny_linear_rows_plan``; inside
     :func:`replayed` ``penny_linear_rows_replay_plan``), the library's product for the rest."""
     dt = x.dtype
-    if dt == w.dtype and (dt == torch.bfloat16 or dt == torch.float32) and x.dim() == 2 and w.dim() == 2 and N.use_native(x):
+    if dt == w.dtype and (dt == torch.bfloat16 or dt == torch.float32) and x.dim() == 2 and w.dim() == 2 and N.use_native(x) and \
+            not torch.is_autocast_enabled():
         (M, K), N_, f32 = x.shape, w.shape[0], dt == torch.float32
         ldx, xp, wp = x.stride(0), x.data_ptr(), w.data_ptr()
         if M <= 2048 and K == w.shape[1] and (xp | wp) % 16 == 0 and ldx % (4 if f32 else 8) == 0 and ldx >= K and x.stride(1) == 1 and \

@@ -123,3 +123,26 @@ def test_the_runner_says_so(monkeypatch):
     r._run_static(3)
     r._run_static(4, filtered=True)
     assert seen == [(3, False, True), (4, True, True)] and not getattr(G._REPLAYED, "on", False)
+
+
+def test_transformed_calls():
+    """The head of the layered decoders under vmap, forward mode, a trace and a tensor class; any product under autocast."""
+    from types import SimpleNamespace
+    from torch.autograd import forward_ad as fw
+    from financial_chatbot_llm_amd.models.layered import LayeredDecoder
+    g = torch.Generator(device="cuda").manual_seed(3)
+    model = SimpleNamespace(head=torch.randn((512, 128), generator=g, device="cuda"))
+    logits = lambda h: LayeredDecoder.logits(model, h)                                 # noqa: E731
+    h, t = (torch.randn((3, 4, 128), generator=g, device="cuda") for _ in range(2))
+    want = torch.nn.functional.linear(h, model.head)
+    assert torch.allclose(torch.vmap(logits)(h), want, atol=1e-4)
+    with fw.dual_level():
+        y, dy = fw.unpack_dual(logits(fw.make_dual(h[0], t[0])))
+    assert torch.allclose(y, want[0], atol=1e-4) and torch.allclose(dy, t[0] @ model.head.t(), atol=1e-4)
+    y, dy = torch.func.jvp(logits, (h[0],), (t[0],))
+    assert torch.allclose(dy, t[0] @ model.head.t(), atol=1e-4)
+    traced = torch.jit.trace(logits, h[0], check_trace=False)
+    assert torch.allclose(traced(h[1]), want[1], atol=1e-4)
+    assert isinstance(logits(torch.nn.Parameter(h[0], requires_grad=False)), torch.Tensor) and logits(h[0]).dtype == torch.float32
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert logits(h[0]).dtype == torch.bfloat16
