@@ -9,8 +9,8 @@
 // projected inputs in slot slot[s] of `state` (f32 [slots, K-1, C]); a segment that starts at position 0 starts from
 // zeros whatever the slot held.  G = 0: queries only (a layer that reads another layer's keys and values).
 //
-// A wave owns one head and TT consecutive rows of a segment: all TT + K - 1 input rows are fetched before the first
-// is used (the loads overlap), the convolution runs from registers and each row's norm is one wave reduction.
+// A wave owns one head and TT consecutive rows of a segment: all TT + K - 1 input rows and the slot's next history are fetched
+// before the first is used (the loads overlap), the convolution runs from registers and the norms of four rows are reduced side by side.
 // Only the wave of a segment's first tile reads the slot's history (TT >= K - 1), and it is the one that replaces it.
 #include "mx_common.h"
 
@@ -25,7 +25,8 @@ conv_heads_kernel(const T* __restrict__ in, long si, const float* __restrict__ w
                   const float* __restrict__ qw, const float* __restrict__ kw, float eps, float tcoef, int tevery,
                   const int* __restrict__ cu, const int* __restrict__ slot, const int* __restrict__ pos,
                   const int* __restrict__ slots, T* __restrict__ cache, T* __restrict__ qout, int S, int per, int H, int G, int D, int P) {
-  static_assert(TT >= KM - 1, "tiles behind the first must not reach the slot's history");
+  static_assert(TT == 1 || TT >= KM - 1, "tiles behind the first must not reach the slot's history; single-row tiles are for segments of one row");
+  constexpr int RB = TT < 4 ? TT : 4;
   typedef T vt __attribute__((ext_vector_type(VE)));
   constexpr int NV = NC * VE;
   int s, t0;
@@ -42,7 +43,9 @@ conv_heads_kernel(const T* __restrict__ in, long si, const float* __restrict__ w
   float* st = state + (sl < 0 ? 0 : (long)sl * (K - 1) * C) + col;
   const int pad = KM - K;                                // taps are aligned to the end of the KM-wide window
 
-  float x[TT + KM - 1][NV], wk[KM][NV];
+  float x[TT + KM - 1][NV], wk[KM][NV], h[KM <= 8 ? KM - 1 : 1][NV];
+  const bool first = t0 == 0, keep = first && sl >= 0;
+  // every load is issued before the first is used: rows behind the segment's end read its last one, and are not used
 #pragma unroll
   for (int r = 0; r < TT + KM - 1; ++r) {
     const int j = t0 - (KM - 1) + r;                     // row of the segment, < 0: history
@@ -52,12 +55,10 @@ conv_heads_kernel(const T* __restrict__ in, long si, const float* __restrict__ w
 #pragma unroll
       for (int e = 0; e < VE; ++e) x[r][c * VE + e] = 0.f;
       if (d < nd) {
-        if (j >= 0) {
-          if (j < n) {
-            const vt v = *reinterpret_cast<const vt*>(in + (long)(r0 + j) * si + col + d);
+        if (r >= KM - 1 || !first) {
+          const vt v = *reinterpret_cast<const vt*>(in + (long)(r0 + max(min(j, n - 1), 0)) * si + col + d);
 #pragma unroll
-            for (int e = 0; e < VE; ++e) x[r][c * VE + e] = (float)v[e];
-          }
+          for (int e = 0; e < VE; ++e) x[r][c * VE + e] = (float)v[e];
         } else if (!fresh && K - 1 + j >= 0) {
 #pragma unroll
           for (int e = 0; e < VE; ++e) x[r][c * VE + e] = st[(long)(K - 1 + j) * C + d + e];
@@ -65,6 +66,20 @@ conv_heads_kernel(const T* __restrict__ in, long si, const float* __restrict__ w
       }
     }
   }
+  if (KM <= 8 && keep)
+#pragma unroll
+    for (int e = 0; e < (KM <= 8 ? KM - 1 : 0); ++e)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int d = (c * 64 + lane) * VE, i = n - (K - 1) + e;
+#pragma unroll
+        for (int q = 0; q < VE; ++q) h[e][c * VE + q] = 0.f;
+        if (d < nd && e < K - 1) {
+#pragma unroll
+          for (int q = 0; q < VE; ++q)
+            h[e][c * VE + q] = i >= 0 ? ldf(in + (long)(r0 + i) * si + col + d + q) : (fresh ? 0.f : st[(long)(e + n) * C + d + q]);
+        }
+      }
 #pragma unroll
   for (int k = 0; k < KM; ++k)
 #pragma unroll
@@ -76,8 +91,18 @@ conv_heads_kernel(const T* __restrict__ in, long si, const float* __restrict__ w
       }
   // the slot's next history: entry e is the input K-1-e rows before the segment's end (entries move down, so each
   // is read before it is overwritten; a lane touches its own channels only)
-  if (t0 == 0 && sl >= 0) {
-    for (int e = 0; e < K - 1; ++e) {
+  if (keep) {
+#pragma unroll
+    for (int e = 0; e < (KM <= 8 ? KM - 1 : 0); ++e)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int d = (c * 64 + lane) * VE;
+        if (d < nd && e < K - 1) {
+#pragma unroll
+          for (int q = 0; q < VE; ++q) st[(long)e * C + d + q] = h[e][c * VE + q];
+        }
+      }
+    for (int e = 0; KM > 8 && e < K - 1; ++e) {
       const int i = n - (K - 1) + e;
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
@@ -102,45 +127,63 @@ conv_heads_kernel(const T* __restrict__ in, long si, const float* __restrict__ w
         nw[c * VE + e] = d < nd ? wn[d] : 0.f;
       }
   const int Wr = G * (D + P);
+  // four rows at a time, so that their reductions run side by side
 #pragma unroll
-  for (int i = 0; i < TT; ++i) {
-    if (t0 + i >= n) break;
-    const long row = r0 + t0 + i;
-    float y[NV], ss = 0.f;
+  for (int i0 = 0; i0 < TT; i0 += RB) {
+    if (t0 + i0 >= n) break;
+    float y[RB][NV], ss[RB];
+    int at[RB];                                           // position of a query, cache row of a key or value
 #pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      float a = 0.f;
+    for (int i = 0; i < RB; ++i) {
+      const long row = r0 + min(t0 + i0 + i, n - 1);
+      at[i] = isq ? (tcoef != 0.f ? pos[row] : 0) : slots[row];
+      ss[i] = 0.f;
 #pragma unroll
-      for (int k = 0; k < KM; ++k) a += wk[k][v] * x[i + k][v];
-      y[v] = a;
-      ss += a * a;
+      for (int v = 0; v < NV; ++v) {
+        float a = 0.f;
+#pragma unroll
+        for (int k = 0; k < KM; ++k) a += wk[k][v] * x[i0 + i + k][v];
+        y[i][v] = a;
+        ss[i] += a * a;
+      }
     }
     if (wn != nullptr) {
-      const float f = 1.0f / sqrtf(mx_wave_sum(ss) / (float)nd + eps);
 #pragma unroll
-      for (int v = 0; v < NV; ++v) y[v] *= f * nw[v];
-    }
-    T* dst;
-    if (isq) {
-      if (tcoef != 0.f) {
-        const float f = 1.0f + tcoef * logf((float)((pos[row] + 1) / tevery + 1));
+      for (int o = 32; o > 0; o >>= 1)
 #pragma unroll
-        for (int v = 0; v < NV; ++v) y[v] *= f;
+        for (int i = 0; i < RB; ++i) ss[i] += __shfl_xor(ss[i], o, 64);
+#pragma unroll
+      for (int i = 0; i < RB; ++i) {
+        const float f = 1.0f / sqrtf(ss[i] / (float)nd + eps);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) y[i][v] *= f * nw[v];
       }
-      dst = qout + row * (long)H * D + (long)unit * D;
-    } else {
-      const int cr = slots[row];
-      if (cr < 0) continue;
-      dst = cache + (long)cr * Wr + (isv ? G * D + (unit - H - G) * P : (unit - H) * D);
     }
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const int d = (c * 64 + lane) * VE;
-      if (d < nd) {
-        vt o;
+    for (int i = 0; i < RB; ++i) {
+      if (t0 + i0 + i >= n) break;
+      const long row = r0 + t0 + i0 + i;
+      T* dst;
+      if (isq) {
+        if (tcoef != 0.f) {
+          const float f = 1.0f + tcoef * logf((float)((at[i] + 1) / tevery + 1));
 #pragma unroll
-        for (int e = 0; e < VE; ++e) o[e] = (T)y[c * VE + e];
-        *reinterpret_cast<vt*>(dst + d) = o;
+          for (int v = 0; v < NV; ++v) y[i][v] *= f;
+        }
+        dst = qout + row * (long)H * D + (long)unit * D;
+      } else {
+        if (at[i] < 0) continue;
+        dst = cache + (long)at[i] * Wr + (isv ? G * D + (unit - H - G) * P : (unit - H) * D);
+      }
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int d = (c * 64 + lane) * VE;
+        if (d < nd) {
+          vt o;
+#pragma unroll
+          for (int e = 0; e < VE; ++e) o[e] = (T)y[i][c * VE + e];
+          *reinterpret_cast<vt*>(dst + d) = o;
+        }
       }
     }
   }
@@ -164,6 +207,9 @@ MX_API int mx_conv_heads(const void* in, long si, int dt, const float* w, int K,
   const size_t al = dt == 1 ? 8 : 4;                       // two elements
   const bool two = D % 2 == 0 && (G == 0 || P % 2 == 0) && si % 2 == 0 && ((size_t)in | (size_t)qout | (size_t)cache) % al == 0;
   const int units = H + 2 * G;
+  // Rows per wave: a wave's rows follow each other's loads, so that few are the shorter way until memory is the bound (bf16, 16 query heads
+  // over 4, four taps, us, before with 8 rows one after the other / 4 / 8: 60 rows 10.3 / 6.8 / 9.0, 400 11.4 / 8.8 / 9.9, 800 12.9 / 11.1 /
+  // 11.9, 1188 15.2 / 15.4 / 14.4, 2048 18.3 / 21.9 / 17.6, 4096 29.6 / 38.5 / 31.4)
 #define CH_LAUNCH(VE, NC, KM, TT)                                                                                     \
   do {                                                                                                                \
     dim3 grid(mx_tile_count(S, rows, max_len, TT, 6), (units + CH_WAVES - 1) / CH_WAVES);                             \
@@ -173,7 +219,9 @@ MX_API int mx_conv_heads(const void* in, long si, int dt, const float* w, int K,
   } while (0)
 #define CH_TAPS(VE, NC)                     \
   do {                                      \
-    if (K <= 4) CH_LAUNCH(VE, NC, 4, 8);    \
+    if (K <= 4 && max_len == 1) CH_LAUNCH(VE, NC, 4, 1); \
+    else if (K <= 4 && rows * (long)units < 24000) CH_LAUNCH(VE, NC, 4, 4); \
+    else if (K <= 4) CH_LAUNCH(VE, NC, 4, 8); \
     else if (K <= 8) CH_LAUNCH(VE, NC, 8, 8); \
     else CH_LAUNCH(VE, NC, 16, 16);         \
   } while (0)

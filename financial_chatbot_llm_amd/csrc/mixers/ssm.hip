@@ -77,26 +77,34 @@ __global__ void conv_silu_kernel(const T* __restrict__ in, long si, const float*
   }
 }
 
-// The same for K = 4 taps and channels by fours (grid ceil(C/1024)): the inputs of eight tokens are fetched together.
-// Bound by memory (4096 rows of 4608 bf16 channels: 41 us, one channel per thread and one input in flight 62).
-constexpr int CONV_V = 8;
-
-template <typename T>
+// The same for K = 4 taps and channels by fours, TT tokens of a segment per thread (grid ceil(C/1024)): every load of a thread, the
+// next history's included, is issued before the first is used, so that a tile takes one trip to memory.
+template <typename T, int TT>
 __global__ void __launch_bounds__(256) conv4_kernel(const T* __restrict__ in, long si, const float* __restrict__ w,
                                                     const float* __restrict__ bias, const float* __restrict__ in_bias, int act,
                                                     float* state, const int* __restrict__ cu,
                                                     const int* __restrict__ slot, const int* __restrict__ pos,
                                                     float* __restrict__ out, int S, int per, int C) {
+  static_assert(TT == 1 || TT >= 3, "a tile behind a segment's first reads three rows back; single-row tiles are for segments of one row");
   int s, t0;
-  if (!mx_tile_place<1>(cu, S, per, CONV_TT, blockIdx.z * gridDim.y + blockIdx.y, s, t0)) return;
+  if (!mx_tile_place<1>(cu, S, per, TT, blockIdx.z * gridDim.y + blockIdx.y, s, t0)) return;
   const int sl = slot[s];
   if (sl < 0) return;
   const int r0 = cu[s], n = cu[s + 1] - r0;
   const int c = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (c >= C) return;
-  const bool fresh = pos[r0] == 0;
+  const bool fresh = pos[r0] == 0, first = t0 == 0;
+  float* st = state + (long)sl * 3 * C + c;
+  const T* seg = in + (long)r0 * si + c;
   const mx_f32x4 zero = mx_f32x4{0.f, 0.f, 0.f, 0.f};
-  const mx_f32x4 ib = in_bias != nullptr ? ldf4(in_bias + c) : zero;   // added to every real input (not to the history)
+  mx_f32x4 x[TT + 3], h[3];              // x[k]: the input at local index t0 - 3 + k; h[j]: the next history
+#pragma unroll
+  for (int i = 0; i < TT; ++i) x[3 + i] = ldf4(seg + min(t0 + i, n - 1) * si);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) x[k] = first ? (fresh ? zero : ldf4(st + (long)k * C)) : ldf4(seg + max(t0 - 3 + k, 0) * si);
+  if (first)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) h[j] = ldf4(seg + max(n - 3 + j, 0) * si);
   mx_f32x4 wk[4];                        // weights [C][4]: channel c + e, tap k
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -104,42 +112,26 @@ __global__ void __launch_bounds__(256) conv4_kernel(const T* __restrict__ in, lo
 #pragma unroll
     for (int k = 0; k < 4; ++k) wk[k][e] = r[k];
   }
+  const mx_f32x4 ib = in_bias != nullptr ? ldf4(in_bias + c) : zero;   // added to every real input (not to the history)
   const mx_f32x4 b = bias != nullptr ? ldf4(bias + c) : zero;
-  mx_f32x4 x[CONV_V + 3];                // x[k]: the input at local index i0 - 3 + k
+  if (first) {                           // x[0 .. 2] is the history: entry j takes input n - 3 + j, or entry j + n of before
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    const int j = t0 - 3 + k;
-    x[k] = zero;
-    if (j >= 0) x[k] = ldf4(in + (long)(r0 + j) * si + c) + ib;
-    else if (!fresh) x[k] = ldf4(state + ((long)sl * 3 + 3 + j) * C + c);
+    for (int j = 0; j < 3; ++j) stf4(st + (long)j * C, n - 3 + j >= 0 ? h[j] + ib : (j + n == 1 ? x[1] : x[2]));
+  } else {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) x[k] += ib;
   }
-  if (t0 == 0) {                         // x[0 .. 2] is the history
-    float* st = state + (long)sl * 3 * C + c;
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const int i = n - 3 + j;
-      const mx_f32x4 old = j + n == 1 ? x[1] : x[2];       // entry j + n, 1 or 2
-      stf4(st + (long)j * C, i >= 0 ? ldf4(in + (long)(r0 + i) * si + c) + ib : old);
+  for (int i = 0; i < TT; ++i) {
+    x[3 + i] += ib;
+    mx_f32x4 y = b;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) y += wk[k] * x[i + k];
+    if (act == 1) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = mx_silu(y[e]);
     }
-  }
-  const int t1 = min(t0 + CONV_TT, n);
-  for (int i0 = t0; i0 < t1; i0 += CONV_V) {
-#pragma unroll
-    for (int i = 0; i < CONV_V; ++i) x[3 + i] = ldf4(in + (long)(r0 + min(i0 + i, n - 1)) * si + c);
-#pragma unroll
-    for (int i = 0; i < CONV_V; ++i) {
-      x[3 + i] += ib;
-      mx_f32x4 y = b;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) y += wk[k] * x[i + k];
-      if (act == 1) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) y[e] = mx_silu(y[e]);
-      }
-      if (i0 + i < t1) stf4(out + (long)(r0 + i0 + i) * C + c, y);
-    }
-#pragma unroll
-    for (int k = 0; k < 3; ++k) x[k] = x[CONV_V + k];
+    if (t0 + i < n) stf4(out + (long)(r0 + t0 + i) * C + c, y);
   }
 }
 
@@ -668,25 +660,33 @@ ssd_scan_kernel(const float* __restrict__ u, int C, const float* __restrict__ Dp
 
 // in: [rows, C] slice (row stride si) of the in-projection; out: f32 [rows, C]; state f32 [slots, K-1, C]
 // act: 0 none, 1 SiLU; in_bias (optional, [C]) is added to every input before the convolution; rows: those of the step
-// By four channels (conv4_kernel) from where memory is the bound: a quarter of the threads with eight inputs each in flight is
-// the slower start for less, and for segments of fewer than eight tokens (bf16, us, by one / by four: 64 single rows of 4608
-// 7.1 / 11.0; 512 rows of 4608 15.6 / 17.1; 1024 19.1 / 18.9; 2048 rows of 8192 36 / 28; 512 segments of 4 rows of 4608 38 / 40).
+// Four taps go by four channels (conv4_kernel), tokens per thread by size: the fewer the shorter a tile's way, the more the fewer
+// halo rows are read again once memory is the bound, and single rows need no tile (bf16, us, one channel and 32 tokens a thread in
+// turn / 1 or 4 tokens / 8 / 16: 64 single rows of 4608 4.8 / 4.1, 512 20.4 / 12.4; one segment of 100 rows 11.8 / 4.4 / 5.6 / 8.1, 400
+// 12.7 / 5.9 / 6.5 / 8.9, 800 14.2 / 9.3 / 9.4 / 10.2, 2048 22.9 / 19.3 / 18.2 / 19.6; 5065 rows behind their projection 41.4 with four
+// channels and 32 tokens in turn, here by 8 38.9).
 MX_API int mx_conv_act(const void* in, long si, int dt, const float* w, const float* bias, const float* in_bias, int act,
                        float* state, const int* cu, const int* slot, const int* pos, float* out, int S, int max_len,
                        int rows, int C, int K, hipStream_t st) {
   if (S <= 0 || max_len <= 0) return 0;
   if (K < 1 || K > MAX_TAPS || act < 0 || act > 1) return (int)hipErrorInvalidValue;
-  const int per = mx_tile_per(S, rows, max_len, CONV_TT, 4), tiles = mx_tile_count(S, rows, max_len, CONV_TT, 4);
-  const int tz = (tiles + 65534) / 65535, ty = (tiles + tz - 1) / tz;
-  if (K == 4 && C % 4 == 0 && rows >= 8L * S && (long)rows * C >= 4500000 && mx_by_four(in, si, dt) &&
+  auto grid = [&](int nx, int tt) {
+    const int tiles = mx_tile_count(S, rows, max_len, tt, 4), tz = (tiles + 65534) / 65535;
+    return dim3(nx, (tiles + tz - 1) / tz, tz);
+  };
+  if (K == 4 && C % 4 == 0 && mx_by_four(in, si, dt) &&
       ((size_t)w | (size_t)bias | (size_t)in_bias | (size_t)state | (size_t)out) % 16 == 0) {
-    const dim3 grid((C / 4 + 255) / 256, ty, tz);
-    MX_DISPATCH(dt, TT, conv4_kernel<TT><<<grid, 256, 0, st>>>((const TT*)in, si, w, bias, in_bias, act, state, cu, slot, pos,
-                                                               out, S, per, C));
+#define CONV4(TT)                                                                                                                  \
+  MX_DISPATCH(dt, TY, conv4_kernel<TY, TT><<<grid((C / 4 + 255) / 256, TT), 256, 0, st>>>((const TY*)in, si, w, bias, in_bias, act, state, cu, \
+                                                                                          slot, pos, out, S, mx_tile_per(S, rows, max_len, TT, 4), C))
+    const long size = (long)rows * C;
+    if (max_len == 1) CONV4(1);
+    else if (size < 8000000 || rows < 8L * S) CONV4(4);
+    else CONV4(8);
+#undef CONV4
   } else {
-    const dim3 grid((C + 255) / 256, ty, tz);
-    MX_DISPATCH(dt, TT, conv_silu_kernel<TT><<<grid, 256, 0, st>>>((const TT*)in, si, w, bias, in_bias, act, state, cu,
-                                                                   slot, pos, out, S, per, C, K));
+    MX_DISPATCH(dt, TT, conv_silu_kernel<TT><<<grid((C + 255) / 256, CONV_TT), 256, 0, st>>>((const TT*)in, si, w, bias, in_bias, act, state, cu,
+                                                                   slot, pos, out, S, mx_tile_per(S, rows, max_len, CONV_TT, 4), C, K));
   }
   MX_RETURN_LAUNCH();
 }

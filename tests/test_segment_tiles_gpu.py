@@ -95,3 +95,61 @@ def test_attention(name):
         return mx.window_attend(f(q), f(cache), f(cu), f(pos), f(bt), 50, D ** -0.5, max(lens), H, G, D, D)
     want, got = run(lambda t: t.float() if t.is_floating_point() else t), run(lambda t: t.cuda()).float().cpu()
     assert ((got - want).abs() <= want.abs() * 2.0 ** -8 + 5 * 2.0 ** -19).all()
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("lens,C", [([1] * 300, 1028), ([2, 1, 5], 2048), ([1000, 3, 1, 9], 8192)])
+def test_convolution_rows_per_thread(lens, C, dt):
+    """Single rows, and sizes at which a thread has 4 and 8 rows; histories of segments shorter than the taps among them."""
+    T, S, K = sum(lens), len(lens), 4
+    g = torch.Generator().manual_seed(T)
+    x, w, b = torch.randn((T, C), generator=g).to(dt), torch.randn((C, K), generator=g), torch.randn(C, generator=g)
+    st, slot = torch.randn((S, K - 1, C), generator=g), torch.randperm(S, generator=g).int()
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    pos = torch.cat([torch.arange(n) + (9 if i % 2 else 0) for i, n in enumerate(lens)]).int()
+    want_st, got_st = st.clone(), st.cuda()
+    want = mx.conv_silu(x, w, b, want_st, cu, slot, pos, max(lens))
+    got = mx.conv_silu(x.cuda(), w.cuda(), b.cuda(), got_st, cu.cuda(), slot.cuda(), pos.cuda(), max(lens))
+    assert torch.allclose(got.cpu(), want, rtol=1e-4, atol=1e-4)           # f32 sums of four terms, SiLU by the fast exponential
+    assert torch.equal(got_st.cpu(), want_st)
+
+
+@pytest.mark.parametrize("K", [3, 4, 7, 9])
+@pytest.mark.parametrize("lens", [[1] * 40, [2, 1, 5, 60], [2390, 1, 9, 2]])
+def test_conv_heads_rows_per_wave(lens, K):
+    """Single rows, and both numbers of rows per wave; histories of segments shorter than the taps among them."""
+    T, S, H, G, D, P = sum(lens), len(lens), 6, 2, 24, 20
+    C = (H + G) * D + G * P
+    g = torch.Generator().manual_seed(T + K)
+    x, w, n = torch.randn((T, C), generator=g), torch.randn((C, K), generator=g), torch.rand(D, generator=g)
+    st, slot, slots = torch.randn((S, K - 1, C), generator=g), torch.randperm(S, generator=g).int(), torch.randperm(T, generator=g).int()
+    slots[T // 2] = -1
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    pos = torch.cat([torch.arange(m) + (9 if i % 2 else 0) for i, m in enumerate(lens)]).int()
+
+    def run(f, st, cache):
+        return mx.conv_heads(f(x), f(w), st, f(n), f(n), 1e-5, f(cu), f(slot), f(pos), f(slots), cache, max(lens), H, G, D, P, 0.1, 16)
+    want_st, want_c, got_st, got_c = st.clone(), torch.zeros(T, G * (D + P)), st.cuda(), torch.zeros(T, G * (D + P), device="cuda")
+    want, got = run(lambda t: t, want_st, want_c), run(lambda t: t.cuda(), got_st, got_c)
+    assert torch.allclose(got.cpu(), want, rtol=1e-4, atol=1e-4) and torch.allclose(got_c.cpu(), want_c, rtol=1e-4, atol=1e-4)
+    assert torch.equal(got_st.cpu(), want_st)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("W", [6, 8, 1100])
+@pytest.mark.parametrize("lens", [[1] * 40, [1, 9, 0, 3], [401] + [1] * 40 + [0, 7]])      # the last: more than 16384 blocks of one row
+def test_embed_pairs(lens, W, dt):
+    T, S, V, B = sum(lens), len(lens), 50, 13
+    g = torch.Generator().manual_seed(T + W)
+    table, pairs = torch.randn((V, W), generator=g).to(dt), torch.randn((B + 1, W), generator=g).to(dt)
+    ids, last = torch.randint(0, V, (T,), generator=g).int(), torch.randint(0, V, (S,), generator=g).int()
+    slot = torch.randperm(S, generator=g).int()
+    slot[1] = -1
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    pos = torch.cat([torch.arange(m) + (9 if i % 2 else 0) for i, m in enumerate(lens)]).int()
+    want_last, got_last = last.clone(), last.cuda()
+    want = mx.embed_pairs(ids, table, pairs, 3, 4, want_last, cu, slot, pos, max(lens))
+    got = mx.embed_pairs(ids.cuda(), table.cuda(), pairs.cuda(), 3, 4, got_last, cu.cuda(), slot.cuda(), pos.cuda(), max(lens))
+    live = torch.ones(T, dtype=torch.bool)
+    live[int(cu[1]):int(cu[2])] = False                                     # a segment without a slot is padding
+    assert torch.equal(got.cpu()[live], want[live]) and torch.equal(got_last.cpu(), want_last)
