@@ -21,6 +21,7 @@
 //     sums the S slabs, which costs S*4 B per output instead of a 1.5-2 us kernel boundary.
 #include "common.h"
 
+#include <cfloat>
 #include <utility>
 
 typedef __attribute__((address_space(3))) void lds_void_t;
@@ -687,7 +688,7 @@ constexpr RowsTile kRowsTiles[] = {{2, 2, 4.6f, 13.6f}, {2, 4, 6.5f, 23.4f}, {4,
 
 }  // namespace
 
-// The tile and split of penny_linear_rows for M rows: nf | mt << 8 | S << 16, or 0 where the library's product is to be taken.
+// The tile and split of penny_linear_rows for M rows: nf | mt << 8 | S << 16, or 0 where another product is to be taken (best: its time).
 //
 // A block's ring takes a CU's LDS, so the blocks run in rounds of 256, each round for as long as its tile's K: a product is the
 // faster the smaller the tile, as long as one round holds all blocks; with few blocks K is cut in 2 or 4 (a second launch and
@@ -706,10 +707,10 @@ constexpr RowsTile kRowsTiles[] = {{2, 2, 4.6f, 13.6f}, {2, 4, 6.5f, 23.4f}, {4,
 // 2048 x 1024 16 rows 8.8 / 6.9; 1024 x 3072 10.9 / 9.0), so up to 256 rows the products of up to 11 us are taken.  Steps at width 1024: 14
 // rows decoding 956 -> 812, 50 1023 -> 916; 200 tokens, where the host is the bound, 1575 -> 1355.  Errors against 64 bits at most the library's
 // (K = 1024 1.6 - 2.9e-7 of the norm against 2.9 - 5.8e-7, K = 3072 2.0 - 2.6e-7 against 5.0e-7).
-PENNY_API int penny_linear_rows_plan(int M, int N, int K, int f32) {
+static int rows_plan(int M, int N, int K, int f32, float& best) {
   if (M <= 0 || M > (f32 ? 256 : 2048) || N < 512 || N % 16 || K <= 0 || K % (f32 ? 32 : 64)) return 0;
   int plan = 0;
-  float best = f32 ? 11.f : M <= 96 ? 60.f : M <= 512 ? 20.f : 20.f - (M - 512) / 128.f;
+  best = f32 ? 11.f : M <= 96 ? 60.f : M <= 512 ? 20.f : 20.f - (M - 512) / 128.f;
   for (int S = 1; S <= (f32 ? 8 : 4); S *= 2) {
     if (S > 1 && (K % (64 * S) || K / S < 256)) break;
     for (int i = 0; i < (f32 ? 4 : (int)(sizeof(kRowsTiles) / sizeof(kRowsTiles[0]))); ++i) {
@@ -721,6 +722,16 @@ PENNY_API int penny_linear_rows_plan(int M, int N, int K, int f32) {
     }
   }
   return plan;
+}
+
+PENNY_API int penny_linear_rows_plan(int M, int N, int K, int f32) {
+  float us;
+  return rows_plan(M, N, K, f32, us);
+}
+// the estimate of the plan for bf16, FLT_MAX where there is none
+extern "C" float penny_linear_rows_us(int M, int N, int K) {
+  float us;
+  return rows_plan(M, N, K, 0, us) ? us : FLT_MAX;
 }
 
 // The same for launches that a graph replays, where the host's share of a library call does not count: only what the device runs faster.

@@ -146,3 +146,67 @@ def test_transformed_calls():
     assert isinstance(logits(torch.nn.Parameter(h[0], requires_grad=False)), torch.Tensor) and logits(h[0]).dtype == torch.float32
     with torch.autocast("cuda", dtype=torch.bfloat16):
         assert logits(h[0]).dtype == torch.bfloat16
+
+
+RING = [(64, 64, 4), (64, 128, 4), (128, 64, 2), (128, 96, 2), (128, 128, 2), (128, 160, 2), (128, 192, 2), (128, 256, 2), (256, 128, 1), (256, 160, 1)]
+
+
+@pytest.mark.parametrize("tile", range(1, 11))
+def test_ring_tiles(tile):
+    """Each tile with less than one of it, whole ones and part-filled ones on both sides; K of one step, fewer than the ring's stages and more; strided
+    rows; nothing written behind the result."""
+    from financial_chatbot_llm_amd.ops import _native as N
+    tn, tm, kg = RING[tile - 1]
+    g = torch.Generator().manual_seed(tile)
+    for M, N_ in ((1, 8), (tm, tn), (tm + 1, tn + 8), (9 * tm - 15, 2 * tn - 24), (3 * tm + 16, 5 * tn + 64)):
+        for K in sorted({32 * max(kg, 2), 64 * max(kg, 2), 384, 1152}):
+            x = torch.randn((M, K + 8), generator=g).bfloat16().cuda()[:, :K]
+            w = (torch.randn((N_, K), generator=g) * K ** -0.5).bfloat16().cuda()
+            y = torch.full((M + 1, N_), 7.0, dtype=torch.bfloat16, device="cuda")
+            N.call("penny_linear_ring", N.ptr(x), K + 8, N.ptr(w), K, N.ptr(y), M, N_, tile, N.stream())
+            want = x.double() @ w.double().t()
+            # one rounding to eight significant bits; f32 sums of K products of values of order K^-0.5, as above
+            assert ((y[:M].double() - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -18 * K ** 0.5).all(), (M, N_, K)
+            assert (y[M] == 7).all()
+    for bad in ((K + 4, 64, K), (K + 8, 60, K), (K + 8, 64, K - 32), (64, 64, K)):
+        with pytest.raises(RuntimeError):
+            N.call("penny_linear_ring", N.ptr(x), bad[0], N.ptr(w), bad[2], N.ptr(y), 1, bad[1], tile, N.stream())
+
+
+def test_ring_rule():
+    """One round of blocks, and the shortest: the streaming tiles and the library keep the rest."""
+    from financial_chatbot_llm_amd.ops import _native as N
+    plan = N.load().penny_linear_ring_plan
+    assert plan(1188, 2048, 2048) == 4 and plan(400, 7216, 2048) == 5 and plan(300, 12288, 2048) > 0 and plan(2600, 2048, 2048) == 7
+    assert plan(256, 2048, 2048) == plan(3073, 1024, 1024) == plan(1000, 12288, 2048) == plan(400, 2044, 2048) == plan(400, 2048, 2080) == 0
+    assert plan(300, 512, 1024) == 0                                    # shorter on the streaming tiles
+    for M in range(257, 3100, 61):
+        for N_ in (512, 1000, 2048, 3208, 7216, 8192, 12864):
+            for K in (64, 192, 1024, 6144):
+                t = plan(M, N_, K)
+                assert t == 0 or (-(-M // RING[t - 1][1]) * -(-N_ // RING[t - 1][0]) <= 256 and K % (32 * RING[t - 1][2]) == 0)
+
+
+@pytest.mark.parametrize("M,N_,K", [(257, 3208, 1024), (400, 7216, 2048), (1188, 2048, 6144), (3072, 1024, 1024)])
+def test_ring_projections(M, N_, K, monkeypatch):
+    """Through ``project``, not-a-numbers and infinities where they belong; rows off the alignment and replays keep their paths."""
+    from financial_chatbot_llm_amd.ops import _native as N
+    calls = []
+    call = N.call
+    monkeypatch.setattr(N, "call", lambda name, *a: (calls.append(name), call(name, *a))[1])
+    g = torch.Generator(device="cuda").manual_seed(M)
+    w = (torch.randn((N_, K), generator=g, device="cuda") * K ** -0.5).bfloat16()
+    rows = torch.randn((M, K + 8), generator=g, device="cuda").bfloat16()
+    for off in (0, 8, 4):
+        x = rows[:, off:off + K]
+        x[5, 7], x[M - 1, K - 1] = float("nan"), float("inf")
+        calls.clear()
+        y, want = G.project(x, w), x.double() @ w.double().t()
+        assert calls == (["penny_linear_ring"] if off % 8 == 0 else [])
+        assert y[5].isnan().all() and torch.allclose(y[M - 1].double(), want[M - 1], equal_nan=True)
+        y[5] = y[M - 1] = want[5] = want[M - 1] = 0
+        assert ((y.double() - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -18 * K ** 0.5).all()
+    with G.replayed():
+        calls.clear()
+        G.project(rows[:, :K], w)
+        assert "penny_linear_ring" not in calls
