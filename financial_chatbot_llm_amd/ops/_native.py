@@ -45,7 +45,11 @@ _SIGS = {
     "penny_linear_rows_plan": [c_int, c_int, c_int, c_int],
     "penny_linear_rows_replay_plan": [c_int, c_int, c_int, c_int],
     "penny_linear_ring_plan": [c_int, c_int, c_int],
-    "penny_linear_ring": [P, c_int, P, c_int, P, c_int, c_int, c_int, P],
+    "penny_ring_slabs_plan": [c_int, c_int, c_int, c_int],
+    "penny_ring_slabs": [P, c_int, P, c_int, P, c_int, c_int, c_int, c_int, P],
+    "penny_qkv_ring_plan": [c_int, c_int, c_int],
+    "penny_qkv_ring": [P, c_int, P, c_int, c_int, P, P, P, P, P, P, c_int, c_int, c_float, c_int, P],
+    "penny_linear_ring": [P, c_int, P, c_int, P, c_int, P, c_int, c_int, c_int, c_int, P],
     "penny_linear_rows": [P, c_int, P, c_int, P, c_int, c_int, P, c_int, c_int, c_int, c_int, c_int, P],
     "penny_lm_head_stream_sample": [P, c_int, P, c_int, c_int, c_int, c_int, c_int, P, P, P, P, P, c_int, c_int,
                                     c_int, P],

@@ -89,6 +89,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, epilogue: Optional[str] = None,
     if M > 256 and prefill_ok(x, w) and epilogue in (None, "silu", "residual"):
         fr = fuse_residual is not None and epilogue is None and residual is None
         c = prefill_choice(M, N_, K, epilogue, slabs and residual is None, fused_residual=fr)
+        # (slabs beyond 24 MB take longer than the sum in place: 4096 x 4096, 640 rows 34.7 / 35.4 us, 768 38.4 / 36.5, 1024 48.0 / 41.4)
+        tile = _ring_residual(x, w, fuse_residual) if fr and (c[0] != "M" or int(c[1:]) * M * N_ > 6 << 20) else 0
+        if tile:
+            N.call("penny_linear_ring", N.ptr(x), x.stride(0), N.ptr(w), K, N.ptr(fuse_residual), fuse_residual.stride(0), N.ptr(fuse_residual),
+                   fuse_residual.stride(0), M, N_, tile, N.stream())
+            return ResidualSum(fuse_residual)
         if c.startswith("K"):
             return splitk_bf16(x, w, N_, int(c[1:]))
         if c == "R":
@@ -99,6 +105,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, epilogue: Optional[str] = None,
         if c.startswith("S"):
             return Slabs(prefill_gemm(x, w, "slabs", int(c[1:])))
         if c.startswith("M"):
+            if slabs and epilogue is None and residual is None and _ring_operands(x, w):
+                tile = N.load().penny_ring_slabs_plan(M, N_, K, int(c[1:]))
+                if tile:
+                    return Slabs(ring_slabs(x, w, int(c[1:]), tile))
             return mid_linear(x, w, int(c[1:]), epilogue, slabs and residual is None, residual)
     # the decode kernels stream either the fragment-tiled copy or (DECODE_WEIGHTS == "rowmajor",
     # or no copy was made) the row-major weight itself
@@ -291,7 +301,7 @@ def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
             tile = lib.penny_linear_ring_plan(M, N_, K) if M > 256 and not (f32 or replay) and M * ldx < 1 << 31 and N_ * K < 1 << 31 else 0
             if tile:
                 y = torch.empty((M, N_), dtype=dt, device=x.device)
-                N.call("penny_linear_ring", xp, ldx, wp, K, y.data_ptr(), M, N_, tile, N.stream())
+                N.call("penny_linear_ring", xp, ldx, wp, K, y.data_ptr(), N_, None, 0, M, N_, tile, N.stream())
                 return y
             plan = lib.penny_linear_rows_replay_plan(M, N_, K, f32) if replay else lib.penny_linear_rows_plan(M, N_, K, f32)
             if plan:
@@ -302,6 +312,36 @@ def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
                        PAIR_MODE != "0", N.stream())
                 return y
     return F.linear(x, w)
+
+
+# Projections that add the residual stream take a single round of ring tiles (penny_linear_ring_plan) up to this K, with the norm behind
+# them, us before / here: 4096 x 4096 (slices of K and slabs to 2048 rows, then 256 x 256 tiles) 374 rows 29.2 / 27.3, 512 32.5 / 28.4, 1024 48.2 /
+# 40.9, 1280 61.6 / 48.7, 2048 77.0 / 69.0, 2133 86.2 / 79.7, 2560 89.0 / 86.2.  A longer K is the shorter in slices: 4096 x 14336 374 rows
+# 72.4 / 92.7, 1024 115 / 141, 2048 201 / 215.
+RING_RESIDUAL_MAX_K = 4096
+
+
+def _ring_operands(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Do the ring tiles read these operands of :func:`prefill_ok` (``PENNY_PREFILL_GEMM=force``: the 256 x 256 tiles take everything)?"""
+    return os.environ.get("PENNY_PREFILL_GEMM", "1") == "1" and x.dtype == w.dtype == torch.bfloat16 and x.shape[0] * x.stride(0) < 1 << 31 and \
+        w.numel() < 1 << 31 and (x.data_ptr() | w.data_ptr()) % 16 == 0
+
+
+def _ring_residual(x: torch.Tensor, w: torch.Tensor, r: torch.Tensor) -> int:
+    """The ring tile for r += x @ w.T in place, or 0 (operands of :func:`prefill_ok`)."""
+    (M, K), N_ = x.shape, w.shape[0]
+    if K > RING_RESIDUAL_MAX_K or r.shape != (M, N_) or r.dtype != torch.bfloat16 or r.stride(1) != 1 or r.stride(0) % 8 or r.data_ptr() % 16 or \
+            not _ring_operands(x, w):
+        return 0
+    return N.load().penny_linear_ring_plan(M, N_, K)
+
+
+def ring_slabs(x: torch.Tensor, w: torch.Tensor, S: int, tile: int) -> torch.Tensor:
+    """f32 split-K partials [S, M, N] of x @ w.T on a tile of the ring (``penny_ring_slabs_plan``)."""
+    (M, K), N_ = x.shape, w.shape[0]
+    P = torch.empty((S, M, N_), dtype=torch.float32, device=x.device)
+    N.call("penny_ring_slabs", N.ptr(x), x.stride(0), N.ptr(w), K, N.ptr(P), M, N_, S, tile, N.stream())
+    return P
 
 
 FEW_FORMS = {"slab": 0, "add": 1, "silu": 2}
@@ -957,6 +997,11 @@ def prefill_qkv_rope(x: torch.Tensor, w: torch.Tensor, positions: torch.Tensor, 
         qr = _rope_ref(qkv[:, :Hq * 128].float().view(M, Hq, 128), positions, cos_sin)   # f32
         return (qr * qscale).to(x.dtype)
     q = torch.empty((M, Hq, 128), dtype=x.dtype, device=x.device)
+    tile = N.load().penny_qkv_ring_plan(M, w.shape[0], K) if _ring_operands(x, w) and cos_sin.data_ptr() % 16 == 0 else 0
+    if tile:
+        N.call("penny_qkv_ring", N.ptr(x), x.stride(0), N.ptr(w), K, M, N.ptr(positions), N.ptr(cos_sin), N.ptr(slots), N.ptr(q), N.ptr(k_cache),
+               N.ptr(v_cache), Hq, Hkv, float(qscale), tile, N.stream())
+        return q
     N.call("penny_gemm_prefill_qkv_rope", N.ptr(x), x.stride(0), N.ptr(w), K, M, N.ptr(positions), N.ptr(cos_sin),
            N.ptr(slots), N.ptr(q), N.ptr(k_cache), N.ptr(v_cache), Hq, Hkv, float(qscale), *tail_workspace(x.device),
            N.stream())

@@ -163,14 +163,18 @@ def test_ring_tiles(tile):
             x = torch.randn((M, K + 8), generator=g).bfloat16().cuda()[:, :K]
             w = (torch.randn((N_, K), generator=g) * K ** -0.5).bfloat16().cuda()
             y = torch.full((M + 1, N_), 7.0, dtype=torch.bfloat16, device="cuda")
-            N.call("penny_linear_ring", N.ptr(x), K + 8, N.ptr(w), K, N.ptr(y), M, N_, tile, N.stream())
+            N.call("penny_linear_ring", N.ptr(x), K + 8, N.ptr(w), K, N.ptr(y), N_, None, 0, M, N_, tile, N.stream())
             want = x.double() @ w.double().t()
             # one rounding to eight significant bits; f32 sums of K products of values of order K^-0.5, as above
             assert ((y[:M].double() - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -18 * K ** 0.5).all(), (M, N_, K)
             assert (y[M] == 7).all()
+            r = torch.randn((M, N_ + 16), generator=g).bfloat16().cuda()[:, :N_]
+            want = (y[:M].float() + r.float()).bfloat16()           # added to the rounded product, in place
+            N.call("penny_linear_ring", N.ptr(x), K + 8, N.ptr(w), K, N.ptr(r), N_ + 16, N.ptr(r), N_ + 16, M, N_, tile, N.stream())
+            assert torch.equal(r, want)
     for bad in ((K + 4, 64, K), (K + 8, 60, K), (K + 8, 64, K - 32), (64, 64, K)):
         with pytest.raises(RuntimeError):
-            N.call("penny_linear_ring", N.ptr(x), bad[0], N.ptr(w), bad[2], N.ptr(y), 1, bad[1], tile, N.stream())
+            N.call("penny_linear_ring", N.ptr(x), bad[0], N.ptr(w), bad[2], N.ptr(y), N_, None, 0, 1, bad[1], tile, N.stream())
 
 
 def test_ring_rule():
@@ -210,3 +214,75 @@ def test_ring_projections(M, N_, K, monkeypatch):
         calls.clear()
         G.project(rows[:, :K], w)
         assert "penny_linear_ring" not in calls
+
+
+@pytest.mark.parametrize("tile", range(1, 11))
+def test_ring_slabs(tile):
+    from financial_chatbot_llm_amd.ops import _native as N
+    tn, tm, kg = RING[tile - 1]
+    g = torch.Generator().manual_seed(tile)
+    step = 64 if kg == 1 else 32 * kg
+    for M, N_, S, n in ((1, 8, 1, 1), (tm + 5, tn + 40, 2, 1), (2 * tm + 16, 3 * tn - 8, 3, 7), (tm, tn, 4, 5)):
+        K = S * n * step + (64 - S * n * step % 64) % 64
+        K = K if K % (S * step) == 0 else S * n * step * 2
+        x = torch.randn((M, K + 8), generator=g).bfloat16().cuda()[:, :K]
+        w = (torch.randn((N_, K), generator=g) * K ** -0.5).bfloat16().cuda()
+        P = G.ring_slabs(x, w, S, tile)
+        want = torch.stack([a.double() @ b.double().t() for a, b in zip(x.chunk(S, 1), w.chunk(S, 1))])
+        assert ((P.double() - want).abs() <= 2.0 ** -18 * K ** 0.5 * K ** -0.5 * K ** 0.5).all(), (M, N_, S, K)
+
+
+@pytest.mark.parametrize("tile", range(3, 11))
+@pytest.mark.parametrize("Hq,Hkv,qs", [(2, 1, 1.0), (5, 1, 0.13)])
+def test_qkv_ring(tile, Hq, Hkv, qs):
+    """Rotated queries and the paged caches of every tile that holds a head, against the torch path: part-filled tiles, a last half tile
+    of heads, tokens without a slot."""
+    from financial_chatbot_llm_amd.ops import _native as N
+    tn, tm, kg = RING[tile - 1]
+    g = torch.Generator().manual_seed(tile)
+    K, N_ = 384, (Hq + 2 * Hkv) * 128
+    for M in (1, tm, 2 * tm + 17):
+        x, w = torch.randn((M, K + 8), generator=g).bfloat16(), (torch.randn((N_, K), generator=g) * K ** -0.5).bfloat16()
+        f = torch.rand((300, 64), generator=g) * 6.28
+        cs, pos, nb = torch.cat([f.cos(), f.sin()], 1), torch.randint(0, 300, (M,), generator=g).int(), M // 64 + 2
+        slots = torch.randperm(nb * 64, generator=g)[:M].int()
+        slots[M // 2] = -1
+        kc, vc = (torch.zeros((nb, Hkv, 64 * 128), dtype=torch.bfloat16) for _ in range(2))
+        dk, dv = kc.cuda(), vc.cuda()
+        dx, dw, dc, dp, ds = x.cuda()[:, :K], w.cuda(), cs.cuda(), pos.cuda(), slots.cuda()
+        q = torch.zeros((M + 1, Hq, 128), dtype=torch.bfloat16, device="cuda")
+        N.call("penny_qkv_ring", N.ptr(dx), K + 8, N.ptr(dw), K, M, N.ptr(dp), N.ptr(dc), N.ptr(ds), N.ptr(q), N.ptr(dk), N.ptr(dv), Hq, Hkv,
+               qs, tile, N.stream())
+        want = G.prefill_qkv_rope(x[:, :K], w, pos, cs, slots, kc, vc, Hq, Hkv, qs)
+        # a sum next to the middle of two bf16 values may be rounded either way: their spacing is up to 2^-7 of them.  That of each of
+        # the pair that turns, and of the result
+        turn = torch.cat([want.float()[..., :64], want.float()[..., 64:]], -1).view(M, Hq, 2, 64).norm(dim=2).repeat(1, 1, 2)
+        assert ((q[:M].cpu().float() - want.float()).abs() <= 2.0 ** -7 * (1.5 * turn + want.float().abs()) + 1e-5).all()
+        assert (q[M] == 0).all()
+        assert ((dv.cpu().float() - vc.float()).abs() <= 2.0 ** -7 * vc.float().abs() + 1e-5).all()
+        assert (dk.cpu().float() - kc.float()).norm() <= 2.0 ** -8 * kc.float().norm() and ((dk.cpu() == 0) == (kc == 0)).float().mean() > 0.999
+
+
+def test_qkv_and_slabs_take_the_ring(monkeypatch):
+    from financial_chatbot_llm_amd.ops import _native as N
+    calls = []
+    call = N.call
+    monkeypatch.setattr(N, "call", lambda name, *a: (calls.append(name), call(name, *a))[1])
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x, w = torch.randn((300, 14336), generator=g, device="cuda").bfloat16(), torch.randn((4096, 14336), generator=g, device="cuda").bfloat16()
+    r = torch.randn((300, 4096), generator=g, device="cuda").bfloat16()
+    P = G.linear(x, w, slabs=True, fuse_residual=r)
+    assert calls == ["penny_ring_slabs"] and isinstance(P, G.Slabs) and P.P.shape == (4, 300, 4096)
+    want = x.double() @ w.double().t()
+    assert ((P.P.double().sum(0) - want).norm() / want.norm()) < 5e-6              # f32 sums of 14336 products
+    calls.clear()
+    x, r = (torch.randn((1300, n), generator=g, device="cuda").bfloat16() for n in (14336, 4096))
+    before = r.clone()
+    y = G.linear(x[:, :4096], w[:, :4096].contiguous(), slabs=True, fuse_residual=r)
+    assert calls == ["penny_linear_ring"] and isinstance(y, G.ResidualSum) and y.t is r
+    want = x[:, :4096].double() @ w[:, :4096].double().t()
+    assert ((r.double() - before.double() - want).abs() <= 2.0 ** -7 * (want.abs() + before.double().abs()) + 1e-3).all()
+    monkeypatch.setenv("PENNY_PREFILL_GEMM", "force")
+    calls.clear()
+    G.linear(x[:, :4096], w[:, :4096].contiguous(), slabs=True, fuse_residual=r)
+    assert calls == ["penny_gemm_prefill"]
