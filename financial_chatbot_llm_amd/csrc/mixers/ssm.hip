@@ -370,24 +370,26 @@ ssm_scan_kernel(const float* __restrict__ u, int C, const TD* __restrict__ dt_ra
 //     S  <- e^(c_63) S + sum_s e^(c_63 - c_s) dt_s x_s B_s^T
 // all in f32 (v_mfma_f32_16x16x4_f32; the sums c in f64, so that their differences are good to f32 however far the
 // chunk decays).  Three launches leave to the serial one only products: ssd_scores_kernel makes C . B of a group, which its
-// heads share, and B in operand order; ssd_decay_kernel the factors of every chunk and head, M[t][s] = (C_t . B_s)
+// heads share, and B and C in operand order; ssd_decay_kernel the factors of every chunk and head, M[t][s] = (C_t . B_s)
 // e^(c_t - c_s) dt_s for s <= t (else 0), E[t] = e^(c_t), F[s] = e^(c_63 - c_s) dt_s; then a block of ssd_scan_kernel owns 16
 // value channels of one head and walks the chunks of its segment: wave w owns tokens 16 w .. 16 w + 15 of the outputs and
-// N / 4 columns of the state, which the waves exchange through LDS, one barrier per chunk.  Every operand is read from memory
-// in the register layout of its product -- K index 16 j + 4 g + e of step (j, e) for lane group g on both sides -- and the
-// loads of the next chunk are issued as soon as the registers are free.
-// Bound by the matrix cores (80 of these products per wave and chunk); 2 prompts of 2048, 64 heads of 64 x 128, 2 groups:
-// 188 us in all, with the factors made in the walk, four value blocks and four waves over, 287 us, token by token 858 us.
+// N / 4 columns of the state, which the waves exchange through LDS, one barrier per chunk.  Every operand but the values is read
+// from memory in the register layout of its product -- K index 16 j + 4 g + e of step (j, e) for lane group g on both sides --
+// and the loads of the next chunk are issued as soon as the registers are free; the values come one 16-byte load a thread, two
+// chunks ahead, and turn through LDS.  Bound by the chunk's chain (1.1 us of its 2.6 to 4 are products: 80 per wave);
+// 2 prompts of 2048, 64 heads of 64 x 128, 2 groups: 158 us in all; with C and the values read from their rows, 64 bytes
+// each and far apart, 183; one prompt 106 and 121.  (Waves of their own for the state and the outputs: 3 % less for one prompt,
+// 20 % more for three uneven ones.)
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int SSD_L = 64;           // tokens per chunk
 constexpr int SSD_LEAST = 32;       // shorter segments of a step in chunks go token by token: a chunk costs about 20 steps
 
 __device__ __forceinline__ f32x4 mma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
-// Scratch of a chunk: per group C . B [64][64] (s up to t's tile of 16) and B in
-// operand order [N / 16][4][64 lanes][4 tokens]; per head M in operand order [10 tiles (w, j <= w)][64 lanes][4], E, F.
+// Scratch of a chunk: per group C . B [64][64] (s up to t's tile of 16), B in operand order [N / 16][4][64 lanes][4 tokens] and C
+// in operand order [4][N / 16][64 lanes][4 columns]; per head M in operand order [10 tiles (w, j <= w)][64 lanes][4], E, F.
 constexpr int SSD_HEAD = 10 * 256 + 2 * SSD_L;
-__host__ __device__ inline long ssd_group_floats(int N) { return 64L * SSD_L + 64L * N; }
+__host__ __device__ inline long ssd_group_floats(int N) { return 64L * SSD_L + 2 * 64L * N; }
 __host__ __device__ inline long ssd_chunk_floats(int N, int G, int H) { return G * ssd_group_floats(N) + (long)H * SSD_HEAD; }
 
 // max_len is a bound: the only segment of a step may be of any length, and needs no fourth launch whatever it is
@@ -445,6 +447,9 @@ __global__ void __launch_bounds__(256, 2) ssd_scores_kernel(const float* __restr
 #pragma unroll
     for (int r = 0; r < 4; ++r) cb[(16 * w + 4 * g + r) * SSD_L + 16 * st + c] = a0[r] + a1[r];
   }
+  float* ct = cb + SSD_L * SSD_L + 64 * N;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) *reinterpret_cast<f32x4*>(ct + ((w * NJ + j) * 64 + lane) * 4) = cv[j];
   // B: wave w's tokens 16 w + 4 g + e, column 16 i + c
   float* bt = cb + SSD_L * SSD_L;
   const float* bp = u + inner + grp * N + c;
@@ -510,6 +515,7 @@ ssd_scan_kernel(const float* __restrict__ u, int C, const float* __restrict__ Dp
                 const int* __restrict__ pos, float* __restrict__ y, int H, int P, int G) {
   constexpr int N = 64 * NTW, NJ = N / 16;
   __shared__ __attribute__((aligned(16))) float sbuf[2][16][N + 4];   // the state, [p][n]: rows 4 banks apart
+  __shared__ __attribute__((aligned(16))) float xbuf[2][16][SSD_L + 4];   // a chunk's values, [p][token]
   const int s = blockIdx.z, h = blockIdx.x, p0 = blockIdx.y * 16;
   const int sl = slot[s], r0 = cu[s], n = cu[s + 1] - r0;
   if (sl < 0 || n < ssd_least(gridDim.z)) return;
@@ -520,8 +526,9 @@ ssd_scan_kernel(const float* __restrict__ u, int C, const float* __restrict__ Dp
   const float* base = ws + (long)ssd_first(r0, s) * step;
   const float* bbase = base + grp * ssd_group_floats(N) + SSD_L * SSD_L + (NTW * w * 256 + lane) * 4;
   const float* hbase = base + G * ssd_group_floats(N) + (long)h * SSD_HEAD;
-  const float* ux = u + (long)r0 * C + h * P + p0 + c;
-  const float* uc = u + (long)r0 * C + inner + (G + grp) * N + 4 * g;
+  const int tok = threadIdx.x >> 2, xp = threadIdx.x & 3;              // the token and the four channels whose values this thread fetches
+  const float* ux = u + (long)r0 * C + h * P + p0 + 4 * xp;
+  const float* cbase = base + grp * ssd_group_floats(N) + SSD_L * SSD_L + 64 * N + (NJ * w * 64 + lane) * 4;
   float* sp = state + (((long)sl * H + h) * P + p0 + 4 * g) * N + 16 * NTW * w + c;
   float* yp = y + (long)(r0 + 16 * w + 4 * g) * inner + h * P + p0 + c;
 
@@ -537,9 +544,9 @@ ssd_scan_kernel(const float* __restrict__ u, int C, const float* __restrict__ Dp
   f32x4 cv[NJ], mv[4], xv[4], bv[NTW][4], fv[4], ev;
   float keep;
   auto load_c = [&](int k) {              // k: the chunk (behind the end: the last one again)
-    const float* p = uc + (long)min(k * SSD_L + 16 * w + c, n - 1) * C;
+    const float* p = cbase + min(k, last) * step;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) cv[j] = *reinterpret_cast<const f32x4*>(p + 16 * j);
+    for (int j = 0; j < NJ; ++j) cv[j] = *reinterpret_cast<const f32x4*>(p + 256 * j);
   };
   auto load_m = [&](int k) {
     const float* p = hbase + min(k, last) * step;
@@ -559,27 +566,25 @@ ssd_scan_kernel(const float* __restrict__ u, int C, const float* __restrict__ Dp
     }
     keep = f[SSD_L - 1];
   };
-  auto load_x = [&](int k) {
-    const int t0 = k * SSD_L + 4 * g;
-    if (k < last) {
-      const float* p = ux + (long)t0 * C;
+  f32x4 xr;
+  auto load_x = [&](int k) { xr = *reinterpret_cast<const f32x4*>(ux + (long)min(k * SSD_L + tok, n - 1) * C); };
+  auto put_x = [&](int k) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) xv[j][e] = p[(16 * j + e) * C];
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) xv[j][e] = ux[(long)min(t0 + 16 * j + e, n - 1) * C];
-    }
+    for (int e = 0; e < 4; ++e) xbuf[k & 1][4 * xp + e][tok] = xr[e];
   };
+  load_x(0);
   load_c(0);
   load_m(0);
-  load_x(0);
   load_b(0);
+  put_x(0);
+  load_x(1);
   for (int k = 0; k <= last; ++k) {
     const int b = k & 1, left = n - k * SSD_L;
+    __syncthreads();                      // the state of the last chunk is in sbuf[b], this one's values in xbuf[b]
+#pragma unroll
+    for (int j = 0; j < 4; ++j) xv[j] = *reinterpret_cast<const f32x4*>(&xbuf[b][c][16 * j + 4 * g]);
+    put_x(k + 1);
+    load_x(k + 2);
     // a value that is not finite spoils the tokens from its own on and its row of the state, nothing before
     int bad = SSD_L;
     const f32x4 xt = w == 0 ? xv[0] : (w == 1 ? xv[1] : (w == 2 ? xv[2] : xv[3]));
@@ -592,7 +597,6 @@ ssd_scan_kernel(const float* __restrict__ u, int C, const float* __restrict__ Dp
       const int at = mx_drop_nonfinite(xv[j], g);
       bad = min(bad, at < 16 ? 16 * j + at : SSD_L);
     }
-    __syncthreads();                      // the state of the last chunk is in sbuf[b]
     // what the state before the chunk gives
     f32x4 y0 = {0.f, 0.f, 0.f, 0.f}, y1 = y0;
 #pragma unroll
@@ -635,7 +639,6 @@ ssd_scan_kernel(const float* __restrict__ u, int C, const float* __restrict__ Dp
 #pragma unroll
         for (int i = 0; i < NTW; ++i) st[i] = mma4(a[e], bv[i][j][e], st[i]);
     }
-    load_x(k + 1);
     load_b(k + 1);
     if (__any(bad < SSD_L)) {
 #pragma unroll

@@ -467,7 +467,7 @@ def ssm_scan(u: torch.Tensor, dt_raw: torch.Tensor, dt_bias: torch.Tensor, A_log
         max_len = max_len or T
         ws = None
         if Ns in (64, 128, 256) and _ssm_in_chunks(T, S, max_len, H * P * Ns):          # the factors: ssd_chunk_floats of the kernels
-            ws = torch.empty((max(1, T // 64 + min(S, T // 32)), G * 64 * (64 + Ns) + H * 2688), dtype=torch.float32, device=u.device)
+            ws = torch.empty((max(1, T // 64 + min(S, T // 32)), G * 64 * (64 + 2 * Ns) + H * 2688), dtype=torch.float32, device=u.device)
         N.mcall("mx_ssm_scan", N.ptr(u), C, N.ptr(_rows(dt_raw)), dt_raw.stride(0), _dt(dt_raw), N.ptr(dt_bias),
                 N.ptr(A_log), N.ptr(D), N.ptr(state), N.ptr(cu), N.ptr(slot), N.ptr(pos), N.ptr(y), S, int(max_len), H, P, Ns, G,
                 T, N.ptr(ws), N.stream())
