@@ -167,3 +167,26 @@ def test_projection_form_follows_its_shape():
     from financial_chatbot_llm_amd.ops.gemm import small_bias_wins as small
     assert all(small(*s) for s in ((768, 2304, 768), (768, 768, 3072), (400, 1152, 384), (18, 384, 1536), (64, 8192, 2048), (511, 4096, 1024)))
     assert not any(small(*s) for s in ((769, 768, 768), (512, 1152, 384), (64, 384, 1536), (128, 8192, 2048), (768, 4096, 1024)))
+
+
+def test_activations_of_tile_products_over_all_bf16():
+    """The tile kernel's tables of GELU and SiLU give what the row kernels work out, bit for bit, for every bf16 value."""
+    from financial_chatbot_llm_amd import ops
+    from financial_chatbot_llm_amd.ops import gemm
+    K, M = 128, 257
+    values = torch.arange(1 << 16, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).cuda()
+    # GELU: products of zero, every value as a bias
+    x, w = torch.zeros(M, K, dtype=torch.bfloat16, device="cuda"), torch.zeros(1 << 16, K, dtype=torch.bfloat16, device="cuda")
+    got = gemm.prefill_gemm(x, w, "bias_gelu", bias=values)
+    want = ops.gelu_(values.clone().view(1, -1)).view(-1)
+    assert torch.equal(torch.nan_to_num(got, 7.0), torch.nan_to_num(want, 7.0).expand(M, -1))
+    # SiLU: row m's entries 1 .. 127 of X reach a gate each through unit rows of W, entry 0 is the factor 1.5 of every `up`
+    fin = values[torch.isfinite(values)]
+    fin = torch.cat([fin, fin.new_zeros(-fin.numel() % (K - 1))]).view(-1, K - 1)
+    x = torch.cat([fin.new_full((fin.shape[0], 1), 1.5), fin], 1).contiguous()
+    eye = torch.eye(K, dtype=torch.bfloat16, device="cuda")
+    up = torch.zeros_like(eye)
+    up[:, 0] = 1.0
+    got = gemm.prefill_gemm(x, gemm.interleave16(eye, up).contiguous(), "silu")
+    want = ops.silu_mul(torch.cat([x, x[:, :1].expand(-1, K)], 1).contiguous())
+    assert torch.equal(got, want)
