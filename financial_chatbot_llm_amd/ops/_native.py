@@ -96,7 +96,8 @@ _SIGS = {
     "penny_moe_gemm_fp8": [P, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, P],
     "penny_moe_combine": [P, P, c_int, c_int, c_int, P, P],
     "penny_moe_combine_weighted": [P, P, P, c_int, c_int, c_int, P, P],
-    "penny_filtered_topk": [P, P, P, c_long, c_int, P, P, P, P, c_int, c_int, P, P, P, c_int, P, P, P, P, P],
+    "penny_topk_filter": [P, P, c_long, c_int, P, P, c_int, P, P, c_int, P],
+    "penny_topk_rank": [P, c_int, P, P, c_int, c_int, P, P, P, c_int, P, P, P, P, P],
 }
 
 

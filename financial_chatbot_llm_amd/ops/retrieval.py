@@ -34,21 +34,21 @@ def filtered_topk_ref(corpus, user_codes, dates, queries, q_user, q_floor, ks, k
 # Candidate lists that no call holds: (device, stream, set), at most eight, the longest unused dropped first.  A set serves the
 # calls of one stream, whatever their sizes; a call takes one (or makes it), so two threads never share it, and hands it back
 # when its kernels have left the counters at zero again -- a call that fails does not.
-_Set = Tuple[torch.Tensor, torch.Tensor, torch.Tensor]
+_Set = Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]
 _FREE: List[Tuple[int, int, _Set]] = []
 _LOCK = threading.Lock()
 _KEEP = 8
 
 
 def _take(n: int, device: torch.device, stream: int) -> _Set:
-    """Counters [64, 32] of zeros, rows and scores of at least ``n`` candidates."""
+    """Counters [64, 32] of zeros, rows and scores of at least ``n`` candidates, 64 result counts in pinned host memory."""
     with _LOCK:
         for i, (d, s, ws) in enumerate(_FREE):
             if d == device.index and s == stream and ws[1].numel() >= n:
                 return _FREE.pop(i)[2]
     n = 1 << (n - 1).bit_length()          # few sizes: a smaller call fits behind a larger one
     return (torch.zeros((64, 32), dtype=torch.int32, device=device), torch.empty(n, dtype=torch.int32, device=device),
-            torch.empty(n, dtype=torch.float32, device=device))
+            torch.empty(n, dtype=torch.float32, device=device), torch.empty(64, dtype=torch.int32, pin_memory=True))
 
 
 def _hand_back(ws: _Set, device: torch.device, stream: int) -> None:
@@ -56,6 +56,10 @@ def _hand_back(ws: _Set, device: torch.device, stream: int) -> None:
         # smaller sets of the stream that nobody holds have no use beside this one
         _FREE[:] = [f for f in _FREE if f[:2] != (device.index, stream) or f[2][1].numel() >= ws[1].numel()][1 - _KEEP:]
         _FREE.append((device.index, stream, ws))
+
+
+def _as(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    return t if t.dtype == dtype and t.is_contiguous() else t.to(dtype).contiguous()
 
 
 def filtered_topk(corpus: torch.Tensor, user_codes: torch.Tensor, dates: torch.Tensor, queries: torch.Tensor,
@@ -73,20 +77,21 @@ def filtered_topk(corpus: torch.Tensor, user_codes: torch.Tensor, dates: torch.T
     cap = max(SORT_CAP, min(cap, corpus.shape[0]))
     stream = N.stream()
     ws = _take(nq * cap, corpus.device, stream)
-    counts, cand, scores = ws                                        # the lists: nq rows of cap entries
-    out_ids = torch.empty((nq, kmax), dtype=torch.int32, device=corpus.device)
-    out_scores = torch.empty((nq, kmax), dtype=torch.float32, device=corpus.device)
-    out_count = torch.empty((nq,), dtype=torch.int32, device=corpus.device)
-    oc = torch.empty((nq,), dtype=torch.int32, pin_memory=True)      # written by the kernel itself
-    queries = queries.to(torch.bfloat16).contiguous()
+    counts, cand, scores, oc = ws                                    # the lists: nq rows of cap entries; oc is written by the kernel itself
     # converted inputs bound to names: as N.ptr(x.to(...)) temporaries they would be freed before
     # the launch and the next conversion could reuse (overwrite) their memory on the stream
-    qu, qf, kk = q_user.to(torch.int32).contiguous(), q_floor.to(torch.int64).contiguous(), ks.to(torch.int32).contiguous()
-    N.call("penny_filtered_topk", N.ptr(corpus), N.ptr(user_codes), N.ptr(dates), corpus.shape[0], D,
-           N.ptr(queries), N.ptr(qu), N.ptr(qf), N.ptr(kk), nq, kmax, N.ptr(counts), N.ptr(cand), N.ptr(scores), cap,
-           N.ptr(out_ids), N.ptr(out_scores), N.ptr(out_count), N.ptr(oc), stream)
-    torch.cuda.current_stream(corpus.device).synchronize()
-    for i, c in enumerate(oc.tolist()):  # > SORT_CAP candidates: finish on device with torch.topk
+    qu, qf = _as(q_user, torch.int32), _as(q_floor, torch.int64)
+    dev, cp = corpus.device, counts.data_ptr()
+    N.call("penny_topk_filter", user_codes.data_ptr(), dates.data_ptr(), corpus.shape[0], D, qu.data_ptr(), qf.data_ptr(), nq, cp,
+           cand.data_ptr(), cap, stream)
+    # beside the filter: the results' memory
+    queries, kk = _as(queries, torch.bfloat16), _as(ks, torch.int32)
+    out_ids = torch.empty((nq, kmax), dtype=torch.int32, device=dev)
+    out_scores = torch.empty((nq, kmax), dtype=torch.float32, device=dev)
+    out_count = torch.empty((nq,), dtype=torch.int32, device=dev)
+    N.call("penny_topk_rank", corpus.data_ptr(), D, queries.data_ptr(), kk.data_ptr(), nq, kmax, cp, cand.data_ptr(), scores.data_ptr(),
+           cap, out_ids.data_ptr(), out_scores.data_ptr(), out_count.data_ptr(), oc.data_ptr(), stream)
+    for i, c in enumerate(oc[:nq].tolist()):  # the call has waited for them; > SORT_CAP candidates: finish on device with torch.topk
         if c >= 0:
             continue
         total = -c

@@ -38,6 +38,23 @@ def test_sizes(sizes, N, D):
         assert torch.equal(got[0].cpu()[small], want[0][small])
 
 
+@pytest.mark.parametrize("D", [8, 520, 1024])
+@pytest.mark.parametrize("nq", [1, 3, 17, 64])
+def test_one_block_and_several(nq, D):
+    """Counts around what one block ranks alone, and more queries than a block each: contiguous rows of a user, which hit whole waves."""
+    sizes = ([128, 129, 127, 2, 1000, 257] * 11)[:nq]
+    x, users, dates, q = corpus(sizes, sum(sizes) + 600, D, nq + D)
+    users = users.sort().values
+    who, ks = torch.arange(1, nq + 1, dtype=torch.int32), torch.full((nq,), 200, dtype=torch.int32)
+    for since in (0, 400):
+        floor = torch.full((nq,), since, dtype=torch.int64)
+        want = ops.filtered_topk(x, users, dates, q[:nq], who, floor, ks, 260)
+        for _ in range(2):                                                 # the counters are back at zero
+            got = ops.filtered_topk(*(t.cuda() for t in (x, users, dates, q[:nq], who, floor, ks)), 260)
+            for g, w in zip(got, want):
+                assert torch.equal(g.cpu(), w)
+
+
 def test_not_a_number():
     x, users, dates, q = corpus([200], 300, 64, 7)
     x[users.nonzero().flatten()[:3]] = float("nan")
