@@ -86,6 +86,34 @@ __global__ void __launch_bounds__(1024) moe_route_kernel(const bf16* __restrict_
 //     scatters the pairs into their buckets (order inside a bucket is irrelevant -- rows are
 //     computed independently -- so the result is deterministic per row).
 // ---------------------------------------------------------------------------------------------
+// token t's experts by one wave, lane e holding logit e
+__device__ __forceinline__ void moe_choose(float l, long t, int E, int K, int* __restrict__ pe, float* __restrict__ pw) {
+  const int lane = threadIdx.x & 63;
+  float mx = l;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  float p = lane < E ? __expf(l - mx) : -1.f;
+  if (p != p) p = 0.f;                     // a total order: K experts are chosen whatever the logits
+  float ws = 0.f, mine = 0.f;
+  int myj = -1;
+  for (int j = 0; j < K; ++j) {
+    float bv = p;
+    int bi = lane;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const float ov = __shfl_xor(bv, o, 64);
+      const int oi = __shfl_xor(bi, o, 64);
+      if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
+    }
+    ws += bv;
+    if (lane == bi) { mine = p; myj = j; p = -1.f; }
+  }
+  if (myj >= 0) {
+    pe[t * K + myj] = lane;
+    pw[t * K + myj] = mine / ws;
+  }
+}
+
 template <int CPT>
 __global__ void __launch_bounds__(256) moe_route_quant_kernel(const bf16* __restrict__ x, int ldx, int H,
                                                               const bf16* __restrict__ logits, int E, int K,
@@ -94,31 +122,7 @@ __global__ void __launch_bounds__(256) moe_route_quant_kernel(const bf16* __rest
   __shared__ float red[4];
   const long t = blockIdx.x;
   const int lane = threadIdx.x & 63;
-  if (threadIdx.x < 64) {
-    float l = lane < E ? (float)logits[t * E + lane] : -INFINITY;
-    float mx = l;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    float p = lane < E ? __expf(l - mx) : -1.f;
-    float ws = 0.f, mine = 0.f;
-    int myj = -1;
-    for (int j = 0; j < K; ++j) {
-      float bv = p;
-      int bi = lane;
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(bv, o, 64);
-        const int oi = __shfl_xor(bi, o, 64);
-        if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-      }
-      ws += bv;
-      if (lane == bi) { mine = p; myj = j; p = -1.f; }
-    }
-    if (myj >= 0) {
-      pe[t * K + myj] = lane;
-      pw[t * K + myj] = mine / ws;
-    }
-  }
+  if (threadIdx.x < 64) moe_choose(lane < E ? (float)logits[t * E + lane] : -INFINITY, t, E, K, pe, pw);
   const uint4* xr = reinterpret_cast<const uint4*>(x + t * ldx);
   const int nchunk = H >> 3;
   float a[CPT][8];
@@ -155,10 +159,10 @@ __global__ void __launch_bounds__(256) moe_route_quant_kernel(const bf16* __rest
   }
 }
 
-__global__ void __launch_bounds__(1024) moe_bucket_kernel(const int* __restrict__ pe, const float* __restrict__ pw,
-                                                          int P, int E, int K, int* __restrict__ sorted_tok,
-                                                          float* __restrict__ sorted_w, int* __restrict__ offsets,
-                                                          int* __restrict__ inv) {
+// pairs by their expert: counts, offsets and the scatter (order inside a bucket is irrelevant), by one block
+__device__ __forceinline__ void moe_bucket(const int* __restrict__ pe, const float* __restrict__ pw, int P, int E, int K,
+                                           int* __restrict__ sorted_tok, float* __restrict__ sorted_w,
+                                           int* __restrict__ offsets, int* __restrict__ inv) {
   __shared__ int cnt[64], cur[64];
   for (int e = threadIdx.x; e < E; e += blockDim.x) cnt[e] = 0;
   __syncthreads();
@@ -182,41 +186,157 @@ __global__ void __launch_bounds__(1024) moe_bucket_kernel(const int* __restrict_
   }
 }
 
+__global__ void __launch_bounds__(1024) moe_bucket_kernel(const int* __restrict__ pe, const float* __restrict__ pw,
+                                                          int P, int E, int K, int* __restrict__ sorted_tok,
+                                                          float* __restrict__ sorted_w, int* __restrict__ offsets,
+                                                          int* __restrict__ inv) {
+  moe_bucket(pe, pw, P, E, K, sorted_tok, sorted_w, offsets, inv);
+}
+
 // ---------------------------------------------------------------------------------------------
 // 2. dynamic per-row fp8 quantisation (one workgroup per row; row length multiple of 8)
 // ---------------------------------------------------------------------------------------------
-__global__ void quant_rows_kernel(const bf16* __restrict__ x, int ld, int n, unsigned char* __restrict__ q,
-                                  float* __restrict__ scale) {
-  __shared__ float red[16];
-  const int row = blockIdx.x;
+// The row stays in registers between the two sweeps, its CPT 16-byte pieces of a thread in one trip (96 rows of 14336: 4.8 us; read
+// twice, a piece at a time, 7.1); a row of more than 8 pieces (16384 values) goes through the caches twice.
+__device__ __forceinline__ uint2 fp8_of(const float (&f)[8], float inv) {
+  uint32_t w0 = 0, w1 = 0;
+  w0 = __builtin_amdgcn_cvt_pk_fp8_f32(f[0] * inv, f[1] * inv, w0, false);
+  w0 = __builtin_amdgcn_cvt_pk_fp8_f32(f[2] * inv, f[3] * inv, w0, true);
+  w1 = __builtin_amdgcn_cvt_pk_fp8_f32(f[4] * inv, f[5] * inv, w1, false);
+  w1 = __builtin_amdgcn_cvt_pk_fp8_f32(f[6] * inv, f[7] * inv, w1, true);
+  return make_uint2(w0, w1);
+}
+template <int CPT>
+__global__ void __launch_bounds__(256) quant_rows_kernel(const bf16* __restrict__ x, int ld, int n, unsigned char* __restrict__ q,
+                                                         float* __restrict__ scale) {
+  constexpr bool HELD = CPT > 0;                             // 0: rows of any length
+  __shared__ float red[4];
+  const int row = blockIdx.x, chunks = n / 8;
   const uint4* xr = reinterpret_cast<const uint4*>(x + (long)row * ld);
+  uint4 v[HELD ? CPT : 1];
   float amax = 0.f;
-  for (int c = threadIdx.x; c < n / 8; c += blockDim.x) {
+  auto most = [&](const uint4& u) {
     float f[8];
-    unpack8(xr[c], f);
+    unpack8(u, f);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(f[i]));
+    for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(f[k]));
+  };
+  if constexpr (HELD) {
+    if (chunks > 0) {                                        // behind the row's end its last piece again
+#pragma unroll
+      for (int i = 0; i < CPT; ++i) v[i] = xr[min((int)threadIdx.x + 256 * i, chunks - 1)];
+#pragma unroll
+      for (int i = 0; i < CPT; ++i) most(v[i]);
+    }
+  } else {
+    for (int c = threadIdx.x; c < chunks; c += 256) most(xr[c]);
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
   __syncthreads();
-  amax = 0.f;
-  for (int i = 0; i < (int)(blockDim.x >> 6); ++i) amax = fmaxf(amax, red[i]);
+  amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
   const float s = amax > 0.f ? amax / FP8_MAX : 1.f;
   const float inv = 1.f / s;
   if (threadIdx.x == 0) scale[row] = s;
   uint2* qr = reinterpret_cast<uint2*>(q + (long)row * n);
-  for (int c = threadIdx.x; c < n / 8; c += blockDim.x) {
+  auto put = [&](const uint4& u, int c) {
     float f[8];
-    unpack8(xr[c], f);
-    uint32_t w0 = 0, w1 = 0;
-    w0 = __builtin_amdgcn_cvt_pk_fp8_f32(f[0] * inv, f[1] * inv, w0, false);
-    w0 = __builtin_amdgcn_cvt_pk_fp8_f32(f[2] * inv, f[3] * inv, w0, true);
-    w1 = __builtin_amdgcn_cvt_pk_fp8_f32(f[4] * inv, f[5] * inv, w1, false);
-    w1 = __builtin_amdgcn_cvt_pk_fp8_f32(f[6] * inv, f[7] * inv, w1, true);
-    qr[c] = make_uint2(w0, w1);
+    unpack8(u, f);
+    qr[c] = fp8_of(f, inv);
+  };
+  if constexpr (HELD) {
+#pragma unroll
+    for (int i = 0; i < CPT; ++i)
+      if ((int)threadIdx.x + 256 * i < chunks) put(v[i], threadIdx.x + 256 * i);
+  } else {
+    for (int c = threadIdx.x; c < chunks; c += 256) put(xr[c], c);
   }
+}
+
+// 2a. decode batches: router, choice, quantised row and buckets in one launch, a block per token.  Every block reads the router
+//     (8 experts of 4096: 64 KB) from the caches; logits are f32 sums rounded to bf16, as a bf16 product's.  The block that draws the
+//     last ticket sorts the pairs into their buckets.  48 tokens: 9 us, for the library's product (13.4), moe_route_kernel (9) and
+//     quant_rows_kernel (4.6).
+template <int CPT, int EM>
+__global__ void __launch_bounds__(256) moe_decode_route_kernel(const bf16* __restrict__ x, int ldx, int H, const bf16* __restrict__ rw,
+                                                               int T, int E, int K, unsigned char* __restrict__ q,
+                                                               float* __restrict__ scale, int* pe, float* pw, int* ticket,
+                                                               int* __restrict__ sorted_tok, float* __restrict__ sorted_w,
+                                                               int* __restrict__ offsets, int* __restrict__ inv_pos) {
+  __shared__ float red[4], part[4][EM];
+  __shared__ int last;
+  const long t = blockIdx.x;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, chunks = H / 8;
+  const uint4* xr = reinterpret_cast<const uint4*>(x + t * ldx);
+  uint4 v[CPT];
+#pragma unroll
+  for (int i = 0; i < CPT; ++i) {
+    const int c = threadIdx.x + 256 * i;
+    v[i] = c < chunks ? xr[c] : uint4{0, 0, 0, 0};
+  }
+  float amax = 0.f, sum[EM];
+#pragma unroll
+  for (int e = 0; e < EM; ++e) sum[e] = 0.f;
+#pragma unroll
+  for (int i = 0; i < CPT; ++i) {
+    const int c = min((int)threadIdx.x + 256 * i, chunks - 1);
+    uint4 r[EM];
+#pragma unroll
+    for (int e = 0; e < EM; ++e) r[e] = reinterpret_cast<const uint4*>(rw + (long)min(e, E - 1) * H)[c];
+    float f[8];
+    unpack8(v[i], f);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(f[k]));
+    if ((int)threadIdx.x + 256 * i >= chunks) continue;      // (not 0 x a weight, which may be infinite)
+#pragma unroll
+    for (int e = 0; e < EM; ++e) {
+      float g[8];
+      unpack8(r[e], g);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) sum[e] += f[k] * g[k];
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+#pragma unroll
+  for (int e = 0; e < EM; ++e) sum[e] = wave_sum(sum[e]);
+  if (lane == 0) {
+    red[w] = amax;
+#pragma unroll
+    for (int e = 0; e < EM; ++e) part[w][e] = sum[e];
+  }
+  __syncthreads();
+  if (w == 0) {
+    const int e = min(lane, EM - 1);
+    const float l = (float)(bf16)((part[0][e] + part[1][e]) + (part[2][e] + part[3][e]));
+    moe_choose(lane < E ? l : -INFINITY, t, E, K, pe, pw);
+  }
+  amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  const float s = amax > 0.f ? amax / FP8_MAX : 1.f;
+  const float inv = 1.f / s;
+  if (threadIdx.x == 0) scale[t] = s;
+  uint2* qr = reinterpret_cast<uint2*>(q + t * (long)H);
+#pragma unroll
+  for (int i = 0; i < CPT; ++i) {
+    const int c = threadIdx.x + 256 * i;
+    if (c >= chunks) continue;
+    float f[8];
+    unpack8(v[i], f);
+    qr[c] = fp8_of(f, inv);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (threadIdx.x == 0) {                                    // of the wave that stored the pairs
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    last = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == T - 1;
+    if (last) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      *ticket = 0;                                           // for the next launch
+    }
+  }
+  __syncthreads();
+  if (last) moe_bucket(pe, pw, T * K, E, K, sorted_tok, sorted_w, offsets, inv_pos);
 }
 
 // 2b. prefill experts: SiLU(gate) * up of the 16-row-interleaved W13 GEMM output, quantised per row
@@ -438,6 +558,33 @@ PENNY_API int penny_moe_route_quant(const void* x, int ldx, const void* logits, 
   PENNY_RETURN_LAUNCH();
 }
 
+// penny_moe_route_quant for decode batches from the router's weight rw [E, H] bf16 in one launch: E <= 16, T K <= 4096, H / 8 <= 2048,
+// 16-byte rows.  ticket: one int, zero at the first call, zero again behind every call.
+PENNY_API int penny_moe_decode_route(const void* x, int ldx, const void* rw, int T, int H, int E, int K, void* xq, float* xs, int* pe,
+                                     float* pw, int* ticket, int* sorted_tok, float* sorted_w, int* offsets, int* inv,
+                                     hipStream_t stream) {
+  if (T <= 0) return 0;
+  if (E < 1 || E > 16 || K < 1 || K > 8 || K > E || (long)T * K > MOE_ROUTE_CAP || H < 8 || H % 8 || H > 16384 || ldx % 8 ||
+      ((size_t)x | (size_t)rw) % 16)
+    return (int)hipErrorInvalidValue;
+  const int cpt = (H / 8 + 255) / 256;
+#define ROUTE(C, EM)                                                                                                             \
+  moe_decode_route_kernel<C, EM><<<T, 256, 0, stream>>>((const bf16*)x, ldx, H, (const bf16*)rw, T, E, K, (unsigned char*)xq, xs, \
+                                                        pe, pw, ticket, sorted_tok, sorted_w, offsets, inv)
+#define ROUTE_E(C)                \
+  do {                            \
+    if (E <= 8) ROUTE(C, 8);      \
+    else ROUTE(C, 16);            \
+  } while (0)
+  if (cpt <= 1) ROUTE_E(1);
+  else if (cpt <= 2) ROUTE_E(2);
+  else if (cpt <= 4) ROUTE_E(4);
+  else ROUTE_E(8);
+#undef ROUTE_E
+#undef ROUTE
+  PENNY_RETURN_LAUNCH();
+}
+
 // gu [rows, 2F] bf16 (16-column-interleaved gate|up) -> q [rows, F] e4m3, scale [rows] f32
 PENNY_API int penny_silu_quant_rows_fp8(const void* gu, int rows, int F, void* q, float* scale, hipStream_t stream) {
   if (rows <= 0) return 0;
@@ -457,8 +604,14 @@ PENNY_API int penny_silu_quant_rows_fp8(const void* gu, int rows, int F, void* q
 PENNY_API int penny_quant_rows_fp8(const void* x, int ld, int rows, int n, void* q, float* scale, hipStream_t stream) {
   if (rows <= 0) return 0;
   if (n % 8) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(quant_rows_kernel, dim3(rows), dim3(256), 0, stream, (const bf16*)x, ld, n, (unsigned char*)q,
-                     scale);
+  const int cpt = (n / 8 + 255) / 256;
+#define QUANT(C) quant_rows_kernel<C><<<rows, 256, 0, stream>>>((const bf16*)x, ld, n, (unsigned char*)q, scale)
+  if (cpt <= 1) QUANT(1);
+  else if (cpt <= 2) QUANT(2);
+  else if (cpt <= 4) QUANT(4);
+  else if (cpt <= 8) QUANT(8);
+  else QUANT(0);
+#undef QUANT
   PENNY_RETURN_LAUNCH();
 }
 

@@ -160,6 +160,14 @@ class MixtralModel(DecoderModel):
         p = f"layers.{i}."
         c = self.cfg
         T = h.shape[0]
+        # fp8 MFMA pipeline while the step is weight-bandwidth-bound; bigger prefill chunks go to
+        # hipBLASLt on the cached bf16 copy of the same quantized experts (compute-bound regime)
+        fp8_limit = 1024 if (self.prefill_dequant_cache or self.prefill_fp8) else 4096
+        if not self.ep and self.fp8 and ops._native.use_native(h) and T * c.top_k_experts <= fp8_limit:
+            out = moe_ops.moe_decode_fp8_routed(h.contiguous(), self.w[p + "router"], self.w[p + "w13_t"],
+                                                self.w[p + "w13_scale"], self.w[p + "w2_t"], self.w[p + "w2_scale"],
+                                                c.top_k_experts, self._moe_workspace(T))
+            return comm.tp_all_reduce(out) if self.tp_size > 1 and reduce else out
         logits = linear(h, self.w[p + "router"])
         if self.ep:
             grouped = None
@@ -178,14 +186,6 @@ class MixtralModel(DecoderModel):
                                                    self.w[p + "w2_t"], self.w[p + "w2_scale"])
             return ep_moe(h, logits, c.top_k_experts, c.num_experts, lambda rows, e: self._expert(p, rows, e),
                           group=pstate().tp_group, grouped_fn=grouped)
-        # fp8 MFMA pipeline while the step is weight-bandwidth-bound; bigger prefill chunks go to
-        # hipBLASLt on the cached bf16 copy of the same quantized experts (compute-bound regime)
-        fp8_limit = 1024 if (self.prefill_dequant_cache or self.prefill_fp8) else 4096
-        if self.fp8 and ops._native.use_native(h) and T * c.top_k_experts <= fp8_limit:
-            out = moe_ops.moe_decode_fp8(h.contiguous(), logits.contiguous(), self.w[p + "w13_t"],
-                                         self.w[p + "w13_scale"], self.w[p + "w2_t"], self.w[p + "w2_scale"],
-                                         c.top_k_experts, self._moe_workspace(T))
-            return comm.tp_all_reduce(out) if self.tp_size > 1 and reduce else out
         if (self.fp8 and ops._native.use_native(h) and (p + "w13_q") in self.w
                 and moe_ops.PREFILL_TILES and self.w[p + "w13_q"].shape[1] % 256 == 0):
             # prefill-size step: grouped fp8 tile GEMMs over device-side expert buckets (no host sync)

@@ -89,6 +89,7 @@ _SIGS = {
     "penny_lm_head_sample_shard": [P, c_int, P, c_int, c_int, c_int, c_int, c_int, P, P, P, P, P],
     "penny_sample_shard": [P, c_int, c_long, P, P, P, P, c_int, c_int, c_int, P],
     "penny_topk_topp_threshold": [P, c_int, c_long, P, P, P, P, c_int, c_int, P],
+    "penny_moe_decode_route": [P, c_int, P, c_int, c_int, c_int, c_int, P, P, P, P, P, P, P, P, P, P],
     "penny_moe_route": [P, c_int, c_int, c_int, P, P, P, P, P],
     "penny_moe_route_quant": [P, c_int, P, c_int, c_int, c_int, c_int, P, P, P, P, P, P, P, P, P],
     "penny_quant_rows_fp8": [P, c_int, c_int, c_int, P, P, P],

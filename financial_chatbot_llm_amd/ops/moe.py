@@ -423,6 +423,25 @@ class MoEWorkspace:
         self.aq = torch.zeros((P, F), dtype=torch.uint8, device=device)
         self.as_ = torch.zeros(P, dtype=torch.float32, device=device)
         self.y2 = torch.zeros((P, H), dtype=torch.bfloat16, device=device)
+        self.pairs = torch.zeros((2, P), **i32)           # expert and weight of each pair, on their way to the buckets
+        self.ticket = torch.zeros(1, **i32)
+
+
+def moe_decode_fp8_routed(h: torch.Tensor, router_w: torch.Tensor, w13t: torch.Tensor, s13: torch.Tensor, w2t: torch.Tensor,
+                          s2: torch.Tensor, top_k: int, ws: "MoEWorkspace") -> torch.Tensor:
+    """:func:`moe_decode_fp8` from the router's weight [E, H]: its product (f32 sums, rounded to bf16), the choice, the quantised rows
+    and the buckets in one launch (``penny_moe_decode_route``) where it takes these operands."""
+    from . import _native as N
+    T, H = h.shape
+    E = router_w.shape[0]
+    if not (h.dtype == router_w.dtype == torch.bfloat16 and E <= 16 and top_k <= min(8, E) and T * top_k <= 4096 and H % 8 == 0 and
+            H <= 16384 and router_w.shape == (s13.shape[0], H) and router_w.is_contiguous() and h.stride(1) == 1 and h.stride(0) % 8 == 0 and
+            (h.data_ptr() | router_w.data_ptr()) % 16 == 0):
+        from .gemm import linear
+        return moe_decode_fp8(h, linear(h, router_w).contiguous(), w13t, s13, w2t, s2, top_k, ws)
+    N.call("penny_moe_decode_route", N.ptr(h), h.stride(0), N.ptr(router_w), T, H, E, top_k, N.ptr(ws.xq), N.ptr(ws.xs), N.ptr(ws.pairs[0]),
+           N.ptr(ws.pairs[1]), N.ptr(ws.ticket), N.ptr(ws.sorted_tok), N.ptr(ws.sorted_w), N.ptr(ws.offsets), N.ptr(ws.inv), N.stream())
+    return _moe_decode_experts(h, w13t, s13, w2t, s2, top_k, ws)
 
 
 def moe_decode_fp8(h: torch.Tensor, router_logits: torch.Tensor, w13t: torch.Tensor, s13: torch.Tensor,
@@ -431,13 +450,22 @@ def moe_decode_fp8(h: torch.Tensor, router_logits: torch.Tensor, w13t: torch.Ten
     grouped GEMM(x routing weight) -> combine.  Returns [T, H] bf16 (TP partial sum)."""
     from . import _native as N
     T, H = h.shape
+    st = N.stream()
+    N.call("penny_moe_route", N.ptr(router_logits), T, s13.shape[0], top_k, N.ptr(ws.sorted_tok), N.ptr(ws.sorted_w),
+           N.ptr(ws.offsets), N.ptr(ws.inv), st)
+    N.call("penny_quant_rows_fp8", N.ptr(h), h.stride(0), T, H, N.ptr(ws.xq), N.ptr(ws.xs), st)
+    return _moe_decode_experts(h, w13t, s13, w2t, s2, top_k, ws)
+
+
+def _moe_decode_experts(h: torch.Tensor, w13t: torch.Tensor, s13: torch.Tensor, w2t: torch.Tensor, s2: torch.Tensor, top_k: int,
+                        ws: "MoEWorkspace") -> torch.Tensor:
+    """The experts of the routed, quantised rows in ``ws``."""
+    from . import _native as N
+    T, H = h.shape
     E, F2 = s13.shape
     F_ = F2 // 2
     P = T * top_k
     st = N.stream()
-    N.call("penny_moe_route", N.ptr(router_logits), T, E, top_k, N.ptr(ws.sorted_tok), N.ptr(ws.sorted_w),
-           N.ptr(ws.offsets), N.ptr(ws.inv), st)
-    N.call("penny_quant_rows_fp8", N.ptr(h), h.stride(0), T, H, N.ptr(ws.xq), N.ptr(ws.xs), st)
     ntf13, ntf2 = MOE_NTF
     N.call("penny_moe_gemm_fp8", N.ptr(ws.xq), N.ptr(ws.xs), N.ptr(ws.sorted_tok), N.ptr(ws.offsets), N.ptr(w13t),
            N.ptr(s13), None, N.ptr(ws.a), E, F2, H, 1, ntf13, st)

@@ -1676,3 +1676,47 @@ def test_mid_gemm_residual_epilogue_and_slab_exactness():
     refP = torch.einsum("smk,snk->smn", x.float().view(M, S, K // S).transpose(0, 1),
                         w.float().view(N_, S, K // S).transpose(0, 1))
     close(P, refP, atol=1e-3 * refP.abs().max().item(), rtol=1e-3)
+
+
+@pytest.mark.parametrize("T,E,H,K", [(1, 8, 8, 2), (48, 8, 4096, 2), (65, 9, 520, 4), (512, 16, 2048, 8), (3, 4, 16384, 1), (7, 3, 10248, 3)])
+def test_moe_decode_route(T, E, H, K):
+    """Router, choice, quantised rows and buckets in one launch: the choice of its own bf16 logits, in buckets that hold every pair once."""
+    from financial_chatbot_llm_amd.ops import _native as N, moe
+    g = torch.Generator().manual_seed(T + E)
+    h, router = rnd(T, H, gen=g), rnd(E, H, scale=H ** -0.5, gen=g)
+    x, rw = h.to(DEV), router.to(DEV)
+    ws = moe.MoEWorkspace(max(T, 8), K, E, H, 16, DEV)
+    z = h.double() @ router.double().t()
+    for _ in range(2):                                                   # the ticket is back at zero
+        N.call("penny_moe_decode_route", N.ptr(x), H, N.ptr(rw), T, H, E, K, N.ptr(ws.xq), N.ptr(ws.xs), N.ptr(ws.pairs[0]),
+               N.ptr(ws.pairs[1]), N.ptr(ws.ticket), N.ptr(ws.sorted_tok), N.ptr(ws.sorted_w), N.ptr(ws.offsets), N.ptr(ws.inv), N.stream())
+        q, s = moe.quant_rows_fp8(x)
+        assert torch.equal(ws.xq[:T], q.view(torch.uint8)) and torch.equal(ws.xs[:T], s)
+        idx, w = ws.pairs[0].flatten()[:T * K].view(T, K).cpu().long(), ws.pairs[1].flatten().view(torch.float32)[:T * K].view(T, K).cpu()
+        assert all(len(set(r.tolist())) == K for r in idx) and int(idx.min()) >= 0 and int(idx.max()) < E
+        # chosen logits within one bf16 step (2^-8 of the largest either way) of the best ones, in order
+        best = z.sort(1, descending=True).values[:, :K]
+        tol = 2 ** -7 * z.abs().amax(1, keepdim=True) + 1e-6
+        assert ((z.gather(1, idx) - best).abs() <= tol).all()
+        want = torch.softmax(z.gather(1, idx), 1)
+        assert ((w - want).abs() <= 2 * tol).all() and torch.allclose(w.sum(1), torch.ones(T), atol=1e-5)
+        off, inv = ws.offsets.cpu().tolist(), ws.inv[:T * K].cpu().long()
+        assert off[0] == 0 and off[-1] == T * K and sorted(inv.tolist()) == list(range(T * K))
+        flat = idx.flatten()
+        assert all(off[e] <= p < off[e + 1] for p, e in zip(inv.tolist(), flat.tolist()))
+        assert torch.equal(ws.sorted_tok.cpu().long()[inv], torch.arange(T * K) // K)
+        assert torch.equal(ws.sorted_w.cpu()[inv], w.flatten())
+
+
+@pytest.mark.parametrize("n", [8, 2040, 2056, 4104, 16384, 16392, 40000])
+def test_quant_rows_sizes(n):
+    """Rows around what a thread holds in one, two, four and eight pieces, and longer ones: scale amax / 448, values the nearest e4m3."""
+    from financial_chatbot_llm_amd.ops import moe
+    x = (torch.randn(3, n + 8, generator=torch.Generator().manual_seed(n)) * 3).to(torch.bfloat16)[:, :n]
+    x[2] = 0
+    q, s = moe.quant_rows_fp8(x.to(DEV))
+    amax = x.float().abs().amax(1)
+    assert torch.equal(s.cpu(), torch.where(amax > 0, amax / 448.0, torch.ones(3)))
+    y, got = x.float() * (1.0 / s.cpu())[:, None], q.cpu().float()
+    # half a step of e4m3: 3 mantissa bits, 2^-10 below 2^-6
+    assert ((got - y).abs() <= y.abs().clamp(min=2.0 ** -6) * 2.0 ** -4 + 1e-6).all()
