@@ -316,8 +316,9 @@ def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 # Projections that add the residual stream take a single round of ring tiles (penny_linear_ring_plan) up to this K, with the norm behind
 # them, us before / here: 4096 x 4096 (slices of K and slabs to 2048 rows, then 256 x 256 tiles) 374 rows 29.2 / 27.3, 512 32.5 / 28.4, 1024 48.2 /
-# 40.9, 1280 61.6 / 48.7, 2048 77.0 / 69.0, 2133 86.2 / 79.7, 2560 89.0 / 86.2.  A longer K is the shorter in slices: 4096 x 14336 374 rows
-# 72.4 / 92.7, 1024 115 / 141, 2048 201 / 215.
+# 40.9, 1280 61.6 / 48.7, 2048 77.0 / 69.0, 2133 86.2 / 79.7, 2560 89.0 / 86.2.  A longer K is the shorter in slices (4096 x 14336 374 rows
+# 72.4 / 92.7, 1024 115 / 141, 2048 193 / 205), which 256 x 256 tiles have while two or more of them fill the 256 CUs; between 129 and 160 such
+# tiles run whole and leave the other CUs idle: 4096 x 14336 2133 rows 254 / 228, 2304 240 / 233, 2560 245 / 232, 2800 (176 tiles) 257 / 352.
 RING_RESIDUAL_MAX_K = 4096
 
 
@@ -330,7 +331,9 @@ def _ring_operands(x: torch.Tensor, w: torch.Tensor) -> bool:
 def _ring_residual(x: torch.Tensor, w: torch.Tensor, r: torch.Tensor) -> int:
     """The ring tile for r += x @ w.T in place, or 0 (operands of :func:`prefill_ok`)."""
     (M, K), N_ = x.shape, w.shape[0]
-    if K > RING_RESIDUAL_MAX_K or r.shape != (M, N_) or r.dtype != torch.bfloat16 or r.stride(1) != 1 or r.stride(0) % 8 or r.data_ptr() % 16 or \
+    if K > RING_RESIDUAL_MAX_K and not 128 < -(-M // 256) * -(-N_ // 256) <= 160:
+        return 0
+    if r.shape != (M, N_) or r.dtype != torch.bfloat16 or r.stride(1) != 1 or r.stride(0) % 8 or r.data_ptr() % 16 or \
             not _ring_operands(x, w):
         return 0
     return N.load().penny_linear_ring_plan(M, N_, K)

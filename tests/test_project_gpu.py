@@ -286,3 +286,20 @@ def test_qkv_and_slabs_take_the_ring(monkeypatch):
     calls.clear()
     G.linear(x[:, :4096], w[:, :4096].contiguous(), slabs=True, fuse_residual=r)
     assert calls == ["penny_gemm_prefill"]
+
+
+@pytest.mark.parametrize("M,ring", [(2049, True), (2560, True), (2561, False)])
+def test_long_sums_take_the_ring_where_whole_tiles_leave_cus_idle(M, ring, monkeypatch):
+    """4096 x 14336 with the residual sum: 129 - 160 tiles of 256 x 256 run on the ring instead, and the two agree."""
+    from financial_chatbot_llm_amd.ops import _native as N
+    calls = []
+    call = N.call
+    monkeypatch.setattr(N, "call", lambda name, *a: (calls.append(name), call(name, *a))[1])
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x, w, r = ((torch.randn(s, generator=g, device="cuda") * f).bfloat16() for s, f in (((M, 14336), 1.0), ((4096, 14336), 0.01), ((M, 4096), 1.0)))
+    before = r.clone()
+    G.linear(x, w, slabs=True, fuse_residual=r)
+    assert calls == ["penny_linear_ring" if ring else "penny_gemm_prefill"]
+    want = x.float() @ w.float().t()
+    # the product and the sum are rounded to bf16 one after the other, half a step of at most 2^-7 each
+    assert ((r.float() - before.float() - want).abs() <= 2.0 ** -7 * (want.abs() + before.float().abs()) + 1e-3).all()
