@@ -29,7 +29,7 @@
 //   then the recurrence itself, where a block of 16 channels walks 256 tokens at a time: each thread
 //   scans 16 tokens of one channel from zero, the sixteen partial maps S -> A S + B are folded through
 //   LDS, and the outputs are corrected by the true start state.  Steps of single rows (decode) take
-//   one fused launch instead.
+//   one fused launch instead.  mx_lru_blocks has the block-diagonal product of zr and zi in the gates' launch as well.
 //
 // mx_mingru_scan: the minimal gated recurrent unit, S <- (1 - z) S + z c per channel with gates that read
 //   only the current token: z = sigmoid(zp + z_bias), u = xp + x_bias, c = u + 1/2 for u >= 0 and
@@ -461,6 +461,103 @@ int dispatch_matrix_scan(int D, bool wide, Args... args) {
 // tokens 509 -> 175 us (50 of them the preparation), four of 2048 865 -> 421, 64 + 40 + 32 tokens 41 -> 26; gla, D = 64,
 // 279 -> 77, 433 -> 140 and 19 -> 16.  Errors against 64 bits are those of the token form.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// -expm1(x) for x <= 0, ex = e^x: the series up to 1/2, where it has lost nothing yet (its next term is 1e-8)
+__device__ __forceinline__ float one_less_exp(float x, float ex) {
+  float p = 1.f / 40320.f;
+  p = fmaf(p, x, 1.f / 5040.f);
+  p = fmaf(p, x, 1.f / 720.f);
+  p = fmaf(p, x, 1.f / 120.f);
+  p = fmaf(p, x, 1.f / 24.f);
+  p = fmaf(p, x, 1.f / 6.f);
+  p = fmaf(p, x, 0.5f);
+  p = fmaf(p, x, 1.f);
+  return x > -0.5f ? -x * p : 1.f - ex;
+}
+
+// The block-diagonal gates with their product: z[.., zr] = a, z[.., zi] = sqrt(1 - a^2) i u, gy = gelu_tanh(y + y_bias), as
+// lru_gates_kernel leaves them.  A block takes 16 UT tokens and 64 channels of one part of bs, both of whose matrices (w [B][2 bs][bs], r
+// over i) it stages with the tokens in three stages of 32 of K by LDS-DMA, 16-byte chunks swizzled by the row; a wave 16 channels, both
+// gates in one lane, each sum in two halves.  Bound by the f32 products (46 us of the first figure) and the transcendentals.  R = 2048, 8 parts,
+// with the library's product and lru_gates_kernel / here: 3453 rows 153 / 97, 1200 60 / 39, 100 25 / 8; operands straight from the caches,
+// whose rows lie a power of two apart, 119.  Errors against 64 bits 1.9e-7 of the norm of a, of the library's product 2.9e-7.
+template <typename TY, int UT>
+__global__ void __launch_bounds__(256) lru_blocks_kernel(const float* __restrict__ u, const float* __restrict__ w, int bs, int T, int R,
+                                                         const float* __restrict__ r_bias, const float* __restrict__ i_bias,
+                                                         const float* __restrict__ lam, const TY* __restrict__ y, long sy,
+                                                         const float* __restrict__ y_bias, float* __restrict__ z, float* __restrict__ gy) {
+  constexpr int NST = 3, ROWS = 128 + 16 * UT, STG = ROWS * 128, PIECES = ROWS / 8, LPS = (PIECES + 3) / 4;
+  __shared__ __attribute__((aligned(1024))) char smem[NST * STG];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, c = lane & 15;
+  const int cb = blockIdx.y * 64, b = cb / bs, jb = cb - b * bs, t0 = blockIdx.x * 16 * UT, n = bs / 32;
+  const char* src[LPS];                            // of this lane in the wave's pieces of a stage: 64 rows for r, 64 for i, the tokens
+#pragma unroll
+  for (int i = 0; i < LPS; ++i) {
+    const int r = min(wv + 4 * i, PIECES - 1) * 8 + (lane >> 3), ch = (lane & 7) ^ ((r >> 1) & 7);
+    const float* row = r < 128 ? w + ((long)b * 2 * bs + (r < 64 ? 0 : bs) + jb + (r & 63)) * bs : u + (long)min(t0 + r - 128, T - 1) * R + b * bs;
+    src[i] = reinterpret_cast<const char*>(row + 4 * ch);
+  }
+  const unsigned lds0 = (unsigned)(uintptr_t)((__attribute__((address_space(3))) char*)smem);
+  auto stage = [&](int t) {
+#pragma unroll
+    for (int i = 0; i < LPS; ++i) {
+      unsigned keep;
+      asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+                   : "=&s"(keep)
+                   : "v"(src[i] + 128 * t), "s"(lds0 + (t % NST) * STG + min(wv + 4 * i, PIECES - 1) * 1024)
+                   : "memory");
+    }
+  };
+  f32x4 acc[2][2][UT];                             // half of the sum, gate, token group
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+      for (int k = 0; k < UT; ++k) acc[h][d][k] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int at[2] = {(g ^ ((c >> 1) & 7)) << 4, ((4 + g) ^ ((c >> 1) & 7)) << 4};
+  stage(0);
+  if (n > 1) stage(1);
+  for (int t = 0; t < n; ++t) {
+    if (t + 1 < n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPS) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();                  // stage t is there, and every wave has read stage t - 1
+    if (t + 2 < n) stage(t + 2);
+    const char* sm = smem + (t % NST) * STG + c * 128;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const f32x4 p = *reinterpret_cast<const f32x4*>(sm + 16 * wv * 128 + at[h]);
+      const f32x4 q = *reinterpret_cast<const f32x4*>(sm + (64 + 16 * wv) * 128 + at[h]);
+      f32x4 x[UT];
+#pragma unroll
+      for (int k = 0; k < UT; ++k) x[k] = *reinterpret_cast<const f32x4*>(sm + (128 + 16 * k) * 128 + at[h]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int k = 0; k < UT; ++k) {
+          acc[e & 1][0][k] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[k][e], p[e], acc[e & 1][0][k], 0, 0, 0);
+          acc[e & 1][1][k] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[k][e], q[e], acc[e & 1][1][k], 0, 0, 0);
+        }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+  const int ch = cb + 16 * wv + c, j = jb + 16 * wv + c;
+  const float rb = r_bias[ch], ib = i_bias[ch], sp = -8.0f * mx_softplus(lam[ch]), yb = y_bias != nullptr ? y_bias[ch] : 0.f;
+#pragma unroll
+  for (int k = 0; k < UT; ++k)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int t = t0 + 16 * k + 4 * g + r;
+      if (t >= T) continue;
+      const float rr = mx_sigmoid(acc[0][0][k][r] + acc[1][0][k][r] + rb), ii = mx_sigmoid(acc[0][1][k][r] + acc[1][1][k][r] + ib);
+      const float la = rr * sp, a = expf(la);
+      float* zp = z + ((long)b * T + t) * 2 * bs + j;
+      zp[0] = a;
+      zp[bs] = sqrtf(one_less_exp(2.0f * la, a * a)) * ii * u[(long)t * R + ch];
+      const float yy = ldf(y + t * sy + ch) + yb;
+      gy[(long)t * R + ch] = yy * mx_sigmoid(1.5957691216057308f * (yy + 0.044715f * yy * yy * yy));      // gelu_tanh
+    }
+}
 constexpr int SCC = 16;                  // tokens per chunk
 constexpr int SCAN_LEAST = 32;           // the longest segment from which the chunk form is taken (two chunks; see above)
 
@@ -913,6 +1010,33 @@ MX_API int mx_lru_scan(float* u, float* z, int blocks, const float* r_bias, cons
                                                                  sy, y_bias, R));
   dim3 grid((R + LRU_CH - 1) / LRU_CH, S);
   MX_DISPATCH(dt_out, TO, lru_scan_kernel<TO><<<grid, 256, 0, st>>>(z, u, R / blocks, (long)T, state, cu, slot, pos, (TO*)out, R));
+  MX_RETURN_LAUNCH();
+}
+
+// mx_lru_scan from the parts' matrices w f32 [blocks][2 R / blocks][R / blocks] (r over i): u f32 [T, R] is only read, z f32 [blocks, T,
+// 2 R / blocks] and gy f32 [T, R] are scratch.  R / blocks in whole 64s, T R below 2^31, 16-byte operands.
+MX_API int mx_lru_blocks(const float* u, const float* w, int blocks, const float* r_bias, const float* i_bias, const float* lam,
+                         const void* y, long sy, int dt_y, const float* y_bias, float* z, float* gy, float* state, const int* cu,
+                         const int* slot, const int* pos, void* out, int dt_out, int S, int R, int T, hipStream_t st) {
+  if (S <= 0 || T <= 0) return 0;
+  if (blocks < 1 || R < 1 || R % blocks || R / blocks % 64 || R / 64 > 65535 || S > 65535 || (long)T * R >= 1L << 31 ||
+      ((size_t)u | (size_t)w) % 16)
+    return (int)hipErrorInvalidValue;
+  const int bs = R / blocks;
+  // tokens per block: the fewest that leave more blocks than fit at once, 16 where the chip is not filled
+  const long parts = R / 64;
+  const int ut = (T + 63) / 64 * parts >= 1024 ? 4 : (T + 31) / 32 * parts >= 256 ? 2 : 1;
+  const dim3 gg((T + 16 * ut - 1) / (16 * ut), (unsigned)parts);
+#define LRU_BLOCKS(UT) \
+  MX_DISPATCH(dt_y, TY, lru_blocks_kernel<TY, UT><<<gg, 256, 0, st>>>(u, w, bs, T, R, r_bias, i_bias, lam, (const TY*)y, sy, y_bias, z, gy))
+  if (ut == 4) LRU_BLOCKS(4);
+  else if (ut == 2) LRU_BLOCKS(2);
+  else LRU_BLOCKS(1);
+#undef LRU_BLOCKS
+  const int rc = (int)hipGetLastError();
+  if (rc) return rc;
+  dim3 grid((R + LRU_CH - 1) / LRU_CH, S);
+  MX_DISPATCH(dt_out, TO, lru_scan_kernel<TO><<<grid, 256, 0, st>>>(z, gy, bs, (long)T, state, cu, slot, pos, (TO*)out, R));
   MX_RETURN_LAUNCH();
 }
 

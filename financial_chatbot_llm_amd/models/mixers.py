@@ -637,8 +637,8 @@ class GatedLRUMixer:
     def load(self, get: Getter, dtype) -> torch.Tensor:
         self.y_b, self.x_b = _f32(get, "y.b"), _f32(get, "x.b")
         self.conv_w, self.conv_b, self.lam = _f32(get, "conv"), _f32(get, "conv.b"), _f32(get, "lam")
-        # both gates' block matrices as one batched operand [B, in, 2 * out], f32 (they enter the recurrence)
-        self.w_ri = torch.cat([_f32(get, "ra").transpose(1, 2), _f32(get, "ri").transpose(1, 2)], 2).contiguous()
+        # both gates' block matrices one over the other [B, 2 * out, in], f32 (they enter the recurrence)
+        self.w_ri = torch.cat([_f32(get, "ra"), _f32(get, "ri")], 1).contiguous()
         self.r_b, self.i_b = _f32(get, "ra.b").reshape(-1), _f32(get, "ri.b").reshape(-1)
         self.o = get("o").to(dtype).contiguous()
         return torch.cat([get("y"), get("x")], 0).to(dtype)
@@ -648,12 +648,11 @@ class GatedLRUMixer:
 
     def forward(self, proj: torch.Tensor, positions: torch.Tensor, meta: AttentionMetadata, cache) -> torch.Tensor:
         st = cache[1]
-        T, R, B, bs = proj.shape[0], self.R, self.B, self.bs
+        R = self.R
         u = mx.conv_act(proj[:, R:2 * R], self.conv_w, self.conv_b, st["conv"], meta.seg_cu, meta.seg_state, positions,
                         meta.seg_max_len, "none", in_bias=self.x_b)
-        z = torch.bmm(u.view(T, B, bs).transpose(0, 1), self.w_ri)             # [B, T, 2 bs]: r | i pre-activations
-        s = mx.lru_scan(u, z, B, self.r_b, self.i_b, self.lam, proj[:, :R], self.y_b, st["S"], meta.seg_cu,
-                        meta.seg_state, positions, proj.dtype, max_len=meta.seg_max_len)
+        s = mx.lru_blocks(u, self.w_ri, self.r_b, self.i_b, self.lam, proj[:, :R], self.y_b, st["S"], meta.seg_cu,
+                          meta.seg_state, positions, proj.dtype, max_len=meta.seg_max_len)
         return project(s, self.o)
 
 

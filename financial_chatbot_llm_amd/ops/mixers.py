@@ -988,6 +988,27 @@ def lru_scan(u: torch.Tensor, z: torch.Tensor, blocks: int, r_bias: torch.Tensor
     return (out * F.gelu(yy, approximate="tanh")).to(out_dtype)
 
 
+def lru_blocks(u: torch.Tensor, w: torch.Tensor, r_bias: torch.Tensor, i_bias: torch.Tensor, lam: torch.Tensor, y: torch.Tensor,
+               y_bias: Optional[torch.Tensor], state: torch.Tensor, cu: torch.Tensor, slot: torch.Tensor, pos: torch.Tensor,
+               out_dtype: torch.dtype, max_len: int = 0) -> torch.Tensor:
+    """:func:`lru_scan` from the block-diagonal gate matrices ``w`` f32 [blocks, 2 bs, bs] (r over i) of ``u`` f32 [T, blocks bs], which
+    is scratch afterwards: product and gates in one launch for blocks in whole 64s, but for single-row steps."""
+    T, R = u.shape
+    B, bs = w.shape[0], w.shape[2]
+    if N.use_native(u) and max_len != 1 and bs % 64 == 0 and 0 < T * R < 1 << 31 and R <= 64 * 65535 and cu.numel() <= 65535 and \
+            u.is_contiguous() and w.is_contiguous() and (u.data_ptr() | w.data_ptr()) % 16 == 0:
+        assert u.dtype == w.dtype == torch.float32 and tuple(w.shape) == (B, 2 * bs, bs) and R == B * bs
+        z = torch.empty((B, T, 2 * bs), dtype=torch.float32, device=u.device)
+        gy = torch.empty((T, R), dtype=torch.float32, device=u.device)
+        out = torch.empty((T, R), dtype=out_dtype, device=u.device)
+        N.mcall("mx_lru_blocks", N.ptr(u), N.ptr(w), B, N.ptr(r_bias), N.ptr(i_bias), N.ptr(lam), N.ptr(_rows(y)), y.stride(0), _dt(y),
+                N.ptr(y_bias), N.ptr(z), N.ptr(gy), N.ptr(state), N.ptr(cu), N.ptr(slot), N.ptr(pos), N.ptr(out), _dt(out),
+                cu.numel() - 1, R, T, N.stream())
+        return out
+    z = torch.bmm(u.view(T, B, bs).transpose(0, 1), w.transpose(1, 2))             # [B, T, 2 bs]: r | i pre-activations
+    return lru_scan(u, z, B, r_bias, i_bias, lam, y, y_bias, state, cu, slot, pos, out_dtype, max_len=max_len)
+
+
 # ----------------------------------------------------------------------------------------------
 # minimal gated recurrent unit
 # ----------------------------------------------------------------------------------------------
