@@ -133,6 +133,22 @@ __device__ __forceinline__ void better(float& bv, int& bi, float v, int i) {
 
 #define PENNY_RETURN_LAUNCH() return (int)hipGetLastError()
 
+// Two 4-column groups of bf16 accumulators, lo = columns 16f + 4g .. +3 and hi = 16(f+1) + 4g .. +3
+// in lane row g (= lane >> 4) -> the 8 CONSECUTIVE columns 16f + 8*(g>>1) + 16*(g&1) .. +7 of this
+// lane, via v_permlane16_swap (odd lane rows of vdst <-> even lane rows of vsrc): one 16-B store
+// instead of two 8-B ones (the epilogue store tail is issue-bound).
+__device__ __forceinline__ uint4 pair16(bf16x4 lo, bf16x4 hi) {
+  union {
+    bf16x4 v;
+    uint2 u;
+  } a, b;
+  a.v = lo;
+  b.v = hi;
+  const auto x = __builtin_amdgcn_permlane16_swap(a.u.x, b.u.x, false, false);
+  const auto y = __builtin_amdgcn_permlane16_swap(a.u.y, b.u.y, false, false);
+  return make_uint4(x[0], y[0], x[1], y[1]);
+}
+
 // GELU as max(x, 0) - |x| erfc(|x| / sqrt 2) / 2, without branches: erfc(z) = t Q(t) exp(-z^2), t = 1 / (1 + 0.3 z), Q of
 // degree 8 fitted to a relative error of 2e-8 over z <= 9.5 (beyond, the result is below the smallest f32).  A third of the
 // instructions of x/2 (1 + erff), which a GEMM's epilogue does not hide (36,400 x 3072 x 768: 208 us, with erff 260, the

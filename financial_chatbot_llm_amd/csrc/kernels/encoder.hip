@@ -17,24 +17,27 @@ union Frag {
   bf16x8 v;
 };
 
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
 __device__ __forceinline__ f32x4 mfma16(const bf16x8& a, const bf16x8& b, const f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
 // grid (query tiles of 64, heads, texts), 4 waves of 16 queries.  qkv [T, ld]: q | k | v, heads side by side.  Per tile of
-// 64 keys: S^T = K Q^T with the keys' rows read from memory as operands (the four waves share them in L1), online softmax
-// in base 2, O^T += V^T P^T with the value tile transposed in LDS and P straight from the score registers (K slot 8 g + i
-// holds keys 4 g + i and 16 + 4 g + i).  Bound by the QKV rows read and the output written: 1024 texts of 6 - 64 tokens
-// (36k), 12 heads of 64: 61 us (3.6 TB/s); the paged form took 202 us for the cache write and 72 us for the attention.
-// Longer texts read each other's keys once per 64 queries and wave, without prefetch: the attention alone is slower than the
-// paged one from 64 tokens on, but not with its cache write (32,768 tokens, us, write + paged / this: texts of 128 239 + 39 / 75, of
-// 256 236 + 65 / 125, of 512 237 + 100 / 227; 8 texts of 512 25 + 20 / 38).
+// 64 keys: keys and values to LDS as they lie, each row once, the rows behind the text's end not at all; S^T = K Q^T, online softmax
+// in base 2, O^T += V^T P^T with the values through the transposing LDS read and P straight from the score registers (K slot 8 g + i
+// holds keys 4 g + i and 16 + 4 g + i); sixteens of keys behind the end are left out.  LDS rows are 16 bytes longer than their values, so
+// that 16 of them start in different banks.  Bound by the QKV rows read and the output written: 1024 texts of 6 - 64 tokens
+// (36k), 12 heads of 64: 40 us (5.6 TB/s); with each wave reading the keys for itself, outputs in 8-byte pieces and the values transposed on
+// the way in 59; the paged form took 202 us for the cache write and 72 us for the attention.
+// Longer texts read each other's keys once per 64 queries, without prefetch (32,768 tokens, us, that form / this / paged write + attention:
+// texts of 128 72 / 47 / 239 + 39, of 512 224 / 160 / 237 + 100; 8 texts of 512 36 / 29 / 25 + 20).
 template <int D>
 __global__ void __launch_bounds__(256) encoder_attention_kernel(const bf16* __restrict__ qkv, long ld,
                                                                 const int* __restrict__ cu, int H, float scale_log2,
                                                                 bf16* __restrict__ out) {
-  constexpr int KS = D / 32, NT = D / 16, LDV = 64 + 8;
-  __shared__ __attribute__((aligned(16))) bf16 vt[D * LDV];
+  constexpr int KS = D / 32, NT = D / 16, CP = D / 8, RB = D + 8, LN = 64 * CP / 256;
+  __shared__ __attribute__((aligned(16))) bf16 kt[64 * RB], vt[64 * RB];
   const int r0 = cu[blockIdx.z], n = cu[blockIdx.z + 1] - r0, t0 = blockIdx.x * 64;
   if (t0 >= n) return;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, c = lane & 15, h = blockIdx.y;
@@ -42,52 +45,53 @@ __global__ void __launch_bounds__(256) encoder_attention_kernel(const bf16* __re
   const bf16* k = q + H * D;
   const bf16* v = k + H * D;
   const int qi = t0 + 16 * w + c;
+  const bool live = t0 + 16 * w < n;                 // this wave has a query
   Frag qf[KS];
+  if (live) {
 #pragma unroll
-  for (int s = 0; s < KS; ++s) qf[s].u = *reinterpret_cast<const uint4*>(q + min(qi, n - 1) * ld + 32 * s + 8 * g);
+    for (int s = 0; s < KS; ++s) qf[s].u = *reinterpret_cast<const uint4*>(q + min(qi, n - 1) * ld + 32 * s + 8 * g);
+  }
   f32x4 o[NT];
 #pragma unroll
   for (int i = 0; i < NT; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
-  const bool live = t0 + 16 * w < n;                 // this wave has a query
   for (int k0 = 0; k0 < n; k0 += 64) {
-    Frag kf[4][KS], vv[D / 64][2][1];
+    uint4 kk[LN], vv[LN];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int s = 0; s < KS; ++s)
-        kf[t][s].u = *reinterpret_cast<const uint4*>(k + min(k0 + 16 * t + c, n - 1) * ld + 32 * s + 8 * g);
-    // value tile: a thread moves a pair of keys x 8 dims (zeros behind the text's end)
-#pragma unroll
-    for (int i = 0; i < D / 64; ++i) {
-      const int e = threadIdx.x + 256 * i, jp = e / (D / 8), d = e % (D / 8) * 8;
-#pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        const int j = k0 + 2 * jp + r;
-        vv[i][r][0].u = *reinterpret_cast<const uint4*>(v + min(j, n - 1) * ld + d);
-        if (j >= n) vv[i][r][0].u = make_uint4(0, 0, 0, 0);
+    for (int i = 0; i < LN; ++i) {                   // a thread's 16 bytes of a key and a value, zeros behind the text's end
+      const int e = threadIdx.x + 256 * i, j = k0 + e / CP;
+      kk[i] = vv[i] = make_uint4(0, 0, 0, 0);
+      if (j < n) {
+        kk[i] = *reinterpret_cast<const uint4*>(k + j * ld + e % CP * 8);
+        vv[i] = *reinterpret_cast<const uint4*>(v + j * ld + e % CP * 8);
       }
     }
     if (k0 > 0) __syncthreads();                     // the previous tile's readers are done
 #pragma unroll
-    for (int i = 0; i < D / 64; ++i) {
-      const int e = threadIdx.x + 256 * i, jp = e / (D / 8), d = e % (D / 8) * 8;
-#pragma unroll
-      for (int x = 0; x < 8; ++x)
-        *reinterpret_cast<bf16x2*>(vt + (d + x) * LDV + 2 * jp) = bf16x2{vv[i][0][0].v[x], vv[i][1][0].v[x]};
+    for (int i = 0; i < LN; ++i) {
+      const int e = threadIdx.x + 256 * i, at = e / CP * RB + e % CP * 8;
+      *reinterpret_cast<uint4*>(kt + at) = kk[i];
+      *reinterpret_cast<uint4*>(vt + at) = vv[i];
     }
     __syncthreads();
     if (!live) continue;
+    const int tiles = min(4, (n - k0 + 15) / 16);    // sixteens of keys
     f32x4 sc[4];
     float mt = -INFINITY;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      sc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      sc[t] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      if (t >= tiles) continue;
+      f32x4 a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int s = 0; s < KS; ++s) sc[t] = mfma16(kf[t][s].v, qf[s].v, sc[t]);
+      for (int s = 0; s < KS; ++s) {
+        Frag kf;
+        kf.u = *reinterpret_cast<const uint4*>(kt + (16 * t + c) * RB + 32 * s + 8 * g);
+        a = mfma16(kf.v, qf[s].v, a);
+      }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        sc[t][r] = k0 + 16 * t + 4 * g + r < n ? sc[t][r] * scale_log2 : -INFINITY;
+        if (k0 + 16 * t + 4 * g + r < n) sc[t][r] = a[r] * scale_log2;
         mt = fmaxf(mt, sc[t][r]);
       }
     }
@@ -100,34 +104,41 @@ __global__ void __launch_bounds__(256) encoder_attention_kernel(const bf16* __re
     for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float p = __builtin_amdgcn_exp2f(sc[t][r] - mn);
+        const float p = t < tiles ? __builtin_amdgcn_exp2f(sc[t][r] - mn) : 0.f;
         ls += p;
         pf[t >> 1].v[4 * (t & 1) + r] = (bf16)p;
       }
     l = l * corr + ls;
     m = mn;
+    const bf16* vr = vt + (4 * g + (c >> 2)) * RB + 4 * (c & 3);
 #pragma unroll
-    for (int i = 0; i < NT; ++i) {
-      o[i] *= corr;
+    for (int i = 0; i < NT; ++i) o[i] *= corr;
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const bf16* vr = vt + (16 * i + c) * LDV + 32 * s + 4 * g;
-        const bf16x4 a0 = *reinterpret_cast<const bf16x4*>(vr), a1 = *reinterpret_cast<const bf16x4*>(vr + 16);
-        o[i] = mfma16(bf16x8{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]}, pf[s].v, o[i]);
+    for (int s = 0; s < 2; ++s) {
+      if (2 * s >= tiles) continue;
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        union {
+          s16x4 s[2];
+          bf16x8 v;
+        } a;
+        a.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vr + 32 * s * RB + 16 * i));
+        a.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vr + (32 * s + 16) * RB + 16 * i));
+        o[i] = mfma16(a.v, pf[s].v, o[i]);
       }
     }
   }
-  if (qi >= n) return;
+  if (qi >= n) return;                               // all four lanes of a query together: their swaps have partners
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
   const float inv = 1.0f / l;
-  bf16* dst = out + ((long)(r0 + qi) * H + h) * D + 4 * g;
+  bf16* dst = out + ((long)(r0 + qi) * H + h) * D + 8 * (g >> 1) + 16 * (g & 1);
 #pragma unroll
-  for (int i = 0; i < NT; ++i) {
-    bf16x4 x;
+  for (int i = 0; i < NT; i += 2) {
+    bf16x4 x, y;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) x[r] = (bf16)(o[i][r] * inv);
-    *reinterpret_cast<bf16x4*>(dst + 16 * i) = x;
+    for (int r = 0; r < 4; ++r) x[r] = (bf16)(o[i][r] * inv), y[r] = (bf16)(o[i + 1][r] * inv);
+    *reinterpret_cast<uint4*>(dst + 16 * i) = pair16(x, y);
   }
 }
 

@@ -141,22 +141,6 @@ union FragPair {
   i32x8 v;
 };
 
-// Two 4-column groups of bf16 accumulators, lo = columns 16f + 4g .. +3 and hi = 16(f+1) + 4g .. +3
-// in lane row g (= lane >> 4) -> the 8 CONSECUTIVE columns 16f + 8*(g>>1) + 16*(g&1) .. +7 of this
-// lane, via v_permlane16_swap (odd lane rows of vdst <-> even lane rows of vsrc): one 16-B store
-// instead of two 8-B ones (the epilogue store tail is issue-bound).
-__device__ __forceinline__ uint4 pair16(bf16x4 lo, bf16x4 hi) {
-  union {
-    bf16x4 v;
-    uint2 u;
-  } a, b;
-  a.v = lo;
-  b.v = hi;
-  const auto x = __builtin_amdgcn_permlane16_swap(a.u.x, b.u.x, false, false);
-  const auto y = __builtin_amdgcn_permlane16_swap(a.u.y, b.u.y, false, false);
-  return make_uint4(x[0], y[0], x[1], y[1]);
-}
-
 // The activation of bf16 values, rounded to bf16, from a table in LDS that each block fills with the function's own results while
 // its first K-tiles are on the way: every value of magnitude 2^-14 up to 16 (GELU) or 128 (SiLU), by magnitude and sign (9 and
 // 10.5 KB).  Beyond, GELU is x / 2 or x or 0 once rounded, and SiLU is worked out; all 65536 results are the function's.  The

@@ -34,19 +34,6 @@ union Frag {
   bf16x8 v;
 };
 
-// lo = columns 16f + 4g .. +3 and hi = 16(f+1) + 4g .. +3 of lane row g -> 8 consecutive columns 8*(g>>1) + 16*(g&1) .. +7 of this lane
-__device__ __forceinline__ uint4 pair16(bf16x4 lo, bf16x4 hi) {
-  union {
-    bf16x4 v;
-    uint2 u;
-  } a, b;
-  a.v = lo;
-  b.v = hi;
-  const auto x = __builtin_amdgcn_permlane16_swap(a.u.x, b.u.x, false, false);
-  const auto y = __builtin_amdgcn_permlane16_swap(a.u.y, b.u.y, false, false);
-  return make_uint4(x[0], y[0], x[1], y[1]);
-}
-
 template <int N_>
 __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N_) : "memory");
