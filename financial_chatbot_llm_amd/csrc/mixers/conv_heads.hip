@@ -80,15 +80,31 @@ conv_heads_kernel(const T* __restrict__ in, long si, const float* __restrict__ w
             h[e][c * VE + q] = i >= 0 ? ldf(in + (long)(r0 + i) * si + col + d + q) : (fresh ? 0.f : st[(long)(e + n) * C + d + q]);
         }
       }
-#pragma unroll
-  for (int k = 0; k < KM; ++k)
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  if (KM % 4 == 0 && K == KM && ((size_t)w & 15) == 0) {     // a channel's taps by fours: one by one, each load touches every line
 #pragma unroll
     for (int c = 0; c < NC; ++c)
 #pragma unroll
       for (int e = 0; e < VE; ++e) {
-        const int d = (c * 64 + lane) * VE + e;
-        wk[k][c * VE + e] = (d < nd && k >= pad) ? w[(long)(col + d) * K + k - pad] : 0.f;
+        const int d = min((c * 64 + lane) * VE + e, nd - 1);
+#pragma unroll
+        for (int k = 0; k < KM; k += 4) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(w + (long)(col + d) * KM + k);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) wk[k + i][c * VE + e] = v[i];
+        }
       }
+  } else {
+#pragma unroll
+    for (int k = 0; k < KM; ++k)
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int e = 0; e < VE; ++e) {
+          const int d = (c * 64 + lane) * VE + e;
+          wk[k][c * VE + e] = (d < nd && k >= pad) ? w[(long)(col + d) * K + k - pad] : 0.f;
+        }
+  }
   // the slot's next history: entry e is the input K-1-e rows before the segment's end (entries move down, so each
   // is read before it is overwritten; a lane touches its own channels only)
   if (keep) {
@@ -208,8 +224,8 @@ MX_API int mx_conv_heads(const void* in, long si, int dt, const float* w, int K,
   const bool two = D % 2 == 0 && (G == 0 || P % 2 == 0) && si % 2 == 0 && ((size_t)in | (size_t)qout | (size_t)cache) % al == 0;
   const int units = H + 2 * G;
   // Rows per wave: a wave's rows follow each other's loads, so that few are the shorter way until memory is the bound (bf16, 16 query heads
-  // over 4, four taps, us, before with 8 rows one after the other / 4 / 8: 60 rows 10.3 / 6.8 / 9.0, 400 11.4 / 8.8 / 9.9, 800 12.9 / 11.1 /
-  // 11.9, 1188 15.2 / 15.4 / 14.4, 2048 18.3 / 21.9 / 17.6, 4096 29.6 / 38.5 / 31.4)
+  // over 4, four taps, us, before with 8 rows one after the other / by the rule: 100 rows 10.2 / 5.9, 400 11.2 / 6.3, 1160 15.2 /
+  // 11.9, 2048 20.2 / 15.0, 4096 29.7 / 26.1, 40 single rows 5.6 / 4.3; of these, the taps by fours were 8.2, 8.8, 14.4, 17.6, 31.4 and 5.6 before)
 #define CH_LAUNCH(VE, NC, KM, TT)                                                                                     \
   do {                                                                                                                \
     dim3 grid(mx_tile_count(S, rows, max_len, TT, 6), (units + CH_WAVES - 1) / CH_WAVES);                             \

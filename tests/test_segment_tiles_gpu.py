@@ -153,3 +153,25 @@ def test_embed_pairs(lens, W, dt):
     live = torch.ones(T, dtype=torch.bool)
     live[int(cu[1]):int(cu[2])] = False                                     # a segment without a slot is padding
     assert torch.equal(got.cpu()[live], want[live]) and torch.equal(got_last.cpu(), want_last)
+
+
+@pytest.mark.parametrize("K", [4, 8, 16])
+@pytest.mark.parametrize("D,P", [(128, 128), (40, 24), (33, 33), (200, 256)])
+def test_conv_heads_taps_by_fours(K, D, P):
+    """Taps read sixteen bytes at a time and one by one (weights that start between two sixteens): the same bits."""
+    from financial_chatbot_llm_amd.ops import mixers as mx
+    g = torch.Generator(device="cuda").manual_seed(K + D)
+    H, G, lens = 3, 1, [21, 1, 9]
+    C, T = (H + G) * D + G * P, sum(lens)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    x, flat, state = rnd(T, C), rnd(C * K + 4), rnd(4, K - 1, C)
+    ix = [torch.tensor(v, dtype=torch.int32, device="cuda") for v in ([0, 21, 22, 31], [0, 1, 3], list(range(21)) + [7] + list(range(3, 12)), range(T))]
+    got = []
+    for off in (0, 1):
+        w = flat[off:off + C * K].view(C, K)
+        w.copy_(torch.arange(C * K, device="cuda").view(C, K).remainder(13) / 13 - 0.4)
+        assert w.data_ptr() % 16 == 4 * off
+        st, cache = state.clone(), torch.zeros(T, G * (D + P), device="cuda")
+        q = mx.conv_heads(x, w, st, state[0, 0, :D], state[0, 1, :D], 1e-5, *ix, cache, max(lens), H, G, D, P)
+        got.append((q, st, cache))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
