@@ -83,6 +83,66 @@ __global__ void qk_norm_write_kernel(const T* __restrict__ q, long sq, const T* 
   for (int i = threadIdx.x; i < nv; i += blockDim.x) dst[nk + i] = vr[i];
 }
 
+// The same by 16 bytes, V entries of a row at a time, at most NV pieces of each row a thread: all of a token's rows in one trip, both
+// sums in one exchange.  nq 2048, nk = nv = 512, bf16, us by single entries / here: 3453 rows 19.2 / 8.7, 300 6.3 / 3.1, 20 5.8 / 2.7.
+template <typename T, int V, int NV>
+__global__ void __launch_bounds__(256) qk_norm_write_vec_kernel(const T* __restrict__ q, long sq, const T* __restrict__ k, long sk,
+                                                                const T* __restrict__ v, long sv, const float* __restrict__ qw,
+                                                                const float* __restrict__ kw, float eps, const int* __restrict__ slots,
+                                                                T* __restrict__ cache, T* __restrict__ qout, int nq, int nk, int nv) {
+  typedef T vec __attribute__((ext_vector_type(V)));
+  typedef float fvec __attribute__((ext_vector_type(V)));
+  __shared__ float part[2][4];
+  const long t = blockIdx.x;
+  const int slot = slots[t];
+  vec a[NV], b[NV], c[NV];
+  const bool keep_q = qout != nullptr;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int e = (threadIdx.x + 256 * i) * V;
+    if (keep_q && e < nq) a[i] = *reinterpret_cast<const vec*>(q + t * sq + e);
+    if (e < nk) b[i] = *reinterpret_cast<const vec*>(k + t * sk + e);
+    if (e < nv) c[i] = *reinterpret_cast<const vec*>(v + t * sv + e);
+  }
+  float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int e = (threadIdx.x + 256 * i) * V;
+    if (keep_q && e < nq)
+#pragma unroll
+      for (int x = 0; x < V; ++x) s0 += (float)a[i][x] * (float)a[i][x];
+    if (e < nk)
+#pragma unroll
+      for (int x = 0; x < V; ++x) s1 += (float)b[i][x] * (float)b[i][x];
+  }
+  s0 = mx_wave_sum(s0);
+  s1 = mx_wave_sum(s1);
+  if ((threadIdx.x & 63) == 0) part[0][threadIdx.x >> 6] = s0, part[1][threadIdx.x >> 6] = s1;
+  __syncthreads();
+  s0 = (part[0][0] + part[0][1]) + (part[0][2] + part[0][3]);
+  s1 = (part[1][0] + part[1][1]) + (part[1][2] + part[1][3]);
+  const float cq = 1.0f / sqrtf(s0 / (float)nq + eps), ck = 1.0f / sqrtf(s1 / (float)nk + eps);
+  auto put = [&](T* dst, const vec& x, const float* w, float f, int e) {
+    if (w == nullptr) {
+      *reinterpret_cast<vec*>(dst + e) = x;
+      return;
+    }
+    const fvec g = *reinterpret_cast<const fvec*>(w + e);
+    vec o;
+#pragma unroll
+    for (int y = 0; y < V; ++y) o[y] = (T)((float)x[y] * f * g[y]);
+    *reinterpret_cast<vec*>(dst + e) = o;
+  };
+  T* dst = cache + (long)max(slot, 0) * (nk + nv);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int e = (threadIdx.x + 256 * i) * V;
+    if (keep_q && e < nq) put(qout + t * nq, a[i], qw, cq, e);
+    if (slot >= 0 && e < nk) put(dst, b[i], kw, ck, e);
+    if (slot >= 0 && e < nv) *reinterpret_cast<vec*>(dst + nk + e) = c[i];
+  }
+}
+
 // The same with a rotation: of each head of D entries the first `rot` are turned by the angle pos * freq[i] (times
 // mscale), pair i being the entries (i, i + rot/2) or, half == 0, (2i, 2i + 1).  Sine and cosine are evaluated
 // once per pair and token and shared by all heads.  V > 1: V-entry accesses (half layout; rot/2, D and every row
@@ -690,6 +750,18 @@ MX_API int mx_qk_norm_write(const void* q, long sq, const void* k, long sk, cons
       else QK_ROPE_LAUNCH(bf16, 1);
     }
 #undef QK_ROPE_LAUNCH
+    MX_RETURN_LAUNCH();
+  }
+  const int V = dt == 1 ? 4 : 8, widest = nq > nk ? (nq > nv ? nq : nv) : (nk > nv ? nk : nv), pieces = (widest + 256 * V - 1) / (256 * V);
+  if (pieces <= 4 && nq % V == 0 && nk % V == 0 && nv % V == 0 && sq % V == 0 && sk % V == 0 && sv % V == 0 &&
+      ((size_t)q | (size_t)k | (size_t)v | (size_t)cache | (size_t)qout | (size_t)qw | (size_t)kw) % 16 == 0) {
+#define QK_VEC(NV)                                                                                                                    \
+  MX_DISPATCH(dt, TT, qk_norm_write_vec_kernel<TT, 16 / sizeof(TT), NV><<<T, 256, 0, st>>>(                                           \
+      (const TT*)q, sq, (const TT*)k, sk, (const TT*)v, sv, qw, kw, eps, slots, (TT*)cache, (TT*)qout, nq, nk, nv))
+    if (pieces <= 1) QK_VEC(1);
+    else if (pieces <= 2) QK_VEC(2);
+    else QK_VEC(4);
+#undef QK_VEC
     MX_RETURN_LAUNCH();
   }
   MX_DISPATCH(dt, TT, qk_norm_write_kernel<TT><<<T, 256, 0, st>>>((const TT*)q, sq, (const TT*)k, sk, (const TT*)v, sv, qw,
