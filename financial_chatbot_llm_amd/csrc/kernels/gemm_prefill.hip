@@ -898,6 +898,24 @@ PENNY_API int penny_gemm_prefill_set_group(int gm) {
   return 0;
 }
 
+// gemm_splitk.hip
+extern "C" int penny_bias_rows_tile(int M, int N, int S);
+extern "C" float penny_bias_rows_us(int M, int N, int K);
+extern "C" int penny_bias_rows(const void* X, int ldx, const void* W, int K, void* Y, int ldy, const void* bias, int M, int N, int gelu, int slices, int nf,
+                               int mt, hipStream_t st);
+
+// The last rows of a product with bias that go to the ring's tiles instead, or 0.  A short K has no tail to split (16 K-tiles each), so a
+// last round of a few tiles costs a whole one: 36,352 rows of 2304 x 768 are 1278 tiles, five rounds of 256 CUs, and 248 rows more a sixth.
+// Where the row tiles behind the last full round are up to 1024 rows, one launch of smaller tiles does them in less (here 6.7 us, the
+// round 23).  Up to K = 1024 both add up K in one chain, so that a row has the same bits on either.
+static int peeled_rows(int M, int N, int K, int cus, bool gelu) {
+  const int Mt = (M + TM - 1) / TM, Nt = N / TN, T = Mt * Nt, over = cus > 0 ? T % cus : 0;
+  if (over == 0 || over == T || K > 1024) return 0;
+  const int p = (over + Nt - 1) / Nt, rows = M - (Mt - p) * TM;
+  if (p >= Mt || rows > 1024) return 0;
+  return penny_bias_rows_us(rows, N, K) * (gelu ? 1.5f : 1.f) + 3.f < 5.f + 1.37f * K / BK ? rows : 0;
+}
+
 // Contract (checked): N % 256 == 0, K % (64*S) == 0, ldx % 8 == 0, rows 16-B aligned; EPI_SILU
 // needs S == 1 and ldy % 8 == 0 (Y is [M, N/2]); EPI_SLAB writes P [S, M, N] f32 (ldy unused);
 // EPI_RESID needs R (row stride ldr, ldr % 8 == 0) and S == 1; EPI_BIAS(_GELU) take the bias [N]
@@ -915,6 +933,15 @@ PENNY_API int penny_gemm_prefill(const void* X, int ldx, const void* W, int K, v
   if (epi == EPI_RESID && (!R || ldr % 8)) return (int)hipErrorInvalidValue;
   if ((epi == EPI_BIAS || epi == EPI_BIAS_GELU) && !R) return (int)hipErrorInvalidValue;
   if ((long)((M + TM - 1) / TM) * (N / TN) * S > (1L << 30)) return (int)hipErrorInvalidValue;
+  if (epi == EPI_BIAS || epi == EPI_BIAS_GELU) {
+    if (const int rows = peeled_rows(M, N, K, cus, epi == EPI_BIAS_GELU)) {
+      M -= rows;
+      const int tile = penny_bias_rows_tile(rows, N, 1);
+      const int rc = penny_bias_rows(static_cast<const bf16*>(X) + (long)M * ldx, ldx, W, K, static_cast<bf16*>(Y) + (long)M * ldy, ldy, R, rows, N,
+                                     epi == EPI_BIAS_GELU, 1, tile & 255, tile >> 8, stream);
+      if (rc) return rc;
+    }
+  }
   TailArgs ta{};
   const dim3 grid = S == 1 ? tail_plan(M, N, K, cus, tail_ws, tail_ws_floats, tail_cnt, tail_ncnt, ta)
                            : grid_for(M, N, S);

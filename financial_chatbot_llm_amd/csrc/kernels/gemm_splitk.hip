@@ -806,6 +806,14 @@ extern "C" int penny_bias_rows_tile(int M, int N, int S) {
   return tile;
 }
 
+// ... and what it takes, by the figures above
+extern "C" float penny_bias_rows_us(int M, int N, int K) {
+  const int tile = penny_bias_rows_tile(M, N, 1);
+  for (const RowsTile& t : kRowsTiles)
+    if (tile == (t.nf | t.mt << 8)) return 2.8f + t.us * K / 2048.f;
+  return FLT_MAX;
+}
+
 // Y [M, N] (row stride ldy) = bf16(X W^T + bias) [-> exact GELU] on the same tiles, for penny_gemm_bias_small; the sums are those of
 // penny_rows_slabs in `slices` slices, added in turn
 extern "C" int penny_bias_rows(const void* X, int ldx, const void* W, int K, void* Y, int ldy, const void* bias, int M, int N, int gelu, int slices, int nf,

@@ -190,3 +190,20 @@ def test_activations_of_tile_products_over_all_bf16():
     got = gemm.prefill_gemm(x, gemm.interleave16(eye, up).contiguous(), "silu")
     want = ops.silu_mul(torch.cat([x, x[:, :1].expand(-1, K)], 1).contiguous())
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("gelu", [False, True])
+@pytest.mark.parametrize("N,K,over", [(2304, 768, 7), (2304, 768, 600), (768, 768, 250), (3072, 768, 1), (512, 1024, 300)])
+def test_rows_behind_the_last_full_round(N, K, over, gelu):
+    """The rows that a last, nearly empty round of tiles would take go to smaller tiles: the same bits as in whole tiles."""
+    from financial_chatbot_llm_amd.ops import _native, gemm
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    nt = N // 256
+    M = (cus // nt if cus // nt else 1) * (1 if cus % nt == 0 else 2) * 256 + over     # row tiles of one or two full rounds, and a few rows
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x, w = (torch.randn(s, generator=g, device="cuda").to(torch.bfloat16) for s in ((M, K), (N, K)))
+    b = torch.randn(N, generator=g, device="cuda").to(torch.bfloat16)
+    y, want = torch.empty((M, N), dtype=torch.bfloat16, device="cuda"), gemm.prefill_gemm(x, w, "bias_gelu" if gelu else "bias", bias=b)
+    _native.call("penny_gemm_prefill", _native.ptr(x), K, _native.ptr(w), K, _native.ptr(y), N, _native.ptr(b), 0, M, N, 1, 6 if gelu else 5,
+                 None, 0, None, 0, 0, _native.stream())                                # no count of CUs: whole tiles only
+    assert torch.equal(want, y)
