@@ -659,6 +659,8 @@ PREFILL_EPI = {None: 0, "silu": 1, "slabs": 2, "residual": 3, "bias": 5, "bias_g
 # wave-quantisation tail (profiles/r3_prefill_policy_v5_tail.jsonl; before the tail:
 # r3_prefill_policy_v3_widestores.jsonl, the residual epilogue: r3_prefill_policy_v4_residual.jsonl):
 # (N, K) -> [(max M, choice), ...], first match wins.
+# Where one round of the ring's tiles holds a product, it goes there first: "fused" by penny_qkv_ring_plan, "M" in slabs by
+# penny_ring_slabs_plan, sums with the residual stream by _ring_residual (figures beside each); the choices below are for the rest.
 #   "lib"  hipBLASLt (+ the separate epilogue pass)       "hip"  tile kernel, fused epilogue
 #   "S<n>" tile kernel split-K into n f32 slabs (only where the consumer reads slabs)
 #   "fused" (QKV only) tile kernel with RoPE + paged-KV-write epilogue (prefill_qkv_rope)
