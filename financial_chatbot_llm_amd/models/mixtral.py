@@ -68,7 +68,9 @@ class MixtralModel(DecoderModel):
         self.ep = moe_parallel == "ep" and self.tp_size > 1
         if self.ep:
             self.expert_lo, self.expert_hi = expert_range(self.cfg.num_experts, self.tp_rank, self.tp_size)
-        self._moe_ws = None
+        # scratch of routed fp8 steps by size, and the ticket that every one of them finds at zero and leaves so
+        self._moe_ws: Dict[int, moe_ops.MoEWorkspace] = {}
+        self._moe_ticket = torch.zeros(1, dtype=torch.int32, device=self.device)
 
     def shard(self, name: str, full: torch.Tensor) -> torch.Tensor:
         if self.ep and name.rsplit(".", 1)[-1] in ("w13", "w2"):
@@ -116,13 +118,17 @@ class MixtralModel(DecoderModel):
         q = moe_ops.untile_fp8_weight(self.w[p + key + "_t"][e:e + 1])[0]
         return moe_ops.dequant_fp8(q, self.w[p + key + "_scale"][e], self.dtype)
 
-    def _moe_workspace(self, T: int):
-        c = self.cfg
-        if self._moe_ws is None or self._moe_ws.max_tokens < T:
+    def _moe_workspace(self, T: int) -> "moe_ops.MoEWorkspace":
+        """Scratch for a routed fp8 step of ``T`` tokens.  Captured graphs hold its addresses, so none is given back while the model
+        lives: the sizes are powers of two from 256 on, of which the routed steps reach four at most."""
+        n = max(256, 1 << (T - 1).bit_length())
+        ws = self._moe_ws.get(n)
+        if ws is None:
+            c = self.cfg
             f_local = self.w["layers.0.w13_scale"].shape[-1] // 2   # per-rank expert FFN width
-            self._moe_ws = moe_ops.MoEWorkspace(max(T, 256), c.top_k_experts, c.num_experts, c.hidden_size,
-                                                f_local, self.device)
-        return self._moe_ws
+            ws = self._moe_ws.setdefault(n, moe_ops.MoEWorkspace(n, c.top_k_experts, c.num_experts, c.hidden_size, f_local,
+                                                                 self.device, self._moe_ticket))
+        return ws
 
     def _expert_fp8(self, p: str, rows: torch.Tensor, e: int, out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """One expert on its routed rows with fp8 x fp8 hipBLASLt GEMMs (prefill-size buckets).

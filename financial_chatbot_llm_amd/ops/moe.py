@@ -5,7 +5,7 @@ gfx950 uses the OCP ``e4m3fn`` encoding (not MI300's ``fnuz``), which is torch.f
 from __future__ import annotations
 
 import os
-from typing import Tuple
+from typing import Optional, Tuple
 
 import torch
 
@@ -407,9 +407,11 @@ MOE_NTF = tuple(int(v) for v in os.environ.get("PENNY_MOE_NTF", "4,4").split(","
 
 
 class MoEWorkspace:
-    """Device buffers for one decode-sized MoE step (reused across layers; graph-capturable)."""
+    """Device buffers for one decode-sized MoE step (reused across layers; graph-capturable).  All of it is written before it is read,
+    but for ``ticket``, which ``penny_moe_decode_route`` expects at zero: one that the caller keeps beyond any graph, or an own one."""
 
-    def __init__(self, max_tokens: int, top_k: int, num_experts: int, H: int, F: int, device):
+    def __init__(self, max_tokens: int, top_k: int, num_experts: int, H: int, F: int, device,
+                 ticket: Optional[torch.Tensor] = None):
         P = max_tokens * top_k
         self.max_tokens = max_tokens
         i32 = dict(dtype=torch.int32, device=device)
@@ -424,7 +426,7 @@ class MoEWorkspace:
         self.as_ = torch.zeros(P, dtype=torch.float32, device=device)
         self.y2 = torch.zeros((P, H), dtype=torch.bfloat16, device=device)
         self.pairs = torch.zeros((2, P), **i32)           # expert and weight of each pair, on their way to the buckets
-        self.ticket = torch.zeros(1, **i32)
+        self.ticket = torch.zeros(1, **i32) if ticket is None else ticket
 
 
 def moe_decode_fp8_routed(h: torch.Tensor, router_w: torch.Tensor, w13t: torch.Tensor, s13: torch.Tensor, w2t: torch.Tensor,

@@ -154,6 +154,27 @@ def test_mixtral_fp8_prefill_scaled_mm_path():
     assert (got.float() - dec.float()).abs().max().item() < 0.05 * scale
 
 
+def test_mixtral_graph_replays_behind_larger_steps():
+    """A captured decode step's scratch and ticket stay its own when larger steps come in between, however the memory is used then."""
+    cfg = get_model_config("mixtral-tiny")
+    m = MixtralModel(cfg, device="cuda", tp_rank=0, tp_size=1, fp8=True).init_random(seed=6, std=0.05)
+    gen = torch.Generator().manual_seed(2)
+    h = torch.randn(8, cfg.hidden_size, generator=gen).to(torch.bfloat16).cuda()
+    want = m.mlp(0, h).clone()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = m.mlp(0, h)
+    junk = []
+    for T in (300, 500, 270):
+        m.mlp(0, torch.randn(T, cfg.hidden_size, generator=gen).to(torch.bfloat16).cuda())
+        junk += [torch.full((n,), 77, dtype=torch.int32, device="cuda") for n in (1, 16, 512, 1024, 4096, 1 << 17) for _ in range(4)]
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and int(m._moe_ticket) == 0
+    assert all(bool((t == 77).all()) for t in junk)
+
+
 def test_bge_encoder_gpu_matches_cpu():
     from financial_chatbot_llm_amd.models.bert import BertEncoder
     cfg = get_model_config("bert-tiny")

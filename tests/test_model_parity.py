@@ -135,3 +135,19 @@ def test_mixtral_fp8_expert_path_cpu():
     # random tiny model: many near-tied logits, so bound the mean error (~3 %) and a loose argmax agreement
     assert (got - ref).abs().mean() < 0.05 * ref.abs().mean()
     assert (got.argmax(-1) == ref.argmax(-1)).float().mean() > 0.7
+
+
+def test_mixtral_routed_scratch_outlives_larger_steps():
+    """Captured decode graphs hold the addresses of the routed steps' scratch and its ticket: a larger step takes other scratch, nothing is
+    given back, and a small step finds its own again."""
+    import weakref
+    m = MixtralModel(get_model_config("mixtral-tiny"), device="cpu", dtype=torch.float32).init_random(seed=3)
+    m.quantize_experts()
+    first = weakref.ref(m._moe_workspace(8))
+    at = {k: v.data_ptr() for k, v in vars(first()).items() if torch.is_tensor(v)}
+    for T in (256, 300, 512, 2048, 513, 1025):
+        ws = m._moe_workspace(T)
+        assert ws.max_tokens >= T and ws.ticket.data_ptr() == at["ticket"] and int(ws.ticket) == 0
+    assert first() is not None and m._moe_workspace(1) is m._moe_workspace(256) is first()
+    assert {k: v.data_ptr() for k, v in vars(first()).items() if torch.is_tensor(v)} == at
+    assert len(m._moe_ws) == 4
