@@ -324,8 +324,14 @@ RING_RESIDUAL_MAX_K = 4096
 
 def _ring_operands(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Do the ring tiles read these operands of :func:`prefill_ok` (``PENNY_PREFILL_GEMM=force``: the 256 x 256 tiles take everything)?"""
-    return os.environ.get("PENNY_PREFILL_GEMM", "1") == "1" and x.dtype == w.dtype == torch.bfloat16 and x.shape[0] * x.stride(0) < 1 << 31 and \
-        w.numel() < 1 << 31 and (x.data_ptr() | w.data_ptr()) % 16 == 0
+    return os.environ.get("PENNY_PREFILL_GEMM", "1") == "1" and x.dtype == w.dtype == torch.bfloat16 and x.stride(0) >= x.shape[1] and \
+        x.shape[0] * x.stride(0) < 1 << 31 and w.numel() < 1 << 31 and (x.data_ptr() | w.data_ptr()) % 16 == 0
+
+
+def _apart(x: torch.Tensor, y: torch.Tensor) -> bool:
+    """Do the memory ranges of two matrices of unit column stride not meet?"""
+    (a, na), (b, nb) = ((t.data_ptr(), ((t.shape[0] - 1) * t.stride(0) + t.shape[1]) * t.element_size()) for t in (x, y))
+    return a + na <= b or b + nb <= a
 
 
 def _ring_residual(x: torch.Tensor, w: torch.Tensor, r: torch.Tensor) -> int:
@@ -333,8 +339,8 @@ def _ring_residual(x: torch.Tensor, w: torch.Tensor, r: torch.Tensor) -> int:
     (M, K), N_ = x.shape, w.shape[0]
     if K > RING_RESIDUAL_MAX_K and not 128 < -(-M // 256) * -(-N_ // 256) <= 160:
         return 0
-    if r.shape != (M, N_) or r.dtype != torch.bfloat16 or r.stride(1) != 1 or r.stride(0) % 8 or r.data_ptr() % 16 or \
-            not _ring_operands(x, w):
+    if r.shape != (M, N_) or r.dtype != torch.bfloat16 or r.stride(1) != 1 or r.stride(0) % 8 or r.stride(0) < N_ or r.data_ptr() % 16 or \
+            not (_ring_operands(x, w) and _apart(x, r)):
         return 0
     return N.load().penny_linear_ring_plan(M, N_, K)
 

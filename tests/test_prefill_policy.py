@@ -93,3 +93,17 @@ def test_context_parallel_prefix_length():
     assert cp_prefix_len(300, 2) == 296
     assert cp_prefix_len(100_001, 8) == 100_000
     assert cp_prefix_len(5, 4) == 0
+
+
+def test_ring_leaves_rows_that_overlap_and_sums_over_their_input():
+    """Rows that share memory (a stride below their length) are the other kernels' to read, and a sum in place never writes over its input."""
+    K = 512
+    w = torch.zeros(K, K, dtype=torch.bfloat16)
+    x = torch.zeros(300, 3 * K, dtype=torch.bfloat16)
+    assert gemm._ring_operands(x[:, :K], w) and gemm._ring_operands(x[:, :K].contiguous(), w)
+    one = torch.zeros(1, K, dtype=torch.bfloat16).expand(300, K)
+    near = torch.zeros(300 * 8 + K, dtype=torch.bfloat16).as_strided((300, K), (8, 1))
+    assert not gemm._ring_operands(one, w) and not gemm._ring_operands(near, w)
+    r = torch.zeros(300, K, dtype=torch.bfloat16)
+    for a, b in ((r, r), (x[:, :K], x[:, K:2 * K]), (r, one), (one, r)):
+        assert gemm._ring_residual(a, w, b) == 0

@@ -303,3 +303,28 @@ def test_long_sums_take_the_ring_where_whole_tiles_leave_cus_idle(M, ring, monke
     want = x.float() @ w.float().t()
     # the product and the sum are rounded to bf16 one after the other, half a step of at most 2^-7 each
     assert ((r.float() - before.float() - want).abs() <= 2.0 ** -7 * (want.abs() + before.float().abs()) + 1e-3).all()
+
+
+@pytest.mark.parametrize("stride", [0, 8])
+def test_rows_that_overlap_are_read_as_before(stride):
+    """Rows of a stride below their length, of which prefill products take any multiple of eight: QKV, slabs and the sum in place."""
+    M, K, N_ = 300, 4096, 4096
+    g = torch.Generator(device="cuda").manual_seed(stride)
+    x = torch.randn(M * 8 + K, generator=g, device="cuda").bfloat16().as_strided((M, K), (stride, 1))
+    w = (torch.randn((N_, K), generator=g, device="cuda") * K ** -0.5).bfloat16()
+    want = x.double() @ w.double().t()
+    y = G.linear(x, w, slabs=True)
+    y = y.P.double().sum(0) if isinstance(y, G.Slabs) else y.double()
+    assert ((y - want).norm() / want.norm()) < 2.0 ** -8
+    r = torch.randn((M, N_), generator=g, device="cuda").bfloat16()
+    before = r.double()
+    s = G.linear(x, w, fuse_residual=r)
+    s = s.t.double() if isinstance(s, G.ResidualSum) else s.double() + before
+    assert ((s - before - want).abs() <= 2.0 ** -7 * (want.abs() + before.abs()) + 1e-3).all()
+    qkv = (torch.randn((6144, K), generator=g, device="cuda") * K ** -0.5).bfloat16()
+    cos_sin = torch.cat([torch.ones(1, 64), torch.zeros(1, 64)], 1).cuda()
+    none = torch.full((M,), -1, dtype=torch.int32, device="cuda")
+    caches = [torch.zeros(1, 8, 64 * 128, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    q = G.prefill_qkv_rope(x, qkv, torch.zeros_like(none), cos_sin, none, *caches, 32, 8)
+    want = x.double() @ qkv[:4096].double().t()
+    assert ((q.view(M, 4096).double() - want).norm() / want.norm()) < 2.0 ** -7
