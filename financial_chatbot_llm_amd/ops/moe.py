@@ -429,15 +429,23 @@ class MoEWorkspace:
         self.ticket = torch.zeros(1, **i32) if ticket is None else ticket
 
 
+def _one_route_launch(T: int, E: int, H: int) -> bool:
+    """Is ``penny_moe_decode_route`` the faster for ``T`` tokens?  Each of its blocks, one per token, reads the whole router, so the library's
+    product, choice and quantisation win in the end.  Us in a replayed graph, three launches / one: 8 experts of 4096, 48 tokens 15.0 / 7.6,
+    256 16.3 / 12.1, 384 16.8 / 14.4, 512 17.0 / 17.4, 2048 34 / 59; 8 of 8192, 384 18.2 / 16.7, 512 18.2 / 20.3; 16 of 8192, 256 21.3 / 20.5, 320
+    21.7 / 22.5; 4 of 1024, 256 10.8 / 10.1, 384 10.7 / 11.9; 16 of 16384, 1 23.2 / 23.8, 256 25.6 / 29.5."""
+    return E * H <= 1 << 17 and T <= (384 if E * H <= 1 << 16 else 256)
+
+
 def moe_decode_fp8_routed(h: torch.Tensor, router_w: torch.Tensor, w13t: torch.Tensor, s13: torch.Tensor, w2t: torch.Tensor,
                           s2: torch.Tensor, top_k: int, ws: "MoEWorkspace") -> torch.Tensor:
     """:func:`moe_decode_fp8` from the router's weight [E, H]: its product (f32 sums, rounded to bf16), the choice, the quantised rows
-    and the buckets in one launch (``penny_moe_decode_route``) where it takes these operands."""
+    and the buckets in one launch (``penny_moe_decode_route``) where it takes these operands and is the faster."""
     from . import _native as N
     T, H = h.shape
     E = router_w.shape[0]
-    if not (h.dtype == router_w.dtype == torch.bfloat16 and E <= 16 and top_k <= min(8, E) and T * top_k <= 4096 and H % 8 == 0 and
-            H <= 16384 and router_w.shape == (s13.shape[0], H) and router_w.is_contiguous() and h.stride(1) == 1 and h.stride(0) % 8 == 0 and
+    if not (h.dtype == router_w.dtype == torch.bfloat16 and E <= 16 and top_k <= min(8, E) and _one_route_launch(T, E, H) and H % 8 == 0 and
+            router_w.shape == (s13.shape[0], H) and router_w.is_contiguous() and h.stride(1) == 1 and h.stride(0) % 8 == 0 and
             (h.data_ptr() | router_w.data_ptr()) % 16 == 0):
         from .gemm import linear
         return moe_decode_fp8(h, linear(h, router_w).contiguous(), w13t, s13, w2t, s2, top_k, ws)

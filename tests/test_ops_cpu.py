@@ -291,3 +291,19 @@ def test_paired_stage_table(monkeypatch):
     assert gemm._wrow(False, 256, 1000, 1000) == 2
     monkeypatch.setattr(gemm, "PAIR_MODE", "0")
     assert gemm._wrow(True, 8, 4096, 4096) == 1
+
+
+def test_routed_step_takes_one_launch_only_for_few_tokens(monkeypatch):
+    """Every block of the routing launch reads the router, so steps of many tokens keep the library's product."""
+    from financial_chatbot_llm_amd.ops import _native as N
+    from financial_chatbot_llm_amd.ops import moe
+    calls = []
+    monkeypatch.setattr(N, "call", lambda name, *a: calls.append(name))
+    monkeypatch.setattr(N, "stream", lambda: 0)
+    for T, E, H, one in ((1, 8, 4096, True), (256, 16, 8192, True), (384, 8, 4096, True), (257, 16, 8192, False), (385, 8, 4096, False),
+                         (512, 8, 4096, False), (2048, 8, 4096, False), (1, 16, 16384, False)):
+        bf = dict(dtype=torch.bfloat16)
+        calls.clear()
+        moe.moe_decode_fp8_routed(torch.zeros(T, H, **bf), torch.zeros(E, H, **bf), None, torch.zeros(E, 32), None, torch.zeros(E, H), 2,
+                                  moe.MoEWorkspace(T, 2, E, H, 16, "cpu"))
+        assert (calls[:1] == ["penny_moe_decode_route"]) is one and ("penny_moe_route" in calls) is not one
