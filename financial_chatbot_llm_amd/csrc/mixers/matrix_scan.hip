@@ -462,24 +462,11 @@ int dispatch_matrix_scan(int D, bool wide, Args... args) {
 // 279 -> 77, 433 -> 140 and 19 -> 16.  Errors against 64 bits are those of the token form.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// -expm1(x) for x <= 0, ex = e^x: the series up to 1/2, where it has lost nothing yet (its next term is 1e-8)
-__device__ __forceinline__ float one_less_exp(float x, float ex) {
-  float p = 1.f / 40320.f;
-  p = fmaf(p, x, 1.f / 5040.f);
-  p = fmaf(p, x, 1.f / 720.f);
-  p = fmaf(p, x, 1.f / 120.f);
-  p = fmaf(p, x, 1.f / 24.f);
-  p = fmaf(p, x, 1.f / 6.f);
-  p = fmaf(p, x, 0.5f);
-  p = fmaf(p, x, 1.f);
-  return x > -0.5f ? -x * p : 1.f - ex;
-}
-
-// The block-diagonal gates with their product: z[.., zr] = a, z[.., zi] = sqrt(1 - a^2) i u, gy = gelu_tanh(y + y_bias), as
-// lru_gates_kernel leaves them.  A block takes 16 UT tokens and 64 channels of one part of bs, both of whose matrices (w [B][2 bs][bs], r
+// The block-diagonal gates with their product: z[.., zr] = a, z[.., zi] = sqrt(1 - a^2) i u, gy = gelu_tanh(y + y_bias), by
+// the functions of lru_gates_kernel: from equal sums the same bits.  A block takes 16 UT tokens and 64 channels of one part of bs, both of whose matrices (w [B][2 bs][bs], r
 // over i) it stages with the tokens in three stages of 32 of K by LDS-DMA, 16-byte chunks swizzled by the row; a wave 16 channels, both
 // gates in one lane, each sum in two halves.  Bound by the f32 products (46 us of the first figure) and the transcendentals.  R = 2048, 8 parts,
-// with the library's product and lru_gates_kernel / here: 3453 rows 153 / 97, 1200 60 / 39, 100 25 / 8; operands straight from the caches,
+// with the library's product and lru_gates_kernel / here: 3453 rows 153 / 99, 1200 60 / 40, 100 25 / 8; operands straight from the caches,
 // whose rows lie a power of two apart, 119.  Errors against 64 bits 1.9e-7 of the norm of a, of the library's product 2.9e-7.
 template <typename TY, int UT>
 __global__ void __launch_bounds__(256) lru_blocks_kernel(const float* __restrict__ u, const float* __restrict__ w, int bs, int T, int R,
@@ -550,12 +537,11 @@ __global__ void __launch_bounds__(256) lru_blocks_kernel(const float* __restrict
       const int t = t0 + 16 * k + 4 * g + r;
       if (t >= T) continue;
       const float rr = mx_sigmoid(acc[0][0][k][r] + acc[1][0][k][r] + rb), ii = mx_sigmoid(acc[0][1][k][r] + acc[1][1][k][r] + ib);
-      const float la = rr * sp, a = expf(la);
+      const float la = rr * sp;
       float* zp = z + ((long)b * T + t) * 2 * bs + j;
-      zp[0] = a;
-      zp[bs] = sqrtf(one_less_exp(2.0f * la, a * a)) * ii * u[(long)t * R + ch];
-      const float yy = ldf(y + t * sy + ch) + yb;
-      gy[(long)t * R + ch] = yy * mx_sigmoid(1.5957691216057308f * (yy + 0.044715f * yy * yy * yy));      // gelu_tanh
+      zp[0] = expf(la);
+      zp[bs] = sqrtf(-expm1f(2.0f * la)) * ii * u[(long)t * R + ch];
+      gy[(long)t * R + ch] = gelu_tanh_f(ldf(y + t * sy + ch) + yb);
     }
 }
 constexpr int SCC = 16;                  // tokens per chunk

@@ -53,8 +53,9 @@ def test_against_float64(dtype, B, bs, lens, gain):
             got = mx.lru_blocks(u.cuda(), w.cuda(), *a, st, *ix, torch.float32, max_len=most)
         assert torch.equal(st[0].cpu(), state[0])
         off.append(max(float((got.double().cpu() - want).norm() / want.norm()), float((st[1:].double().cpu() - ends).norm() / ends.norm())))
-    # f32 sums of bs products inside a sigmoid and an exponential, then a recurrence that forgets
-    assert off[0] < 2e-6 and off[0] <= 1.5 * off[1] + 1e-7, off
+    # f32 sums of bs products inside a sigmoid and an exponential, then a recurrence that forgets; the gates are the same functions and the
+    # sums here in two halves, so that the whole is no further off than with the library's: 2^-24 for the last rounding
+    assert off[0] < 2e-6 and off[0] <= off[1] + 2.0 ** -24, off
 
 
 def test_gates_at_their_ends():
@@ -75,3 +76,22 @@ def test_gates_at_their_ends():
     want, _ = exact(v, w.double(), zero.double(), zero.double(), lam.double(), y.double(), None, None, [T], [0])
     assert torch.isfinite(got[:30]).all()
     assert (got[:30].double() - want[:30]).abs().max() <= 2e-6 * want.abs().max()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_gates_are_those_of_the_scan(dtype):
+    """From pre-activations without a rounding of their own (matrices of zero) the two forms agree bit for bit: decays, inputs and the GeLU
+    branch over the range of each."""
+    from financial_chatbot_llm_amd.ops import mixers as mx
+    g = torch.Generator().manual_seed(4)
+    B, bs, T = 2, 128, 500
+    R = B * bs
+    u, y = torch.randn(T, R, generator=g), (torch.randn(T, R, generator=g) * 3).to(dtype)
+    rb, ib, lam, yb = torch.linspace(-9, 9, R), torch.linspace(5, -5, R), torch.randn(R, generator=g) * 3 - 2, torch.randn(R, generator=g)
+    ix = [torch.tensor(v, dtype=torch.int32, device="cuda") for v in ([0, 200, T], [1, 0], list(range(T)))]
+    arg = [t.cuda() for t in (rb, ib, lam, y, yb)]
+    state = torch.randn(2, R, generator=g)
+    s0, s1 = state.cuda(), state.cuda()
+    got = mx.lru_blocks(u.cuda(), torch.zeros(B, 2 * bs, bs, device="cuda"), *arg, s0, *ix, torch.float32, max_len=300)
+    want = mx.lru_scan(u.cuda(), torch.zeros(B, T, 2 * bs, device="cuda"), B, *arg, s1, *ix, torch.float32, max_len=300)
+    assert torch.equal(got, want) and torch.equal(s0, s1)
