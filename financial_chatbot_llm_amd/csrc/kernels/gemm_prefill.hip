@@ -142,20 +142,25 @@ union FragPair {
 };
 
 // The activation of bf16 values, rounded to bf16, from a table in LDS that each block fills with the function's own results while
-// its first K-tiles are on the way: every value of magnitude 2^-14 up to 16 (GELU) or 128 (SiLU), by magnitude and sign (9 and
-// 10.5 KB).  Beyond, GELU is x / 2 or x or 0 once rounded, and SiLU is worked out; all 65536 results are the function's.  The
-// functions themselves are 18 to 26 instructions a value that no product of the block runs beside: 36,600 x 3072 x 768 with GELU
-// 210 us -> 177, without an activation 163; gate|up of 28672 x 4096, 1024 rows 213 -> 204, 3400 rows 633 -> 623.
-constexpr int ACT_LO = 0x3880;                            // bf16 bits of 2^-14
+// its first K-tiles are on the way, by magnitude and sign (9 KB).  All 65536 results are the function's.
+//   * GELU: every value of magnitude 2^-14 up to 16.  Beyond, it is x / 2 or x or 0 once rounded.
+//   * SiLU: every value of 2^-10 up to 128, as the bits' distance from the result's.  Below it is x / 2, whose distance is that of the
+//     table's first entry down to 2^-125, so that gates may be small; where x / 2 is no normal number, and from 128 on (x, or -0), it is worked out.
+// The functions themselves are 18 to 26 instructions a value that no product of the block runs beside.  Us, with them / here: 36,600 x 3072 x 768
+// with GELU of values of deviation 1, 0.1 and 0.01 212 / 175, 214 / 181, 212 / 204, without an activation 163; gate|up of 28672 x 4096, 3400 rows,
+// gates of 1, 0.01 and 0.001 617 / 611, 620 / 618, 614 / 609 (results in place of distances, gates below 2^-14 by the function: 610, 632, 633).
 template <bool GELU>
-constexpr int act_values() { return 2 * 128 * (GELU ? 18 : 21); }
-__device__ __forceinline__ bf16 silu_bf16(float x) { return (bf16)(x / (1.f + __expf(-x))); }
+constexpr int act_lo() { return GELU ? 0x3880 : 0x3a80; }     // bf16 bits of 2^-14, 2^-10
+template <bool GELU>
+constexpr int act_values() { return 2 * 128 * (GELU ? 18 : 17); }
 
 template <bool GELU>
 __device__ __forceinline__ void act_fill(unsigned short* tab) {
   for (int i = threadIdx.x; i < act_values<GELU>(); i += 512) {
-    const float x = __uint_as_float((unsigned)(ACT_LO + (i >> 1) + ((i & 1) << 15)) << 16);
-    tab[i] = __builtin_bit_cast(unsigned short, GELU ? (bf16)gelu_erf(x) : silu_bf16(x));
+    const unsigned short bits = act_lo<GELU>() + (i >> 1) + ((i & 1) << 15);
+    const float x = __uint_as_float((unsigned)bits << 16);
+    if constexpr (GELU) tab[i] = __builtin_bit_cast(unsigned short, (bf16)gelu_erf(x));
+    else tab[i] = bits - __builtin_bit_cast(unsigned short, (bf16)(x / (1.f + __expf(-x))));
   }
 }
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
@@ -169,17 +174,38 @@ __device__ __forceinline__ bf16x4 act_read(const unsigned short* tab, bf16x4 v) 
   bool off = false;
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
-    const u16x2 at = ((in.p[k] << (unsigned short)1) | (in.p[k] >> (unsigned short)15)) - (u16x2)(unsigned short)(2 * ACT_LO);
+    const u16x2 mag = (in.p[k] << (unsigned short)1) | (in.p[k] >> (unsigned short)15), lo = (u16x2)(unsigned short)(2 * act_lo<GELU>());
+    u16x2 at;
+    if constexpr (GELU) at = mag - lo;
+    else at = __builtin_elementwise_sub_sat(mag, lo);
     const u16x2 to = __builtin_elementwise_min(at, (u16x2)(unsigned short)(act_values<GELU>() - 1));
     off |= __builtin_bit_cast(unsigned, at) != __builtin_bit_cast(unsigned, to);
     out.p[k] = u16x2{tab[to.x], tab[to.y]};
+    if constexpr (!GELU) {
+      const u16x2 least = (u16x2)(unsigned short)0x200;        // 2^-125
+      out.p[k] = in.p[k] - out.p[k];
+      off |= __builtin_bit_cast(unsigned, __builtin_elementwise_min(mag, least)) != __builtin_bit_cast(unsigned, least);
+    }
   }
   if (__any(off)) {
+    bool large = false;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const float x = (float)v[r], a = fabsf(x);
-      if constexpr (!GELU) out.v[r] = silu_bf16(x);
-      else if (!(a >= 6.103515625e-05f && a < 16.f)) out.v[r] = (bf16)(a < 1.f ? 0.5f * x : x < 0.f ? 0.f : x);
+      if constexpr (GELU) {
+        if (!(a >= 6.103515625e-05f && a < 16.f)) out.v[r] = (bf16)(a < 1.f ? 0.5f * x : x < 0.f ? 0.f : x);
+      } else {
+        const bf16 half = (bf16)(0.5f * x);
+        if (a < 2.350988702e-38f) out.v[r] = half;
+        large |= !(a < 128.f);
+      }
+    }
+    if (!GELU && __any(large)) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float x = (float)v[r];
+        if (!(fabsf(x) < 128.f)) out.v[r] = (bf16)(x > 0.f ? x : 0.f * x);      // of -inf: NaN
+      }
     }
   }
   return out.v;

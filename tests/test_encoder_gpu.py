@@ -179,7 +179,8 @@ def test_activations_of_tile_products_over_all_bf16():
     x, w = torch.zeros(M, K, dtype=torch.bfloat16, device="cuda"), torch.zeros(1 << 16, K, dtype=torch.bfloat16, device="cuda")
     got = gemm.prefill_gemm(x, w, "bias_gelu", bias=values)
     want = ops.gelu_(values.clone().view(1, -1)).view(-1)
-    assert torch.equal(torch.nan_to_num(got, 7.0), torch.nan_to_num(want, 7.0).expand(M, -1))
+    bits = lambda t: torch.nan_to_num(t, 7.0, 8.0, 9.0).view(torch.int16)  # noqa: E731  (and the sign of zeros)
+    assert torch.equal(bits(got), bits(want).expand(M, -1))
     # SiLU: row m's entries 1 .. 127 of X reach a gate each through unit rows of W, entry 0 is the factor 1.5 of every `up`
     fin = values[torch.isfinite(values)]
     fin = torch.cat([fin, fin.new_zeros(-fin.numel() % (K - 1))]).view(-1, K - 1)
@@ -188,8 +189,13 @@ def test_activations_of_tile_products_over_all_bf16():
     up = torch.zeros_like(eye)
     up[:, 0] = 1.0
     got = gemm.prefill_gemm(x, gemm.interleave16(eye, up).contiguous(), "silu")
-    want = ops.silu_mul(torch.cat([x, x[:, :1].expand(-1, K)], 1).contiguous())
-    assert torch.equal(got, want)
+    want = ops.silu_mul(torch.cat([x + 0.0, x[:, :1].expand(-1, K)], 1).contiguous())          # a sum is no -0
+    assert torch.equal(bits(got), bits(want))
+    # gates beyond what f32 holds
+    x[:, 1::2], x[:, 2::2] = 3e38, -3e38
+    got = gemm.prefill_gemm(x, gemm.interleave16(2 * eye, up).contiguous(), "silu")
+    want = ops.silu_mul(torch.cat([2 * x, x[:, :1].expand(-1, K)], 1).contiguous())
+    assert torch.isinf(want[:, 1]).all() and torch.isnan(want[:, 2]).all() and torch.equal(bits(got), bits(want))
 
 
 @pytest.mark.parametrize("gelu", [False, True])
