@@ -934,7 +934,8 @@ extern "C" int penny_bias_rows(const void* X, int ldx, const void* W, int K, voi
 // last round of a few tiles costs a whole one: 36,352 rows of 2304 x 768 are 1278 tiles, five rounds of 256 CUs, and 248 rows more a sixth.
 // Where the row tiles behind the last full round are up to 1024 rows, one launch of smaller tiles does them in less (here 6.7 us, the
 // round 23).  Up to K = 1024 both add up K in one chain, so that a row has the same bits on either.
-static int peeled_rows(int M, int N, int K, int cus, bool gelu) {
+PENNY_API int penny_bias_peeled_rows(int M, int N, int K, int cus, int gelu) {
+  if (M <= 0 || N <= 0 || N % TN || K <= 0 || K % BK || (long)((M + TM - 1) / TM) * (N / TN) > (1L << 30)) return 0;
   const int Mt = (M + TM - 1) / TM, Nt = N / TN, T = Mt * Nt, over = cus > 0 ? T % cus : 0;
   if (over == 0 || over == T || K > 1024) return 0;
   const int p = (over + Nt - 1) / Nt, rows = M - (Mt - p) * TM;
@@ -960,7 +961,7 @@ PENNY_API int penny_gemm_prefill(const void* X, int ldx, const void* W, int K, v
   if ((epi == EPI_BIAS || epi == EPI_BIAS_GELU) && !R) return (int)hipErrorInvalidValue;
   if ((long)((M + TM - 1) / TM) * (N / TN) * S > (1L << 30)) return (int)hipErrorInvalidValue;
   if (epi == EPI_BIAS || epi == EPI_BIAS_GELU) {
-    if (const int rows = peeled_rows(M, N, K, cus, epi == EPI_BIAS_GELU)) {
+    if (const int rows = penny_bias_peeled_rows(M, N, K, cus, epi == EPI_BIAS_GELU)) {
       M -= rows;
       const int tile = penny_bias_rows_tile(rows, N, 1);
       const int rc = penny_bias_rows(static_cast<const bf16*>(X) + (long)M * ldx, ldx, W, K, static_cast<bf16*>(Y) + (long)M * ldy, ldy, R, rows, N,

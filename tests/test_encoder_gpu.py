@@ -206,6 +206,9 @@ def test_rows_behind_the_last_full_round(N, K, over, gelu):
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     nt = N // 256
     M = (cus // nt if cus // nt else 1) * (1 if cus % nt == 0 else 2) * 256 + over     # row tiles of one or two full rounds, and a few rows
+    peeled = _native.load().penny_bias_peeled_rows
+    assert peeled(M, N, K, cus, gelu) == over and peeled(M, N, K, 0, gelu) == 0          # the two sides below are two paths
+    assert peeled(M - over, N, K, cus, gelu) == 0 and peeled(M, N, K + 1024, cus, gelu) == 0
     g = torch.Generator(device="cuda").manual_seed(M)
     x, w = (torch.randn(s, generator=g, device="cuda").to(torch.bfloat16) for s in ((M, K), (N, K)))
     b = torch.randn(N, generator=g, device="cuda").to(torch.bfloat16)
