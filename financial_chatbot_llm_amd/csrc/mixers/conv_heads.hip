@@ -225,7 +225,9 @@ MX_API int mx_conv_heads(const void* in, long si, int dt, const float* w, int K,
   const int units = H + 2 * G;
   // Rows per wave: a wave's rows follow each other's loads, so that few are the shorter way until memory is the bound (bf16, 16 query heads
   // over 4, four taps, us, before with 8 rows one after the other / by the rule: 100 rows 10.2 / 5.9, 400 11.2 / 6.3, 1160 15.2 /
-  // 11.9, 2048 20.2 / 15.0, 4096 29.7 / 26.1, 40 single rows 5.6 / 4.3; of these, the taps by fours were 8.2, 8.8, 14.4, 17.6, 31.4 and 5.6 before)
+  // 11.9, 2048 20.2 / 15.0, 4096 29.7 / 26.1, 40 single rows 5.6 / 4.3; of these, the taps by fours were 8.2, 8.8, 14.4, 17.6, 31.4 and 5.6 before).
+  // A wave of 8 or 16 rows fetches as many for a segment of one: five taps, 1, 64 and 200 single rows, with 8 rows one after the other / by 8
+  // side by side / by one 5.4 / 6.2 / 5.0, 6.8 / 7.6 / 6.2, 10.9 / 11.8 / 10.0.
 #define CH_LAUNCH(VE, NC, KM, TT)                                                                                     \
   do {                                                                                                                \
     dim3 grid(mx_tile_count(S, rows, max_len, TT, 6), (units + CH_WAVES - 1) / CH_WAVES);                             \
@@ -238,7 +240,9 @@ MX_API int mx_conv_heads(const void* in, long si, int dt, const float* w, int K,
     if (K <= 4 && max_len == 1) CH_LAUNCH(VE, NC, 4, 1); \
     else if (K <= 4 && rows * (long)units < 24000) CH_LAUNCH(VE, NC, 4, 4); \
     else if (K <= 4) CH_LAUNCH(VE, NC, 4, 8); \
+    else if (K <= 8 && max_len == 1) CH_LAUNCH(VE, NC, 8, 1); \
     else if (K <= 8) CH_LAUNCH(VE, NC, 8, 8); \
+    else if (max_len == 1) CH_LAUNCH(VE, NC, 16, 1); \
     else CH_LAUNCH(VE, NC, 16, 16);         \
   } while (0)
   if (two) {
