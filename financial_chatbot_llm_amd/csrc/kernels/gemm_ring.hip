@@ -310,6 +310,15 @@ PENNY_API int penny_linear_ring_plan(int M, int N, int K) {
   float us = penny_linear_rows_us(M, N, K);
   return ring_plan(M, N, K, 0, us);
 }
+// The same for products that the library does otherwise (ops.gemm.project), or 0.  Where W's rows are in whole 256s the library's large tiles
+// have no remainder, and from 128 x 256 on the ring's are slower (weights beyond the caches, library / here: 4096 x 2048, 1600 rows 33.9 / 37.9, 2557
+// 44.3 / 47.2; 5120 x 2048, 1200 - 1450 rows 0.94 of its rate, 1724 0.91; 2560 x 1024, 2400 - 3000 rows 0.97; 4096 x 6144, 2557 rows 111.6 / 119.4; a few
+// sizes that the library does badly are faster here: 6144 x 1024, 1458 rows 1.26); beside other widths they are the faster at all sizes (5168 x 2048 1.03 -
+// 1.10, 3592 x 1024 1.09 - 1.26).
+PENNY_API int penny_project_ring_plan(int M, int N, int K) {
+  const int tile = penny_linear_ring_plan(M, N, K);
+  return tile && N % 256 == 0 && K >= 1024 && kRingTiles[tile - 1].tn * kRingTiles[tile - 1].tm >= 128 * 256 ? 0 : tile;
+}
 // The tile of penny_qkv_ring for heads of 128, or 0: the 256 x 256 tiles of gemm_prefill.hip are left what no single round holds
 // (6144 x 4096 with rotation and scattered cache rows, us there / here: 300 rows 73 / 37, 476 77 / 48, 768 90 / 66, 1176 114 / 94, 1600 115 /
 // 107; 10240 x 8192 374 rows 118 / 89, 900 198 / 176)

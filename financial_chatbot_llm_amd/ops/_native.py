@@ -46,6 +46,7 @@ _SIGS = {
     "penny_linear_rows_plan": [c_int, c_int, c_int, c_int],
     "penny_linear_rows_replay_plan": [c_int, c_int, c_int, c_int],
     "penny_linear_ring_plan": [c_int, c_int, c_int],
+    "penny_project_ring_plan": [c_int, c_int, c_int],
     "penny_ring_slabs_plan": [c_int, c_int, c_int, c_int],
     "penny_ring_slabs": [P, c_int, P, c_int, P, c_int, c_int, c_int, c_int, P],
     "penny_qkv_ring_plan": [c_int, c_int, c_int],

@@ -289,7 +289,7 @@ def transformed(x: torch.Tensor) -> bool:
 def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """y = x @ w.T in bf16 or f32: the streaming kernels for up to about two thousand rows (``penny_linear_rows_plan``; inside
     :func:`replayed` ``penny_linear_rows_replay_plan``), deep rings of larger tiles where one round of them holds 257 to 3072 rows in
-    bf16 (``penny_linear_ring_plan``), the library's product for the rest."""
+    bf16 (``penny_project_ring_plan``), the library's product for the rest."""
     dt = x.dtype
     if dt == w.dtype and (dt == torch.bfloat16 or dt == torch.float32) and x.dim() == 2 and w.dim() == 2 and N.use_native(x) and \
             not torch.is_autocast_enabled():
@@ -298,7 +298,7 @@ def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         if M <= 3072 and K == w.shape[1] and (xp | wp) % 16 == 0 and ldx % (4 if f32 else 8) == 0 and ldx >= K and x.stride(1) == 1 and \
                 w.is_contiguous() and w.device == x.device and not (w.requires_grad or x.requires_grad):
             lib, replay = N.load(), M > 32 and getattr(_REPLAYED, "on", False)
-            tile = lib.penny_linear_ring_plan(M, N_, K) if M > 256 and not (f32 or replay) and M * ldx < 1 << 31 and N_ * K < 1 << 31 else 0
+            tile = lib.penny_project_ring_plan(M, N_, K) if M > 256 and not (f32 or replay) and M * ldx < 1 << 31 and N_ * K < 1 << 31 else 0
             if tile:
                 y = torch.empty((M, N_), dtype=dt, device=x.device)
                 N.call("penny_linear_ring", xp, ldx, wp, K, y.data_ptr(), N_, None, 0, M, N_, tile, N.stream())

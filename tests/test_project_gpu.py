@@ -191,6 +191,17 @@ def test_ring_rule():
                 assert t == 0 or (-(-M // RING[t - 1][1]) * -(-N_ // RING[t - 1][0]) <= 256 and K % (32 * RING[t - 1][2]) == 0)
 
 
+def test_ring_leaves_even_widths_in_large_tiles_to_the_library():
+    from financial_chatbot_llm_amd.ops import _native as N
+    ring, plan = N.load().penny_linear_ring_plan, N.load().penny_project_ring_plan
+    assert plan(1600, 4096, 2048) == plan(2557, 4096, 2048) == plan(1300, 5120, 2048) == plan(2600, 2560, 1024) == 0
+    assert ring(1600, 4096, 2048) == 8 and ring(2557, 4096, 2048) == 10 and ring(2600, 2560, 1024) == 9      # sums in place stay there
+    assert plan(1600, 5168, 2048) == 10 and plan(2123, 2048, 64) == 9 and plan(1300, 4096, 2048) == 7
+    for M in range(257, 3100, 61):
+        for N_, K in ((512, 1024), (3592, 1024), (2048, 6144), (4096, 512)):
+            assert plan(M, N_, K) == ring(M, N_, K) or (N_ % 256 == 0 and K >= 1024 and ring(M, N_, K) >= 8)
+
+
 @pytest.mark.parametrize("M,N_,K", [(257, 3208, 1024), (400, 7216, 2048), (1188, 2048, 6144), (3072, 1024, 1024)])
 def test_ring_projections(M, N_, K, monkeypatch):
     """Through ``project``, not-a-numbers and infinities where they belong; rows off the alignment and replays keep their paths."""
