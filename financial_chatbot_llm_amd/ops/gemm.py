@@ -90,7 +90,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, epilogue: Optional[str] = None,
         fr = fuse_residual is not None and epilogue is None and residual is None
         c = prefill_choice(M, N_, K, epilogue, slabs and residual is None, fused_residual=fr)
         # (slabs beyond 24 MB take longer than the sum in place: 4096 x 4096, 640 rows 34.7 / 35.4 us, 768 38.4 / 36.5, 1024 48.0 / 41.4)
-        tile = _ring_residual(x, w, fuse_residual) if fr and (c[0] != "M" or int(c[1:]) * M * N_ > 6 << 20) else 0
+        tile = _ring_residual(x, w, fuse_residual, c) if fr and (c[0] != "M" or int(c[1:]) * M * N_ > 6 << 20) else 0
         if tile:
             N.call("penny_linear_ring", N.ptr(x), x.stride(0), N.ptr(w), K, N.ptr(fuse_residual), fuse_residual.stride(0), N.ptr(fuse_residual),
                    fuse_residual.stride(0), M, N_, tile, N.stream())
@@ -318,7 +318,8 @@ def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 # them, us before / here: 4096 x 4096 (slices of K and slabs to 2048 rows, then 256 x 256 tiles) 374 rows 29.2 / 27.3, 512 32.5 / 28.4, 1024 48.2 /
 # 40.9, 1280 61.6 / 48.7, 2048 77.0 / 69.0, 2133 86.2 / 79.7, 2560 89.0 / 86.2.  A longer K is the shorter in slices (4096 x 14336 374 rows
 # 72.4 / 92.7, 1024 115 / 141, 2048 193 / 205), which 256 x 256 tiles have while two or more of them fill the 256 CUs; between 129 and 160 such
-# tiles run whole and leave the other CUs idle: 4096 x 14336 2133 rows 254 / 228, 2304 240 / 233, 2560 245 / 232, 2800 (176 tiles) 257 / 352.
+# tiles run whole and leave the other CUs idle: 4096 x 14336 2133 rows 254 / 228, 2304 240 / 233, 2560 245 / 232, 2800 (176 tiles) 257 / 352.  Where
+# the choice is the library's product, which deals K over all CUs, it stays: 3072 x 8192 2900 rows 141 / 155.
 RING_RESIDUAL_MAX_K = 4096
 
 
@@ -334,10 +335,10 @@ def _apart(x: torch.Tensor, y: torch.Tensor) -> bool:
     return a + na <= b or b + nb <= a
 
 
-def _ring_residual(x: torch.Tensor, w: torch.Tensor, r: torch.Tensor) -> int:
-    """The ring tile for r += x @ w.T in place, or 0 (operands of :func:`prefill_ok`)."""
+def _ring_residual(x: torch.Tensor, w: torch.Tensor, r: torch.Tensor, choice: str) -> int:
+    """The ring tile for r += x @ w.T in place, or 0 (operands of :func:`prefill_ok`, of which ``prefill_choice`` is ``choice``)."""
     (M, K), N_ = x.shape, w.shape[0]
-    if K > RING_RESIDUAL_MAX_K and not 128 < -(-M // 256) * -(-N_ // 256) <= 160:
+    if K > RING_RESIDUAL_MAX_K and not (choice in ("R", "hip") and 128 < -(-M // 256) * -(-N_ // 256) <= 160):
         return 0
     if r.shape != (M, N_) or r.dtype != torch.bfloat16 or r.stride(1) != 1 or r.stride(0) % 8 or r.stride(0) < N_ or r.data_ptr() % 16 or \
             not (_ring_operands(x, w) and _apart(x, r)):

@@ -106,4 +106,15 @@ def test_ring_leaves_rows_that_overlap_and_sums_over_their_input():
     assert not gemm._ring_operands(one, w) and not gemm._ring_operands(near, w)
     r = torch.zeros(300, K, dtype=torch.bfloat16)
     for a, b in ((r, r), (x[:, :K], x[:, K:2 * K]), (r, one), (one, r)):
-        assert gemm._ring_residual(a, w, b) == 0
+        assert gemm._ring_residual(a, w, b, "R") == 0
+
+
+def test_long_sums_in_place_leave_the_library_its_product(monkeypatch):
+    """Beyond K = 4096 the ring stands in for whole 256 x 256 tiles only, never for the library's product."""
+    monkeypatch.delenv("PENNY_PREFILL_GEMM", raising=False)
+    monkeypatch.setattr(gemm, "_ring_operands", lambda x, w: True)
+    monkeypatch.setattr(gemm.N, "load", lambda: type("L", (), {"penny_linear_ring_plan": staticmethod(lambda M, N, K: 10)}))
+    for M, N_, K, ring in ((2133, 4096, 14336, True), (1200, 8192, 8192, True), (2900, 3072, 8192, False), (2100, 4096, 8192, False), (1700, 4096, 14336, False)):
+        x, w, r = (torch.empty(s, dtype=torch.bfloat16, device="meta") for s in ((M, K), (N_, K), (M, N_)))
+        monkeypatch.setattr(gemm, "_apart", lambda a, b: True)
+        assert (gemm._ring_residual(x, w, r, gemm.prefill_choice(M, N_, K, None, True, fused_residual=True)) == 10) is ring
