@@ -152,7 +152,8 @@ __device__ __forceinline__ uint4 pair16(bf16x4 lo, bf16x4 hi) {
 // GELU as max(x, 0) - |x| erfc(|x| / sqrt 2) / 2, without branches: erfc(z) = t Q(t) exp(-z^2), t = 1 / (1 + 0.3 z), Q of
 // degree 8 fitted to a relative error of 2e-8 over z <= 9.5 (beyond, the result is below the smallest f32).  A third of the
 // instructions of x/2 (1 + erff), which a GEMM's epilogue does not hide (36,400 x 3072 x 768: 208 us, with erff 260, the
-// product and bias alone 163; from gemm_prefill.hip's table of these results 177), and without its cancellation for negative x: relative error 1.5e-6 for |x| < 5, there 5e-2.
+// product and bias alone 163; from gemm_prefill.hip's table of these results 177), and without its cancellation for negative x:
+// relative error 1.5e-6 for |x| < 5, there 5e-2.
 __device__ __forceinline__ float gelu_erf(float x) {
   const float t = __builtin_amdgcn_rcpf(fmaf(fabsf(x), 0.2121320366859436f, 1.f));
   float q = -0.06471703946590424f;

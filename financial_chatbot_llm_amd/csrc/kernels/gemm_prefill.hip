@@ -835,8 +835,7 @@ __global__ void __launch_bounds__(512) gemm_prefill_kernel(const void* __restric
       const int col0 = ((n0 + wa * 128) >> 5) * 16;
       bf16x4 o[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-      {
+      for (int q = 0; q < 4; ++q) {
         // same roundings as GEMM -> bf16 gate|up -> silu_mul (HF: silu in the activation dtype)
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[q][r] = (bf16)acc[2 * q][t][r];

@@ -1,9 +1,9 @@
-// Projections of some hundred to three thousand rows (prompts of the layered decoders):
+// Projections of 257 to 3072 rows (prompts):
 //   Y[m, n] = sum_k X[m, k] * W[n, k]          X [M, K] bf16 (row stride ldx), W [N, K] bf16 row-major, Y [M, N] bf16
 //
 // At these sizes a product is one round of blocks over the 256 CUs, and what counts is that the round is well filled and that a
 // block's chain of K steps never waits for memory.  So: ten tiles, from 64 x 64 to 256 x 160, of which penny_linear_ring_plan takes
-// the one whose single round is the shortest; one block of eight waves per CU; and as many stages of K as LDS holds (2 to 6, 96 -
+// the one whose single round is the shortest; one block of eight waves per CU; and as many stages of K as LDS holds (3 to 6, 140 -
 // 160 KB) in flight by LDS-DMA, with counted waits.
 //   * A wave's sub-tile is 64 W rows by a part of the tokens.  Tiles of up to 128 W rows have fewer sub-tiles than waves: KG groups
 //     of waves then take every KG-th 32 of K of a stage, so that each still has a large sub-tile (operand reads from LDS are the
@@ -17,9 +17,9 @@
 // 2048 x 6144 800 rows 39.0 / 33.8; 4096 x 2048 800 rows 24.3 / 20.9; 7216 x 2048 400 rows 25.2 / 19.9, 1188 41.9 / 39.3; 1024 x 1024 1000
 // rows 9.6 / 7.4; 3592 x 1024 1500 rows 20.3 / 16.4.  A stage of 128 x 128 takes 0.48 us: LDS is busy for 0.32 of it, the matrix
 // cores for 0.21.
-// Epilogues: the rounded product; the residual stream added to it; f32 slabs of S slices of K, which the consumer adds; and of a QKV projection (heads of 128) rotation and the paged
-// cache's layout, each with the roundings of gemm_prefill.hip's.  For the last a wave's W rows are 32 of a head's first half and
-// the 32 that they turn with, so that both meet in one lane.
+// Epilogues: the rounded product; the residual stream added to it; f32 slabs of S slices of K, which the consumer adds; and of a QKV
+// projection (heads of 128) rotation and the paged cache's layout, each with the roundings of gemm_prefill.hip's.  For the last a
+// wave's W rows are 32 of a head's first half and the 32 that they turn with, so that both meet in one lane.
 #include "common.h"
 #include "kv_layout.h"
 

@@ -463,8 +463,8 @@ int dispatch_matrix_scan(int D, bool wide, Args... args) {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // The block-diagonal gates with their product: z[.., zr] = a, z[.., zi] = sqrt(1 - a^2) i u, gy = gelu_tanh(y + y_bias), by
-// the functions of lru_gates_kernel: from equal sums the same bits.  A block takes 16 UT tokens and 64 channels of one part of bs, both of whose matrices (w [B][2 bs][bs], r
-// over i) it stages with the tokens in three stages of 32 of K by LDS-DMA, 16-byte chunks swizzled by the row; a wave 16 channels, both
+// the functions of lru_gates_kernel: from equal sums the same bits.  A block takes 16 UT tokens and 64 channels of one part of bs, both of
+// whose matrices (w [B][2 bs][bs], r over i) it stages with the tokens in three stages of 32 of K by LDS-DMA, 16-byte chunks swizzled by the row; a wave 16 channels, both
 // gates in one lane, each sum in two halves.  Bound by the f32 products (46 us of the first figure) and the transcendentals.  R = 2048, 8 parts,
 // with the library's product and lru_gates_kernel / here: 3453 rows 153 / 99, 1200 60 / 40, 100 25 / 8; operands straight from the caches,
 // whose rows lie a power of two apart, 119.  Errors against 64 bits 1.9e-7 of the norm of a, of the library's product 2.9e-7.

@@ -992,7 +992,9 @@ def lru_blocks(u: torch.Tensor, w: torch.Tensor, r_bias: torch.Tensor, i_bias: t
                y_bias: Optional[torch.Tensor], state: torch.Tensor, cu: torch.Tensor, slot: torch.Tensor, pos: torch.Tensor,
                out_dtype: torch.dtype, max_len: int = 0) -> torch.Tensor:
     """:func:`lru_scan` from the block-diagonal gate matrices ``w`` f32 [blocks, 2 bs, bs] (r over i) of ``u`` f32 [T, blocks bs], which
-    is scratch afterwards: product and gates in one launch for blocks in whole 64s, but for single-row steps."""
+    is scratch afterwards: product and gates in one launch for blocks in whole 64s, but for single-row steps.  Those keep the batched
+    product, on this layout as on its transpose (us in a replayed graph, transpose / this: 8 blocks of 256, 1 row 4.2 / 4.0, 32 4.8 / 4.5, 64
+    5.2 / 5.8, 128 6.8 / 6.0; 4 of 256, 64 4.7 / 6.4; 8 of 128, 1 6.0 / 6.4, 128 19.8 / 19.9; 10 of 256, 64 8.2 / 9.6, 128 14.8 / 8.9)."""
     T, R = u.shape
     B, bs = w.shape[0], w.shape[2]
     if N.use_native(u) and max_len != 1 and bs % 64 == 0 and 0 < T * R < 1 << 31 and R <= 64 * 65535 and cu.numel() <= 65535 and \
