@@ -763,14 +763,14 @@ extern "C" int penny_rows_slabs(const void* X, int ldx, const void* W, int K, fl
 }
 
 // Y [M, N] = X [M, K] x W [N, K]^T in bf16 or f32 (f32 != 0) for up to about two thousand rows, W row-major: slabs == null streams W once (S = 1), else
-// S slices of K leave f32 slabs [S, M, N] that a second launch adds.  One entry for both, so that a step that the host bounds
-// pays for one call.  nf, mt: a block's columns and rows in units of 16, one of kRowsTiles.  Contract (checked): N % 16 == 0 (the last
+// S slices of K leave f32 slabs [S, M, N] that a second launch adds, or with Y null the reader.  One entry for both, so that a step that
+// the host bounds pays for one call.  nf, mt: a block's columns and rows in units of 16, one of kRowsTiles.  Contract (checked): N % 16 == 0 (the last
 // tile may be part-filled), K % (64 * S) == 0 (f32: 32 * S), rows of x in whole 16 bytes, y contiguous.
 PENNY_API int penny_linear_rows(const void* X, int ldx, const void* W, int K, void* Y, int M, int N, void* slabs, int S, int nf, int mt,
                                 int f32, int paired, hipStream_t st) {
   if (M <= 0) return 0;
-  if (M > (1 << 20) || N <= 0 || N % 16 || S < 1 || (S > 1) != (slabs != nullptr) || K <= 0 || K % ((f32 ? 32 : 64) * S) ||
-      K > (1 << 28) || ldx % (f32 ? 4 : 8))
+  if (M > (1 << 20) || N <= 0 || N % 16 || S < 1 || (S > 1) != (slabs != nullptr) || (S == 1 && Y == nullptr) || K <= 0 ||
+      K % ((f32 ? 32 : 64) * S) || K > (1 << 28) || ldx % (f32 ? 4 : 8))
     return (int)hipErrorInvalidValue;
   float* p = static_cast<float*>(f32 && S == 1 ? Y : slabs);
   int rc;
@@ -788,7 +788,7 @@ PENNY_API int penny_linear_rows(const void* X, int ldx, const void* W, int K, vo
   ROWS_TILES(LR_CASE)
   return (int)hipErrorInvalidValue;
 #undef LR_CASE
-  if (rc || S == 1) return rc;
+  if (rc || S == 1 || Y == nullptr) return rc;
   if (!f32) return penny_splitk_reduce(slabs, S, M, N, Y, N, nullptr, 0, st);
   const long quads = (long)M * N / 4;
   splitk_reduce_f32_kernel<<<dim3((unsigned)((quads + 255) / 256)), 256, 0, st>>>((const f32x4*)slabs, S, quads, (f32x4*)Y);

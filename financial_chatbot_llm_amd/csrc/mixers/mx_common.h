@@ -105,6 +105,68 @@ template <typename T> __device__ __forceinline__ void stf4(T* p, mx_f32x4 x) {
 // rows of `stride` elements of type code dt (1: f32) may be read and written by four
 inline bool mx_by_four(const void* p, long stride, int dt) { return stride % 4 == 0 && (size_t)p % (dt == 1 ? 16 : 8) == 0; }
 
+// A sublayer's output as the norm behind it reads it, so that what would only add it up needs no launch of its own (a step of 64 rows:
+// the sum of a product's K slices 4.4 us, of a token's experts 4.9): rows p [T, ld] of the storage type, `slabs` f32 slices of K of them
+// (slab elements apart, their sum rounded to the type), or nothing (p null); with top > 0 a token's routed rows besides, added to those in
+// turn: row pos[t, k] of ys times wts[t, k] (null: 1), or for an entry idx[t, k] >= E the token's own row of h.  The order of
+// the sums and the roundings are those of the launches that write it out.
+struct MxPart {
+  const void* p;
+  long ld, slab;
+  const void* ys;
+  long sy;
+  const int* pos;
+  const int* idx;
+  const float* wts;
+  const void* h;
+  long sh;
+  int slabs, E, top;
+};
+// columns c .. c + 3 of row t
+template <typename T> __device__ __forceinline__ mx_f32x4 mx_part4(const MxPart& a, long t, int c) {
+  mx_f32x4 v = mx_f32x4{0.f, 0.f, 0.f, 0.f};
+  if (a.slabs > 0) {
+    const float* p = static_cast<const float*>(a.p) + t * a.ld + c;
+    v = ldf4(p);
+    for (int s = 1; s < a.slabs; s += 4) {                 // four loads at a time
+      mx_f32x4 u[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) u[j] = ldf4(p + min(s + j, a.slabs - 1) * a.slab);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (s + j < a.slabs) v += u[j];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = (float)(T)v[e];
+  } else if (a.p != nullptr) {
+    v = ldf4(static_cast<const T*>(a.p) + t * a.ld + c);
+  }
+  if (a.top == 0) return v;
+  for (int k = 0; k < a.top; k += 4) {
+    mx_f32x4 u[4];
+    float w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const long i = t * a.top + min(k + j, a.top - 1);
+      w[j] = k + j < a.top ? (a.wts != nullptr ? a.wts[i] : 1.f) : 0.f;
+      u[j] = ldf4(a.idx[i] >= a.E ? static_cast<const T*>(a.h) + t * a.sh + c : static_cast<const T*>(a.ys) + a.pos[i] * a.sy + c);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (w[j] != 0.f)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += w[j] * u[j][e];
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = (float)(T)v[e];
+  return v;
+}
+// rows of it may be read by four (type code dt)
+inline bool mx_part_by_four(const MxPart& a, int dt) {
+  return mx_by_four(a.p, a.ld, a.slabs > 0 ? 1 : dt) && a.slab % 4 == 0 && a.slabs >= 0 && (a.slabs == 0 || a.p != nullptr) &&
+         (a.top == 0 || (a.top > 0 && a.pos != nullptr && a.idx != nullptr && mx_by_four(a.ys, a.sy, dt) && mx_by_four(a.h, a.sh, dt)));
+}
+
 // A token whose value is not finite must not reach the tokens before it through the zeros of a triangular factor: such
 // elements of a tile (rows 4 g + r of column lane % 16) become zero, and the first one's row is returned (16: none).
 __device__ __forceinline__ int mx_drop_nonfinite(mx_f32x4& x, int g) {

@@ -99,9 +99,11 @@ __global__ void post_norm_kernel(float* __restrict__ x, const TA* __restrict__ a
 
 // The same with the row in registers, by fours, R pieces per thread: one read of every input (2400 rows of 2048 f32 with a
 // bf16 addend and copy: 19 us, through LDS element by element 34).
-template <typename TA, typename TO, int R>
+// OPEN: the sublayer outputs are pa and pb (a and b say only which of them there are)
+template <typename TA, typename TO, int R, bool OPEN>
 __global__ void __launch_bounds__(256) post_norm_vec_kernel(float* __restrict__ x, const TA* __restrict__ a, long sa,
                                                             const float* __restrict__ wa, const TA* __restrict__ b, long sb,
+                                                            MxPart pa, MxPart pb,
                                                             const float* __restrict__ wb, const float* __restrict__ w,
                                                             float eps, TO* __restrict__ out, int W) {
   __shared__ float scratch[16];
@@ -116,8 +118,13 @@ __global__ void __launch_bounds__(256) post_norm_vec_kernel(float* __restrict__ 
     m[c] = xv[c] = u[c] = zero;
     if (i >= W) continue;
     xv[c] = ldf4(x + t * W + i);
-    m[c] = a == nullptr ? xv[c] : ldf4(a + t * sa + i);
-    if (b != nullptr) u[c] = ldf4(b + t * sb + i);
+    if (OPEN) {
+      m[c] = mx_part4<TA>(pa, t, i);
+      if (b != nullptr) u[c] = mx_part4<TA>(pb, t, i);
+    } else {
+      m[c] = a == nullptr ? xv[c] : ldf4(a + t * sa + i);
+      if (b != nullptr) u[c] = ldf4(b + t * sb + i);
+    }
   }
   if (b != nullptr) {
     float sa2 = 0.f, sb2 = 0.f;
@@ -350,8 +357,8 @@ MX_API int mx_post_norm(float* x, const void* a, long sa, const float* wa, const
       (a == nullptr || mx_by_four(a, sa, dt_ab)) && (b == nullptr || (a != nullptr && mx_by_four(b, sb, dt_ab))) &&
       mx_by_four(out, W, dt_out)) {
 #define POST_NORM(R)                                                                                                     \
-  MX_DISPATCH(dt_ab, TA, MX_DISPATCH(dt_out, TO, post_norm_vec_kernel<TA, TO, R><<<T, 256, 0, st>>>(                     \
-      x, (const TA*)a, sa, wa, (const TA*)b, sb, wb, w, eps, (TO*)out, W)))
+  MX_DISPATCH(dt_ab, TA, MX_DISPATCH(dt_out, TO, post_norm_vec_kernel<TA, TO, R, false><<<T, 256, 0, st>>>(              \
+      x, (const TA*)a, sa, wa, (const TA*)b, sb, MxPart{}, MxPart{}, wb, w, eps, (TO*)out, W)))
     if (W <= 1024) POST_NORM(1);
     else if (W <= 2048) POST_NORM(2);
     else POST_NORM(4);
@@ -361,6 +368,25 @@ MX_API int mx_post_norm(float* x, const void* a, long sa, const float* wa, const
   const int nt = W >= 1024 ? 512 : 256;
   MX_DISPATCH(dt_ab, TA, MX_DISPATCH(dt_out, TO, post_norm_kernel<TA, TO><<<T, nt, (size_t)W * sizeof(float), st>>>(
       x, (const TA*)a, sa, wa, (const TA*)b, sb, wb, w, eps, (TO*)out, W)));
+  MX_RETURN_LAUNCH();
+}
+
+// The same for sublayer outputs that are still apart (b may be null).  W and all rows in whole fours, W <= 4096.
+MX_API int mx_post_norm_parts(float* x, const MxPart* a, const float* wa, const MxPart* b, const float* wb, int dt_ab, const float* w,
+                              float eps, void* out, int dt_out, int T, int W, hipStream_t st) {
+  if (T <= 0) return 0;
+  if (a == nullptr || W <= 0 || W % 4 || W > 4096 || !mx_part_by_four(*a, dt_ab) ||
+      (b != nullptr && (!mx_part_by_four(*b, dt_ab) || wa == nullptr || wb == nullptr)) || w == nullptr ||
+      ((size_t)x | (size_t)w | (size_t)wa | (size_t)wb) % 16 || !mx_by_four(out, W, dt_out))
+    return (int)hipErrorInvalidValue;
+  const MxPart pb = b != nullptr ? *b : MxPart{};
+#define POST_NORM(R)                                                                                                     \
+  MX_DISPATCH(dt_ab, TA, MX_DISPATCH(dt_out, TO, post_norm_vec_kernel<TA, TO, R, true><<<T, 256, 0, st>>>(               \
+      x, (const TA*)a, 0, wa, (const TA*)b, 0, *a, pb, wb, w, eps, (TO*)out, W)))
+  if (W <= 1024) POST_NORM(1);
+  else if (W <= 2048) POST_NORM(2);
+  else POST_NORM(4);
+#undef POST_NORM
   MX_RETURN_LAUNCH();
 }
 

@@ -67,10 +67,11 @@ __global__ void residual_norm_kernel(float* __restrict__ x, const TA* __restrict
 }
 
 // the same with four adjacent columns per access and the row in registers between its two passes: a thread owns NC
-// groups of columns; every row start and W are multiples of four elements
-template <typename TA, typename TO, int NC>
+// groups of columns; every row start and W are multiples of four elements.  OPEN: the sublayer outputs are pa and pb (a and b
+// say only which of them there are)
+template <typename TA, typename TO, int NC, bool OPEN>
 __global__ void residual_norm_vec_kernel(float* __restrict__ x, const TA* __restrict__ a, long sa,
-                                         const TA* __restrict__ b, long sb, float mult, float mult_b,
+                                         const TA* __restrict__ b, long sb, MxPart pa, MxPart pb, float mult, float mult_b,
                                          const TA* __restrict__ gate, long sg, const float* __restrict__ gate_bias,
                                          const int* __restrict__ ids, const TA* __restrict__ table, int vocab, int fresh,
                                          const float* __restrict__ w, float eps, TO* __restrict__ out, int W) {
@@ -91,13 +92,17 @@ __global__ void residual_norm_vec_kernel(float* __restrict__ x, const TA* __rest
     if (i >= W) continue;
     if (!fresh) v[c] = *reinterpret_cast<const vf*>(xr + i);
     if (upd) {
-      va av = va{}, bv = va{};
-      if (a != nullptr) av = *reinterpret_cast<const va*>(a + t * sa + i);
-      if (b != nullptr) bv = *reinterpret_cast<const va*>(b + t * sb + i);
+      vf av = vf{0.f, 0.f, 0.f, 0.f}, bv = av;
+      if (OPEN) {
+        if (a != nullptr) av = mx_part4<TA>(pa, t, i);
+        if (b != nullptr) bv = mx_part4<TA>(pb, t, i);
+      } else {
+        if (a != nullptr) av = ldf4(a + t * sa + i);
+        if (b != nullptr) bv = ldf4(b + t * sb + i);
+      }
       vf s;
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        s[e] = mult == mult_b ? mult * ((float)av[e] + (float)bv[e]) : mult * (float)av[e] + mult_b * (float)bv[e];
+      for (int e = 0; e < 4; ++e) s[e] = mult == mult_b ? mult * (av[e] + bv[e]) : mult * av[e] + mult_b * bv[e];
       if (gate != nullptr) {
         const va gv = *reinterpret_cast<const va*>(gate + t * sg + i);
 #pragma unroll
@@ -227,9 +232,10 @@ __global__ void relu2_kernel(const T* __restrict__ in, long si, T* __restrict__ 
 }
 
 // grid (row groups, column chunks): a thread owns V adjacent columns and walks `rows` rows, its weights in
-// registers.  a null: the first form reads table rows (ids) and REPLACES x; both a and table null: out only.
-template <typename TA, typename TO, int V>
-__global__ void dyn_tanh_kernel(float* __restrict__ x, const TA* __restrict__ a, long sa, const int* __restrict__ ids,
+// registers.  a null: the first form reads table rows (ids) and REPLACES x; both a and table null: out only.  OPEN: the sublayer's
+// output is pa (a: not null), V = 4.
+template <typename TA, typename TO, int V, bool OPEN>
+__global__ void dyn_tanh_kernel(float* __restrict__ x, const TA* __restrict__ a, long sa, MxPart pa, const int* __restrict__ ids,
                                 const TA* __restrict__ table, int vocab, float scale, float alpha1,
                                 const float* __restrict__ w1, const float* __restrict__ b1, float alpha2,
                                 const float* __restrict__ w2, const float* __restrict__ b2, TO* __restrict__ out, int W,
@@ -253,7 +259,12 @@ __global__ void dyn_tanh_kernel(float* __restrict__ x, const TA* __restrict__ a,
   for (long t = t0; t < t1; ++t) {
     float* xr = x + t * W + c;
     vf v = {};
-    if (a != nullptr) {
+    if constexpr (OPEN) {
+      v = *reinterpret_cast<const vf*>(xr);
+      const vf y = mx_part4<TA>(pa, t, c);
+#pragma unroll
+      for (int e = 0; e < V; ++e) v[e] += mx_tanh(alpha1 * y[e]) * w1r[e] + b1r[e];
+    } else if (a != nullptr) {
       const va y = *reinterpret_cast<const va*>(a + t * sa + c);
       v = *reinterpret_cast<const vf*>(xr);
 #pragma unroll
@@ -426,9 +437,9 @@ MX_API int mx_residual_norm(float* x, const void* a, long sa, const void* b, lon
   if (vec) {
     const int cols = W / 4, ntv = cols >= 512 ? 512 : (cols + 63) / 64 * 64;
 #define RESIDUAL_VEC(NC)                                                                                              \
-  MX_DISPATCH(dt_ab, TA, MX_DISPATCH(dt_out, TO, residual_norm_vec_kernel<TA, TO, NC><<<T, ntv, 0, st>>>(             \
-      x, (const TA*)a, sa, (const TA*)b, sb, mult, mult_b, (const TA*)gate, sg, gate_bias, ids, (const TA*)table,     \
-      vocab, fresh, w, eps, (TO*)out, W)))
+  MX_DISPATCH(dt_ab, TA, MX_DISPATCH(dt_out, TO, residual_norm_vec_kernel<TA, TO, NC, false><<<T, ntv, 0, st>>>(      \
+      x, (const TA*)a, sa, (const TA*)b, sb, MxPart{}, MxPart{}, mult, mult_b, (const TA*)gate, sg, gate_bias, ids,   \
+      (const TA*)table, vocab, fresh, w, eps, (TO*)out, W)))
     if (cols <= ntv) RESIDUAL_VEC(1);
     else if (cols <= 2 * ntv) RESIDUAL_VEC(2);
     else RESIDUAL_VEC(4);
@@ -439,6 +450,27 @@ MX_API int mx_residual_norm(float* x, const void* a, long sa, const void* b, lon
   MX_DISPATCH(dt_ab, TA, MX_DISPATCH(dt_out, TO, residual_norm_kernel<TA, TO><<<T, nt, 0, st>>>(
       x, (const TA*)a, sa, (const TA*)b, sb, mult, mult_b, (const TA*)gate, sg, gate_bias, ids,
       (const TA*)table, vocab, fresh, w, eps, (TO*)out, W)));
+  MX_RETURN_LAUNCH();
+}
+
+// x <- x + mult * a + mult_b * b and its norm as above for sublayer outputs that are still apart (b may be null).  W and all rows in
+// whole fours, W <= 8192.
+MX_API int mx_residual_norm_parts(float* x, const MxPart* a, const MxPart* b, int dt_ab, float mult, float mult_b, const float* w,
+                                  float eps, void* out, int dt_out, int T, int W, hipStream_t st) {
+  if (T <= 0) return 0;
+  if (a == nullptr || W <= 0 || W % 4 || W > 8192 || !mx_part_by_four(*a, dt_ab) || (b != nullptr && !mx_part_by_four(*b, dt_ab)) ||
+      ((size_t)x | (size_t)w) % 16 || !mx_by_four(out, W, dt_out) || (out != nullptr && w == nullptr))
+    return (int)hipErrorInvalidValue;
+  const int cols = W / 4, nt = cols >= 512 ? 512 : (cols + 63) / 64 * 64;
+  const MxPart pb = b != nullptr ? *b : MxPart{};
+#define RESIDUAL_PARTS(NC)                                                                                            \
+  MX_DISPATCH(dt_ab, TA, MX_DISPATCH(dt_out, TO, residual_norm_vec_kernel<TA, TO, NC, true><<<T, nt, 0, st>>>(        \
+      x, (const TA*)a, 0, (const TA*)b, 0, *a, pb, mult, mult_b, (const TA*)nullptr, 0, nullptr, nullptr,             \
+      (const TA*)nullptr, 0, 0, w, eps, (TO*)out, W)))
+  if (cols <= nt) RESIDUAL_PARTS(1);
+  else if (cols <= 2 * nt) RESIDUAL_PARTS(2);
+  else RESIDUAL_PARTS(4);
+#undef RESIDUAL_PARTS
   MX_RETURN_LAUNCH();
 }
 
@@ -460,11 +492,26 @@ MX_API int mx_dyn_tanh(float* x, const void* a, long sa, const int* ids, const v
   const int rows = T >= 2048 ? 4 : (T >= 1024 ? 2 : 1);
   dim3 grid((T + rows - 1) / rows, (cols + nt - 1) / nt);
   if (vec)
-    MX_DISPATCH(dt_a, TA, MX_DISPATCH(dt_out, TO, dyn_tanh_kernel<TA, TO, 4><<<grid, nt, 0, st>>>(
-        x, (const TA*)a, sa, ids, (const TA*)table, vocab, scale, alpha1, w1, b1, alpha2, w2, b2, (TO*)out, W, rows, T)));
+    MX_DISPATCH(dt_a, TA, MX_DISPATCH(dt_out, TO, dyn_tanh_kernel<TA, TO, 4, false><<<grid, nt, 0, st>>>(
+        x, (const TA*)a, sa, MxPart{}, ids, (const TA*)table, vocab, scale, alpha1, w1, b1, alpha2, w2, b2, (TO*)out, W, rows, T)));
   else
-    MX_DISPATCH(dt_a, TA, MX_DISPATCH(dt_out, TO, dyn_tanh_kernel<TA, TO, 1><<<grid, nt, 0, st>>>(
-        x, (const TA*)a, sa, ids, (const TA*)table, vocab, scale, alpha1, w1, b1, alpha2, w2, b2, (TO*)out, W, rows, T)));
+    MX_DISPATCH(dt_a, TA, MX_DISPATCH(dt_out, TO, dyn_tanh_kernel<TA, TO, 1, false><<<grid, nt, 0, st>>>(
+        x, (const TA*)a, sa, MxPart{}, ids, (const TA*)table, vocab, scale, alpha1, w1, b1, alpha2, w2, b2, (TO*)out, W, rows, T)));
+  MX_RETURN_LAUNCH();
+}
+
+// x <- x + D1(a) and out = D2(x) (out may be null) for a sublayer output that is still apart; W and all rows in whole fours
+MX_API int mx_dyn_tanh_parts(float* x, const MxPart* a, int dt_a, float alpha1, const float* w1, const float* b1, float alpha2,
+                             const float* w2, const float* b2, void* out, int dt_out, int T, int W, hipStream_t st) {
+  if (T <= 0) return 0;
+  if (a == nullptr || w1 == nullptr || b1 == nullptr || (out != nullptr && (w2 == nullptr || b2 == nullptr)) || W <= 0 || W % 4 ||
+      !mx_part_by_four(*a, dt_a) || ((size_t)x | (size_t)w1 | (size_t)b1 | (size_t)w2 | (size_t)b2) % 16 || !mx_by_four(out, W, dt_out))
+    return (int)hipErrorInvalidValue;
+  const int cols = W / 4, nt = cols >= 256 ? 256 : (cols + 63) / 64 * 64;
+  const int rows = T >= 2048 ? 4 : (T >= 1024 ? 2 : 1);
+  const dim3 grid((T + rows - 1) / rows, (cols + nt - 1) / nt);
+  MX_DISPATCH(dt_a, TA, MX_DISPATCH(dt_out, TO, dyn_tanh_kernel<TA, TO, 4, true><<<grid, nt, 0, st>>>(
+      x, (const TA*)a, 0, *a, nullptr, (const TA*)nullptr, 0, 1.f, alpha1, w1, b1, alpha2, w2, b2, (TO*)out, W, rows, T)));
   MX_RETURN_LAUNCH();
 }
 

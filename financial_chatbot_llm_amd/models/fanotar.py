@@ -86,6 +86,7 @@ class _Layer(Layer):
             self.ff = RoutedFF(mlp, width, score="sigmoid", renorm=True)
         else:
             raise ValueError(f"layer {i}: unknown feed-forward kind {mlp['kind']!r}")
+        self.leave_parts()
         self.width = width
         self.w_ff = None
         self.dt = {}             # norm name -> mx.DynTanh

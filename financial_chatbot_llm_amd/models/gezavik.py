@@ -68,6 +68,7 @@ class _Layer(Layer):
             self.ff = RoutedFF(mlp, width, alpha=1.702)
         else:
             raise ValueError(f"layer {i}: unknown feed-forward kind {mlp['kind']!r}")
+        self.leave_parts()
 
 
 class GezavikModel(LayeredDecoder):

@@ -43,6 +43,13 @@ class Layer:
     def norms(self):
         return self.norm_names
 
+    def leave_parts(self) -> None:
+        """The sublayers' outputs go to a norm that adds up their parts itself (:data:`..ops.mixers.Sublayer`: a product's K slices,
+        a token's routed rows): they are left so."""
+        for m in (self.mixer, getattr(self.mixer, "left", None), getattr(self.mixer, "right", None), self.ff):
+            if m is not None:
+                m.parts = True
+
     def extra_shapes(self) -> Dict[str, tuple]:
         """Further per-layer tensors of the design: {name after the layer prefix: shape}."""
         return {}

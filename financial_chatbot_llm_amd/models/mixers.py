@@ -139,6 +139,7 @@ class _ExpertBank:
 
 class Mamba2Mixer:
     kind = "mamba2"
+    parts = False              # leave the output to the norm behind it (``Layer.leave_parts``)
 
     def __init__(self, spec: Dict, width: int, eps: float):
         self.H, self.P, self.N = int(spec["heads"]), int(spec["vdim"]), int(spec["state"])
@@ -181,7 +182,7 @@ class Mamba2Mixer:
                         self.H, self.P, self.N, self.G, meta.seg_max_len)
         # the gate comes before the norm: rms over silu(z) * y, in norm_groups equal parts
         yn = mx.group_norm(y, self.norm_w, self.eps, self.norm_groups, gate=z, out_dtype=proj.dtype)
-        return project(yn, self.o)
+        return project(yn, self.o, self.parts)
 
 
 class LatentAttentionMixer:
@@ -191,6 +192,7 @@ class LatentAttentionMixer:
     :func:`..ops.mixers.rope_freqs`); score = (q . k + q_rot . k_rot) * scale; position i sees j with
     0 <= i - j < mask.size (no ``mask`` entry: every j <= i); head h's output times sigmoid(W_g h)_h; W_o."""
     kind = "latent_attention"
+    parts = False              # leave the output to the norm behind it (``Layer.leave_parts``)
     gated = True               # output gate per head (tensor ``g``)
     sinks = False              # exp(sink[h]) in the softmax denominator (tensor ``sink``)
     exact_weights = False      # f32 softmax weights in the value product also in bf16
@@ -258,7 +260,7 @@ class LatentAttentionMixer:
         q_lat = self.uk(q_nope)                                              # [T, H, R]
         o_lat = mx.latent_attend(q_lat, q_rot, rows, meta.seg_cu, positions, meta.seg_bt, self.window, self.scale,
                                  meta.seg_max_len, gate=gate, sink=self.sink, exact_weights=self.exact_weights)
-        return project(self.uv(o_lat).view(T, H * self.dv), self.o)
+        return project(self.uv(o_lat).view(T, H * self.dv), self.o, self.parts)
 
 
 class SinkLatentAttentionMixer(LatentAttentionMixer):
@@ -272,6 +274,8 @@ class DenseFF:
     """W_down act(W_up h), ``act`` = "relu2" (the square of relu) | gelu_tanh | silu; or, ``gated``,
     W_down (act(W_gate h) * (W_up h)) with ``act`` in silu | gelu_tanh, or with ``act`` = "clamped" the unit
     g * sigmoid(alpha g) * (u + 1) of g = min(W_gate h, limit), u = clamp(W_up h, +-limit) (the spec's ``limit``)."""
+
+    parts = False              # leave the output to the norm behind it (``Layer.leave_parts``)
 
     def __init__(self, spec: Dict, width: int, act: str = "relu2", gated: bool = False, alpha: float = 1.702):
         self.ff, self.width, self.act, self.gated = int(spec["ff"]), width, act, gated
@@ -299,10 +303,10 @@ class DenseFF:
         if self.gated:
             gate, up = proj[:, :self.ff], proj[:, self.ff:2 * self.ff]
             if self.act == "clamped":
-                return project(mx.glu_clamp(gate, up, self.limit, self.alpha), self.down)
-            return project(mx.glu_act(gate, up, self.act), self.down)
+                return project(mx.glu_clamp(gate, up, self.limit, self.alpha), self.down, self.parts)
+            return project(mx.glu_act(gate, up, self.act), self.down, self.parts)
         up = proj[:, :self.ff]
-        return project(mx.relu2(up) if self.act == "relu2" else mx.glu_act(up, None, self.act), self.down)
+        return project(mx.relu2(up) if self.act == "relu2" else mx.glu_act(up, None, self.act), self.down, self.parts)
 
 
 class RoutedFF:
@@ -315,6 +319,8 @@ class RoutedFF:
     instead of ``correction``), the ``top`` largest are chosen and the weights are the softmax over the chosen
     logits.  An identity expert returns its input.  Expert: g = min(W_g h, limit), u = clamp(W_u h, +-limit),
     W_d (g * sigmoid(alpha g) * (u + 1)).  A shared expert of the same form runs for every token."""
+
+    parts = False              # leave the output to the norm behind it (``Layer.leave_parts``)
 
     def __init__(self, spec: Dict, width: int, alpha: float = 1.702, score: str = "softmax", renorm: bool = False):
         r = spec["router"]
@@ -360,13 +366,15 @@ class RoutedFF:
         shared = None
         if self.Fs:
             shared = project(mx.glu_clamp(proj[:, :self.Fs], proj[:, self.Fs:2 * self.Fs], self.limit_s, self.alpha),
-                             self.down_s)
+                             self.down_s, self.parts)
         if self.score == "softmax_top":
             wts, idx = mx.router_scores(h, self.router, self.correction, top, "softmax_top")
         else:
             wts, idx = mx.router_biased(h, self.router, self.correction, top, self.score, self.renorm, self.w_scale)
         ys, pos = self.bank.run(h, idx, "clamped", self.limit, self.alpha)
-        return mx.moe_combine(ys, pos, idx, wts, h, shared, self.E)
+        if self.parts and self.bank.native:
+            return mx.Routed(ys, pos, idx, wts, h, shared, self.E, self.I > 0)
+        return mx.moe_combine(ys, pos, idx, wts, h, mx.whole(shared), self.E)
 
 
 class InputScaledRoutedFF:
@@ -377,6 +385,8 @@ class InputScaledRoutedFF:
     multiplies the expert's INPUT: out = sum_e expert_e(s_e h), expert(x) = W_d (act(W_g x) * (W_u x)).
     Since W (s h) = s (W h), the experts' first projections run on h itself and the activation
     kernel applies s to both halves."""
+
+    parts = False              # leave the output to the norm behind it (``Layer.leave_parts``)
 
     def __init__(self, spec: Dict, width: int, act: str = "silu", score: str = "sigmoid"):
         r = spec["router"]
@@ -408,6 +418,8 @@ class InputScaledRoutedFF:
         unrounded values (fewer swapped near-ties against an exact evaluation)."""
         wts, idx = mx.router_scores(x32 if x32 is not None else h, self.router, None, self.top, self.score)
         ys, pos = self.bank.run(h, idx, self.act, scale=wts)
+        if self.parts and self.bank.native:
+            return mx.Routed(ys, pos, idx, None, h, None, self.E, False)
         return mx.moe_combine(ys, pos, idx, None, h, None, self.E)
 
 
@@ -470,6 +482,7 @@ class ChannelDeltaMixer:
     Output: o / rms(o) * w_norm * sigmoid(W_g2 W_g1 h), then W_o.  Slot state: S and the last
     taps - 1 inputs of the three convolutions."""
     kind = "channel_delta"
+    parts = False              # leave the output to the norm behind it (``Layer.leave_parts``)
 
     def __init__(self, spec: Dict, width: int, eps: float):
         self.H, self.G = int(spec["heads"]), int(spec.get("kv_heads", spec["heads"]))
@@ -515,7 +528,7 @@ class ChannelDeltaMixer:
                            meta.seg_state, positions, H, self.G, self.D, self.P, "delta", A_log=self.A_log, beta=beta,
                            max_len=meta.seg_max_len)
         gate = project(proj[:, C + H + self.ra:C + H + self.ra + self.rg], self.g2)
-        return project(mx.head_norm_gate(o, self.norm_w, self.eps, gate, H, "sigmoid", proj.dtype), self.o)
+        return project(mx.head_norm_gate(o, self.norm_w, self.eps, gate, H, "sigmoid", proj.dtype), self.o, self.parts)
 
 
 class GLAMixer:
@@ -524,6 +537,7 @@ class GLAMixer:
     S [dim, vdim]: S <- diag(alpha) S + k v^T, o = S^T q.  Output: RMS norm of each head's o times
     w_norm, times silu(W_g h), then W_o."""
     kind = "gla"
+    parts = False              # leave the output to the norm behind it (``Layer.leave_parts``)
 
     def __init__(self, spec: Dict, width: int, eps: float):
         self.H, self.D, self.P = int(spec["heads"]), int(spec["dim"]), int(spec["vdim"])
@@ -560,7 +574,7 @@ class GLAMixer:
                            meta.seg_cu, meta.seg_state, positions, self.H, self.H, self.D, self.P, "gla", tau=self.tau,
                            max_len=meta.seg_max_len)
         gate = proj[:, 2 * nq + nv:2 * nq + 2 * nv]
-        return project(mx.head_norm_gate(o, self.norm_w, self.eps, gate, self.H, "silu", proj.dtype), self.o)
+        return project(mx.head_norm_gate(o, self.norm_w, self.eps, gate, self.H, "silu", proj.dtype), self.o, self.parts)
 
 
 class WindowAttentionMixer:
@@ -570,6 +584,7 @@ class WindowAttentionMixer:
     0 <= i - j < mask.size (no ``mask`` entry: plain causal); head h's output times
     sigmoid(W_g h)_h; then W_o.  The cache holds one row [k | v] per token."""
     kind = "window_attention"
+    parts = False              # leave the output to the norm behind it (``Layer.leave_parts``)
 
     def __init__(self, spec: Dict, width: int, eps: float):
         self.H, self.G = int(spec["heads"]), int(spec.get("kv_heads", spec["heads"]))
@@ -607,7 +622,7 @@ class WindowAttentionMixer:
         gate = proj[:, nq + nk + nv:nq + nk + nv + self.H]
         o = mx.window_attend(q, rows, meta.seg_cu, positions, meta.seg_bt, self.window, self.scale, meta.seg_max_len,
                              self.H, self.G, self.D, self.P, gate=gate)
-        return project(o, self.o)
+        return project(o, self.o, self.parts)
 
 
 class GatedLRUMixer:
@@ -617,6 +632,7 @@ class GatedLRUMixer:
     a = exp(-8 r softplus(lam));  S <- a S + sqrt(1 - a^2) i u (from S = 0, no special first token);
     output W_o (S * y).  Slot state: S (f32) and the last taps - 1 biased convolution inputs."""
     kind = "gated_lru"
+    parts = False              # leave the output to the norm behind it (``Layer.leave_parts``)
 
     def __init__(self, spec: Dict, width: int, eps: float):
         self.R, self.B, self.K = int(spec["width"]), int(spec["blocks"]), int(spec["conv"])
@@ -653,7 +669,7 @@ class GatedLRUMixer:
                         meta.seg_max_len, "none", in_bias=self.x_b)
         s = mx.lru_blocks(u, self.w_ri, self.r_b, self.i_b, self.lam, proj[:, :R], self.y_b, st["S"], meta.seg_cu,
                           meta.seg_state, positions, proj.dtype, max_len=meta.seg_max_len)
-        return project(s, self.o)
+        return project(s, self.o, self.parts)
 
 
 def _decays(spec: Dict, heads: int) -> torch.Tensor:
@@ -1086,6 +1102,7 @@ class ConvAttentionMixer:
     With ``kv_from`` = j the layer has no keys and values of its own: it attends over layer j's cache rows
     (``forward``'s ``kv_cache``) and convolves its queries only."""
     kind = "conv_attention"
+    parts = False              # leave the output to the norm behind it (``Layer.leave_parts``)
 
     def __init__(self, spec: Dict, width: int, eps: float):
         self.H, self.G = int(spec["heads"]), int(spec.get("kv_heads", spec["heads"]))
@@ -1148,7 +1165,7 @@ class ConvAttentionMixer:
         o = mx.window_attend(q, rows, meta.seg_cu, positions, meta.seg_bt, self.window, self.scale, meta.seg_max_len,
                              self.H, self.G, self.D, self.P, gate=proj[:, self.C:self.C + self.no], slopes=self.slopes,
                              sink=self.sink)
-        return project(o, self.o)
+        return project(o, self.o, self.parts)
 
 
 class _GroupedAttention:

@@ -76,6 +76,7 @@ class _Layer(Layer):
             self.ff = InputScaledRoutedFF(mlp, width, act="silu", score="sigmoid")
         else:
             raise ValueError(f"layer {i}: unknown feed-forward kind {mlp['kind']!r}")
+        self.leave_parts()
         self.w_ff = None
         self.norm2 = None
 

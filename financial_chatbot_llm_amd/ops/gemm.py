@@ -20,6 +20,7 @@ with ``bench/kernels.py`` (profiles named next to each table).
 from __future__ import annotations
 
 import contextlib
+import functools
 import os
 import threading
 from typing import Dict, List, Optional, Tuple, Union
@@ -286,10 +287,11 @@ def transformed(x: torch.Tensor) -> bool:
         torch.jit.is_tracing()
 
 
-def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+def project(x: torch.Tensor, w: torch.Tensor, slabs: bool = False) -> Union[torch.Tensor, "Slabs"]:
     """y = x @ w.T in bf16 or f32: the streaming kernels for up to about two thousand rows (``penny_linear_rows_plan``; inside
     :func:`replayed` ``penny_linear_rows_replay_plan``), deep rings of larger tiles where one round of them holds 257 to 3072 rows in
-    bf16 (``penny_project_ring_plan``), the library's product for the rest."""
+    bf16 (``penny_project_ring_plan``), the library's product for the rest.  ``slabs``: a product in slices of K is left as
+    :class:`Slabs` for a reader that sums them itself."""
     dt = x.dtype
     if dt == w.dtype and (dt == torch.bfloat16 or dt == torch.float32) and x.dim() == 2 and w.dim() == 2 and N.use_native(x) and \
             not torch.is_autocast_enabled():
@@ -306,11 +308,11 @@ def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
             plan = lib.penny_linear_rows_replay_plan(M, N_, K, f32) if replay else lib.penny_linear_rows_plan(M, N_, K, f32)
             if plan:
                 S = plan >> 16
-                y = torch.empty((M, N_), dtype=dt, device=x.device)
-                slabs = torch.empty((S, M, N_), dtype=torch.float32, device=x.device) if S > 1 else None
-                N.call("penny_linear_rows", xp, ldx, wp, K, y.data_ptr(), M, N_, N.ptr(slabs), S, plan & 255, plan >> 8 & 255, f32,
+                P = torch.empty((S, M, N_), dtype=torch.float32, device=x.device) if S > 1 else None
+                y = None if slabs and S > 1 else torch.empty((M, N_), dtype=dt, device=x.device)
+                N.call("penny_linear_rows", xp, ldx, wp, K, N.ptr(y), M, N_, N.ptr(P), S, plan & 255, plan >> 8 & 255, f32,
                        PAIR_MODE != "0", N.stream())
-                return y
+                return Slabs(P, dt) if y is None else y
     return F.linear(x, w)
 
 
@@ -612,19 +614,21 @@ class ResidualSum:
 class Slabs:
     """A split-K GEMM output left unreduced: f32 partial sums ``P`` [S, M, N].  Consumers that
     read the activation anyway (``ops.rms_norm``, ``ops.rope_kv_write``) sum the slabs inside
-    their own row pass; anything else calls :meth:`materialize`."""
+    their own row pass; anything else calls :meth:`materialize`.  ``dtype``: the output's type, to which the sum is rounded."""
 
-    __slots__ = ("P",)
+    __slots__ = ("P", "dtype")
 
-    def __init__(self, P: torch.Tensor):
-        self.P = P
+    def __init__(self, P: torch.Tensor, dtype: torch.dtype = torch.bfloat16):
+        self.P, self.dtype = P, dtype
 
     @property
     def shape(self) -> Tuple[int, int]:
         return (self.P.shape[1], self.P.shape[2])
 
     def materialize(self) -> torch.Tensor:
-        return splitk_reduce(self.P)
+        if self.dtype == torch.bfloat16:
+            return splitk_reduce(self.P)
+        return functools.reduce(torch.add, self.P.unbind(0)).to(self.dtype)
 
 
 def splitk_partials(x: torch.Tensor, wt: torch.Tensor, N_: int, S: int, nf: int,

@@ -32,13 +32,15 @@ segment whose first row is at position 0 starts from zero state whatever its slo
 """
 from __future__ import annotations
 
+import ctypes
 import functools
-from typing import NamedTuple, Optional, Tuple
+from typing import NamedTuple, Optional, Tuple, Union
 
 import torch
 import torch.nn.functional as F
 
 from . import _native as N
+from .gemm import Slabs
 
 PAGE = 64
 
@@ -61,6 +63,92 @@ def _rows(t: torch.Tensor) -> torch.Tensor:
 # ----------------------------------------------------------------------------------------------
 # residual stream
 # ----------------------------------------------------------------------------------------------
+class Routed(NamedTuple):
+    """A routed feed-forward's output whose rows the norm behind it adds up (the operands of :func:`moe_combine`)."""
+    ys: torch.Tensor
+    pos: torch.Tensor
+    idx: torch.Tensor
+    wts: Optional[torch.Tensor]
+    h: torch.Tensor
+    shared: Union[torch.Tensor, Slabs, None]
+    num_experts: int
+    identity: bool = True        # entries >= num_experts may occur
+
+    @property
+    def dtype(self) -> torch.dtype:
+        return self.ys.dtype
+
+    def materialize(self) -> torch.Tensor:
+        return moe_combine(self.ys, self.pos, self.idx, self.wts, self.h, whole(self.shared), self.num_experts)
+
+
+Sublayer = Union[torch.Tensor, Slabs, Routed]
+
+
+def whole(v: Optional[Sublayer]) -> Optional[torch.Tensor]:
+    """A sublayer's output written out."""
+    return v if v is None or isinstance(v, torch.Tensor) else v.materialize()
+
+
+class _Part(ctypes.Structure):
+    """``MxPart`` of ``csrc/mixers/mx_common.h``."""
+    _fields_ = [("p", ctypes.c_void_p), ("ld", ctypes.c_long), ("slab", ctypes.c_long), ("ys", ctypes.c_void_p), ("sy", ctypes.c_long),
+                ("pos", ctypes.c_void_p), ("idx", ctypes.c_void_p), ("wts", ctypes.c_void_p), ("h", ctypes.c_void_p), ("sh", ctypes.c_long),
+                ("slabs", ctypes.c_int), ("E", ctypes.c_int), ("top", ctypes.c_int)]
+
+
+def _by_four(t: torch.Tensor) -> bool:
+    ld, one = t.stride()
+    return one == 1 and ld % 4 == 0 and t.data_ptr() % (16 if t.dtype == torch.float32 else 8) == 0
+
+
+def _part(v: Sublayer, T: int, W: int) -> Optional[_Part]:
+    """The parts of a sublayer output [T, W] for the kernels that add them up, or None: rows that they do not read by four."""
+    r = v if isinstance(v, Routed) else None
+    base = v if r is None else r.shared
+    p, ld, slab, slabs = None, 0, 0, 0
+    if base is not None:
+        if base.shape != (T, W) or base.dtype != v.dtype:
+            raise ValueError(f"a sublayer's output is [{T}, {W}], all of one type")
+        if isinstance(base, Slabs):
+            p, ld, slab, slabs = base.P.data_ptr(), W, T * W, base.P.shape[0]
+            if p % 16 or not base.P.is_contiguous():
+                return None
+        elif _by_four(base):
+            p, ld = base.data_ptr(), base.stride(0)
+        else:
+            return None
+    if r is None:
+        return _Part(p, ld, slab, None, 0, None, None, None, None, 0, slabs, 0, 0)
+    ys, pos, idx, wts, h = r[:5]
+    many = idx.shape
+    if len(many) != 2 or many[0] != T or pos.shape != many or ys.shape[1] != W or h.shape != (T, W) or ys.dtype != h.dtype or \
+            (wts is not None and wts.shape != many):
+        raise ValueError("a routed output has an entry per token and choice")
+    if not (_by_four(ys) and _by_four(h) and idx.is_contiguous() and pos.is_contiguous() and (wts is None or wts.is_contiguous())):
+        return None
+    # (no identity entries: h, which may be the stream that is written, is not read)
+    return _Part(p, ld, slab, ys.data_ptr(), ys.stride(0), pos.data_ptr(), idx.data_ptr(), N.ptr(wts), h.data_ptr() if r.identity else None,
+                 h.stride(0), slabs, r.num_experts if r.identity else 0x7fffffff, many[1])
+
+
+def _parts(x: torch.Tensor, a: Optional[Sublayer], b: Optional[Sublayer], widest: int):
+    """(parts of a, parts of b) where a kernel of rows up to ``widest`` columns adds them up into ``x``, else None."""
+    if (a is None or type(a) is torch.Tensor) and (b is None or type(b) is torch.Tensor):
+        return None
+    T, W = x.shape
+    if a is None or W % 4 or W > widest or x.data_ptr() % 16 or (b is not None and a.dtype != b.dtype) or not N.use_native(x):
+        return None
+    for v in (a, b):
+        if isinstance(v, Routed) and v.identity and v.h.untyped_storage().data_ptr() == x.untyped_storage().data_ptr():
+            return None
+    p = _part(a, T, W)
+    if p is None or b is None:
+        return None if p is None else (ctypes.byref(p), None)
+    q = _part(b, T, W)
+    return None if q is None else (ctypes.byref(p), ctypes.byref(q))
+
+
 def embed_f32(ids: torch.Tensor, table: torch.Tensor) -> torch.Tensor:
     """Token rows of ``table`` (bf16 or f32) as an f32 residual stream [T, W]."""
     T, (V, W) = ids.numel(), table.shape
@@ -72,8 +160,8 @@ def embed_f32(ids: torch.Tensor, table: torch.Tensor) -> torch.Tensor:
     return table[ids.long().clamp(0, V - 1)].float()
 
 
-def residual_norm(x: torch.Tensor, w: Optional[torch.Tensor], eps: float, a: Optional[torch.Tensor] = None,
-                  b: Optional[torch.Tensor] = None, mult: float = 1.0,
+def residual_norm(x: torch.Tensor, w: Optional[torch.Tensor], eps: float, a: Optional[Sublayer] = None,
+                  b: Optional[Sublayer] = None, mult: float = 1.0,
                   out_dtype: torch.dtype = torch.bfloat16, mult_b: Optional[float] = None,
                   gate: Optional[torch.Tensor] = None, gate_bias: Optional[torch.Tensor] = None,
                   ids: Optional[torch.Tensor] = None, table: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
@@ -96,8 +184,15 @@ def embed_norm(ids: torch.Tensor, table: torch.Tensor, w: torch.Tensor, eps: flo
 def _residual_norm(x, w, eps, a, b, mult, out_dtype, mult_b, gate, gate_bias, ids, table, fresh):
     T, W = x.shape
     assert x.dtype == torch.float32 and x.is_contiguous()
-    ab = a if a is not None else b
     mult_b = mult if mult_b is None else mult_b
+    parts = _parts(x, a, b, 8192) if gate is None and table is None and w is not None and w.data_ptr() % 16 == 0 else None
+    if parts is not None:
+        out = torch.empty((T, W), dtype=out_dtype, device=x.device)
+        N.mcall("mx_residual_norm_parts", N.ptr(x), parts[0], parts[1], int(a.dtype == torch.float32), float(mult), float(mult_b), N.ptr(w),
+                float(eps), N.ptr(out), _dt(out), T, W, N.stream())
+        return out
+    a, b = whole(a), whole(b)
+    ab = a if a is not None else b
     if gate is not None and ab is None:
         raise ValueError("a gate needs a sublayer output to act on")
     if table is not None and (ids is None or ids.numel() != T or table.shape[1] != W):
@@ -173,11 +268,21 @@ def dyn_tanh_embed(ids: torch.Tensor, table: torch.Tensor, scale: float, norm: D
     return x, post.plain(x).to(out_dtype) if post is not None else None
 
 
-def dyn_tanh_residual(x: torch.Tensor, y: Optional[torch.Tensor], norm: Optional[DynTanh], post: Optional[DynTanh] = None,
+def dyn_tanh_residual(x: torch.Tensor, y: Optional[Sublayer], norm: Optional[DynTanh], post: Optional[DynTanh] = None,
                       out_dtype: torch.dtype = torch.bfloat16) -> Optional[torch.Tensor]:
     """``x`` (f32 [T, W], in place) <- x + norm(y) for a sublayer's output ``y`` (None: x stays), then post(x) in
     ``out_dtype`` (the next sublayer's input; ``post`` None: the update only), in one pass."""
     T, W = x.shape
+    parts = _parts(x, y, None, 1 << 30) if norm is not None and all(
+        (d.w.data_ptr() | d.b.data_ptr()) % 16 == 0 for d in (norm, post) if d is not None) else None
+    if parts is not None:
+        assert x.dtype == torch.float32 and x.is_contiguous()
+        out = torch.empty((T, W), dtype=out_dtype, device=x.device) if post is not None else None
+        N.mcall("mx_dyn_tanh_parts", N.ptr(x), parts[0], int(y.dtype == torch.float32), norm.alpha, N.ptr(norm.w), N.ptr(norm.b),
+                post.alpha if post is not None else 0.0, N.ptr(post.w) if post is not None else None,
+                N.ptr(post.b) if post is not None else None, N.ptr(out), _dt(out) if out is not None else 1, T, W, N.stream())
+        return out
+    y = whole(y)
     assert x.dtype == torch.float32 and x.is_contiguous() and (y is None or (y.shape == x.shape and norm is not None))
     if N.use_native(x):
         out = torch.empty((T, W), dtype=out_dtype, device=x.device) if post is not None else None
@@ -730,8 +835,8 @@ def layer_norm_out(x: torch.Tensor, w: torch.Tensor, eps: float, out_dtype: torc
     return _ln(x, w, eps).to(out_dtype)
 
 
-def post_norm_add(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, eps: float, out_dtype: Optional[torch.dtype] = None,
-                  b: Optional[torch.Tensor] = None, wa: Optional[torch.Tensor] = None,
+def post_norm_add(x: torch.Tensor, a: Sublayer, w: torch.Tensor, eps: float, out_dtype: Optional[torch.dtype] = None,
+                  b: Optional[Sublayer] = None, wa: Optional[torch.Tensor] = None,
                   wb: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """``x`` (f32 [T, W], in place) <- x + LayerNorm(m) * w, the norm on the sublayer's output only.
     m = a, or with a second branch m = (RMSnorm(a) * wa + RMSnorm(b) * wb) / 2 (two mixers side by
@@ -740,6 +845,13 @@ def post_norm_add(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, eps: float,
     T, W = x.shape
     assert x.dtype == torch.float32 and x.is_contiguous()
     want = out_dtype is not None and out_dtype != torch.float32
+    parts = _parts(x, a, b, 4096) if (w.data_ptr() | (N.ptr(wa) or 0) | (N.ptr(wb) or 0)) % 16 == 0 else None
+    if parts is not None:
+        out = torch.empty((T, W), dtype=out_dtype, device=x.device) if want else None
+        N.mcall("mx_post_norm_parts", N.ptr(x), parts[0], N.ptr(wa), parts[1], N.ptr(wb), int(a.dtype == torch.float32), N.ptr(w), float(eps),
+                N.ptr(out), _dt(out) if want else 1, T, W, N.stream())
+        return out if want else x
+    a, b = whole(a), whole(b)
     if N.use_native(x):
         out = torch.empty((T, W), dtype=out_dtype, device=x.device) if want else None
         if b is not None:
