@@ -193,7 +193,7 @@ __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restr
   X += (long)m0 * ldx;
   if constexpr (EPI == SK_SILU || EPI == SK_BF16 || EPI == SK_BIAS) Y += (long)m0 * ldy;
   PENNY_DASSERT(M > 0 && (EPI != SK_SAMPLE || gridDim.y == 1));
-  PENNY_DASSERT((tile + 1) * 16 * NF <= N || (WROW && N % 16 == 0 && tile * 16 * NF < N && (EPI == SK_BF16 || EPI == SK_BIAS || EPI == SK_SLAB || EPI == SK_F32)));
+  PENNY_DASSERT((tile + 1) * 16 * NF <= N || (WROW && N % 8 == 0 && tile * 16 * NF < N && (EPI == SK_BF16 || EPI == SK_BIAS || EPI == SK_SLAB || EPI == SK_F32)));
   PENNY_DASSERT(K % (64 * BKM * S) == 0);
   const int n0 = tile * 16 * NF;
   const int kc = K / S, k0 = s * kc;
@@ -326,10 +326,11 @@ __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restr
       if (m >= M) continue;
 #pragma unroll
       for (int f = 0; f < FW; ++f) {
-        if (WROW && n0 + (wa * FW + f) * 16 >= N) break;
+        const int n = n0 + (wa * FW + f) * 16 + 4 * g;
+        if (WROW && n >= N) break;
         bf16x4 o;
         if constexpr (EPI == SK_BIAS) {
-          const bf16x4 bv = *reinterpret_cast<const bf16x4*>(sa.bias + n0 + (wa * FW + f) * 16 + 4 * g);
+          const bf16x4 bv = *reinterpret_cast<const bf16x4*>(sa.bias + n);
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const bf16 v = (bf16)(acc[f][t][r] + (float)bv[r]);
@@ -339,7 +340,7 @@ __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restr
 #pragma unroll
           for (int r = 0; r < 4; ++r) o[r] = (bf16)acc[f][t][r];
         }
-        *reinterpret_cast<bf16x4*>(Y + (long)m * ldy + n0 + (wa * FW + f) * 16 + 4 * g) = o;
+        *reinterpret_cast<bf16x4*>(Y + (long)m * ldy + n) = o;
       }
     }
     return;
@@ -704,13 +705,15 @@ constexpr RowsTile kRowsTiles[] = {{2, 2, 4.6f, 13.6f}, {2, 4, 6.5f, 23.4f}, {4,
 //
 // f32 (a sixteenth of the matrix rate; the four smallest tiles): the library's tiles are 1.1 - 1.3 times faster from 40 - 100 rows on where
 // the device counts (1024 x 3072, 64 rows 10.6 / 12.3; 2048 x 1024 at 150 11.4 / 14.7) and slower below (1024 x 1024 1 row 8.3 / 6.2, 64 8.7 / 7.3;
-// 2048 x 1024 16 rows 8.8 / 6.9; 1024 x 3072 10.9 / 9.0), so up to 256 rows the products of up to 11 us are taken.  Steps at width 1024: 14
-// rows decoding 956 -> 812, 50 1023 -> 916; 200 tokens, where the host is the bound, 1575 -> 1355.  Errors against 64 bits at most the library's
+// 2048 x 1024 16 rows 8.8 / 6.9; 1024 x 3072 10.9 / 9.0), so up to 64 rows, which may be a captured step, the products of up to 11 us are taken, and
+// beyond, where the host is the bound, up to 20.  Steps at width 1024: 14 rows decoding 956 -> 812, 50 1023 -> 916; prompts (11 us up to 256 rows / 20):
+// 74 tokens 1472 / 1141, 150 beside 9 rows 1457 / 1177, 120 beside 4 1423 / 1220, 100 beside 6 1277 / 1114, 200 1440 / 1349 (of which the widths of
+// 3112 - 4136 that are no multiples of 16 a part; decoding in bf16 they alone are 30 rows 677 / 625 and 695 / 649).  Errors against 64 bits at most the library's
 // (K = 1024 1.6 - 2.9e-7 of the norm against 2.9 - 5.8e-7, K = 3072 2.0 - 2.6e-7 against 5.0e-7).
 static int rows_plan(int M, int N, int K, int f32, float& best) {
-  if (M <= 0 || M > (f32 ? 256 : 2048) || N < 512 || N % 16 || K <= 0 || K % (f32 ? 32 : 64)) return 0;
+  if (M <= 0 || M > (f32 ? 256 : 2048) || N < 512 || N % 8 || K <= 0 || K % (f32 ? 32 : 64)) return 0;
   int plan = 0;
-  best = f32 ? 11.f : M <= 96 ? 60.f : M <= 512 ? 20.f : 20.f - (M - 512) / 128.f;
+  best = f32 ? (M <= 64 ? 11.f : 20.f) : M <= 96 ? 60.f : M <= 512 ? 20.f : 20.f - (M - 512) / 128.f;
   for (int S = 1; S <= (f32 ? 8 : 4); S *= 2) {
     if (S > 1 && (K % (64 * S) || K / S < 256)) break;
     for (int i = 0; i < (f32 ? 4 : (int)(sizeof(kRowsTiles) / sizeof(kRowsTiles[0]))); ++i) {
@@ -754,7 +757,7 @@ PENNY_API int penny_linear_rows_replay_plan(int M, int N, int K, int f32) {
 extern "C" int penny_rows_slabs(const void* X, int ldx, const void* W, int K, float* slabs, int M, int N, int S, int nf, int mt, int paired,
                                 hipStream_t st) {
   if (M <= 0) return 0;
-  if (M > (1 << 20) || N <= 0 || N % 16 || S < 1 || K <= 0 || K % (64 * S) || ldx % 8) return (int)hipErrorInvalidValue;
+  if (M > (1 << 20) || N <= 0 || N % 8 || S < 1 || K <= 0 || K % (64 * S) || ldx % 8) return (int)hipErrorInvalidValue;
 #define SLABS_CASE(NF_, MT_, WA_) \
   if (nf == NF_ && mt == MT_) return launch<NF_, MT_, WA_, true>(X, ldx, W, K, slabs, M, N, S, paired ? 3 : 1, st);
   ROWS_TILES(SLABS_CASE)
@@ -764,12 +767,12 @@ extern "C" int penny_rows_slabs(const void* X, int ldx, const void* W, int K, fl
 
 // Y [M, N] = X [M, K] x W [N, K]^T in bf16 or f32 (f32 != 0) for up to about two thousand rows, W row-major: slabs == null streams W once (S = 1), else
 // S slices of K leave f32 slabs [S, M, N] that a second launch adds, or with Y null the reader.  One entry for both, so that a step that
-// the host bounds pays for one call.  nf, mt: a block's columns and rows in units of 16, one of kRowsTiles.  Contract (checked): N % 16 == 0 (the last
+// the host bounds pays for one call.  nf, mt: a block's columns and rows in units of 16, one of kRowsTiles.  Contract (checked): N % 8 == 0 (the last
 // tile may be part-filled), K % (64 * S) == 0 (f32: 32 * S), rows of x in whole 16 bytes, y contiguous.
 PENNY_API int penny_linear_rows(const void* X, int ldx, const void* W, int K, void* Y, int M, int N, void* slabs, int S, int nf, int mt,
                                 int f32, int paired, hipStream_t st) {
   if (M <= 0) return 0;
-  if (M > (1 << 20) || N <= 0 || N % 16 || S < 1 || (S > 1) != (slabs != nullptr) || (S == 1 && Y == nullptr) || K <= 0 ||
+  if (M > (1 << 20) || N <= 0 || N % 8 || S < 1 || (S > 1) != (slabs != nullptr) || (S == 1 && Y == nullptr) || K <= 0 ||
       K % ((f32 ? 32 : 64) * S) || K > (1 << 28) || ldx % (f32 ? 4 : 8))
     return (int)hipErrorInvalidValue;
   float* p = static_cast<float*>(f32 && S == 1 ? Y : slabs);

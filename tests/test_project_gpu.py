@@ -55,6 +55,23 @@ def test_every_tile():
         N.call("penny_linear_rows", N.ptr(x), 512, N.ptr(w), 512, N.ptr(y), 150, 528, None, 1, 2, 16, 0, 1, N.stream())
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M", [1, 16, 33, 100, 256])
+@pytest.mark.parametrize("N_,K", [(520, 64), (536, 512), (3208, 1024), (3112, 1024), (1032, 4096)])
+def test_widths_in_eights(dt, M, N_, K):
+    """The last sixteen of columns half filled: one launch, slices of K, and the slices left to the reader."""
+    g = torch.Generator(device="cuda").manual_seed(M + N_)
+    w = (torch.randn((N_, K), generator=g, device="cuda") * K ** -0.5).to(dt)
+    x = torch.randn((M, K), generator=g, device="cuda").to(dt)
+    want = x.double() @ w.double().t()
+    e = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -20
+    assert rows_config(M, N_, K, dt) is not None or dt == torch.float32
+    y = G.project(x, w)
+    assert ((y.double() - want).abs() <= want.abs() * e + 2.0 ** -18 * K ** 0.5).all()
+    p = G.project(x, w, slabs=True)
+    assert torch.equal(p.materialize() if isinstance(p, G.Slabs) else p, y)
+
+
 def test_rule():
     assert rows_config(64, 2048, 4096) == (2, 4, 4) and rows_config(64, 4096, 2048) == (2, 2, 1) and rows_config(1, 7216, 2048) == (2, 2, 1)
     assert rows_config(256, 2048, 2048) == (2, 4, 1) and rows_config(512, 1024, 1024) == (2, 4, 1)
