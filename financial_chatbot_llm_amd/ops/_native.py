@@ -43,6 +43,7 @@ _SIGS = {
     "penny_few_rows": [P, c_int, P, c_float, P, c_int, c_int, P, c_int, c_int, c_int, P],
     "penny_bias_rows_plan": [c_int, c_int, c_int],
     "penny_bias_peeled_rows": [c_int, c_int, c_int, c_int, c_int],
+    "penny_linear_rows_f32_plan": [c_int, c_int, c_int],
     "penny_linear_rows_plan": [c_int, c_int, c_int, c_int],
     "penny_linear_rows_replay_plan": [c_int, c_int, c_int, c_int],
     "penny_linear_ring_plan": [c_int, c_int, c_int],

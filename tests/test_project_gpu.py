@@ -72,6 +72,21 @@ def test_widths_in_eights(dt, M, N_, K):
     assert torch.equal(p.materialize() if isinstance(p, G.Slabs) else p, y)
 
 
+@pytest.mark.parametrize("M,N_,K,here", [(256, 1024, 1024, True), (257, 1024, 1024, True), (384, 1024, 64, True), (338, 520, 32, True), (385, 1024, 64, False),
+                                         (338, 6144, 1024, False)])
+def test_short_f32_products(M, N_, K, here, monkeypatch):
+    """Around the rows up to which short f32 products stay here."""
+    from financial_chatbot_llm_amd.ops import _native as N
+    calls, call = [], N.call
+    monkeypatch.setattr(N, "call", lambda name, *a: (calls.append(name), call(name, *a))[1])
+    g = torch.Generator(device="cuda").manual_seed(M)
+    w, x = torch.randn((N_, K), generator=g, device="cuda") * K ** -0.5, torch.randn((M, K), generator=g, device="cuda")
+    y = G.project(x, w)
+    assert bool(calls) is here
+    want = x.double() @ w.double().t()
+    assert ((y.double() - want).abs() <= want.abs() * 2.0 ** -20 + 2.0 ** -18 * K ** 0.5).all()
+
+
 def test_rule():
     assert rows_config(64, 2048, 4096) == (2, 4, 4) and rows_config(64, 4096, 2048) == (2, 2, 1) and rows_config(1, 7216, 2048) == (2, 2, 1)
     assert rows_config(256, 2048, 2048) == (2, 4, 1) and rows_config(512, 1024, 1024) == (2, 4, 1)
