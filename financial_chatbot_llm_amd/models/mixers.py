@@ -523,11 +523,11 @@ class ChannelDeltaMixer:
         u = mx.conv_act(proj[:, :C], self.conv_w, None, st["conv"], meta.seg_cu, meta.seg_state, positions,
                         meta.seg_max_len, "silu")
         beta = proj[:, C:C + H]
-        a = project(proj[:, C + H:C + H + self.ra].float(), self.a2)
+        at = C + H + self.ra
+        a, gate = mx.low_rank(proj[:, C + H:at], self.a2, proj[:, at:at + self.rg], self.g2)
         o = mx.matrix_scan(u[:, :nq], u[:, nq:2 * nq], u[:, 2 * nq:], a, self.dt_bias, st["S"], meta.seg_cu,
                            meta.seg_state, positions, H, self.G, self.D, self.P, "delta", A_log=self.A_log, beta=beta,
                            max_len=meta.seg_max_len)
-        gate = project(proj[:, C + H + self.ra:C + H + self.ra + self.rg], self.g2)
         return project(mx.head_norm_gate(o, self.norm_w, self.eps, gate, H, "sigmoid", proj.dtype), self.o, self.parts)
 
 
@@ -569,7 +569,7 @@ class GLAMixer:
     def forward(self, proj: torch.Tensor, positions: torch.Tensor, meta: AttentionMetadata, cache) -> torch.Tensor:
         st = cache[1]
         nq, nv = self.nq, self.nv
-        a = project(proj[:, 2 * nq + 2 * nv:2 * nq + 2 * nv + self.ra].float(), self.a2)
+        a, _ = mx.low_rank(proj[:, 2 * nq + 2 * nv:2 * nq + 2 * nv + self.ra], self.a2)
         o = mx.matrix_scan(proj[:, :nq], proj[:, nq:2 * nq], proj[:, 2 * nq:2 * nq + nv], a, self.a2_b, st["S"],
                            meta.seg_cu, meta.seg_state, positions, self.H, self.H, self.D, self.P, "gla", tau=self.tau,
                            max_len=meta.seg_max_len)

@@ -116,6 +116,7 @@ _MIXER_SIGS = {
     "mx_post_norm_parts": [P, P, P, P, P, c_int, P, c_float, P, c_int, c_int, c_int, P],
     "mx_dyn_tanh_parts": [P, P, c_int, c_float, P, P, c_float, P, P, P, c_int, c_int, c_int, P],
     "mx_group_norm": [P, c_long, c_int, P, c_long, c_int, P, c_float, P, c_long, c_int, c_int, c_int, c_int, P],
+    "mx_low_rank": [P, P, c_long, P, c_int, c_int, P, c_int, c_int, P, P, c_int, c_int, P],
     "mx_relu2": [P, c_long, P, c_long, c_int, c_int, c_int, P],
     "mx_glu_clamp": [P, c_long, P, c_long, c_float, c_float, P, c_long, c_int, c_int, c_int, P],
     "mx_route_biased": [P, P, c_int, c_int, c_int, c_int, c_float, P, P, c_int, P],

@@ -40,7 +40,7 @@ import torch
 import torch.nn.functional as F
 
 from . import _native as N
-from .gemm import Slabs
+from .gemm import Slabs, project
 
 PAGE = 64
 
@@ -1035,6 +1035,25 @@ def matrix_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.Tens
             out[r0 + t] = torch.einsum("hdp,hd->hp", St, qq[t]).reshape(-1)
         state[sll[s]] = St
     return out
+
+
+def low_rank(ua: torch.Tensor, wa: torch.Tensor, ug: Optional[torch.Tensor] = None,
+             wg: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
+    """The second factors of two low-rank projections: ``ua wa^T`` in f32 (``ua`` [T, ra] bf16 or f32, ``wa`` f32) and, given, ``ug wg^T`` in
+    the type of ``ug``.  One launch for ranks of 32 and 64 (``mx_low_rank``), else a product each."""
+    (T, ra), na = ua.shape, wa.shape[0]
+    if N.use_native(ua) and T > 0 and ra in (32, 64) and na % 16 == 0 and wa.dtype == torch.float32 and wa.shape[1] == ra and wa.is_contiguous() and \
+            ua.dtype in (torch.bfloat16, torch.float32) and ua.stride(1) == 1 and ua.stride(0) * ua.element_size() % 16 == 0 and ua.stride(0) >= ra and \
+            (ua.data_ptr() | wa.data_ptr()) % 16 == 0 and T <= 1 << 23:
+        ng = 0 if ug is None else wg.shape[0]
+        if ng == 0 or (ug.shape[0] == T and ug.shape[1] in (32, 64) and ug.shape[1] <= ug.stride(0) and wg.shape[1] == ug.shape[1] and ng % 16 == 0 and ug.stride() == ua.stride() and
+                       ug.dtype == wg.dtype == ua.dtype and wg.is_contiguous() and (ug.data_ptr() | wg.data_ptr()) % 16 == 0):
+            a = torch.empty((T, na), dtype=torch.float32, device=ua.device)
+            g = torch.empty((T, ng), dtype=ua.dtype, device=ua.device) if ng else None
+            N.mcall("mx_low_rank", N.ptr(ua), N.ptr(ug), ua.stride(0), N.ptr(wa), ra, na, N.ptr(wg), ug.shape[1] if ng else 0, ng, N.ptr(a), N.ptr(g),
+                    _dt(ua), T, N.stream())
+            return a, g
+    return project(ua.float(), wa), project(ug, wg) if ug is not None else None
 
 
 def head_norm_gate(o: torch.Tensor, w: torch.Tensor, eps: float, gate: torch.Tensor, heads: int, act: str,
