@@ -401,7 +401,7 @@ latent_attend_mfma_kernel(const bf16* __restrict__ q_lat, const bf16* __restrict
     }
   }
   if (!qok) return;
-  if (nsplit > 1) {                          // unnormalised part: o | m | l, merged by latent_merge_kernel
+  if (nsplit > 1) {                          // unnormalised part: o | m | l, merged by attend_merge_kernel
     float* w = ws + ((row * H + h) * nsplit + split) * (long)(R + 2);
 #pragma unroll
     for (int nt = 0; nt < NTM; ++nt)
@@ -429,32 +429,6 @@ latent_attend_mfma_kernel(const bf16* __restrict__ q_lat, const bf16* __restrict
         if (r < R) dst[r] = (bf16)(o[nt][i] * gsc);
       }
     }
-  }
-}
-
-// grid (rows, H): combine the nsplit parts of one (row, head)
-template <typename T>
-__global__ void latent_merge_kernel(const float* __restrict__ ws, const T* __restrict__ gate, long sgate,
-                                    const float* __restrict__ sink, T* __restrict__ out, int H, int R, int nsplit) {
-  const long row = blockIdx.x;
-  const int h = blockIdx.y;
-  const float* w = ws + (row * H + h) * nsplit * (long)(R + 2);
-  float M = sink != nullptr ? sink[h] : -INFINITY;
-  for (int i = 0; i < nsplit; ++i) M = fmaxf(M, w[i * (R + 2) + R]);
-  float L = sink != nullptr ? expf(sink[h] - M) : 0.f;      // the sink counts once, not once per part
-  for (int i = 0; i < nsplit; ++i) {
-    const float mi = w[i * (R + 2) + R];
-    if (mi != -INFINITY) L += w[i * (R + 2) + R + 1] * expf(mi - M);
-  }
-  float gsc = 1.0f / L;
-  if (gate != nullptr) gsc *= mx_sigmoid(ldf(gate + row * sgate + h));
-  for (int r = threadIdx.x; r < R; r += blockDim.x) {
-    float a = 0.f;
-    for (int i = 0; i < nsplit; ++i) {
-      const float mi = w[i * (R + 2) + R];
-      if (mi != -INFINITY) a += w[i * (R + 2) + r] * expf(mi - M);
-    }
-    stf(out + (row * H + h) * R + r, a * gsc);
   }
 }
 
@@ -495,7 +469,7 @@ MX_API int mx_latent_attend(const void* q_lat, const void* q_rot, const void* ca
                             int window, float scale, void* out, int dt, int S, int max_len, int H, int R, int Dr,
                             int nsplit, float* ws, int rows, hipStream_t st) {
   if (S <= 0 || max_len <= 0) return 0;
-  if (R > 64 * ATT_RPL) return (int)hipErrorInvalidValue;
+  if (R > 64 * ATT_RPL || nsplit > 64) return (int)hipErrorInvalidValue;
   const int D = R + Dr;
   // rows_attend.h for the latent of 256 with a rotated part of 32 or none, the sizes of this framework's decoders (window 1024,
   // before -> after; 32 heads, bf16: 2048 rows of three segments 217 -> 64 us, 256 rows and 30 single ones 405 -> 75, 64 single
@@ -520,8 +494,7 @@ MX_API int mx_latent_attend(const void* q_lat, const void* q_rot, const void* ca
       else rows_attend_kernel<bf16, 256, 0, 256, true, 1, 4, 64, false, false><<<grid, 256, 0, st>>>(a);
     }
     if (nsplit > 1)
-      MX_DISPATCH(dt, TT, latent_merge_kernel<TT><<<dim3(rows, H), 128, 0, st>>>(ws, (const TT*)gate, sgate, sink, (TT*)out, H,
-                                                                                R, nsplit));
+      MX_DISPATCH(dt, TT, attend_merge(ws, (const TT*)gate, sgate, 0, sink, (TT*)out, rows, H, R, nsplit, 0, st));
     MX_RETURN_LAUNCH();
   }
   if (dt == 0 && D <= 320 && R <= 256 && mx_use_mfma()) {
@@ -544,10 +517,8 @@ MX_API int mx_latent_attend(const void* q_lat, const void* q_rot, const void* ca
       else LATENT_LAUNCH(10, 16, false);
     }
 #undef LATENT_LAUNCH
-    if (nsplit > 1) {
-      dim3 g2(S, H);           // single-row segments: row index == segment index
-      latent_merge_kernel<bf16><<<g2, R >= 128 ? 128 : 64, 0, st>>>(ws, (const bf16*)gate, sgate, sink, (bf16*)out, H, R, nsplit);
-    }
+    // (single-row segments: row index == segment index)
+    if (nsplit > 1) attend_merge(ws, (const bf16*)gate, sgate, 0, sink, (bf16*)out, S, H, R, nsplit, 0, st);
     MX_RETURN_LAUNCH();
   }
   const int esz = dt == 1 ? 4 : 2;

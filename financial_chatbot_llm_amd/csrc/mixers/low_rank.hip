@@ -1,6 +1,6 @@
 // The second factors of low-rank projections in one launch: A = U_a W_a^T in f32 (a decay's pre-activation) and beside it
 // G = U_g W_g^T in the storage type (an output gate), U_a [T, ra] and U_g [T, rg] columns of a stacked projection, ranks of 32 or 64.
-// Replaces a conversion to f32 and two products (bf16, 15 rows: three launches of 4.6 us; 3453 rows of 2048 + 2048: 38 us).  Bound by the
+// Replaces a conversion to f32 and two products (bf16, 15 rows: three launches of 4.6 us, now one of 5.3; 3453 rows of 2048 + 2048: 38, now 22 us).  Bound by the
 // results written.
 //
 // A wave keeps 64 rows of W in registers and walks token tiles of 16.  With bf16 rows each f32 weight is the sum of three bf16 pieces,
@@ -141,8 +141,8 @@ MX_API int mx_low_rank(const void* ua, const void* ug, long ldu, const float* wa
       (ng > 0 && ldu < rg) || ((size_t)ua | (size_t)wa | (size_t)ya) % 16 || (ng > 0 && ((size_t)ug | (size_t)wg | (size_t)yg) % 16) || T > (1 << 24))
     return (int)hipErrorInvalidValue;
   const int ba = (na + 255) / 256, bg = (ng + 255) / 256, tt = (T + 15) / 16;
-  // as many token tiles a block as still leave eight blocks for every CU
-  int tiles = (int)((long)tt * (ba + bg) / 2048);
+  // as many token tiles a block as still leave two blocks for every CU
+  int tiles = (int)((long)tt * (ba + bg) / 512);
   tiles = tiles < 1 ? 1 : (tiles > 8 ? 8 : tiles);
   const LowRank a{{ua, ug}, {wa, wg}, {ya, yg}, {na, ng}, ba, ldu, T, tiles};
   const dim3 grid(ba + bg, (tt + tiles - 1) / tiles);

@@ -379,7 +379,7 @@ window_attend_kernel(const T* __restrict__ q, long sq, const T* __restrict__ cac
 //                        terms hi + lo so that the f32 softmax weights are not cut to 8 bits
 // Feature dimensions are zero-padded to multiples of 32 (keys) / 16 (values) in LDS and registers.
 // Single-row segments (decode) may split each row's key range over nsplit blocks; the parts
-// (unnormalised output, running maximum, sum) are combined by window_merge_kernel.
+// (unnormalised output, running maximum, sum) are combined by attend_merge_kernel.
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 constexpr int MKT = 32;             // keys per tile
 constexpr int MLDV = MKT + 8;       // row stride of the transposed value tile
@@ -620,7 +620,7 @@ window_attend_mfma_kernel(const bf16* __restrict__ q, long sq, const bf16* __res
     }
   }
   if (!qok) return;
-  if (nsplit > 1) {                          // unnormalised part: o | m | l, merged by window_merge_kernel
+  if (nsplit > 1) {                          // unnormalised part: o | m | l, merged by attend_merge_kernel
     float* w = ws + ((row * H + h) * nsplit + split) * (long)(P + 2);
 #pragma unroll
     for (int nt = 0; nt < NTM; ++nt)
@@ -668,44 +668,6 @@ window_attend_mfma_kernel(const bf16* __restrict__ q, long sq, const bf16* __res
         if (r < P) dst[r] = (bf16)(o[nt][i] * gsc * (ge != nullptr ? mx_sigmoid((float)ge[r]) : 1.0f));
       }
     }
-  }
-}
-
-// grid (rows, H): combine the nsplit parts of one (row, head)
-// (sigm: the parts are plain sums of independently weighted values)
-template <typename T>
-__global__ void window_merge_kernel(const float* __restrict__ ws, const T* __restrict__ gate, long sgate,
-                                    int gate_elem, const float* __restrict__ sink, T* __restrict__ out, int H, int P,
-                                    int nsplit, int sigm) {
-  const long row = blockIdx.x;
-  const int h = blockIdx.y;
-  const float* w = ws + (row * H + h) * nsplit * (long)(P + 2);
-  const T* ge = gate_elem ? gate + row * sgate + (long)h * P : nullptr;
-  if (sigm) {
-    const float gs = gate != nullptr && !gate_elem ? mx_sigmoid(ldf(gate + row * sgate + h)) : 1.0f;
-    for (int r = threadIdx.x; r < P; r += blockDim.x) {
-      float a = 0.f;
-      for (int i = 0; i < nsplit; ++i) a += w[i * (P + 2) + r];
-      out[(row * H + h) * P + r] = (T)(a * gs * (ge != nullptr ? mx_sigmoid(ldf(ge + r)) : 1.0f));
-    }
-    return;
-  }
-  float M = sink != nullptr ? sink[h] : -INFINITY;
-  for (int i = 0; i < nsplit; ++i) M = fmaxf(M, w[i * (P + 2) + P]);
-  float L = sink != nullptr ? expf(sink[h] - M) : 0.f;      // the sink counts once, not once per part
-  for (int i = 0; i < nsplit; ++i) {
-    const float mi = w[i * (P + 2) + P];
-    if (mi != -INFINITY) L += w[i * (P + 2) + P + 1] * expf(mi - M);
-  }
-  float gsc = 1.0f / L;
-  if (gate != nullptr && !gate_elem) gsc *= mx_sigmoid(ldf(gate + row * sgate + h));
-  for (int r = threadIdx.x; r < P; r += blockDim.x) {
-    float a = 0.f;
-    for (int i = 0; i < nsplit; ++i) {
-      const float mi = w[i * (P + 2) + P];
-      if (mi != -INFINITY) a += w[i * (P + 2) + r] * expf(mi - M);
-    }
-    out[(row * H + h) * P + r] = (T)(a * gsc * (ge != nullptr ? mx_sigmoid(ldf(ge + r)) : 1.0f));
   }
 }
 
@@ -789,7 +751,7 @@ MX_API int mx_window_attend(const void* q, long sq, const void* cache, const int
                             const float* sink, float scale, void* out, int dt, int S, int max_len, int H, int G,
                             int D, int P, int nsplit, float* ws, int rows, hipStream_t st) {
   if (S <= 0 || max_len <= 0) return 0;
-  if (P > 64 * WA_CPL || G < 1 || H % G || window < 1 || keep < 0 ||
+  if (P > 64 * WA_CPL || nsplit > 64 || G < 1 || H % G || window < 1 || keep < 0 ||
       (gate_elem && gate == nullptr) || (sink != nullptr && head_bias != nullptr) || (rel != nullptr && rel_len < 1))
     return (int)hipErrorInvalidValue;
   // 2: gate rows that 8-byte accesses may read (bf16)
@@ -816,8 +778,7 @@ MX_API int mx_window_attend(const void* q, long sq, const void* cache, const int
       else rows_attend_kernel<bf16, 128, 0, 128, false, 1, 4, 32, false, true><<<grid, 256, 0, st>>>(a);
     }
     if (nsplit > 1)
-      MX_DISPATCH(dt, TT, window_merge_kernel<TT><<<dim3(rows, H), 128, 0, st>>>(
-          ws, (const TT*)gate, sgate, gate_elem, sink, (TT*)out, H, P, nsplit, 0));
+      MX_DISPATCH(dt, TT, attend_merge(ws, (const TT*)gate, sgate, gate_elem, sink, (TT*)out, rows, H, P, nsplit, 0, st));
     MX_RETURN_LAUNCH();
   }
   const bool forms = (cap <= 0.f || head_bias == nullptr) &&
@@ -853,11 +814,8 @@ MX_API int mx_window_attend(const void* q, long sq, const void* cache, const int
     else WINDOW_FORM(8, 16);
 #undef WINDOW_FORM
 #undef WINDOW_LAUNCH
-    if (nsplit > 1) {
-      dim3 g2(S, H);           // single-row segments: row index == segment index
-      window_merge_kernel<bf16><<<g2, P >= 128 ? 128 : 64, 0, st>>>(ws, (const bf16*)gate, sgate, ge, sink, (bf16*)out, H, P,
-                                                              nsplit, head_bias != nullptr ? 1 : 0);
-    }
+    // (single-row segments: row index == segment index)
+    if (nsplit > 1) attend_merge(ws, (const bf16*)gate, sgate, ge, sink, (bf16*)out, S, H, P, nsplit, head_bias != nullptr ? 1 : 0, st);
     MX_RETURN_LAUNCH();
   }
   const int esz = dt == 1 ? 4 : 2;
