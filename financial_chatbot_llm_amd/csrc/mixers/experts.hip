@@ -1,9 +1,9 @@
 // Routed feed-forwards: the chosen experts of every token as two grouped matrix products over rows sorted by expert,
 //     act[r] = unit(W1[e] x[token(r)])      W1 [N1, W] per expert (gated: gate and up rows in turns of 16)
 //     ys[r]  = W2[e] act[r]                 W2 [W, F] per expert
-// Three launches and no host read of the bucket sizes:
+// At most three launches and no host read of the bucket sizes:
 //   plan    a stable counting sort of the (token, choice) pairs by expert and the list of row tiles: one block, beyond 1024 pairs one
-//           per expert
+//           per expert; no launch of its own for up to 1024 pairs in the stream form below
 //   GEMM 1  gathers the tokens' rows while it stages them, applies the gated unit in its epilogue
 //   GEMM 2  sorted rows in and out; mx_moe_combine sums a token's rows
 // Weights are stored as the MFMA reads them: pieces of 1 KiB, [row group of 16][K step of 64 bytes][64 lanes][16 B],
@@ -55,6 +55,11 @@ struct ExpertGemm {
   int unit;
   float limit, alpha;
   const float* scale;   // per pair, on the expert's input (or null)
+  // stream form with a plan of its own (plan_tile): the pairs' experts, and where the plan goes for what comes after
+  const int* idx;
+  int pairs, experts;
+  int *pos, *src_out;
+  int4* tiles_out;
 };
 
 // One block: pairs 0 .. P-1 (expert idx[i], identity experts >= E stay out) in a stable order by expert.  Every wave
@@ -235,11 +240,11 @@ __device__ __forceinline__ float unit_value(int unit, float g, float u, float li
 
 // four adjacent output columns c .. c + 3 of sorted row r: gate and up sums, or one sum
 template <typename T, bool GLU>
-__device__ __forceinline__ void expert_store(const ExpertGemm& a, long r, int c, f32x4 g, f32x4 u) {
+__device__ __forceinline__ void expert_store(const ExpertGemm& a, long r, int c, f32x4 g, f32x4 u, int pair = -1) {
   if (c >= a.ncol) return;
   typedef T vec __attribute__((ext_vector_type(4)));
   if (GLU && a.scale != nullptr) {
-    const float s = a.scale[a.src[r]];
+    const float s = a.scale[pair >= 0 ? pair : a.src[r]];
 #pragma unroll
     for (int j = 0; j < 4; ++j) g[j] *= s, u[j] *= s;
   }
@@ -553,12 +558,85 @@ __global__ void __launch_bounds__(512) expert_wide_kernel(ExpertGemm a) {
 }
 
 // ---- stream form -------------------------------------------------------------------------------------------------
+// Up to 1024 pairs over up to 64 experts: every block finds its own tile (blockIdx.y) and the pairs in it, in the order of
+// expert_plan_kernel, whose launch is left out; the first of a tile's blocks leaves the plan for the second product and the
+// reader of its rows.  Bound by latency: one read of the indices and three passes through LDS, 1 - 3 us of the product for the 4 of the
+// launch (passes of 1 - 64 rows with four such layers 1 - 13 us shorter: f32 1 row 592 / 583, 60 rows of width 1024 665 / 652, of 2048 1027 / 1020).
+// own: the tile's pairs.  Returns (expert, first sorted row, rows, -).
+__device__ __forceinline__ int4 plan_tile(const ExpertGemm& a, int* own) {
+  __shared__ int count[64], found[4][4];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, y = blockIdx.y, E = a.experts;
+  const bool leave = blockIdx.x == 0;
+  int held[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int i = threadIdx.x + 256 * c;
+    held[c] = i < a.pairs ? a.idx[i] : E;
+  }
+  if (threadIdx.x < 64) count[threadIdx.x] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    if ((unsigned)held[c] < (unsigned)E) atomicAdd(count + held[c], 1);
+  __syncthreads();
+  const int n = lane < E ? count[lane] : 0;
+  int rows = n, upto = (n + 15) / 16;                        // this expert's and all before
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int r = __shfl_up(rows, o, 64), t = __shfl_up(upto, o, 64);
+    if (lane >= o) rows += r, upto += t;
+  }
+  const unsigned long long past = __ballot(upto > y);
+  int4 tile = make_int4(0, 0, 0, 0);
+  int first = 0;                                             // of the tile among its expert's rows
+  if (past != 0) {
+    const int e = __ffsll(past) - 1, ne = __builtin_amdgcn_readlane(n, e);
+    first = (y - (__builtin_amdgcn_readlane(upto, e) - (ne + 15) / 16)) * 16;
+    tile = make_int4(e, __builtin_amdgcn_readlane(rows, e) - ne + first, min(16, ne - first), 0);
+  }
+  if (leave && threadIdx.x == 0) a.tiles_out[y] = tile;
+  if (leave && y == 0)
+#pragma unroll
+    for (int c = 0; c < 4; ++c)                              // identity entries have no row
+      if (threadIdx.x + 256 * c < a.pairs && (unsigned)held[c] >= (unsigned)E) a.pos[threadIdx.x + 256 * c] = 0;
+  if (tile.z == 0) return tile;
+  int before[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const unsigned long long m = __ballot(held[c] == tile.x);
+    before[c] = __popcll(m & ((1ull << lane) - 1));
+    if (lane == 0) found[c][w] = __popcll(m);
+  }
+  __syncthreads();
+  int at = -first;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int r = at + before[c];
+      if (v == w && held[c] == tile.x && r >= 0 && r < 16) {
+        const int i = threadIdx.x + 256 * c;
+        own[r] = i;
+        if (leave) {
+          a.pos[i] = tile.y + r;
+          a.src_out[tile.y + r] = i;
+        }
+      }
+      at += found[c][v];
+    }
+  __syncthreads();
+  return tile;
+}
+
 // NF row groups x 16 tokens per block; wave w takes the w-th quarter of the pieces, the partial sums meet in LDS.
-template <typename T, int NF, bool GLU>
+template <typename T, int NF, bool GLU, bool PLAN>
 __global__ void __launch_bounds__(256) expert_stream_kernel(ExpertGemm a) {
   constexpr int ES = sizeof(T), UN = 8;
   __shared__ f32x4 red[4][NF][64];
-  const int4 tile = a.tiles[blockIdx.y];
+  __shared__ int own[16];
+  int4 tile;
+  if constexpr (PLAN) tile = plan_tile(a, own);
+  else tile = a.tiles[blockIdx.y];
   const int rows = tile.z;
   if (rows == 0) return;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, col = lane & 15;
@@ -567,7 +645,8 @@ __global__ void __launch_bounds__(256) expert_stream_kernel(ExpertGemm a) {
 #pragma unroll
   for (int f = 0; f < NF; ++f)
     wp[f] = reinterpret_cast<const uint4*>(a.w + tile.x * a.wstride + (long)min(G + f, a.groups - 1) * a.kt * 1024) + lane;
-  const char* xp = expert_row(a, tile.y + min(col, rows - 1), ES) + 16 * g;
+  const char* xp = (PLAN ? static_cast<const char*>(a.x) + own[min(col, rows - 1)] / a.top * a.ldx * ES
+                         : expert_row(a, tile.y + min(col, rows - 1), ES)) + 16 * g;
   const char* zero = reinterpret_cast<const char*>(&g_zero16);
   f32x4 acc[NF];
 #pragma unroll
@@ -609,7 +688,7 @@ __global__ void __launch_bounds__(256) expert_stream_kernel(ExpertGemm a) {
     if (col >= rows) continue;
     if (GLU) {
       if (G + 2 * f < a.groups)
-        expert_store<T, true>(a, tile.y + col, (G / 2 + f) * 16 + 4 * g, total(2 * f), total(2 * f + 1));
+        expert_store<T, true>(a, tile.y + col, (G / 2 + f) * 16 + 4 * g, total(2 * f), total(2 * f + 1), PLAN ? own[col] : -1);
     } else if (G + f < a.groups) {
       const f32x4 s = total(f);
       expert_store<T, false>(a, tile.y + col, (G + f) * 16 + 4 * g, s, s);
@@ -697,8 +776,11 @@ int expert_launch(const ExpertGemm& a, int mt, hipStream_t st) {
     if (a.ntiles > 65535) return (int)hipErrorInvalidValue;
     const bool wide = (long)a.ntiles * (a.groups / 4) >= 512;       // enough blocks of 64 W rows to fill the chip
     const dim3 grid((a.groups + (wide ? 3 : 1)) / (wide ? 4 : 2), a.ntiles);
-    if (wide) expert_stream_kernel<T, 4, GLU><<<grid, 256, 0, st>>>(a);
-    else expert_stream_kernel<T, 2, GLU><<<grid, 256, 0, st>>>(a);
+    if (a.idx != nullptr) {
+      if (wide) expert_stream_kernel<T, 4, GLU, true><<<grid, 256, 0, st>>>(a);
+      else expert_stream_kernel<T, 2, GLU, true><<<grid, 256, 0, st>>>(a);
+    } else if (wide) expert_stream_kernel<T, 4, GLU, false><<<grid, 256, 0, st>>>(a);
+    else expert_stream_kernel<T, 2, GLU, false><<<grid, 256, 0, st>>>(a);
   }
   return (int)hipGetLastError();
 }
@@ -746,7 +828,9 @@ MX_API int mx_experts(const void* h, long ldh, const int* idx, int T, int top, i
   const size_t lds = (size_t)(nw + 1) * E * 4;
 #define PLAN(NC) expert_plan_kernel<NC><<<1, nw * 64, lds, st>>>(idx, (int)P, E, bits, mt, ntiles, pos, src, tiles)
 #define WIDE(NC) expert_plan_wide_kernel<NC><<<E, 1024, (size_t)17 * E * 4, st>>>(idx, (int)P, E, mt, ntiles, pos, src, tiles)
-  if (wide && P <= 4 * 1024) WIDE(4);
+  const bool own = mt == 16 && P <= 1024 && E <= 64;         // the first product's blocks plan for themselves
+  if (own) {
+  } else if (wide && P <= 4 * 1024) WIDE(4);
   else if (wide && P <= 8 * 1024) WIDE(8);
   else if (wide && P <= 16 * 1024) WIDE(16);
   else if (wide && P <= 32 * 1024) WIDE(32);
@@ -761,9 +845,9 @@ MX_API int mx_experts(const void* h, long ldh, const int* idx, int T, int top, i
   int rc = (int)hipGetLastError();
   if (rc) return rc;
   ExpertGemm a{h, ldh, W * es, src, top, tiles, ntiles, (const char*)w1, (long)g1 * k1 * 1024, k1, g1, act, lda, (int)lda,
-               unit, limit, alpha, scale};
+               unit, limit, alpha, scale, own ? idx : nullptr, (int)P, E, pos, src, tiles};
   ExpertGemm b{act, lda, (int)lda * es, src, 0, tiles, ntiles, (const char*)w2, (long)g2 * k2 * 1024, k2, g2, ys, W, W,
-               UNIT_NONE, 0.f, 0.f, nullptr};
+               UNIT_NONE, 0.f, 0.f, nullptr, nullptr, 0, 0, nullptr, nullptr, nullptr};
   if (glu) MX_DISPATCH(dt, TT, rc = expert_launch<TT, true>(a, mt, st));
   else MX_DISPATCH(dt, TT, rc = expert_launch<TT, false>(a, mt, st));
   if (rc) return rc;

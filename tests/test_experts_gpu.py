@@ -160,3 +160,12 @@ def test_expert_plan_is_the_stable_sort(E, T):
 ])
 def test_experts_of_many_rows(T, W, F_, E, top, unit, kw):
     check(torch.bfloat16, T, W, F_, E, top, unit, **kw)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,E,top,ident,skew", [(1, 64, 1, 0, False), (256, 64, 4, 0, False), (341, 64, 3, 5, True), (342, 64, 3, 0, True), (256, 65, 4, 0, False),
+                                                (17, 2, 1, 0, False), (64, 33, 1, 31, True)])
+def test_blocks_that_plan_for_themselves(dtype, T, E, top, ident, skew):
+    """Around 1024 pairs and 64 experts, beyond which the plan is a launch: buckets of one tile, of several and empty ones, identity entries."""
+    check(dtype, T, 256, 64, E, top, "clamped", ident=ident, skew=skew)
+    check(dtype, T, 256, 64, E, top, "silu", ident=ident, skew=skew)
