@@ -7,6 +7,8 @@
 //          exchanges, the choice) and by the router's bytes, which every block reads from L2.
 //   tile   16 tokens per block on the f32 matrix cores, 8 waves split K, the partial sums meet in LDS.  Bound by the f32 products.
 // Either way products and sums are f32 and the choice runs on one lane per expert, by rank (ties: the lower index).
+// The clamped unit of a shared expert's gate and up columns, which needs nothing of the router, may run in blocks behind the router's: a launch
+// less for work that fits beside a kernel that waits for latency (gezavik, four such layers: 17 rows 552 -> 541 us, 64 1275 -> 1265, 130 mixed 1040 -> 1015).
 #include "mx_common.h"
 
 namespace {
@@ -37,7 +39,33 @@ struct Router {
   int E, top, W, T;
   float* outw;
   int* outi;
+  // blocks from `blocks` on: out = unit(gate, up), rows of nv 16-byte pieces
+  int blocks;
+  const void *gate, *up;
+  long sgate, sup;
+  float limit, alpha;
+  void* out;
+  int nv;
 };
+
+// glu_clamp_vec_kernel's values, a piece of 16 bytes per thread
+template <typename T> __device__ __forceinline__ void router_glu(const Router& a) {
+  constexpr int V = 16 / sizeof(T);
+  typedef T vec __attribute__((ext_vector_type(V)));
+  const long i = (long)(blockIdx.x - a.blocks) * blockDim.x + threadIdx.x, t = i / a.nv;
+  const int c = (int)(i - t * a.nv);
+  if (t >= a.T) return;
+  const vec gv = *reinterpret_cast<const vec*>(static_cast<const T*>(a.gate) + t * a.sgate + (long)c * V);
+  const vec uv = *reinterpret_cast<const vec*>(static_cast<const T*>(a.up) + t * a.sup + (long)c * V);
+  vec o;
+#pragma unroll
+  for (int e = 0; e < V; ++e) {
+    const float g = fminf((float)gv[e], a.limit);
+    const float u = fminf(fmaxf((float)uv[e], -a.limit), a.limit);
+    o[e] = (T)(g * mx_sigmoid(a.alpha * g) * (u + 1.0f));
+  }
+  *reinterpret_cast<vec*>(static_cast<T*>(a.out) + (t * a.nv + c) * V) = o;
+}
 
 // The choice of one token by one wave: z is lane e's logit (e < E).  An entry's rank is the number of those before it: larger,
 // or equal with a lower index; what is not a number comes last.
@@ -91,6 +119,7 @@ template <int O> __device__ __forceinline__ float halve(float x, float y) {
 template <typename T, int EP, int TB>
 __global__ void __launch_bounds__(1024) router_rows_kernel(Router a) {
   __shared__ float part[TB][4][4][16];                       // token, group, wave, expert of the group
+  if ((int)blockIdx.x >= a.blocks) return router_glu<T>(a);
   const long t0 = (long)blockIdx.x * TB;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, q = threadIdx.x >> 8;
   const T* h[TB];
@@ -143,6 +172,7 @@ template <typename T, int NF>
 __global__ void __launch_bounds__(512, 4) router_tile_kernel(Router a) {
   __shared__ f32x4 red[8][NF][64];
   __shared__ float zt[16][16 * NF + 1];
+  if ((int)blockIdx.x >= a.blocks) return router_glu<T>(a);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, c = lane & 15, t0 = blockIdx.x * 16;
   const T* h = static_cast<const T*>(a.h) + (long)min(t0 + c, a.T - 1) * a.ldh + 8 * g;
   const float* r[NF];
@@ -183,11 +213,14 @@ __global__ void __launch_bounds__(512, 4) router_tile_kernel(Router a) {
   }
 }
 
-template <typename T, int NF> void router_launch(const Router& a, hipStream_t st) {
-  if (a.T <= ROWS_1) router_rows_kernel<T, 4 * NF, 1><<<a.T, 1024, 0, st>>>(a);
+template <typename T, int NF> void router_launch(Router a, hipStream_t st) {
+  const int tokens = a.T <= ROWS_1 ? 1 : a.T <= ROWS_4 ? 4 : 16, threads = a.T <= ROWS_4 ? 1024 : 512;
+  a.blocks = (a.T + tokens - 1) / tokens;
+  const unsigned grid = a.blocks + (unsigned)(((long)a.T * a.nv + threads - 1) / threads);
+  if (a.T <= ROWS_1) router_rows_kernel<T, 4 * NF, 1><<<grid, 1024, 0, st>>>(a);
   else if (a.T <= ROWS_4) {
-    if constexpr (NF <= 3) router_rows_kernel<T, 4 * NF, 4><<<(a.T + 3) / 4, 1024, 0, st>>>(a);
-  } else if constexpr (sizeof(T) == 2) router_tile_kernel<T, NF><<<(a.T + 15) / 16, 512, 0, st>>>(a);
+    if constexpr (NF <= 3) router_rows_kernel<T, 4 * NF, 4><<<grid, 1024, 0, st>>>(a);
+  } else if constexpr (sizeof(T) == 2) router_tile_kernel<T, NF><<<grid, 512, 0, st>>>(a);
 }
 
 }  // namespace
@@ -196,16 +229,18 @@ template <typename T, int NF> void router_launch(const Router& a, hipStream_t st
 // entries, 1 sigmoid, 2 softmax over the chosen logits.  biased != 0: the largest score + bias (f32 [E] or null) are chosen,
 // weighted by the score itself; else the largest logits.  renorm != 0: weights divided by their sum (+ 1e-20); times wscale.
 // outw, outi [T, top].  E <= 64, W % 32 == 0, 16-byte rows.  The tile form is for bf16: f32 takes at most ROWS_4 rows.  More than 48
-// entries take no rows between ROWS_1 and ROWS_4.
+// entries take no rows between ROWS_1 and ROWS_4.  n > 0: act [T, n] = mx_glu_clamp of the columns gate and up besides, all of type dt in whole 16 bytes.
 MX_API int mx_router(const void* h, long ldh, int dt, const float* w, const float* zbias, const float* bias, int biased,
-                     int score, int renorm, float wscale, int E, int top, int W, float* outw, int* outi, int T,
-                     hipStream_t st) {
+                     int score, int renorm, float wscale, int E, int top, int W, float* outw, int* outi, const void* gate, long sgate,
+                     const void* up, long sup, float limit, float alpha, void* act, int n, int T, hipStream_t st) {
   if (T <= 0) return 0;
+  const int V = dt == 1 ? 4 : 8;
   if (E < 1 || E > 64 || top < 1 || top > E || W < 32 || W % 32 || ldh * (dt == 1 ? 4 : 2) % 16 ||
       ((size_t)h | (size_t)w) % 16 || score < 0 || score > 2 || (biased && score == ROUTE_SOFTMAX_TOP) || (dt == 1 && T > ROWS_4) ||
-      (E > 48 && T > ROWS_1 && T <= ROWS_4))
+      (E > 48 && T > ROWS_1 && T <= ROWS_4) || n < 0 || (n > 0 && (n % V || sgate % V || sup % V || ((size_t)gate | (size_t)up | (size_t)act) % 16)) ||
+      (long)T * (n / V) > 1L << 36)
     return (int)hipErrorInvalidValue;
-  const Router a{h, ldh, w, zbias, bias, biased, score, renorm, wscale, E, top, W, T, outw, outi};
+  const Router a{h, ldh, w, zbias, bias, biased, score, renorm, wscale, E, top, W, T, outw, outi, 0, gate, up, sgate, sup, limit, alpha, act, n / V};
   MX_DISPATCH(dt, TT, switch ((E + 15) / 16) {
     case 1: router_launch<TT, 1>(a, st); break;
     case 2: router_launch<TT, 2>(a, st); break;

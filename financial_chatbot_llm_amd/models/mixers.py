@@ -363,14 +363,13 @@ class RoutedFF:
 
     def forward(self, h: torch.Tensor, proj: Optional[torch.Tensor]) -> torch.Tensor:
         top = self.top
-        shared = None
-        if self.Fs:
-            shared = project(mx.glu_clamp(proj[:, :self.Fs], proj[:, self.Fs:2 * self.Fs], self.limit_s, self.alpha),
-                             self.down_s, self.parts)
+        glu = mx.Glu(proj[:, :self.Fs], proj[:, self.Fs:2 * self.Fs], self.limit_s, self.alpha) if self.Fs else None
         if self.score == "softmax_top":
             wts, idx = mx.router_scores(h, self.router, self.correction, top, "softmax_top")
+            act = mx.glu_clamp(*glu) if glu is not None else None
         else:
-            wts, idx = mx.router_biased(h, self.router, self.correction, top, self.score, self.renorm, self.w_scale)
+            wts, idx, act = mx.router_glu(h, self.router, self.correction, top, self.score, self.renorm, self.w_scale, glu)
+        shared = project(act, self.down_s, self.parts) if act is not None else None
         ys, pos = self.bank.run(h, idx, "clamped", self.limit, self.alpha)
         if self.parts and self.bank.native:
             return mx.Routed(ys, pos, idx, wts, h, shared, self.E, self.I > 0)

@@ -132,7 +132,8 @@ _MIXER_SIGS = {
     "mx_embed_pairs": [P, P, P, c_int, c_int, c_int, c_int, P, P, P, P, P, c_int, c_int, c_int, c_int, P],
     "mx_post_norm": [P, P, c_long, P, P, c_long, P, c_int, P, c_float, P, c_int, c_int, c_int, P],
     "mx_glu_act": [P, c_long, P, c_long, P, c_int, P, c_long, c_int, c_int, c_int, P],
-    "mx_router": [P, c_long, c_int, P, P, P, c_int, c_int, c_int, c_float, c_int, c_int, c_int, P, P, c_int, P],
+    "mx_router": [P, c_long, c_int, P, P, P, c_int, c_int, c_int, c_float, c_int, c_int, c_int, P, P, P, c_long, P, c_long, c_float, c_float, P,
+                  c_int, c_int, P],
     "mx_route_scores": [P, c_int, c_int, c_int, P, P, c_int, P],
     "mx_head_norm_gate": [P, c_long, c_int, P, c_float, P, c_long, c_int, c_int, P, c_int, c_int, c_int, c_int, P],
     "mx_matrix_scan": [P, c_long, P, c_long, P, c_long, c_int, P, c_long, P, P, P, c_long, c_int, c_float, c_int, P, P, P, P,

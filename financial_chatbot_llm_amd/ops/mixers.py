@@ -386,9 +386,17 @@ def router_takes(T: int, E: int, W: int, f32: bool) -> bool:
     return T > 1024 and (W <= 1024 or (W <= 2048 and T <= 4096))
 
 
-def _router(h: torch.Tensor, w: torch.Tensor, zbias, bias, biased: bool, top: int, score: str, renorm: bool, scale: float):
-    """``mx_router`` where it serves the call (up to 64 entries, whole groups of 32 columns, 16-byte rows) and is the faster way
-    (:func:`router_takes`), else None."""
+class Glu(NamedTuple):
+    """Operands of :func:`glu_clamp` that a router's launch may take along."""
+    gate: torch.Tensor
+    up: torch.Tensor
+    limit: float
+    alpha: float
+
+
+def _router(h: torch.Tensor, w: torch.Tensor, zbias, bias, biased: bool, top: int, score: str, renorm: bool, scale: float, glu: Optional[Glu] = None):
+    """(weights, indices, act) by ``mx_router`` where it serves the call (up to 64 entries, whole groups of 32 columns, 16-byte rows) and is the
+    faster way (:func:`router_takes`), else None.  act: :func:`glu_clamp` of ``glu`` where its rows are in whole 16 bytes, else None."""
     T, W = h.shape
     E = w.shape[0]
     es = h.element_size()
@@ -397,19 +405,23 @@ def _router(h: torch.Tensor, w: torch.Tensor, zbias, bias, biased: bool, top: in
         return None
     outw = torch.empty((T, top), dtype=torch.float32, device=h.device)
     outi = torch.empty((T, top), dtype=torch.int32, device=h.device)
+    act, more = None, (None, 0, None, 0, 0.0, 0.0, None, 0)
+    if glu is not None:
+        g, u = glu.gate, glu.up
+        n, (sg, one), (su, one_) = g.shape[1], g.stride(), u.stride()
+        if g.shape == u.shape and g.shape[0] == T and g.dtype == u.dtype == h.dtype and one == one_ == 1 and n > 0 and \
+                (n * es | sg * es | su * es | g.data_ptr() | u.data_ptr()) % 16 == 0 and T * n < 1 << 36:
+            act = torch.empty((T, n), dtype=h.dtype, device=h.device)
+            more = (g.data_ptr(), sg, u.data_ptr(), su, float(glu.limit), float(glu.alpha), act.data_ptr(), n)
     N.mcall("mx_router", N.ptr(h), h.stride(0), _dt(h), N.ptr(w), N.ptr(zbias), N.ptr(bias), 1 if biased else 0, ROUTE_SCORES[score],
-            1 if renorm else 0, float(scale), E, top, W, N.ptr(outw), N.ptr(outi), T, N.stream())
-    return outw, outi
+            1 if renorm else 0, float(scale), E, top, W, N.ptr(outw), N.ptr(outi), *more, T, N.stream())
+    return outw, outi, act
 
 
 def router_biased(h: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], top: int, score: str = "softmax",
                   renorm: bool = False, scale: float = 1.0) -> Tuple[torch.Tensor, torch.Tensor]:
     """:func:`route_biased` of the logits ``h w^T`` in f32 (``h`` [T, W] bf16 or f32, ``w`` f32 [E, W])."""
-    assert w.dtype == torch.float32 and w.shape[1] == h.shape[1] and 1 <= top <= w.shape[0]
-    if score not in ("softmax", "sigmoid"):
-        raise ValueError(f"unknown routing score {score!r}")
-    r = _router(h, w, None, bias, True, top, score, renorm, scale)
-    return r if r is not None else route_biased(F.linear(h.float(), w), bias, top, score, renorm, scale)
+    return router_glu(h, w, bias, top, score, renorm, scale)[:2]
 
 
 def router_scores(h: torch.Tensor, w: torch.Tensor, zbias: Optional[torch.Tensor], top: int,
@@ -419,7 +431,19 @@ def router_scores(h: torch.Tensor, w: torch.Tensor, zbias: Optional[torch.Tensor
     if score not in ROUTE_SCORES:
         raise ValueError(f"unknown routing score {score!r}")
     r = _router(h, w, zbias, None, False, top, score, False, 1.0)
-    return r if r is not None else route_scores(F.linear(h.float(), w, zbias), top, score)
+    return r[:2] if r is not None else route_scores(F.linear(h.float(), w, zbias), top, score)
+
+
+def router_glu(h: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], top: int, score: str = "softmax", renorm: bool = False,
+               scale: float = 1.0, glu: Optional[Glu] = None) -> Tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]:
+    """:func:`router_biased` and, given, :func:`glu_clamp` of ``glu``, in one launch where one serves both."""
+    assert w.dtype == torch.float32 and w.shape[1] == h.shape[1] and 1 <= top <= w.shape[0]
+    if score not in ("softmax", "sigmoid"):
+        raise ValueError(f"unknown routing score {score!r}")
+    r = _router(h, w, None, bias, True, top, score, renorm, scale, glu)
+    if r is None:
+        r = *route_biased(F.linear(h.float(), w), bias, top, score, renorm, scale), None
+    return r if glu is None or r[2] is not None else (r[0], r[1], glu_clamp(*glu))
 
 
 class ExpertRows(NamedTuple):

@@ -95,3 +95,22 @@ def test_rule(T, E, W, f32, native, monkeypatch):
     z = (h.double() @ r.double().t()).cpu()
     s = torch.softmax(z, -1)
     check(w, i, z, s, lambda i: s.gather(1, i), top, 2.0 ** -22 * W ** 0.5 + 2.0 ** -20)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,E", [(1, 34), (5, 8), (256, 34), (257, 34), (1024, 16), (1030, 34), (300, 60)])
+@pytest.mark.parametrize("n,pad", [(8, 0), (136, 8), (2048, 0), (72, 3), (20, 0)])
+def test_a_units_columns_beside_the_router(dt, T, E, n, pad):
+    """The clamped unit in the router's launch, and where it has to stay its own (other layouts, calls that the launch does not serve): the
+    same values either way."""
+    g = torch.Generator(device="cuda").manual_seed(T + n)
+    h, w, b = (torch.randn(s, generator=g, device="cuda") for s in ((T, 256), (E, 256), (E,)))
+    h, w = h.to(dt), w * 256 ** -0.5
+    rows = (2.0 * torch.randn((T, 2 * n + pad), generator=g, device="cuda")).to(dt)
+    rows[0, 0], rows[0, n] = float("inf"), float("nan")
+    gate, up = rows[:, :n], rows[:, n + pad:] if pad == 3 else rows[:, n:2 * n]
+    rw, ri = mx.router_biased(h, w, b, 4, "sigmoid", True, 1.5)
+    gw, gi, act = mx.router_glu(h, w, b, 4, "sigmoid", True, 1.5, mx.Glu(gate, up, 1.3, 1.702))
+    want = mx.glu_clamp(gate, up, 1.3, 1.702)
+    assert torch.equal(rw, gw) and torch.equal(ri, gi) and act.shape == want.shape and torch.equal(act.view(torch.int16 if dt == torch.bfloat16 else torch.int32),
+                                                                                             want.view(torch.int16 if dt == torch.bfloat16 else torch.int32))
