@@ -19,6 +19,7 @@
 //            the current chunk's dependent steps run; the chunk's outputs leave through LDS as
 //            whole runs.  Steps with few (segment, head) pairs take the variant with more lanes per
 //            column so that the grid still covers the chip.
+//   single rows with D <= 256 and P a multiple of four go through state_step_kernel instead, which reads the state by rows.
 //   gla and delta with D <= 256 take chunks of 16 tokens on the f32 matrix instructions instead (further down) in steps
 //   with a segment of 32 rows or more, but for those that run_matrix_scan keeps here.
 //
@@ -417,6 +418,103 @@ __global__ void mingru_step_kernel(const TI* __restrict__ zp, long sz, const TI*
   }
 }
 
+// Single rows (decode): the token of matrix_scan_kernel's ONE form with the state read and written as it lies.  A block takes 32 of a head's
+// value columns and all of its keys: eight lanes by four columns are 128 bytes of a row, 32 rows side by side, RPT of them a thread,
+// all asked for before anything else.  The sums over the keys meet by lane exchanges and once through LDS.  Bound by the state's bytes and,
+// for few rows, by latency.  16 heads, 15 rows, by columns (16-byte pieces of a row per lane group) / here, us: delta, 128 x 128 22.7 / 11.0, gla, 64 x
+// 128 14.8 / 7.3; 8 heads, one row in f32 6.5 / 5.4 and 5.3 / 4.8.
+template <typename TQ, int MODE, int RPT>
+__global__ void __launch_bounds__(256)
+state_step_kernel(const TQ* __restrict__ q, long sq, const TQ* __restrict__ k, long sk, const TQ* __restrict__ v, long sv,
+                  const float* __restrict__ a, long sa, float* __restrict__ state, const int* __restrict__ cu, const int* __restrict__ slot,
+                  const int* __restrict__ pos, float* __restrict__ out, int H, int G, int D, int P, const float* __restrict__ a_bias,
+                  const float* __restrict__ A_log, const void* __restrict__ beta, long sbeta, int beta_code, float tau_inv, int most) {
+  constexpr bool DELTA = MODE == 1, FIXED = MODE == 2;
+  constexpr int DP = 32 * RPT;
+  __shared__ float qs[DP], ks[DP], gs[DP], norm[2][4];
+  __shared__ mx_f32x4 red[2][4][8];
+  const int s = blockIdx.z, sl = slot[s];
+  if (sl < 0) return;
+  const long t = cu[s];
+  const int n = cu[s + 1] - (int)t;
+  if (n <= 0 || n > most) return;
+  const int h = blockIdx.y, kvh = h / (H / G), tid = threadIdx.x, lane = tid & 63, w = tid >> 6, cg = tid & 7, rg = tid >> 3;
+  const int c = blockIdx.x * 32 + 4 * cg, cc = min(c, P - 4);
+  const bool fresh = pos[t] == 0;
+  float* srec = state + (((long)sl * H + h) * D) * P + cc;
+  mx_f32x4 S[RPT];
+#pragma unroll
+  for (int i = 0; i < RPT; ++i) {
+    const int d = 32 * i + rg;
+    S[i] = !fresh && d < D ? ldf4(srec + (long)d * P) : mx_f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  mx_f32x4 u;
+  const int fact = beta_code & 15, vcode = beta_code >> 4;
+  const long vi = t * sv + h * P + cc;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) u[e] = FIXED ? ld_code(v, vcode, vi + e) : ldf(v + vi + e);
+  float b = 1.f;
+  if (DELTA) b = mx_sigmoid(ld_code(beta, beta_code, t * sbeta + h));
+  const float qscale = 1.0f / sqrtf((float)D), gfix = FIXED ? a_bias[h] : 1.f;
+  if (w < (DP + 63) / 64) {
+    float qv = 0.f, kv = 0.f, gv = 1.f;
+    if (tid < D) {
+      qv = ldf(q + t * sq + kvh * D + tid);
+      kv = ldf(k + t * sk + kvh * D + tid);
+      if (!FIXED) {
+        const float z = a[t * sa + h * D + tid] + a_bias[h * D + tid];
+        gv = DELTA ? expf(-expf(A_log[h]) * mx_softplus(z)) : expf(-mx_softplus(-z) * tau_inv);
+      }
+      if (FIXED && fact == 1) qv = mx_silu(qv), kv = mx_silu(kv);
+    }
+    if (tid < DP) qs[tid] = qv, ks[tid] = kv, gs[tid] = gv;
+    if (DELTA) {
+      const float qq = mx_wave_sum(qv * qv), kk = mx_wave_sum(kv * kv);
+      if (lane == 0) norm[0][w] = qq, norm[1][w] = kk;
+    }
+  }
+  if (FIXED && fact == 1)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) u[e] = mx_silu(u[e]);
+  __syncthreads();
+  float fq = 1.f, fk = 1.f;
+  if (DELTA) {                             // q and k become unit vectors, q also scaled
+    float qq = 0.f, kk = 0.f;
+#pragma unroll
+    for (int i = 0; i < (DP + 63) / 64; ++i) qq += norm[0][i], kk += norm[1][i];
+    fq = qscale / sqrtf(qq + 1e-6f);
+    fk = 1.0f / sqrtf(kk + 1e-6f);
+  }
+  auto total = [&](mx_f32x4 x, int at) {   // over all keys of this thread's columns
+#pragma unroll
+    for (int o = 8; o < 64; o <<= 1)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] += __shfl_xor(x[e], o, 64);
+    if (lane < 8) red[at][w][lane] = x;
+    __syncthreads();
+    return (red[at][0][cg] + red[at][1][cg]) + (red[at][2][cg] + red[at][3][cg]);
+  };
+#pragma unroll
+  for (int i = 0; i < RPT; ++i) S[i] *= FIXED ? gfix : gs[32 * i + rg];
+  if (DELTA) {
+    mx_f32x4 x = mx_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) x += S[i] * (ks[32 * i + rg] * fk);
+    x = total(x, 0);
+    u = b * (u - x);
+  }
+  mx_f32x4 o = mx_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < RPT; ++i) {
+    const int d = 32 * i + rg;
+    S[i] += u * (ks[d] * fk);
+    o += S[i] * (qs[d] * fq);
+    if (d < D && c < P) stf4(srec + (long)d * P, S[i]);
+  }
+  o = total(o, 1);
+  if (tid < 8 && c < P) stf4(out + t * H * P + h * P + c, DELTA ? o : o * (FIXED ? tau_inv : qscale));
+}
+
 template <typename TQ, int RPL, int LPC, int DELTA>
 int launch_matrix_scan(const void* q, long sq, const void* k, long sk, const void* v, long sv, const float* g, long sa,
                        const float* aux, float* state, const int* cu, const int* slot, const int* pos, float* out, int S,
@@ -435,9 +533,32 @@ int launch_matrix_scan(const void* q, long sq, const void* k, long sk, const voi
   MX_RETURN_LAUNCH();
 }
 
+// the steps of single rows that state_step_kernel takes
+template <typename TQ, int MODE>
+int launch_state_step(bool& done, const void* q, long sq, const void* k, long sk, const void* v, long sv, const float* g, long sa, const float*,
+                      float* state, const int* cu, const int* slot, const int* pos, float* out, int S, int H, int G, int D, int P,
+                      const float* a_bias, const float* A_log, const void* beta, long sbeta, int beta_dt, float tau_inv, bool one, int most,
+                      hipStream_t st) {
+  done = one && D <= 256 && P % 4 == 0 && ((size_t)state | (size_t)out) % 16 == 0;
+  if (!done) return 0;
+  const dim3 grid((P + 31) / 32, H, S);
+#define STATE_STEP(RPT)                                                                                                             \
+  state_step_kernel<TQ, MODE, RPT><<<grid, 256, 0, st>>>((const TQ*)q, sq, (const TQ*)k, sk, (const TQ*)v, sv, g, sa, state, cu, slot, pos, \
+                                                         out, H, G, D, P, a_bias, A_log, beta, sbeta, beta_dt, tau_inv, most)
+  if (D <= 32) STATE_STEP(1);
+  else if (D <= 64) STATE_STEP(2);
+  else if (D <= 128) STATE_STEP(4);
+  else STATE_STEP(8);
+#undef STATE_STEP
+  MX_RETURN_LAUNCH();
+}
+
 // the variant with 16 lanes per column when the narrow one would leave most of the chip idle
 template <typename TQ, int DELTA, typename... Args>
 int dispatch_matrix_scan(int D, bool wide, Args... args) {
+  bool done;
+  const int rc = launch_state_step<TQ, DELTA>(done, args...);
+  if (done) return rc;
   if (D <= 32) return launch_matrix_scan<TQ, 8, 4, DELTA>(args...);
   if (D <= 64) return wide ? launch_matrix_scan<TQ, 4, 16, DELTA>(args...) : launch_matrix_scan<TQ, 16, 4, DELTA>(args...);
   if (D <= 128) return wide ? launch_matrix_scan<TQ, 8, 16, DELTA>(args...) : launch_matrix_scan<TQ, 32, 4, DELTA>(args...);

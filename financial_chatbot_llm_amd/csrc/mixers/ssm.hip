@@ -158,6 +158,59 @@ __device__ __forceinline__ float row_sum16(float v) {
   return v;
 }
 
+// A step of single rows (decode): a block takes a head, its threads 16 of the value channels at a time with 16 lanes by fours along
+// the state's NJ 64s, up to 64 channels' states asked for at once; B and C, the same for all of them, stay in registers.  Bound by the
+// state's bytes: 64 rows of 64 heads of 64 x 128 47 us (5.7 TB/s), by the scan below, whose chunk of staged rows leaves room for three blocks a
+// CU, 62; 17 rows of 32 heads 9.6, 13.4.
+template <typename TD, int NJ>
+__global__ void __launch_bounds__(256)
+ssm_step_kernel(const float* __restrict__ u, int C, const TD* __restrict__ dt_raw, long sdt, const float* __restrict__ dt_bias,
+                const float* __restrict__ A_log, const float* __restrict__ Dp, float* __restrict__ state, const int* __restrict__ cu,
+                const int* __restrict__ slot, const int* __restrict__ pos, float* __restrict__ y, int H, int P, int G) {
+  constexpr int N = 64 * NJ, PU = NJ <= 2 ? 4 : 2;
+  const int s = blockIdx.y, sl = slot[s];
+  if (sl < 0) return;
+  const long t = cu[s];
+  if (cu[s + 1] - (int)t <= 0) return;
+  const int h = blockIdx.x, ns = threadIdx.x & 15, pl = threadIdx.x >> 4, inner = H * P;
+  const bool fresh = pos[t] == 0;
+  const float* ur = u + t * C;
+  float* sh = state + ((long)sl * H + h) * P * N + 4 * ns;
+  const float* Br = ur + inner + (long)(h / (H / G)) * N + 4 * ns;
+  mx_f32x4 B[NJ], Cv[NJ], S[PU][NJ];
+  float x[PU];
+  auto load = [&](int p0) {
+#pragma unroll
+    for (int i = 0; i < PU; ++i) {
+      const int p = min(p0 + 16 * i + pl, P - 1);
+      x[i] = ur[h * P + p];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) S[i][j] = fresh ? mx_f32x4{0.f, 0.f, 0.f, 0.f} : ldf4(sh + (long)p * N + 64 * j);
+    }
+  };
+  load(0);
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) B[j] = ldf4(Br + 64 * j), Cv[j] = ldf4(Br + (long)G * N + 64 * j);
+  const float dt = mx_softplus(ldf(dt_raw + t * sdt + h) + dt_bias[h]), a = expf(-expf(A_log[h]) * dt), Dh = Dp[h];
+  for (int p0 = 0; p0 < P; p0 += 16 * PU) {
+    if (p0 > 0) load(p0);
+#pragma unroll
+    for (int i = 0; i < PU; ++i) {
+      const int p = p0 + 16 * i + pl;
+      const float dx = dt * x[i];
+      mx_f32x4 acc = mx_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        S[i][j] = a * S[i][j] + dx * B[j];
+        acc += S[i][j] * Cv[j];
+        if (p < P) stf4(sh + (long)p * N + 64 * j, S[i][j]);
+      }
+      const float o = row_sum16((acc[0] + acc[1]) + (acc[2] + acc[3]));
+      if (ns == 0 && p < P) y[t * inner + h * P + p] = o + Dh * x[i];
+    }
+  }
+}
+
 // VEC: B | C rows are fetched and staged as 16-byte pieces (N, H*P and the row stride multiples of 4)
 template <typename TD, int NI, bool VEC>
 __global__ void __launch_bounds__(SCAN_NT) __attribute__((amdgpu_waves_per_eu(NI <= 8 ? 3 : 2)))   // blocks per CU that hide the step latency
@@ -729,6 +782,16 @@ MX_API int mx_ssm_scan(const float* u, int C, const void* dt_raw, long sdt, int 
 #undef SSD
     const int rc = (int)hipGetLastError();
     if (rc || S == 1) return rc;
+  }
+  if (max_len == 1 && (N == 64 || N == 128 || N == 256) && vecu && ((size_t)u | (size_t)state) % 16 == 0 && S <= 65535) {
+#define SSM_STEP(NJ)                                                                                                               \
+  MX_DISPATCH(dt_code, TT, ssm_step_kernel<TT, NJ><<<dim3(H, S), 256, 0, st>>>(u, C, (const TT*)dt_raw, sdt, dt_bias, A_log, D, state, cu, \
+                                                                               slot, pos, y, H, P, G))
+    if (N == 64) SSM_STEP(1);
+    else if (N == 128) SSM_STEP(2);
+    else SSM_STEP(4);
+#undef SSM_STEP
+    MX_RETURN_LAUNCH();
   }
   const int below = chunked ? SSD_LEAST : 0x7fffffff;
   dim3 grid((P + SCAN_PT - 1) / SCAN_PT, H, S);

@@ -1,0 +1,69 @@
+"""Steps of single rows of the matrix-state and state-space recurrences against the CPU forms: key sizes around a thread's share, value
+columns around a block's, padding rows, fresh and carried states, and the shapes that keep the longer form."""
+import pytest
+import torch
+
+from financial_chatbot_llm_amd.ops import mixers as mx
+
+pytestmark = pytest.mark.gpu
+
+S = 5
+SLOT = torch.tensor([3, 0, -1, 5, 1], dtype=torch.int32)
+POS = torch.tensor([7, 0, 3, 0, 1000], dtype=torch.int32)
+CU = torch.arange(S + 1, dtype=torch.int32)
+LIVE = (SLOT >= 0).nonzero().flatten()
+
+
+def near(got, want, n):
+    # sums of n products in f32, in another order: a few 2^-24 of each of them
+    err = (got.double().cpu() - want.double()).abs()
+    assert bool((err <= 2.0 ** -21 * n ** 0.5 * (1.0 + want.double().abs())).all()), float(err.max())
+
+
+def cuda(*ts):
+    return [t.cuda() if isinstance(t, torch.Tensor) else t for t in ts]
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("mode", ["gla", "delta", "decay", "decay silu"])
+@pytest.mark.parametrize("D,P", [(1, 4), (31, 36), (32, 32), (33, 128), (64, 100), (100, 8), (128, 128), (129, 64), (256, 60), (257, 32), (64, 30)])
+def test_matrix_states(dt, mode, D, P):
+    g = torch.Generator().manual_seed(D * 1000 + P)
+    rnd = lambda *s: torch.randn(s, generator=g)  # noqa: E731
+    H, G = 4, 4 if mode != "delta" else 2
+    q, k, v = rnd(S, G * D + 8).to(dt)[:, 8:], (rnd(S, G * D) * D ** -0.5).to(dt), rnd(S, H * P).to(dt)
+    state = rnd(6, H, D, P)
+    cs, ds = state.clone(), state.cuda()
+    meta = (CU, SLOT, POS)
+    if mode in ("gla", "delta"):
+        a, bias, A = rnd(S, H * D), rnd(H * D), rnd(H) * 0.3
+        kw = dict(A_log=A, beta=rnd(S, H).to(dt)) if mode == "delta" else dict(tau=3.0)
+        want = mx.matrix_scan(q, k, v, a.clone(), bias, cs, *meta, H, G, D, P, mode, max_len=1, **kw)
+        got = mx.matrix_scan(*cuda(q, k, v, a, bias), ds, *cuda(*meta), H, G, D, P, mode, max_len=1,
+                             **{n: t.cuda() if isinstance(t, torch.Tensor) else t for n, t in kw.items()})
+    else:
+        decay = torch.rand(H, generator=g)
+        act = "silu" if mode.endswith("silu") else "none"
+        want = mx.decay_scan(q, k, v, decay, cs, *meta, H, D, P, act=act, max_len=1)
+        got = mx.decay_scan(*cuda(q, k, v, decay), ds, *cuda(*meta), H, D, P, act=act, max_len=1)
+    near(got.cpu()[LIVE], want[LIVE], 4 * D)
+    near(ds, cs, 4)
+    for s in (2, 4):                                     # slots of no row
+        assert torch.equal(ds[s].cpu(), state[s])
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,P,G", [(64, 5, 1), (64, 64, 2), (128, 50, 2), (128, 64, 1), (128, 100, 4), (256, 16, 2), (256, 70, 1), (96, 64, 2), (24, 20, 2)])
+def test_state_space(dt, N, P, G):
+    g = torch.Generator().manual_seed(N * 1000 + P)
+    rnd = lambda *s: torch.randn(s, generator=g)  # noqa: E731
+    H = 4
+    u, dtr = rnd(S, H * P + 2 * G * N), rnd(S, H + 4).to(dt)[:, :H]
+    bias, A, Dp, state = rnd(H), rnd(H), rnd(H), rnd(6, H, P, N)
+    cs, ds = state.clone(), state.cuda()
+    want = mx.ssm_scan(u, dtr, bias, A, Dp, cs, CU, SLOT, POS, H, P, N, G, 1)
+    got = mx.ssm_scan(*cuda(u, dtr, bias, A, Dp), ds, *cuda(CU, SLOT, POS), H, P, N, G, 1)
+    near(got.cpu()[LIVE], want[LIVE], 16 * N)
+    near(ds, cs, 4)
+    for s in (2, 4):
+        assert torch.equal(ds[s].cpu(), state[s])
