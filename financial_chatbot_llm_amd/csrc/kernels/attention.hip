@@ -920,13 +920,40 @@ __global__ void __launch_bounds__(HPW * D) decode_lean_reduce_kernel(const int* 
     np = lw - fw + 1;
   }
   const long base = ((long)b * Hq + hq) * part_stride;
-  float M = -INFINITY;
-  for (int i = 0; i < np; ++i) M = fmaxf(M, part_m[base + i]);
-  float L = 0.f, O = 0.f;
-  for (int i = 0; i < np; ++i) {
-    const float f = exp2f(part_m[base + i] - M);
-    L += part_l[base + i] * f;
-    O += part_o[(base + i) * D + d] * f;
+  float M = -INFINITY, L = 0.f, O = 0.f;
+  const auto few = [&](auto most) {   // all parts asked for at once: one trip instead of two and one a part
+    constexpr int N = decltype(most)::value;
+    float m[N], l[N], o[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (i < np) {
+        m[i] = part_m[base + i];
+        l[i] = part_l[base + i];
+        o[i] = part_o[(base + i) * D + d];
+      }
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (i < np) M = fmaxf(M, m[i]);
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (i < np) {
+        const float f = exp2f(m[i] - M);
+        L += l[i] * f;
+        O += o[i] * f;
+      }
+  };
+  if (np <= 4) {
+    few(std::integral_constant<int, 4>{});
+  } else if (np <= 16) {
+    few(std::integral_constant<int, 16>{});
+  } else {
+    for (int i = 0; i < np; ++i) M = fmaxf(M, part_m[base + i]);
+#pragma unroll 4
+    for (int i = 0; i < np; ++i) {
+      const float f = exp2f(part_m[base + i] - M);
+      L += part_l[base + i] * f;
+      O += part_o[(base + i) * D + d] * f;
+    }
   }
   out[((long)b * Hq + hq) * D + d] = (bf16)(L > 0.f ? O / L : 0.f);
 }

@@ -23,17 +23,23 @@ __global__ void __launch_bounds__(1024) rmsnorm_kernel(const bf16* __restrict__ 
   const int nchunk = H >> 3;
   const uint4* xr = reinterpret_cast<const uint4*>(x + (size_t)row * H);
   uint4* rr = reinterpret_cast<uint4*>(res + (size_t)row * H);
+  const uint4* wr = reinterpret_cast<const uint4*>(w);
   float v[CPT][8];
+  constexpr bool EARLY = CPT <= 4;   // the weight with the row: behind the sum it is a second trip (8: no registers)
+  uint4 wv[CPT];
   float ss = 0.f;
 #pragma unroll
   for (int c = 0; c < CPT; ++c) {
     const int idx = threadIdx.x + c * blockDim.x;
     if (idx < nchunk) {
+      uint4 rv;
+      if (ADD_RES) rv = rr[idx];
+      if (EARLY) wv[c] = wr[idx];
       if (SLAB) load8_slabs(P + (size_t)row * H + 8 * idx, S, (long)T * H, v[c]);
       else unpack8(xr[idx], v[c]);
       if (ADD_RES) {
         float r[8];
-        unpack8(rr[idx], r);
+        unpack8(rv, r);
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[c][i] = (float)(bf16)(v[c][i] + r[i]);  // residual kept in bf16
         rr[idx] = pack8(v[c]);
@@ -43,14 +49,13 @@ __global__ void __launch_bounds__(1024) rmsnorm_kernel(const bf16* __restrict__ 
     }
   }
   const float inv = rsqrtf(block_sum(ss, scratch) / (float)H + eps);
-  const uint4* wr = reinterpret_cast<const uint4*>(w);
   uint4* yr = reinterpret_cast<uint4*>(y + (size_t)row * H);
 #pragma unroll
   for (int c = 0; c < CPT; ++c) {
     const int idx = threadIdx.x + c * blockDim.x;
     if (idx < nchunk) {
       float g[8], o[8];
-      unpack8(wr[idx], g);
+      unpack8(EARLY ? wv[c] : wr[idx], g);
 #pragma unroll
       for (int i = 0; i < 8; ++i) o[i] = (float)(bf16)(v[c][i] * inv) * g[i];
       yr[idx] = pack8(o);

@@ -13,6 +13,7 @@
 // Rotation is the HF/"neox" rotate-half form used by Llama-3 checkpoints.
 #include "common.h"
 #include "kv_layout.h"
+#include <algorithm>
 
 // SLAB: the QKV activation arrives as the S f32 split-K slabs [S, T, width] of the QKV GEMM
 // (gemm_splitk.hip) and is reduced here, in the same pass that rotates and scatters it.
@@ -47,15 +48,16 @@ __global__ void rope_kv_kernel(const bf16* __restrict__ qkv, const int* __restri
   for (int u = threadIdx.x + blockIdx.y * blockDim.x; u < total; u += blockDim.x * gridDim.y) {
     if (u < n_rot) {
       const int h = u / RU, c = u % RU;
-      float x1[8], x2[8];
-      load8(h * D + c * 8, x1);
-      load8(h * D + HALF + c * 8, x2);
-      if (apply_rope) {
-        float co[8], si[8];   // 4 x 16-B loads instead of 16 scalar loads
+      float x1[8], x2[8], co[8], si[8];
+      if (apply_rope) {   // 4 x 16-B loads instead of 16 scalar loads
         *reinterpret_cast<float4*>(co) = *reinterpret_cast<const float4*>(cs + c * 8);
         *reinterpret_cast<float4*>(co + 4) = *reinterpret_cast<const float4*>(cs + c * 8 + 4);
         *reinterpret_cast<float4*>(si) = *reinterpret_cast<const float4*>(cs + HALF + c * 8);
         *reinterpret_cast<float4*>(si + 4) = *reinterpret_cast<const float4*>(cs + HALF + c * 8 + 4);
+      }
+      load8(h * D + c * 8, x1);
+      load8(h * D + HALF + c * 8, x2);
+      if (apply_rope) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const float a = x1[i], b = x2[i];
@@ -95,8 +97,11 @@ static int launch_rope_kv(const void* qkv, const float* P, int S, const int* pos
                           const int* slots, void* q_out, void* k_cache, void* v_cache, int T, int Hq, int Hkv, int D,
                           int apply_rope, hipStream_t stream) {
   if (T <= 0) return 0;
-  const int threads = 256;
-  const dim3 grid(T, T <= 512 ? 2 : 1);
+  const int total = (Hq + Hkv) * (D / 16) + Hkv * (D / 8);
+  // a few tokens: smaller workgroups, so that a token's units lie on more CUs (a 32-layer step of 64 rows 7369 us in two
+  // workgroups a token, 7340 in seven; 16 rows 4544 and 4493)
+  const int threads = T <= 64 ? 64 : T <= 128 ? 128 : 256;
+  const dim3 grid(T, T <= 128 ? std::min(8, (total + threads - 1) / threads) : T <= 512 ? 2 : 1);
   if (D == 128) {
     hipLaunchKernelGGL((rope_kv_kernel<128, SLAB>), grid, dim3(threads), 0, stream, (const bf16*)qkv, positions,
                        cos_sin, slots, (bf16*)q_out, (bf16*)k_cache, (bf16*)v_cache, Hq, Hkv, apply_rope, P, S, T);
