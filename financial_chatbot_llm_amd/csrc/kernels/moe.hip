@@ -397,110 +397,147 @@ __global__ void __launch_bounds__(256) silu_quant_rows_kernel(const bf16* __rest
 #define MOE_EPI_SILU 1
 #define MOE_EPI_ROUTEW 2
 
-template <int NTF, int NW, int EPI>
-__global__ void __launch_bounds__(NW * 64) moe_gemm_kernel(
-    const unsigned char* __restrict__ Xq, const float* __restrict__ xs, const int* __restrict__ rows,
-    const int* __restrict__ offsets, const unsigned char* __restrict__ Wt, const float* __restrict__ ws,
-    const float* __restrict__ route_w, bf16* __restrict__ Y, int N, int K) {
-  constexpr int NR = 16 * NTF;
-  extern __shared__ __attribute__((aligned(16))) float red[];  // [NW][NR][64]
-  const int e = blockIdx.y;
-  const int p0 = offsets[e], p1 = offsets[e + 1];
-  if (p1 <= p0) return;
+// One chunk of up to 16 * MT pairs (c0 ..) of expert e against the workgroup's 16 * NTF weight rows.  The weights are streamed once and
+// bound the kernel, so what counts is how they stream: D k-pairs of weights and activations are asked for ahead of the MFMAs, past the
+// caches' replacement (ONCE), and only the MT token tiles that hold pairs are read and multiplied.  8 experts of 2 x 14336 x 4096, 48
+// tokens: first product 182 -> 145 us (6.4 TB/s; 138, 6.8, for 16 tokens), second 87 -> 72; one k-pair ahead, four token tiles whatever
+// the rows and 64 KB of LDS a workgroup before.  Without ONCE 152 and 80; four pairs or six ahead the same; four workgroups a CU
+// instead of three 197 and 100.
+template <int NTF, int NW, int EPI, int MT, int D, bool ONCE = true>
+__device__ __forceinline__ void moe_chunk(const unsigned char* __restrict__ Xq, const float* __restrict__ xs, const int* __restrict__ rows,
+                                          const unsigned char* __restrict__ We, const float* __restrict__ wse,
+                                          const float* __restrict__ route_w, bf16* __restrict__ Y, int N, int K, int n0, int c0, int nrow,
+                                          float* red) {
+  constexpr int NR = 16 * NTF, RS = 20;                       // RS: a row's 16 sums; 4 rows on, the banks behind them
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, col = lane & 15;
-  const int n0 = blockIdx.x * NR;
-  const int kper = K / NW, kb = w * kper;
+  const int kper = K / NW, kb = w * kper, kp = kper / 64;
   const long kpairs = K / 64;
-  const unsigned char* We = Wt + (long)e * N * K;
-  for (int c0 = p0; c0 < p1; c0 += 64) {  // token chunks of 64 pairs
-    const int nrow = min(64, p1 - c0);
-    f32x4 acc[NTF][4];
+  // lane (g, col) owns physical k = 64p + 16g .. +15 of its token row: one 16-B load per row tile
+  // and k-pair, matching the weight tiling (ops/moe.py tile_fp8_weight); bytes 0-7 feed the
+  // first MFMA of the pair, bytes 8-15 the second
+  const unsigned char* xr[MT];
 #pragma unroll
-    for (int f = 0; f < NTF; ++f)
+  for (int m = 0; m < MT; ++m) {
+    const int pr = c0 + min(16 * m + col, nrow - 1);
+    xr[m] = Xq + (long)(rows ? rows[pr] : pr) * K + kb + 16 * g;
+  }
+  const unsigned char* wr = We + ((n0 / 16 * kpairs + kb / 64) * 64 + lane) * 16;
+  f32x4 acc[NTF][MT];
 #pragma unroll
-      for (int m = 0; m < 4; ++m) acc[f][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // lane (g, col) owns physical k = 64p + 16g .. +15 of its token row: one 16-B load per row tile
-    // and k-pair, matching the weight tiling (ops/moe.py tile_fp8_weight); bytes 0-7 feed the
-    // first MFMA of the pair, bytes 8-15 the second
-    const unsigned char* xr[4];
+  for (int f = 0; f < NTF; ++f)
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const int pr = c0 + min(16 * m + col, nrow - 1);
-      const int src = rows ? rows[pr] : pr;
-      xr[m] = Xq + (long)src * K + kb + 16 * g;
+    for (int m = 0; m < MT; ++m) acc[f][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+  u32x4_t wv[D][NTF], xv[D][MT];
+  auto fetch = [&](int slot, int p) {
+#pragma unroll
+    for (int f = 0; f < NTF; ++f) {
+      const u32x4_t* src = reinterpret_cast<const u32x4_t*>(wr + (f * kpairs + p) * 1024);
+      wv[slot][f] = ONCE ? __builtin_nontemporal_load(src) : *src;
     }
-    // one k-pair of W (NTF fragments) and X (4 token tiles) in flight ahead of the MFMAs using
-    // the previous one (register double buffer)
-    uint4 wn[NTF], xn[4];
-    auto fetch = [&](int k) {
 #pragma unroll
-      for (int f = 0; f < NTF; ++f)
-        wn[f] = *reinterpret_cast<const uint4*>(We + (((long)(n0 / 16 + f) * kpairs + (kb + k) / 64) * 64 + lane) * 16);
+    for (int m = 0; m < MT; ++m) xv[slot][m] = *reinterpret_cast<const u32x4_t*>(xr[m] + 64 * p);
+  };
+  auto use = [&](int slot) {
+    // both k-halves of one accumulator back to back (a dependent MFMA pair): interleaving the
+    // halves across all accumulators made hipcc shuffle them between AGPRs every pair
 #pragma unroll
-      for (int m = 0; m < 4; ++m) xn[m] = *reinterpret_cast<const uint4*>(xr[m] + k);
-    };
-    fetch(0);
-    for (int k = 0; k < kper; k += 64) {
-      uint4 wv[NTF], xv[4];
+    for (int f = 0; f < NTF; ++f) {
+      const long a0 = ((long)wv[slot][f].y << 32 | wv[slot][f].x), a1 = ((long)wv[slot][f].w << 32 | wv[slot][f].z);
 #pragma unroll
-      for (int f = 0; f < NTF; ++f) wv[f] = wn[f];
-#pragma unroll
-      for (int m = 0; m < 4; ++m) xv[m] = xn[m];
-      if (k + 64 < kper) fetch(k + 64);
-#pragma unroll
-      // both k-halves of one accumulator back to back (a dependent MFMA pair): interleaving the
-      // halves across all NTF*4 accumulators made hipcc shuffle them between AGPRs every pair
-      for (int f = 0; f < NTF; ++f) {
-        const long a0 = ((long)wv[f].y << 32 | wv[f].x), a1 = ((long)wv[f].w << 32 | wv[f].z);
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-          const long b0 = ((long)xv[m].y << 32 | xv[m].x), b1 = ((long)xv[m].w << 32 | xv[m].z);
-          acc[f][m] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a0, b0, acc[f][m], 0, 0, 0);
-          acc[f][m] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a1, b1, acc[f][m], 0, 0, 0);
-        }
+      for (int m = 0; m < MT; ++m) {
+        const long b0 = ((long)xv[slot][m].y << 32 | xv[slot][m].x), b1 = ((long)xv[slot][m].w << 32 | xv[slot][m].z);
+        acc[f][m] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a0, b0, acc[f][m], 0, 0, 0);
+        acc[f][m] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a1, b1, acc[f][m], 0, 0, 0);
       }
     }
-    float* mine = red + w * NR * 64;
+  };
 #pragma unroll
-    for (int f = 0; f < NTF; ++f)
+  for (int d = 0; d < D; ++d)
+    if (d < kp) fetch(d, d);
+  int p = 0;
+  for (; p + 2 * D <= kp; p += D) {
 #pragma unroll
-      for (int m = 0; m < 4; ++m)
+    for (int d = 0; d < D; ++d) {
+      use(d);
+      fetch(d, p + D + d);
+      if (MT == 1) __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  for (; p < kp; p += D) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) mine[(16 * f + 4 * g + r) * 64 + 16 * m + col] = acc[f][m][r];
+    for (int d = 0; d < D; ++d) {
+      if (p + d < kp) use(d);
+      if (p + D + d < kp) fetch(d, p + D + d);
+    }
+  }
+  // the waves' sums of K, one token tile at a time; a thread has two neighbouring outputs of a pair
+  constexpr int OUTN = (EPI == MOE_EPI_SILU) ? NR / 2 : NR;
+  const int ldy = (EPI == MOE_EPI_SILU) ? N / 2 : N;
+  for (int m = 0; m < MT; ++m) {
+    if (16 * m >= nrow) break;
+    __syncthreads();                                          // the tile before has been read
+    float* mine = red + w * NR * RS;
+#pragma unroll
+    for (int mm = 0; mm < MT; ++mm)
+      if (mm == m)
+#pragma unroll
+        for (int f = 0; f < NTF; ++f)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) mine[(16 * f + 4 * g + r) * RS + col] = acc[f][mm][r];
     __syncthreads();
-    constexpr int OUTN = (EPI == MOE_EPI_SILU) ? NR / 2 : NR;
-    const int ldy = (EPI == MOE_EPI_SILU) ? N / 2 : N;
-    for (int idx = threadIdx.x; idx < 64 * (OUTN / 8); idx += NW * 64) {
-      const int m = idx / (OUTN / 8), c8 = (idx % (OUTN / 8)) * 8;
-      if (m >= nrow) continue;
-      const int pr = c0 + m;
+    for (int idx = threadIdx.x; idx < 16 * (OUTN / 2); idx += NW * 64) {
+      const int mr = idx / (OUTN / 2), c = idx % (OUTN / 2) * 2;
+      if (16 * m + mr >= nrow) continue;
+      const int pr = c0 + 16 * m + mr;
       const float sx = xs[rows ? rows[pr] : pr];
-      float o[8];
+      bf16 o[2];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
+      for (int j = 0; j < 2; ++j) {
         if (EPI == MOE_EPI_SILU) {
-          const int c = c8 + j, pair = c >> 4, jj = c & 15;
-          const int rg = 32 * pair + jj, ru = rg + 16;
+          const int rg = 32 * (c >> 4) + (c & 15) + j, ru = rg + 16;
           float gs = 0.f, us = 0.f;
 #pragma unroll
           for (int ww = 0; ww < NW; ++ww) {
-            gs += red[(ww * NR + rg) * 64 + m];
-            us += red[(ww * NR + ru) * 64 + m];
+            gs += red[(ww * NR + rg) * RS + mr];
+            us += red[(ww * NR + ru) * RS + mr];
           }
-          const float gv = (float)(bf16)(gs * sx * ws[(long)e * N + n0 + rg]);
-          const float uv = (float)(bf16)(us * sx * ws[(long)e * N + n0 + ru]);
-          o[j] = (float)(bf16)(gv / (1.f + __expf(-gv))) * uv;
+          const float gv = (float)(bf16)(gs * sx * wse[n0 + rg]);
+          const float uv = (float)(bf16)(us * sx * wse[n0 + ru]);
+          o[j] = (bf16)((float)(bf16)(gv / (1.f + __expf(-gv))) * uv);
         } else {
           float s = 0.f;
 #pragma unroll
-          for (int ww = 0; ww < NW; ++ww) s += red[(ww * NR + c8 + j) * 64 + m];
-          o[j] = s * sx * ws[(long)e * N + n0 + c8 + j] * route_w[pr];
+          for (int ww = 0; ww < NW; ++ww) s += red[(ww * NR + c + j) * RS + mr];
+          o[j] = (bf16)(s * sx * wse[n0 + c + j] * route_w[pr]);
         }
       }
-      const int ncol = (EPI == MOE_EPI_SILU) ? (n0 / 2 + c8) : (n0 + c8);
-      *reinterpret_cast<uint4*>(Y + (long)pr * ldy + ncol) = pack8(o);
+      const int ncol = (EPI == MOE_EPI_SILU) ? n0 / 2 + c : n0 + c;
+      *reinterpret_cast<uint32_t*>(Y + (long)pr * ldy + ncol) = *reinterpret_cast<const uint32_t*>(o);
     }
-    __syncthreads();
+  }
+}
+
+// (two waves a SIMD asked for: left to itself the compiler packs the wide workgroup's registers for three, 128 tokens 198 us instead of 175)
+template <int NTF, int NW, int EPI>
+__global__ void __launch_bounds__(NW * 64, NTF == 4 ? 2 : 1) moe_gemm_kernel(
+    const unsigned char* __restrict__ Xq, const float* __restrict__ xs, const int* __restrict__ rows,
+    const int* __restrict__ offsets, const unsigned char* __restrict__ Wt, const float* __restrict__ ws,
+    const float* __restrict__ route_w, bf16* __restrict__ Y, int N, int K) {
+  __shared__ float red[NW * 16 * NTF * 20];
+  const int e = blockIdx.y;
+  const int p0 = offsets[e], p1 = offsets[e + 1];
+  if (p1 <= p0) return;
+  const int n0 = blockIdx.x * 16 * NTF;
+  const unsigned char* We = Wt + (long)e * N * K;
+  for (int c0 = p0; c0 < p1; c0 += 64) {  // token chunks of 64 pairs
+    const int nrow = min(64, p1 - c0);
+#define CHUNK(...) moe_chunk<NTF, NW, EPI, __VA_ARGS__>(Xq, xs, rows, We, ws + (long)e * N, route_w, Y, N, K, n0, c0, nrow, red)
+    if (nrow <= 16) CHUNK(1, 4);
+    else if (nrow <= 32) CHUNK(2, 3);
+    else if (p1 - p0 <= 64) CHUNK(4, 2);
+    else CHUNK(4, 2, false);   // (the next chunk reads the weights again)
+#undef CHUNK
   }
 }
 
@@ -620,20 +657,23 @@ static int moe_gemm_launch(const void* Xq, const float* xs, const int* rows, con
                            const float* ws, const float* route_w, void* Y, int E, int N, int K, int epi,
                            hipStream_t stream) {
   dim3 grid(N / (16 * NTF), E);
-  // waves split K: as many as divide it into whole 64-wide k-pairs (4 for every real model)
+  // Waves split K into whole 64-wide k-pairs.  Thin workgroups (NTF 2) want long streams a wave: 2 waves up to K = 8192 (4096, 48 / 64 / 96
+  // tokens: 143 / 154 / 180 us, 4 waves 146 / 162 / 190), 8 beyond, where they are taken because few of them fill the chip (14336, one
+  // token 18.7, 4 waves 24.7).  NTF 4: 4 waves (4096, 128 tokens 175, 2 waves 184).
 #define MOE_LAUNCH(NW_)                                                                                          \
   {                                                                                                              \
-    const size_t lds = (size_t)NW_ * 16 * NTF * 64 * sizeof(float);                                             \
     if (epi == MOE_EPI_SILU)                                                                                     \
-      hipLaunchKernelGGL((moe_gemm_kernel<NTF, NW_, MOE_EPI_SILU>), grid, dim3(NW_ * 64), lds, stream,          \
+      hipLaunchKernelGGL((moe_gemm_kernel<NTF, NW_, MOE_EPI_SILU>), grid, dim3(NW_ * 64), 0, stream,            \
                          (const unsigned char*)Xq, xs, rows, offsets, (const unsigned char*)Wt, ws, route_w,     \
                          (bf16*)Y, N, K);                                                                        \
     else                                                                                                         \
-      hipLaunchKernelGGL((moe_gemm_kernel<NTF, NW_, MOE_EPI_ROUTEW>), grid, dim3(NW_ * 64), lds, stream,        \
+      hipLaunchKernelGGL((moe_gemm_kernel<NTF, NW_, MOE_EPI_ROUTEW>), grid, dim3(NW_ * 64), 0, stream,          \
                          (const unsigned char*)Xq, xs, rows, offsets, (const unsigned char*)Wt, ws, route_w,     \
                          (bf16*)Y, N, K);                                                                        \
   }
-  if (K % 256 == 0) MOE_LAUNCH(4)
+  if (NTF == 2 && K % 128 == 0 && K < 8192) MOE_LAUNCH(2)
+  else if (NTF == 2 && K % 512 == 0) MOE_LAUNCH(8)
+  else if (K % 256 == 0) MOE_LAUNCH(4)
   else if (K % 128 == 0) MOE_LAUNCH(2)
   else MOE_LAUNCH(1)
 #undef MOE_LAUNCH

@@ -123,7 +123,7 @@ def moe_prefill_fp8(h: torch.Tensor, router_logits: torch.Tensor, w13t: torch.Te
     xq, xs, offsets, tok_idx, tok_w, inv = _route_and_quant(h, router_logits, top_k, E)
     st = N.stream()
     a = torch.empty((P, F_), dtype=torch.bfloat16, device=h.device)
-    ntf13, ntf2 = MOE_NTF
+    ntf13, ntf2 = moe_ntf(P, E, F2, H)
     N.call("penny_moe_gemm_fp8", N.ptr(xq), N.ptr(xs), N.ptr(tok_idx), N.ptr(offsets), N.ptr(w13t), N.ptr(s13), None,
            N.ptr(a), E, F2, H, 1, ntf13, st)
     aq = torch.empty((P, F_), dtype=torch.uint8, device=h.device)
@@ -201,7 +201,7 @@ def moe_grouped_fp8(x: torch.Tensor, expert_ids: torch.Tensor, w13t: torch.Tenso
     xs = torch.empty(M, dtype=torch.float32, device=x.device)
     N.call("penny_quant_rows_fp8", N.ptr(x), x.stride(0), M, H, N.ptr(xq), N.ptr(xs), st)
     a = torch.zeros((M, F_), dtype=torch.bfloat16, device=x.device)
-    ntf13, ntf2 = MOE_NTF
+    ntf13, ntf2 = moe_ntf(M, E, F2, H)
     N.call("penny_moe_gemm_fp8", N.ptr(xq), N.ptr(xs), N.ptr(rows), N.ptr(offsets), N.ptr(w13t), N.ptr(s13), None,
            N.ptr(a), E, F2, H, 1, ntf13, st)
     aq = torch.empty((M, F_), dtype=torch.uint8, device=x.device)
@@ -401,9 +401,18 @@ def moe_fp8_reference(h, router_w, w13q, s13, w2q, s2, top_k, quant_act=False):
     return out.to(h.dtype)
 
 
-# 16-row weight groups per workgroup for the (W13, W2) grouped fp8 GEMMs (PENNY_MOE_NTF="a,b"):
-# 4,4 measured 6-16 % faster than 2,2 at T = 64-256 decode tokens (profiles/r1_moe_ntf.jsonl)
-MOE_NTF = tuple(int(v) for v in os.environ.get("PENNY_MOE_NTF", "4,4").split(","))
+# 16-row weight groups per workgroup for the (W13, W2) grouped fp8 GEMMs: PENNY_MOE_NTF="a,b", or by moe_ntf's rule
+MOE_NTF = tuple(int(v) for v in os.environ["PENNY_MOE_NTF"].split(",")) if "PENNY_MOE_NTF" in os.environ else None
+
+
+def moe_ntf(P: int, E: int, F2: int, H: int) -> tuple:
+    """(W13, W2) row groups for P pairs over E experts.  W13: 2 while an expert has about 20 pairs, as its weights then stream faster (8
+    experts of 4096 -> 28672, 16 / 48 / 64 / 80 / 96 tokens: 138 / 146 / 154 / 165 / 180 us, 4 groups 164 / 163 / 163 / 166 / 167); 4
+    beyond, for half the reads of activations.  W2: 2 where 4 would leave fewer than 512 workgroups (14336 -> 4096, 1 / 4 tokens: 18.7 /
+    36.1, 4 groups 23.4 / 37.1), else 4 (48 / 64 tokens 72 / 74, 2 groups 75 / 84)."""
+    if MOE_NTF is not None:
+        return MOE_NTF
+    return 2 if P <= 20 * E and F2 % 64 == 0 else 4, 2 if min(P, E) * H < 64 * 512 and H % 64 == 0 else 4
 
 
 class MoEWorkspace:
@@ -476,7 +485,7 @@ def _moe_decode_experts(h: torch.Tensor, w13t: torch.Tensor, s13: torch.Tensor, 
     F_ = F2 // 2
     P = T * top_k
     st = N.stream()
-    ntf13, ntf2 = MOE_NTF
+    ntf13, ntf2 = moe_ntf(P, E, F2, H)
     N.call("penny_moe_gemm_fp8", N.ptr(ws.xq), N.ptr(ws.xs), N.ptr(ws.sorted_tok), N.ptr(ws.offsets), N.ptr(w13t),
            N.ptr(s13), None, N.ptr(ws.a), E, F2, H, 1, ntf13, st)
     N.call("penny_quant_rows_fp8", N.ptr(ws.a), F_, P, F_, N.ptr(ws.aq), N.ptr(ws.as_), st)
