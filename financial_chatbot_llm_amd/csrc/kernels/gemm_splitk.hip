@@ -184,7 +184,12 @@ __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restr
   constexpr int SLOT = BKM * SBYTES;
   __shared__ __attribute__((aligned(1024))) char smem[NBUF * SLOT];
 
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, col = lane & 15;
+  // The tiled weight past the caches (nt): the stream is faster, its loads take longer.  Ahead while the ring holds many stages (gate|up of
+  // 28672 x 4096, 16 / 32 rows: 45.7 -> 43.4, 45.5 -> 42.9 us; QKV of 6144 11.3 -> 10.8, 11.7 -> 11.3), and with K in slices for wide
+  // tiles to 64 rows (4096 x 14336, 32 / 48 / 64 rows: 22.4 -> 20.5, 23.8 -> 22.6, 24.2 -> 23.3); behind otherwise (gate|up of 64 rows 44.2
+  // and 45.4, 128 rows 53 and 61; 4096 x 4096, 64 rows 9.8 and 10.3).
+  constexpr bool ONCE = !WROW && (MT <= 2 || (MT <= 4 && EPI == SK_SLAB && NF >= 6));
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, col = lane & 15;
   const int s = blockIdx.x % S, tile = blockIdx.x / S;
   // token chunks (blockIdx.y): rows m0 .. m0 + 16*MT - 1 of X / Y / the slabs; one chunk for decode
   // batches, ceil(M / (16*MT)) for the small prefill steps of narrow TP shards
@@ -234,14 +239,15 @@ __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restr
   }
   auto stage = [&](int j) {
     char* base = smem + (j % NBUF) * SLOT;
-    // default cache policy on W too: the nt hint measured 4-7 % slower at M >= 48 (2-3 % faster
-    // only at M <= 32; profiles/r1_splitk_v5_qkv_nont.jsonl vs r1_splitk_v4_qkv.jsonl)
 #pragma unroll
     for (int i = 0; i < LOADS; ++i)
 #pragma unroll
-      for (int u = 0; u < BKM; ++u)
-        __builtin_amdgcn_global_load_lds((gbl_void_t*)(src[i] + (j * BKM + u) * step[i]),
-                                         (lds_void_t*)(base + u * SBYTES + dst[i]), 16, 0, 0);
+      for (int u = 0; u < BKM; ++u) {
+        gbl_void_t* from = (gbl_void_t*)(src[i] + (j * BKM + u) * step[i]);
+        lds_void_t* to = (lds_void_t*)(base + u * SBYTES + dst[i]);
+        if (ONCE && w * LOADS + i < 2 * NF) __builtin_amdgcn_global_load_lds(from, to, 16, 0, 2);   // nt
+        else __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
+      }
   };
 
   constexpr int SUMS = EPI == SK_F32 ? 4 : 1;
