@@ -563,20 +563,22 @@ __global__ void __launch_bounds__(512) expert_wide_kernel(ExpertGemm a) {
 // reader of its rows.  Bound by latency: one read of the indices and three passes through LDS, 1 - 3 us of the product for the 4 of the
 // launch (passes of 1 - 64 rows with four such layers 1 - 13 us shorter: f32 1 row 592 / 583, 60 rows of width 1024 665 / 652, of 2048 1027 / 1020).
 // own: the tile's pairs.  Returns (expert, first sorted row, rows, -).
+template <int NW>
 __device__ __forceinline__ int4 plan_tile(const ExpertGemm& a, int* own) {
-  __shared__ int count[64], found[4][4];
+  constexpr int THREADS = NW * 64, C = 1024 / THREADS;
+  __shared__ int count[64], found[C][NW];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, y = blockIdx.y, E = a.experts;
   const bool leave = blockIdx.x == 0;
-  int held[4];
+  int held[C];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int i = threadIdx.x + 256 * c;
+  for (int c = 0; c < C; ++c) {
+    const int i = threadIdx.x + THREADS * c;
     held[c] = i < a.pairs ? a.idx[i] : E;
   }
   if (threadIdx.x < 64) count[threadIdx.x] = 0;
   __syncthreads();
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
+  for (int c = 0; c < C; ++c)
     if ((unsigned)held[c] < (unsigned)E) atomicAdd(count + held[c], 1);
   __syncthreads();
   const int n = lane < E ? count[lane] : 0;
@@ -597,12 +599,12 @@ __device__ __forceinline__ int4 plan_tile(const ExpertGemm& a, int* own) {
   if (leave && threadIdx.x == 0) a.tiles_out[y] = tile;
   if (leave && y == 0)
 #pragma unroll
-    for (int c = 0; c < 4; ++c)                              // identity entries have no row
-      if (threadIdx.x + 256 * c < a.pairs && (unsigned)held[c] >= (unsigned)E) a.pos[threadIdx.x + 256 * c] = 0;
+    for (int c = 0; c < C; ++c)                              // identity entries have no row
+      if (threadIdx.x + THREADS * c < a.pairs && (unsigned)held[c] >= (unsigned)E) a.pos[threadIdx.x + THREADS * c] = 0;
   if (tile.z == 0) return tile;
-  int before[4];
+  int before[C];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
+  for (int c = 0; c < C; ++c) {
     const unsigned long long m = __ballot(held[c] == tile.x);
     before[c] = __popcll(m & ((1ull << lane) - 1));
     if (lane == 0) found[c][w] = __popcll(m);
@@ -610,12 +612,12 @@ __device__ __forceinline__ int4 plan_tile(const ExpertGemm& a, int* own) {
   __syncthreads();
   int at = -first;
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
+  for (int c = 0; c < C; ++c)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
+    for (int v = 0; v < NW; ++v) {
       const int r = at + before[c];
       if (v == w && held[c] == tile.x && r >= 0 && r < 16) {
-        const int i = threadIdx.x + 256 * c;
+        const int i = threadIdx.x + THREADS * c;
         own[r] = i;
         if (leave) {
           a.pos[i] = tile.y + r;
@@ -628,71 +630,85 @@ __device__ __forceinline__ int4 plan_tile(const ExpertGemm& a, int* own) {
   return tile;
 }
 
-// NF row groups x 16 tokens per block; wave w takes the w-th quarter of the pieces, the partial sums meet in LDS.
-template <typename T, int NF, bool GLU, bool PLAN>
-__global__ void __launch_bounds__(256) expert_stream_kernel(ExpertGemm a) {
-  constexpr int ES = sizeof(T), UN = 8;
-  __shared__ f32x4 red[4][NF][64];
+// Two row groups x 16 tokens per block; the NW waves share the pieces of K, their partial sums meet in LDS.  Bound by the weights' stream,
+// past the caches as each is read once: four steps of weights and rows are always in flight per wave, and thin blocks of long streams
+// keep many of them at it.  Both products in us, four groups x 4 waves that drain every eight steps (before) / the same drained never /
+// two groups x 4 waves / two groups x 2 waves: 32 experts of 1024 x 2048, top 4, 1 token 19.5 / 15.9 / 15.9 / 15.8, 16 tokens 71 / 70 / 62 / 61, 64 tokens 80 /
+// 79 / 70 / 70 (5.8 TB/s), f32 156 / 164 / 142 / 135; 8 of 2048 x 4096, 16 tokens 85 / 90 / 76 / 71; 16 of 512 x 1024, 8 tokens 17.3 / 14.8
+// / 14.8 / 14.7.  Eight steps in flight measured the same.
+template <typename T, bool GLU, bool PLAN, int NW>
+__global__ void __launch_bounds__(NW * 64) expert_stream_kernel(ExpertGemm a) {
+  constexpr int ES = sizeof(T), NF = 2, D = 4;
+  __shared__ f32x4 red[NW][NF][64];
   __shared__ int own[16];
   int4 tile;
-  if constexpr (PLAN) tile = plan_tile(a, own);
+  if constexpr (PLAN) tile = plan_tile<NW>(a, own);
   else tile = a.tiles[blockIdx.y];
   const int rows = tile.z;
   if (rows == 0) return;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, col = lane & 15;
+  // (a wave's number of steps has to be uniform to the compiler: matrix instructions run whatever the lanes' mask)
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, col = lane & 15;
   const int G = blockIdx.x * NF;
-  const uint4* wp[NF];
+  const int k0 = a.kt * w / NW, steps = a.kt * (w + 1) / NW - k0;
+  const char* wp[NF];
 #pragma unroll
   for (int f = 0; f < NF; ++f)
-    wp[f] = reinterpret_cast<const uint4*>(a.w + tile.x * a.wstride + (long)min(G + f, a.groups - 1) * a.kt * 1024) + lane;
+    wp[f] = reinterpret_cast<const char*>(a.w) + (tile.x * a.wstride + (long)min(G + f, a.groups - 1) * a.kt * 1024 + k0 * 1024) + 16 * lane;
   const char* xp = (PLAN ? static_cast<const char*>(a.x) + own[min(col, rows - 1)] / a.top * a.ldx * ES
-                         : expert_row(a, tile.y + min(col, rows - 1), ES)) + 16 * g;
+                         : expert_row(a, tile.y + min(col, rows - 1), ES)) + 16 * g + k0 * 64;
+  const int behind = a.kbytes - 16 * g - k0 * 64;            // the row's bytes from this lane's first chunk on
   const char* zero = reinterpret_cast<const char*>(&g_zero16);
   f32x4 acc[NF];
 #pragma unroll
   for (int f = 0; f < NF; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int k0 = a.kt * w / 4, k1 = a.kt * (w + 1) / 4;
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-  auto steps = [&](int k, auto count) {
-    constexpr int U = decltype(count)::value;
-    uint4 av[U][NF], bv[U];
+  uint4 av[D][NF], bv[D];
+  auto fetch = [&](int d, int k) {
 #pragma unroll
-    for (int j = 0; j < U; ++j) {
-#pragma unroll
-      for (int f = 0; f < NF; ++f) {
-        const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wp[f] + (long)(k + j) * 64));
-        av[j][f] = make_uint4(v.x, v.y, v.z, v.w);
-      }
-      const int off = (k + j) * 64;
-      bv[j] = *reinterpret_cast<const uint4*>(off + 16 * g < a.kbytes ? xp + off : zero);
+    for (int f = 0; f < NF; ++f) {
+      const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wp[f] + k * 1024));
+      av[d][f] = make_uint4(v.x, v.y, v.z, v.w);
     }
-#pragma unroll
-    for (int j = 0; j < U; ++j)
-#pragma unroll
-      for (int f = 0; f < NF; ++f) acc[f] = mma16<T>(av[j][f], bv[j], acc[f]);
+    bv[d] = *reinterpret_cast<const uint4*>(k * 64 < behind ? xp + k * 64 : zero);
   };
-  int k = k0;
-  for (; k + UN <= k1; k += UN) steps(k, Steps<UN>{});
-  for (; k < k1; ++k) steps(k, Steps<1>{});
+  auto use = [&](int d) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) acc[f] = mma16<T>(av[d][f], bv[d], acc[f]);
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (d < steps) fetch(d, d);
+  int k = 0;
+  for (; k + 2 * D <= steps; k += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      use(d);
+      fetch(d, k + D + d);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  for (; k < steps; k += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      if (k + d < steps) use(d);
+      if (k + D + d < steps) fetch(d, k + D + d);
+    }
+  }
 #pragma unroll
   for (int f = 0; f < NF; ++f) red[w][f][lane] = acc[f];
   __syncthreads();
   auto total = [&](int i) {
     f32x4 s = red[0][i][lane];
 #pragma unroll
-    for (int v = 1; v < 4; ++v) s += red[v][i][lane];
+    for (int v = 1; v < NW; ++v) s += red[v][i][lane];
     return s;
   };
-  constexpr int ITEMS = GLU ? NF / 2 : NF;
-  for (int f = w; f < ITEMS; f += 4) {
-    if (col >= rows) continue;
-    if (GLU) {
-      if (G + 2 * f < a.groups)
-        expert_store<T, true>(a, tile.y + col, (G / 2 + f) * 16 + 4 * g, total(2 * f), total(2 * f + 1), PLAN ? own[col] : -1);
-    } else if (G + f < a.groups) {
-      const f32x4 s = total(f);
-      expert_store<T, false>(a, tile.y + col, (G + f) * 16 + 4 * g, s, s);
-    }
+  if (col >= rows) return;
+  if (GLU) {
+    if (w == 0 && G < a.groups) expert_store<T, true>(a, tile.y + col, G / 2 * 16 + 4 * g, total(0), total(1), PLAN ? own[col] : -1);
+  } else if (w < NF && G + w < a.groups) {
+    const f32x4 s = total(w);
+    expert_store<T, false>(a, tile.y + col, (G + w) * 16 + 4 * g, s, s);
   }
 }
 
@@ -774,13 +790,14 @@ int expert_launch(const ExpertGemm& a, int mt, hipStream_t st) {
     expert_tile_kernel<T, 2, GLU><<<(unsigned)grid, 256, 0, st>>>(a);
   } else {
     if (a.ntiles > 65535) return (int)hipErrorInvalidValue;
-    const bool wide = (long)a.ntiles * (a.groups / 4) >= 512;       // enough blocks of 64 W rows to fill the chip
-    const dim3 grid((a.groups + (wide ? 3 : 1)) / (wide ? 4 : 2), a.ntiles);
+    const dim3 grid((a.groups + 1) / 2, a.ntiles);
+    // two waves a block where the blocks alone fill the chip, four otherwise (us of both products: above)
+    const bool many = (long)a.ntiles * (a.groups / 4) >= 512;
     if (a.idx != nullptr) {
-      if (wide) expert_stream_kernel<T, 4, GLU, true><<<grid, 256, 0, st>>>(a);
-      else expert_stream_kernel<T, 2, GLU, true><<<grid, 256, 0, st>>>(a);
-    } else if (wide) expert_stream_kernel<T, 4, GLU, false><<<grid, 256, 0, st>>>(a);
-    else expert_stream_kernel<T, 2, GLU, false><<<grid, 256, 0, st>>>(a);
+      if (many) expert_stream_kernel<T, GLU, true, 2><<<grid, 128, 0, st>>>(a);
+      else expert_stream_kernel<T, GLU, true, 4><<<grid, 256, 0, st>>>(a);
+    } else if (many) expert_stream_kernel<T, GLU, false, 2><<<grid, 128, 0, st>>>(a);
+    else expert_stream_kernel<T, GLU, false, 4><<<grid, 256, 0, st>>>(a);
   }
   return (int)hipGetLastError();
 }
