@@ -446,7 +446,7 @@ state_step_kernel(const TQ* __restrict__ q, long sq, const TQ* __restrict__ k, l
 #pragma unroll
   for (int i = 0; i < RPT; ++i) {
     const int d = 32 * i + rg;
-    S[i] = !fresh && d < D ? ldf4(srec + (long)d * P) : mx_f32x4{0.f, 0.f, 0.f, 0.f};
+    S[i] = !fresh && d < D ? ldf4_once(srec + (long)d * P) : mx_f32x4{0.f, 0.f, 0.f, 0.f};
   }
   mx_f32x4 u;
   const int fact = beta_code & 15, vcode = beta_code >> 4;
@@ -509,7 +509,7 @@ state_step_kernel(const TQ* __restrict__ q, long sq, const TQ* __restrict__ k, l
     const int d = 32 * i + rg;
     S[i] += u * (ks[d] * fk);
     o += S[i] * (qs[d] * fq);
-    if (d < D && c < P) stf4(srec + (long)d * P, S[i]);
+    if (d < D && c < P) stf4_once(srec + (long)d * P, S[i]);
   }
   o = total(o, 1);
   if (tid < 8 && c < P) stf4(out + t * H * P + h * P + c, DELTA ? o : o * (FIXED ? tau_inv : qscale));

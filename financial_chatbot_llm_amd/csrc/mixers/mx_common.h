@@ -102,6 +102,9 @@ template <typename T> __device__ __forceinline__ void stf4(T* p, mx_f32x4 x) {
   typedef T v4 __attribute__((ext_vector_type(4)));
   *reinterpret_cast<v4*>(p) = v4{(T)x[0], (T)x[1], (T)x[2], (T)x[3]};
 }
+// what a launch reads or writes once and nobody needs before much else has passed (recurrent states): not kept in the caches
+__device__ __forceinline__ mx_f32x4 ldf4_once(const float* p) { return __builtin_nontemporal_load(reinterpret_cast<const mx_f32x4*>(p)); }
+__device__ __forceinline__ void stf4_once(float* p, mx_f32x4 x) { __builtin_nontemporal_store(x, reinterpret_cast<mx_f32x4*>(p)); }
 // rows of `stride` elements of type code dt (1: f32) may be read and written by four
 inline bool mx_by_four(const void* p, long stride, int dt) { return stride % 4 == 0 && (size_t)p % (dt == 1 ? 16 : 8) == 0; }
 

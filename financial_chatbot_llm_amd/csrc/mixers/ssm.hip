@@ -160,7 +160,8 @@ __device__ __forceinline__ float row_sum16(float v) {
 
 // A step of single rows (decode): a block takes a head, its threads 16 of the value channels at a time with 16 lanes by fours along
 // the state's NJ 64s, up to 64 channels' states asked for at once; B and C, the same for all of them, stay in registers.  Bound by the
-// state's bytes: 64 rows of 64 heads of 64 x 128 47 us (5.7 TB/s), by the scan below, whose chunk of staged rows leaves room for three blocks a
+// state's bytes, which do not stay in the caches on either way: 64 rows of 64 heads of 64 x 128 46 us (5.8 TB/s; 48 where they stay, and
+// the step's other launches longer: 8 layers 1157 / 1117, 17 rows 504 / 480), by the scan below, whose chunk of staged rows leaves room for three blocks a
 // CU, 62; 17 rows of 32 heads 9.6, 13.4.
 template <typename TD, int NJ>
 __global__ void __launch_bounds__(256)
@@ -185,7 +186,7 @@ ssm_step_kernel(const float* __restrict__ u, int C, const TD* __restrict__ dt_ra
       const int p = min(p0 + 16 * i + pl, P - 1);
       x[i] = ur[h * P + p];
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) S[i][j] = fresh ? mx_f32x4{0.f, 0.f, 0.f, 0.f} : ldf4(sh + (long)p * N + 64 * j);
+      for (int j = 0; j < NJ; ++j) S[i][j] = fresh ? mx_f32x4{0.f, 0.f, 0.f, 0.f} : ldf4_once(sh + (long)p * N + 64 * j);
     }
   };
   load(0);
@@ -203,7 +204,7 @@ ssm_step_kernel(const float* __restrict__ u, int C, const TD* __restrict__ dt_ra
       for (int j = 0; j < NJ; ++j) {
         S[i][j] = a * S[i][j] + dx * B[j];
         acc += S[i][j] * Cv[j];
-        if (p < P) stf4(sh + (long)p * N + 64 * j, S[i][j]);
+        if (p < P) stf4_once(sh + (long)p * N + 64 * j, S[i][j]);
       }
       const float o = row_sum16((acc[0] + acc[1]) + (acc[2] + acc[3]));
       if (ns == 0 && p < P) y[t * inner + h * P + p] = o + Dh * x[i];
