@@ -161,7 +161,15 @@ __device__ __forceinline__ void stage_mma(const char* __restrict__ base, f32x4 (
 // whole 128-B lines and the fragment reads stay conflict-free.
 // RKB: LDS ring budget in KiB (150: one workgroup per CU; ~72: two co-resident workgroups, so one's
 // pipeline ramp overlaps the other's stream when a CU runs several tiles in sequence).
-template <int NF, int MT, int WA, int EPI = SK_SLAB, bool WROW = false, int RKB = 150, int MAXB = 8, int BKM = 1>
+// ONCE: the weight past the caches (nt), so that what the launches around it read -- rows, slabs, states, small weights -- stays in them.
+// Its loads take longer: by itself a launch gains while its ring holds many stages (gate|up of 28672 x 4096, 16 / 32 / 64 / 128 rows, the
+// weight through the caches / past them: 45.7 / 43.4, 45.5 / 42.9, 44.2 / 45.4, 53 / 61 us), but a step gains beyond that: 32 such layers
+// with the tiled weight past the caches to no rows / 32 / 64 / 128: 64 rows 7504 / 7400 / 7220 / 7190 us, 96 rows 6115 / 6035 / 6015 / 5750, 128 rows
+// 7330 / 7260 / 7190 / 6960; at 192 and 256 rows nothing.  Row-major weights in one chunk of rows: 8 hybrid layers of width 2048, 64 rows
+// 1129 / 1078 us, 15 rows 817 / 778, 3 rows 625 / 575, f32 1 row 562 / 516, 90 rows 1231 / 1180; in several chunks, which all read the weight, 1154 and 1186
+// for 100 rows.  Not for the encoder (SK_BIAS), whose weights stay on the chip from pass to pass: 60 tokens 446 and 490 us.
+template <int NF, int MT, int WA, int EPI = SK_SLAB, bool WROW = false, int RKB = 150, int MAXB = 8, int BKM = 1,
+          bool ONCE = !WROW && MT <= 8>
 __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restrict__ X, int ldx,
                                                              const bf16* __restrict__ Wt, int K,
                                                              float* __restrict__ P, int M, int N, int S,
@@ -184,11 +192,6 @@ __global__ void __launch_bounds__(256, 1) splitk_gemm_kernel(const bf16* __restr
   constexpr int SLOT = BKM * SBYTES;
   __shared__ __attribute__((aligned(1024))) char smem[NBUF * SLOT];
 
-  // The tiled weight past the caches (nt): the stream is faster, its loads take longer.  Ahead while the ring holds many stages (gate|up of
-  // 28672 x 4096, 16 / 32 rows: 45.7 -> 43.4, 45.5 -> 42.9 us; QKV of 6144 11.3 -> 10.8, 11.7 -> 11.3), and with K in slices for wide
-  // tiles to 64 rows (4096 x 14336, 32 / 48 / 64 rows: 22.4 -> 20.5, 23.8 -> 22.6, 24.2 -> 23.3); behind otherwise (gate|up of 64 rows 44.2
-  // and 45.4, 128 rows 53 and 61; 4096 x 4096, 64 rows 9.8 and 10.3).
-  constexpr bool ONCE = !WROW && (MT <= 2 || (MT <= 4 && EPI == SK_SLAB && NF >= 6));
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, col = lane & 15;
   const int s = blockIdx.x % S, tile = blockIdx.x / S;
   // token chunks (blockIdx.y): rows m0 .. m0 + 16*MT - 1 of X / Y / the slabs; one chunk for decode
@@ -445,6 +448,18 @@ constexpr bool pair_fits() {
   return Ring<NF, MT, RKB, MAXB, 2>::NBUF >= 3;
 }
 
+// row-major weights: past the caches in one chunk of rows (ONCE above)
+template <int NF, int MT, int WA, int EPI, int MAXB, int BKM, class... A>
+void launch_rows(dim3 grid, hipStream_t st, A... args) {
+  if constexpr (MT <= 8 && EPI != SK_BIAS) {
+    if (grid.y == 1) {
+      hipLaunchKernelGGL((splitk_gemm_kernel<NF, MT, WA, EPI, true, 150, MAXB, BKM, true>), grid, dim3(256), 0, st, args...);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((splitk_gemm_kernel<NF, MT, WA, EPI, true, 150, MAXB, BKM, false>), grid, dim3(256), 0, st, args...);
+}
+
 // one launch of splitk_gemm_kernel<NF, MT, WA, EPI, *, 150, MAXB, *> with the W layout / stage pairing
 // of wrow (runtime) mapped onto the template arguments.  ROWS: row-major weights only (the entries whose last tile of columns may be
 // part-filled, which the tiled copy's form does not know).
@@ -454,12 +469,12 @@ int launch_any(int wrow, bool pair_ok, dim3 grid, hipStream_t st, A... args) {
   if (ROWS && !rm) return (int)hipErrorInvalidValue;
   if constexpr (pair_fits<NF, MT, 150, MAXB>()) {
     if ((wrow & 2) && pair_ok) {
-      if (rm) hipLaunchKernelGGL((splitk_gemm_kernel<NF, MT, WA, EPI, true, 150, MAXB, 2>), grid, dim3(256), 0, st, args...);
+      if (rm) launch_rows<NF, MT, WA, EPI, MAXB, 2>(grid, st, args...);
       else if constexpr (!ROWS) hipLaunchKernelGGL((splitk_gemm_kernel<NF, MT, WA, EPI, false, 150, MAXB, 2>), grid, dim3(256), 0, st, args...);
       return (int)hipGetLastError();
     }
   }
-  if (rm) hipLaunchKernelGGL((splitk_gemm_kernel<NF, MT, WA, EPI, true, 150, MAXB>), grid, dim3(256), 0, st, args...);
+  if (rm) launch_rows<NF, MT, WA, EPI, MAXB, 1>(grid, st, args...);
   else if constexpr (!ROWS) hipLaunchKernelGGL((splitk_gemm_kernel<NF, MT, WA, EPI, false, 150, MAXB>), grid, dim3(256), 0, st, args...);
   return (int)hipGetLastError();
 }
@@ -475,13 +490,11 @@ int launch_f32(const void* X, int ldx, const void* W, int K, float* P, int M, in
   const dim3 grid(((N + 16 * NF - 1) / (16 * NF)) * S, (M + 16 * MT - 1) / (16 * MT));
   if constexpr (pair_fits<NF, MT, 150, 16>()) {
     if (paired && (K / S) % 64 == 0) {
-      hipLaunchKernelGGL((splitk_gemm_kernel<NF, MT, WA, SK_F32, true, 150, 16, 2>), grid, dim3(256), 0, st, (const bf16*)X, 2 * ldx,
-                         (const bf16*)W, 2 * K, P, M, N, S, (bf16*)nullptr, 0, SkSample{});
+      launch_rows<NF, MT, WA, SK_F32, 16, 2>(grid, st, (const bf16*)X, 2 * ldx, (const bf16*)W, 2 * K, P, M, N, S, (bf16*)nullptr, 0, SkSample{});
       return (int)hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((splitk_gemm_kernel<NF, MT, WA, SK_F32, true, 150, 16>), grid, dim3(256), 0, st, (const bf16*)X, 2 * ldx, (const bf16*)W,
-                     2 * K, P, M, N, S, (bf16*)nullptr, 0, SkSample{});
+  launch_rows<NF, MT, WA, SK_F32, 16, 1>(grid, st, (const bf16*)X, 2 * ldx, (const bf16*)W, 2 * K, P, M, N, S, (bf16*)nullptr, 0, SkSample{});
   return (int)hipGetLastError();
 }
 
