@@ -12,8 +12,8 @@
 // step j takes K element 4 g + j of both operands).  Accumulation is f32; the unit sees the f32 sums.
 //
 // Three forms, chosen by the rows an expert gets on average (the bucket sizes stay on the device):
-//   tile    128 W rows x 64 or 128 tokens per block, both operands through a two-stage LDS ring filled by LDS-DMA,
-//           two or three blocks per CU: bound by the operand reads.  4096 tokens, width 2048, 32 experts of 1024, top 4,
+//   tile    128 W rows x 64 or 128 tokens per block (64 x 64 for few in f32), both operands through an LDS ring of two or three stages
+//           filled by LDS-DMA, two or three blocks per CU: bound by the operand reads.  4096 tokens, width 2048, 32 experts of 1024, top 4,
 //           bf16: 300 us for both products (650 TFLOP/s); 31 pairs of library products and the host's wait for the
 //           bucket sizes took 1.3 ms.
 //   wide    256 W rows x 256 tokens per block, bf16: bound by the matrix cores and, with few rounds of blocks, by the last one
@@ -300,32 +300,42 @@ __device__ __forceinline__ bool expert_place(const ExpertGemm& a, int cols, int&
 }
 
 // ---- tile form ---------------------------------------------------------------------------------------------------
-// 256 threads = 4 waves as 2 (W rows) x 2 (tokens), a wave's 64 x 16 MF sub-tile as 4 x MF accumulators (A = W: a
-// lane's four registers are adjacent output columns).  A stage is 128 bytes of K: the W image keeps the pieces'
-// order, the X image has rows of 128 B whose 16-B chunks are swizzled by (row / 2) % 8 (conflict-free b128 reads).
-template <typename T, int MF, bool GLU>
-__global__ void __launch_bounds__(256, MF == 4 ? 2 : 3) expert_tile_kernel(ExpertGemm a) {
-  constexpr int MT = 32 * MF, WIMG = 16384, STG = WIMG + MT * 128, ES = sizeof(T);
-  constexpr int XP = MT / 32;             // 1-KiB pieces of the X image per wave
-  __shared__ __attribute__((aligned(1024))) char smem[2 * STG];
+// WR row groups of W x MT tokens per block, 256 threads = 4 waves: 4 x 1 in blocks of 8 groups x 64 tokens, else 2 (W) x 2 (every other group
+// of 16 tokens), a wave's sub-tile as FW x U accumulators (A = W: a lane's four registers are adjacent output columns).  A stage is 128
+// bytes of K, ST of them in LDS: the W image keeps the pieces' order, the X image has rows of 128 B whose 16-B chunks are swizzled by
+// (row / 2) % 8 (conflict-free b128 reads).  An expert's last tile is half full on average and with few rows its only one: groups of
+// 16 tokens without a row are not multiplied (nor staged, with two stages), and the rest is dealt evenly over the waves.  f32 is bound by the matrix
+// cores, whose work is a block's chain of 14 us (8 groups, K = 1024) for each 16 of its tokens: both products in us, every group multiplied / 8
+// groups of W / 4 with three stages, 32 experts of 1024 x 512, buckets even and (spread by a factor of three): 338 tokens, top 4, 118 / 106 / 100
+// (118 / 117 / 101), 800 180 / 168 / 158 (181 / 181 / 159), 520 119 / 119 / 104 (118 / 118 / 130), 1600 235 / 238 / 245 (236 / 235 / 243).  bf16 is
+// bound by the way of the operands to LDS: 0 - 4 % shorter, and longer with blocks of 4 groups (1188 tokens of 2048 x 1024 145, 158) or a
+// third stage (146 and 155 for 142 and 146).
+template <typename T, int MT, int WR, int ST, bool GLU>
+__global__ void __launch_bounds__(256, 163840 / (ST * (WR * 2048 + MT * 128))) expert_tile_kernel(ExpertGemm a) {
+  constexpr int WIMG = WR * 2048, STG = WIMG + MT * 128, ES = sizeof(T);
+  constexpr int WP = WR / 2, XP = MT / 32;     // 1-KiB pieces of the two images per wave
+  constexpr int WB = MT == 64 && WR == 8 ? 1 : 2;             // waves over the tokens
+  constexpr int FW = WR * WB / 4, U = MT / 16 / WB;           // a wave's row groups of W and of tokens
+  __shared__ __attribute__((aligned(1024))) char smem[ST * STG];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wa = w >> 1, wb = w & 1, g = lane >> 4, col = lane & 15;
+  // (the half with the odd group of tokens in turn: a wave's place in its block is its SIMD)
+  const int wa = w / WB, wb = WB == 1 ? 0 : (w ^ (blockIdx.x >> 3)) & 1, g = lane >> 4, col = lane & 15;
   int t, nb;
-  if (!expert_place(a, (a.groups + 7) / 8, t, nb)) return;
+  if (!expert_place(a, (a.groups + WR - 1) / WR, t, nb)) return;
   const int4 tile = a.tiles[t];
-  const int rows = tile.z;
+  const int rows = __builtin_amdgcn_readfirstlane(tile.z), live = (rows + 15) / 16;
 
-  const char* wsrc[4];
+  const char* wsrc[WP];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {           // piece p = 4 w + i of the stage: row group p / 2, K step p % 2
-    const int p = 4 * w + i;
-    wsrc[i] = a.w + tile.x * a.wstride + ((long)min(nb * 8 + p / 2, a.groups - 1) * a.kt + p % 2) * 1024 + lane * 16;
+  for (int i = 0; i < WP; ++i) {          // piece p = WP w + i of the stage: row group p / 2, K step p % 2
+    const int p = WP * w + i;
+    wsrc[i] = a.w + tile.x * a.wstride + ((long)min(nb * WR + p / 2, a.groups - 1) * a.kt + p % 2) * 1024 + lane * 16;
   }
   const char* xsrc[XP];
   int xoff[XP];
 #pragma unroll
   for (int i = 0; i < XP; ++i) {
-    const int r = 8 * (w * XP + i) + lane / 8;
+    const int r = 8 * (4 * i + w) + lane / 8;
     xsrc[i] = expert_row(a, tile.y + min(r, rows - 1), ES);
     xoff[i] = 16 * ((lane % 8) ^ ((r >> 1) & 7));
   }
@@ -339,57 +349,69 @@ __global__ void __launch_bounds__(256, MF == 4 ? 2 : 3) expert_tile_kernel(Exper
                  : "memory");
   };
   auto stage = [&](int s) {
-    const unsigned buf = lds0 + (s & 1) * STG;
+    const unsigned buf = lds0 + (s % ST) * STG;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) load(wsrc[i] + (long)s * 2048, buf + (4 * w + i) * 1024);
+    for (int i = 0; i < WP; ++i) load(wsrc[i] + (long)s * 2048, buf + (WP * w + i) * 1024);
 #pragma unroll
     for (int i = 0; i < XP; ++i) {
+      if (ST == 2 && 8 * (4 * i + w) >= 16 * live) break;
       const int off = s * 128 + xoff[i];
-      load(off < a.kbytes ? xsrc[i] + off : zero, buf + WIMG + (w * XP + i) * 1024);
+      load(off < a.kbytes ? xsrc[i] + off : zero, buf + WIMG + (4 * i + w) * 1024);
     }
   };
-  f32x4 acc[4][MF];
+  f32x4 acc[FW][U];
 #pragma unroll
-  for (int f = 0; f < 4; ++f)
+  for (int f = 0; f < FW; ++f)
 #pragma unroll
-    for (int u = 0; u < MF; ++u) acc[f][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < U; ++u) acc[f][u] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int ns = a.kt / 2;
-  stage(0);
-  for (int s = 0; s < ns; ++s) {
-    // this wave's pieces have landed, then everybody's; all reads of the other buffer are done
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (s + 1 < ns) stage(s + 1);
-    const char* wi = smem + (s & 1) * STG + wa * 8192 + lane * 16;
-    const char* xi = smem + (s & 1) * STG + WIMG + (wb * 16 * MF + col) * 128;
-    uint4 av[4][2], bv[MF][2];
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
+  for (int s = 0; s < ST - 1; ++s)
+    if (s < ns) stage(s);
+  auto walk = [&](auto count) {           // all stages with this wave's first NU groups of tokens; every wave meets the same barriers
+    constexpr int NU = decltype(count)::value;
+    for (int s = 0; s < ns; ++s) {
+      // this wave's pieces have landed, then everybody's; all reads of the other buffer are done
+      if (ST == 2 || s + ST - 1 > ns) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((ST - 2) * (WP + XP)) : "memory");
+      if (s + ST - 1 < ns) stage(s + ST - 1);
+      const char* wi = smem + (s % ST) * STG + wa * FW * 2048 + lane * 16;
+      const char* xi = smem + (s % ST) * STG + WIMG + (wb * 16 + col) * 128;
+      uint4 av[FW][2], bv[NU][2];
 #pragma unroll
-      for (int f = 0; f < 4; ++f) av[f][kk] = *reinterpret_cast<const uint4*>(wi + (2 * f + kk) * 1024);
+      for (int kk = 0; kk < 2; ++kk) {
 #pragma unroll
-      for (int u = 0; u < MF; ++u)
-        bv[u][kk] = *reinterpret_cast<const uint4*>(xi + u * 2048 + (((4 * kk + g) ^ ((col >> 1) & 7)) << 4));
+        for (int f = 0; f < FW; ++f) av[f][kk] = *reinterpret_cast<const uint4*>(wi + (2 * f + kk) * 1024);
+#pragma unroll
+        for (int u = 0; u < NU; ++u)
+          bv[u][kk] = *reinterpret_cast<const uint4*>(xi + u * WB * 2048 + (((4 * kk + g) ^ ((col >> 1) & 7)) << 4));
+      }
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int f = 0; f < FW; ++f)
+#pragma unroll
+          for (int u = 0; u < NU; ++u) acc[f][u] = mma16<T>(av[f][kk], bv[u][kk], acc[f][u]);
     }
+  };
+  const int mine = (live - wb + WB - 1) / WB;   // (a wave of the second half may have none: it multiplies one that is not stored)
+  if (U == 4 && mine >= 4) walk(Steps<U>{});
+  else if (U == 4 && mine == 3) walk(Steps<U < 3 ? U : 3>{});
+  else if (mine >= 2) walk(Steps<2>{});
+  else walk(Steps<1>{});
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-      for (int f = 0; f < 4; ++f)
-#pragma unroll
-        for (int u = 0; u < MF; ++u) acc[f][u] = mma16<T>(av[f][kk], bv[u][kk], acc[f][u]);
-  }
-#pragma unroll
-  for (int u = 0; u < MF; ++u) {
-    const int m = wb * 16 * MF + u * 16 + col;
+  for (int u = 0; u < U; ++u) {
+    const int m = (u * WB + wb) * 16 + col;
     if (m >= rows) continue;
-    const int G = nb * 8 + wa * 4;
+    const int G = nb * WR + wa * FW;
     if (GLU) {
 #pragma unroll
-      for (int q = 0; q < 2; ++q)
+      for (int q = 0; q < FW / 2; ++q)
         if (G + 2 * q < a.groups)
           expert_store<T, true>(a, tile.y + m, (G / 2 + q) * 16 + 4 * g, acc[2 * q][u], acc[2 * q + 1][u]);
     } else {
 #pragma unroll
-      for (int f = 0; f < 4; ++f)
+      for (int f = 0; f < FW; ++f)
         if (G + f < a.groups) expert_store<T, false>(a, tile.y + m, (G + f) * 16 + 4 * g, acc[f][u], acc[f][u]);
     }
   }
@@ -782,12 +804,14 @@ int expert_launch(const ExpertGemm& a, int mt, hipStream_t st) {
     const long grid = (long)a.ntiles * ((a.groups + 7) / 8);
     if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
     if constexpr (sizeof(T) == 2) {
-      if (mt == 128) {
-        expert_tile_kernel<T, 4, GLU><<<(unsigned)grid, 256, 0, st>>>(a);
-        return (int)hipGetLastError();
-      }
+      if (mt == 128) expert_tile_kernel<T, 128, 8, 2, GLU><<<(unsigned)grid, 256, 0, st>>>(a);
+      else expert_tile_kernel<T, 64, 8, 2, GLU><<<(unsigned)grid, 256, 0, st>>>(a);
+    } else if (grid <= 768) {
+      // f32 blocks that all lie on the chip at once: whichever CU got one more takes a block's whole time longer, so halves of them (above)
+      expert_tile_kernel<T, 64, 4, 3, GLU><<<(unsigned)(a.ntiles * ((a.groups + 3) / 4)), 256, 0, st>>>(a);
+    } else {
+      expert_tile_kernel<T, 64, 8, 2, GLU><<<(unsigned)grid, 256, 0, st>>>(a);
     }
-    expert_tile_kernel<T, 2, GLU><<<(unsigned)grid, 256, 0, st>>>(a);
   } else {
     if (a.ntiles > 65535) return (int)hipErrorInvalidValue;
     const dim3 grid((a.groups + 1) / 2, a.ntiles);

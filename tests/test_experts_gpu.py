@@ -72,6 +72,11 @@ def check(dtype, T, W, F_, E, top, unit, ident=0, skew=False, strided=False):
     (140, 160, 72, 5, 2, "relu2"),         # 56: the last of bf16's 64-row tiles
     (143, 160, 72, 5, 2, "gelu_tanh"),     # 57: the first of 128
     (700, 256, 264, 6, 2, "clamped"),      # a column block beyond the last group
+    (33, 192, 128, 1, 1, "silu"),          # one expert, three groups of 16 tokens with rows
+    (49, 128, 64, 1, 1, "relu2"),          # four, fewer stages of K than the ring holds
+    (65, 192, 128, 1, 1, "clamped"),       # one row in the second tile
+    (145, 192, 128, 1, 1, "silu"),         # bf16's second tile of 128: an odd number of groups
+    (3072, 2048, 64, 1, 1, "clamped"),     # f32's second product beyond 768 blocks
     (515, 192, 128, 2, 2, "silu"),
 ])
 def test_experts_against_float64(dtype, T, W, F_, E, top, unit):
