@@ -27,6 +27,9 @@ from .configs import ModelConfig
 LAYER = ("qkv", "qkv_b", "o", "o_b", "ln1_g", "ln1_b", "fc1", "fc1_b", "fc2", "fc2_b", "ln2_g", "ln2_b")
 
 
+EMBED_ARGS = 960             # ints that travel with penny_encoder_embed_host's launch
+
+
 class BertEncoder:
     def __init__(self, cfg: ModelConfig, device="cuda", dtype=torch.bfloat16):
         self.cfg = cfg
@@ -68,11 +71,15 @@ class BertEncoder:
             self.w[k] = v.to(self.device, self.dtype).contiguous()
         return self
 
+    def _embed_rows(self) -> Optional[list]:
+        """The embedding's five tensors where the native pass takes them."""
+        rows = [self.w[n] for n in ("word_emb", "pos_emb", "type_emb", "emb_ln_g", "emb_ln_b")]
+        return rows if N.use_native(rows[0]) and self.H in (256, 512, 768, 1024) and \
+            all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.shape[-1] == self.H for t in rows) else None
+
     def _embed(self, ids: torch.Tensor, pos: torch.Tensor) -> torch.Tensor:
-        c, w = self.cfg, self.w
-        rows = [w[n] for n in ("word_emb", "pos_emb", "type_emb", "emb_ln_g", "emb_ln_b")]
-        if N.use_native(rows[0]) and self.H in (256, 512, 768, 1024) and \
-                all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.shape[-1] == self.H for t in rows):
+        c, w, rows = self.cfg, self.w, self._embed_rows()
+        if rows is not None:
             x = torch.empty((ids.numel(), self.H), dtype=torch.bfloat16, device=ids.device)
             word, position, kind, g, b = rows
             N.call("penny_encoder_embed", N.ptr(ids), N.ptr(pos), N.ptr(word), word.shape[0], N.ptr(position),
@@ -118,10 +125,18 @@ class BertEncoder:
         meta[:T] = np.fromiter((t for x in ids_list for t in x), np.int32, T)
         meta[T:2 * T] = np.arange(T, dtype=np.int64) - np.repeat(cu[:-1], lens)
         meta[2 * T:] = cu
-        ids_t, pos_t, cu_t = torch.from_numpy(meta).to(dev).split([T, T, len(cu)])
         longest = int(lens.max())
-        w = self.w
-        x = self._embed(ids_t, pos_t)
+        w, rows = self.w, self._embed_rows()
+        # a recorded launch would hold this call's ids: a capture meets the copy
+        if 0 < T and len(meta) <= EMBED_ARGS and rows is not None and not torch.cuda.is_current_stream_capturing():
+            word, position, kind, g, b = rows
+            x = torch.empty((T, self.H), dtype=torch.bfloat16, device=dev)
+            cu_t = torch.empty(len(cu), dtype=torch.int32, device=dev)
+            N.call("penny_encoder_embed_host", meta.ctypes.data, len(cu), N.ptr(word), word.shape[0], N.ptr(position), position.shape[0],
+                   N.ptr(kind), N.ptr(g), N.ptr(b), N.ptr(x), T, self.H, float(c.norm_eps), N.ptr(cu_t), N.stream())
+        else:
+            ids_t, pos_t, cu_t = torch.from_numpy(meta).to(dev).split([T, T, len(cu)])
+            x = self._embed(ids_t, pos_t)
         if self._small_batch(x, cu_t, longest):
             return x, cu, cu_t
         scale = 1.0 / math.sqrt(self.D)

@@ -29,6 +29,7 @@ _SIGS = {
     "penny_rmsnorm": [P, P, P, P, c_int, c_int, c_float, c_int, P],
     "penny_rmsnorm_slabs": [P, c_int, P, P, P, c_int, c_int, c_float, c_int, P],
     "penny_encoder_embed": [P, P, P, c_int, P, c_int, P, P, P, P, c_int, c_int, c_float, P],
+    "penny_encoder_embed_host": [P, c_int, P, c_int, P, c_int, P, P, P, P, c_int, c_int, c_float, P, P],
     "penny_encoder_pool": [P, P, c_int, c_int, P, P],
     "penny_encoder_layers": [P, c_int, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, P],
     "penny_gemm_bias_small_split": [P, c_int, P, c_int, P, c_int, P, c_int, c_int, P, c_int, P],

@@ -162,6 +162,24 @@ def test_encoder_embed_edges():
         assert float((y.float() - want.float()).abs().max()) <= 2.0 ** -6      # a rounding to bf16 below 4
 
 
+def test_ids_that_travel_with_the_launch(monkeypatch):
+    """Small batches whose ids are the launch's own arguments against ids copied to the device, bit by bit: the largest that fits and the
+    first that does not (960 ints of ids, positions and bounds), ids outside the table, positions beyond theirs, calls in a row."""
+    from financial_chatbot_llm_amd.models import bert
+    from financial_chatbot_llm_amd.models.configs import ModelConfig
+    cfg = ModelConfig("bert-r", "bert", 300, 256, 2, 4, 4, 64, 512, max_position=160, norm_eps=1e-12, type_vocab_size=2)
+    m = bert.BertEncoder.build(cfg, device="cuda", seed=3)
+    batches = [[[(5 * i + j) % 300 for j in range(n)] for i, n in enumerate(lens)]
+               for lens in ([1], [4], [5, 1, 18], [479], [480], [3] * 137, [3] * 138, [2, 0, 3])]
+    batches += [[[-1, 299, 300, 2]], [[2 ** 31 - 1, 0, 1]]]
+    got = [m.encode(b) for b in batches for _ in range(2)]
+    with pytest.raises(OverflowError):
+        m.encode([[2 ** 31]])
+    monkeypatch.setattr(bert, "EMBED_ARGS", 0)
+    want = [m.encode(b) for b in batches for _ in range(2)]
+    assert all(torch.equal(a.nan_to_num(), b.nan_to_num()) for a, b in zip(got, want))
+
+
 def test_projection_form_follows_its_shape():
     """Shapes of which each form was measured faster."""
     from financial_chatbot_llm_amd.ops.gemm import small_bias_wins as small
