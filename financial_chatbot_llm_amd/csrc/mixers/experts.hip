@@ -12,7 +12,7 @@
 // step j takes K element 4 g + j of both operands).  Accumulation is f32; the unit sees the f32 sums.
 //
 // Three forms, chosen by the rows an expert gets on average (the bucket sizes stay on the device):
-//   tile    128 W rows x 64 or 128 tokens per block (64 x 64 for few in f32), both operands through an LDS ring of two or three stages
+//   tile    128 W rows x 64, 128 or 192 tokens per block (64 x 64 for few in f32), both operands through an LDS ring of two or three stages
 //           filled by LDS-DMA, two or three blocks per CU: bound by the operand reads.  4096 tokens, width 2048, 32 experts of 1024, top 4,
 //           bf16: 300 us for both products (650 TFLOP/s); 31 pairs of library products and the host's wait for the
 //           bucket sizes took 1.3 ms.
@@ -61,6 +61,14 @@ struct ExpertGemm {
   int *pos, *src_out;
   int4* tiles_out;
 };
+
+// Rows of each of the tiles of an expert with c rows but the last, which has the rest: even shares in whole groups of 16, as the tile form's
+// blocks cost what they hold and the longest is waited for (5065 tokens in tiles of 192 351 -> 337 us, 3453 254 -> 249; tiles of 128
+// level); tiles of 256 cost halves
+__device__ __forceinline__ int tile_share(int c, int mt) {
+  const int k = max((c + mt - 1) / mt, 1);
+  return mt == 256 ? mt : ((c + k - 1) / k + 15) / 16 * 16;
+}
 
 // One block: pairs 0 .. P-1 (expert idx[i], identity experts >= E stay out) in a stable order by expert.  Every wave
 // owns a contiguous run of pairs; lanes with equal experts find each other by ballots over the index bits, so no
@@ -120,8 +128,9 @@ __global__ void __launch_bounds__(1024) expert_plan_kernel(const int* __restrict
       }
       const int r0 = rows + sc - c, t0 = nt + st - t;
       if (e < E) base[e] = r0;
+      const int share = tile_share(c, mt);
       for (int k = 0; k < t; ++k)
-        if (t0 + k < ntiles) tiles[t0 + k] = make_int4(e, r0 + k * mt, min(mt, c - k * mt), 0);
+        if (t0 + k < ntiles) tiles[t0 + k] = make_int4(e, r0 + k * share, min(share, c - k * share), 0);
       rows += __shfl(sc, 63, 64);
       nt += __shfl(st, 63, 64);
     }
@@ -204,9 +213,10 @@ __global__ void __launch_bounds__(1024) expert_plan_wide_kernel(const int* __res
   }
   __syncthreads();
   const int row0 = own[0], tile0 = own[1], small0 = own[2], all = own[3], n = total[me];
+  const int share = tile_share(n, mt);
   for (int k = threadIdx.x; k * mt < n; k += 1024) {
     const int at = n - k * mt < mt && begun(n) ? small0 : tile0 + k;
-    if (at < ntiles) tiles[at] = make_int4(me, row0 + k * mt, min(mt, n - k * mt), 0);
+    if (at < ntiles) tiles[at] = make_int4(me, row0 + k * share, min(share, n - k * share), 0);
   }
   if (me == 0)
     for (int t = all + threadIdx.x; t < ntiles; t += 1024) tiles[t] = make_int4(0, 0, 0, 0);
@@ -348,6 +358,7 @@ __global__ void __launch_bounds__(256, 163840 / (ST * (WR * 2048 + MT * 128))) e
                  : "v"(gp), "s"(dst)
                  : "memory");
   };
+  const int ns = a.kt / 2;
   auto stage = [&](int s) {
     const unsigned buf = lds0 + (s % ST) * STG;
 #pragma unroll
@@ -364,7 +375,6 @@ __global__ void __launch_bounds__(256, 163840 / (ST * (WR * 2048 + MT * 128))) e
   for (int f = 0; f < FW; ++f)
 #pragma unroll
     for (int u = 0; u < U; ++u) acc[f][u] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int ns = a.kt / 2;
 #pragma unroll
   for (int s = 0; s < ST - 1; ++s)
     if (s < ns) stage(s);
@@ -395,8 +405,10 @@ __global__ void __launch_bounds__(256, 163840 / (ST * (WR * 2048 + MT * 128))) e
     }
   };
   const int mine = (live - wb + WB - 1) / WB;   // (a wave of the second half may have none: it multiplies one that is not stored)
-  if (U == 4 && mine >= 4) walk(Steps<U>{});
-  else if (U == 4 && mine == 3) walk(Steps<U < 3 ? U : 3>{});
+  if (U == 6 && mine >= 6) walk(Steps<U>{});
+  else if (U == 6 && mine == 5) walk(Steps<U < 5 ? U : 5>{});
+  else if (U >= 4 && mine >= 4) walk(Steps<U < 4 ? U : 4>{});
+  else if (U >= 4 && mine == 3) walk(Steps<U < 3 ? U : 3>{});
   else if (mine >= 2) walk(Steps<2>{});
   else walk(Steps<1>{});
 #pragma unroll
@@ -747,8 +759,8 @@ __global__ void __launch_bounds__(NW * 64) expert_stream_kernel(ExpertGemm a) {
 // tiles of 16 / 64: 32 rows on average 58 / 132, f32 126 / 569, 96 rows 120 / 122; 8 of 8192 x 2048: 24 rows 165 / 238, 48 rows
 // 274 / 245; 2 of 4096 x 1024: 64 rows 32 / 87; 16 of 768 x 2048: 24 rows 35 / 48, 48 rows 56 / 50.
 //
-// Among the larger tiles the choice is by an estimate too: the rounds of blocks over the CUs (3, 2 and 1 blocks of 64, 128 and 256
-// rows on each) times a block's stages at 1.35 (1.15 where the CUs are not full), 1.38 and 1.85 us; an expert's last tile is half
+// Among the larger tiles the choice is by an estimate too: the rounds of blocks over the CUs (3, 2, 2 and 1 blocks of 64, 128, 192 and 256
+// rows on each) times a block's stages at 1.35 (1.15 where the CUs are not full), 1.38, 1.84 and 1.85 us; an expert's last tile is half
 // full on average, and a small one of 256 rows takes half the time.  Us for tiles of 64 / 128 / 256, bf16, experts' rows spread by a
 // factor of about 1.3 (5 for the second figures): 32 experts of 1024 x 2048: 64 rows on average 102 / 100 / 95 (96 / 127 / 117), 128:
 // 129 / 138 / 114 (132 / 139 / 142),
@@ -766,9 +778,9 @@ double wide_time(double avg, int experts, int mt, const Product* p) {
   for (int i = 0; i < 2; ++i) {
     const int cols = mt == 256 ? (p[i].groups + 15) / 16 : (p[i].groups + 7) / 8;
     double r = mt == 256 ? experts * (avg / 256 + 0.25) * cols / 256 + 0.2
-                         : experts * (avg / mt + 0.5) * cols / (mt == 128 ? 512 : 768);
+                         : experts * (avg / mt + 0.5) * cols / (mt == 64 ? 768 : 512);
     if (r < 3) r = floor(r) + fmin(1.0, 2 * (r - floor(r)));      // the last of a few rounds leaves CUs idle
-    us += fmax(r, 1.0) * (p[i].kt / 2 * (mt == 256 ? 1.85 : mt == 128 ? 1.38 : r < 1 ? 1.15 : 1.35) + (mt == 256 ? 5 : 0));
+    us += fmax(r, 1.0) * (p[i].kt / 2 * (mt == 256 ? 1.85 : mt == 192 ? 1.84 : mt == 128 ? 1.38 : r < 1 ? 1.15 : 1.35) + (mt == 256 ? 5 : 0));
   }
   return us;
 }
@@ -791,6 +803,14 @@ int tile_rows(long pairs, int experts, int dt, const Product* p, bool whole) {
   // 64 where it is clearly the shorter, and while most experts' only tile is less than half of one of 128: uneven buckets then pay for
   // the wider (plan and products, 200 and 300 tokens most of which go to an eighth of the experts: 64 of 512 x 1024, top 6, 128 rows 66 and 71 us,
   // 64 rows 47 and 51; 32 of 1024 x 2048, top 4, 120 and 126, 94 and 97; evenly spread 43 - 45 and 42, 91 - 92 and 86)
+  // 192 takes a sixth less of the operands' way to LDS per row than 128, but its rounds are longer, and an expert with more rows than a tile starts
+  // another of them: far beyond the 136 rows from which most experts fill more than one of 128 it has to be little worse by the
+  // estimate, which is 5 - 10 % too low for two or three rounds of 128, else clearly better.  Us, 128 / 192 (even and spread buckets): 32 experts of 1024 x
+  // 2048, 148 rows 142 / 145 (139 / 149), 192: 180 / 164 (180 / 164), 256: 190 / 175 (187 / 173), 338: 240 / 220 (234 / 216), 431: 265 / 250 (280 /
+  // 252); of 512 x 1024, 256: 75 / 63, 432: 88 / 99, 633: 125 / 118; 64 of 768 x 2048, 141: 209 / 196 (201 / 187), 375: 372 / 340 (381 / 358);
+  // 8 of 2048 x 4096, 150: 133 / 156, 250: 218 / 157 (211 / 157).
+  const double t192 = wide_time((double)pairs / experts, experts, 192, p);
+  if (avg >= 136 && t192 < (avg >= 176 ? 1.07 : 0.92) * fmin(t64, t128)) return 192;
   return avg <= 56 || t64 < 0.95 * t128 ? 64 : 128;
 }
 
@@ -804,7 +824,8 @@ int expert_launch(const ExpertGemm& a, int mt, hipStream_t st) {
     const long grid = (long)a.ntiles * ((a.groups + 7) / 8);
     if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
     if constexpr (sizeof(T) == 2) {
-      if (mt == 128) expert_tile_kernel<T, 128, 8, 2, GLU><<<(unsigned)grid, 256, 0, st>>>(a);
+      if (mt == 192) expert_tile_kernel<T, 192, 8, 2, GLU><<<(unsigned)grid, 256, 0, st>>>(a);
+      else if (mt == 128) expert_tile_kernel<T, 128, 8, 2, GLU><<<(unsigned)grid, 256, 0, st>>>(a);
       else expert_tile_kernel<T, 64, 8, 2, GLU><<<(unsigned)grid, 256, 0, st>>>(a);
     } else if (grid <= 768) {
       // f32 blocks that all lie on the chip at once: whichever CU got one more takes a block's whole time longer, so halves of them (above)

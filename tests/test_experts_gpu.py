@@ -125,6 +125,14 @@ def test_few_experts(dtype, T, W, F_, E, top, unit):
     check(dtype, T, W, F_, E, top, unit)
 
 
+@pytest.mark.parametrize("T,skew", [(2048, False), (1905, True)])
+def test_tiles_of_192(T, skew):
+    """Even shares of an expert's rows in one and two tiles of 192, and of thousands of rows beside experts of a few."""
+    from financial_chatbot_llm_amd.ops import _native as N
+    assert N.load_mixers().mx_experts_tile(T * 4, 32, 0, 64, 32, 64, 16, 1) == 192
+    check(torch.bfloat16, T, 1024, 512, 32, 4, "clamped", skew=skew)
+
+
 def test_tile_rule():
     """Few rows per expert on average keep tiles of 64 whatever the estimate says of even buckets."""
     from financial_chatbot_llm_amd.ops import _native as N
