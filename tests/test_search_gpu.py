@@ -117,3 +117,26 @@ def test_workspaces(monkeypatch):
     for t in threads:
         t.join()
     assert not errors and len(retrieval._FREE) <= 8
+
+
+def test_calls_in_a_row():
+    """The host goes on when it knows the counts: calls behind one another, whose lists, counters and told counts are one set, with
+    rows ranked alone, by several blocks, by sorting and on the host's side."""
+    sizes = [90, 200, 1500, 9000, 0, 3]
+    x, users, dates, q = corpus(sizes, 14000, 64, 11)
+    rows = [t.cuda() for t in (x, users, dates)]
+    calls = []
+    for i in range(24):
+        pick = [(i + j) % 6 for j in range(1 + i % 5)]
+        if i % 3:                                                          # most calls without a wait of their own
+            pick = [u for u in pick if u != 3] or [0]
+        who = torch.tensor([u + 1 for u in pick], dtype=torch.int32)
+        floor, ks = torch.full((len(pick),), 13 * i), torch.full((len(pick),), 40 + i, dtype=torch.int32)
+        calls.append((q[pick], who, floor, ks, [u != 3 for u in pick]))
+    dev = [[t.cuda() for t in c[:4]] for c in calls]
+    torch.cuda.synchronize()
+    got = [ops.filtered_topk(*rows, *c, 64) for c in dev]
+    for c, (ids, scores, counts) in zip(calls, got):
+        want = ops.filtered_topk(x, users, dates, *c[:4], 64)
+        assert torch.equal(counts.cpu(), want[2]) and torch.equal(scores.cpu(), want[1])
+        assert torch.equal(ids.cpu()[c[4]], want[0][c[4]])
