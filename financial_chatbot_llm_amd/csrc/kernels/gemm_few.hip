@@ -20,7 +20,7 @@ constexpr int FEW_ROWS = 4;              // tokens at most
 constexpr int FEW_CHUNKS = 7168;         // 16-byte chunks of the rows at most: 4 x 14336, 3 x 18944, 2 x 28672, 1 x 57344 values in 112 KiB
 constexpr int FEW_PAD = 64;              // bytes behind a token's row in LDS: four tokens at one k meet different banks
 
-enum { FEW_SLAB = 0, FEW_ADD = 1, FEW_SILU = 2, FEW_ROPE = 3, FEW_ROWS_OUT = 4 };
+enum { FEW_SLAB = 0, FEW_ADD = 1, FEW_SILU = 2, FEW_ROPE = 3 };
 
 struct FewRows {
   const bf16* x;                         // [M, K], row stride ldx
@@ -216,10 +216,7 @@ __global__ void __launch_bounds__(NW * 64) few_rows_kernel(FewRows a) {
   } else {
     bf16x4* y = reinterpret_cast<bf16x4*>(static_cast<bf16*>(a.y) + col * a.ldy + n);
     bf16x4 o;
-    if constexpr (EPI == FEW_ROWS_OUT) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = (bf16)sum[0][i];
-    } else if constexpr (EPI == FEW_ADD) {
+    if constexpr (EPI == FEW_ADD) {
       const bf16x4 r = *y;
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[i] = (bf16)((float)(bf16)sum[0][i] + (float)r[i]);   // as rmsnorm_kernel with slabs
@@ -238,13 +235,11 @@ __global__ void __launch_bounds__(NW * 64) few_rows_kernel(FewRows a) {
 // waves x 16 pieces 39.6 (40.3), 8 x 8 39.5 (40.6), 4 x 16 40.9 (40.2), 16 x 8 41.0 (45.7); QKV of 6144 x 4096: 8 x 12 10.4 (12.5), 8 x 16
 // 11.3 (12.8), 4 x 16 11.2 (11.5); the adding form, 4096 x 14336: 16 x 8 20.4 (20.9), 8 x 24 21.0 (22.2), 4096 x 4096: 7.7 (8.4) and 9.1
 // (9.8); QKV with its rotation and cache write behind it 16 x 8 10.7 (12.7), 16 x 12 11.3 (13.0), 8 x 16 13.8 (14.9), as two launches 13.2 (15.5).
-// With loads that stay in the caches these were 42.3, 11.0, 22.8 and 8.5.  Plain rows, 128256 x 4096: 16 x 8 152 (152; 7 TB/s), 16 x 4 151
-// (154), 8 x 8 158 (158), the library 183 (182); 32000 x 4096 41.5 (42.4), the library 60.
+// With loads that stay in the caches these were 42.3, 11.0, 22.8 and 8.5.
 template <int EPI, bool NORM>
 int launch_few(const FewRows& a, hipStream_t st) {
   const dim3 grid(a.N / (EPI == FEW_SILU || EPI == FEW_ROPE ? 32 : 16));
-  constexpr int NW = EPI == FEW_SILU || EPI == FEW_SLAB ? 8 : 16;
-  constexpr int D = EPI == FEW_SILU ? 16 : EPI == FEW_SLAB ? 12 : 8;
+  constexpr int NW = EPI == FEW_ADD || EPI == FEW_ROPE ? 16 : 8, D = EPI == FEW_SILU ? 16 : EPI == FEW_SLAB ? 12 : 8;
   if (a.M * (a.K / 8) <= 2048) few_rows_kernel<EPI, NORM, 2048, NW, D><<<grid, NW * 64, 0, st>>>(a);
   else if constexpr (!NORM) few_rows_kernel<EPI, NORM, FEW_CHUNKS, NW, D><<<grid, NW * 64, 0, st>>>(a);
   return (int)hipGetLastError();
@@ -253,19 +248,18 @@ int launch_few(const FewRows& a, hipStream_t st) {
 }  // namespace
 
 // y = [norm of] X [M, K] x W [N, K]^T, W as tile_weight's copy.  form 0: norm, f32 [M, N]; 1: added to the bf16 rows of y in place;
-// 2: norm, W is the interleave16 gate|up weight, y bf16 [M, N / 2] = SiLU(gate) * up; 4: the rows as they are, bf16 [M, N].
+// 2: norm, W is the interleave16 gate|up weight, y bf16 [M, N / 2] = SiLU(gate) * up.
 // Contract (checked): 1 <= M <= 4, N % 16 == 0 (form 2: 32), K % 512 == 0, M * K <= 8 * FEW_CHUNKS; with a norm
 // K <= 4096; ldx % 8 == 0, ldy % 4 == 0; x, norm, W and f32 y in whole 16 bytes, bf16 y in 8.
 PENNY_API int penny_few_rows(const void* X, int ldx, const void* norm, float eps, const void* Wt, int K, int N, void* y, int ldy,
                              int M, int form, hipStream_t stream) {
   if (M <= 0) return 0;
-  if (M > FEW_ROWS || N <= 0 || K <= 0 || N % (form == FEW_SILU ? 32 : 16) || K % 512 || ldx % 8 || ldy % 4 || form < 0 ||
-      form > FEW_ROWS_OUT || form == FEW_ROPE || (long)M * K > 8 * FEW_CHUNKS || (form == FEW_ADD || form == FEW_ROWS_OUT ? norm != nullptr : !norm || K > 4096) ||
+  if (M > FEW_ROWS || N <= 0 || K <= 0 || N % (form == FEW_SILU ? 32 : 16) || K % 512 || ldx % 8 || ldy % 4 || form < 0 || form > 2 ||
+      (long)M * K > 8 * FEW_CHUNKS || (form == FEW_ADD ? norm != nullptr : !norm || K > 4096) ||
       ((size_t)X | (size_t)norm | (size_t)Wt) % 16 || !X || !Wt || !y || (size_t)y % (form == FEW_SLAB ? 16 : 8))
     return (int)hipErrorInvalidValue;
   const FewRows a{(const bf16*)X, (const bf16*)norm, (const char*)Wt, y, ldx, ldy, M, N, K, eps};
-  return form == FEW_SLAB ? launch_few<FEW_SLAB, true>(a, stream) : form == FEW_ADD ? launch_few<FEW_ADD, false>(a, stream) :
-         form == FEW_ROWS_OUT ? launch_few<FEW_ROWS_OUT, false>(a, stream) : launch_few<FEW_SILU, true>(a, stream);
+  return form == FEW_SLAB ? launch_few<FEW_SLAB, true>(a, stream) : form == FEW_ADD ? launch_few<FEW_ADD, false>(a, stream) : launch_few<FEW_SILU, true>(a, stream);
 }
 
 // QKV [norm of] X [M, K] x W^T of heads of 128 with the rotation and the paged cache's write behind it (rope_kv.hip): q [M, Hq, 128] bf16,

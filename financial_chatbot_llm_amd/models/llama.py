@@ -38,7 +38,7 @@ def _dual_stream(device) -> "torch.cuda.Stream":
         _DUAL_STREAMS[key] = torch.cuda.Stream(device=device)
     return _DUAL_STREAMS[key]
 from ..ops.gemm import (few_ok, few_qkv_rope, few_rows, interleave16, linear, linear_tiled, prefill_qkv_rope, qkv_rope_fused, tile_weight,
-                        tiled_only, uses_tiled_weight, vocab_rows)
+                        tiled_only, uses_tiled_weight)
 from ..parallel.layers import shard_cols, shard_rows, shard_sections, vocab_range
 from .common import AttentionMetadata, KVCache, random_tensor
 from .configs import ModelConfig
@@ -513,7 +513,7 @@ class DecoderModel:
         return self.w["embed"] if self.cfg.tie_embeddings else self.w["lm_head"]
 
     def logits(self, h: torch.Tensor) -> torch.Tensor:
-        out = vocab_rows(h, self.lm_weight(), self.lm_tiled())
+        out = linear(h, self.lm_weight())
         return comm.tp_all_gather_last(out) if self.tp_size > 1 else out
 
     def sample_vocab_parallel(self, h: torch.Tensor, temps: torch.Tensor, seeds: torch.Tensor) -> torch.Tensor:
@@ -527,7 +527,7 @@ class DecoderModel:
         if pad is not None and ops.fused_lm_head_ok(h, pad):
             pairs = ops.lm_head_sample_shard(h, pad, w.shape[0], self.vocab_start, temps, seeds, wt=self.lm_tiled())
         else:
-            pairs = ops.sample_shard(vocab_rows(h, w, self.lm_tiled()), temps, seeds, self.vocab_start, self.cfg.vocab_size)
+            pairs = ops.sample_shard(linear(h, w), temps, seeds, self.vocab_start, self.cfg.vocab_size)
         return ops.pick_pairs(comm.tp_all_gather_pairs(pairs))
 
 

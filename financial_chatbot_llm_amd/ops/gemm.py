@@ -359,7 +359,7 @@ def ring_slabs(x: torch.Tensor, w: torch.Tensor, S: int, tile: int) -> torch.Ten
     return P
 
 
-FEW_FORMS = {"slab": 0, "add": 1, "silu": 2, "rows": 4}
+FEW_FORMS = {"slab": 0, "add": 1, "silu": 2}
 
 
 def few_ok(M: int, wt: Optional[torch.Tensor], norm: bool) -> bool:
@@ -391,14 +391,14 @@ def few_rows(x: torch.Tensor, wt: torch.Tensor, form: str, norm: Optional[torch.
              residual: Optional[torch.Tensor] = None) -> Union[torch.Tensor, "Slabs"]:
     """One to four rows through a ``tile_weight`` copy in one launch (``penny_few_rows``).  "slab": RMS-normed with ``norm`` first, f32 sums
     as one slab; "add": added to ``residual`` in place; "silu": normed, ``wt`` the interleave16 gate|up weight and the result
-    SiLU(gate) * up; "rows": the product in bf16."""
+    SiLU(gate) * up."""
     x, norm = _few_operands(x, wt, norm)
     M, K = x.shape
     N_ = wt.shape[0] * 16
     if form == "slab":
         y = torch.empty((1, M, N_), dtype=torch.float32, device=x.device)
-    elif form in ("silu", "rows"):
-        y = torch.empty((M, N_ // 2 if form == "silu" else N_), dtype=x.dtype, device=x.device)
+    elif form == "silu":
+        y = torch.empty((M, N_ // 2), dtype=x.dtype, device=x.device)
     else:
         y = residual
         if y is None or y.dtype != x.dtype or y.shape != (M, N_) or y.stride(1) != 1:
@@ -406,26 +406,6 @@ def few_rows(x: torch.Tensor, wt: torch.Tensor, form: str, norm: Optional[torch.
     N.call("penny_few_rows", N.ptr(x), x.stride(0), N.ptr(norm), float(eps), N.ptr(wt), K, N_, N.ptr(y), y.stride(-2), M, FEW_FORMS[form],
            N.stream())
     return Slabs(y) if form == "slab" else y
-
-
-def vocab_rows(x: torch.Tensor, w: torch.Tensor, wt: Optional[torch.Tensor]) -> torch.Tensor:
-    """``x @ w.T`` in bf16 of a vocabulary projection, on its ``tile_weight`` copy ``wt`` where that is the faster one.
-
-    us (weights beyond the caches; the library's product of ``w``): 128256 x 4096, 1 / 4 rows 152 / 152 (183 / 182) by ``few_rows``, 16 / 32 /
-    64 / 128 rows 177 / 184 / 203 / 224 (188 / 197 / 210 / 234) by the split-K kernel without a split, 192 rows 268 (255); 32000 x 4096, 1 /
-    16 / 48 / 128 rows 42 / 49 / 50 / 56 (60 / 61 / 66 / 64), 192 rows 71 (70).  Narrower projections have too few tiles for the chip."""
-    M, K = x.shape
-    N_ = w.shape[0]
-    if wt is None or not 1 <= M <= 128 or N_ < 24576 or N_ % 128 or K % 64 or wt.shape[0] * 16 != N_ or not N.use_native(x) or x.dtype != torch.bfloat16 \
-            or wt.dtype != torch.bfloat16 or os.environ.get("PENNY_SPLITK", "1") == "0" \
-            or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
-        return linear(x, w)
-    if few_ok(M, wt, False):
-        return few_rows(x, wt, "rows")
-    x, _ = _few_operands(x, wt, None)
-    y = torch.empty((M, N_), dtype=x.dtype, device=x.device)
-    N.call("penny_splitk_gemm_bf16", N.ptr(x), x.stride(0), N.ptr(wt), K, N.ptr(y), N_, M, N_, 4 if M <= 32 else 8, 2, N.stream())
-    return y
 
 
 def few_qkv_rope(x: torch.Tensor, wt: torch.Tensor, norm: torch.Tensor, eps: float, positions: torch.Tensor, cos_sin: torch.Tensor,

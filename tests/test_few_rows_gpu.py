@@ -181,15 +181,3 @@ def test_decoder_step_of_prompts(D, prompts, rows, monkeypatch):
     for a, b in zip(*outs):
         # both round the same values to eight bits in a different order of f32 sums: at most a unit per layer of the largest
         assert (a - b).abs().max() <= 4 * 2.0 ** -8 * b.abs().max()
-
-
-@pytest.mark.parametrize("M", [1, 2, 4, 5, 16, 17, 32, 33, 64, 65, 127, 128, 129])
-@pytest.mark.parametrize("V,K", [(24576, 512), (24704, 576), (32000, 2048)])
-def test_vocabulary_rows(M, V, K):
-    g = torch.Generator().manual_seed(M)
-    x = torch.randn(M, K + 8, generator=g).to(torch.bfloat16).cuda()[:, :K]
-    w = (torch.randn(V, K, generator=g) * K ** -0.5).to(torch.bfloat16).cuda()
-    y = G.vocab_rows(x, w, G.tile_weight(w))
-    ref, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
-    assert y.shape == (M, V) and bool(((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + K * 2.0 ** -24 * size).all())
-    assert torch.equal(G.vocab_rows(x, w, None), G.linear(x, w))
