@@ -65,8 +65,7 @@ def _as(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
 def filtered_topk(corpus: torch.Tensor, user_codes: torch.Tensor, dates: torch.Tensor, queries: torch.Tensor,
                   q_user: torch.Tensor, q_floor: torch.Tensor, ks: torch.Tensor, kmax: int,
                   cap: int = 65536) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    """-> (row ids [nq,kmax] int32, scores [nq,kmax] f32, counts [nq] int32), best first; written, like any operation's results, when
-    the current stream comes to them."""
+    """-> (row ids [nq,kmax] int32, scores [nq,kmax] f32, counts [nq] int32), best first."""
     nq, D = queries.shape
     if not N.use_native(corpus):
         return filtered_topk_ref(corpus, user_codes, dates, queries, q_user.tolist(), q_floor.tolist(),
@@ -92,7 +91,7 @@ def filtered_topk(corpus: torch.Tensor, user_codes: torch.Tensor, dates: torch.T
     out_count = torch.empty((nq,), dtype=torch.int32, device=dev)
     N.call("penny_topk_rank", corpus.data_ptr(), D, queries.data_ptr(), kk.data_ptr(), nq, kmax, cp, cand.data_ptr(), scores.data_ptr(),
            cap, out_ids.data_ptr(), out_scores.data_ptr(), out_count.data_ptr(), oc.data_ptr(), stream)
-    for i, c in enumerate(oc[:nq].tolist()):  # the call has waited for these; > SORT_CAP candidates: finish on device with torch.topk
+    for i, c in enumerate(oc[:nq].tolist()):  # the call has waited for them; > SORT_CAP candidates: finish on device with torch.topk
         if c >= 0:
             continue
         total = -c

@@ -120,8 +120,8 @@ def test_workspaces(monkeypatch):
 
 
 def test_calls_in_a_row():
-    """The host goes on when it knows the counts: calls behind one another, whose lists, counters and told counts are one set, with
-    rows ranked alone, by several blocks, by sorting and on the host's side."""
+    """Calls behind one another, whose lists, counters and counts for the host are one set, with rows ranked alone, by several blocks, by
+    sorting and on the host's side."""
     sizes = [90, 200, 1500, 9000, 0, 3]
     x, users, dates, q = corpus(sizes, 14000, 64, 11)
     rows = [t.cuda() for t in (x, users, dates)]
@@ -140,3 +140,27 @@ def test_calls_in_a_row():
         want = ops.filtered_topk(x, users, dates, *c[:4], 64)
         assert torch.equal(counts.cpu(), want[2]) and torch.equal(scores.cpu(), want[1])
         assert torch.equal(ids.cpu()[c[4]], want[0][c[4]])
+
+
+@pytest.mark.parametrize("before", [0, 40])
+def test_results_are_complete_on_return(before):
+    """Nothing of a call is left on its stream when it returns, also behind a few milliseconds of other work: another stream may read its
+    results at once."""
+    sizes = [4000] * 16 + [90, 0, 200]
+    x, users, dates, q = corpus(sizes, sum(sizes) + 50, 256, 5)
+    nq, other, own = len(sizes), torch.cuda.Stream(), torch.cuda.Stream()
+    who, floor, ks = torch.arange(1, nq + 1, dtype=torch.int32), torch.zeros(nq, dtype=torch.int64), torch.full((nq,), 300, dtype=torch.int32)
+    dev = [t.cuda() for t in (x, users, dates, q[:nq], who, floor, ks)]
+    want = ops.filtered_topk(x, users, dates, q[:nq], who, floor, ks, 300)
+    busy = torch.randn((4096, 4096), device="cuda")
+    torch.cuda.synchronize()
+    for _ in range(3):
+        with torch.cuda.stream(own):
+            for _ in range(before):
+                busy @ busy
+            got = ops.filtered_topk(*dev, 300)
+            assert own.query()
+        with torch.cuda.stream(other):
+            for g, w in zip(got, want):
+                assert torch.equal(g.cpu(), w)
+        torch.cuda.synchronize()
