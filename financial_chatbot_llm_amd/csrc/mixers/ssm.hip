@@ -158,11 +158,46 @@ __device__ __forceinline__ float row_sum16(float v) {
   return v;
 }
 
+// The sum over 64 entries of the state, four in each of 16 lanes, in the order of a lane of the scan below, which owns 4 NJ entries side by side:
+// a run of NJ lanes passes its two partial sums on, then the runs meet as row_sum16 adds the scan's lanes.
+template <int NJ>
+__device__ __forceinline__ float run_sum(mx_f32x4 s, mx_f32x4 c, int ns) {
+  float even = 0.f, odd = 0.f;
+  const auto chain = [&] {
+    even = fmaf(s[2], c[2], fmaf(s[0], c[0], even));
+    odd = fmaf(s[3], c[3], fmaf(s[1], c[1], odd));
+  };
+  const auto from = [](float v, auto ctrl) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), decltype(ctrl)::value, 0xF, 0xF, true));
+  };
+  chain();
+#pragma unroll
+  for (int hop = 1; hop < NJ; ++hop) {         // quad_perm [3,0,1,2]: the lane before
+    even = from(even, std::integral_constant<int, 0x93>{});
+    odd = from(odd, std::integral_constant<int, 0x93>{});
+    if (ns % NJ == 0) even = odd = 0.f;
+    chain();
+  }
+  float v = even + odd;
+  if (NJ == 1) return row_sum16(v);
+  if (NJ == 2) {                               // each pair's second lane has it: quad_perm [1,1,3,3], then pairs, eights, the row
+    v = from(v, std::integral_constant<int, 0xF5>{});
+    v += from(v, std::integral_constant<int, 0x4E>{});
+  } else {
+    v = from(v, std::integral_constant<int, 0xFF>{});
+  }
+  v += from(v, std::integral_constant<int, 0x141>{});
+  return v + from(v, std::integral_constant<int, 0x140>{});
+}
+
 // A step of single rows (decode): a block takes a head, its threads 16 of the value channels at a time with 16 lanes by fours along
 // the state's NJ 64s, up to 64 channels' states asked for at once; B and C, the same for all of them, stay in registers.  Bound by the
 // state's bytes, which do not stay in the caches on either way: 64 rows of 64 heads of 64 x 128 46 us (5.8 TB/s; 48 where they stay, and
 // the step's other launches longer: 8 layers 1157 / 1117, 17 rows 504 / 480), by the scan below, whose chunk of staged rows leaves room for three blocks a
-// CU, 62; 17 rows of 32 heads 9.6, 13.4.
+// CU, 62; 17 rows of 32 heads 9.6, 13.4.  Every product, sum and rounding is that of the scan's single token, so that a row's results do not
+// depend on which of the two its step takes: the lanes' passing on is free beside the bytes (44.2 us added up as the lanes lie, 44.4 so), and
+// added up as they lie, values and states of 64 entries were 5 and 9 % further from 64 bits than the scan's.  (Entries side by side in a lane,
+// as the scan reads them, break the loads past the caches into halves of lines: 69 us.)
 template <typename TD, int NJ>
 __global__ void __launch_bounds__(256)
 ssm_step_kernel(const float* __restrict__ u, int C, const TD* __restrict__ dt_raw, long sdt, const float* __restrict__ dt_bias,
@@ -199,15 +234,16 @@ ssm_step_kernel(const float* __restrict__ u, int C, const TD* __restrict__ dt_ra
     for (int i = 0; i < PU; ++i) {
       const int p = p0 + 16 * i + pl;
       const float dx = dt * x[i];
-      mx_f32x4 acc = mx_f32x4{0.f, 0.f, 0.f, 0.f};
+      float part[NJ];
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        S[i][j] = a * S[i][j] + dx * B[j];
-        acc += S[i][j] * Cv[j];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[i][j][e] = NJ == 1 ? fmaf(a, S[i][j][e], dx * B[j][e]) : fmaf(dx, B[j][e], a * S[i][j][e]);
         if (p < P) stf4_once(sh + (long)p * N + 64 * j, S[i][j]);
+        part[j] = run_sum<NJ>(S[i][j], Cv[j], ns);
       }
-      const float o = row_sum16((acc[0] + acc[1]) + (acc[2] + acc[3]));
-      if (ns == 0 && p < P) y[t * inner + h * P + p] = o + Dh * x[i];
+      const float o = NJ == 4 ? (part[0] + part[1 % NJ]) + (part[2 % NJ] + part[3 % NJ]) : NJ == 2 ? part[0] + part[1 % NJ] : part[0];
+      if (ns == 0 && p < P) y[t * inner + h * P + p] = fmaf(Dh, x[i], o);
     }
   }
 }

@@ -67,3 +67,20 @@ def test_state_space(dt, N, P, G):
     near(ds, cs, 4)
     for s in (2, 4):
         assert torch.equal(ds[s].cpu(), state[s])
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,P,G", [(64, 5, 1), (64, 64, 2), (128, 50, 2), (128, 64, 1), (256, 16, 2), (256, 70, 1)])
+def test_state_space_step_is_the_scan(dt, N, P, G):
+    """Single rows have the bits of the scan's single tokens, which a step that may hold longer segments takes."""
+    g = torch.Generator().manual_seed(N + P)
+    rnd = lambda *s: torch.randn(s, generator=g)  # noqa: E731
+    H = 4
+    u, dtr = rnd(S, H * P + 2 * G * N), rnd(S, H).to(dt)
+    u[0, 3], u[4, H * P + 5] = float("inf"), float("nan")
+    args = cuda(u, dtr, rnd(H), rnd(H), rnd(H))
+    state = rnd(6, H, P, N)
+    a, b = state.cuda(), state.cuda()
+    ya = mx.ssm_scan(*args, a, *cuda(CU, SLOT, POS), H, P, N, G, 1)
+    yb = mx.ssm_scan(*args, b, *cuda(CU, SLOT, POS), H, P, N, G, 2)
+    assert torch.allclose(ya[LIVE], yb[LIVE], rtol=0, atol=0, equal_nan=True) and torch.allclose(a, b, rtol=0, atol=0, equal_nan=True)
