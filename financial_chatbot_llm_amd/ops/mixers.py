@@ -1064,9 +1064,10 @@ def matrix_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.Tens
 def low_rank(ua: torch.Tensor, wa: torch.Tensor, ug: Optional[torch.Tensor] = None,
              wg: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
     """The second factors of two low-rank projections: ``ua wa^T`` in f32 (``ua`` [T, ra] bf16 or f32, ``wa`` f32) and, given, ``ug wg^T`` in
-    the type of ``ug``.  One launch for ranks of 32 and 64 (``mx_low_rank``), else a product each."""
+    the type of ``ug``.  One launch for ranks of 32 and 64 (``mx_low_rank``), else, and under autocast or for gradients, a product each."""
     (T, ra), na = ua.shape, wa.shape[0]
-    if N.use_native(ua) and T > 0 and ra in (32, 64) and na % 16 == 0 and wa.dtype == torch.float32 and wa.shape[1] == ra and wa.is_contiguous() and \
+    plain = not torch.is_autocast_enabled() and not any(t is not None and t.requires_grad for t in (ua, wa, ug, wg))
+    if plain and N.use_native(ua) and T > 0 and ra in (32, 64) and na % 16 == 0 and wa.dtype == torch.float32 and wa.shape[1] == ra and wa.is_contiguous() and \
             ua.dtype in (torch.bfloat16, torch.float32) and ua.stride(1) == 1 and ua.stride(0) * ua.element_size() % 16 == 0 and ua.stride(0) >= ra and \
             (ua.data_ptr() | wa.data_ptr()) % 16 == 0 and T <= 1 << 23:
         ng = 0 if ug is None else wg.shape[0]

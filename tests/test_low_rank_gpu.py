@@ -59,3 +59,25 @@ def test_other_layouts_keep_the_products(dt, ra, na, rg, ng, pad):
     ua, wa, ug, wg = operands(dt, 20, ra, na, rg, ng, pad)
     a, g = mx.low_rank(ua, wa, ug, wg)
     check(a, g, ua, wa, ug, wg, dt)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_autocast_and_gradients(dt):
+    """As the two products: autocast's type, and gradients for rows and weights."""
+    ua, wa, ug, wg = operands(dt, 20, 64, 64, 32, 80)
+    with torch.autocast("cuda", dtype=torch.float16):
+        a, g = mx.low_rank(ua, wa, ug, wg)
+        want = torch.nn.functional.linear(ua.float(), wa), torch.nn.functional.linear(ug, wg)
+    assert a.dtype == g.dtype == torch.float16 and torch.equal(a, want[0]) and torch.equal(g, want[1])
+    for i in range(4):
+        ts = [t.detach().clone() for t in (ua, wa, ug, wg)]
+        ts[i].requires_grad_()
+        a, g = mx.low_rank(*ts)
+        (a if i < 2 else g).sum().backward()
+        u, w = ts[:2] if i < 2 else ts[2:]
+        want = (w if i % 2 == 0 else u).double().sum(0)
+        # sums of at most 80 products with ones: f32, and in bf16 the result rounded to eight significant bits
+        e = 2.0 ** -8 if ts[i].dtype == torch.bfloat16 else 0.0
+        size = (w if i % 2 == 0 else u).double().abs().sum(0)
+        assert ((ts[i].grad.double() - want).abs() <= e * want.abs() + 80 * 2.0 ** -24 * size).all()
+    assert not any(t.requires_grad for t in mx.low_rank(ua, wa, ug, wg))
