@@ -469,7 +469,7 @@ MX_API int mx_latent_attend(const void* q_lat, const void* q_rot, const void* ca
                             int window, float scale, void* out, int dt, int S, int max_len, int H, int R, int Dr,
                             int nsplit, float* ws, int rows, hipStream_t st) {
   if (S <= 0 || max_len <= 0) return 0;
-  if (R > 64 * ATT_RPL || nsplit > 64) return (int)hipErrorInvalidValue;
+  if (R > 64 * ATT_RPL) return (int)hipErrorInvalidValue;
   const int D = R + Dr;
   // rows_attend.h for the latent of 256 with a rotated part of 32 or none, the sizes of this framework's decoders (window 1024,
   // before -> after; 32 heads, bf16: 2048 rows of three segments 217 -> 64 us, 256 rows and 30 single ones 405 -> 75, 64 single

@@ -259,8 +259,8 @@ inline int mx_tile_count(int S, int rows, int max_len, int tile, int slack = 0) 
 constexpr int PAGE_ROWS = 64;            // tokens per cache page
 
 // The parts that several blocks left of one (row, head)'s attention, ws [rows, H, nsplit, P + 2]: unnormalised values, running maximum and
-// sum (sigm: plain sums of independently weighted values).  grid (rows, H), a thread per value; nsplit <= 64.  Bound by latency: every
-// load is asked for at once, the maxima and sums by a lane each (as three loops over the parts, 17 rows of 8 heads of 256 took 8.9 us
+// sum (sigm: plain sums of independently weighted values).  grid (rows, H), a thread per value.  Bound by latency: every
+// load is asked for at once, the maxima and sums of 64 parts by a lane each (as three loops over the parts, 17 rows of 8 heads of 256 took 8.9 us
 // and 22 of 16 of 128 6.3; now 4.6 and 4.8, 78 of 16 7.4 and 4.0).
 template <typename T>
 __global__ void attend_merge_kernel(const float* __restrict__ ws, const T* __restrict__ gate, long sgate, int gate_elem,
@@ -268,8 +268,13 @@ __global__ void attend_merge_kernel(const float* __restrict__ ws, const T* __res
   const long row = blockIdx.x;
   const int h = blockIdx.y, lane = threadIdx.x & 63, r = threadIdx.x;
   const float* w = ws + (row * H + h) * nsplit * (long)(P + 2);
-  const float* part = w + (long)min(lane, nsplit - 1) * (P + 2) + P;
-  const float m = lane < nsplit && !sigm ? part[0] : -INFINITY, l = part[1];
+  float m, l;
+  auto stats = [&](int from) {             // of the 64 parts from there on
+    const float* part = w + (long)min(from + lane, nsplit - 1) * (P + 2) + P;
+    m = from + lane < nsplit && !sigm ? part[0] : -INFINITY;
+    l = part[1];
+  };
+  stats(0);
   const float sk = sink != nullptr ? sink[h] : -INFINITY;
   const float gh = gate != nullptr && !gate_elem ? ldf(gate + row * sgate + h) : 0.f;
   const float ge = gate != nullptr && gate_elem && r < P ? ldf(gate + row * sgate + (long)h * P + r) : 0.f;
@@ -280,20 +285,32 @@ __global__ void attend_merge_kernel(const float* __restrict__ ws, const T* __res
     for (int i = 0; i < B; ++i) v[i] = w[(long)min(b + i, nsplit - 1) * (P + 2) + min(r, P - 1)];
   };
   load(0);
-  const float M = fmaxf(mx_wave_max(m), sk);
-  const float e = m != -INFINITY ? expf(m - M) : 0.f;
+  float M = fmaxf(mx_wave_max(m), sk);
+  if (nsplit > 64) {
+    for (int from = 64; from < nsplit; from += 64) {
+      stats(from);
+      M = fmaxf(M, mx_wave_max(m));
+    }
+    stats(0);
+  }
+  float e = m != -INFINITY ? expf(m - M) : 0.f;
   auto of = [](float x, int i) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), i)); };
   float L = sink != nullptr ? expf(sk - M) : 0.f, a = 0.f;      // the sink counts once, not once per part
   for (int b = 0; b < nsplit; b += B) {
     if (b > 0) load(b);
+    if (b > 0 && b % 64 == 0) {
+      stats(b);
+      e = m != -INFINITY ? expf(m - M) : 0.f;
+    }
 #pragma unroll
     for (int i = 0; i < B; ++i) {
       if (b + i >= nsplit) break;
+      const int at = (b + i) & 63;
       if (sigm) {
         a += v[i];
-      } else if (of(m, b + i) != -INFINITY) {
-        L += of(l, b + i) * of(e, b + i);
-        a += v[i] * of(e, b + i);
+      } else if (of(m, at) != -INFINITY) {
+        L += of(l, at) * of(e, at);
+        a += v[i] * of(e, at);
       }
     }
   }

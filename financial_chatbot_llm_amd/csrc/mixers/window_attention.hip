@@ -751,7 +751,7 @@ MX_API int mx_window_attend(const void* q, long sq, const void* cache, const int
                             const float* sink, float scale, void* out, int dt, int S, int max_len, int H, int G,
                             int D, int P, int nsplit, float* ws, int rows, hipStream_t st) {
   if (S <= 0 || max_len <= 0) return 0;
-  if (P > 64 * WA_CPL || nsplit > 64 || G < 1 || H % G || window < 1 || keep < 0 ||
+  if (P > 64 * WA_CPL || G < 1 || H % G || window < 1 || keep < 0 ||
       (gate_elem && gate == nullptr) || (sink != nullptr && head_bias != nullptr) || (rel != nullptr && rel_len < 1))
     return (int)hipErrorInvalidValue;
   // 2: gate rows that 8-byte accesses may read (bf16)

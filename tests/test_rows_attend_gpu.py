@@ -170,6 +170,16 @@ def test_any_number_of_parts(dt, nsplit, monkeypatch):
     test_window(dt, SINGLES, (8, 1), {"window": 130, "keep_first": 70, "gate": "head", "sink": True})
 
 
+@pytest.mark.parametrize("nsplit", [63, 64, 65, 128, 150])
+def test_more_parts_than_lanes(nsplit, monkeypatch):
+    """A merging wave reads the statistics of 64 parts at a time: up to 150 parts, with and without keys of their own, in every group of 64."""
+    monkeypatch.setattr(mx, "_key_parts", lambda *a: nsplit)
+    segs = [(1, 6000), (2, 70), (1, 4500)]
+    test_window(torch.float32, segs, (4, 2), {"window": 1 << 40, "gate": "head", "sink": True})
+    test_window(torch.bfloat16, segs, (4, 4), {"window": 5000, "slopes": True, "gate": "elem"})
+    test_latent_f32(segs, 8, 32, 1 << 40)
+
+
 @pytest.mark.parametrize("segs", [SINGLES, RAGGED, LONG], ids=["singles", "ragged", "long"])
 @pytest.mark.parametrize("H,Dr,window", [(1, 32, 1), (8, 32, 1024), (70, 0, 1 << 40), (3, 0, 64), (32, 32, 65)])
 def test_latent_f32(segs, H, Dr, window):
