@@ -729,10 +729,15 @@ constexpr RowsTile kRowsTiles[] = {{2, 2, 4.6f, 13.6f}, {2, 4, 6.5f, 23.4f}, {4,
 // 74 tokens 1472 / 1141, 150 beside 9 rows 1457 / 1177, 120 beside 4 1423 / 1220, 100 beside 6 1277 / 1114, 200 1440 / 1349 (of which the widths of
 // 3112 - 4136 that are no multiples of 16 a part; decoding in bf16 they alone are 30 rows 677 / 625 and 695 / 649).  Errors against 64 bits at most the library's
 // (K = 1024 1.6 - 2.9e-7 of the norm against 2.9 - 5.8e-7, K = 3072 2.0 - 2.6e-7 against 5.0e-7).
-static int rows_plan(int M, int N, int K, int f32, float& best, int most = 256) {
-  if (M <= 0 || M > (f32 ? most : 2048) || N < 512 || N % 8 || K <= 0 || K % (f32 ? 32 : 64)) return 0;
+//
+// Beyond 256 rows of f32 the device's time meets the host's, and the line falls with the rows as that of bf16 does: from 20 us to 14.7 at 384, from
+// where whole passes are level or behind (none beyond 256 rows / this line; 8 layers of width 1024, two hybrid decoders and one whose passes the device bounds
+// earlier): 270 rows 1620 / 1480, 1604 / 1411, 1608 / 1505; 320 1624 / 1490, 1710 / 1531, 1628 / 1653; 350 1624 / 1600, 1696 / 1520, 1656 / 1674; 384 1631 /
+// 1642, 1689 / 1524, 1722 / 1743; products of up to 15 us at 400 rows 1778 / 1807, 1682 / 1630, 1762 / 1776, at 512 1784 / 1811, 1682 / 1717, 1901 / 1919.
+static int rows_plan(int M, int N, int K, int f32, float& best) {
+  if (M <= 0 || M > (f32 ? 384 : 2048) || N < 512 || N % 8 || K <= 0 || K % (f32 ? 32 : 64)) return 0;
   int plan = 0;
-  best = f32 ? (M <= 64 ? 11.f : M <= 256 ? 20.f : 15.f) : M <= 96 ? 60.f : M <= 512 ? 20.f : 20.f - (M - 512) / 128.f;
+  best = f32 ? (M <= 64 ? 11.f : M <= 256 ? 20.f : 20.f - (M - 256) / 24.f) : M <= 96 ? 60.f : M <= 512 ? 20.f : 20.f - (M - 512) / 128.f;
   for (int S = 1; S <= (f32 ? 8 : 4); S *= 2) {
     if (S > 1 && (K % (64 * S) || K / S < 256)) break;
     for (int i = 0; i < (f32 ? 4 : (int)(sizeof(kRowsTiles) / sizeof(kRowsTiles[0]))); ++i) {
@@ -748,14 +753,12 @@ static int rows_plan(int M, int N, int K, int f32, float& best, int most = 256) 
 
 PENNY_API int penny_linear_rows_plan(int M, int N, int K, int f32) {
   float us;
-  return rows_plan(M, N, K, f32, us);
+  return f32 && M > 256 ? 0 : rows_plan(M, N, K, f32, us);
 }
-// The same for f32 products of 257 to 384 rows, where the host's and the device's times meet: short ones (estimated up to 15 us: 1024 x 1024 338
-// rows 12 of the library / 14 here, and 1024 x 64 5.8 / 3.1), of which a step has enough to end up bound by the device (338 rows of 8 layers of width
-// 1024: host 1730 -> 1347 us, the whole 1695 -> 1693; 300 rows 1590 -> 1489; at 400 and more level or 1 % behind).
+// f32 of any number of rows: the rows beyond 256 are for calls whose host's time counts, no launches that a graph replays
 PENNY_API int penny_linear_rows_f32_plan(int M, int N, int K) {
   float us;
-  return M > 256 ? rows_plan(M, N, K, 1, us, 384) : 0;
+  return rows_plan(M, N, K, 1, us);
 }
 // the estimate of the plan for bf16, FLT_MAX where there is none
 extern "C" float penny_linear_rows_us(int M, int N, int K) {

@@ -305,10 +305,10 @@ def project(x: torch.Tensor, w: torch.Tensor, slabs: bool = False) -> Union[torc
                 y = torch.empty((M, N_), dtype=dt, device=x.device)
                 N.call("penny_linear_ring", xp, ldx, wp, K, y.data_ptr(), N_, None, 0, M, N_, tile, N.stream())
                 return y
-            if f32 and M > 256:
-                plan = 0 if replay else lib.penny_linear_rows_f32_plan(M, N_, K)
+            if replay:
+                plan = lib.penny_linear_rows_replay_plan(M, N_, K, f32)
             else:
-                plan = lib.penny_linear_rows_replay_plan(M, N_, K, f32) if replay else lib.penny_linear_rows_plan(M, N_, K, f32)
+                plan = lib.penny_linear_rows_f32_plan(M, N_, K) if f32 else lib.penny_linear_rows_plan(M, N_, K, 0)
             if plan:
                 S = plan >> 16
                 P = torch.empty((S, M, N_), dtype=torch.float32, device=x.device) if S > 1 else None
