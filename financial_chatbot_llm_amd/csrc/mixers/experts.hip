@@ -814,8 +814,20 @@ int tile_rows(long pairs, int experts, int dt, const Product* p, bool whole) {
   return avg <= 56 || t64 < 0.95 * t128 ? 64 : 128;
 }
 
+// f32 products in tiles of 64 tokens: four row groups of W a block, or eight (false)?  The matrix cores bound them, so what counts is how many
+// blocks the fullest CU has, and halves even that out where whole ones leave a round of 256 up to half empty: `likely` tiles (an expert's last
+// one half full) give x whole blocks a CU, of which halves cost half of ceil(2 x).  Both products in us, eight / four (three spreads of the buckets
+// by three seeds each): 32 experts of 1024 x 512, 33 rows on average (x = 1.02) 77 / 75, 50 (1.28) 97 / 89, 65 (1.52) 115 / 107, but 80 (1.75) 114 /
+// 127, 100 (2.06) 152 / 142, 120 (2.38) 177 / 155, 150 (2.84) 179 / 181; 8 of 2048 x 1024: 120 (1.19) 214 / 180, 200 (1.81) 217 / 245; 64 of 512 x 768
+// 60 (4.31) 148 / 137; from 8 rounds on level.  The line at 0.65 is for the estimate, which is a tile or two off: over 55 such sets of both products
+// 0.6 % and at most 5 % are lost to the better choice of each, with halves for all 1.2 % and 13 %, eight for all 4.2 % and 19 %.
+bool half_blocks(double likely, int groups) {
+  const double x = likely * ((groups + 7) / 8) / 256;
+  return x < 8 && x - floor(x) <= 0.65;
+}
+
 template <typename T, bool GLU>
-int expert_launch(const ExpertGemm& a, int mt, hipStream_t st) {
+int expert_launch(const ExpertGemm& a, int mt, double likely, hipStream_t st) {
   if (mt == 256) {
     const long grid = (long)a.ntiles * ((a.groups + 15) / 16);
     if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
@@ -827,8 +839,7 @@ int expert_launch(const ExpertGemm& a, int mt, hipStream_t st) {
       if (mt == 192) expert_tile_kernel<T, 192, 8, 2, GLU><<<(unsigned)grid, 256, 0, st>>>(a);
       else if (mt == 128) expert_tile_kernel<T, 128, 8, 2, GLU><<<(unsigned)grid, 256, 0, st>>>(a);
       else expert_tile_kernel<T, 64, 8, 2, GLU><<<(unsigned)grid, 256, 0, st>>>(a);
-    } else if (grid <= 768) {
-      // f32 blocks that all lie on the chip at once: whichever CU got one more takes a block's whole time longer, so halves of them (above)
+    } else if (half_blocks(likely, a.groups)) {
       expert_tile_kernel<T, 64, 4, 3, GLU><<<(unsigned)(a.ntiles * ((a.groups + 3) / 4)), 256, 0, st>>>(a);
     } else {
       expert_tile_kernel<T, 64, 8, 2, GLU><<<(unsigned)grid, 256, 0, st>>>(a);
@@ -906,13 +917,14 @@ MX_API int mx_experts(const void* h, long ldh, const int* idx, int T, int top, i
 #undef PLAN
   int rc = (int)hipGetLastError();
   if (rc) return rc;
+  const double likely = (double)P / mt + 0.5 * (P < E ? P : E);
   ExpertGemm a{h, ldh, W * es, src, top, tiles, ntiles, (const char*)w1, (long)g1 * k1 * 1024, k1, g1, act, lda, (int)lda,
                unit, limit, alpha, scale, own ? idx : nullptr, (int)P, E, pos, src, tiles};
   ExpertGemm b{act, lda, (int)lda * es, src, 0, tiles, ntiles, (const char*)w2, (long)g2 * k2 * 1024, k2, g2, ys, W, W,
                UNIT_NONE, 0.f, 0.f, nullptr, nullptr, 0, 0, nullptr, nullptr, nullptr};
-  if (glu) MX_DISPATCH(dt, TT, rc = expert_launch<TT, true>(a, mt, st));
-  else MX_DISPATCH(dt, TT, rc = expert_launch<TT, false>(a, mt, st));
+  if (glu) MX_DISPATCH(dt, TT, rc = expert_launch<TT, true>(a, mt, likely, st));
+  else MX_DISPATCH(dt, TT, rc = expert_launch<TT, false>(a, mt, likely, st));
   if (rc) return rc;
-  MX_DISPATCH(dt, TT, rc = expert_launch<TT, false>(b, mt, st));
+  MX_DISPATCH(dt, TT, rc = expert_launch<TT, false>(b, mt, likely, st));
   return rc;
 }

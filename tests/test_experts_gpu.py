@@ -76,7 +76,9 @@ def check(dtype, T, W, F_, E, top, unit, ident=0, skew=False, strided=False):
     (49, 128, 64, 1, 1, "relu2"),          # four, fewer stages of K than the ring holds
     (65, 192, 128, 1, 1, "clamped"),       # one row in the second tile
     (145, 192, 128, 1, 1, "silu"),         # bf16's second tile of 128: an odd number of groups
-    (3072, 2048, 64, 1, 1, "clamped"),     # f32's second product beyond 768 blocks
+    (3072, 2048, 64, 1, 1, "clamped"),     # f32's second product in blocks of four row groups ...
+    (2900, 2048, 64, 1, 1, "clamped"),     # ... and of eight
+    (320, 256, 1024, 8, 2, "silu"),        # f32's first product in blocks of eight
     (515, 192, 128, 2, 2, "silu"),
 ])
 def test_experts_against_float64(dtype, T, W, F_, E, top, unit):
