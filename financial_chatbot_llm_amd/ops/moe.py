@@ -406,13 +406,19 @@ MOE_NTF = tuple(int(v) for v in os.environ["PENNY_MOE_NTF"].split(",")) if "PENN
 
 
 def moe_ntf(P: int, E: int, F2: int, H: int) -> tuple:
-    """(W13, W2) row groups for P pairs over E experts.  W13: 2 while an expert has about 20 pairs, as its weights then stream faster (8
+    """(W13, W2) row groups for P pairs over E experts.  W13: 2 while an expert has fewer than 20 pairs, as its weights then stream faster (8
     experts of 4096 -> 28672, 16 / 48 / 64 / 80 / 96 tokens: 138 / 146 / 154 / 165 / 180 us, 4 groups 164 / 163 / 163 / 166 / 167); 4
-    beyond, for half the reads of activations.  W2: 2 where 4 would leave fewer than 512 workgroups (14336 -> 4096, 1 / 4 tokens: 18.7 /
-    36.1, 4 groups 23.4 / 37.1), else 4 (48 / 64 tokens 72 / 74, 2 groups 75 / 84)."""
+    beyond, for half the reads of activations.  W2: with as few pairs 2 where 4 would leave fewer than 512 workgroups (14336 -> 4096, 1 / 4
+    tokens: 18.7 / 36.1, 4 groups 23.4 / 37.1), else 4 (48 / 64 tokens 72 / 74, 2 groups 75 / 84).  Two-layer steps of seven sizes (8 to 64
+    experts, widths of 1024 to 8192, 1 to 200 tokens) take at most 4 % longer than with the best of the four pairs, and up to 10 % less than with 4
+    for both.
+
+    The number of groups also sets how many waves share the sum over K, and so the order of its f32 additions: a token's expert rows are
+    those of another batch but for that order (its rounding to bf16 may fall the other way), as with the split of K in the dense products."""
     if MOE_NTF is not None:
         return MOE_NTF
-    return 2 if P <= 20 * E and F2 % 64 == 0 else 4, 2 if min(P, E) * H < 64 * 512 and H % 64 == 0 else 4
+    few = P < 20 * E
+    return 2 if few and F2 % 64 == 0 else 4, 2 if few and min(P, E) * H < 64 * 512 and H % 64 == 0 else 4
 
 
 class MoEWorkspace:

@@ -49,6 +49,31 @@ def test_pairs_by_expert(K, epi, ntf):
     assert bool((err <= tol).all()), float((err / tol).max())
 
 
+@pytest.mark.parametrize("K", [256, 1536, 4096, 14336])
+def test_widths_agree(K):
+    """One token's row of an expert in a small batch and in a large one, whose products split K over other numbers of waves."""
+    g = torch.Generator().manual_seed(K)
+    n, P = 128, 40
+    w8, s = moe.quantize_fp8_rowwise(torch.randn(1, n, K, generator=g) * K ** -0.5)
+    x8 = torch.randn(P, K, generator=g).to(torch.float8_e4m3fn)
+    xs, rw = torch.rand(P, generator=g) + 0.5, torch.ones(P)
+    wt, d = moe.tile_fp8_weight(w8.cuda()), [t.cuda().contiguous() for t in (x8.view(torch.uint8), xs, s, rw)]
+
+    def rows(first, count, ntf):
+        y = torch.zeros(count, n, dtype=torch.bfloat16, device="cuda")
+        off = torch.tensor([0, count], dtype=torch.int32, device="cuda")
+        N.call("penny_moe_gemm_fp8", N.ptr(d[0][first:]), N.ptr(d[1][first:]), None, N.ptr(off), N.ptr(wt), N.ptr(d[2]), N.ptr(d[3][first:]), N.ptr(y),
+               1, n, K, 2, ntf, N.stream())
+        return y.double()
+    thin, wide = rows(7, 1, 2), rows(0, P, 4)[7:8]
+    W = w8.view(torch.float8_e4m3fn).double().cuda()[0] * s.double().cuda()[0][:, None]
+    size = (x8.double().cuda()[7:8] * xs.double().cuda()[7]).abs() @ W.abs().t()
+    # either sum is within K 2^-24 of the magnitudes and the matrix unit's own cut (above), and is rounded to bf16
+    assert ((thin - wide).abs() <= 2 * (K * 2.0 ** -24 + 2.0 ** -17) * size + 2.0 ** -7 * wide.abs()).all()
+    assert torch.equal(rows(7, 1, 4), wide)                    # of one width, whatever the batch: the same bits
+
+
 def test_row_groups():
     assert moe.moe_ntf(96, 8, 28672, 4096) == (2, 4) and moe.moe_ntf(320, 8, 28672, 4096) == (4, 4)
+    assert moe.moe_ntf(159, 8, 28672, 2048) == (2, 2) and moe.moe_ntf(160, 8, 28672, 2048) == (4, 4)
     assert moe.moe_ntf(2, 8, 28672, 4096) == (2, 2) and moe.moe_ntf(16, 8, 28688, 4080) == (4, 4)
