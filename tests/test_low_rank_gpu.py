@@ -40,6 +40,22 @@ def test_against_float64(dt, T, ra, na, rg, ng, monkeypatch):
     check(a, g, ua, wa, ug, wg, dt)
 
 
+@pytest.mark.parametrize("K", [32, 64])
+@pytest.mark.parametrize("spread", [0.0, 2.0])
+def test_no_less_exact_than_the_f32_product(K, spread):
+    """The sums over exact pieces of the weights against those of the product that they stand for, on f32 rows of the same values: weights of one size,
+    and spread over some orders of magnitude."""
+    ua, wa, _, _ = operands(torch.bfloat16, 1500, K, 2048, 0, 0, seed=K)
+    g = torch.Generator(device="cuda").manual_seed(K)
+    wa = wa * torch.exp(spread * torch.randn(wa.shape, generator=g, device="cuda"))
+    want, size = ua.double() @ wa.double().t(), ua.double().abs() @ wa.double().abs().t()
+    here, before = ((y.double() - want).abs() for y in (mx.low_rank(ua, wa)[0], torch.nn.functional.linear(ua.float(), wa)))
+    assert here.norm() <= before.norm()
+    # three products for each 32 of K, each of which adds 32 terms to the sum: K / 32 * 3 roundings of at most 2^-24 of the magnitudes, and as much again
+    # for what the unit cuts while it aligns a product's terms
+    assert (here <= K / 32 * 6 * 2.0 ** -24 * size).all(), float((here / size).max() * 2 ** 24)
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 def test_values_that_are_not_finite(dt):
     ua, wa, ug, wg = operands(dt, 40, 64, 96, 64, 96)

@@ -72,6 +72,30 @@ def test_widths_in_eights(dt, M, N_, K):
     assert torch.equal(p.materialize() if isinstance(p, G.Slabs) else p, y)
 
 
+@pytest.mark.parametrize("f32,nf,mt", [(1, 2, 2), (1, 2, 4), (1, 4, 2), (1, 2, 6), (0, 2, 2), (0, 2, 8), (0, 4, 4), (0, 8, 8), (0, 4, 12)])
+def test_widths_in_eights_by_tile(f32, nf, mt):
+    """The half-filled last sixteen in the native launch itself, whatever the rule of ``project`` says: tiles that end before, in and behind it, rows in one
+    and several chunks, whole K and slices, which are also read as they are left; nothing is written behind the result."""
+    from financial_chatbot_llm_amd.ops import _native as N
+    g = torch.Generator(device="cuda").manual_seed(nf * 100 + mt)
+    dt = torch.float32 if f32 else torch.bfloat16
+    for N_, K in ((520, 512), (1032, 1024), (3208, 512)):
+        w = (torch.randn((N_, K), generator=g, device="cuda") * K ** -0.5).to(dt)
+        for M in (1, 16 * mt, 16 * mt + 1, 3 * 16 * mt - 5):
+            x = torch.randn((M, K), generator=g, device="cuda").to(dt)
+            want = x.double() @ w.double().t()
+            bound = want.abs() * (2.0 ** -22 if f32 else 2.0 ** -8) + 2.0 ** -22 * K ** 0.5        # as in test_every_tile
+            for S in (1, 2, 4):
+                y = torch.full((M + 1, N_), 7.0, dtype=dt, device="cuda")
+                slabs = torch.full((S + 1, M, N_), 7.0, device="cuda") if S > 1 else None
+                for out in (y, None) if S > 1 else (y,):
+                    N.call("penny_linear_rows", N.ptr(x), K, N.ptr(w), K, N.ptr(out), M, N_, N.ptr(slabs), S, nf, mt, f32, 1, N.stream())
+                    if S > 1:
+                        assert ((slabs[:S].double().sum(0) - want).abs() <= 2.0 ** -22 * (want.abs() + K ** 0.5)).all(), (N_, M, S)
+                        assert (slabs[S] == 7).all()
+                assert ((y[:M].double() - want).abs() <= bound).all() and (y[M] == 7).all(), (N_, M, S)
+
+
 @pytest.mark.parametrize("M,N_,K,here", [(256, 1024, 1024, True), (257, 1024, 1024, True), (384, 1024, 64, True), (338, 520, 32, True), (385, 1024, 64, False),
                                          (338, 6144, 1024, False)])
 def test_short_f32_products(M, N_, K, here, monkeypatch):
