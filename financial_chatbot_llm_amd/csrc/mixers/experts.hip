@@ -597,9 +597,8 @@ __global__ void __launch_bounds__(512) expert_wide_kernel(ExpertGemm a) {
 // reader of its rows.  Bound by latency: one read of the indices and three passes through LDS, 1 - 3 us of the product for the 4 of the
 // launch (passes of 1 - 64 rows with four such layers 1 - 13 us shorter: f32 1 row 592 / 583, 60 rows of width 1024 665 / 652, of 2048 1027 / 1020).
 // own: the tile's pairs.  Returns (expert, first sorted row, rows, -).
-template <int NW>
 __device__ __forceinline__ int4 plan_tile(const ExpertGemm& a, int* own) {
-  constexpr int THREADS = NW * 64, C = 1024 / THREADS;
+  constexpr int NW = 4, THREADS = NW * 64, C = 1024 / THREADS;
   __shared__ int count[64], found[C][NW];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, y = blockIdx.y, E = a.experts;
   const bool leave = blockIdx.x == 0;
@@ -664,19 +663,20 @@ __device__ __forceinline__ int4 plan_tile(const ExpertGemm& a, int* own) {
   return tile;
 }
 
-// Two row groups x 16 tokens per block; the NW waves share the pieces of K, their partial sums meet in LDS.  Bound by the weights' stream,
+// Two row groups x 16 tokens per block; the four waves share the pieces of K, their partial sums meet in LDS.  Bound by the weights' stream,
 // past the caches as each is read once: four steps of weights and rows are always in flight per wave, and thin blocks of long streams
 // keep many of them at it.  Both products in us, four groups x 4 waves that drain every eight steps (before) / the same drained never /
-// two groups x 4 waves / two groups x 2 waves: 32 experts of 1024 x 2048, top 4, 1 token 19.5 / 15.9 / 15.9 / 15.8, 16 tokens 71 / 70 / 62 / 61, 64 tokens 80 /
-// 79 / 70 / 70 (5.8 TB/s), f32 156 / 164 / 142 / 135; 8 of 2048 x 4096, 16 tokens 85 / 90 / 76 / 71; 16 of 512 x 1024, 8 tokens 17.3 / 14.8
-// / 14.8 / 14.7.  Eight steps in flight measured the same.
-template <typename T, bool GLU, bool PLAN, int NW>
-__global__ void __launch_bounds__(NW * 64) expert_stream_kernel(ExpertGemm a) {
-  constexpr int ES = sizeof(T), NF = 2, D = 4;
+// two groups x 4 waves: 32 experts of 1024 x 2048, top 4, 1 token 19.5 / 15.9 / 15.9, 16 tokens 71 / 70 / 62, 64 tokens 80 / 79 / 70 (5.8 TB/s), f32
+// 156 / 164 / 142; 8 of 2048 x 4096, 16 tokens 85 / 90 / 76; 16 of 512 x 1024, 8 tokens 17.3 / 14.8 / 14.8.  Eight steps in flight measured the
+// same.  Two waves a block where the blocks alone fill the chip gained up to 6 % more (f32 135, 16 tokens of the large ones 71), but then the order of
+// a row's sum, and with it the rounding of its result, depends on how many rows the step has.
+template <typename T, bool GLU, bool PLAN>
+__global__ void __launch_bounds__(256) expert_stream_kernel(ExpertGemm a) {
+  constexpr int ES = sizeof(T), NF = 2, NW = 4, D = 4;
   __shared__ f32x4 red[NW][NF][64];
   __shared__ int own[16];
   int4 tile;
-  if constexpr (PLAN) tile = plan_tile<NW>(a, own);
+  if constexpr (PLAN) tile = plan_tile(a, own);
   else tile = a.tiles[blockIdx.y];
   const int rows = tile.z;
   if (rows == 0) return;
@@ -847,13 +847,8 @@ int expert_launch(const ExpertGemm& a, int mt, double likely, hipStream_t st) {
   } else {
     if (a.ntiles > 65535) return (int)hipErrorInvalidValue;
     const dim3 grid((a.groups + 1) / 2, a.ntiles);
-    // two waves a block where the blocks alone fill the chip, four otherwise (us of both products: above)
-    const bool many = (long)a.ntiles * (a.groups / 4) >= 512;
-    if (a.idx != nullptr) {
-      if (many) expert_stream_kernel<T, GLU, true, 2><<<grid, 128, 0, st>>>(a);
-      else expert_stream_kernel<T, GLU, true, 4><<<grid, 256, 0, st>>>(a);
-    } else if (many) expert_stream_kernel<T, GLU, false, 2><<<grid, 128, 0, st>>>(a);
-    else expert_stream_kernel<T, GLU, false, 4><<<grid, 256, 0, st>>>(a);
+    if (a.idx != nullptr) expert_stream_kernel<T, GLU, true><<<grid, 256, 0, st>>>(a);
+    else expert_stream_kernel<T, GLU, false><<<grid, 256, 0, st>>>(a);
   }
   return (int)hipGetLastError();
 }

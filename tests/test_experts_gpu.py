@@ -184,3 +184,18 @@ def test_blocks_that_plan_for_themselves(dtype, T, E, top, ident, skew):
     """Around 1024 pairs and 64 experts, beyond which the plan is a launch: buckets of one tile, of several and empty ones, identity entries."""
     check(dtype, T, 256, 64, E, top, "clamped", ident=ident, skew=skew)
     check(dtype, T, 256, 64, E, top, "silu", ident=ident, skew=skew)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rows_do_not_depend_on_the_step(dtype):
+    """A token's expert rows alone and among 64 tokens, both in the stream form: the same bits."""
+    from financial_chatbot_llm_amd.ops import mixers as mx
+    T, E, W, F_, top = 64, 32, 1024, 512, 4
+    g = torch.Generator().manual_seed(2)
+    w1 = mx.pack_experts([tuple((torch.randn(F_, W, generator=g) * W ** -0.5).to("cuda", dtype) for _ in range(2)) for _ in range(E)], dtype)
+    w2 = mx.pack_experts([(torch.randn(W, F_, generator=g) * F_ ** -0.5).to("cuda", dtype) for _ in range(E)], dtype)
+    h, idx = torch.randn(T, W, generator=g).to("cuda", dtype), torch.rand(T, E, generator=g).topk(top, -1).indices.int().cuda()
+    ys, pos = mx.experts(h, idx, w1, w2, "clamped", LIMIT, ALPHA)
+    for t in (0, 17, 63):
+        y1, p1 = mx.experts(h[t:t + 1], idx[t:t + 1].contiguous(), w1, w2, "clamped", LIMIT, ALPHA)
+        assert torch.equal(ys[pos[t].long()], y1[p1[0].long()])
