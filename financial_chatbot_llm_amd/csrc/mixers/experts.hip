@@ -55,7 +55,7 @@ struct ExpertGemm {
   int unit;
   float limit, alpha;
   const float* scale;   // per pair, on the expert's input (or null)
-  // stream form with a plan of its own (plan_tile): the pairs' experts, and where the plan goes for what comes after
+  // stream form with a plan of its own (plan_tile): the pairs' experts (null: without), and where the plan goes for what comes after
   const int* idx;
   int pairs, experts;
   int *pos, *src_out;
@@ -597,8 +597,9 @@ __global__ void __launch_bounds__(512) expert_wide_kernel(ExpertGemm a) {
 // reader of its rows.  Bound by latency: one read of the indices and three passes through LDS, 1 - 3 us of the product for the 4 of the
 // launch (passes of 1 - 64 rows with four such layers 1 - 13 us shorter: f32 1 row 592 / 583, 60 rows of width 1024 665 / 652, of 2048 1027 / 1020).
 // own: the tile's pairs.  Returns (expert, first sorted row, rows, -).
+template <int NW>
 __device__ __forceinline__ int4 plan_tile(const ExpertGemm& a, int* own) {
-  constexpr int NW = 4, THREADS = NW * 64, C = 1024 / THREADS;
+  constexpr int THREADS = NW * 64, C = 1024 / THREADS;
   __shared__ int count[64], found[C][NW];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, y = blockIdx.y, E = a.experts;
   const bool leave = blockIdx.x == 0;
@@ -663,20 +664,20 @@ __device__ __forceinline__ int4 plan_tile(const ExpertGemm& a, int* own) {
   return tile;
 }
 
-// Two row groups x 16 tokens per block; the four waves share the pieces of K, their partial sums meet in LDS.  Bound by the weights' stream,
+// Two row groups x 16 tokens per block; the NW waves share the four quarters of K, whose sums meet in LDS.  Bound by the weights' stream,
 // past the caches as each is read once: four steps of weights and rows are always in flight per wave, and thin blocks of long streams
 // keep many of them at it.  Both products in us, four groups x 4 waves that drain every eight steps (before) / the same drained never /
-// two groups x 4 waves: 32 experts of 1024 x 2048, top 4, 1 token 19.5 / 15.9 / 15.9, 16 tokens 71 / 70 / 62, 64 tokens 80 / 79 / 70 (5.8 TB/s), f32
-// 156 / 164 / 142; 8 of 2048 x 4096, 16 tokens 85 / 90 / 76; 16 of 512 x 1024, 8 tokens 17.3 / 14.8 / 14.8.  Eight steps in flight measured the
-// same.  Two waves a block where the blocks alone fill the chip gained up to 6 % more (f32 135, 16 tokens of the large ones 71), but then the order of
-// a row's sum, and with it the rounding of its result, depends on how many rows the step has.
-template <typename T, bool GLU, bool PLAN>
-__global__ void __launch_bounds__(256) expert_stream_kernel(ExpertGemm a) {
-  constexpr int ES = sizeof(T), NF = 2, NW = 4, D = 4;
-  __shared__ f32x4 red[NW][NF][64];
+// two groups x 4 waves / two groups x 2 waves: 32 experts of 1024 x 2048, top 4, 1 token 19.5 / 15.9 / 15.9 / 15.8, 16 tokens 71 / 70 / 62 / 61, 64 tokens 80 /
+// 79 / 70 / 70 (5.8 TB/s), f32 156 / 164 / 142 / 135; 8 of 2048 x 4096, 16 tokens 85 / 90 / 76 / 71; 16 of 512 x 1024, 8 tokens 17.3 / 14.8
+// / 14.8 / 14.7.  Eight steps in flight measured the same.  Two waves have two quarters each, summed apart: the order of a row's sum, and with it
+// its bits, must not follow from how many rows the step has.
+template <typename T, bool GLU, bool PLAN, int NW>
+__global__ void __launch_bounds__(NW * 64) expert_stream_kernel(ExpertGemm a) {
+  constexpr int ES = sizeof(T), NF = 2, D = 4, QW = 4 / NW;
+  __shared__ f32x4 red[4][NF][64];
   __shared__ int own[16];
   int4 tile;
-  if constexpr (PLAN) tile = plan_tile(a, own);
+  if constexpr (PLAN) tile = plan_tile<NW>(a, own);
   else tile = a.tiles[blockIdx.y];
   const int rows = tile.z;
   if (rows == 0) return;
@@ -684,6 +685,7 @@ __global__ void __launch_bounds__(256) expert_stream_kernel(ExpertGemm a) {
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, col = lane & 15;
   const int G = blockIdx.x * NF;
   const int k0 = a.kt * w / NW, steps = a.kt * (w + 1) / NW - k0;
+  const int mid = QW == 2 ? a.kt * (2 * w + 1) / 4 - k0 : 0;  // the wave's second quarter begins
   const char* wp[NF];
 #pragma unroll
   for (int f = 0; f < NF; ++f)
@@ -705,7 +707,12 @@ __global__ void __launch_bounds__(256) expert_stream_kernel(ExpertGemm a) {
     }
     bv[d] = *reinterpret_cast<const uint4*>(k * 64 < behind ? xp + k * 64 : zero);
   };
-  auto use = [&](int d) {
+  auto first = [&] {                                         // quarter done: its sum aside
+#pragma unroll
+    for (int f = 0; f < NF; ++f) red[QW * w][f][lane] = acc[f], acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  auto use = [&](int d, int k) {
+    if (QW == 2 && k == mid) first();
 #pragma unroll
     for (int f = 0; f < NF; ++f) acc[f] = mma16<T>(av[d][f], bv[d], acc[f]);
   };
@@ -716,7 +723,7 @@ __global__ void __launch_bounds__(256) expert_stream_kernel(ExpertGemm a) {
   for (; k + 2 * D <= steps; k += D) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      use(d);
+      use(d, k + d);
       fetch(d, k + D + d);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -724,17 +731,18 @@ __global__ void __launch_bounds__(256) expert_stream_kernel(ExpertGemm a) {
   for (; k < steps; k += D) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      if (k + d < steps) use(d);
+      if (k + d < steps) use(d, k + d);
       if (k + D + d < steps) fetch(d, k + D + d);
     }
   }
+  if (QW == 2 && mid >= steps) first();
 #pragma unroll
-  for (int f = 0; f < NF; ++f) red[w][f][lane] = acc[f];
+  for (int f = 0; f < NF; ++f) red[QW * w + QW - 1][f][lane] = acc[f];
   __syncthreads();
   auto total = [&](int i) {
     f32x4 s = red[0][i][lane];
 #pragma unroll
-    for (int v = 1; v < NW; ++v) s += red[v][i][lane];
+    for (int v = 1; v < 4; ++v) s += red[v][i][lane];
     return s;
   };
   if (col >= rows) return;
@@ -847,8 +855,14 @@ int expert_launch(const ExpertGemm& a, int mt, double likely, hipStream_t st) {
   } else {
     if (a.ntiles > 65535) return (int)hipErrorInvalidValue;
     const dim3 grid((a.groups + 1) / 2, a.ntiles);
-    if (a.idx != nullptr) expert_stream_kernel<T, GLU, true><<<grid, 256, 0, st>>>(a);
-    else expert_stream_kernel<T, GLU, false><<<grid, 256, 0, st>>>(a);
+    // two waves a block where the blocks alone fill the chip, four otherwise (us of both products: above) and for the more rows of f32, whose
+    // matrix work then counts (32 experts of 2048 x 2048, 24 rows each 531 with two, 510; 12 rows 317 and 313, 2 rows 240 and 245)
+    const bool many = (long)a.ntiles * (a.groups / 4) >= 512 && a.pairs <= 12L * a.experts;
+    if (a.idx != nullptr) {
+      if (many) expert_stream_kernel<T, GLU, true, 2><<<grid, 128, 0, st>>>(a);
+      else expert_stream_kernel<T, GLU, true, 4><<<grid, 256, 0, st>>>(a);
+    } else if (many) expert_stream_kernel<T, GLU, false, 2><<<grid, 128, 0, st>>>(a);
+    else expert_stream_kernel<T, GLU, false, 4><<<grid, 256, 0, st>>>(a);
   }
   return (int)hipGetLastError();
 }
@@ -916,7 +930,7 @@ MX_API int mx_experts(const void* h, long ldh, const int* idx, int T, int top, i
   ExpertGemm a{h, ldh, W * es, src, top, tiles, ntiles, (const char*)w1, (long)g1 * k1 * 1024, k1, g1, act, lda, (int)lda,
                unit, limit, alpha, scale, own ? idx : nullptr, (int)P, E, pos, src, tiles};
   ExpertGemm b{act, lda, (int)lda * es, src, 0, tiles, ntiles, (const char*)w2, (long)g2 * k2 * 1024, k2, g2, ys, W, W,
-               UNIT_NONE, 0.f, 0.f, nullptr, nullptr, 0, 0, nullptr, nullptr, nullptr};
+               UNIT_NONE, 0.f, 0.f, nullptr, nullptr, (int)P, E, nullptr, nullptr, nullptr};
   if (glu) MX_DISPATCH(dt, TT, rc = expert_launch<TT, true>(a, mt, likely, st));
   else MX_DISPATCH(dt, TT, rc = expert_launch<TT, false>(a, mt, likely, st));
   if (rc) return rc;
