@@ -1069,7 +1069,7 @@ def low_rank(ua: torch.Tensor, wa: torch.Tensor, ug: Optional[torch.Tensor] = No
     plain = not torch.is_autocast_enabled() and not any(t is not None and t.requires_grad for t in (ua, wa, ug, wg))
     if plain and N.use_native(ua) and T > 0 and ra in (32, 64) and na % 16 == 0 and wa.dtype == torch.float32 and wa.shape[1] == ra and wa.is_contiguous() and \
             ua.dtype in (torch.bfloat16, torch.float32) and ua.stride(1) == 1 and ua.stride(0) * ua.element_size() % 16 == 0 and ua.stride(0) >= ra and \
-            (ua.data_ptr() | wa.data_ptr()) % 16 == 0 and T <= 1 << 23:
+            (ua.data_ptr() | wa.data_ptr()) % 16 == 0 and T <= 128 * 65535:
         ng = 0 if ug is None else wg.shape[0]
         if ng == 0 or (ug.shape[0] == T and ug.shape[1] in (32, 64) and ug.shape[1] <= ug.stride(0) and wg.shape[1] == ug.shape[1] and ng % 16 == 0 and ug.stride() == ua.stride() and
                        ug.dtype == wg.dtype == ua.dtype and wg.is_contiguous() and (ug.data_ptr() | wg.data_ptr()) % 16 == 0):

@@ -97,3 +97,14 @@ def test_autocast_and_gradients(dt):
         size = (w if i % 2 == 0 else u).double().abs().sum(0)
         assert ((ts[i].grad.double() - want).abs() <= e * want.abs() + 80 * 2.0 ** -24 * size).all()
     assert not any(t.requires_grad for t in mx.low_rank(ua, wa, ug, wg))
+
+
+@pytest.mark.parametrize("T,here", [(128 * 65535, True), (128 * 65535 + 1, False), (1 << 23, False)])
+def test_most_rows(T, here, monkeypatch):
+    """The launch has a block of its grid for each 128 rows; more rows are the product's."""
+    ua = torch.ones((T, 32), dtype=torch.bfloat16, device="cuda")
+    ua[-1] = 2.0
+    calls, mcall = [], N.mcall
+    monkeypatch.setattr(N, "mcall", lambda name, *a: (calls.append(name), mcall(name, *a))[1])
+    a, _ = mx.low_rank(ua, torch.ones((16, 32), device="cuda"))
+    assert bool(calls) is here and (a[:-1] == 32.0).all() and (a[-1] == 64.0).all()
